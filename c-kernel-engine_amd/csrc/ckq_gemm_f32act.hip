@@ -1,0 +1,360 @@
+/*
+ * ckq_gemm_f32act.hip - several tokens of fp32 activations against Q4_K, Q6_K or Q8_0 weights, nothing
+ * quantized, on the bf16 matrix cores with fp32 precision.
+ *
+ *   C[t][n] = sum over scale groups s:  scale(n,s) * sum_{k in s} q(n,k) * x(t,k)  [- dmin * m(n,s) * sum_{k in s} x(t,k)]  (+ bias[n])
+ * (reference: gemm_kernels_q4k.c:53-101, gemm_kernels_q6k.c:39-76, gemm_kernels_q8_0.c:254-277, under the token
+ * loops of gemm_nt_q4_k / _q6_k / _q8_0).
+ *
+ * Exactness.  The integers q (4 to 8 bits) are exact in bf16.  An fp32 activation is cut into three bf16 parts,
+ * x = hi + mid + lo, each the leading 8 bits of what is left: 24 bits, so the cut is exact.  Every product of an
+ * integer and a part fits fp32, the matrix core adds in fp32, and the scale is applied to the sum of a group in
+ * fp32: the only roundings are those of fp32 additions, one per group and one per product as before.
+ *
+ * Mapping.  v_mfma_f32_32x32x16_bf16, tokens as rows (A), weight rows as columns (B): a lane holds ONE weight row,
+ * so its scale is a register of the lane and one multiply-add per output and group applies it.  A lane (column
+ * l % 32, half l / 32) takes the elements its half of the raw bytes holds, straight from memory; the activations are
+ * read in the same order, so no byte moves between lanes.  The min term of Q4_K is one more MFMA per 64 elements:
+ * the lane's share of the two sub-block sums of x, cut in three like x, against the two mins.
+ *
+ * Block = 8 waves on one tile of 32 tokens x 32 R weight rows; the waves cut K into eight contiguous runs and add
+ * their partial tiles through LDS in wave order.  Each wave loads its own activations one step ahead, 256 contiguous bytes
+ * per token, and turns them through LDS (a lane loading its own row would touch 64 cache lines per instruction: 40 us
+ * instead of 36 at 96 x 4096 x 4096, Q6_K; one token per pass over the weights, as the streaming kernel does it, 245 us);
+ * no other wave reads them, so the loop has no barrier.  Cutting the activations in a launch of its own and reading the
+ * parts back (6 bytes per element instead of 4) was slower: 41 us.
+ *
+ * Grid: token groups fastest, so the blocks that share weights run side by side.
+ * Bound: what a CU can load from L2 (8 KiB of activations and 64 rows of weights per wave and step) next to VALU issue
+ * (per 64 elements and 32 rows: 60-110 operations to form the integers and apply the scales, 210 / R to cut x).
+ */
+#include "ckq_gemm_common.hpp"
+#include "ckq_gemm_f32act.hpp"
+
+namespace {
+
+constexpr int F32_WAVES = 8;
+
+__device__ __forceinline__ u32 pack_bf16(float lo, float hi)      /* two floats whose low 16 bits are to be dropped */
+{
+    return __builtin_amdgcn_perm(__builtin_bit_cast(u32, hi), __builtin_bit_cast(u32, lo), 0x07060302u);
+}
+
+/* eight floats -> their three bf16 parts as MFMA operands */
+struct Cut { ckq_v4i hi, mid, lo; };
+__device__ __forceinline__ float top16(float v) { return __builtin_bit_cast(float, __builtin_bit_cast(u32, v) & 0xffff0000u); }
+/* The lower parts are taken from v clamped to the finite range: of an infinity only the first part matters, and it
+ * must not meet the NaN that inf - inf would leave in the others. */
+__device__ __forceinline__ float finite(float v) { return __builtin_amdgcn_fmed3f(v, -3.402823466e38f, 3.402823466e38f); }
+__device__ __forceinline__ void cut8(const float *x, Cut &c)
+{
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float m[2], l[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const float v = finite(x[2 * i + j]);
+            m[j] = v - top16(v);
+            l[j] = m[j] - top16(m[j]);
+        }
+        c.hi[i]  = (int)pack_bf16(x[2 * i], x[2 * i + 1]);
+        c.mid[i] = (int)pack_bf16(m[0], m[1]);
+        c.lo[i]  = (int)pack_bf16(l[0], l[1]);
+    }
+}
+
+__device__ __forceinline__ ckq_v16f mfma_bf16(ckq_v4i a, ckq_v4i b, ckq_v16f c)
+{
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(ckq_v8bf, a), __builtin_bit_cast(ckq_v8bf, b), c, 0, 0, 0);
+}
+
+/* Signed byte i of a dword as a float, in one instruction (the compiler extends the byte with an instruction of its own). */
+__device__ __forceinline__ float sbyte_f32(u32 v, int i)
+{
+    float f;
+    switch (i) {
+    case 0: asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_0" : "=v"(f) : "v"(v)); break;
+    case 1: asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_1" : "=v"(f) : "v"(v)); break;
+    case 2: asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_2" : "=v"(f) : "v"(v)); break;
+    default: asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_3" : "=v"(f) : "v"(v)); break;
+    }
+    return f;
+}
+
+/* Eight signed bytes -> bf16x8 (exact). */
+__device__ __forceinline__ ckq_v4i bytes_to_bf16(u32 b0, u32 b1)
+{
+    ckq_v4i o;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        o[i]     = (int)pack_bf16(sbyte_f32(b0, 2 * i), sbyte_f32(b0, 2 * i + 1));
+        o[2 + i] = (int)pack_bf16(sbyte_f32(b1, 2 * i), sbyte_f32(b1, 2 * i + 1));
+    }
+    return o;
+}
+
+/* ---- formats ------------------------------------------------------------------------------------
+ * STEP elements of K per step, NG scale groups of 8 * NK elements per lane half in it.
+ *   Raw / load      the step's bytes of one weight row that this lane's half decodes
+ *   src_elem(c)     first element of 16-byte chunk c (0..15) of the step's activations
+ *   chunk(g, h, i)  which chunk holds floats 4 i .. 4 i + 3 of group g for lane half h
+ *   operand(g, i)   bf16x8 of the lane's elements 8 i .. 8 i + 7 of group g
+ *   scale(g)        fp32 factor of the group; MIN: min_operand / dmin for the min term */
+struct F32Q4K {
+    static constexpr int STEP = 64, NG = 2, NK = 2;
+    static constexpr bool MIN = true;
+    struct Raw { u32 hdr[4], qs[4]; };
+    static __device__ __forceinline__ void load(Raw &w, const uint8_t *row, int step, int h, int)
+    {
+        const uint8_t *blk = row + (u32)(step >> 2) * 144u;
+        ld16<4>(w.hdr, blk);
+        ld16<4>(w.qs, blk + 16 + 32 * (step & 3) + 16 * h);
+    }
+    static __device__ __forceinline__ u32 src_elem(int step, int c, int) { return 64u * (u32)step + 4u * c; }
+    static __device__ __forceinline__ int chunk(int g, int h, int i) { return 8 * g + 4 * h + i; }
+    static __device__ __forceinline__ bool live(int, int, int) { return true; }
+    struct Dec { float s[2], dmin; ckq_v4i mins; };
+    static __device__ __forceinline__ void decode(Dec &d, const Raw &w, int step)
+    {
+        u32 sc2, mn2;
+        k4_scale_pair(w.hdr[1], w.hdr[2], w.hdr[3], step & 3, &sc2, &mn2);
+        const float dd = h2f(w.hdr[0] & 0xffff);
+        d.s[0] = dd * (float)(sc2 & 0xff);
+        d.s[1] = dd * (float)((sc2 >> 8) & 0xff);
+        d.dmin = h2f(w.hdr[0] >> 16);
+        const float m0 = (float)(mn2 & 0xff), m1 = (float)((mn2 >> 8) & 0xff);
+        d.mins = ckq_v4i{(int)pack_bf16(m0, m0), (int)pack_bf16(m0, m1), (int)pack_bf16(m1, m1), 0};
+    }
+    static __device__ __forceinline__ ckq_v4i operand(const Raw &w, int g, int i)
+    {
+        const u32 a = g ? w.qs[2 * i] >> 4 : w.qs[2 * i], b = g ? w.qs[2 * i + 1] >> 4 : w.qs[2 * i + 1];
+        return bytes_to_bf16(a & 0x0f0f0f0fu, b & 0x0f0f0f0fu);
+    }
+};
+
+struct F32Q6K {
+    static constexpr int STEP = 64, NG = 4, NK = 1;       /* a step: 16-runs o of the four 32-runs of one 128-half n */
+    static constexpr bool MIN = false;
+    struct Raw { u32 ql0[2], ql1[2], qh[2], sc[2], d; };
+    static __device__ __forceinline__ void load(Raw &w, const uint8_t *row, int step, int h, int)
+    {
+        const uint8_t *blk = row + (u32)(step >> 2) * 210u;
+        const int n = (step >> 1) & 1, o = step & 1;
+        ld8<2>(w.ql0, blk + 64 * n + 16 * o + 8 * h);
+        ld8<2>(w.ql1, blk + 64 * n + 32 + 16 * o + 8 * h);
+        ld8<2>(w.qh, blk + 128 + 32 * n + 16 * o + 8 * h);
+        ld8<2>(w.sc, blk + 192 + 8 * n);
+        w.d = ld2(blk + 208);
+    }
+    static __device__ __forceinline__ u32 src_elem(int step, int c, int)
+    {
+        return 128u * (u32)(step >> 1) + 16u * (step & 1) + 32u * (c >> 2) + 4u * (c & 3);
+    }
+    static __device__ __forceinline__ int chunk(int g, int h, int i) { return 4 * g + 2 * h + i; }
+    static __device__ __forceinline__ bool live(int, int, int) { return true; }
+    struct Dec { float s[4]; };
+    static __device__ __forceinline__ void decode(Dec &d, const Raw &w, int step)
+    {
+        const float dd = h2f(w.d);
+        const int o = step & 1;
+        d.s[0] = dd * (float)sbyte(w.sc[0], o);
+        d.s[1] = dd * (float)sbyte(w.sc[0], o + 2);
+        d.s[2] = dd * (float)sbyte(w.sc[1], o);
+        d.s[3] = dd * (float)sbyte(w.sc[1], o + 2);
+    }
+    static __device__ __forceinline__ ckq_v4i operand(const Raw &w, int g, int)
+    {
+        u32 q[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const u32 l = (g & 1) ? w.ql1[j] : w.ql0[j];
+            const u32 nib = (g >> 1) ? (l >> 4) & 0x0f0f0f0fu : l & 0x0f0f0f0fu;
+            const u32 hb = g == 0 ? w.qh[j] << 4 : g == 1 ? w.qh[j] << 2 : g == 2 ? w.qh[j] : w.qh[j] >> 2;
+            const u32 v = nib | (hb & 0x30303030u);
+            q[j] = ((v | 0x80808080u) - 0x20202020u) ^ 0x80808080u;      /* no borrows between bytes */
+        }
+        return bytes_to_bf16(q[0], q[1]);
+    }
+};
+
+struct F32Q80 {
+    static constexpr int STEP = 64, NG = 2, NK = 2;       /* two 32-blocks; the second is missing in the last step of an odd count */
+    static constexpr bool MIN = false;
+    struct Raw { u32 q[2][4]; u32 d[2]; };
+    static __device__ __forceinline__ void load(Raw &w, const uint8_t *row, int step, int h, int K)
+    {
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            const uint8_t *blk = row + (u32)min(2 * step + g, K / 32 - 1) * 34u;
+            w.d[g] = ld2(blk);
+            ld16<2>(w.q[g], blk + 2 + 16 * h);
+        }
+    }
+    static __device__ __forceinline__ u32 src_elem(int step, int c, int K)
+    {
+        return 32u * (u32)min(2 * step + (c >> 3), K / 32 - 1) + 4u * (c & 7);
+    }
+    static __device__ __forceinline__ int chunk(int g, int h, int i) { return 8 * g + 4 * h + i; }
+    static __device__ __forceinline__ bool live(int step, int g, int K) { return 2 * step + g < K / 32; }
+    struct Dec { float s[2]; };
+    static __device__ __forceinline__ void decode(Dec &d, const Raw &w, int) { d.s[0] = h2f(w.d[0]); d.s[1] = h2f(w.d[1]); }
+    static __device__ __forceinline__ ckq_v4i operand(const Raw &w, int g, int i)
+    {
+        return bytes_to_bf16(w.q[g][2 * i], w.q[g][2 * i + 1]);
+    }
+};
+
+template <class F, int R>
+__global__ void __launch_bounds__(64 * F32_WAVES, 2)
+gemm_f32act_kernel(const float *__restrict__ A, const uint8_t *__restrict__ B, const float *__restrict__ bias, float *__restrict__ C,
+                   int M, int N, int K, long wrow, long ldc, int ntg)
+{
+    /* a wave's activations of one step, token t at 256 t, chunk c in slot c ^ (t & 15); at the end the partial tiles */
+    __shared__ __attribute__((aligned(16))) uint8_t xs_all[F32_WAVES][32 * 256];
+    const int lane = threadIdx.x & 63, wave = wave_in_block();
+    const int col = lane & 31, half = lane >> 5;
+    const int t0 = (int)(blockIdx.x % (u32)ntg) * 32, n0 = (int)(blockIdx.x / (u32)ntg) * 32 * R;
+    const int steps = (K + F::STEP - 1) / F::STEP, per = (steps + F32_WAVES - 1) / F32_WAVES;
+    const int s0 = wave * per, s1 = min(steps, s0 + per);
+
+    const float *xsrc[8];          /* row of the token this lane fetches in load instruction j */
+#pragma unroll
+    for (int j = 0; j < 8; ++j) xsrc[j] = A + (size_t)min(t0 + 4 * j + (lane >> 4), M - 1) * (size_t)K;
+    const uint8_t *wr[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) wr[r] = B + (size_t)min(n0 + 32 * r + col, N - 1) * (size_t)wrow;
+
+    ckq_v16f acc[R], zero;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) zero[i] = 0.0f;
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = zero;
+
+    uint8_t *const xs = xs_all[wave];
+    typename F::Raw w[R], wn[R];
+    ckq_v4i xn[8];
+    auto fetch = [&](int s) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) xn[j] = *reinterpret_cast<const ckq_v4i *>(xsrc[j] + F::src_elem(s, lane & 15, K));
+#pragma unroll
+        for (int r = 0; r < R; ++r) F::load(wn[r], wr[r], s, half, K);
+    };
+    auto take = [&]() {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int t = 4 * j + (lane >> 4);
+            *reinterpret_cast<ckq_v4i *>(xs + 256 * t + 16 * ((lane & 15) ^ (t & 15))) = xn[j];
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) w[r] = wn[r];
+    };
+    auto compute = [&](int s) {
+        typename F::Dec dec[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) F::decode(dec[r], w[r], s);
+        float p[F::NG];
+#pragma unroll
+        for (int g = 0; g < F::NG; ++g) {
+            if (!F::live(s, g, K)) break;                        /* uniform */
+            Cut c[F::NK];
+            float x[F::NK * 8];
+#pragma unroll
+            for (int i = 0; i < 2 * F::NK; ++i) {
+                const ckq_v4i v = *reinterpret_cast<const ckq_v4i *>(xs + 256 * col + 16 * (F::chunk(g, half, i) ^ (col & 15)));
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int e = v[j];
+                    x[4 * i + j] = __builtin_bit_cast(float, e);
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < F::NK; ++k) cut8(x + 8 * k, c[k]);
+            if constexpr (F::MIN)
+                p[g] = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7])) +
+                       (((x[8] + x[9]) + (x[10] + x[11])) + ((x[12] + x[13]) + (x[14] + x[15])));
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                ckq_v16f sum = zero;
+#pragma unroll
+                for (int k = 0; k < F::NK; ++k) {
+                    const ckq_v4i b = F::operand(w[r], g, k);
+                    sum = mfma_bf16(c[k].lo, b, sum);
+                    sum = mfma_bf16(c[k].mid, b, sum);
+                    sum = mfma_bf16(c[k].hi, b, sum);
+                }
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[r][i] = fmaf(dec[r].s[g], sum[i], acc[r][i]);
+            }
+        }
+        if constexpr (F::MIN) {
+            /* this half's share of the two sub-block sums, cut in three; the MFMA adds the halves */
+            const float p0 = finite(p[0]), p1 = finite(p[1]);
+            const float m0 = p0 - top16(p0), m1 = p1 - top16(p1);
+            const ckq_v4i pa = {(int)pack_bf16(m0 - top16(m0), m0), (int)pack_bf16(p[0], m1 - top16(m1)), (int)pack_bf16(m1, p[1]), 0};
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const ckq_v16f i2 = mfma_bf16(pa, dec[r].mins, zero);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[r][i] = fmaf(-dec[r].dmin, i2[i], acc[r][i]);
+            }
+        }
+    };
+    if (s0 < s1) fetch(s0);
+    for (int s = s0; s < s1; ++s) {
+        take();
+        if (s + 1 < s1) fetch(s + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(s);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+
+    constexpr int RP = R < 2 ? 1 : 2;
+    float *const red = reinterpret_cast<float *>(&xs_all[0][0]);     /* [wave][RP * 16][64] */
+    static_assert(F32_WAVES * RP * 16 * 64 * sizeof(float) <= sizeof(xs_all), "the partial tiles fit the activations' place");
+    __syncthreads();                         /* every wave is done with its activations */
+    /* the eight partial tiles through LDS, two row tiles at a time; wave w finishes sixteenths 2 w .. of every lane */
+#pragma unroll
+    for (int q = 0; q < R; q += RP) {
+        __syncthreads();                     /* every wave is done with the buffer (and its loads have landed) */
+#pragma unroll
+        for (int r = 0; r < RP; ++r)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) red[(wave * RP * 16 + 16 * r + i) * 64 + lane] = acc[q + r][i];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 2 * RP; ++j) {
+            const int o = 2 * RP * wave + j, i = o & 15;
+            float v = red[o * 64 + lane];
+#pragma unroll
+            for (int k = 1; k < F32_WAVES; ++k) v += red[(k * RP * 16 + o) * 64 + lane];
+            const int n = n0 + 32 * (q + (o >> 4)) + col, t = t0 + 8 * (i >> 2) + 4 * half + (i & 3);
+            if (n < N && t < M) C[(size_t)t * ldc + n] = bias ? v + bias[n] : v;
+        }
+    }
+}
+
+template <class F>
+int launch_f32act(const float *A, const uint8_t *B, const float *bias, float *C, int M, int N, int K, long wrow, long ldc, hipStream_t s)
+{
+    const long long ntg = (M + 31) / 32;
+    /* two row tiles per wave share the cut of x; one where that would leave CUs without a block */
+    const int R = ntg * ((N + 63) / 64) >= 192 ? 2 : 1;
+    const long long grid = ntg * ((N + 32 * R - 1) / (32 * R));
+    if (grid > 0x7fffffffll) return CKQ_ESHAPE;
+    if (R == 2) hipLaunchKernelGGL((gemm_f32act_kernel<F, 2>), dim3((unsigned)grid), dim3(64 * F32_WAVES), 0, s, A, B, bias, C, M, N, K, wrow, ldc, (int)ntg);
+    else hipLaunchKernelGGL((gemm_f32act_kernel<F, 1>), dim3((unsigned)grid), dim3(64 * F32_WAVES), 0, s, A, B, bias, C, M, N, K, wrow, ldc, (int)ntg);
+    return (int)hipGetLastError();
+}
+
+} // namespace
+
+int launch_gemm_f32act(int fmt, const float *A, const void *B, const float *bias, float *C, int M, int N, int K, long ldc, hipStream_t s)
+{
+    const uint8_t *W = (const uint8_t *)B;
+    switch (fmt) {
+    case CKQ_KERNEL_Q4K_F32: return launch_f32act<F32Q4K>(A, W, bias, C, M, N, K, (long)(K / 256) * 144, ldc, s);
+    case CKQ_KERNEL_Q6K_F32: return launch_f32act<F32Q6K>(A, W, bias, C, M, N, K, (long)(K / 256) * 210, ldc, s);
+    case CKQ_KERNEL_Q80_F32: return launch_f32act<F32Q80>(A, W, bias, C, M, N, K, (long)(K / 32) * 34, ldc, s);
+    default: return CKQ_EFORMAT;
+    }
+}

@@ -74,8 +74,28 @@ static bool gemm_on_matrix_cores(int ntok, size_t weight_bytes, size_t budget_mb
     return passes * per > (budget_mb << 20);
 }
 
+/* fp32 activations.  The streaming kernel decodes the weights again for every token; the matrix-core kernel
+ * (ckq_gemm_f32act.hip) decodes them once per 32 tokens.  Fitted to launches of both over 141..11008 rows, widths
+ * of 512..8192 and 1..200 tokens (us): streaming 4 + 0.125 / 0.18 / 0.16 (Q4_K / Q6_K / Q8_0) per million products; matrix cores
+ * 6 + 0.017 / 0.024 / 0.024 per million products of the tokens rounded up to 32, but never less than 5 + 1.35 for every
+ * 64 elements a wave walks through (an eighth of K).  4096 x 4096 Q6_K: 4 tokens 14.5 against 19 (streams), 8 tokens 26 against
+ * 19, 96 tokens 270 against 36; 141 x 8192 streams up to 96 tokens. */
+static bool f32act_on_matrix_cores(int fmt, int ntok, int nrows, int K)
+{
+    const int policy = g_gemm_policy.load(std::memory_order_relaxed);
+    if (ntok < 2 || policy == 2) return false;
+    if (policy == 1) return true;
+    const float per = fmt == CKQ_KERNEL_Q4K_F32 ? 0.125f : fmt == CKQ_KERNEL_Q6K_F32 ? 0.18f : 0.16f;
+    const float per_matrix = fmt == CKQ_KERNEL_Q4K_F32 ? 0.017f : 0.024f;
+    const float mw = (float)nrows * (float)K * 1e-6f;
+    const float t_stream = 4.0f + per * mw * (float)ntok;
+    const float t_matrix = fmaxf(5.0f + 1.35f * (float)((K + 511) / 512), 6.0f + per_matrix * mw * (float)((ntok + 31) / 32 * 32));
+    return t_stream > t_matrix;
+}
+
 #include "ckq_gemv.hpp"
 #include "ckq_gemm_common.hpp"
+#include "ckq_gemm_f32act.hpp"
 
 /* C = bias + partial 0 + partial 1 + ... in that order: the result does not
  * depend on which block finished first.  One thread per output. */
@@ -382,16 +402,19 @@ static int launch_gemv_args(int fmt_flags, GemvArgs &a, const GemvGroup &grp, in
     case CKQ_KERNEL_Q80_F32:
         if (K % 32) return CKQ_ESHAPE;
         if (dump || grp.n > 1) return CKQ_EINVAL;
+        if (whole && f32act_on_matrix_cores(fmt, ntok, nrows, K)) return launch_gemm_f32act(fmt, (const float *)X, W, bias, y, ntok, nrows, K, ldy, s);
         a.npos = K / 32; a.wrow = (long)(K / 32) * 34; a.xrow = (long)K * 4; a.nsub_row = K / 32;
         return ckq_gemv_launch_q80_f32(a, grp, s);
     case CKQ_KERNEL_Q4K_F32:
         if (K % 256) return CKQ_ESHAPE;
         if (dump || grp.n > 1) return CKQ_EINVAL;
+        if (whole && f32act_on_matrix_cores(fmt, ntok, nrows, K)) return launch_gemm_f32act(fmt, (const float *)X, W, bias, y, ntok, nrows, K, ldy, s);
         a.npos = K / 64; a.wrow = (long)(K / 256) * 144; a.xrow = (long)K * 4; a.nsub_row = K / 64;
         return ckq_gemv_launch_q4k_f32(a, grp, s);
     case CKQ_KERNEL_Q6K_F32:
         if (K % 256) return CKQ_ESHAPE;
         if (dump || grp.n > 1) return CKQ_EINVAL;
+        if (whole && f32act_on_matrix_cores(fmt, ntok, nrows, K)) return launch_gemm_f32act(fmt, (const float *)X, W, bias, y, ntok, nrows, K, ldy, s);
         a.npos = K / 64; a.wrow = (long)(K / 256) * 210; a.xrow = (long)K * 4; a.nsub_row = K / 64;
         return ckq_gemv_launch_q6k_f32(a, grp, s);
     default:

@@ -1189,3 +1189,43 @@ def test_host_inputs_stored_straight_into_device_memory_are_never_stale():
         got = P.gemm_nt("q4_k", xq, Wh[K], None if bi < 0 else biases[bi], 1, N, K).reshape(-1)
         bad += int(not np.array_equal(got, want[(K, i, bi)]))
     assert bad == 0, "%d of 3000 calls read stale inputs" % bad
+
+
+# ---- fp32 activations on the matrix cores -------------------------------------------------------
+
+@pytest.mark.parametrize("fmt", F32_FMTS)
+def test_f32act_matrix_cores_vs_fp64(fmt):
+    """The matrix-core kernel (forced; up to 32 tokens per tile) at the edges of its tiles: one token and
+    one more than a tile, row counts around 32 and 64, fewer steps of K than the eight waves of a block and
+    one more, an odd number of 32-blocks (Q8_0); against dequantize-then-matmul in fp64, with a bias and a
+    padded C, and with infinite activations where the exact result is infinite."""
+    import torch
+    L = ckq.lib()
+    blk = 32 if fmt == "q8_0" else 256
+    shapes = [(2, 1, blk), (31, 33, 2 * blk), (32, 64, 512), (33, 65, 2304), (70, 31, 17 * blk), (97, 200, 1024), (200, 2085, 768)]
+    L.ckq_set_gemm_policy(1)
+    try:
+        for M, N, K in shapes:
+            W, xf, _ = make_case(fmt, N, K, "enc", 9000 + M + K, tokens=M)
+            bias = T.normal(N, 0.0, 0.5, seed=N)
+            say("f32act matrix cores", fmt, M, N, K)
+            ldc = N + 3
+            c = torch.full((M, ldc), 7.0, dtype=torch.float32, device="cuda")
+            x_d, W_d, b_d = P.to_device(xf), P.to_device(W), P.to_device(bias)
+            P.check(L.ckq_gemm_nt_f32act_dev(P.FMT[fmt], P._dp(x_d), P._dp(W_d), P._dp(b_d), P._dp(c), M, N, K, ldc, P._stream()), "f32act")
+            got = c.cpu().numpy()
+            want = xf.reshape(M, K).astype(np.float64) @ T.np_dequant(fmt, W).reshape(N, K).T + bias
+            assert T.norm_err(got[:, :N], want) <= 2e-6, (M, N, K)
+            assert np.all(got[:, N:] == 7.0), (M, N, K)
+        M, N, K = 40, 64, 512
+        W = np.tile(T.synth_weights(fmt, 1, K, seed=5), N)
+        w0 = T.np_dequant(fmt, W[:T.row_bytes(fmt, K)])
+        x = T.normal(M * K, 0.0, 1.0, seed=6).reshape(M, K)
+        k = int(np.argmax(np.abs(w0)))
+        x[3, k] = np.inf
+        got = P.dev_gemm_nt_f32act(fmt, P.to_device(x.reshape(-1)), P.to_device(W), None, M, N, K).cpu().numpy().reshape(M, N)
+        assert np.all(np.isfinite(np.delete(got, 3, axis=0)))
+        if fmt != "q4_k":            # in Q4_K the min term subtracts the same infinity
+            assert np.all(got[3] == np.copysign(np.inf, w0[k]))
+    finally:
+        L.ckq_set_gemm_policy(0)
