@@ -38,6 +38,7 @@
  * each see a weight tile once.
  */
 #include "ckq_gemm_q4k.hpp"
+#include "ckq_gemm_rows16.hpp"
 #include <atomic>
 #include <type_traits>
 
@@ -371,6 +372,15 @@ static bool q4k_take_t96(int M, int tiles64, int blocks96)
     return 2 * blocks96 >= 3 * SLOTS;
 }
 
+GemmChains gemm_q4k_chains(int M, int N, int K)
+{
+    const int nb = K / 256, tiles = ((M + GEMM_BM - 1) / GEMM_BM) * ((N + GEMM_BN - 1) / GEMM_BN);
+    GemmChains c = gemm_chains_split(tiles, nb);
+    const int sp = gemm_choose_splits(tiles, nb);
+    if (tiles * sp <= 256 && (nb + sp - 1) / sp >= 8) c.kg = 2;
+    return c;
+}
+
 int launch_gemm_q4k_mfma(const void *A, const void *B, const float *bias, float *C,
                          int M, int N, int K, long ldc, const GemmOpts &opts, hipStream_t s)
 {
@@ -404,6 +414,13 @@ int launch_gemm_q4k_mfma(const void *A, const void *B, const float *bias, float 
     }
     if (two_groups) return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 2>, g, (unsigned)(g.ntt * nnt8), g.nb, s, 512);
     return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 1>, g, (unsigned)(g.ntt * nnt8), g.nb, s, 256);
+}
+
+bool gemm_q4k_group_chains(const GemmGroupIn &in, int M, int K, GemmChains *ch)
+{
+    const int tiles = gemm_group_tiles(in, M, GEMM_BM);
+    *ch = {1, K / 256, tiles <= 256 && K / 256 >= 8 ? 2 : 1};
+    return tiles >= GEMM_GROUP_MIN_TILES;
 }
 
 int launch_gemm_q4k_mfma_group(const void *A, const GemmGroupIn &in, int M, int K, hipStream_t s)

@@ -29,7 +29,7 @@
  *
  * Block = 4 waves = 64 tokens x 128 weight rows; wave w owns rows 32w..32w+31.
  */
-#include "ckq_gemm_common.hpp"
+#include "ckq_gemm_rows16.hpp"
 #include <atomic>
 #include <type_traits>
 
@@ -452,6 +452,11 @@ static bool q5k_take_pair(int tiles)
     return forced ? forced == 2 : tiles > 256;
 }
 
+GemmChains gemm_q5k_chains(int M, int N, int K)
+{
+    return gemm_chains_split(((M + GEMM5_BM - 1) / GEMM5_BM) * ((N + GEMM5_BN - 1) / GEMM5_BN), K / 256);
+}
+
 int launch_gemm_q5k_mfma(const void *A, const void *B, const float *bias, float *C,
                          int M, int N, int K, long ldc, const GemmOpts &opts, hipStream_t s)
 {
@@ -481,6 +486,12 @@ int launch_gemm_q5k_mfma(const void *A, const void *B, const float *bias, float 
     if (sums) return CKQ_ENODUMP;
 #endif
     return gemm_launch_split(gemm_q5k_mfma_kernel<false>, g, (unsigned)(g.ntt * nnt8), g.nb, s);
+}
+
+bool gemm_q5k_group_chains(const GemmGroupIn &in, int M, int K, GemmChains *ch)
+{
+    *ch = {1, K / 256, 1};
+    return gemm_group_tiles(in, M, GEMM5_BM) >= GEMM_GROUP_MIN_TILES;
 }
 
 int launch_gemm_q5k_mfma_group(const void *A, const GemmGroupIn &in, int M, int K, hipStream_t s)

@@ -30,7 +30,7 @@
  *   slab s and larger token tiles (TH = 4) amortise it where the grid is big
  *   enough to fill the chip with them.
  */
-#include "ckq_gemm_common.hpp"
+#include "ckq_gemm_rows16.hpp"
 #include <atomic>
 #include <type_traits>
 
@@ -469,6 +469,12 @@ static bool q6k_take_pair(int tiles128, int tiles64)
     return 4 * rounds * 256 >= 5 * tiles128;        /* ceil(r) / r >= 1.25 */
 }
 
+GemmChains gemm_q6k_chains(int M, int N, int K)
+{
+    const int nnt = (N + GEMM6_BN - 1) / GEMM6_BN, t4 = (M + 127) / 128 * nnt, t2 = (M + 63) / 64 * nnt;
+    return gemm_chains_split(q6k_take_pair(t4, t2) || t4 <= 128 ? t2 : t4, K / 256);
+}
+
 int launch_gemm_q6k_mfma(const void *A, const void *B, const float *bias, float *C,
                          int M, int N, int K, long ldc, const GemmOpts &opts, hipStream_t s)
 {
@@ -510,6 +516,12 @@ int launch_gemm_q6k_mfma(const void *A, const void *B, const float *bias, float 
     if (sums) return CKQ_ENODUMP;
 #endif
     return gemm_launch_split(gemm_q6k_mfma_kernel<2>, g, (unsigned)(g.ntt * nnt8), g.nb, s);
+}
+
+bool gemm_q6k_group_chains(const GemmGroupIn &in, int M, int K, GemmChains *ch)
+{
+    *ch = {1, K / 256, 1};
+    return gemm_group_tiles(in, M, 64) >= GEMM_GROUP_MIN_TILES;
 }
 
 int launch_gemm_q6k_mfma_group(const void *A, const GemmGroupIn &in, int M, int K, hipStream_t s)

@@ -1,0 +1,466 @@
+/*
+ * ckq_gemm_rows16.hip - K-quant weights x Q8_K activations for a few to a few dozen tokens, on the gfx950 int8 matrix
+ * cores, with the weights streamed from memory through LDS private to a wave.
+ *
+ * Where the tile kernels (ckq_gemm_q4k.hip and its siblings) move 128-row tiles through LDS and need hundreds of tokens
+ * to pay for it, and the streaming kernel (ckq_gemv.hpp) spends one v_dot4 per four products and token, this kernel has
+ * one WAVE multiply 16 weight rows with 16 tokens: the matrix instruction takes 16 tokens for the price of one, the
+ * planes of a weight are formed once, and as in the streaming kernel the waves run on their own and nothing waits at
+ * a barrier before the end.
+ *
+ * v_mfma_i32_16x16x64_i8: A = 16 tokens x 64 k, B = 64 k x 16 weight rows, D = 16 x 16 int32.  Lane l = 16 q + i holds
+ * token / row i and the 16 k of quarter q; of D it holds row i and tokens 4 q .. 4 q + 3.  The 64 k of an instruction are
+ * those a lane of the streaming kernel takes, ordered so that a lane's sixteen are one 16-byte run of the raw block's
+ * quants (low or high nibbles) inside one scale; the activations are read in the same order.  The planes are those of the tile kernels: Q4_K (sc >> 3) q and
+ * (sc & 7) q, Q5_K / Q6_K the two bytes of the 16-bit product, each summed over the 256-block; the min term of Q4_K / Q5_K is
+ * a bf16 MFMA of the mins and the bsum pairs split in two (ckq_gemm_q4k.hip).  All integers are exact.
+ *
+ * The integers being exact, only the order of the fp32 additions is left to choose, and it is that of the kernel the shape
+ * would otherwise run on: the streaming kernel's term per 64 elements and tree (TREE), or the tile kernels' term per
+ * 256-block and chains (GemmChains).  The terms meet in LDS; one thread per output adds them.
+ *
+ * Bound: VALU issue (150-300 operations per 256-block of 16 rows) next to HBM and, for small matrices, one latency after
+ * another.  Measured, weights from HBM, against the kernel that served the shape before (us): Q4_K 4096 x 4096 at 8 / 13 / 32
+ * tokens 7.5 -> 6.1, 10.0 -> 6.5, 13.1 -> 8.1; 11008 x 4096 at 8 / 13: 14.7 -> 10.3, 15.6 -> 9.7; Q6_K 32000 x 4096 at
+ * 8 / 13: 40.6 -> 27.1, 46.2 -> 28.3; 4096 x 11008 at 13: 20.7 -> 15.8; Q5_K 1024 x 4864 at 64: 16.8 -> 8.0.
+ */
+#include "ckq_formats.hpp"
+#include "ckq_blocks.h"
+#include "ckq_gemm_rows16.hpp"
+#include "ckq_gemm_q4k.hpp"
+#include <atomic>
+
+namespace {
+
+typedef float ckq_v4f __attribute__((ext_vector_type(4)));
+
+/* What a lane keeps of its row's block header. */
+struct Head {
+    u32     sc[2];           /* Q4_K, Q5_K: scale of sub-block 2 g + q / 2 in byte 2 (g & 1) of [g / 2]; Q6_K: that of 16-run (n, q, odd) in byte odd of [n] */
+    ckq_v4i mins;            /* bf16 m_2q, m_2q+1, m_2q, m_2q+1, 0... (Q4_K, Q5_K) */
+    float   dw, dmin;
+};
+
+/* Header of a Q4_K / Q5_K block: the packed 6-bit scales and mins (layout: ckq_formats.hpp). */
+__device__ __forceinline__ void head_k45(Head &p, const uint8_t *r, int q)
+{
+    const ckq_v4i hv = *reinterpret_cast<const ckq_v4i *>(r);
+    const u32 h0 = (u32)hv[0], h1 = (u32)hv[1], h2 = (u32)hv[2], h3 = (u32)hv[3];
+    const int s8 = 8 * (q >> 1), s16 = 16 * (q & 1);
+    p.sc[0] = (h1 & 0x3f3f3f3fu) >> s8;
+    p.sc[1] = ((h3 & 0x0f0f0f0fu) | ((h1 >> 2) & 0x30303030u)) >> s8;
+    const u32 lo = (h2 >> s16) & 0x3f3fu, hi = ((h3 >> (s16 + 4)) & 0x0f0fu) | (((h2 >> s16) >> 2) & 0x3030u);
+    const u32 mn = q < 2 ? lo : hi;
+    const u32 pair = bf16_pair((float)(mn & 0xff), (float)((mn >> 8) & 0xff));
+    p.mins = ckq_v4i{(int)pair, (int)pair, 0, 0};
+    p.dw = h2f(h0 & 0xffff);
+    p.dmin = h2f(h0 >> 16);
+}
+
+/* Four bytes times a 16-bit factor (+ add), split into the signed low and the high bytes of the products. */
+__device__ __forceinline__ void byte_planes(u32 v, u32 sc2, u32 add2, int &lo, int &hi)
+{
+    const u32 e = __builtin_amdgcn_perm(0u, v, 0x0c020c00u), o = __builtin_amdgcn_perm(0u, v, 0x0c030c01u);
+    const u32 te = pk_mad_u16(e, sc2, add2), to = pk_mad_u16(o, sc2, add2);      /* product + 128 */
+    lo = (int)(__builtin_amdgcn_perm(to, te, 0x06020400u) ^ 0x80808080u);
+    hi = (int)__builtin_amdgcn_perm(to, te, 0x07030501u);
+}
+
+__device__ __forceinline__ ckq_v4i lds16(const uint8_t *p) { return *reinterpret_cast<const ckq_v4i *>(p); }
+
+/* Formats.  Position g of a 256-block: the 64 elements of one instruction, of which lane quarter q supplies the sixteen
+ * from a_elem(g, q).  planes() forms them from the raw block of the lane's row at r (in LDS). */
+struct R16Q4K {
+    static constexpr int WBLOCK = 144, SHIFT = 3, CHUNKS = 9, PITCH = 144;
+    static constexpr bool MIN = true;
+    static __device__ __forceinline__ u32 chunk_ofs(int c) { return 16u * (u32)c; }
+    static __device__ __forceinline__ u32 a_elem(int g, int q) { return 64u * g + 16u * q; }
+    static __device__ __forceinline__ void head(Head &p, const uint8_t *r, int q) { head_k45(p, r, q); }
+    static __device__ __forceinline__ void planes(ckq_v4i &h, ckq_v4i &l, const Head &p, const uint8_t *r, int g, int q)
+    {
+        const ckq_v4i qs = lds16(r + 16 + 32 * g + 16 * (q & 1));
+        auto pair_of_byte = [](u32 v, int k) { return __builtin_amdgcn_perm(0u, v, 0x0c000c00u | (u32)k | ((u32)k << 16)); };
+        const u32 mh = pair_of_byte((p.sc[g >> 1] >> 3) & 0x07070707u, 2 * (g & 1)), ml = pair_of_byte(p.sc[g >> 1] & 0x07070707u, 2 * (g & 1));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const u32 n = ((u32)qs[i] >> (4 * (q >> 1))) & 0x0f0f0f0fu;
+            h[i] = mul_bytes(n, mh);
+            l[i] = mul_bytes(n, ml);
+        }
+    }
+};
+
+struct R16Q5K {
+    static constexpr int WBLOCK = 176, SHIFT = 8, CHUNKS = 11, PITCH = 176;
+    static constexpr bool MIN = true;
+    static __device__ __forceinline__ u32 chunk_ofs(int c) { return 16u * (u32)c; }
+    static __device__ __forceinline__ u32 a_elem(int g, int q) { return 64u * g + 16u * q; }
+    static __device__ __forceinline__ void head(Head &p, const uint8_t *r, int q) { head_k45(p, r, q); }
+    static __device__ __forceinline__ void planes(ckq_v4i &h, ckq_v4i &l, const Head &p, const uint8_t *r, int g, int q)
+    {
+        const ckq_v4i qs = lds16(r + 48 + 32 * g + 16 * (q & 1)), qh = lds16(r + 16 + 16 * (q & 1));
+        const u32 sc2 = __builtin_amdgcn_perm(0u, p.sc[g >> 1], (g & 1) ? 0x0c020c02u : 0x0c000c00u);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const u32 n = ((u32)qs[i] >> (4 * (q >> 1))) & 0x0f0f0f0fu;
+            const u32 hb = ((u32)qh[i] >> (2 * g + (q >> 1))) & 0x01010101u;              /* fifth bits of sub-block 2 g + q / 2 */
+            int lo, hi;
+            byte_planes(n | (hb << 4), sc2, 0x00800080u, lo, hi);
+            h[i] = hi;
+            l[i] = lo;
+        }
+    }
+};
+
+struct R16Q6K {
+    /* a 210-byte block as fourteen chunks, the last from byte 194 so that no load passes the block's end */
+    static constexpr int WBLOCK = 210, SHIFT = 8, CHUNKS = 14, PITCH = 240;
+    static constexpr bool MIN = false;
+    static __device__ __forceinline__ u32 chunk_ofs(int c) { return c < 13 ? 16u * (u32)c : 194u; }
+    /* position g = 2 n + odd: the halves `odd` of the four 32-runs of 128-half n */
+    static __device__ __forceinline__ u32 a_elem(int g, int q) { return 128u * (g >> 1) + 32u * q + 16u * (g & 1); }
+    static __device__ __forceinline__ void head(Head &p, const uint8_t *r, int q)
+    {
+        const ckq_v4i sc = lds16(r + 192);
+#pragma unroll
+        for (int n = 0; n < 2; ++n) p.sc[n] = (u32)(q < 2 ? sc[2 * n] : sc[2 * n + 1]) >> (16 * (q & 1));
+        p.dw = h2f(*reinterpret_cast<const uint16_t *>(r + 222));
+        p.dmin = 0.0f;
+    }
+    static __device__ __forceinline__ void planes(ckq_v4i &h, ckq_v4i &l, const Head &p, const uint8_t *r, int g, int q)
+    {
+        const int n = g >> 1, odd = g & 1;
+        const ckq_v4i ql = lds16(r + 64 * n + 32 * (q & 1) + 16 * odd), qh = lds16(r + 128 + 32 * n + 16 * odd);
+        const int sc = __builtin_amdgcn_sbfe((int)p.sc[n], 8 * odd, 8);
+        const u32 sc2 = __builtin_amdgcn_perm((u32)sc, (u32)sc, 0x05040504u);
+        const u32 add = pk_mad_u16(sc2, 0xFFE0FFE0u, 0x00800080u);                   /* 128 - 32 sc */
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const u32 n4 = ((u32)ql[i] >> (4 * (q >> 1))) & 0x0f0f0f0fu, hb = (((u32)qh[i] >> (2 * q)) & 0x03030303u) << 4;
+            int lo, hi;
+            byte_planes(n4 | hb, sc2, add, lo, hi);
+            h[i] = hi;
+            l[i] = lo;
+        }
+    }
+};
+
+/* Shape of a launch: what a block needs besides its problem. */
+struct Rows16Shape { int M, nb; };
+
+/* LDS of one wave: the 16 weight blocks of an item, the quants of NT tokens (256 bytes each, 16-byte chunk c in slot
+ * c ^ token) and their bsums (32 bytes each). */
+template <class F, int NT> constexpr int rows16_wave_lds() { return 16 * F::PITCH + NT * 288; }
+
+/* One block computes a tile of 16 rows for NT (8 or 16) tokens.  Wave w takes the 256-blocks w, w + waves, ... of the
+ * rows.  A block's bytes are loaded in memory order - 16 adjacent lanes read a token's 256 quants, 9 to 14 lanes a weight
+ * block: a lane loading its own operand would touch a cache line of its own with every 16 bytes, and the address unit
+ * would bound the launch (10.6 us instead of 9.4 at 11008 x 4096, 13 tokens, Q4_K; 44 instead of 27 at 32000 x 4096,
+ * Q6_K) - and turned through LDS of the wave's own, the next block's loads in flight meanwhile.  A 256-block leaves
+ * u = dw I1 - dmin I2 of its NT x 16 outputs in LDS; when all are done, one thread per output runs the chains of
+ * multiply-adds over them in order, so that any wave may take any block whatever the chains.
+ * More rows or more tokens (32, planes shared) per block were slower: fewer waves per CU fit the LDS. */
+template <class F, int NT, bool TREE, bool GRP>
+__global__ void __launch_bounds__(1024)
+gemm_rows16_kernel(const uint8_t *W, const uint8_t *X, int N, Rows16Shape S, float *y, const float *bias, long ldy, GemmChains ch, Rows16Args grp)
+{
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const int tid = threadIdx.x, nthr = blockDim.x, nwave = nthr >> 6;
+    const int lane = tid & 63, wave = wave_in_block();
+    const int i16 = lane & 15, q = lane >> 4;
+    const int M = S.M, nb = S.nb;
+    int bid = (int)blockIdx.x;
+    if constexpr (GRP) {
+        if (bid >= grp.p[1].id0) {
+            Rows16Problem p = grp.p[1];
+            if (grp.n > 2 && bid >= grp.p[2].id0) p = grp.p[2];
+            if (grp.n > 3 && bid >= grp.p[3].id0) p = grp.p[3];
+            W = p.W; X = p.X; N = p.N; y = p.y; bias = p.bias; ldy = p.ldy; ch = p.ch;
+            bid -= p.id0;
+        }
+    }
+    const int n0 = bid * 16, t0 = (int)blockIdx.y * NT;
+    const u32 xrow = (u32)nb * 292u, wpitch = (u32)nb * (u32)F::WBLOCK;
+    uint8_t *const wl = smem + wave * rows16_wave_lds<F, NT>();           /* this wave's weights, quants, bsums */
+    uint8_t *const al = wl + 16 * F::PITCH, *const bl = al + NT * 256;
+    float *const us = reinterpret_cast<float *>(smem + nwave * rows16_wave_lds<F, NT>()), *const dxs = us + (TREE ? min(nb, 16) : nb) * (NT * 16);
+    /* uniform bases, 32-bit lane offsets */
+    const uint8_t *const wbase = W + (size_t)n0 * wpitch;
+    const uint8_t *const xbase = X + (size_t)t0 * xrow;
+
+    /* copy roles: weight chunk 64 j + lane -> (row, chunk), token chunk 64 j + lane -> (token, one of 16 of quants or 2 of bsums) */
+    constexpr int NWL = (16 * F::CHUNKS + 63) / 64, NAL = (NT * 18 + 63) / 64;
+    u32 wsrc[NWL], wdst[NWL], asrc[NAL], adst[NAL];
+#pragma unroll
+    for (int j = 0; j < NWL; ++j) {
+        const int e = min(64 * j + lane, 16 * F::CHUNKS - 1), r = e / F::CHUNKS, c = e % F::CHUNKS;
+        wsrc[j] = (u32)min(r, N - 1 - n0) * wpitch + F::chunk_ofs(c);
+        wdst[j] = (u32)(r * F::PITCH + 16 * c);
+    }
+#pragma unroll
+    for (int j = 0; j < NAL; ++j) {
+        const int e = min(64 * j + lane, NT * 18 - 1), t = e / 18, c = e % 18;
+        asrc[j] = (u32)min(t, M - 1 - t0) * xrow + 4u + 16u * (u32)c;
+        adst[j] = (u32)(c < 16 ? 256 * t + 16 * (c ^ (t & 15)) : NT * 256 + 32 * t + 16 * (c - 16));
+    }
+    u32 aofs[4];
+    constexpr int QL = NT / 4;                       /* quarters of the result that hold tokens */
+    const int ta = i16 & (NT - 1);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) aofs[m] = (u32)(256 * ta + 16 * ((int)(F::a_elem(m, q) >> 4) ^ ta));
+
+    ckq_v4i wr[NWL], ar[NAL];
+    auto fetch = [&](int b) {
+        const uint8_t *wb = wbase + (size_t)((u32)b * (u32)F::WBLOCK), *xb = xbase + (size_t)((u32)b * 292u);
+#pragma unroll
+        for (int j = 0; j < NWL; ++j) {
+            u32 t[4];
+            ld16<F::WBLOCK % 4 == 0 ? 4 : 2>(t, wb + wsrc[j]);
+            wr[j] = ckq_v4i{(int)t[0], (int)t[1], (int)t[2], (int)t[3]};
+        }
+#pragma unroll
+        for (int j = 0; j < NAL; ++j) {
+            u32 t[4];
+            ld16<4>(t, xb + asrc[j]);
+            ar[j] = ckq_v4i{(int)t[0], (int)t[1], (int)t[2], (int)t[3]};
+        }
+    };
+    auto take = [&]() {
+#pragma unroll
+        for (int j = 0; j < NWL; ++j) *reinterpret_cast<ckq_v4i *>(wl + wdst[j]) = wr[j];
+#pragma unroll
+        for (int j = 0; j < NAL; ++j) *reinterpret_cast<ckq_v4i *>(al + adst[j]) = ar[j];
+    };
+    /* the two bsum pairs of position q as lo + 64 hi, exact in bf16 (ckq_gemm_q4k.hip) */
+    auto bsum_operand = [&]() {
+        const int2 bs = *reinterpret_cast<const int2 *>(bl + 32 * ta + 8 * q);
+        const int p0 = (int)(int16_t)(bs.x & 0xffff) + (bs.x >> 16), p1 = (int)(int16_t)(bs.y & 0xffff) + (bs.y >> 16);
+        return ckq_v4i{(int)bf16_pair((float)(p0 & 63), (float)(p1 & 63)), (int)bf16_pair((float)(64 * (p0 >> 6)), (float)(64 * (p1 >> 6))), 0, 0};
+    };
+    auto min_mfma = [&](const ckq_v4i &am, const ckq_v4i &mins) {
+        const ckq_v4f z = {0.0f, 0.0f, 0.0f, 0.0f};
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(ckq_v8bf, am), __builtin_bit_cast(ckq_v8bf, mins), z, 0, 0, 0);
+    };
+    /* lane 16 q + i holds tokens 4 q .. 4 q + 3; of eight tokens the upper two quarters are copies */
+    auto put = [&](int b, const float (&v)[4]) {
+        float *u = us + b * (NT * 16) + lane;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (NT > 8 || q < 2) u[r * (16 * QL)] = v[r];
+    };
+    const ckq_v4i zero = {0, 0, 0, 0};
+    const uint8_t *const wrow = wl + i16 * F::PITCH;
+
+    /* CHAIN: the integers of the whole 256-block, u = dw I1 - dmin I2 */
+    auto block_term = [&](int b) {
+        Head hd;
+        F::head(hd, wrow, q);
+        ckq_v4i sh, sl;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            ckq_v4i ph, pl;
+            F::planes(ph, pl, hd, wrow, g, q);
+            const ckq_v4i a = lds16(al + aofs[g]);
+            sh = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, ph, g ? sh : zero, 0, 0, 0);
+            sl = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, pl, g ? sl : zero, 0, 0, 0);
+        }
+        float out[4];
+        if constexpr (F::MIN) {
+            const ckq_v4f i2 = min_mfma(bsum_operand(), hd.mins);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float f = (float)((sh[r] << F::SHIFT) + sl[r]);
+                out[r] = hd.dw * f - hd.dmin * i2[r];
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) out[r] = hd.dw * (float)((sh[r] << F::SHIFT) + sl[r]);
+        }
+        put(b, out);
+    };
+
+    /* TREE: the fp32 terms of the four positions, added to the sums their lanes of the streaming kernel would hold */
+    auto position_terms = [&](int b, float (&acc)[4][4]) {
+        Head hd;
+        F::head(hd, wrow, q);
+        const ckq_v4i dxi = lds16(reinterpret_cast<const uint8_t *>(dxs + b * NT + 4 * (q & (QL - 1))));
+        ckq_v4i am;
+        if (F::MIN) am = bsum_operand();
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            ckq_v4i ph, pl;
+            F::planes(ph, pl, hd, wrow, g, q);
+            const ckq_v4i a = lds16(al + aofs[g]);
+            const ckq_v4i sh = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, ph, zero, 0, 0, 0);
+            const ckq_v4i sl = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, pl, zero, 0, 0, 0);
+            ckq_v4f i2;
+            if constexpr (F::MIN) i2 = min_mfma(am, q == g ? hd.mins : zero);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int di = dxi[r];
+                const float dx = __builtin_bit_cast(float, di), f = (float)((sh[r] << F::SHIFT) + sl[r]);
+                float v;
+                if constexpr (F::MIN) v = (hd.dw * dx) * f - (hd.dmin * dx) * i2[r];
+                else                  v = (hd.dw * dx) * f;
+                asm volatile("" : "+v"(v));                  /* rounded before it is added, as there */
+                acc[g][r] += v;
+            }
+        }
+    };
+
+    /* block scales of the tokens, [block][NT]: their loads go out first, so that waiting for them waits for nothing else */
+    constexpr int ND = 2;
+    const int nd = nb * NT;
+    float dxv[ND];
+    auto dx_load = [&](int e) {
+        const int t = e % NT, b = e / NT;
+        return __builtin_bit_cast(float, ld4<4>(xbase + (size_t)((u32)min(t, M - 1 - t0) * xrow + (u32)b * 292u)));
+    };
+#pragma unroll
+    for (int k = 0; k < ND; ++k) dxv[k] = dx_load(min(tid + k * nthr, nd - 1));
+    if (wave < nb) fetch(wave);
+#pragma unroll
+    for (int k = 0; k < ND; ++k)
+        if (tid + k * nthr < nd) dxs[tid + k * nthr] = dxv[k];
+    for (int e = tid + ND * nthr; e < nd; e += nthr) dxs[e] = dx_load(e);        /* long rows */
+    if constexpr (TREE) {
+        __syncthreads();                                                         /* for the scales only: the blocks' loads stay in flight */
+        /* a lane of the streaming kernel holds positions l, l + 64, ...: blocks b, b + 16, ... meet in one sum per position */
+        for (int b0 = wave; b0 < min(nb, 16); b0 += nwave) {
+            float acc[4][4];
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[g][r] = 0.0f;
+            for (int b = b0; b < nb; b += 16) {
+                take();
+                const int next = b + 16 < nb ? b + 16 : b0 + nwave;
+                if (next < nb && (b + 16 < nb || next < 16)) fetch(next);
+                __builtin_amdgcn_sched_barrier(0);
+                position_terms(b, acc);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            float out[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) out[r] = (acc[0][r] + acc[1][r]) + (acc[2][r] + acc[3][r]);
+            put(b0, out);
+        }
+    } else {
+        for (int b = wave; b < nb; b += nwave) {
+            take();
+            if (b + nwave < nb) fetch(b + nwave);
+            __builtin_amdgcn_sched_barrier(0);
+            block_term(b);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    __syncthreads();
+    for (int e = tid; e < NT * 16; e += nthr) {
+        const int l = e % (16 * QL), r = e / (16 * QL);
+        const int tok = 4 * (l >> 4) + r;
+        const float *u = us + r * (16 * QL) + l, *dx = dxs + tok;
+        float v = 0.0f;
+        if constexpr (TREE) {
+            /* the streaming kernel's fixed tree over the lanes of a row, four of them per block */
+            float t[16];
+#pragma unroll
+            for (int b = 0; b < 16; ++b) t[b] = b < nb ? u[b * (NT * 16)] : 0.0f;
+#pragma unroll
+            for (int w = 1; w < 16; w *= 2)
+#pragma unroll
+                for (int b = 0; b < 16; b += 2 * w) t[b] += t[b + w];
+            v = t[0];
+        } else {
+            for (int sp = 0; sp < ch.splits; ++sp) {
+                const int b0 = sp * ch.per, b1 = min(nb, b0 + ch.per);
+                float c[2] = {0.0f, 0.0f};
+                for (int b = b0; b < b1; b += 4) {
+                    float uu[4], dd[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const int bk = min(b + k, b1 - 1);
+                        uu[k] = u[bk * (NT * 16)];
+                        dd[k] = dx[bk * NT];
+                    }
+                    if (ch.kg == 2) {
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) c[k & 1] = b + k < b1 ? fmaf(dd[k], uu[k], c[k & 1]) : c[k & 1];
+                    } else {
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) c[0] = b + k < b1 ? fmaf(dd[k], uu[k], c[0]) : c[0];
+                    }
+                }
+                if (ch.kg == 2) c[0] += c[1];
+                v = sp ? v + c[0] : c[0];
+            }
+        }
+        const int n = n0 + (l & 15), t = t0 + tok;
+        if (n < N && t < M) y[(size_t)t * ldy + n] = bias ? v + bias[n] : v;
+    }
+}
+
+/* Waves per block: with two tiles per CU and more, blocks of four waves overlap each other's beginnings and ends
+ * (32000 x 4096, 13 tokens: 27 us, with eight 41); with fewer, a tile's blocks spread over more waves. */
+int rows16_waves(int tiles, int nb)
+{
+    int waves = tiles >= 512 ? 4 : tiles > 64 ? 8 : 16;
+    while (waves > 4 && waves / 2 >= nb) waves /= 2;
+    return waves;
+}
+
+template <class F, int NT, bool TREE>
+int launch_rows16_nt(Rows16Args &a, hipStream_t s)
+{
+    unsigned grid = 0;
+    for (int i = 0; i < a.n; ++i) {
+        a.p[i].id0 = (int)grid;
+        grid += (unsigned)((a.p[i].N + 15) / 16);
+    }
+    const unsigned gy = (unsigned)((a.M + NT - 1) / NT);
+    if (gy > 65535) return CKQ_ESHAPE;
+    auto lds_bytes = [&](int w) { return (size_t)w * rows16_wave_lds<F, NT>() + (size_t)(TREE && a.nb > 16 ? 16 : a.nb) * (NT * 64) + (size_t)a.nb * (NT * 4); };
+    int waves = rows16_waves((int)(grid * gy), TREE ? (a.nb < 16 ? a.nb : 16) : a.nb);
+    while (waves > 4 && lds_bytes(waves) > 160 * 1024) waves -= 4;
+    const size_t lds = lds_bytes(waves);
+    if (lds > 160 * 1024) return CKQ_ESHAPE;
+    if (lds > 64 * 1024) {
+        /* more than 64 KB of dynamic LDS is an opt-in per function and device; asked for once */
+        static std::atomic<uint64_t> done[2];
+        int dev = 0;
+        hipError_t e = hipGetDevice(&dev);
+        if (e != hipSuccess) return (int)e;
+        const uint64_t bit = 1ull << (dev & 63);
+        if (!(done[a.n > 1].load(std::memory_order_acquire) & bit)) {
+            e = hipFuncSetAttribute(a.n > 1 ? (const void *)gemm_rows16_kernel<F, NT, TREE, true> : (const void *)gemm_rows16_kernel<F, NT, TREE, false>,
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+            if (e != hipSuccess) return (int)e;
+            done[a.n > 1].fetch_or(bit, std::memory_order_release);
+        }
+    }
+    const Rows16Problem &p = a.p[0];
+    const Rows16Shape S = {a.M, a.nb};
+    if (a.n > 1)
+        hipLaunchKernelGGL((gemm_rows16_kernel<F, NT, TREE, true>), dim3(grid, gy), dim3(64 * waves), lds, s, p.W, p.X, p.N, S, p.y, p.bias, p.ldy, p.ch, a);
+    else
+        hipLaunchKernelGGL((gemm_rows16_kernel<F, NT, TREE, false>), dim3(grid, gy), dim3(64 * waves), lds, s, p.W, p.X, p.N, S, p.y, p.bias, p.ldy, p.ch, a);
+    return (int)hipGetLastError();
+}
+
+template <class F>
+int launch_rows16(Rows16Args &a, hipStream_t s)
+{
+    if (a.tree) return a.M <= 8 ? launch_rows16_nt<F, 8, true>(a, s) : launch_rows16_nt<F, 16, true>(a, s);
+    return a.M <= 8 ? launch_rows16_nt<F, 8, false>(a, s) : launch_rows16_nt<F, 16, false>(a, s);
+}
+
+} // namespace
+
+int launch_gemm_rows16(int fmt, Rows16Args &a, hipStream_t s)
+{
+    switch (fmt) {
+    case CKQ_FMT_Q4_K: return launch_rows16<R16Q4K>(a, s);
+    case CKQ_FMT_Q5_K: return launch_rows16<R16Q5K>(a, s);
+    case CKQ_FMT_Q6_K: return launch_rows16<R16Q6K>(a, s);
+    default: return CKQ_EFORMAT;
+    }
+}

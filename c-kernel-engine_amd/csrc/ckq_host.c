@@ -698,6 +698,7 @@ void ckq_weights_set_cache(int enabled)
 void ckq_set_gemm_policy(int policy) { ckq_launch_set_gemm_policy(policy); }
 void ckq_set_prefill_variant(int fmt, int variant)
 {
+    ckq_launch_set_rows16(fmt, variant == 16);
     if (fmt == CKQ_FMT_Q4_K) ckq_launch_set_q4k_tile(variant);
     else if (fmt == CKQ_FMT_Q6_K) ckq_launch_set_q6k_variant(variant);
     else if (fmt == CKQ_FMT_Q5_K) ckq_launch_set_q5k_variant(variant);

@@ -96,6 +96,7 @@ static bool f32act_on_matrix_cores(int fmt, int ntok, int nrows, int K)
 #include "ckq_gemv.hpp"
 #include "ckq_gemm_common.hpp"
 #include "ckq_gemm_f32act.hpp"
+#include "ckq_gemm_rows16.hpp"
 
 /* C = bias + partial 0 + partial 1 + ... in that order: the result does not
  * depend on which block finished first.  One thread per output. */
@@ -258,6 +259,64 @@ static bool weights_dword_aligned(const GemvArgs &a, const GemvGroup &grp)
     return (bits & 3) == 0;
 }
 
+/* Whether the matrix-core kernel on 16-row tiles (ckq_gemm_rows16.hip) takes a matmul of `rows` rows (all matrices of a
+ * launch) that would otherwise go to the tile kernels (`tiles`) or to the streaming kernel.  The results are the same bits
+ * either way, so only time decides.  Fitted to launches of all three over 128..32000 rows, widths of 1024..11008 and 5..128
+ * tokens (us; nb: 256-blocks of a row, mb: megabytes of weights, n16: thousands of 256-blocks of 16 rows times groups of 16
+ * tokens); over all of them the rule's choices are within 1 % of always taking the faster:
+ *   rows16     3.6 + 0.12 nb + (Q4_K 0.36, Q5_K 0.65, Q6_K 0.71) n16
+ *   tiles      11 + 0.2 mb + 0.0015 tokens mb, an under-estimate almost everywhere
+ *   streaming  the larger of 4.35 + 0.07 nb and 3.05 + 0.11 nb + (0.24, 0.245, 0.29) mb for every eight tokens, 5 to 8 as 10
+ * Three and four tokens, one pass of half the width, only move for long rows of large matrices (4096 x 11008 Q6_K:
+ * 17.0 -> 13.4); two never do.  The forced policies keep their kernels: 1 the tile kernels, and 2 the streaming kernels,
+ * whose order this one keeps where `tiles` is false. */
+static std::atomic<int> g_rows16_forced{0};           /* bit per format tag */
+extern "C" void ckq_launch_set_rows16(int fmt, int on)
+{
+    if (fmt < 0 || fmt > 31) return;
+    if (on) g_rows16_forced.fetch_or(1 << fmt);
+    else g_rows16_forced.fetch_and(~(1 << fmt));
+}
+static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles)
+{
+    if (ntok < 2 || K > ROWS16_MAX_K) return false;
+    if (g_rows16_forced.load(std::memory_order_relaxed) >> fmt & 1) return true;
+    if (ntok < 3) return false;
+    if (tiles && g_gemm_policy.load(std::memory_order_relaxed) == 1) return false;
+    const int f = fmt == CKQ_FMT_Q4_K ? 0 : fmt == CKQ_FMT_Q5_K ? 1 : 2;
+    static const float per_block[3] = {0.36f, 0.65f, 0.71f}, per_pass[3] = {0.24f, 0.245f, 0.29f};
+    const float nb = (float)(K / 256), mb = (float)rows * nb * (f == 0 ? 144e-6f : f == 1 ? 176e-6f : 210e-6f);
+    if (ntok <= 4) return K > 4096 && mb >= 20.0f;
+    const float passes = ntok <= 8 ? 1.25f : (float)((ntok + 7) / 8);
+    const float t_rows = 3.6f + 0.12f * nb + per_block[f] * 1e-3f * nb * (float)((rows + 15) / 16) * (float)((ntok + 15) / 16);
+    const float t_stream = 3.05f + 0.11f * nb + per_pass[f] * mb * passes, t_least = 4.35f + 0.07f * nb;
+    const float t_else = tiles ? 11.0f + (0.2f + 0.0015f * (float)ntok) * mb : t_stream > t_least ? t_stream : t_least;
+    return t_rows < t_else;
+}
+
+/* The chains of multiply-adds of such a launch: those of the tile kernel where it stands in for one, so that the result
+ * has the tile kernel's bits. */
+static GemmChains rows16_chains(int fmt, int ntok, int nrows, int K, bool tiles)
+{
+    if (!tiles) return {1, K / 256, 1};
+    return fmt == CKQ_FMT_Q4_K ? gemm_q4k_chains(ntok, nrows, K) : fmt == CKQ_FMT_Q5_K ? gemm_q5k_chains(ntok, nrows, K) : gemm_q6k_chains(ntok, nrows, K);
+}
+
+/* K-quants: does a matmul of this size go to the tile kernels (or, at their sizes, to the 16-row tiles)? */
+static bool kquant_on_matrix_cores(int fmt, int ntok, size_t rows, int K)
+{
+    return gemm_on_matrix_cores(ntok, rows * (size_t)(K / 256) * (fmt == CKQ_FMT_Q4_K ? 144 : fmt == CKQ_FMT_Q5_K ? 176 : 210), fmt == CKQ_FMT_Q5_K ? 40 : 20);
+}
+
+static int launch_rows16_one(int fmt, const GemvArgs &a, bool tiles, int K, hipStream_t s)
+{
+    Rows16Args r = {};
+    r.tree = !tiles;
+    r.M = a.ntok; r.nb = K / 256; r.n = 1;
+    r.p[0] = {a.W, a.X, a.y, a.bias, a.ldy, a.nrows, 0, rows16_chains(fmt, a.ntok, a.nrows, K, tiles)};
+    return launch_gemm_rows16(fmt, r, s);
+}
+
 static const GemvGroup k_no_group = {{}, {}, {}, {}, {}, {}, 1};
 
 static int launch_gemv_args(int fmt, GemvArgs &a, const GemvGroup &grp, int K, void *stream, const GemmOpts &opts = GemmOpts{});
@@ -332,6 +391,33 @@ extern "C" int ckq_launch_gemv_group(int fmt, int n, float *const *y, const void
         }
         return 0;
     }
+    /* Matrices that the 16-row tiles take when launched alone share a launch of theirs, the others one of the streaming
+     * kernel: every result keeps the bits of its single launch. */
+    if (!subdots && (fmt == CKQ_FMT_Q4_K || fmt == CKQ_FMT_Q5_K || fmt == CKQ_FMT_Q6_K) && K % 256 == 0) {
+        Rows16Args r = {};
+        r.M = ntok; r.nb = K / 256; r.tree = true;
+        int rest[CKQ_GROUP_MAX], nrest = 0;
+        for (int i = 0; i < n; ++i) {
+            if (take_rows16(fmt, ntok, (size_t)rows[i], K, false))
+                r.p[r.n++] = {(const uint8_t *)W[i], (const uint8_t *)X[i], y[i], bias ? bias[i] : nullptr, ldys[i], rows[i], 0, {}};
+            else
+                rest[nrest++] = i;
+        }
+        if (r.n) {
+            int rc = launch_gemm_rows16(fmt, r, (hipStream_t)stream);
+            if (rc || !nrest) return rc;
+            float *ry[CKQ_GROUP_MAX];
+            const void *rW[CKQ_GROUP_MAX], *rX[CKQ_GROUP_MAX];
+            const float *rb[CKQ_GROUP_MAX];
+            int rrows[CKQ_GROUP_MAX];
+            long rld[CKQ_GROUP_MAX];
+            for (int i = 0; i < nrest; ++i) {
+                const int k = rest[i];
+                ry[i] = y[k]; rW[i] = W[k]; rX[i] = X[k]; rb[i] = bias ? bias[k] : nullptr; rrows[i] = rows[k]; rld[i] = ldys[k];
+            }
+            return ckq_launch_gemv_group(fmt, nrest, ry, rW, rX, rb, rrows, rld, K, ntok, nullptr, stream);
+        }
+    }
     GemvArgs a = {};
     GemvGroup grp = k_no_group;
     a.y = subdots ? nullptr : y[0]; a.W = (const uint8_t *)W[0]; a.X = (const uint8_t *)X[0];
@@ -361,20 +447,29 @@ static int launch_gemv_args(int fmt_flags, GemvArgs &a, const GemvGroup &grp, in
     switch (fmt) {
     case CKQ_FMT_Q4_K:
         if (K % 256) return CKQ_ESHAPE;
-        if (whole && gemm_on_matrix_cores(ntok, (size_t)nrows * (K / 256) * 144, 20))
-            return launch_gemm_q4k_mfma(X, W, bias, y, ntok, nrows, K, ldy, opts, s);
+        if (whole) {
+            const bool tiles = kquant_on_matrix_cores(fmt, ntok, (size_t)nrows, K);
+            if (take_rows16(fmt, ntok, (size_t)nrows, K, tiles)) return launch_rows16_one(fmt, a, tiles, K, s);
+            if (tiles) return launch_gemm_q4k_mfma(X, W, bias, y, ntok, nrows, K, ldy, opts, s);
+        }
         a.npos = K / 64; a.wrow = (long)(K / 256) * 144; a.xrow = (long)(K / 256) * 292; a.nsub_row = K / 32;
         return ckq_gemv_launch_q4k(a, grp, s);
     case CKQ_FMT_Q5_K:
         if (K % 256) return CKQ_ESHAPE;
-        if (whole && gemm_on_matrix_cores(ntok, (size_t)nrows * (K / 256) * 176, 40))
-            return launch_gemm_q5k_mfma(X, W, bias, y, ntok, nrows, K, ldy, opts, s);
+        if (whole) {
+            const bool tiles = kquant_on_matrix_cores(fmt, ntok, (size_t)nrows, K);
+            if (take_rows16(fmt, ntok, (size_t)nrows, K, tiles)) return launch_rows16_one(fmt, a, tiles, K, s);
+            if (tiles) return launch_gemm_q5k_mfma(X, W, bias, y, ntok, nrows, K, ldy, opts, s);
+        }
         a.npos = K / 64; a.wrow = (long)(K / 256) * 176; a.xrow = (long)(K / 256) * 292; a.nsub_row = K / 32;
         return ckq_gemv_launch_q5k(a, grp, s);
     case CKQ_FMT_Q6_K:
         if (K % 256) return CKQ_ESHAPE;
-        if (whole && gemm_on_matrix_cores(ntok, (size_t)nrows * (K / 256) * 210, 20))
-            return launch_gemm_q6k_mfma(X, W, bias, y, ntok, nrows, K, ldy, opts, s);
+        if (whole) {
+            const bool tiles = kquant_on_matrix_cores(fmt, ntok, (size_t)nrows, K);
+            if (take_rows16(fmt, ntok, (size_t)nrows, K, tiles)) return launch_rows16_one(fmt, a, tiles, K, s);
+            if (tiles) return launch_gemm_q6k_mfma(X, W, bias, y, ntok, nrows, K, ldy, opts, s);
+        }
         a.npos = K / 64; a.wrow = (long)(K / 256) * 210; a.xrow = (long)(K / 256) * 292; a.nsub_row = K / 16;
         return ckq_gemv_launch_q6k(a, grp, s);
     case CKQ_FMT_Q8_0:
@@ -444,18 +539,38 @@ extern "C" int ckq_launch_gemm_group(int fmt, int n, float *const *C, const void
         aligned = aligned && ((uintptr_t)B[p] % 4 == 0);
     }
     hipStream_t s = (hipStream_t)stream;
+    if ((fmt == CKQ_FMT_Q4_K || fmt == CKQ_FMT_Q5_K || fmt == CKQ_FMT_Q6_K) && K % 256 == 0) {
+        /* 16-row tiles: in place of the tile kernels' shared launch where they would take it, else of the single launches
+         * (of one kind, as a launch has one order of its sums), with the bits of either */
+        GemmChains shared = {};
+        const bool grouped = kquant_on_matrix_cores(fmt, M, rows, K) &&
+                             (fmt == CKQ_FMT_Q4_K   ? gemm_q4k_group_chains(in, M, K, &shared)
+                              : fmt == CKQ_FMT_Q5_K ? gemm_q5k_group_chains(in, M, K, &shared)
+                                                    : gemm_q6k_group_chains(in, M, K, &shared));
+        bool tiles[GEMM_GROUP_MAX], alike = true;
+        for (int p = 0; p < n; ++p) {
+            tiles[p] = grouped || kquant_on_matrix_cores(fmt, M, (size_t)N[p], K);
+            alike = alike && tiles[p] == tiles[0];
+        }
+        if (alike && take_rows16(fmt, M, rows, K, tiles[0])) {
+            Rows16Args r = {};
+            r.M = M; r.nb = K / 256; r.n = n; r.tree = !tiles[0];
+            for (int p = 0; p < n; ++p)
+                r.p[p] = {(const uint8_t *)B[p], (const uint8_t *)A, C[p], bias ? bias[p] : nullptr, ldc[p], N[p], 0,
+                          grouped ? shared : rows16_chains(fmt, M, N[p], K, tiles[p])};
+            return launch_gemm_rows16(fmt, r, s);
+        }
+        if (!grouped) return CKQ_ENOGROUP;
+    }
     switch (fmt) {
     case CKQ_FMT_Q4_K:
         if (K % 256) return CKQ_ESHAPE;
-        if (!gemm_on_matrix_cores(M, rows * (K / 256) * 144, 20)) return CKQ_ENOGROUP;
         return launch_gemm_q4k_mfma_group(A, in, M, K, s);
     case CKQ_FMT_Q5_K:
         if (K % 256) return CKQ_ESHAPE;
-        if (!gemm_on_matrix_cores(M, rows * (K / 256) * 176, 40)) return CKQ_ENOGROUP;
         return launch_gemm_q5k_mfma_group(A, in, M, K, s);
     case CKQ_FMT_Q6_K:
         if (K % 256) return CKQ_ESHAPE;
-        if (!gemm_on_matrix_cores(M, rows * (K / 256) * 210, 20)) return CKQ_ENOGROUP;
         return launch_gemm_q6k_mfma_group(A, in, M, K, s);
     case CKQ_FMT_Q8_0:
         if (K % 32) return CKQ_ESHAPE;

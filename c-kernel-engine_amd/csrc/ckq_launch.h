@@ -79,6 +79,8 @@ void ckq_launch_set_q4k_tile(int tokens);
 void ckq_launch_set_q6k_variant(int variant);
 /* Q5_K x Q8_K matrix-core GEMM: 0 = by tile count (default), 1 = one block per CU always, 2 = the paired kernel always. */
 void ckq_launch_set_q5k_variant(int variant);
+/* K-quants: 1 = the 16-row tiles take every matmul of two and more tokens (K up to 16384), 0 = by shape (default). */
+void ckq_launch_set_rows16(int fmt, int on);
 
 /* fp32 [rows x k] -> Q8_K / Q8_0 blocks, row-major. */
 int ckq_launch_quantize_q8_k(const float *x, void *y, int rows, int k, void *stream);

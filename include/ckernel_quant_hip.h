@@ -438,6 +438,8 @@ void ckq_set_gemm_policy(int policy);
  *                 quarter or more of its last round (CKQ_Q6K_VARIANT=1|2);
  *   CKQ_FMT_Q5_K: 1 = one block per CU, three LDS stages deep, 2 = two blocks per CU with one LDS image of the weights,
  *                 taken for more tiles than CUs (CKQ_Q5K_VARIANT=1|2).
+ *   16 with any of the three: matmuls of two and more tokens run on 16-row tiles whatever their shape (taken by default from
+ *                 three to a few dozen tokens, by shape; K up to 16384).  The bits are those of the kernel it stands in for.
  * Q8_0 has one variant. */
 void ckq_set_prefill_variant(int fmt, int variant);
 /* Last error of the calling process (0 = none), its text, and a reset for

@@ -1229,3 +1229,62 @@ def test_f32act_matrix_cores_vs_fp64(fmt):
             assert np.all(got[3] == np.copysign(np.inf, w0[k]))
     finally:
         L.ckq_set_gemm_policy(0)
+
+
+# ---- 16-row tiles: a few to a few dozen tokens of the K-quants -------------------------------------
+
+@pytest.mark.parametrize("fmt", ["q4_k", "q5_k", "q6_k"])
+def test_16_row_tiles_vs_oracle_and_the_kernels_they_stand_in_for(fmt):
+    """The kernel forced at the edges of its tiles - two tokens, eight and sixteen and one more, row counts
+    around 16, one K-block, more K-blocks than waves, the longest row it takes - against the oracle, with a
+    bias and a padded C.  It has the bits of the kernel that would otherwise run: of the streaming kernel at
+    these sizes, of the tile kernels, K split and wave groups included, at those of the matrix cores; three
+    matrices of one input share a launch."""
+    import torch
+    L = ckq.lib()
+    tag = P.FMT[fmt]
+    try:
+        for M, N, K in [(2, 1, 256), (8, 15, 512), (9, 16, 1024), (16, 17, 2304), (17, 33, 43 * 256), (13, 70, 64 * 256), (40, 100, 5 * 256)]:
+            W, _, xq = make_case(fmt, N, K, "rand" if N % 2 else "enc", 9100 + M + N, tokens=M)
+            bias = T.normal(N, 0.0, 0.5, seed=N)
+            say("16-row tiles", fmt, M, N, K)
+            L.ckq_set_prefill_variant(tag, 16)
+            c = torch.full((M, N + 3), 7.0, dtype=torch.float32, device="cuda")
+            x_d, W_d, b_d = P.to_device(xq), P.to_device(W), P.to_device(bias)
+            P.check(L.ckq_gemm_nt_dev(tag, P._dp(x_d), P._dp(W_d), P._dp(b_d), P._dp(c), M, N, K, N + 3, P._stream()), "ckq_gemm_nt_dev")
+            got = c.cpu().numpy()
+            assert T.norm_err(got[:, :N], T.oracle_gemm_nt(fmt, xq, W, bias, M, N, K)) <= TOL, (M, N, K)
+            assert np.all(got[:, N:] == 7.0), (M, N, K)
+            rb = x_d.numel() // M
+            for m in {0, M // 2, M - 1}:
+                one = P.dev_gemm_nt(fmt, x_d[m * rb:(m + 1) * rb].clone(), W_d, b_d, 1, N, K)
+                assert torch.equal(c[m, :N], one.view(N)), (M, N, K, m)
+        for M, N, K in [(9, 11008, 2048), (17, 4096, 4096), (33, 4096, 11008), (12, 32000, 512), (100, 4864, 4096)]:
+            xq = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, seed=M)), "q8_k", rows=M)
+            W = P.to_device(T.random_blocks(fmt, N * K // 256, 9200 + M))
+            say("16-row tiles against the tile kernels", fmt, M, N, K)
+            L.ckq_set_prefill_variant(tag, 16)
+            L.ckq_set_gemm_policy(0)
+            a = P.dev_gemm_nt(fmt, xq, W, None, M, N, K).clone()
+            L.ckq_set_prefill_variant(tag, 0)
+            L.ckq_set_gemm_policy(1)
+            b = P.dev_gemm_nt(fmt, xq, W, None, M, N, K).clone()
+            L.ckq_set_gemm_policy(0)
+            budget = (40 if fmt == "q5_k" else 20) << 20
+            if (M + 7) // 8 * max(N * T.row_bytes(fmt, K), 3 << 20) > budget:      # the streaming kernel's part ends here
+                assert torch.equal(a, b), (M, N, K)
+            else:
+                assert torch.allclose(a, b, rtol=0, atol=2e-6 * float(b.abs().max())), (M, N, K)
+        M, K, Ns = 12, 1024, [640, 33, 16]
+        L.ckq_set_prefill_variant(tag, 16)
+        xq = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, seed=3)), "q8_k", rows=M)
+        Ws = [P.to_device(T.synth_weights(fmt, n, K, seed=9300 + i)) for i, n in enumerate(Ns)]
+        ys = [torch.zeros(M * n, dtype=torch.float32, device="cuda") for n in Ns]
+        for m in (M, 5):
+            say("16-row tiles, grouped", fmt, m)
+            P.dev_matmul_sequence([(fmt, xq, W, None, y, m, n, K) for W, y, n in zip(Ws, ys, Ns)])
+            for W, y, n in zip(Ws, ys, Ns):
+                assert torch.equal(y[:m * n].view(m, n), P.dev_gemm_nt(fmt, xq, W, None, m, n, K).view(m, n)), (m, n)
+    finally:
+        L.ckq_set_gemm_policy(0)
+        L.ckq_set_prefill_variant(tag, 0)
