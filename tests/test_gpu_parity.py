@@ -1288,3 +1288,37 @@ def test_16_row_tiles_vs_oracle_and_the_kernels_they_stand_in_for(fmt):
     finally:
         L.ckq_set_gemm_policy(0)
         L.ckq_set_prefill_variant(tag, 0)
+
+
+@pytest.mark.parametrize("blocks", [1, 2, 3, 4, 5, 6, 7, 8, 13, 37, 64])
+def test_gemm_mfma_q8_0_row_alignment_and_k_remainders(blocks):
+    """Rows of odd and even numbers of 32-blocks (odd ones start on dwords every other row), K ending after one, two, three
+    and four blocks of the last step, operands that start two bytes past a dword, an infinite weight scale."""
+    import torch
+    L = ckq.lib()
+    K = 32 * blocks
+    try:
+        L.ckq_set_gemm_policy(1)
+        for M, N, wo, xo in [(9, 5, 0, 0), (64, 128, 2, 0), (70, 200, 0, 2), (65, 131, 2, 2)]:
+            W, _, xq = make_case("q8_0", N, K, "rand", 9400 + M + blocks, tokens=M)
+            if M == 70:
+                W = W.copy()
+                W.reshape(N, -1)[3, :2] = (0x00, 0x7C)
+            bias = T.normal(N, 0.0, 0.5, seed=N)
+            say("q8_0 alignment", M, N, K, wo, xo)
+            ref = T.oracle_gemm_nt("q8_0", xq, W, bias, M, N, K)
+            wd = torch.zeros(len(W) + 4, dtype=torch.uint8, device="cuda")
+            xd = torch.zeros(len(xq) + 4, dtype=torch.uint8, device="cuda")
+            wd[wo:wo + len(W)] = P.to_device(W)
+            xd[xo:xo + len(xq)] = P.to_device(xq)
+            c = torch.full((M, N + 1), 7.0, dtype=torch.float32, device="cuda")
+            b = P.to_device(bias)
+            P.check(L.ckq_gemm_nt_dev(P.FMT["q8_0"], xd.data_ptr() + xo, wd.data_ptr() + wo, P._dp(b), P._dp(c), M, N, K,
+                                      N + 1, P._stream()), "ckq_gemm_nt_dev")
+            got = c.cpu().numpy()
+            assert np.all(got[:, N] == 7.0)
+            ok = np.isfinite(ref)
+            assert np.array_equal(np.isnan(got[:, :N]), np.isnan(ref)) and np.array_equal(got[:, :N][~ok & ~np.isnan(ref)], ref[~ok & ~np.isnan(ref)])
+            assert T.norm_err(np.where(ok, got[:, :N], 0.0), np.where(ok, ref, 0.0)) <= TOL, (M, N, K)
+    finally:
+        L.ckq_set_gemm_policy(0)
