@@ -84,6 +84,22 @@ __device__ __forceinline__ T group_sum(T v)
     return v;
 }
 
+/* Largest of a wave's 64 values, none of them negative, in every lane (through a scalar register); NaNs are passed over
+ * as fmaxf does.  Six DPP steps of one VALU instruction and its wait states: the shuffles through LDS that this replaced
+ * (ds_bpermute) cost a round trip of some 120 cycles a step, one after another, in kernels that are one chain of
+ * latencies when a launch is a single row. */
+__device__ __forceinline__ float wave_max(float v)
+{
+    v = fmaxf(v, dpp_get<0xB1>(v));               /* quad_perm [1,0,3,2] */
+    v = fmaxf(v, dpp_get<0x4E>(v));               /* quad_perm [2,3,0,1] */
+    v = fmaxf(v, dpp_get<0x141>(v));              /* row_half_mirror */
+    v = fmaxf(v, dpp_get<0x140>(v));              /* row_mirror: every lane of a row of 16 has the row's */
+    const int i = __builtin_bit_cast(int, v);     /* the four rows, not through row_bcast: an all-NaN row stays NaN */
+    const float a = __builtin_bit_cast(float, __builtin_amdgcn_readlane(i, 0)), b = __builtin_bit_cast(float, __builtin_amdgcn_readlane(i, 16));
+    const float c = __builtin_bit_cast(float, __builtin_amdgcn_readlane(i, 32)), d = __builtin_bit_cast(float, __builtin_amdgcn_readlane(i, 48));
+    return fmaxf(fmaxf(a, b), fmaxf(c, d));
+}
+
 /* x86 cvtps2dq + saturating packs (quantize_row_q8_k_sse.c:61-68): round to
  * nearest even; NaN, +-inf and anything outside int32 convert to INT_MIN, which
  * the packs saturate to -128 - also for +inf and for values >= 2^31 (a block of
@@ -103,19 +119,16 @@ __device__ __forceinline__ int rne_sat_i8(float p)
  * zero bytes. */
 __device__ __forceinline__ void q8k_quantize_block(const float (&e)[4], int lane, uint8_t *out)
 {
-    float amax = 0.0f, smax = 0.0f;
-    int idx = 4 * lane;
+    float lmax = 0.0f, smax = 0.0f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const float ax = fabsf(e[i]);
-        if (ax > amax) { amax = ax; smax = e[i]; idx = 4 * lane + i; }
+        if (ax > lmax) { lmax = ax; smax = e[i]; }
     }
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const float oa = __shfl_xor(amax, off), os = __shfl_xor(smax, off);
-        const int   oi = __shfl_xor(idx, off);
-        if (oa > amax || (oa == amax && oi < idx)) { amax = oa; smax = os; idx = oi; }
-    }
+    /* elements go up with the lane: the first lane that holds the maximum has the first of the largest elements */
+    const float amax = wave_max(lmax);
+    const int first = __builtin_ctzll(__builtin_amdgcn_ballot_w64(lmax == amax));
+    smax = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, smax), first));
     if (amax == 0.0f) {
         reinterpret_cast<u32 *>(out)[lane] = 0;
         if (lane < 9) reinterpret_cast<u32 *>(out)[64 + lane] = 0;

@@ -41,32 +41,56 @@ __device__ __forceinline__ void pro_quantize_block(const float *__restrict__ x, 
  * ulp and quants flip: eight strided lanes (lane j takes x[8i+j]) each a chain
  * of fused multiply-adds, combined as ((l0+l4)+(l1+l5)) + ((l2+l6)+(l3+l7)). */
 
-/* Thread j < 8 of the block walks chain j over the row staged in LDS at xs
- * (D floats, D a multiple of 256) and leaves its sum at xs[D + j].  The chain
- * is serial; sixteen LDS reads are kept in flight ahead of it. */
+/* The row lies in LDS chain by chain: element 8 i + j at xs[j * rms_pitch(D) + i], so that a chain is read 16 bytes at a
+ * time.  The pitch of D/8 + 8 floats puts the eight chains' reads, and the 64 lanes of a staging store, on different banks
+ * (D/8 is a multiple of 32). */
+__host__ __device__ __forceinline__ constexpr int rms_pitch(int D) { return D / 8 + 8; }
+__host__ __device__ __forceinline__ constexpr size_t rms_lds_bytes(size_t D) { return (8 * (D / 8 + 8) + 8) * sizeof(float); }
+
+/* Lane l of a wave stores elements 4 l .. 4 l + 3 of 256-block b. */
+__device__ __forceinline__ void rms_stage(float *xs, int D, int b, int lane, const float4 v)
+{
+    float *p = xs + 4 * (lane & 1) * rms_pitch(D) + 32 * b + (lane >> 1);
+    p[0] = v.x;
+    p[rms_pitch(D)] = v.y;
+    p[2 * rms_pitch(D)] = v.z;
+    p[3 * rms_pitch(D)] = v.w;
+}
+
+/* Thread j < 8 of the block walks chain j and leaves its sum behind the row.  The chain is serial, one multiply-add
+ * after another; the 32 values of the next 256-block are read while those of this one are added. */
 __device__ __forceinline__ void rms_chain(float *xs, int D, int j)
 {
-    float acc = 0.0f, cur[16], nxt[16];
+    const float4 *x = reinterpret_cast<const float4 *>(xs + j * rms_pitch(D));
+    float acc = 0.0f;
+    float4 cur[8], nxt[8];
 #pragma unroll
-    for (int u = 0; u < 16; ++u) cur[u] = xs[j + 8 * u];
-    for (int d = 0; d < D; d += 128) {
-        const int dn = d + 128 < D ? d + 128 : d;
+    for (int u = 0; u < 8; ++u) cur[u] = x[u];
+    const int nb = D / 256;
+    for (int b = 0; b < nb; ++b) {
+        const float4 *xn = x + 8 * (b + 1 < nb ? b + 1 : b);
 #pragma unroll
-        for (int u = 0; u < 16; ++u) nxt[u] = xs[dn + j + 8 * u];
+        for (int u = 0; u < 8; ++u) nxt[u] = xn[u];
 #pragma unroll
-        for (int u = 0; u < 16; ++u) acc = __fmaf_rn(cur[u], cur[u], acc);
+        for (int u = 0; u < 8; ++u) {
+            acc = __fmaf_rn(cur[u].x, cur[u].x, acc);
+            acc = __fmaf_rn(cur[u].y, cur[u].y, acc);
+            acc = __fmaf_rn(cur[u].z, cur[u].z, acc);
+            acc = __fmaf_rn(cur[u].w, cur[u].w, acc);
+        }
 #pragma unroll
-        for (int u = 0; u < 16; ++u) cur[u] = nxt[u];
+        for (int u = 0; u < 8; ++u) cur[u] = nxt[u];
     }
-    xs[D + j] = acc;
+    xs[8 * rms_pitch(D) + j] = acc;
 }
 
 /* rstd from the eight chain sums (every thread derives the same value).
  * sqrtf and '/' are the correctly rounded ones (the __fsqrt_rn intrinsic is not). */
 __device__ __forceinline__ float rms_rstd(const float *xs, int D, float eps)
 {
-    const float s04 = xs[D + 0] + xs[D + 4], s15 = xs[D + 1] + xs[D + 5];
-    const float s26 = xs[D + 2] + xs[D + 6], s37 = xs[D + 3] + xs[D + 7];
+    const float4 *l = reinterpret_cast<const float4 *>(xs + 8 * rms_pitch(D));
+    const float4 a = l[0], b = l[1];
+    const float s04 = a.x + b.x, s15 = a.y + b.y, s26 = a.z + b.z, s37 = a.w + b.w;
     const float sum_sq = (s04 + s15) + (s26 + s37);
     return 1.0f / sqrtf(sum_sq / (float)D + eps);
 }
@@ -78,9 +102,7 @@ __device__ __forceinline__ void rms_quant_block(const float4 xv, const float4 gv
 {
     const float e[4] = {__fmul_rn(__fmul_rn(xv.x, rstd), gv.x), __fmul_rn(__fmul_rn(xv.y, rstd), gv.y),
                         __fmul_rn(__fmul_rn(xv.z, rstd), gv.z), __fmul_rn(__fmul_rn(xv.w, rstd), gv.w)};
-    float amax = fmaxf(fmaxf(fabsf(e[0]), fabsf(e[1])), fmaxf(fabsf(e[2]), fabsf(e[3])));
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+    const float amax = wave_max(fmaxf(fmaxf(fabsf(e[0]), fabsf(e[1])), fmaxf(fabsf(e[2]), fabsf(e[3]))));
     if (amax == 0.0f) {
         reinterpret_cast<u32 *>(out)[lane] = 0;
         if (lane < 9) reinterpret_cast<u32 *>(out)[64 + lane] = 0;
@@ -100,35 +122,34 @@ __device__ __forceinline__ void rms_quant_block(const float4 xv, const float4 gv
     if (lane == 0) *reinterpret_cast<float *>(out) = __fdiv_rn(1.0f, iscale);
 }
 
-/* One block of NW waves turns row x (D floats) into its D/256 Q8_K blocks at
- * y.  Wave w owns 256-blocks w, w + NW, ...; the gamma of its first GREG
- * blocks is loaded at the start and kept in registers across the chain, so a
- * single row costs one round trip to memory, not one per 256-block (x itself
- * comes back from LDS).  smem: D floats + 8. */
-template <int NW, int GREG>
+/* A block of nw waves turns row x (D floats) into its D/256 Q8_K blocks at y.  Wave w owns 256-blocks w, w + nw, ...;
+ * the x and gamma of its first GREG blocks are loaded at the start and kept in registers across the chain, so a row of
+ * up to GREG * nw blocks costs one round trip to memory.  smem: rms_lds_bytes(D). */
+template <int GREG>
 __device__ __forceinline__ void rms_row(const float *__restrict__ x, const float *__restrict__ gamma,
                                         uint8_t *__restrict__ y, int D, float eps, float *xs)
 {
-    const int tid = threadIdx.x, lane = tid & 63, wave = wave_in_block();
+    const int tid = threadIdx.x, lane = tid & 63, wave = wave_in_block(), nw = blockDim.x >> 6;
     const int nb = D / 256;
-    float4 gv[GREG];
+    float4 xv[GREG], gv[GREG];
 #pragma unroll
-    for (int r = 0; r < GREG; ++r) {
-        const int b = wave + NW * r;
-        gv[r] = reinterpret_cast<const float4 *>(gamma + 256 * (b < nb ? b : nb - 1))[lane];
-    }
-    for (int b = wave; b < nb; b += NW)
-        reinterpret_cast<float4 *>(xs + 256 * b)[lane] = reinterpret_cast<const float4 *>(x + 256 * b)[lane];
+    for (int r = 0; r < GREG; ++r) xv[r] = reinterpret_cast<const float4 *>(x + 256 * min(wave + nw * r, nb - 1))[lane];
+#pragma unroll
+    for (int r = 0; r < GREG; ++r) gv[r] = reinterpret_cast<const float4 *>(gamma + 256 * min(wave + nw * r, nb - 1))[lane];
+#pragma unroll
+    for (int r = 0; r < GREG; ++r)
+        if (wave + nw * r < nb) rms_stage(xs, D, wave + nw * r, lane, xv[r]);
+    for (int b = wave + nw * GREG; b < nb; b += nw) rms_stage(xs, D, b, lane, reinterpret_cast<const float4 *>(x + 256 * b)[lane]);
     __syncthreads();
     if (tid < 8) rms_chain(xs, D, tid);
     __syncthreads();
     const float rstd = rms_rstd(xs, D, eps);
 #pragma unroll
     for (int r = 0; r < GREG; ++r) {
-        const int b = wave + NW * r;
-        if (b < nb) rms_quant_block(reinterpret_cast<const float4 *>(xs + 256 * b)[lane], gv[r], rstd, lane, y + (size_t)b * 292);
+        const int b = wave + nw * r;
+        if (b < nb) rms_quant_block(xv[r], gv[r], rstd, lane, y + (size_t)b * 292);
     }
-    for (int b = wave + NW * GREG; b < nb; b += NW)
-        rms_quant_block(reinterpret_cast<const float4 *>(xs + 256 * b)[lane],
-                        reinterpret_cast<const float4 *>(gamma + 256 * b)[lane], rstd, lane, y + (size_t)b * 292);
+    for (int b = wave + nw * GREG; b < nb; b += nw)
+        rms_quant_block(reinterpret_cast<const float4 *>(x + 256 * b)[lane], reinterpret_cast<const float4 *>(gamma + 256 * b)[lane], rstd, lane,
+                        y + (size_t)b * 292);
 }

@@ -407,6 +407,30 @@ def test_rmsnorm_q8_k_fused_golden_host_and_device():
     assert np.array_equal(out, G["rms_out"])
 
 
+@pytest.mark.parametrize("tokens,D,stride", [(513, 256, 256), (513, 1024, 1028), (520, 4096, 4096), (513, 4352, 4352), (2, 4352, 4352),
+                                             (3, 8192, 8200), (512, 768, 768), (1, 40704, 40704)])
+def test_rmsnorm_q8_k_fused_launch_shapes_bit_exact(tokens, D, stride):
+    """Both sides of the token count that takes four waves a row, one to many 256-blocks a wave, rows that no wave count
+    divides, padded rows, the longest row that fits."""
+    x = T.normal(tokens * stride, 0.0, 3.0, 60 + D)
+    x.reshape(tokens, stride)[-1, :256] = 0.0
+    g = T.normal(D, 1.0, 0.3, 61 + D)
+    say("rmsnorm_q8_k_fused", tokens, D, stride)
+    ref = np.zeros(tokens * (D // 256) * 292, np.uint8)
+    T.oracle().orc_rmsnorm_q8_k_fused(T.ptr(x), T.ptr(g), T.ptr(ref), tokens, D, stride, ctypes.c_float(1e-6))
+    out = P.dev_rmsnorm_q8_k_fused(P.to_device(x), P.to_device(g), tokens, D, stride, 1e-6).cpu().numpy()
+    assert np.array_equal(out, ref)
+
+
+@pytest.mark.parametrize("where", [(0, 3), (3, 252), (17, 18), (62, 255), (31, 32), (0, 255)])
+def test_q8_k_scale_is_the_first_of_the_largest(where):
+    """Two elements of the largest magnitude and opposite signs: the scale's sign is the first one's, in whichever lanes they are."""
+    x = np.clip(T.normal(512, 0.0, 1.0, 71), -3.0, 3.0)
+    x[where[0]], x[where[1]] = -7.0, 7.0
+    x[256 + where[0]], x[256 + where[1]] = 7.0, -7.0
+    assert np.array_equal(P.dev_quantize(P.to_device(x), "q8_k").cpu().numpy(), T.oracle_quantize(x, "q8_k"))
+
+
 @pytest.mark.parametrize("tokens,D,std,seed", [(1, 256, 1.0, 1), (5, 4096, 1.0, 2), (64, 1024, 30.0, 3),
                                                 (3, 11008 // 256 * 256, 1e-3, 4), (512, 4096, 2.0, 5)])
 def test_rmsnorm_q8_k_fused_bit_exact_vs_oracle(tokens, D, std, seed):
