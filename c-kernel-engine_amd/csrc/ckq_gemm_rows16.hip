@@ -399,6 +399,190 @@ gemm_rows16_kernel(const uint8_t *W, const uint8_t *X, int N, Rows16Shape S, flo
     }
 }
 
+/* Short rows, several token groups: a block has a wave for every 256-block of its 16 rows (at most KEEP_NB of them) and goes
+ * through `per` groups of 16 tokens, the planes and scales of its weights formed once and kept in registers.  The kernel above
+ * forms them again for every group, and they are half of what bounds it there, VALU issue (counted at 2 x 4864 x 1024, Q5_K,
+ * 93 tokens: 587 operations a wave for a 256-block and group, 78 % of the busy cycles; 21 us, here 15).  The terms and their order are
+ * the same. */
+constexpr int KEEP_NB = 8;
+template <class F> constexpr int rows16_keep_wave_lds() { return 16 * (F::PITCH > 288 ? F::PITCH : 288); }
+template <class F, bool TREE, bool GRP>
+__global__ void __launch_bounds__(64 * KEEP_NB)
+gemm_rows16_keep_kernel(const uint8_t *W, const uint8_t *X, int N, int M, int parts, int per, float *y, const float *bias, long ldy, GemmChains ch, Rows16Args grp)
+{
+    constexpr int NT = 16;
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const int tid = threadIdx.x, nthr = blockDim.x, nb = nthr >> 6;
+    const int lane = tid & 63, wave = wave_in_block();
+    const int i16 = lane & 15, q = lane >> 4;
+    /* the `parts` blocks of a row tile follow one another on one XCD: blocks are dealt to the eight in turn */
+    const int each = gridDim.x >> 3, odd = gridDim.x & 7, xcd = blockIdx.x & 7;
+    const int id = xcd * each + min(xcd, odd) + (int)(blockIdx.x >> 3);
+    int tile = id / parts;
+    const int g0 = (id - tile * parts) * per, g1 = min(g0 + per, (M + NT - 1) / NT);
+    if constexpr (GRP) {
+        if (tile >= grp.p[1].id0) {
+            Rows16Problem p = grp.p[1];
+            if (grp.n > 2 && tile >= grp.p[2].id0) p = grp.p[2];
+            if (grp.n > 3 && tile >= grp.p[3].id0) p = grp.p[3];
+            W = p.W; X = p.X; N = p.N; y = p.y; bias = p.bias; ldy = p.ldy; ch = p.ch;
+            tile -= p.id0;
+        }
+    }
+    const int n0 = tile * 16;
+    const u32 xrow = (u32)nb * 292u, wpitch = (u32)nb * (u32)F::WBLOCK;
+    uint8_t *const al = smem + wave * rows16_keep_wave_lds<F>(), *const bl = al + NT * 256;   /* the weights first, then each group's quants and bsums */
+    float *const us = reinterpret_cast<float *>(smem + nb * rows16_keep_wave_lds<F>());       /* two groups' terms: one written while the other is read */
+    float *const dxs = us + 2 * nb * (NT * 16);
+    const uint8_t *const wbase = W + (size_t)n0 * wpitch + (u32)wave * (u32)F::WBLOCK;
+    const uint8_t *xbase = X + (size_t)(g0 * NT) * xrow + (u32)wave * 292u;
+
+    /* copy roles as in gemm_rows16_kernel; lanes 0..15 fetch the tokens' scales */
+    constexpr int NWL = (16 * F::CHUNKS + 63) / 64, NAL = (NT * 18 + 63) / 64;
+    u32 asrc[NAL], adst[NAL], dsrc = 0;
+    auto token_offsets = [&](int last) {
+#pragma unroll
+        for (int j = 0; j < NAL; ++j) {
+            const int e = min(64 * j + lane, NT * 18 - 1);
+            asrc[j] = (u32)min(e / 18, last) * xrow + 4u + 16u * (u32)(e % 18);
+        }
+        dsrc = (u32)min(i16, last) * xrow;
+    };
+#pragma unroll
+    for (int j = 0; j < NAL; ++j) {
+        const int e = min(64 * j + lane, NT * 18 - 1), t = e / 18, c = e % 18;
+        adst[j] = (u32)(c < 16 ? 256 * t + 16 * (c ^ (t & 15)) : NT * 256 + 32 * t + 16 * (c - 16));
+    }
+    token_offsets(min(NT, M - g0 * NT) - 1);
+    ckq_v4i wr[NWL], ar[NAL];
+    float dr;
+    auto fetch = [&]() {
+#pragma unroll
+        for (int j = 0; j < NAL; ++j) {
+            u32 t[4];
+            ld16<4>(t, xbase + asrc[j]);
+            ar[j] = ckq_v4i{(int)t[0], (int)t[1], (int)t[2], (int)t[3]};
+        }
+        dr = __builtin_bit_cast(float, ld4<4>(xbase + dsrc));
+    };
+    u32 wdst[NWL];
+#pragma unroll
+    for (int j = 0; j < NWL; ++j) {
+        const int e = min(64 * j + lane, 16 * F::CHUNKS - 1), r = e / F::CHUNKS, c = e % F::CHUNKS;
+        u32 t[4];
+        ld16<F::WBLOCK % 4 == 0 ? 4 : 2>(t, wbase + ((u32)min(r, N - 1 - n0) * wpitch + F::chunk_ofs(c)));
+        wr[j] = ckq_v4i{(int)t[0], (int)t[1], (int)t[2], (int)t[3]};
+        wdst[j] = (u32)(r * F::PITCH + 16 * c);
+    }
+    fetch();
+#pragma unroll
+    for (int j = 0; j < NWL; ++j) *reinterpret_cast<ckq_v4i *>(al + wdst[j]) = wr[j];
+    __builtin_amdgcn_wave_barrier();
+    Head hd;
+    ckq_v4i ph[4], pl[4];
+    const uint8_t *const wrow = al + i16 * F::PITCH;
+    F::head(hd, wrow, q);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) F::planes(ph[g], pl[g], hd, wrow, g, q);
+    __builtin_amdgcn_wave_barrier();                  /* the wave's own LDS accesses stay in this order */
+
+    const ckq_v4i zero = {0, 0, 0, 0};
+    for (int gr = g0, p = 0; gr < g1; ++gr, p ^= 1) {
+        float *const u = us + p * nb * (NT * 16), *const dx = dxs + p * nb * NT;
+#pragma unroll
+        for (int j = 0; j < NAL; ++j) *reinterpret_cast<ckq_v4i *>(al + adst[j]) = ar[j];
+        if (lane < NT) dx[wave * NT + lane] = dr;
+        if (gr + 1 < g1) {
+            xbase += (size_t)NT * xrow;
+            if ((gr + 2) * NT > M) token_offsets(M - 1 - (gr + 1) * NT);
+            fetch();
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_wave_barrier();
+        ckq_v4f i2s = {0.0f, 0.0f, 0.0f, 0.0f};
+        ckq_v4i am = zero;
+        if constexpr (F::MIN) {
+            const int2 bs = *reinterpret_cast<const int2 *>(bl + 32 * i16 + 8 * q);
+            const int p0 = (int)(int16_t)(bs.x & 0xffff) + (bs.x >> 16), p1 = (int)(int16_t)(bs.y & 0xffff) + (bs.y >> 16);
+            am = ckq_v4i{(int)bf16_pair((float)(p0 & 63), (float)(p1 & 63)), (int)bf16_pair((float)(64 * (p0 >> 6)), (float)(64 * (p1 >> 6))), 0, 0};
+        }
+        auto min_mfma = [&](const ckq_v4i &mins) {
+            const ckq_v4f z = {0.0f, 0.0f, 0.0f, 0.0f};
+            return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(ckq_v8bf, am), __builtin_bit_cast(ckq_v8bf, mins), z, 0, 0, 0);
+        };
+        float out[4];
+        if constexpr (TREE) {
+            const ckq_v4i dxi = lds16(reinterpret_cast<const uint8_t *>(dx + wave * NT + 4 * q));
+            float t[4][4];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const ckq_v4i a = lds16(al + 256 * i16 + 16 * ((int)(F::a_elem(g, q) >> 4) ^ i16));
+                const ckq_v4i sh = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, ph[g], zero, 0, 0, 0);
+                const ckq_v4i sl = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, pl[g], zero, 0, 0, 0);
+                if constexpr (F::MIN) i2s = min_mfma(q == g ? hd.mins : zero);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int di = dxi[r];
+                    const float d = __builtin_bit_cast(float, di), f = (float)((sh[r] << F::SHIFT) + sl[r]);
+                    float v;
+                    if constexpr (F::MIN) v = (hd.dw * d) * f - (hd.dmin * d) * i2s[r];
+                    else                  v = (hd.dw * d) * f;
+                    asm volatile("" : "+v"(v));              /* rounded before it is added, as in the streaming kernel */
+                    t[g][r] = 0.0f + v;
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) out[r] = (t[0][r] + t[1][r]) + (t[2][r] + t[3][r]);
+        } else {
+            ckq_v4i sh, sl;
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const ckq_v4i a = lds16(al + 256 * i16 + 16 * ((int)(F::a_elem(g, q) >> 4) ^ i16));
+                sh = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, ph[g], g ? sh : zero, 0, 0, 0);
+                sl = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, pl[g], g ? sl : zero, 0, 0, 0);
+            }
+            if constexpr (F::MIN) i2s = min_mfma(hd.mins);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float f = (float)((sh[r] << F::SHIFT) + sl[r]);
+                out[r] = F::MIN ? hd.dw * f - hd.dmin * i2s[r] : hd.dw * f;
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) u[wave * (NT * 16) + 64 * r + lane] = out[r];
+        /* one barrier a group: the terms of the group after next overwrite these, behind the next group's barrier */
+        __syncthreads();
+        for (int e = tid; e < NT * 16; e += nthr) {
+            const int tok = 4 * ((e & 63) >> 4) + (e >> 6), n = n0 + (e & 15), t = gr * NT + tok;
+            float v = 0.0f;
+            if constexpr (TREE) {
+                float w[KEEP_NB];
+#pragma unroll
+                for (int b = 0; b < KEEP_NB; ++b) w[b] = b < nb ? u[b * (NT * 16) + e] : 0.0f;
+#pragma unroll
+                for (int k = 1; k < KEEP_NB; k *= 2)
+#pragma unroll
+                    for (int b = 0; b < KEEP_NB; b += 2 * k) w[b] += w[b + k];
+                v = w[0] + 0.0f;                      /* the other half of the tree, empty */
+            } else {
+                for (int sp = 0; sp < ch.splits; ++sp) {
+                    const int b0 = sp * ch.per, b1 = min(nb, b0 + ch.per);
+                    float c[2] = {0.0f, 0.0f};
+                    for (int b = b0; b < b1; ++b) {
+                        const int k = ch.kg == 2 ? (b - b0) & 1 : 0;
+                        const float uu = u[b * (NT * 16) + e], dd = dx[b * NT + tok];
+                        if (k) c[1] = fmaf(dd, uu, c[1]);
+                        else   c[0] = fmaf(dd, uu, c[0]);
+                    }
+                    if (ch.kg == 2) c[0] += c[1];
+                    v = sp ? v + c[0] : c[0];
+                }
+            }
+            if (n < N && t < M) y[(size_t)t * ldy + n] = bias ? v + bias[n] : v;
+        }
+    }
+}
+
 /* Waves per block: with two tiles per CU and more, blocks of four waves overlap each other's beginnings and ends
  * (32000 x 4096, 13 tokens: 27 us, with eight 41); with fewer, a tile's blocks spread over more waves. */
 int rows16_waves(int tiles, int nb)
@@ -446,21 +630,77 @@ int launch_rows16_nt(Rows16Args &a, hipStream_t s)
     return (int)hipGetLastError();
 }
 
-template <class F>
-int launch_rows16(Rows16Args &a, hipStream_t s)
+/* Blocks per row tile of the kernel that keeps its planes, 0: the other kernel; its time in us.  Both times are fitted to launches
+ * of 1024 x 1024 to 12000 x 2048, 17 to 256 tokens, one to eight blocks a row tile, mostly within 15 %: here 2.5 (Q4_K 3) +
+ * (groups of a block + 1.5) (0.45 + 0.27 waves a SIMD of the fullest CU + 0.25 (4 / nb - 1) where nb < 4), there 3.2 + 0.15 nb +
+ * (a nb + b) thousands of tiles.  Against the other kernel (us): Q5_K 4864 x 1024 at 64 / 96 / 128 tokens 8.3 -> 6.5,
+ * 10.8 -> 7.9, 10.9 -> 8.6, 12000 x 1024 at 32 / 96 9.8 -> 6.8, 19.0 -> 11.6, 4096 x 2048 at 96 12.0 -> 9.1; Q6_K 11008 x 2048
+ * at 64 22.0 -> 16.4; Q4_K, whose planes are quickly formed, 12000 x 1024 at 64 11.1 -> 8.7.  It loses where the other's waves
+ * have a SIMD to themselves anyway (Q4_K 1782 x 1536 at 43: 5.1 against 7.0) and for Q4_K rows of five blocks and more (11008 x 2048
+ * at 32: 9.6 against 10.3).  Over 260 random shapes of 9 to 400 tokens, all routes: 1.036 on the geometric mean, the largest loss
+ * 5.1 -> 6.1 (Q5_K 1172 x 768 at 208), the largest gain 12.0 -> 6.5 (Q6_K 3293 x 256 at 278). */
+int rows16_keep_parts(int fmt, long tiles, int groups, int nb, float *time)
 {
+    if (nb > (fmt == CKQ_FMT_Q4_K ? 4 : KEEP_NB) || groups < 2 || tiles > 1 << 20 || groups > 1 << 10) return 0;
+    int best = 0;
+    float least = 0.0f;
+    for (int parts = 1; parts <= groups / 2 + 1; ++parts) {
+        const int per = (groups + parts - 1) / parts;
+        if (per < 2) break;
+        const float waves = 0.25f * (float)((tiles * parts + 255) / 256) * (float)nb;
+        const float t = (fmt == CKQ_FMT_Q4_K ? 3.0f : 2.5f) + (1.5f + (float)per) * (0.45f + 0.27f * waves + (nb < 4 ? 1.0f / (float)nb - 0.25f : 0.0f));
+        if (!best || t <= least) { least = t; best = (groups + per - 1) / per; }
+    }
+    const float a = fmt == CKQ_FMT_Q4_K ? 0.29f : fmt == CKQ_FMT_Q5_K ? 0.36f : 0.59f, b = fmt == CKQ_FMT_Q4_K ? 1.6f : fmt == CKQ_FMT_Q5_K ? 2.1f : 1.1f;
+    if (least >= 3.2f + 0.15f * (float)nb + 1e-3f * (a * (float)nb + b) * (float)(tiles * groups)) return 0;
+    if (time) *time = least;
+    return best;
+}
+
+template <class F, bool TREE>
+int launch_rows16_keep(Rows16Args &a, int parts, hipStream_t s)
+{
+    int tiles = 0;
+    for (int i = 0; i < a.n; ++i) {
+        a.p[i].id0 = tiles;
+        tiles += (a.p[i].N + 15) / 16;
+    }
+    const int groups = (a.M + 15) / 16, per = (groups + parts - 1) / parts;
+    const size_t lds = (size_t)a.nb * (rows16_keep_wave_lds<F>() + 2 * 1024 + 2 * 64);
+    const Rows16Problem &p = a.p[0];
+    const dim3 grid((unsigned)(tiles * parts)), block((unsigned)(64 * a.nb));
+    if (a.n > 1)
+        hipLaunchKernelGGL((gemm_rows16_keep_kernel<F, TREE, true>), grid, block, lds, s, p.W, p.X, p.N, a.M, parts, per, p.y, p.bias, p.ldy, p.ch, a);
+    else
+        hipLaunchKernelGGL((gemm_rows16_keep_kernel<F, TREE, false>), grid, block, lds, s, p.W, p.X, p.N, a.M, parts, per, p.y, p.bias, p.ldy, p.ch, a);
+    return (int)hipGetLastError();
+}
+
+template <class F>
+int launch_rows16(int fmt, Rows16Args &a, hipStream_t s)
+{
+    long tiles = 0;
+    for (int i = 0; i < a.n; ++i) tiles += (a.p[i].N + 15) / 16;
+    const int parts = rows16_keep_parts(fmt, tiles, (a.M + 15) / 16, a.nb, nullptr);
+    if (parts) return a.tree ? launch_rows16_keep<F, true>(a, parts, s) : launch_rows16_keep<F, false>(a, parts, s);
     if (a.tree) return a.M <= 8 ? launch_rows16_nt<F, 8, true>(a, s) : launch_rows16_nt<F, 16, true>(a, s);
     return a.M <= 8 ? launch_rows16_nt<F, 8, false>(a, s) : launch_rows16_nt<F, 16, false>(a, s);
 }
 
 } // namespace
 
+float gemm_rows16_keep_time(int fmt, size_t rows, int ntok, int nb)
+{
+    float t = 0.0f;
+    return rows16_keep_parts(fmt, (long)((rows + 15) / 16), (ntok + 15) / 16, nb, &t) ? t : 0.0f;
+}
+
 int launch_gemm_rows16(int fmt, Rows16Args &a, hipStream_t s)
 {
     switch (fmt) {
-    case CKQ_FMT_Q4_K: return launch_rows16<R16Q4K>(a, s);
-    case CKQ_FMT_Q5_K: return launch_rows16<R16Q5K>(a, s);
-    case CKQ_FMT_Q6_K: return launch_rows16<R16Q6K>(a, s);
+    case CKQ_FMT_Q4_K: return launch_rows16<R16Q4K>(fmt, a, s);
+    case CKQ_FMT_Q5_K: return launch_rows16<R16Q5K>(fmt, a, s);
+    case CKQ_FMT_Q6_K: return launch_rows16<R16Q6K>(fmt, a, s);
     default: return CKQ_EFORMAT;
     }
 }

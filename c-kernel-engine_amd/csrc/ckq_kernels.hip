@@ -264,7 +264,8 @@ static bool weights_dword_aligned(const GemvArgs &a, const GemvGroup &grp)
  * either way, so only time decides.  Fitted to launches of all three over 128..32000 rows, widths of 1024..11008 and 5..128
  * tokens (us; nb: 256-blocks of a row, mb: megabytes of weights, n16: thousands of 256-blocks of 16 rows times groups of 16
  * tokens); over all of them the rule's choices are within 1 % of always taking the faster:
- *   rows16     3.6 + 0.12 nb + (Q4_K 0.36, Q5_K 0.65, Q6_K 0.71) n16
+ *   rows16     3.6 + 0.12 nb + (Q4_K 0.36, Q5_K 0.65, Q6_K 0.71) n16; up to 256 tokens of short rows gemm_rows16_keep_time
+ *              (Q5_K 4864 x 1024 at 192 tokens: 10.3, tiles 13.7; 4096 x 2048 at 256: 17.2, tiles 19.5)
  *   tiles      11 + 0.2 mb + 0.0015 tokens mb, an under-estimate almost everywhere
  *   streaming  the larger of 4.35 + 0.07 nb and 3.05 + 0.11 nb + (0.24, 0.245, 0.29) mb for every eight tokens, 5 to 8 as 10
  * Three and four tokens, one pass of half the width, only move for long rows of large matrices (4096 x 11008 Q6_K:
@@ -288,7 +289,8 @@ static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles)
     const float nb = (float)(K / 256), mb = (float)rows * nb * (f == 0 ? 144e-6f : f == 1 ? 176e-6f : 210e-6f);
     if (ntok <= 4) return K > 4096 && mb >= 20.0f;
     const float passes = ntok <= 8 ? 1.25f : (float)((ntok + 7) / 8);
-    const float t_rows = 3.6f + 0.12f * nb + per_block[f] * 1e-3f * nb * (float)((rows + 15) / 16) * (float)((ntok + 15) / 16);
+    const float t_keep = ntok <= 256 ? gemm_rows16_keep_time(fmt, rows, ntok, K / 256) : 0.0f;
+    const float t_rows = t_keep > 0.0f ? t_keep : 3.6f + 0.12f * nb + per_block[f] * 1e-3f * nb * (float)((rows + 15) / 16) * (float)((ntok + 15) / 16);
     const float t_stream = 3.05f + 0.11f * nb + per_pass[f] * mb * passes, t_least = 4.35f + 0.07f * nb;
     const float t_else = tiles ? 11.0f + (0.2f + 0.0015f * (float)ntok) * mb : t_stream > t_least ? t_stream : t_least;
     return t_rows < t_else;

@@ -1314,6 +1314,47 @@ def test_16_row_tiles_vs_oracle_and_the_kernels_they_stand_in_for(fmt):
         L.ckq_set_prefill_variant(tag, 0)
 
 
+@pytest.mark.parametrize("fmt", ["q4_k", "q5_k", "q6_k"])
+def test_16_row_tiles_of_short_rows_and_several_token_groups(fmt):
+    """The kernel that keeps the planes of its weights across token groups: one to eight K-blocks (waves), two groups and many,
+    groups dealt evenly to a row tile's blocks and not, the last rows and tokens of the matrix.  In the order of the streaming
+    kernel (policy 2) and of the tile kernels (1), bit for bit; and several matrices in one launch."""
+    import torch
+    L = ckq.lib()
+    tag = P.FMT[fmt]
+    try:
+        for M, N, K in [(93, 9729, 1024), (70, 12001, 256), (17, 33, 2048), (33, 16, 1792), (21, 20011, 768), (500, 100, 1280)]:
+            xq = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, seed=M)), "q8_k", rows=M)
+            W, bias = P.to_device(T.random_blocks(fmt, N * K // 256, 9400 + M)), P.to_device(T.normal(N, 0.0, 0.5, seed=N))
+            say("16-row tiles, several token groups", fmt, M, N, K)
+            L.ckq_set_prefill_variant(tag, 16)
+            L.ckq_set_gemm_policy(2)
+            tree = P.dev_gemm_nt(fmt, xq, W, bias, M, N, K).clone().view(M, N)
+            L.ckq_set_gemm_policy(1)
+            chain = P.dev_gemm_nt(fmt, xq, W, bias, M, N, K).clone()
+            L.ckq_set_prefill_variant(tag, 0)
+            assert torch.equal(chain, P.dev_gemm_nt(fmt, xq, W, bias, M, N, K)), (M, N, K)
+            L.ckq_set_gemm_policy(0)
+            rb = xq.numel() // M
+            for m in range(0, M, max(1, M // 12)):
+                one = P.dev_gemm_nt(fmt, xq[m * rb:(m + 1) * rb].clone(), W, bias, 1, N, K)
+                assert torch.equal(tree[m], one.view(N)), (M, N, K, m)
+        M, K, Ns = 77, 1024, [9000, 33, 4861, 250]
+        xq = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, seed=4)), "q8_k", rows=M)
+        Ws = [P.to_device(T.random_blocks(fmt, n * K // 256, 9500 + i)) for i, n in enumerate(Ns)]
+        for policy in (1, 0):
+            L.ckq_set_prefill_variant(tag, 16)
+            L.ckq_set_gemm_policy(policy)
+            ys = [torch.zeros(M, n, dtype=torch.float32, device="cuda") for n in Ns]
+            say("16-row tiles, several token groups, grouped", fmt, policy)
+            P.dev_matmul_sequence([(fmt, xq, W, None, y, M, n, K) for W, y, n in zip(Ws, ys, Ns)])
+            for W, y, n in zip(Ws, ys, Ns):
+                assert torch.allclose(y, P.dev_gemm_nt(fmt, xq, W, None, M, n, K).view(M, n), rtol=0, atol=2e-6 * float(y.abs().max())), (policy, n)
+    finally:
+        L.ckq_set_gemm_policy(0)
+        L.ckq_set_prefill_variant(tag, 0)
+
+
 @pytest.mark.parametrize("blocks", [1, 2, 3, 4, 5, 6, 7, 8, 13, 37, 64])
 def test_gemm_mfma_q8_0_row_alignment_and_k_remainders(blocks):
     """Rows of odd and even numbers of 32-blocks (odd ones start on dwords every other row), K ending after one, two, three
