@@ -315,6 +315,20 @@ static int launch_mt(const GemvArgs &a, const GemvGroup &grp, int max_mt, hipStr
         return launch_tile<F, LPR, PPL, 1, 1, 4>(a, grp, s);
     }
     if constexpr (F::TOKEN_TILES) {
+        /* Two rows per slot serve the staged tokens twice, but leave CUs without a block where the matrix is small: then one row
+         * per slot, and smaller token tiles while that too leaves some.  Measured (us; 2, 4 and 7 tokens): Q5_K 1024 x 4864
+         * 3.9 -> 3.2, 5.2 -> 3.9, 7.5 -> 5.2; 4096 x 1024 at 4 and 7 3.5 -> 2.8, 4.5 -> 3.3; Q6_K 1024 x 11008 at 2 and 4 6.5 -> 5.2,
+         * 9.0 -> 7.3; Q4_K 2048 x 2048 at 7 4.5 -> 3.2; 12000 x 1024 at 4 4.4 -> 4.1, Q8_0 at 7 6.7 -> 5.8.  Rows that take a wave
+         * each lose from 256 blocks of two rows per slot on (2048 x 8192, Q6_K at 4: 7.4 -> 8.2), shorter ones from 512. */
+        constexpr long few = LPR < 64 ? 512 : 256;
+        const long slots = ((long)launch_rows(a, grp) * LPR + 255) / 256 * (long)grp.n;      /* blocks of one row per slot and a token tile */
+        if (slots < 2 * few) {
+            int mt = a.ntok == 2 ? 2 : a.ntok <= 4 ? 4 : 8;
+            while (mt > 2 && slots * ((a.ntok + mt - 1) / mt) <= 256) mt /= 2;
+            if (mt == 2) return launch_tile<F, LPR, PPL, 2, 1, 4>(a, grp, s);
+            if (mt == 4) return launch_tile<F, LPR, PPL, 4, 1, 4>(a, grp, s);
+            return launch_tile<F, LPR, PPL, 8, 1, 4>(a, grp, s);
+        }
         if (a.ntok == 2) return launch_tile<F, LPR, PPL, 2, 2, 4>(a, grp, s);
         if (a.ntok <= 4) return launch_tile<F, LPR, PPL, 4, 2, 4>(a, grp, s);
         return launch_tile<F, LPR, PPL, 8, 2, 4>(a, grp, s);   /* two rows per slot: the staged tile serves twice the weights */

@@ -1314,6 +1314,30 @@ def test_16_row_tiles_vs_oracle_and_the_kernels_they_stand_in_for(fmt):
         L.ckq_set_prefill_variant(tag, 0)
 
 
+@pytest.mark.parametrize("fmt", ["q4_k", "q5_k", "q6_k", "q8_0", "q5_0"])
+@pytest.mark.parametrize("N,K", [(7, 256), (250, 1024), (16383, 512), (16385, 512), (1023, 4864), (1025, 4864), (2047, 4096), (2049, 4096), (300, 11008)])
+def test_streamed_tokens_have_the_bits_of_single_ones(fmt, N, K):
+    """Token tiles of the streaming kernel on both sides of the row counts that take one or two rows per slot and smaller token
+    tiles: every token's outputs are those of a call with that token alone - of the K-quants bit for bit, of Q8_0 and Q5_0, whose
+    scaling the compiler may contract into a multiply-add or not per instantiation, but for one rounding a block."""
+    import torch
+    L = ckq.lib()
+    W, bias = P.to_device(T.random_blocks(fmt, N * K // ckq.api.BLOCK_ELEMS[fmt], 9700 + N % 97)), P.to_device(T.normal(N, 0.0, 0.5, seed=N))
+    try:
+        L.ckq_set_gemm_policy(2)
+        for M in (2, 3, 4, 5, 8):
+            xq = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, seed=M)), P.act_format(fmt), rows=M)
+            rb = xq.numel() // M
+            say("streamed tokens", fmt, M, N, K)
+            y = P.dev_gemm_nt(fmt, xq, W, bias, M, N, K).view(M, N)
+            for m in range(M):
+                one = P.dev_gemm_nt(fmt, xq[m * rb:(m + 1) * rb].clone(), W, bias, 1, N, K).view(N)
+                same = torch.equal(y[m], one) if fmt[-1] == "k" else torch.allclose(y[m], one, rtol=0, atol=2e-6 * float(one.abs().max()))
+                assert same, (M, m)
+    finally:
+        L.ckq_set_gemm_policy(0)
+
+
 @pytest.mark.parametrize("fmt", ["q4_k", "q5_k", "q6_k"])
 def test_16_row_tiles_of_short_rows_and_several_token_groups(fmt):
     """The kernel that keeps the planes of its weights across token groups: one to eight K-blocks (waves), two groups and many,
