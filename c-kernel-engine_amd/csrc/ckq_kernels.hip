@@ -267,7 +267,8 @@ static bool weights_dword_aligned(const GemvArgs &a, const GemvGroup &grp)
  *   rows16     3.6 + 0.12 nb + (Q4_K 0.36, Q5_K 0.65, Q6_K 0.71) n16; up to 256 tokens of short rows gemm_rows16_keep_time
  *              (Q5_K 4864 x 1024 at 192 tokens: 10.3, tiles 13.7; 4096 x 2048 at 256: 17.2, tiles 19.5)
  *   tiles      11 + 0.2 mb + 0.0015 tokens mb, an under-estimate almost everywhere
- *   streaming  the larger of 4.35 + 0.07 nb and 3.05 + 0.11 nb + (0.24, 0.245, 0.29) mb for every eight tokens, 5 to 8 as 10
+ *   streaming  the larger of 4.35 + 0.07 nb (to eight tokens 3.5, where smaller tiles fill the chip: Q5_K 1024 x 2048 at 5
+ *              4.5 -> 3.7 us, Q4_K 1024 x 1024 3.9 -> 3.6) and 3.05 + 0.11 nb + (0.24, 0.245, 0.29) mb for every eight tokens, 5 to 8 as 10
  * Three and four tokens, one pass of half the width, only move for long rows of large matrices (4096 x 11008 Q6_K:
  * 17.0 -> 13.4); two never do.  The forced policies keep their kernels: 1 the tile kernels, and 2 the streaming kernels,
  * whose order this one keeps where `tiles` is false. */
@@ -291,7 +292,7 @@ static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles)
     const float passes = ntok <= 8 ? 1.25f : (float)((ntok + 7) / 8);
     const float t_keep = ntok <= 256 ? gemm_rows16_keep_time(fmt, rows, ntok, K / 256) : 0.0f;
     const float t_rows = t_keep > 0.0f ? t_keep : 3.6f + 0.12f * nb + per_block[f] * 1e-3f * nb * (float)((rows + 15) / 16) * (float)((ntok + 15) / 16);
-    const float t_stream = 3.05f + 0.11f * nb + per_pass[f] * mb * passes, t_least = 4.35f + 0.07f * nb;
+    const float t_stream = 3.05f + 0.11f * nb + per_pass[f] * mb * passes, t_least = (ntok <= 8 ? 3.5f : 4.35f) + 0.07f * nb;
     const float t_else = tiles ? 11.0f + (0.2f + 0.0015f * (float)ntok) * mb : t_stream > t_least ? t_stream : t_least;
     return t_rows < t_else;
 }
