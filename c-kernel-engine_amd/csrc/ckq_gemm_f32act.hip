@@ -7,9 +7,11 @@
  * loops of gemm_nt_q4_k / _q6_k / _q8_0).
  *
  * Exactness.  The integers q (4 to 8 bits) are exact in bf16.  An fp32 activation is cut into three bf16 parts,
- * x = hi + mid + lo, each the leading 8 bits of what is left: 24 bits, so the cut is exact.  Every product of an
- * integer and a part fits fp32, the matrix core adds in fp32, and the scale is applied to the sum of a group in
- * fp32: the only roundings are those of fp32 additions, one per group and one per product as before.
+ * x = hi + mid + lo, each the leading 8 bits of what is left: 24 bits, so the cut is exact (of x 2^24, so that the parts of the
+ * smallest numbers are normal too; the scales carry the 2^-24).  Every product of an integer and a part fits fp32, the matrix
+ * core adds in fp32, and the scale is applied to the sum of a group in fp32: the only roundings are those of fp32 additions.
+ * Results that are not finite - an activation is not, or is beyond 2^90 or so - are summed again term by term (exact_output),
+ * as the kernel for one token forms them.
  *
  * Mapping.  v_mfma_f32_32x32x16_bf16, tokens as rows (A), weight rows as columns (B): a lane holds ONE weight row,
  * so its scale is a register of the lane and one multiply-add per output and group applies it.  A lane (column
@@ -34,18 +36,16 @@
 namespace {
 
 constexpr int F32_WAVES = 8;
+constexpr float X_UP = 16777216.0f, X_DOWN = 1.0f / 16777216.0f;      /* factors of the activations and of the scales */
 
 __device__ __forceinline__ u32 pack_bf16(float lo, float hi)      /* two floats whose low 16 bits are to be dropped */
 {
     return __builtin_amdgcn_perm(__builtin_bit_cast(u32, hi), __builtin_bit_cast(u32, lo), 0x07060302u);
 }
 
-/* eight floats -> their three bf16 parts as MFMA operands */
+/* eight floats -> their three bf16 parts as MFMA operands (of an infinity or a NaN: NaNs) */
 struct Cut { ckq_v4i hi, mid, lo; };
 __device__ __forceinline__ float top16(float v) { return __builtin_bit_cast(float, __builtin_bit_cast(u32, v) & 0xffff0000u); }
-/* The lower parts are taken from v clamped to the finite range: of an infinity only the first part matters, and it
- * must not meet the NaN that inf - inf would leave in the others. */
-__device__ __forceinline__ float finite(float v) { return __builtin_amdgcn_fmed3f(v, -3.402823466e38f, 3.402823466e38f); }
 __device__ __forceinline__ void cut8(const float *x, Cut &c)
 {
 #pragma unroll
@@ -53,7 +53,7 @@ __device__ __forceinline__ void cut8(const float *x, Cut &c)
         float m[2], l[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            const float v = finite(x[2 * i + j]);
+            const float v = x[2 * i + j];
             m[j] = v - top16(v);
             l[j] = m[j] - top16(m[j]);
         }
@@ -99,7 +99,8 @@ __device__ __forceinline__ ckq_v4i bytes_to_bf16(u32 b0, u32 b1)
  *   src_elem(c)     first element of 16-byte chunk c (0..15) of the step's activations
  *   chunk(g, h, i)  which chunk holds floats 4 i .. 4 i + 3 of group g for lane half h
  *   operand(g, i)   bf16x8 of the lane's elements 8 i .. 8 i + 7 of group g
- *   scale(g)        fp32 factor of the group; MIN: min_operand / dmin for the min term */
+ *   scale(g)        fp32 factor of the group; MIN: min_operand / dmin for the min term
+ *   weight(blk, e, i)  element e + i of a block, e a multiple of 16 and i below 16, for exact_output */
 struct F32Q4K {
     static constexpr int STEP = 64, NG = 2, NK = 2;
     static constexpr bool MIN = true;
@@ -118,10 +119,10 @@ struct F32Q4K {
     {
         u32 sc2, mn2;
         k4_scale_pair(w.hdr[1], w.hdr[2], w.hdr[3], step & 3, &sc2, &mn2);
-        const float dd = h2f(w.hdr[0] & 0xffff);
+        const float dd = h2f(w.hdr[0] & 0xffff) * X_DOWN;
         d.s[0] = dd * (float)(sc2 & 0xff);
         d.s[1] = dd * (float)((sc2 >> 8) & 0xff);
-        d.dmin = h2f(w.hdr[0] >> 16);
+        d.dmin = h2f(w.hdr[0] >> 16) * X_DOWN;
         const float m0 = (float)(mn2 & 0xff), m1 = (float)((mn2 >> 8) & 0xff);
         d.mins = ckq_v4i{(int)pack_bf16(m0, m0), (int)pack_bf16(m0, m1), (int)pack_bf16(m1, m1), 0};
     }
@@ -129,6 +130,16 @@ struct F32Q4K {
     {
         const u32 a = g ? w.qs[2 * i] >> 4 : w.qs[2 * i], b = g ? w.qs[2 * i + 1] >> 4 : w.qs[2 * i + 1];
         return bytes_to_bf16(a & 0x0f0f0f0fu, b & 0x0f0f0f0fu);
+    }
+    static constexpr int BLOCK = 256, WBLOCK = 144;
+    static __device__ __forceinline__ float weight(const uint8_t *blk, int e, int i)
+    {
+        u32 sc2, mn2;
+        k4_scale_pair(ld4<4>(blk + 4), ld4<4>(blk + 8), ld4<4>(blk + 12), e >> 6, &sc2, &mn2);
+        const int odd = (e >> 5) & 1;
+        const float s = h2f(ld2(blk)) * (float)((sc2 >> (8 * odd)) & 0xff), m = h2f(ld2(blk + 2)) * (float)((mn2 >> (8 * odd)) & 0xff);
+        const u32 b = blk[16 + 32 * (e >> 6) + (e & 31) + i];
+        return s * (float)(odd ? b >> 4 : b & 15u) - m;
     }
 };
 
@@ -155,7 +166,7 @@ struct F32Q6K {
     struct Dec { float s[4]; };
     static __device__ __forceinline__ void decode(Dec &d, const Raw &w, int step)
     {
-        const float dd = h2f(w.d);
+        const float dd = h2f(w.d) * X_DOWN;
         const int o = step & 1;
         d.s[0] = dd * (float)sbyte(w.sc[0], o);
         d.s[1] = dd * (float)sbyte(w.sc[0], o + 2);
@@ -174,6 +185,14 @@ struct F32Q6K {
             q[j] = ((v | 0x80808080u) - 0x20202020u) ^ 0x80808080u;      /* no borrows between bytes */
         }
         return bytes_to_bf16(q[0], q[1]);
+    }
+    static constexpr int BLOCK = 256, WBLOCK = 210;
+    static __device__ __forceinline__ float weight(const uint8_t *blk, int e, int i)
+    {
+        const int n = e >> 7, r = (e >> 5) & 3, l = (e & 31) + i;
+        const u32 lo = blk[64 * n + 32 * (r & 1) + l], hi = blk[128 + 32 * n + l];
+        const int q = (int)(((r >> 1) ? lo >> 4 : lo & 15u) | ((hi >> (2 * r)) & 3u) << 4) - 32;
+        return h2f(ld2(blk + 208)) * (float)(int8_t)blk[192 + (e >> 4)] * (float)q;
     }
 };
 
@@ -197,12 +216,28 @@ struct F32Q80 {
     static __device__ __forceinline__ int chunk(int g, int h, int i) { return 8 * g + 4 * h + i; }
     static __device__ __forceinline__ bool live(int step, int g, int K) { return 2 * step + g < K / 32; }
     struct Dec { float s[2]; };
-    static __device__ __forceinline__ void decode(Dec &d, const Raw &w, int) { d.s[0] = h2f(w.d[0]); d.s[1] = h2f(w.d[1]); }
+    static __device__ __forceinline__ void decode(Dec &d, const Raw &w, int) { d.s[0] = h2f(w.d[0]) * X_DOWN; d.s[1] = h2f(w.d[1]) * X_DOWN; }
     static __device__ __forceinline__ ckq_v4i operand(const Raw &w, int g, int i)
     {
         return bytes_to_bf16(w.q[g][2 * i], w.q[g][2 * i + 1]);
     }
+    static constexpr int BLOCK = 32, WBLOCK = 34;
+    static __device__ __forceinline__ float weight(const uint8_t *blk, int e, int i) { return h2f(ld2(blk)) * (float)(int8_t)blk[2 + e + i]; }
 };
+
+/* One output term by term; a NaN stays one. */
+template <class F>
+__device__ __forceinline__ float exact_output(const uint8_t *w, const float *x, int K)
+{
+    float sum = 0.0f;
+#pragma unroll 1
+    for (int k = 0; k < K && sum == sum; k += 16) {
+        const uint8_t *const blk = w + (u32)(k / F::BLOCK) * (u32)F::WBLOCK;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sum += F::weight(blk, k % F::BLOCK, i) * x[k + i];
+    }
+    return sum;
+}
 
 template <class F, int R>
 __global__ void __launch_bounds__(64 * F32_WAVES, 2)
@@ -264,7 +299,7 @@ gemm_f32act_kernel(const float *__restrict__ A, const uint8_t *__restrict__ B, c
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const int e = v[j];
-                    x[4 * i + j] = __builtin_bit_cast(float, e);
+                    x[4 * i + j] = __builtin_bit_cast(float, e) * X_UP;
                 }
             }
 #pragma unroll
@@ -288,8 +323,7 @@ gemm_f32act_kernel(const float *__restrict__ A, const uint8_t *__restrict__ B, c
         }
         if constexpr (F::MIN) {
             /* this half's share of the two sub-block sums, cut in three; the MFMA adds the halves */
-            const float p0 = finite(p[0]), p1 = finite(p[1]);
-            const float m0 = p0 - top16(p0), m1 = p1 - top16(p1);
+            const float m0 = p[0] - top16(p[0]), m1 = p[1] - top16(p[1]);
             const ckq_v4i pa = {(int)pack_bf16(m0 - top16(m0), m0), (int)pack_bf16(p[0], m1 - top16(m1)), (int)pack_bf16(m1, p[1]), 0};
 #pragma unroll
             for (int r = 0; r < R; ++r) {
@@ -311,6 +345,7 @@ gemm_f32act_kernel(const float *__restrict__ A, const uint8_t *__restrict__ B, c
     constexpr int RP = R < 2 ? 1 : 2;
     float *const red = reinterpret_cast<float *>(&xs_all[0][0]);     /* [wave][RP * 16][64] */
     static_assert(F32_WAVES * RP * 16 * 64 * sizeof(float) <= sizeof(xs_all), "the partial tiles fit the activations' place");
+    bool fix = false;
     __syncthreads();                         /* every wave is done with its activations */
     /* the eight partial tiles through LDS, two row tiles at a time; wave w finishes sixteenths 2 w .. of every lane */
 #pragma unroll
@@ -328,7 +363,20 @@ gemm_f32act_kernel(const float *__restrict__ A, const uint8_t *__restrict__ B, c
 #pragma unroll
             for (int k = 1; k < F32_WAVES; ++k) v += red[(k * RP * 16 + o) * 64 + lane];
             const int n = n0 + 32 * (q + (o >> 4)) + col, t = t0 + 8 * (i >> 2) + 4 * half + (i & 3);
+            fix = fix || !(fabsf(v) < __builtin_inff());
             if (n < N && t < M) C[(size_t)t * ldc + n] = bias ? v + bias[n] : v;
+        }
+    }
+    if (fix) {
+#pragma unroll 1
+        for (int j = 0; j < 2 * R; ++j) {
+            const int o = 2 * RP * wave + j % (2 * RP), i = o & 15;
+            const int n = n0 + 32 * (j / (2 * RP) * RP + (o >> 4)) + col, t = t0 + 8 * (i >> 2) + 4 * half + (i & 3);
+            if (n >= N || t >= M) continue;
+            float *const out = C + (size_t)t * ldc + n;
+            if (fabsf(*out) < __builtin_inff()) continue;
+            const float v = exact_output<F>(B + (size_t)n * (size_t)wrow, A + (size_t)t * (size_t)K, K);
+            *out = bias ? v + bias[n] : v;
         }
     }
 }

@@ -1249,10 +1249,52 @@ def test_f32act_matrix_cores_vs_fp64(fmt):
         x[3, k] = np.inf
         got = P.dev_gemm_nt_f32act(fmt, P.to_device(x.reshape(-1)), P.to_device(W), None, M, N, K).cpu().numpy().reshape(M, N)
         assert np.all(np.isfinite(np.delete(got, 3, axis=0)))
-        if fmt != "q4_k":            # in Q4_K the min term subtracts the same infinity
-            assert np.all(got[3] == np.copysign(np.inf, w0[k]))
+        assert np.all(got[3] == np.copysign(np.inf, w0[k]))
     finally:
         L.ckq_set_gemm_policy(0)
+
+
+@pytest.mark.parametrize("fmt", F32_FMTS)
+def test_f32act_matrix_cores_infinite_huge_and_tiny_activations(fmt):
+    """Infinities, NaNs (with a payload in the low 16 bits alone), finite activations whose products with the integers pass the
+    fp32 range where those with the weights do not, denormal activations, blocks whose scale is zero: what the oracle gives,
+    token by token."""
+    import torch
+    L = ckq.lib()
+    M, N, K = 37, 70, 1024
+    W = T.synth_weights(fmt, N, K, seed=15)
+    rows = W.reshape(N, -1)
+    if fmt == "q4_k":
+        rows[5, 4:16] &= 0x30                       # some sub-block scales and mins become zero
+        rows[6, 0:2] = 0                            # d = 0: every weight of the block is -dmin mn
+    x = T.normal(M * K, 0.0, 1.0, seed=16).reshape(M, K)
+    x[2, 100] = np.inf
+    x[3, 700] = -np.inf
+    x[4, 3], x[4, 900] = np.inf, -np.inf
+    x[5, 17:18].view(np.uint32)[:] = 0x7F800001
+    x[6] *= np.float32(2.0 ** 122)
+    x[7, 40] = 3.0e38
+    x[8] *= np.float32(2.0 ** 105)
+    x[9] *= np.float32(2.0 ** -120)
+    x[10] *= np.float32(2.0 ** -130)
+    x[11] = 0.0
+    x[35, 1023] = np.inf
+    with np.errstate(all="ignore"):
+        want = T.oracle_gemm_nt_f32act(fmt, x.reshape(-1), W, None, M, N, K)
+    L.ckq_set_gemm_policy(1)
+    try:
+        say("fp32 activations at the ends of the range", fmt)
+        got = P.dev_gemm_nt_f32act(fmt, P.to_device(x.reshape(-1)), P.to_device(W), None, M, N, K).cpu().numpy().reshape(M, N)
+    finally:
+        L.ckq_set_gemm_policy(0)
+    for t in range(M):
+        fin = np.isfinite(want[t])
+        assert np.array_equal(np.isnan(got[t]), np.isnan(want[t])), t
+        assert np.array_equal(got[t][np.isinf(want[t])], want[t][np.isinf(want[t])]), t
+        if fin.any():
+            scale = float(np.abs(want[t][fin]).max())
+            # a sum of 1024 fp32 products; denormal terms are rounded to multiples of 2^-149 each
+            assert float(np.abs(got[t][fin].astype(np.float64) - want[t][fin]).max()) <= 1e-5 * scale + 1024 * 2.0 ** -149, t
 
 
 # ---- 16-row tiles: a few to a few dozen tokens of the K-quants -------------------------------------
