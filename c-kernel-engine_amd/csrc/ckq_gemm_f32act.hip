@@ -2,25 +2,36 @@
  * ckq_gemm_f32act.hip - several tokens of fp32 activations against Q4_K, Q6_K or Q8_0 weights, nothing
  * quantized, on the bf16 matrix cores with fp32 precision.
  *
- *   C[t][n] = sum over scale groups s:  scale(n,s) * sum_{k in s} q(n,k) * x(t,k)  [- dmin * m(n,s) * sum_{k in s} x(t,k)]  (+ bias[n])
+ *   C[t][n] = sum over scale groups s:  scale(n,s) * sum_{k in s} q(n,k) * x(t,k)  (+ bias[n]);   Q4_K below
  * (reference: gemm_kernels_q4k.c:53-101, gemm_kernels_q6k.c:39-76, gemm_kernels_q8_0.c:254-277, under the token
  * loops of gemm_nt_q4_k / _q6_k / _q8_0).
  *
  * Exactness.  The integers q (4 to 8 bits) are exact in bf16.  An fp32 activation is cut into three bf16 parts,
  * x = hi + mid + lo, each the leading 8 bits of what is left: 24 bits, so the cut is exact (of x 2^24, so that the parts of the
  * smallest numbers are normal too; the scales carry the 2^-24).  Every product of an integer and a part fits fp32, the matrix
- * core adds in fp32, and the scale is applied to the sum of a group in fp32: the only roundings are those of fp32 additions.
+ * core adds in fp32, and the scale is applied to the sum of a group in fp32.
+ *
+ * Precision: rms error against 64 bits no larger than the one-token kernel's (4096 wide, activations of mean 0: Q4_K 1.0e-7
+ * against 1.6e-7, Q6_K 1.0e-7 against 1.6e-7, Q8_0 1.0e-7 against 1.25e-7; 11008 wide 1.2 / 1.4 / 1.2e-7 against 1.65 / 1.6 / 1.3e-7;
+ * the same for mean 1 and 4).  Three things keep it there:
+ * - A weight of Q4_K is s q - m (s = d sc, m = dmin mn, per 32 elements), and s sum(q x) - m sum(x) would cancel after both
+ *   sums were rounded (2.4e-7, with activations of mean 1 1.4e-6).  So the integers are centred: c = rint(m / s) brings q - c
+ *   around zero, and what is left of the min, m - c s, at most s / 2, multiplies sum(x).
+ * - The matrix core cuts off the bits of a sum below its largest term's, towards minus infinity: every sum comes out a little
+ *   low, and hundreds of groups add that up (a third of the error at 4096, more than half at 11008).  Every other group
+ *   therefore multiplies -x, its scale negated too.
+ * - Two groups are added before they meet the running sum, which then takes half as many roundings.
  * Results that are not finite - an activation is not, or is beyond 2^90 or so - are summed again term by term (exact_output),
  * as the kernel for one token forms them.
  *
  * Mapping.  v_mfma_f32_32x32x16_bf16, tokens as rows (A), weight rows as columns (B): a lane holds ONE weight row,
  * so its scale is a register of the lane and one multiply-add per output and group applies it.  A lane (column
  * l % 32, half l / 32) takes the elements its half of the raw bytes holds, straight from memory; the activations are
- * read in the same order, so no byte moves between lanes.  The min term of Q4_K is one more MFMA per 64 elements:
- * the lane's share of the two sub-block sums of x, cut in three like x, against the two mins.
+ * read in the same order, so no byte moves between lanes.  The rest of the min in Q4_K is one more MFMA per group:
+ * the lane's share of the group's sum of x against the row's factor, both cut in three.
  *
  * Block = 8 waves on one tile of 32 tokens x 32 R weight rows; the waves cut K into eight contiguous runs and add
- * their partial tiles through LDS in wave order.  Each wave loads its own activations one step ahead, 256 contiguous bytes
+ * their partial tiles through LDS, in pairs.  Each wave loads its own activations one step ahead, 256 contiguous bytes
  * per token, and turns them through LDS (a lane loading its own row would touch 64 cache lines per instruction: 40 us
  * instead of 36 at 96 x 4096 x 4096, Q6_K; one token per pass over the weights, as the streaming kernel does it, 245 us);
  * no other wave reads them, so the loop has no barrier.  Cutting the activations in a launch of its own and reading the
@@ -28,7 +39,8 @@
  *
  * Grid: token groups fastest, so the blocks that share weights run side by side.
  * Bound: what a CU can load from L2 (8 KiB of activations and 64 rows of weights per wave and step) next to VALU issue
- * (per 64 elements and 32 rows: 60-110 operations to form the integers and apply the scales, 210 / R to cut x).
+ * (per 64 elements 220-260 operations to cut x, shared by the R row tiles, and per row tile 211 / 226 / 123 for Q4_K / Q6_K /
+ * Q8_0 to form the integers and apply the scales; the centring of Q4_K is about 60 of them: 96 x 4096 x 4096 23 -> 27 us).
  */
 #include "ckq_gemm_common.hpp"
 #include "ckq_gemm_f32act.hpp"
@@ -36,7 +48,9 @@
 namespace {
 
 constexpr int F32_WAVES = 8;
-constexpr float X_UP = 16777216.0f, X_DOWN = 1.0f / 16777216.0f;      /* factors of the activations and of the scales */
+/* factors of the activations and of the scales of group g of a step */
+__device__ constexpr float x_up(int g) { return g & 1 ? -16777216.0f : 16777216.0f; }
+__device__ constexpr float x_down(int g) { return 1.0f / x_up(g); }
 
 __device__ __forceinline__ u32 pack_bf16(float lo, float hi)      /* two floats whose low 16 bits are to be dropped */
 {
@@ -99,7 +113,7 @@ __device__ __forceinline__ ckq_v4i bytes_to_bf16(u32 b0, u32 b1)
  *   src_elem(c)     first element of 16-byte chunk c (0..15) of the step's activations
  *   chunk(g, h, i)  which chunk holds floats 4 i .. 4 i + 3 of group g for lane half h
  *   operand(g, i)   bf16x8 of the lane's elements 8 i .. 8 i + 7 of group g
- *   scale(g)        fp32 factor of the group; MIN: min_operand / dmin for the min term
+ *   scale(g)        fp32 factor of the group; MIN: rest(g), the factor of the group's sum of x
  *   weight(blk, e, i)  element e + i of a block, e a multiple of 16 and i below 16, for exact_output */
 struct F32Q4K {
     static constexpr int STEP = 64, NG = 2, NK = 2;
@@ -113,23 +127,32 @@ struct F32Q4K {
     }
     static __device__ __forceinline__ u32 src_elem(int step, int c, int) { return 64u * (u32)step + 4u * c; }
     static __device__ __forceinline__ int chunk(int g, int h, int i) { return 8 * g + 4 * h + i; }
-    static __device__ __forceinline__ bool live(int, int, int) { return true; }
-    struct Dec { float s[2], dmin; ckq_v4i mins; };
-    static __device__ __forceinline__ void decode(Dec &d, const Raw &w, int step)
+    struct Dec { float s[2], rest[2]; u32 off[2]; };          /* off: 128 - c in every byte */
+    static __device__ __forceinline__ void decode(Dec &d, const Raw &w, int step, int)
     {
         u32 sc2, mn2;
         k4_scale_pair(w.hdr[1], w.hdr[2], w.hdr[3], step & 3, &sc2, &mn2);
-        const float dd = h2f(w.hdr[0] & 0xffff) * X_DOWN;
-        d.s[0] = dd * (float)(sc2 & 0xff);
-        d.s[1] = dd * (float)((sc2 >> 8) & 0xff);
-        d.dmin = h2f(w.hdr[0] >> 16) * X_DOWN;
-        const float m0 = (float)(mn2 & 0xff), m1 = (float)((mn2 >> 8) & 0xff);
-        d.mins = ckq_v4i{(int)pack_bf16(m0, m0), (int)pack_bf16(m0, m1), (int)pack_bf16(m1, m1), 0};
+        const float dd = h2f(w.hdr[0] & 0xffff), dm = h2f(w.hdr[0] >> 16);
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            const float m = dm * x_down(g) * (float)((mn2 >> (8 * g)) & 0xff);
+            d.s[g] = dd * x_down(g) * (float)((sc2 >> (8 * g)) & 0xff);
+            /* 0 to 127, so that q - c is a byte; 0 for a scale of 0 (m / 0 or 0 / 0) and for a min of the other sign */
+            float c = __builtin_rintf(m * __builtin_amdgcn_rcpf(d.s[g]));
+            c = d.s[g] == 0.0f ? 0.0f : fminf(fmaxf(c, 0.0f), 127.0f);
+            d.off[g] = 0x80808080u - __builtin_amdgcn_perm(0u, (u32)c, 0u);
+            d.rest[g] = fmaf(-c, d.s[g], m);
+        }
     }
-    static __device__ __forceinline__ ckq_v4i operand(const Raw &w, int g, int i)
+    static __device__ __forceinline__ ckq_v4i operand(const Raw &w, const Dec &d, int g, int i)
     {
-        const u32 a = g ? w.qs[2 * i] >> 4 : w.qs[2 * i], b = g ? w.qs[2 * i + 1] >> 4 : w.qs[2 * i + 1];
-        return bytes_to_bf16(a & 0x0f0f0f0fu, b & 0x0f0f0f0fu);
+        u32 v[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const u32 q = g ? w.qs[2 * i + j] >> 4 : w.qs[2 * i + j];
+            v[j] = ((q & 0x0f0f0f0fu) + d.off[g]) ^ 0x80808080u;      /* no carries between bytes */
+        }
+        return bytes_to_bf16(v[0], v[1]);
     }
     static constexpr int BLOCK = 256, WBLOCK = 144;
     static __device__ __forceinline__ float weight(const uint8_t *blk, int e, int i)
@@ -162,18 +185,15 @@ struct F32Q6K {
         return 128u * (u32)(step >> 1) + 16u * (step & 1) + 32u * (c >> 2) + 4u * (c & 3);
     }
     static __device__ __forceinline__ int chunk(int g, int h, int i) { return 4 * g + 2 * h + i; }
-    static __device__ __forceinline__ bool live(int, int, int) { return true; }
     struct Dec { float s[4]; };
-    static __device__ __forceinline__ void decode(Dec &d, const Raw &w, int step)
+    static __device__ __forceinline__ void decode(Dec &d, const Raw &w, int step, int)
     {
-        const float dd = h2f(w.d) * X_DOWN;
+        const float dd = h2f(w.d);
         const int o = step & 1;
-        d.s[0] = dd * (float)sbyte(w.sc[0], o);
-        d.s[1] = dd * (float)sbyte(w.sc[0], o + 2);
-        d.s[2] = dd * (float)sbyte(w.sc[1], o);
-        d.s[3] = dd * (float)sbyte(w.sc[1], o + 2);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) d.s[g] = dd * x_down(g) * (float)sbyte(w.sc[g >> 1], o + 2 * (g & 1));
     }
-    static __device__ __forceinline__ ckq_v4i operand(const Raw &w, int g, int)
+    static __device__ __forceinline__ ckq_v4i operand(const Raw &w, const Dec &, int g, int)
     {
         u32 q[2];
 #pragma unroll
@@ -214,10 +234,13 @@ struct F32Q80 {
         return 32u * (u32)min(2 * step + (c >> 3), K / 32 - 1) + 4u * (c & 7);
     }
     static __device__ __forceinline__ int chunk(int g, int h, int i) { return 8 * g + 4 * h + i; }
-    static __device__ __forceinline__ bool live(int step, int g, int K) { return 2 * step + g < K / 32; }
     struct Dec { float s[2]; };
-    static __device__ __forceinline__ void decode(Dec &d, const Raw &w, int) { d.s[0] = h2f(w.d[0]) * X_DOWN; d.s[1] = h2f(w.d[1]) * X_DOWN; }
-    static __device__ __forceinline__ ckq_v4i operand(const Raw &w, int g, int i)
+    static __device__ __forceinline__ void decode(Dec &d, const Raw &w, int step, int K)
+    {
+        d.s[0] = h2f(w.d[0]) * x_down(0);
+        d.s[1] = 2 * step + 1 < K / 32 ? h2f(w.d[1]) * x_down(1) : 0.0f;
+    }
+    static __device__ __forceinline__ ckq_v4i operand(const Raw &w, const Dec &, int g, int i)
     {
         return bytes_to_bf16(w.q[g][2 * i], w.q[g][2 * i + 1]);
     }
@@ -286,50 +309,62 @@ gemm_f32act_kernel(const float *__restrict__ A, const uint8_t *__restrict__ B, c
     auto compute = [&](int s) {
         typename F::Dec dec[R];
 #pragma unroll
-        for (int r = 0; r < R; ++r) F::decode(dec[r], w[r], s);
-        float p[F::NG];
+        for (int r = 0; r < R; ++r) F::decode(dec[r], w[r], s, K);
+        /* two groups at a time: their two terms are added before they meet the sum so far */
 #pragma unroll
-        for (int g = 0; g < F::NG; ++g) {
-            if (!F::live(s, g, K)) break;                        /* uniform */
-            Cut c[F::NK];
-            float x[F::NK * 8];
+        for (int g0 = 0; g0 < F::NG; g0 += 2) {
+            Cut c[2][F::NK];
+            ckq_v4i pa[2];
 #pragma unroll
-            for (int i = 0; i < 2 * F::NK; ++i) {
-                const ckq_v4i v = *reinterpret_cast<const ckq_v4i *>(xs + 256 * col + 16 * (F::chunk(g, half, i) ^ (col & 15)));
+            for (int g = 0; g < 2; ++g) {
+                float x[F::NK * 8];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int e = v[j];
-                    x[4 * i + j] = __builtin_bit_cast(float, e) * X_UP;
+                for (int i = 0; i < 2 * F::NK; ++i) {
+                    const ckq_v4i v = *reinterpret_cast<const ckq_v4i *>(xs + 256 * col + 16 * (F::chunk(g0 + g, half, i) ^ (col & 15)));
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int e = v[j];
+                        x[4 * i + j] = __builtin_bit_cast(float, e) * x_up(g);
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < F::NK; ++k) cut8(x + 8 * k, c[g][k]);
+                if constexpr (F::MIN) {
+                    /* this half's share of the group's sum of x, cut in three; against the cut rest of the min, the six
+                     * products that matter in one MFMA, which also adds the halves */
+                    const float p = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7])) +
+                                    (((x[8] + x[9]) + (x[10] + x[11])) + ((x[12] + x[13]) + (x[14] + x[15])));
+                    const float m = p - top16(p), l = m - top16(m);
+                    pa[g] = ckq_v4i{(int)pack_bf16(p, p), (int)pack_bf16(m, m), (int)pack_bf16(p, l), 0};
                 }
             }
 #pragma unroll
-            for (int k = 0; k < F::NK; ++k) cut8(x + 8 * k, c[k]);
-            if constexpr (F::MIN)
-                p[g] = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7])) +
-                       (((x[8] + x[9]) + (x[10] + x[11])) + ((x[12] + x[13]) + (x[14] + x[15])));
-#pragma unroll
             for (int r = 0; r < R; ++r) {
-                ckq_v16f sum = zero;
+                ckq_v16f two, sum;
+                if constexpr (F::MIN) {
+                    two = zero;
 #pragma unroll
-                for (int k = 0; k < F::NK; ++k) {
-                    const ckq_v4i b = F::operand(w[r], g, k);
-                    sum = mfma_bf16(c[k].lo, b, sum);
-                    sum = mfma_bf16(c[k].mid, b, sum);
-                    sum = mfma_bf16(c[k].hi, b, sum);
+                    for (int g = 0; g < 2; ++g) {
+                        const float h = dec[r].rest[g0 + g], m = h - top16(h), l = m - top16(m);
+                        two = mfma_bf16(pa[g], ckq_v4i{(int)pack_bf16(h, m), (int)pack_bf16(h, m), (int)pack_bf16(l, h), 0}, two);
+                    }
                 }
 #pragma unroll
-                for (int i = 0; i < 16; ++i) acc[r][i] = fmaf(dec[r].s[g], sum[i], acc[r][i]);
-            }
-        }
-        if constexpr (F::MIN) {
-            /* this half's share of the two sub-block sums, cut in three; the MFMA adds the halves */
-            const float m0 = p[0] - top16(p[0]), m1 = p[1] - top16(p[1]);
-            const ckq_v4i pa = {(int)pack_bf16(m0 - top16(m0), m0), (int)pack_bf16(p[0], m1 - top16(m1)), (int)pack_bf16(m1, p[1]), 0};
+                for (int g = 0; g < 2; ++g) {
+                    sum = zero;
 #pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const ckq_v16f i2 = mfma_bf16(pa, dec[r].mins, zero);
+                    for (int k = 0; k < F::NK; ++k) {
+                        const ckq_v4i b = F::operand(w[r], dec[r], g0 + g, k);
+                        sum = mfma_bf16(c[g][k].lo, b, sum);
+                        sum = mfma_bf16(c[g][k].mid, b, sum);
+                        sum = mfma_bf16(c[g][k].hi, b, sum);
+                    }
 #pragma unroll
-                for (int i = 0; i < 16; ++i) acc[r][i] = fmaf(-dec[r].dmin, i2[i], acc[r][i]);
+                    for (int i = 0; i < 16; ++i)
+                        two[i] = F::MIN || g ? fmaf(dec[r].s[g0 + g], sum[i], F::MIN && !g ? -two[i] : two[i]) : dec[r].s[g0 + g] * sum[i];
+                }
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[r][i] += two[i];
             }
         }
     };
@@ -359,9 +394,10 @@ gemm_f32act_kernel(const float *__restrict__ A, const uint8_t *__restrict__ B, c
 #pragma unroll
         for (int j = 0; j < 2 * RP; ++j) {
             const int o = 2 * RP * wave + j, i = o & 15;
-            float v = red[o * 64 + lane];
+            float p[F32_WAVES];
 #pragma unroll
-            for (int k = 1; k < F32_WAVES; ++k) v += red[(k * RP * 16 + o) * 64 + lane];
+            for (int k = 0; k < F32_WAVES; ++k) p[k] = red[(k * RP * 16 + o) * 64 + lane];
+            const float v = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
             const int n = n0 + 32 * (q + (o >> 4)) + col, t = t0 + 8 * (i >> 2) + 4 * half + (i & 3);
             fix = fix || !(fabsf(v) < __builtin_inff());
             if (n < N && t < M) C[(size_t)t * ldc + n] = bias ? v + bias[n] : v;

@@ -77,7 +77,7 @@ static bool gemm_on_matrix_cores(int ntok, size_t weight_bytes, size_t budget_mb
 /* fp32 activations.  The streaming kernel decodes the weights again for every token; the matrix-core kernel
  * (ckq_gemm_f32act.hip) decodes them once per 32 tokens.  Fitted to launches of both over 141..11008 rows, widths
  * of 512..8192 and 1..200 tokens (us): streaming 4 + 0.125 / 0.18 / 0.16 (Q4_K / Q6_K / Q8_0) per million products; matrix cores
- * 6 + 0.017 / 0.024 / 0.024 per million products of the tokens rounded up to 32, but never less than 5 + 1.35 for every
+ * 6 + 0.020 / 0.024 / 0.024 per million products of the tokens rounded up to 32, but never less than 5 + 1.35 (Q4_K 1.5) for every
  * 64 elements a wave walks through (an eighth of K).  4096 x 4096 Q6_K: 4 tokens 14.5 against 19 (streams), 8 tokens 26 against
  * 19, 96 tokens 270 against 36; 141 x 8192 streams up to 96 tokens. */
 static bool f32act_on_matrix_cores(int fmt, int ntok, int nrows, int K)
@@ -86,10 +86,10 @@ static bool f32act_on_matrix_cores(int fmt, int ntok, int nrows, int K)
     if (ntok < 2 || policy == 2) return false;
     if (policy == 1) return true;
     const float per = fmt == CKQ_KERNEL_Q4K_F32 ? 0.125f : fmt == CKQ_KERNEL_Q6K_F32 ? 0.18f : 0.16f;
-    const float per_matrix = fmt == CKQ_KERNEL_Q4K_F32 ? 0.017f : 0.024f;
+    const float per_matrix = fmt == CKQ_KERNEL_Q4K_F32 ? 0.020f : 0.024f, per_step = fmt == CKQ_KERNEL_Q4K_F32 ? 1.5f : 1.35f;
     const float mw = (float)nrows * (float)K * 1e-6f;
     const float t_stream = 4.0f + per * mw * (float)ntok;
-    const float t_matrix = fmaxf(5.0f + 1.35f * (float)((K + 511) / 512), 6.0f + per_matrix * mw * (float)((ntok + 31) / 32 * 32));
+    const float t_matrix = fmaxf(5.0f + per_step * (float)((K + 511) / 512), 6.0f + per_matrix * mw * (float)((ntok + 31) / 32 * 32));
     return t_stream > t_matrix;
 }
 

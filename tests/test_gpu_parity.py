@@ -1255,6 +1255,37 @@ def test_f32act_matrix_cores_vs_fp64(fmt):
 
 
 @pytest.mark.parametrize("fmt", F32_FMTS)
+@pytest.mark.parametrize("mean", [0.0, 1.0, 4.0])
+def test_f32act_matrix_cores_are_as_exact_as_one_token_at_a_time(fmt, mean):
+    """Error of both kernels for fp32 activations against 64 bits, for activations of mean 0, 1 and 4 (the min term of Q4_K is
+    then a large part of what the scales sum to): encoded weights, random blocks, and Q4_K blocks whose min is many times the
+    scale or has the other sign.  An error is the rms over 512 rows of a row's relative one, of 32 tokens, and within 1 % or so
+    of its expectation; the matrix cores' is not the larger one."""
+    import torch
+    L = ckq.lib()
+    M, N = 32, 512
+    for kind, K in (("enc", 1024), ("enc", 4096), ("enc", 11008), ("rand", 2048), ("odd", 2048)):
+        W = T.synth_weights(fmt, N, K, seed=40 + K) if kind == "enc" else T.random_blocks(fmt, N * K // T.ELEMS[fmt], 43)
+        if kind == "odd" and fmt == "q4_k":
+            blocks = W.reshape(-1, 144)
+            blocks[0::3, 0:2] = (0x01, 0x00)         # d = 2^-24
+            blocks[1::3, 3] ^= 0x80                  # dmin negated
+        x = T.normal(M * K, mean, 1.0, seed=41 + K)
+        want = x.reshape(M, K).astype(np.float64) @ T.np_dequant(fmt, W).reshape(N, K).T
+        err = []
+        for policy in (2, 1):
+            say("fp32 activations, error", fmt, mean, kind, K, policy)
+            L.ckq_set_gemm_policy(policy)
+            try:
+                got = P.dev_gemm_nt_f32act(fmt, P.to_device(x), P.to_device(W), None, M, N, K).cpu().numpy().reshape(M, N)
+            finally:
+                L.ckq_set_gemm_policy(0)
+            err.append(float(np.sqrt(np.mean(np.sum((got - want) ** 2, axis=0) / np.sum(want ** 2, axis=0)))))
+        say("   one token at a time %.3e  matrix cores %.3e" % tuple(err))
+        assert err[1] <= 1.03 * err[0], (kind, K, err)
+
+
+@pytest.mark.parametrize("fmt", F32_FMTS)
 def test_f32act_matrix_cores_infinite_huge_and_tiny_activations(fmt):
     """Infinities, NaNs (with a payload in the low 16 bits alone), finite activations whose products with the integers pass the
     fp32 range where those with the weights do not, denormal activations, blocks whose scale is zero: what the oracle gives,
