@@ -270,8 +270,8 @@ static bool weights_dword_aligned(const GemvArgs &a, const GemvGroup &grp)
  *   streaming  the larger of 4.35 + 0.07 nb (to eight tokens 3.5, where smaller tiles fill the chip: Q5_K 1024 x 2048 at 5
  *              4.5 -> 3.7 us, Q4_K 1024 x 1024 3.9 -> 3.6) and 3.05 + 0.11 nb + (0.24, 0.245, 0.29) mb for every eight tokens, 5 to 8 as 10
  * Three and four tokens, one pass of half the width, only move for long rows of large matrices (4096 x 11008 Q6_K:
- * 17.0 -> 13.4); two never do.  The forced policies keep their kernels: 1 the tile kernels, and 2 the streaming kernels,
- * whose order this one keeps where `tiles` is false. */
+ * 17.0 -> 13.4); two never do.  The forced policies keep their kernels: 1 the tile kernels, 2 the streaming kernel at any number of
+ * tokens.  Forced itself (ckq_launch_set_rows16) it goes before both, in the order of the kernel they ask for. */
 static std::atomic<int> g_rows16_forced{0};           /* bit per format tag */
 extern "C" void ckq_launch_set_rows16(int fmt, int on)
 {
@@ -283,8 +283,8 @@ static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles)
 {
     if (ntok < 2 || K > ROWS16_MAX_K) return false;
     if (g_rows16_forced.load(std::memory_order_relaxed) >> fmt & 1) return true;
-    if (ntok < 3) return false;
-    if (tiles && g_gemm_policy.load(std::memory_order_relaxed) == 1) return false;
+    const int policy = g_gemm_policy.load(std::memory_order_relaxed);
+    if (ntok < 3 || policy == 2 || (tiles && policy == 1)) return false;
     const int f = fmt == CKQ_FMT_Q4_K ? 0 : fmt == CKQ_FMT_Q5_K ? 1 : 2;
     static const float per_block[3] = {0.36f, 0.65f, 0.71f}, per_pass[3] = {0.24f, 0.245f, 0.29f};
     const float nb = (float)(K / 256), mb = (float)rows * nb * (f == 0 ? 144e-6f : f == 1 ? 176e-6f : 210e-6f);
@@ -297,18 +297,35 @@ static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles)
     return t_rows < t_else;
 }
 
+/* K-quants: does a matmul of this size go to the tile kernels (or, at their sizes, to the 16-row tiles)? */
+static bool kquant_on_matrix_cores(int fmt, int ntok, size_t rows, int K)
+{
+    return gemm_on_matrix_cores(ntok, rows * (size_t)(K / 256) * (fmt == CKQ_FMT_Q4_K ? 144 : fmt == CKQ_FMT_Q5_K ? 176 : 210), fmt == CKQ_FMT_Q5_K ? 40 : 20);
+}
+
+/* Where a matmul of a whole matrix goes. */
+extern "C" int ckq_launch_route(int fmt, int nrows, int K, int ntok, int aligned)
+{
+    bool tiles;
+    switch (fmt) {
+    case CKQ_FMT_Q4_K: case CKQ_FMT_Q5_K: case CKQ_FMT_Q6_K:
+        tiles = kquant_on_matrix_cores(fmt, ntok, (size_t)nrows, K);
+        if (take_rows16(fmt, ntok, (size_t)nrows, K, tiles)) return tiles ? CKQ_ROUTE_ROWS16_TILES : CKQ_ROUTE_ROWS16_STREAM;
+        break;
+    case CKQ_FMT_Q8_0: tiles = gemm_q80_on_matrix_cores(ntok, (size_t)nrows * (K / 32) * 34, K % 64 == 0 && aligned); break;
+    case CKQ_FMT_Q5_0: tiles = gemm_on_matrix_cores(ntok, (size_t)nrows * (K / 32) * 22, 20); break;
+    case CKQ_KERNEL_Q80_F32: case CKQ_KERNEL_Q4K_F32: case CKQ_KERNEL_Q6K_F32: tiles = f32act_on_matrix_cores(fmt, ntok, nrows, K); break;
+    default: return CKQ_EFORMAT;
+    }
+    return tiles ? CKQ_ROUTE_TILES : CKQ_ROUTE_STREAM;
+}
+
 /* The chains of multiply-adds of such a launch: those of the tile kernel where it stands in for one, so that the result
  * has the tile kernel's bits. */
 static GemmChains rows16_chains(int fmt, int ntok, int nrows, int K, bool tiles)
 {
     if (!tiles) return {1, K / 256, 1};
     return fmt == CKQ_FMT_Q4_K ? gemm_q4k_chains(ntok, nrows, K) : fmt == CKQ_FMT_Q5_K ? gemm_q5k_chains(ntok, nrows, K) : gemm_q6k_chains(ntok, nrows, K);
-}
-
-/* K-quants: does a matmul of this size go to the tile kernels (or, at their sizes, to the 16-row tiles)? */
-static bool kquant_on_matrix_cores(int fmt, int ntok, size_t rows, int K)
-{
-    return gemm_on_matrix_cores(ntok, rows * (size_t)(K / 256) * (fmt == CKQ_FMT_Q4_K ? 144 : fmt == CKQ_FMT_Q5_K ? 176 : 210), fmt == CKQ_FMT_Q5_K ? 40 : 20);
 }
 
 static int launch_rows16_one(int fmt, const GemvArgs &a, bool tiles, int K, hipStream_t s)
@@ -447,41 +464,33 @@ static int launch_gemv_args(int fmt_flags, GemvArgs &a, const GemvGroup &grp, in
     hipStream_t s = (hipStream_t)stream;
     const bool dump = a.sub != nullptr;
     const bool whole = !dump && grp.n == 1 && row0 == 0 && row1 == nrows;   /* what a matrix-core GEMM can take */
+    const bool aligned = weights_dword_aligned(a, grp);
+    const int route = whole ? ckq_launch_route(fmt, nrows, K, ntok, aligned) : CKQ_ROUTE_STREAM;
     switch (fmt) {
     case CKQ_FMT_Q4_K:
         if (K % 256) return CKQ_ESHAPE;
-        if (whole) {
-            const bool tiles = kquant_on_matrix_cores(fmt, ntok, (size_t)nrows, K);
-            if (take_rows16(fmt, ntok, (size_t)nrows, K, tiles)) return launch_rows16_one(fmt, a, tiles, K, s);
-            if (tiles) return launch_gemm_q4k_mfma(X, W, bias, y, ntok, nrows, K, ldy, opts, s);
-        }
+        if (route == CKQ_ROUTE_ROWS16_STREAM || route == CKQ_ROUTE_ROWS16_TILES) return launch_rows16_one(fmt, a, route == CKQ_ROUTE_ROWS16_TILES, K, s);
+        if (route == CKQ_ROUTE_TILES) return launch_gemm_q4k_mfma(X, W, bias, y, ntok, nrows, K, ldy, opts, s);
         a.npos = K / 64; a.wrow = (long)(K / 256) * 144; a.xrow = (long)(K / 256) * 292; a.nsub_row = K / 32;
         return ckq_gemv_launch_q4k(a, grp, s);
     case CKQ_FMT_Q5_K:
         if (K % 256) return CKQ_ESHAPE;
-        if (whole) {
-            const bool tiles = kquant_on_matrix_cores(fmt, ntok, (size_t)nrows, K);
-            if (take_rows16(fmt, ntok, (size_t)nrows, K, tiles)) return launch_rows16_one(fmt, a, tiles, K, s);
-            if (tiles) return launch_gemm_q5k_mfma(X, W, bias, y, ntok, nrows, K, ldy, opts, s);
-        }
+        if (route == CKQ_ROUTE_ROWS16_STREAM || route == CKQ_ROUTE_ROWS16_TILES) return launch_rows16_one(fmt, a, route == CKQ_ROUTE_ROWS16_TILES, K, s);
+        if (route == CKQ_ROUTE_TILES) return launch_gemm_q5k_mfma(X, W, bias, y, ntok, nrows, K, ldy, opts, s);
         a.npos = K / 64; a.wrow = (long)(K / 256) * 176; a.xrow = (long)(K / 256) * 292; a.nsub_row = K / 32;
         return ckq_gemv_launch_q5k(a, grp, s);
     case CKQ_FMT_Q6_K:
         if (K % 256) return CKQ_ESHAPE;
-        if (whole) {
-            const bool tiles = kquant_on_matrix_cores(fmt, ntok, (size_t)nrows, K);
-            if (take_rows16(fmt, ntok, (size_t)nrows, K, tiles)) return launch_rows16_one(fmt, a, tiles, K, s);
-            if (tiles) return launch_gemm_q6k_mfma(X, W, bias, y, ntok, nrows, K, ldy, opts, s);
-        }
+        if (route == CKQ_ROUTE_ROWS16_STREAM || route == CKQ_ROUTE_ROWS16_TILES) return launch_rows16_one(fmt, a, route == CKQ_ROUTE_ROWS16_TILES, K, s);
+        if (route == CKQ_ROUTE_TILES) return launch_gemm_q6k_mfma(X, W, bias, y, ntok, nrows, K, ldy, opts, s);
         a.npos = K / 64; a.wrow = (long)(K / 256) * 210; a.xrow = (long)(K / 256) * 292; a.nsub_row = K / 16;
         return ckq_gemv_launch_q6k(a, grp, s);
     case CKQ_FMT_Q8_0:
         if (K % 32) return CKQ_ESHAPE;
-        if (whole && gemm_q80_on_matrix_cores(ntok, (size_t)nrows * (K / 32) * 34, K % 64 == 0 && weights_dword_aligned(a, grp)))
-            return launch_gemm_q80_mfma(X, W, bias, y, ntok, nrows, K, ldy, opts, s);
+        if (route == CKQ_ROUTE_TILES) return launch_gemm_q80_mfma(X, W, bias, y, ntok, nrows, K, ldy, opts, s);
         a.wrow = (long)(K / 32) * 34; a.xrow = (long)(K / 32) * 34; a.nsub_row = K / 32;
         /* rows of an even number of blocks at dword-aligned addresses: two blocks per position, aligned loads */
-        if (K % 64 == 0 && weights_dword_aligned(a, grp)) {
+        if (K % 64 == 0 && aligned) {
             a.npos = K / 64;
             return ckq_gemv_launch_q80p(a, grp, s);
         }
@@ -491,7 +500,7 @@ static int launch_gemv_args(int fmt_flags, GemvArgs &a, const GemvGroup &grp, in
         if (K % 32) return CKQ_ESHAPE;
         /* prefill: the blocks are rewritten as Q8_0 blocks (same scale, values
          * q - 16: every dot product is unchanged) and go to the Q8_0 GEMM */
-        if (whole && gemm_on_matrix_cores(ntok, (size_t)nrows * (K / 32) * 22, 20)) {
+        if (route == CKQ_ROUTE_TILES) {
             if (opts.scratch) return CKQ_ESCRATCH;       /* the rewritten weights would need an allocation */
             return launch_gemm_q50_via_q80(X, W, bias, y, ntok, nrows, K, ldy, s);
         }
@@ -500,19 +509,19 @@ static int launch_gemv_args(int fmt_flags, GemvArgs &a, const GemvGroup &grp, in
     case CKQ_KERNEL_Q80_F32:
         if (K % 32) return CKQ_ESHAPE;
         if (dump || grp.n > 1) return CKQ_EINVAL;
-        if (whole && f32act_on_matrix_cores(fmt, ntok, nrows, K)) return launch_gemm_f32act(fmt, (const float *)X, W, bias, y, ntok, nrows, K, ldy, s);
+        if (route == CKQ_ROUTE_TILES) return launch_gemm_f32act(fmt, (const float *)X, W, bias, y, ntok, nrows, K, ldy, s);
         a.npos = K / 32; a.wrow = (long)(K / 32) * 34; a.xrow = (long)K * 4; a.nsub_row = K / 32;
         return ckq_gemv_launch_q80_f32(a, grp, s);
     case CKQ_KERNEL_Q4K_F32:
         if (K % 256) return CKQ_ESHAPE;
         if (dump || grp.n > 1) return CKQ_EINVAL;
-        if (whole && f32act_on_matrix_cores(fmt, ntok, nrows, K)) return launch_gemm_f32act(fmt, (const float *)X, W, bias, y, ntok, nrows, K, ldy, s);
+        if (route == CKQ_ROUTE_TILES) return launch_gemm_f32act(fmt, (const float *)X, W, bias, y, ntok, nrows, K, ldy, s);
         a.npos = K / 64; a.wrow = (long)(K / 256) * 144; a.xrow = (long)K * 4; a.nsub_row = K / 64;
         return ckq_gemv_launch_q4k_f32(a, grp, s);
     case CKQ_KERNEL_Q6K_F32:
         if (K % 256) return CKQ_ESHAPE;
         if (dump || grp.n > 1) return CKQ_EINVAL;
-        if (whole && f32act_on_matrix_cores(fmt, ntok, nrows, K)) return launch_gemm_f32act(fmt, (const float *)X, W, bias, y, ntok, nrows, K, ldy, s);
+        if (route == CKQ_ROUTE_TILES) return launch_gemm_f32act(fmt, (const float *)X, W, bias, y, ntok, nrows, K, ldy, s);
         a.npos = K / 64; a.wrow = (long)(K / 256) * 210; a.xrow = (long)K * 4; a.nsub_row = K / 64;
         return ckq_gemv_launch_q6k_f32(a, grp, s);
     default:

@@ -70,9 +70,14 @@ int ckq_launch_gemm_group(int fmt, int n, float *const *C, const void *const *B,
 int ckq_launch_gemm_block_sums(int fmt, const void *A, const void *B, const float *bias, float *C, int32_t *sums,
                                int M, int N, int K, long ldc, void *stream);
 
-/* Kernel choice for more than eight tokens: 0 = by token count and weight size
- * (default), 1 = always the matrix-core GEMM, 2 = always the streaming kernel. */
+/* Kernel choice: 0 = by token count and weight size (default), 1 = above eight tokens always the matrix-core GEMM (fp32
+ * activations: from two on), 2 = always the streaming kernel. */
 void ckq_launch_set_gemm_policy(int policy);
+/* Where ckq_launch_gemv sends a matmul of a whole matrix (K a multiple of the block size; `aligned`: the weights start on a
+ * dword, which Q8_0 looks at): the streaming kernel, the tile kernels of the matrix cores, or the 16-row tiles in the order of
+ * either.  Host arithmetic; exported for the test of the rules. */
+enum { CKQ_ROUTE_STREAM = 0, CKQ_ROUTE_TILES = 1, CKQ_ROUTE_ROWS16_STREAM = 2, CKQ_ROUTE_ROWS16_TILES = 3 };
+int ckq_launch_route(int fmt, int nrows, int K, int ntok, int aligned);
 /* Token tile of the Q4_K x Q8_K matrix-core GEMM: 0 = by shape (default), 64 or 96 = always that kernel. */
 void ckq_launch_set_q4k_tile(int tokens);
 /* Q6_K x Q8_K matrix-core GEMM: 0 = by shape (default), 1 = one block per CU always, 2 = the paired 64-token kernel always. */

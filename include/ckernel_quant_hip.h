@@ -418,13 +418,16 @@ void ckq_set_prefill_grouping(int enabled);
  * and download instead of nth serialized ones: 5 to 9 times faster per
  * dispatch); a negative value restores the default. */
 void ckq_set_parallel_whole(int enabled);
-/* Which kernel serves a matmul of more than eight tokens (up to eight always
- * take the weight-streaming kernel, one pass over the weights).  AUTO, the
- * default, picks by token count and weight size: the streaming kernel while
- * its passes over the weights are cheaper than the matrix-core GEMM's fixed
- * cost, the matrix cores beyond.  MATRIX and STREAM force one of them (tests,
- * tuning); CKQ_GEMM_POLICY=matrix|stream sets it from the environment.  Both
- * kernels meet the same tolerance; their fp32 summation orders differ. */
+/* Which kernel serves a matmul of several tokens.  AUTO, the default, picks by
+ * token count and weight size: the weight-streaming kernel while its passes
+ * over the weights, of up to eight tokens each, are cheaper than the
+ * matrix-core GEMM's fixed cost, the matrix cores beyond; K-quants of three to
+ * a few dozen tokens may run on 16-row tiles of the matrix cores, with the bits
+ * of the kernel they stand in for.  STREAM always streams; MATRIX takes the
+ * GEMM for every matmul of more than eight tokens (fp32 activations: of two
+ * and more); tests, tuning.  CKQ_GEMM_POLICY=matrix|stream sets it from the
+ * environment.  Both kernels meet the same tolerance; their fp32 summation
+ * orders differ. */
 enum { CKQ_GEMM_AUTO = 0, CKQ_GEMM_MATRIX = 1, CKQ_GEMM_STREAM = 2 };
 void ckq_set_gemm_policy(int policy);
 /* Variants of the matrix-core GEMMs (tests, tuning; 0, the default, picks by shape).  Every variant of a format computes

@@ -153,6 +153,37 @@ def test_grid_chunk_index_arithmetic(L):
         assert covered == total and c == -(-total // per)
 
 
+STREAM, TILES, ROWS16_STREAM, ROWS16_TILES = range(4)
+ROUTE_SHAPES = [(n, k) for n in (1, 128, 1000, 4096, 16383, 32000) for k in (256, 512, 1024, 4096, 11008, 16640)]
+ROUTE_TOKENS = (1, 2, 3, 4, 5, 8, 9, 16, 33, 93, 512)
+
+
+def route(L, fmt, n, k, tokens, f32=False, aligned=1):
+    tag = {"q4_k": 17, "q6_k": 18, "q8_0": 16}[fmt] if f32 else ckq.parity.FMT[fmt]
+    return L.ckq_launch_route(tag, n, k, tokens, aligned)
+
+
+def test_forced_policies_keep_their_kernels(L):
+    """STREAM streams at every token count, MATRIX takes the tile kernels above eight tokens (fp32 activations: from two on), over
+    all formats and sizes; the automatic choice uses the 16-row tiles somewhere at either side of eight tokens."""
+    fmts = [(f, False) for f in ("q4_k", "q5_k", "q6_k", "q8_0", "q5_0")] + [(f, True) for f in ("q4_k", "q6_k", "q8_0")]
+    try:
+        seen = set()
+        for fmt, f32 in fmts:
+            for n, k in ROUTE_SHAPES:
+                for t in ROUTE_TOKENS:
+                    L.ckq_set_gemm_policy(0)
+                    seen.add((route(L, fmt, n, k, t, f32), t > 8))
+                    L.ckq_set_gemm_policy(2)
+                    assert route(L, fmt, n, k, t, f32) == STREAM, (fmt, f32, n, k, t)
+                    L.ckq_set_gemm_policy(1)
+                    if t > (1 if f32 else 8):
+                        assert route(L, fmt, n, k, t, f32) == TILES, (fmt, f32, n, k, t)
+        assert {(ROWS16_STREAM, False), (ROWS16_STREAM, True), (ROWS16_TILES, True)} <= seen
+    finally:
+        L.ckq_set_gemm_policy(0)
+
+
 def test_workspace_slot_bookkeeping(L):
     """Slot choice of the per-(device, stream, kind) scratch table of the K-split
     GEMMs: a known key finds its slot, a new key takes the first free slot, and
