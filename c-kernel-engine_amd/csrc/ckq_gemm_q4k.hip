@@ -361,6 +361,7 @@ __global__ void __launch_bounds__(256 * KG, KG == 2 ? 1 : WPE) gemm_q4k_mfma_ker
  * blocks compete with 64-token tiles that all fit one round (960 x 4096: 52.6 against 45.4).  `tiles64`: tiles of the 64-token kernel, `blocks96`: blocks of the 96-token one. */
 static std::atomic<int> g_q4k_tile{0};
 extern "C" void ckq_launch_set_q4k_tile(int tokens) { g_q4k_tile.store(tokens == 64 || tokens == 96 ? tokens : 0); }
+bool gemm_q4k_forced() { return g_q4k_tile.load(std::memory_order_relaxed) != 0; }
 static bool q4k_take_t96(int M, int tiles64, int blocks96)
 {
     const int forced = g_q4k_tile.load(std::memory_order_relaxed);

@@ -446,6 +446,7 @@ __global__ void __launch_bounds__(256, 2) gemm_q5k_pair_kernel(GemmArgs a)
  * itself (256 tiles: 81.7 against 83.0).  variant: 0 = by tile count, 1 = one block per CU always, 2 = paired always. */
 static std::atomic<int> g_q5k_variant{0};
 extern "C" void ckq_launch_set_q5k_variant(int variant) { g_q5k_variant.store(variant == 1 || variant == 2 ? variant : 0); }
+bool gemm_q5k_forced() { return g_q5k_variant.load(std::memory_order_relaxed) != 0; }
 static bool q5k_take_pair(int tiles)
 {
     const int forced = g_q5k_variant.load(std::memory_order_relaxed);

@@ -460,6 +460,7 @@ __global__ void __launch_bounds__(256, 2) gemm_q6k_pair_kernel(GemmArgs a)
  * paired 78.7) and there are at least 512 blocks of 64 tokens.  variant: 0 = by shape, 1 = never, 2 = always. */
 static std::atomic<int> g_q6k_variant{0};
 extern "C" void ckq_launch_set_q6k_variant(int variant) { g_q6k_variant.store(variant == 1 || variant == 2 ? variant : 0); }
+bool gemm_q6k_forced() { return g_q6k_variant.load(std::memory_order_relaxed) != 0; }
 static bool q6k_take_pair(int tiles128, int tiles64)
 {
     const int forced = g_q6k_variant.load(std::memory_order_relaxed);

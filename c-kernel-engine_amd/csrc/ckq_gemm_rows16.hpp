@@ -21,6 +21,10 @@ static inline GemmChains gemm_chains_split(int tiles, int steps)
 GemmChains gemm_q4k_chains(int M, int N, int K);
 GemmChains gemm_q5k_chains(int M, int N, int K);
 GemmChains gemm_q6k_chains(int M, int N, int K);
+/* Has the caller asked for one of the tile kernels (ckq_set_prefill_variant)? */
+bool gemm_q4k_forced();
+bool gemm_q5k_forced();
+bool gemm_q6k_forced();
 /* Those of a shared launch of several matrices; false: launch_gemm_*_mfma_group would not take it. */
 bool gemm_q4k_group_chains(const GemmGroupIn &in, int M, int K, GemmChains *ch);
 bool gemm_q5k_group_chains(const GemmGroupIn &in, int M, int K, GemmChains *ch);

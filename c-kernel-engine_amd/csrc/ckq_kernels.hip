@@ -271,7 +271,8 @@ static bool weights_dword_aligned(const GemvArgs &a, const GemvGroup &grp)
  *              4.5 -> 3.7 us, Q4_K 1024 x 1024 3.9 -> 3.6) and 3.05 + 0.11 nb + (0.24, 0.245, 0.29) mb for every eight tokens, 5 to 8 as 10
  * Three and four tokens, one pass of half the width, only move for long rows of large matrices (4096 x 11008 Q6_K:
  * 17.0 -> 13.4); two never do.  The forced policies keep their kernels: 1 the tile kernels, 2 the streaming kernel at any number of
- * tokens.  Forced itself (ckq_launch_set_rows16) it goes before both, in the order of the kernel they ask for. */
+ * tokens; and so does a tile kernel that the caller asked for.  Forced itself (ckq_launch_set_rows16) it goes before all of them, in
+ * the order of the kernel that the policy asks for. */
 static std::atomic<int> g_rows16_forced{0};           /* bit per format tag */
 extern "C" void ckq_launch_set_rows16(int fmt, int on)
 {
@@ -284,8 +285,9 @@ static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles)
     if (ntok < 2 || K > ROWS16_MAX_K) return false;
     if (g_rows16_forced.load(std::memory_order_relaxed) >> fmt & 1) return true;
     const int policy = g_gemm_policy.load(std::memory_order_relaxed);
-    if (ntok < 3 || policy == 2 || (tiles && policy == 1)) return false;
     const int f = fmt == CKQ_FMT_Q4_K ? 0 : fmt == CKQ_FMT_Q5_K ? 1 : 2;
+    const bool tile_forced = f == 0 ? gemm_q4k_forced() : f == 1 ? gemm_q5k_forced() : gemm_q6k_forced();
+    if (ntok < 3 || policy == 2 || (tiles && (policy == 1 || tile_forced))) return false;
     static const float per_block[3] = {0.36f, 0.65f, 0.71f}, per_pass[3] = {0.24f, 0.245f, 0.29f};
     const float nb = (float)(K / 256), mb = (float)rows * nb * (f == 0 ? 144e-6f : f == 1 ? 176e-6f : 210e-6f);
     if (ntok <= 4) return K > 4096 && mb >= 20.0f;

@@ -78,11 +78,13 @@ void ckq_launch_set_gemm_policy(int policy);
  * either.  Host arithmetic; exported for the test of the rules. */
 enum { CKQ_ROUTE_STREAM = 0, CKQ_ROUTE_TILES = 1, CKQ_ROUTE_ROWS16_STREAM = 2, CKQ_ROUTE_ROWS16_TILES = 3 };
 int ckq_launch_route(int fmt, int nrows, int K, int ntok, int aligned);
-/* Token tile of the Q4_K x Q8_K matrix-core GEMM: 0 = by shape (default), 64 or 96 = always that kernel. */
+/* Token tile of the Q4_K x Q8_K matrix-core GEMM: 0 = by shape (default), 64 or 96 = that kernel wherever the GEMM is taken. */
 void ckq_launch_set_q4k_tile(int tokens);
-/* Q6_K x Q8_K matrix-core GEMM: 0 = by shape (default), 1 = one block per CU always, 2 = the paired 64-token kernel always. */
+/* Q6_K x Q8_K matrix-core GEMM: 0 = by shape (default), 1 = one block per CU, 2 = the paired 64-token kernel,
+ * wherever the GEMM is taken. */
 void ckq_launch_set_q6k_variant(int variant);
-/* Q5_K x Q8_K matrix-core GEMM: 0 = by tile count (default), 1 = one block per CU always, 2 = the paired kernel always. */
+/* Q5_K x Q8_K matrix-core GEMM: 0 = by tile count (default), 1 = one block per CU, 2 = the paired kernel,
+ * wherever the GEMM is taken. */
 void ckq_launch_set_q5k_variant(int variant);
 /* K-quants: 1 = the 16-row tiles take every matmul of two and more tokens (K up to 16384), 0 = by shape (default). */
 void ckq_launch_set_rows16(int fmt, int on);

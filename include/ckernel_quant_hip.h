@@ -430,7 +430,8 @@ void ckq_set_parallel_whole(int enabled);
  * orders differ. */
 enum { CKQ_GEMM_AUTO = 0, CKQ_GEMM_MATRIX = 1, CKQ_GEMM_STREAM = 2 };
 void ckq_set_gemm_policy(int policy);
-/* Variants of the matrix-core GEMMs (tests, tuning; 0, the default, picks by shape).  Every variant of a format computes
+/* Variants of the matrix-core GEMMs (tests, tuning; 0, the default, picks by shape); 64, 96, 1 and 2 say which kernel runs where
+ * the policy above takes the GEMM, 16 also where it would stream.  Every variant of a format computes
  * the same sums in the same order: results are bit-identical wherever neither launch splits K or puts two wave groups
  * on a tile.
  *   CKQ_FMT_Q4_K: 64 or 96 = tiles of 128 rows x 64 tokens, or x 96 tokens - fewer instructions per token in blocks that run

@@ -184,6 +184,28 @@ def test_forced_policies_keep_their_kernels(L):
         L.ckq_set_gemm_policy(0)
 
 
+@pytest.mark.parametrize("fmt,variants", [("q4_k", (64, 96)), ("q5_k", (1, 2)), ("q6_k", (1, 2))])
+def test_forced_variants_keep_their_kernels(L, fmt, variants):
+    """A tile kernel that was asked for serves every size that the automatic policy takes off the streaming kernel; variant 16
+    sends everything from two tokens on (K up to 16384) to the 16-row tiles, in the order of the kernel they stand in for."""
+    tag = ckq.parity.FMT[fmt]
+    try:
+        for n, k in ROUTE_SHAPES:
+            for t in ROUTE_TOKENS:
+                L.ckq_set_prefill_variant(tag, 0)
+                auto = route(L, fmt, n, k, t)
+                for v in variants:
+                    L.ckq_set_prefill_variant(tag, v)
+                    assert route(L, fmt, n, k, t) == (TILES if auto in (TILES, ROWS16_TILES) else auto), (v, n, k, t)
+                L.ckq_set_prefill_variant(tag, 16)
+                if t >= 2 and k <= 16384:
+                    assert route(L, fmt, n, k, t) == (ROWS16_TILES if auto in (TILES, ROWS16_TILES) else ROWS16_STREAM), (n, k, t)
+                else:
+                    assert route(L, fmt, n, k, t) == auto
+    finally:
+        L.ckq_set_prefill_variant(tag, 0)
+
+
 def test_workspace_slot_bookkeeping(L):
     """Slot choice of the per-(device, stream, kind) scratch table of the K-split
     GEMMs: a known key finds its slot, a new key takes the first free slot, and
