@@ -280,8 +280,10 @@ int launch_gemm_q80_mfma_group(const void *A, const GemmGroupIn &in, int M, int 
     g.A = (const uint8_t *)A; g.M = M; g.nb = K / 32;
     if ((long long)g.nb * 34 * GEMM8_BN >= (1ll << 31)) return (int)hipErrorInvalidValue;
     g.ntt = (M + GEMM8_BM - 1) / GEMM8_BM;
-    bool dword_rows = true;
-    for (int p = 0; p < in.n; ++p) dword_rows = dword_rows && gemm_q80_dword_rows(g.nb, A, in.B[p]);
+    /* every matrix keeps the kernel, and with it the order of sums, of its single launch: of two kinds, no common launch */
+    const bool dword_rows = gemm_q80_dword_rows(g.nb, A, in.B[0]);
+    for (int p = 1; p < in.n; ++p)
+        if (gemm_q80_dword_rows(g.nb, A, in.B[p]) != dword_rows) return CKQ_ENOGROUP;
     if (dword_rows) return gemm_q80_dw_launch_group(g, in, s);
     return gemm_launch_grouped(gemm_q80_mfma_kernel<false>, g, in, s);
 }

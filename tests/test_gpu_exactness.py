@@ -495,6 +495,31 @@ def test_grouped_prefill_launch_equals_single_launches(fmt, K):
         L.ckq_set_gemm_policy(0)
 
 
+@pytest.mark.parametrize("offset", [(0, 2, 0), (2, 2, 2)])
+def test_grouped_q8_0_launch_of_mixed_alignment(offset):
+    """Q8_0 matrices that start on a dword and ones that do not, against the same activations as consecutive sequence entries:
+    each has the bits of its single launch (the two kernels add in different orders)."""
+    import torch
+    L = ckq.lib()
+    M, K, Ns = 500, 512, [1536, 640, 392]
+    xq = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, seed=331)), "q8_0", rows=M)
+    Ws = []
+    for i, (n, o) in enumerate(zip(Ns, offset)):
+        w = P.to_device(T.synth_weights("q8_0", n, K, seed=332 + i))
+        buf = torch.zeros(w.numel() + 4, dtype=torch.uint8, device="cuda")
+        buf[o:o + w.numel()] = w
+        Ws.append(buf[o:o + w.numel()])
+    ys = [torch.zeros(M * n, dtype=torch.float32, device="cuda") for n in Ns]
+    L.ckq_set_gemm_policy(1)
+    try:
+        say("grouped q8_0 launch, mixed alignment", offset)
+        P.dev_matmul_sequence([("q8_0", xq, W, None, y, M, n, K) for W, y, n in zip(Ws, ys, Ns)])
+        for W, y, n in zip(Ws, ys, Ns):
+            assert torch.equal(y, P.dev_gemm_nt("q8_0", xq, W, None, M, n, K).view(-1)), n
+    finally:
+        L.ckq_set_gemm_policy(0)
+
+
 def test_grouped_prefill_launch_two_wave_groups_and_fallback():
     """Q4_K, K = 2048: 168 tiles with eight K-steps take the two-wave-group form of the
     kernel (each single launch would be split along K instead, so the comparison is
@@ -614,16 +639,21 @@ def test_embedding_context_window_beyond_grid_y():
 
 
 def test_f32act_gemv_with_more_tokens_than_grid_y():
-    """The fp32-activation kernels take one token per launch row; 70 000 tokens
-    go out as two launches over consecutive token ranges."""
+    """The streaming fp32-activation kernels take one token per launch row; 70 000 tokens
+    go out as two launches over consecutive token ranges.  And the automatic choice."""
     fmt, N, K, M = "q8_0", 8, 64, 70000
     W = T.random_blocks(fmt, N * (K // 32), 81)
     A = T.normal(M * K, 0.0, 1.0, 82)
-    say("fp32-activation GEMM with 70 000 tokens")
-    got = P.dev_gemm_nt_f32act(fmt, P.to_device(A), P.to_device(W), None, M, N, K).cpu().numpy().reshape(M, N)
     want = T.oracle_gemm_nt_f32act(fmt, A, W, None, M, N, K)
-    assert T.norm_err(got, want) <= TOL
-    assert T.norm_err(got[65530:65540], want[65530:65540]) <= TOL
+    for policy in (2, 0):
+        say("fp32-activation GEMM with 70 000 tokens, policy", policy)
+        ckq.lib().ckq_set_gemm_policy(policy)
+        try:
+            got = P.dev_gemm_nt_f32act(fmt, P.to_device(A), P.to_device(W), None, M, N, K).cpu().numpy().reshape(M, N)
+        finally:
+            ckq.lib().ckq_set_gemm_policy(0)
+        assert T.norm_err(got, want) <= TOL
+        assert T.norm_err(got[65530:65540], want[65530:65540]) <= TOL
 
 
 # ---- Q4_K x Q8_K on 96-token tiles -------------------------------------------------------------------
