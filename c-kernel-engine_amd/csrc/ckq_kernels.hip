@@ -413,6 +413,18 @@ extern "C" int ckq_launch_gemv_group(int fmt, int n, float *const *y, const void
         }
         return 0;
     }
+    auto launch_some = [&](const int *which, int count) {
+        float *sy[CKQ_GROUP_MAX];
+        const void *sW[CKQ_GROUP_MAX], *sX[CKQ_GROUP_MAX];
+        const float *sb[CKQ_GROUP_MAX];
+        int srows[CKQ_GROUP_MAX];
+        long sld[CKQ_GROUP_MAX];
+        for (int i = 0; i < count; ++i) {
+            const int k = which[i];
+            sy[i] = y[k]; sW[i] = W[k]; sX[i] = X[k]; sb[i] = bias ? bias[k] : nullptr; srows[i] = rows[k]; sld[i] = ldys[k];
+        }
+        return ckq_launch_gemv_group(fmt, count, sy, sW, sX, sb, srows, sld, K, ntok, nullptr, stream);
+    };
     /* Matrices that the 16-row tiles take when launched alone share a launch of theirs, the others one of the streaming
      * kernel: every result keeps the bits of its single launch. */
     if (!subdots && (fmt == CKQ_FMT_Q4_K || fmt == CKQ_FMT_Q5_K || fmt == CKQ_FMT_Q6_K) && K % 256 == 0) {
@@ -426,18 +438,20 @@ extern "C" int ckq_launch_gemv_group(int fmt, int n, float *const *y, const void
                 rest[nrest++] = i;
         }
         if (r.n) {
-            int rc = launch_gemm_rows16(fmt, r, (hipStream_t)stream);
-            if (rc || !nrest) return rc;
-            float *ry[CKQ_GROUP_MAX];
-            const void *rW[CKQ_GROUP_MAX], *rX[CKQ_GROUP_MAX];
-            const float *rb[CKQ_GROUP_MAX];
-            int rrows[CKQ_GROUP_MAX];
-            long rld[CKQ_GROUP_MAX];
-            for (int i = 0; i < nrest; ++i) {
-                const int k = rest[i];
-                ry[i] = y[k]; rW[i] = W[k]; rX[i] = X[k]; rb[i] = bias ? bias[k] : nullptr; rrows[i] = rows[k]; rld[i] = ldys[k];
-            }
-            return ckq_launch_gemv_group(fmt, nrest, ry, rW, rX, rb, rrows, rld, K, ntok, nullptr, stream);
+            const int rc = launch_gemm_rows16(fmt, r, (hipStream_t)stream);
+            return rc || !nrest ? rc : launch_some(rest, nrest);
+        }
+    }
+    /* Q8_0 rows of an even number of blocks: matrices that start on a dword and ones that do not run different kernels */
+    if (!subdots && fmt == CKQ_FMT_Q8_0 && K % 64 == 0) {
+        int on[CKQ_GROUP_MAX], off[CKQ_GROUP_MAX], non = 0, noff = 0;
+        for (int i = 0; i < n; ++i) {
+            if ((uintptr_t)W[i] % 4 == 0) on[non++] = i;
+            else off[noff++] = i;
+        }
+        if (non && noff) {
+            const int rc = launch_some(on, non);
+            return rc ? rc : launch_some(off, noff);
         }
     }
     GemvArgs a = {};

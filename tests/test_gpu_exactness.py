@@ -501,7 +501,7 @@ def test_grouped_q8_0_launch_of_mixed_alignment(offset):
     each has the bits of its single launch (the two kernels add in different orders)."""
     import torch
     L = ckq.lib()
-    M, K, Ns = 500, 512, [1536, 640, 392]
+    M, K, Ns = 500, 4160, [1536, 640, 392]
     xq = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, seed=331)), "q8_0", rows=M)
     Ws = []
     for i, (n, o) in enumerate(zip(Ns, offset)):
@@ -512,10 +512,11 @@ def test_grouped_q8_0_launch_of_mixed_alignment(offset):
     ys = [torch.zeros(M * n, dtype=torch.float32, device="cuda") for n in Ns]
     L.ckq_set_gemm_policy(1)
     try:
-        say("grouped q8_0 launch, mixed alignment", offset)
-        P.dev_matmul_sequence([("q8_0", xq, W, None, y, M, n, K) for W, y, n in zip(Ws, ys, Ns)])
-        for W, y, n in zip(Ws, ys, Ns):
-            assert torch.equal(y, P.dev_gemm_nt("q8_0", xq, W, None, M, n, K).view(-1)), n
+        for m, k in ((M, 512), (4, 4160), (1, 4160)):
+            say("grouped q8_0 launch, mixed alignment", offset, m, k)
+            P.dev_matmul_sequence([("q8_0", xq, W, None, y, m, n, k) for W, y, n in zip(Ws, ys, Ns)])
+            for W, y, n in zip(Ws, ys, Ns):
+                assert torch.equal(y[:m * n], P.dev_gemm_nt("q8_0", xq, W, None, m, n, k).view(-1)), (m, n)
     finally:
         L.ckq_set_gemm_policy(0)
 
