@@ -637,8 +637,7 @@ int launch_rows16_nt(Rows16Args &a, hipStream_t s)
  * 10.8 -> 7.9, 10.9 -> 8.6, 12000 x 1024 at 32 / 96 9.8 -> 6.8, 19.0 -> 11.6, 4096 x 2048 at 96 12.0 -> 9.1; Q6_K 11008 x 2048
  * at 64 22.0 -> 16.4; Q4_K, whose planes are quickly formed, 12000 x 1024 at 64 11.1 -> 8.7.  It loses where the other's waves
  * have a SIMD to themselves anyway (Q4_K 1782 x 1536 at 43: 5.1 against 7.0) and for Q4_K rows of five blocks and more (11008 x 2048
- * at 32: 9.6 against 10.3).  Over 260 random shapes of 9 to 400 tokens, all routes: 1.036 on the geometric mean, the largest loss
- * 5.1 -> 6.1 (Q5_K 1172 x 768 at 208), the largest gain 12.0 -> 6.5 (Q6_K 3293 x 256 at 278). */
+ * at 32: 9.6 against 10.3). */
 int rows16_keep_parts(int fmt, long tiles, int groups, int nb, float *time)
 {
     if (nb > (fmt == CKQ_FMT_Q4_K ? 4 : KEEP_NB) || groups < 2 || tiles > 1 << 20 || groups > 1 << 10) return 0;
@@ -684,7 +683,7 @@ int launch_rows16(int fmt, Rows16Args &a, hipStream_t s)
     const int parts = rows16_keep_parts(fmt, tiles, (a.M + 15) / 16, a.nb, nullptr);
     if (parts) return a.tree ? launch_rows16_keep<F, true>(a, parts, s) : launch_rows16_keep<F, false>(a, parts, s);
     if (a.tree) return a.M <= 8 ? launch_rows16_nt<F, 8, true>(a, s) : launch_rows16_nt<F, 16, true>(a, s);
-    return a.M <= 8 ? launch_rows16_nt<F, 8, false>(a, s) : launch_rows16_nt<F, 16, false>(a, s);
+    return launch_rows16_nt<F, 16, false>(a, s);           /* the tile kernels start above eight tokens */
 }
 
 } // namespace

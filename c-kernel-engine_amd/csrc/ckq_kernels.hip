@@ -261,18 +261,28 @@ static bool weights_dword_aligned(const GemvArgs &a, const GemvGroup &grp)
 
 /* Whether the matrix-core kernel on 16-row tiles (ckq_gemm_rows16.hip) takes a matmul of `rows` rows (all matrices of a
  * launch) that would otherwise go to the tile kernels (`tiles`) or to the streaming kernel.  The results are the same bits
- * either way, so only time decides.  Fitted to launches of all three over 128..32000 rows, widths of 1024..11008 and 5..128
+ * either way, so only time decides.  Fitted to launches of all three over 128..16000 rows, widths of 256..11008 and 3..400
  * tokens (us; nb: 256-blocks of a row, mb: megabytes of weights, n16: thousands of 256-blocks of 16 rows times groups of 16
- * tokens); over all of them the rule's choices are within 1 % of always taking the faster:
+ * tokens); the rule's choices cost 0.3 % (against streaming) and 1.3 % (against the tiles) more than always taking the faster, single
+ * shapes up to a third (Q6_K 14911 x 1536 at 75 tokens: 22, tiles 17; Q4_K 4556 x 9984 at 30: 22, tiles 18):
  *   rows16     3.6 + 0.12 nb + (Q4_K 0.36, Q5_K 0.65, Q6_K 0.71) n16; up to 256 tokens of short rows gemm_rows16_keep_time
  *              (Q5_K 4864 x 1024 at 192 tokens: 10.3, tiles 13.7; 4096 x 2048 at 256: 17.2, tiles 19.5)
  *   tiles      11 + 0.2 mb + 0.0015 tokens mb, an under-estimate almost everywhere
- *   streaming  the larger of 4.35 + 0.07 nb (to eight tokens 3.5, where smaller tiles fill the chip: Q5_K 1024 x 2048 at 5
- *              4.5 -> 3.7 us, Q4_K 1024 x 1024 3.9 -> 3.6) and 3.05 + 0.11 nb + (0.24, 0.245, 0.29) mb for every eight tokens, 5 to 8 as 10
- * Three and four tokens, one pass of half the width, only move for long rows of large matrices (4096 x 11008 Q6_K:
- * 17.0 -> 13.4); two never do.  The forced policies keep their kernels: 1 the tile kernels, 2 the streaming kernel at any number of
- * tokens; and so does a tile kernel that the caller asked for.  Forced itself (ckq_launch_set_rows16) it goes before all of them, in
- * the order of the kernel that the policy asks for. */
+ *   streaming  above eight tokens the larger of 2.9 and 2.2 + 0.0075 lanes + (23.5, 23.5, 29) million lanes of all rows and passes,
+ *              a row's 64-element positions being dealt to 8, 16, 32 or 64 lanes or to 2 to 4 passes of 64 (stream_lanes): small
+ *              matrices stream at up to some 60 tokens (Q5_K 290 x 1792 at 25: 3.0, here 4.6; Q6_K 435 x 1536 at 13 3.0, here 4.8);
+ *              several matrices take a launch each; 5 to 8 tokens the larger of 3.5 + 0.07 nb and 3.05 + 0.11 nb + (0.24, 0.245, 0.29) mb for 10 tokens
+ * Three and four tokens, one pass of half the width, only move for long rows of large Q6_K matrices whose positions leave a
+ * tenth of those lanes idle (4096 x 11008 at 4: 14.2 -> 12.3, at 4 8192 x 4608 13.1 -> 11.4; but 4096 x 8192, no lane idle, 9.6 against
+ * 9.9, and Q5_K 4096 x 8192 7.6 against 9.5); two never do.  The forced policies keep their kernels: 1 the tile kernels, 2 the
+ * streaming kernel at any number of tokens; and so does a tile kernel that the caller asked for.  Forced itself
+ * (ckq_launch_set_rows16) it goes before all of them, in the order of the kernel that the policy asks for. */
+static int stream_lanes(int positions)
+{
+    for (int n : {8, 16, 32, 64, 128, 192})
+        if (positions <= n) return n;
+    return (positions + 255) / 256 * 256;
+}
 static std::atomic<int> g_rows16_forced{0};           /* bit per format tag */
 extern "C" void ckq_launch_set_rows16(int fmt, int on)
 {
@@ -280,7 +290,7 @@ extern "C" void ckq_launch_set_rows16(int fmt, int on)
     if (on) g_rows16_forced.fetch_or(1 << fmt);
     else g_rows16_forced.fetch_and(~(1 << fmt));
 }
-static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles)
+static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles, int launches = 1)
 {
     if (ntok < 2 || K > ROWS16_MAX_K) return false;
     if (g_rows16_forced.load(std::memory_order_relaxed) >> fmt & 1) return true;
@@ -288,14 +298,19 @@ static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles)
     const int f = fmt == CKQ_FMT_Q4_K ? 0 : fmt == CKQ_FMT_Q5_K ? 1 : 2;
     const bool tile_forced = f == 0 ? gemm_q4k_forced() : f == 1 ? gemm_q5k_forced() : gemm_q6k_forced();
     if (ntok < 3 || policy == 2 || (tiles && (policy == 1 || tile_forced))) return false;
-    static const float per_block[3] = {0.36f, 0.65f, 0.71f}, per_pass[3] = {0.24f, 0.245f, 0.29f};
+    static const float per_block[3] = {0.36f, 0.65f, 0.71f}, per_pass[3] = {0.24f, 0.245f, 0.29f}, per_lane[3] = {23.5f, 23.5f, 29.0f};
     const float nb = (float)(K / 256), mb = (float)rows * nb * (f == 0 ? 144e-6f : f == 1 ? 176e-6f : 210e-6f);
-    if (ntok <= 4) return K > 4096 && mb >= 20.0f;
-    const float passes = ntok <= 8 ? 1.25f : (float)((ntok + 7) / 8);
+    const int lanes = stream_lanes(K / 64);
+    if (ntok <= 4) return f == 2 && K > 4096 && mb >= 20.0f && 10 * lanes >= 11 * (K / 64);
     const float t_keep = ntok <= 256 ? gemm_rows16_keep_time(fmt, rows, ntok, K / 256) : 0.0f;
     const float t_rows = t_keep > 0.0f ? t_keep : 3.6f + 0.12f * nb + per_block[f] * 1e-3f * nb * (float)((rows + 15) / 16) * (float)((ntok + 15) / 16);
-    const float t_stream = 3.05f + 0.11f * nb + per_pass[f] * mb * passes, t_least = (ntok <= 8 ? 3.5f : 4.35f) + 0.07f * nb;
-    const float t_else = tiles ? 11.0f + (0.2f + 0.0015f * (float)ntok) * mb : t_stream > t_least ? t_stream : t_least;
+    float t_else;
+    if (tiles) t_else = 11.0f + (0.2f + 0.0015f * (float)ntok) * mb;
+    else if (ntok <= 8) t_else = fmaxf(3.5f + 0.07f * nb, 3.05f + 0.11f * nb + 1.25f * per_pass[f] * mb);
+    else {
+        const float t_launch = 2.2f + 0.0075f * (float)lanes;
+        t_else = fmaxf(2.9f, t_launch + per_lane[f] * 1e-6f * (float)rows * (float)lanes * (float)((ntok + 7) / 8)) + (float)(launches - 1) * t_launch;
+    }
     return t_rows < t_else;
 }
 
@@ -580,7 +595,7 @@ extern "C" int ckq_launch_gemm_group(int fmt, int n, float *const *C, const void
             tiles[p] = grouped || kquant_on_matrix_cores(fmt, M, (size_t)N[p], K);
             alike = alike && tiles[p] == tiles[0];
         }
-        if (alike && take_rows16(fmt, M, rows, K, tiles[0])) {
+        if (alike && take_rows16(fmt, M, rows, K, tiles[0], n)) {
             Rows16Args r = {};
             r.M = M; r.nb = K / 256; r.n = n; r.tree = !tiles[0];
             for (int p = 0; p < n; ++p)

@@ -206,6 +206,16 @@ def test_forced_variants_keep_their_kernels(L, fmt, variants):
         L.ckq_set_prefill_variant(tag, 0)
 
 
+@pytest.mark.parametrize("fmt,n,k,tokens,want", [
+    ("q5_k", 290, 1792, 25, STREAM), ("q6_k", 435, 1536, 13, STREAM), ("q4_k", 1024, 1024, 16, STREAM),
+    ("q5_k", 4096, 8192, 4, STREAM), ("q4_k", 4096, 11008, 4, STREAM), ("q6_k", 4096, 8192, 4, STREAM),
+    ("q6_k", 4096, 11008, 4, ROWS16_STREAM), ("q5_k", 5000, 1024, 24, ROWS16_STREAM), ("q4_k", 5345, 1280, 26, ROWS16_STREAM),
+    ("q6_k", 4096, 4096, 13, ROWS16_TILES), ("q5_k", 4864, 1024, 93, ROWS16_STREAM), ("q4_k", 11008, 4096, 512, TILES)])
+def test_16_row_tiles_where_they_are_the_faster_ones(L, fmt, n, k, tokens, want):
+    """Shapes at which the kernels were timed against each other; the faster one is taken."""
+    assert route(L, fmt, n, k, tokens) == want
+
+
 def test_workspace_slot_bookkeeping(L):
     """Slot choice of the per-(device, stream, kind) scratch table of the K-split
     GEMMs: a known key finds its slot, a new key takes the first free slot, and
