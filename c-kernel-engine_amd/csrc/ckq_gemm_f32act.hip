@@ -40,7 +40,8 @@
  * Grid: token groups fastest, so the blocks that share weights run side by side.
  * Bound: what a CU can load from L2 (8 KiB of activations and 64 rows of weights per wave and step) next to VALU issue
  * (per 64 elements 220-260 operations to cut x, shared by the R row tiles, and per row tile 211 / 226 / 123 for Q4_K / Q6_K /
- * Q8_0 to form the integers and apply the scales; the centring of Q4_K is about 60 of them: 96 x 4096 x 4096 23 -> 27 us).
+ * Q8_0 to form the integers and apply the scales; counted at 96 x 4096 x 4096 on 192 CUs, vector issue takes 78 / 61 / 44 % of their
+ * cycles and the matrix cores 24 / 16 / 16 %; the centring of Q4_K is about 60 of them: 96 x 4096 x 4096 23 -> 27 us).
  */
 #include "ckq_gemm_common.hpp"
 #include "ckq_gemm_f32act.hpp"

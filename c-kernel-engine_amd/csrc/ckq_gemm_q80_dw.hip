@@ -4,27 +4,24 @@
  *
  *   C[t][n] = sum_j dx(t,j) * (dw(n,j) * S(t,n,j))   (+ bias[n]),   S = the integer dot of 32-block j
  *
- * What bounds it: first, the copies.  Fetched block by block from 2-byte aligned addresses, as the other kernel has to, every
- * lane of a copy is a memory access of its own, and the copies alone take longer than the arithmetic.  Here rows travel as
- * they lie in memory, in dword-aligned 16-byte chunks, and are read where they are (image below): 177 us instead of 239 for
- * the copies of 2048 x 11008 x 4096 (109 if rows were whole cache lines).  Second, the scaling of the integers, which cannot be
- * summed over blocks before it:
+ * What bounds it: the scaling of the integers, which cannot be summed over blocks before it, once the copies are out of the way:
+ * - Fetched block by block from 2-byte aligned addresses, as the other kernel has to, every lane of a copy is a memory access of
+ *   its own and the requests bound the launch.  Here rows travel as they lie in memory, in dword-aligned 16-byte chunks, and are
+ *   read where they are (image below).
  * - v_mfma_i32_16x16x32_i8, K = 32 being one block, starts from the accumulator 0x4B400000, so that its result read as fp32 is
  *   exactly M + S (M = 1.5 * 2^23, |S| < 2^20).  t = fma(dw, M + S, -dw M) is dw S rounded once (dw M has 13 bits), and acc =
- *   fma(dx, t, acc): two plain fp32 operations per output and block.  Conversions and DPP operands (the other kernel's
- *   convert, product, multiply-add with a lane broadcast) issue at 5.4 cycles per wave, plain ones at 3.2; matrix
- *   instructions do not run under the VALU work of their SIMD but add to it (per wave and block 168 cycles of VALU, 128 of MFMA).
+ *   fma(dx, t, acc): two plain fp32 operations per output and block, against the other kernel's convert, product and
+ *   multiply-add with a lane broadcast.
  *   A row whose fp16 scale is infinite gives NaN that way; such outputs are summed again term by term at the end.
  * - Tokens are the A operand, weight rows the B operand: lane 16 q + i holds ONE weight row and tokens 4 q .. 4 q + 3 of a
  *   16 x 16 result.  LDS row 64 h + 16 g + i is weight row 64 h + 4 i + g, so a lane ends with four adjacent rows.
  * - K advances 128 (four blocks) per iteration, two stages.  Of the eight waves, four take two of the blocks and four the
  *   other two, each 64 rows x 32 tokens; the partial tiles are added through LDS at the end.  That gives a tile alone on its
- *   CU two waves per SIMD and two tiles four.  (32x32x32 instructions on 128 x 32 per wave, one block of two waves per SIMD and
- *   three stages need fewer operations and half again the time: 2048 x 11008 x 4096 517 us.)
+ *   CU two waves per SIMD and two tiles four.
  *
- * Measured, us, the other kernel -> this one: 333 tokens x 4864 x 4096 51.3 -> 38.0, 512 x 9728 x 896 35.6 -> 26.8, 2048 x 11008
- * x 4096 466 -> 325, 464 x 37134 x 2048 236 -> 161, 24 x 4864 x 4096 17.1 -> 15.3.  A block's iteration takes 2040 cycles, of
- * which issue 1730.
+ * Measured, us, the other kernel (weights two bytes off) -> this one: 333 tokens x 4864 x 4096 51.3 -> 37.8, 512 x 9728 x 896
+ * 34.7 -> 25.5, 2048 x 11008 x 4096 426 -> 322, 464 x 37134 x 2048 218 -> 154, 24 x 4864 x 4096 15.7 -> 13.9.  At 2048 tokens a block's
+ * iteration takes 1970 cycles of its CU, of which the vector instructions issue 1260 and the matrix instructions 510 (counters).
  *
  * Block = 8 waves = 64 tokens x 128 weight rows.
  */

@@ -401,9 +401,9 @@ gemm_rows16_kernel(const uint8_t *W, const uint8_t *X, int N, Rows16Shape S, flo
 
 /* Short rows, several token groups: a block has a wave for every 256-block of its 16 rows (at most KEEP_NB of them) and goes
  * through `per` groups of 16 tokens, the planes and scales of its weights formed once and kept in registers.  The kernel above
- * forms them again for every group, and they are half of what bounds it there, VALU issue (2 x 4864 x 1024, Q5_K,
- * 93 tokens: 587 operations a wave for a 256-block and group, 78 % of the busy cycles; 21 us, here 15).  The terms and their order are
- * the same. */
+ * forms them again for every group, and they are a good third of what bounds it there, VALU issue (Q5_K, 93 tokens: 480 vector
+ * instructions a 256-block and group at 1024 x 4864, 64 % of the busy CUs' issue cycles; here 301 and 63 % at 2 x 4864 x 1024, which took
+ * 20.9 us in the kernel above and takes 15.1).  The terms and their order are the same. */
 constexpr int KEEP_NB = 8;
 template <class F> constexpr int rows16_keep_wave_lds() { return 16 * (F::PITCH > 288 ? F::PITCH : 288); }
 template <class F, bool TREE, bool GRP>

@@ -52,7 +52,9 @@ extern "C" void ckq_launch_set_gemm_policy(int policy) { g_gemm_policy.store(pol
  * loads), matrix cores max(14, 9 + MB / 2.5).  LM head 151936x896 (145 MB):
  * 9-16 tokens stream (63-66 us against 67-69), 17 and more go to the matrix
  * cores (89 against 69); 4864x896 (4.6 MB) streams up to 72 tokens (64 tokens:
- * 11.8 us against 15.3). */
+ * 11.8 us against 15.3).  The matrix-core side is that of ckq_gemm_q80.hip; rows on
+ * dwords run the faster ckq_gemm_q80_dw.hip (24 tokens, 4864x4096: 15.7 -> 13.9), so
+ * for them the line lies on the late side. */
 static bool gemm_q80_on_matrix_cores(int ntok, size_t weight_bytes, bool aligned_rows)
 {
     const int policy = g_gemm_policy.load(std::memory_order_relaxed);
@@ -358,8 +360,8 @@ static const GemvGroup k_no_group = {{}, {}, {}, {}, {}, {}, 1};
 
 static int launch_gemv_args(int fmt, GemvArgs &a, const GemvGroup &grp, int K, void *stream, const GemmOpts &opts = GemmOpts{});
 
-/* `subdots`, when non-NULL, selects the dump build of the instantiation the
- * same call would run without it: out[(t * nrows + row) * nsub + i], nothing
+/* `subdots`, when non-NULL, selects the dump build of the streaming kernel's
+ * instantiation for these sizes: out[(t * nrows + row) * nsub + i], nothing
  * is written to y. */
 extern "C" int ckq_launch_gemv(int fmt, float *y, const void *W, const void *X, const float *bias,
                                int nrows, int K, int ntok, long ldy, int row0, int row1,

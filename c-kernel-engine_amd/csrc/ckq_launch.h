@@ -40,8 +40,10 @@ extern "C" {
  * `row0`/`row1` restrict the computed rows to [row0,row1) (thread-split entry
  * points); outputs outside the range are not touched.
  * `subdots`, when non-NULL (at most eight tokens), runs the dump build of the
- * instantiation the call would otherwise run and receives the raw integer
- * sub-block dots, subdots[(t * nrows + row) * nsub + i]; y is not written.
+ * streaming kernel's instantiation for these sizes and receives the raw integer
+ * sub-block dots, subdots[(t * nrows + row) * nsub + i]; y is not written.  (The
+ * 16-row tiles, which some K-quant calls of three to eight tokens run instead,
+ * have the streaming kernel's bits and no dump of their own.)
  */
 int ckq_launch_gemv(int fmt, float *y, const void *W, const void *X, const float *bias,
                     int nrows, int K, int ntok, long ldy, int row0, int row1,
@@ -50,7 +52,9 @@ int ckq_launch_gemv(int fmt, float *y, const void *W, const void *X, const float
 /* n (at most 4) independent matmuls of one format, input width and token count
  * (at most eight tokens; a token tile that does not fit in LDS is issued as
  * separate launches), problem i with rows[i] weight rows and output row stride
- * ldys[i], in one launch of the streaming kernel; the arrays are host arrays
+ * ldys[i], in one launch of the streaming kernel (K-quant matrices that run on
+ * the 16-row tiles when launched alone share one of those, and Q8_0 matrices on
+ * and off dword boundaries have a launch each); the arrays are host arrays
  * (of device pointers), bias may be NULL or hold NULL entries.  `subdots`
  * non-NULL runs the dump build of the grouped kernel instead (y, ldys and bias
  * are then ignored): subdots[((g * ntok + t) * max_rows + row) * nsub + i]. */
@@ -59,7 +63,7 @@ int ckq_launch_gemv_group(int fmt, int n, float *const *y, const void *const *W,
                           int32_t *subdots, void *stream);
 
 /* n (2..4) weight matrices of one format against the same M x K quantized activations as one
- * matrix-core launch; CKQ_ENOGROUP when the matrices should be launched one by one instead. */
+ * matrix-core launch (tile kernels or 16-row tiles); CKQ_ENOGROUP when the matrices should be launched one by one instead. */
 int ckq_launch_gemm_group(int fmt, int n, float *const *C, const void *const *B, const void *A,
                           const float *const *bias, const int *N, const long *ldc, int K, int M, void *stream);
 

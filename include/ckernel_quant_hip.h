@@ -330,8 +330,9 @@ int ckq_matmul_sequence_dev(const ckq_matmul_op *ops, int nops, int repeat, void
 int ckq_subblock_dots_dev(int fmt, int32_t *out, const void *W, const void *x_q8, int M, int K, void *stream);
 
 /* The same dump for up to eight tokens, taken from the instantiation of the
- * streaming kernel that ckq_gemm_nt_dev would run for this shape and token
- * count (token tile, rows per wave, block size, staged activations):
+ * streaming kernel for this shape and token count (token tile, rows per wave,
+ * block size, staged activations), which ckq_gemm_nt_dev runs too, or a kernel
+ * with the same bits (16-row tiles, K-quants of three and more tokens):
  * out[(t * M + row) * (K/sub) + i]. */
 int ckq_subblock_dots_tokens_dev(int fmt, int32_t *out, const void *W, const void *X_q8, int M, int K, int ntok, void *stream);
 /* And from the grouped launch of n (2..4) matmuls of one format, input width
