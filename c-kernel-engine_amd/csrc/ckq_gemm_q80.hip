@@ -280,10 +280,14 @@ int launch_gemm_q80_mfma_group(const void *A, const GemmGroupIn &in, int M, int 
     g.A = (const uint8_t *)A; g.M = M; g.nb = K / 32;
     if ((long long)g.nb * 34 * GEMM8_BN >= (1ll << 31)) return (int)hipErrorInvalidValue;
     g.ntt = (M + GEMM8_BM - 1) / GEMM8_BM;
-    /* every matrix keeps the kernel, and with it the order of sums, of its single launch: of two kinds, no common launch */
-    const bool dword_rows = gemm_q80_dword_rows(g.nb, A, in.B[0]);
-    for (int p = 1; p < in.n; ++p)
-        if (gemm_q80_dword_rows(g.nb, A, in.B[p]) != dword_rows) return CKQ_ENOGROUP;
-    if (dword_rows) return gemm_q80_dw_launch_group(g, in, s);
-    return gemm_launch_grouped(gemm_q80_mfma_kernel<false>, g, in, s);
+    /* every matrix keeps the kernel, and with it the order of sums, of its single launch: of two kinds, two launches (still
+     * without a K split, so that a group never needs scratch) */
+    GemmGroupIn kind[2] = {};
+    for (int p = 0; p < in.n; ++p) {
+        GemmGroupIn &k = kind[gemm_q80_dword_rows(g.nb, A, in.B[p])];
+        k.B[k.n] = in.B[p]; k.bias[k.n] = in.bias[p]; k.C[k.n] = in.C[p]; k.N[k.n] = in.N[p]; k.ldc[k.n] = in.ldc[p];
+        ++k.n;
+    }
+    const int rc = kind[1].n ? gemm_q80_dw_launch_group(g, kind[1], s) : 0;
+    return rc || !kind[0].n ? rc : gemm_launch_grouped(gemm_q80_mfma_kernel<false>, g, kind[0], s);
 }
