@@ -31,20 +31,26 @@
  * the lane's share of the group's sum of x against the row's factor, both cut in three.
  *
  * Block = 8 waves on one tile of 32 tokens x 32 R weight rows; the waves cut K into eight contiguous runs and add
- * their partial tiles through LDS, in pairs.  Each wave loads its own activations one step ahead, 256 contiguous bytes
- * per token, and turns them through LDS (a lane loading its own row would touch 64 cache lines per instruction: 40 us
+ * their partial tiles through LDS, in pairs.  Each wave loads its own activations one step (Q4_K) or half a step ahead, a
+ * contiguous run per token, and turns them through LDS (a lane loading its own row would touch 64 cache lines per instruction: 40 us
  * instead of 36 at 96 x 4096 x 4096, Q6_K; one token per pass over the weights, as the streaming kernel does it, 245 us);
  * no other wave reads them, so the loop has no barrier.  Cutting the activations in a launch of its own and reading the
- * parts back (6 bytes per element instead of 4) was slower: 41 us.
+ * parts back (6 bytes per element instead of 4) gains what the launch costs.
+ *
+ * Weights.  The address path takes a wave's load in 16 to 22 cycles where quads of lanes read adjacent bytes, in 64 where every lane
+ * has a row of its own, and in 160 where the rows' bytes are not on dwords either (measured, 16 bytes a lane, L2).  Q6_K
+ * and Q8_0, whose blocks are only 2-byte aligned, therefore come in memory order like the activations (gemm_f32run_kernel, 96 x 4096 x
+ * 4096: Q6_K 36.1 -> 31.7 us, Q8_0 36.3 -> 28.2, same bits; 40 shapes of 1..158 tokens 1.03 on average).  Q4_K, 16-byte
+ * aligned and two loads a step, loses that way (27.5 -> 29.3) and keeps its own loads (gemm_f32act_q4k_kernel).
  *
  * Grid: token groups fastest, so the blocks that share weights run side by side.
- * Bound: what a CU can load from L2 (8 KiB of activations and 64 rows of weights per wave and step) next to VALU issue
- * (per 64 elements 220-260 operations to cut x, shared by the R row tiles, and per row tile 211 / 226 / 123 for Q4_K / Q6_K /
- * Q8_0 to form the integers and apply the scales; counted at 96 x 4096 x 4096 on 192 CUs, vector issue takes 78 / 61 / 44 % of their
- * cycles and the matrix cores 24 / 16 / 16 %; the centring of Q4_K is about 60 of them: 96 x 4096 x 4096 23 -> 27 us).
+ * Bound: VALU issue: per 64 elements 220-260 operations to cut x, shared by the R row tiles, and per row tile some 210 / 230 / 130 for
+ * Q4_K / Q6_K / Q8_0 to form the integers and apply the scales, half of them at half rate (conversions, byte permutes); the matrix
+ * cores are busy a quarter of the time.  The centring of Q4_K is about 60 of them: 96 x 4096 x 4096 23 -> 27 us.
  */
 #include "ckq_gemm_common.hpp"
 #include "ckq_gemm_f32act.hpp"
+#include <type_traits>
 
 namespace {
 
@@ -110,26 +116,27 @@ __device__ __forceinline__ ckq_v4i bytes_to_bf16(u32 b0, u32 b1)
 
 /* ---- formats ------------------------------------------------------------------------------------
  * STEP elements of K per step, NG scale groups of 8 * NK elements per lane half in it.
- *   Raw / load      the step's bytes of one weight row that this lane's half decodes
- *   src_elem(c)     first element of 16-byte chunk c (0..15) of the step's activations
- *   chunk(g, h, i)  which chunk holds floats 4 i .. 4 i + 3 of group g for lane half h
+ *   Raw / load      the step's bytes of one weight row that this lane's half decodes: Q4_K from memory, the others from LDS
+ *   src_elem(c)     first element of 16-byte chunk c of the activations: of the step (Q4_K, 16 chunks), of its phase p (8)
+ *   chunk(g, h, i)  (Q4_K) which chunk holds floats 4 i .. 4 i + 3 of group g for lane half h
+ *   RUN, BYTES      steps of a run of weights in LDS and its bytes; LANES lanes bring a row's, one row is PITCH bytes from the next;
+ *                   SHIFT: they come from the dword they start in and are shifted into place
  *   operand(g, i)   bf16x8 of the lane's elements 8 i .. 8 i + 7 of group g
  *   scale(g)        fp32 factor of the group; MIN: rest(g), the factor of the group's sum of x
  *   weight(blk, e, i)  element e + i of a block, e a multiple of 16 and i below 16, for exact_output */
 struct F32Q4K {
-    static constexpr int STEP = 64, NG = 2, NK = 2;
-    static constexpr bool MIN = true;
+    static constexpr int STEP = 64, NK = 2;
     struct Raw { u32 hdr[4], qs[4]; };
-    static __device__ __forceinline__ void load(Raw &w, const uint8_t *row, int step, int h, int)
+    static __device__ __forceinline__ void load(Raw &w, const uint8_t *row, int step, int h)
     {
         const uint8_t *blk = row + (u32)(step >> 2) * 144u;
         ld16<4>(w.hdr, blk);
         ld16<4>(w.qs, blk + 16 + 32 * (step & 3) + 16 * h);
     }
-    static __device__ __forceinline__ u32 src_elem(int step, int c, int) { return 64u * (u32)step + 4u * c; }
+    static __device__ __forceinline__ u32 src_elem(int step, int c) { return 64u * (u32)step + 4u * c; }
     static __device__ __forceinline__ int chunk(int g, int h, int i) { return 8 * g + 4 * h + i; }
     struct Dec { float s[2], rest[2]; u32 off[2]; };          /* off: 128 - c in every byte */
-    static __device__ __forceinline__ void decode(Dec &d, const Raw &w, int step, int)
+    static __device__ __forceinline__ void decode(Dec &d, const Raw &w, int step)
     {
         u32 sc2, mn2;
         k4_scale_pair(w.hdr[1], w.hdr[2], w.hdr[3], step & 3, &sc2, &mn2);
@@ -169,23 +176,26 @@ struct F32Q4K {
 
 struct F32Q6K {
     static constexpr int STEP = 64, NG = 4, NK = 1;       /* a step: 16-runs o of the four 32-runs of one 128-half n */
-    static constexpr bool MIN = false;
+    static constexpr int RUN = 4, BYTES = 210, LANES = 16, PITCH = 240;
+    static constexpr bool SHIFT = true;
     struct Raw { u32 ql0[2], ql1[2], qh[2], sc[2], d; };
-    static __device__ __forceinline__ void load(Raw &w, const uint8_t *row, int step, int h, int)
+    static __device__ __forceinline__ void load(Raw &w, const uint8_t *row, int step, int h)
     {
-        const uint8_t *blk = row + (u32)(step >> 2) * 210u;
         const int n = (step >> 1) & 1, o = step & 1;
-        ld8<2>(w.ql0, blk + 64 * n + 16 * o + 8 * h);
-        ld8<2>(w.ql1, blk + 64 * n + 32 + 16 * o + 8 * h);
-        ld8<2>(w.qh, blk + 128 + 32 * n + 16 * o + 8 * h);
-        ld8<2>(w.sc, blk + 192 + 8 * n);
-        w.d = ld2(blk + 208);
+        auto two = [&](u32 *d, int ofs) {
+            const int2 v = *reinterpret_cast<const int2 *>(row + ofs);
+            d[0] = (u32)v.x; d[1] = (u32)v.y;
+        };
+        two(w.ql0, 64 * n + 16 * o + 8 * h);
+        two(w.ql1, 64 * n + 32 + 16 * o + 8 * h);
+        two(w.qh, 128 + 32 * n + 16 * o + 8 * h);
+        two(w.sc, 192 + 8 * n);
+        w.d = *reinterpret_cast<const u32 *>(row + 208) & 0xffffu;
     }
-    static __device__ __forceinline__ u32 src_elem(int step, int c, int)
+    static __device__ __forceinline__ u32 src_elem(int step, int p, int c, int)
     {
-        return 128u * (u32)(step >> 1) + 16u * (step & 1) + 32u * (c >> 2) + 4u * (c & 3);
+        return 128u * (u32)(step >> 1) + 16u * (step & 1) + 32u * (u32)(2 * p + (c >> 2)) + 4u * (u32)(c & 3);
     }
-    static __device__ __forceinline__ int chunk(int g, int h, int i) { return 4 * g + 2 * h + i; }
     struct Dec { float s[4]; };
     static __device__ __forceinline__ void decode(Dec &d, const Raw &w, int step, int)
     {
@@ -219,22 +229,28 @@ struct F32Q6K {
 
 struct F32Q80 {
     static constexpr int STEP = 64, NG = 2, NK = 2;       /* two 32-blocks; the second is missing in the last step of an odd count */
-    static constexpr bool MIN = false;
+    static constexpr int RUN = 2, BYTES = 136, LANES = 9, PITCH = 144;
+    static constexpr bool SHIFT = false;
     struct Raw { u32 q[2][4]; u32 d[2]; };
-    static __device__ __forceinline__ void load(Raw &w, const uint8_t *row, int step, int h, int K)
+    static __device__ __forceinline__ void load(Raw &w, const uint8_t *row, int step, int h)
     {
+        /* quants of block j start at byte 34 j + 2: two aligned reads around them */
+        auto block = [&](auto jc) __attribute__((always_inline)) {
+            constexpr int j = decltype(jc)::value, first = (34 * j + 2) / 4, base = first & ~3, sh = (34 * j + 2) & 2, g = j & 1;
+            const ckq_v4i a = *reinterpret_cast<const ckq_v4i *>(row + 4 * base + 16 * h), b = *reinterpret_cast<const ckq_v4i *>(row + 4 * base + 16 + 16 * h);
+            auto dw = [&](int i) { return (u32)(i < 4 ? a[i] : b[i - 4]); };
 #pragma unroll
-        for (int g = 0; g < 2; ++g) {
-            const uint8_t *blk = row + (u32)min(2 * step + g, K / 32 - 1) * 34u;
-            w.d[g] = ld2(blk);
-            ld16<2>(w.q[g], blk + 2 + 16 * h);
-        }
+            for (int i = 0; i < 4; ++i) {
+                const int k = first - base + i;
+                w.q[g][i] = sh ? __builtin_amdgcn_alignbyte(dw(k + 1), dw(k), 2) : dw(k);
+            }
+            const u32 d = *reinterpret_cast<const u32 *>(row + ((34 * j) & ~3));
+            w.d[g] = (34 * j) & 2 ? d >> 16 : d & 0xffffu;
+        };
+        if (step & 1) { block(std::integral_constant<int, 2>{}); block(std::integral_constant<int, 3>{}); }
+        else          { block(std::integral_constant<int, 0>{}); block(std::integral_constant<int, 1>{}); }
     }
-    static __device__ __forceinline__ u32 src_elem(int step, int c, int K)
-    {
-        return 32u * (u32)min(2 * step + (c >> 3), K / 32 - 1) + 4u * (c & 7);
-    }
-    static __device__ __forceinline__ int chunk(int g, int h, int i) { return 8 * g + 4 * h + i; }
+    static __device__ __forceinline__ u32 src_elem(int step, int p, int c, int K) { return 32u * (u32)min(2 * step + p, K / 32 - 1) + 4u * (u32)c; }
     struct Dec { float s[2]; };
     static __device__ __forceinline__ void decode(Dec &d, const Raw &w, int step, int K)
     {
@@ -263,11 +279,13 @@ __device__ __forceinline__ float exact_output(const uint8_t *w, const float *x, 
     return sum;
 }
 
-template <class F, int R>
+/* Q4_K */
+template <int R>
 __global__ void __launch_bounds__(64 * F32_WAVES, 2)
-gemm_f32act_kernel(const float *__restrict__ A, const uint8_t *__restrict__ B, const float *__restrict__ bias, float *__restrict__ C,
+gemm_f32act_q4k_kernel(const float *__restrict__ A, const uint8_t *__restrict__ B, const float *__restrict__ bias, float *__restrict__ C,
                    int M, int N, int K, long wrow, long ldc, int ntg)
 {
+    typedef F32Q4K F;
     /* a wave's activations of one step, token t at 256 t, chunk c in slot c ^ (t & 15); at the end the partial tiles */
     __shared__ __attribute__((aligned(16))) uint8_t xs_all[F32_WAVES][32 * 256];
     const int lane = threadIdx.x & 63, wave = wave_in_block();
@@ -294,9 +312,9 @@ gemm_f32act_kernel(const float *__restrict__ A, const uint8_t *__restrict__ B, c
     ckq_v4i xn[8];
     auto fetch = [&](int s) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) xn[j] = *reinterpret_cast<const ckq_v4i *>(xsrc[j] + F::src_elem(s, lane & 15, K));
+        for (int j = 0; j < 8; ++j) xn[j] = *reinterpret_cast<const ckq_v4i *>(xsrc[j] + F::src_elem(s, lane & 15));
 #pragma unroll
-        for (int r = 0; r < R; ++r) F::load(wn[r], wr[r], s, half, K);
+        for (int r = 0; r < R; ++r) F::load(wn[r], wr[r], s, half);
     };
     auto take = [&]() {
 #pragma unroll
@@ -310,10 +328,9 @@ gemm_f32act_kernel(const float *__restrict__ A, const uint8_t *__restrict__ B, c
     auto compute = [&](int s) {
         typename F::Dec dec[R];
 #pragma unroll
-        for (int r = 0; r < R; ++r) F::decode(dec[r], w[r], s, K);
-        /* two groups at a time: their two terms are added before they meet the sum so far */
-#pragma unroll
-        for (int g0 = 0; g0 < F::NG; g0 += 2) {
+        for (int r = 0; r < R; ++r) F::decode(dec[r], w[r], s);
+        /* the step's two groups: their two terms are added before they meet the sum so far */
+        {
             Cut c[2][F::NK];
             ckq_v4i pa[2];
 #pragma unroll
@@ -321,7 +338,7 @@ gemm_f32act_kernel(const float *__restrict__ A, const uint8_t *__restrict__ B, c
                 float x[F::NK * 8];
 #pragma unroll
                 for (int i = 0; i < 2 * F::NK; ++i) {
-                    const ckq_v4i v = *reinterpret_cast<const ckq_v4i *>(xs + 256 * col + 16 * (F::chunk(g0 + g, half, i) ^ (col & 15)));
+                    const ckq_v4i v = *reinterpret_cast<const ckq_v4i *>(xs + 256 * col + 16 * (F::chunk(g, half, i) ^ (col & 15)));
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
                         const int e = v[j];
@@ -330,7 +347,7 @@ gemm_f32act_kernel(const float *__restrict__ A, const uint8_t *__restrict__ B, c
                 }
 #pragma unroll
                 for (int k = 0; k < F::NK; ++k) cut8(x + 8 * k, c[g][k]);
-                if constexpr (F::MIN) {
+                {
                     /* this half's share of the group's sum of x, cut in three; against the cut rest of the min, the six
                      * products that matter in one MFMA, which also adds the halves */
                     const float p = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7])) +
@@ -341,28 +358,25 @@ gemm_f32act_kernel(const float *__restrict__ A, const uint8_t *__restrict__ B, c
             }
 #pragma unroll
             for (int r = 0; r < R; ++r) {
-                ckq_v16f two, sum;
-                if constexpr (F::MIN) {
-                    two = zero;
+                ckq_v16f two = zero, sum;
 #pragma unroll
-                    for (int g = 0; g < 2; ++g) {
-                        const float h = dec[r].rest[g0 + g], m = h - top16(h), l = m - top16(m);
-                        two = mfma_bf16(pa[g], ckq_v4i{(int)pack_bf16(h, m), (int)pack_bf16(h, m), (int)pack_bf16(l, h), 0}, two);
-                    }
+                for (int g = 0; g < 2; ++g) {
+                    const float h = dec[r].rest[g], m = h - top16(h), l = m - top16(m);
+                    two = mfma_bf16(pa[g], ckq_v4i{(int)pack_bf16(h, m), (int)pack_bf16(h, m), (int)pack_bf16(l, h), 0}, two);
                 }
 #pragma unroll
                 for (int g = 0; g < 2; ++g) {
                     sum = zero;
 #pragma unroll
                     for (int k = 0; k < F::NK; ++k) {
-                        const ckq_v4i b = F::operand(w[r], dec[r], g0 + g, k);
+                        const ckq_v4i b = F::operand(w[r], dec[r], g, k);
                         sum = mfma_bf16(c[g][k].lo, b, sum);
                         sum = mfma_bf16(c[g][k].mid, b, sum);
                         sum = mfma_bf16(c[g][k].hi, b, sum);
                     }
 #pragma unroll
                     for (int i = 0; i < 16; ++i)
-                        two[i] = F::MIN || g ? fmaf(dec[r].s[g0 + g], sum[i], F::MIN && !g ? -two[i] : two[i]) : dec[r].s[g0 + g] * sum[i];
+                        two[i] = fmaf(dec[r].s[g], sum[i], g ? two[i] : -two[i]);
                 }
 #pragma unroll
                 for (int i = 0; i < 16; ++i) acc[r][i] += two[i];
@@ -418,6 +432,218 @@ gemm_f32act_kernel(const float *__restrict__ A, const uint8_t *__restrict__ B, c
     }
 }
 
+template <class F, int R>
+__global__ void __launch_bounds__(64 * F32_WAVES, 2)
+gemm_f32run_kernel(const float *__restrict__ A, const uint8_t *__restrict__ B, const float *__restrict__ bias, float *__restrict__ C,
+                   int M, int N, int K, long wrow, long ldc, int ntg)
+{
+    constexpr int ROWS = 32 * R, RPI = 64 / F::LANES, NWL = (ROWS + RPI - 1) / RPI;      /* rows per load instruction, instructions per run */
+    constexpr int WLDS = ROWS * F::PITCH, XLDS = 32 * 128, RED = F32_WAVES * (R < 2 ? 1 : 2) * 16 * 64 * 4;
+    /* of each wave: the weights of a run, and the activations of a phase, token t at 128 t, chunk c in slot c ^ (t / 2 % 8); at
+     * the end the partial tiles */
+    __shared__ __attribute__((aligned(16))) uint8_t smem[F32_WAVES * (WLDS + XLDS) > RED ? F32_WAVES * (WLDS + XLDS) : RED];
+    const int lane = threadIdx.x & 63, wave = wave_in_block();
+    const int col = lane & 31, half = lane >> 5;
+    const int t0 = (int)(blockIdx.x % (u32)ntg) * 32, n0 = (int)(blockIdx.x / (u32)ntg) * ROWS;
+    const int steps = (K + F::STEP - 1) / F::STEP, per = (steps + F32_WAVES - 1) / F32_WAVES;
+    const int s0 = wave * per, s1 = min(steps, s0 + per);
+    uint8_t *const wl = smem + wave * (WLDS + XLDS), *const xs = wl + WLDS;
+
+    /* weights: row and chunk of this lane in load instruction j */
+    const int w_row = lane / F::LANES, w_chunk = lane % F::LANES;
+    const uint8_t *const wbase = B + (size_t)n0 * (size_t)wrow;
+    const int left = N - 1 - n0;
+    const u32 row_bytes = (u32)wrow, par = (u32)(uintptr_t)wbase & 2u;
+    ckq_v4i wn[NWL];
+    auto run_bytes = [&](int run) { return min((u32)F::BYTES, row_bytes - (u32)run * (u32)F::BYTES); };
+    auto w_src = [&](int j, int run) {
+        int r = RPI * j + min(w_row, RPI - 1);
+        asm volatile("" : "+v"(r));                          /* formed when it is needed, not kept for every j */
+        return (size_t)min(r, left) * row_bytes + (u32)run * (u32)F::BYTES;
+    };
+    auto fetch_w = [&](int run) {
+#pragma unroll
+        for (int j = 0; j < NWL; ++j) {
+            u32 t[4];
+            if constexpr (F::SHIFT) {
+                /* from the dword the block starts in; the last chunk from byte 196 of it, so that no load passes the dword the block ends in */
+                ld16<4>(t, wbase - par + (((w_src(j, run) + par) & ~(size_t)3) + (u32)(w_chunk < 13 ? 16 * w_chunk : 196)));
+            } else ld16<2>(t, wbase + (w_src(j, run) + min(16u * (u32)w_chunk, run_bytes(run) - 16u)));
+            wn[j] = ckq_v4i{(int)t[0], (int)t[1], (int)t[2], (int)t[3]};
+        }
+    };
+    auto take_w = [&](int run) {
+#pragma unroll
+        for (int j = 0; j < NWL; ++j) {
+            const int row = RPI * j + w_row;
+            uint8_t *const d = wl + row * F::PITCH;
+            const bool on = w_row < RPI && row < ROWS;
+            if constexpr (F::SHIFT) {
+                const u32 sh = ((u32)w_src(j, run) + par) & 2u;
+                u32 v[5];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = (u32)wn[j][i];
+                /* the neighbour's first dword; lane 13 holds dwords 49 .. 52 of the block's 53 */
+                v[4] = (u32)dpp_get<0x101>((int)(w_chunk == 13 ? v[3] : v[0]));
+                ckq_v4i o;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[i] = (int)__builtin_amdgcn_alignbyte(v[i + 1], v[i], sh);
+                if (on && w_chunk < 13) *reinterpret_cast<ckq_v4i *>(d + 16 * w_chunk) = o;
+                if (on && w_chunk == 13) *reinterpret_cast<u32 *>(d + 208) = v[3] >> (8 * sh);
+            } else if (run_bytes(run) == (u32)F::BYTES) {
+                if (on && 16 * w_chunk + 16 <= F::BYTES) *reinterpret_cast<ckq_v4i *>(d + 16 * w_chunk) = wn[j];
+                else if (on) *reinterpret_cast<int2 *>(d + 16 * w_chunk) = int2{wn[j][2], wn[j][3]};         /* the last 16 of 136 bytes */
+            } else if (on) {
+                uint16_t *const e = reinterpret_cast<uint16_t *>(d + min(16u * (u32)w_chunk, run_bytes(run) - 16u));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    e[2 * i] = (uint16_t)((u32)wn[j][i] & 0xffffu);
+                    e[2 * i + 1] = (uint16_t)((u32)wn[j][i] >> 16);
+                }
+            }
+        }
+        __builtin_amdgcn_wave_barrier();                     /* the wave's own LDS accesses stay in this order */
+    };
+
+    const float *xsrc[4];          /* row of the token this lane fetches in load instruction j */
+#pragma unroll
+    for (int j = 0; j < 4; ++j) xsrc[j] = A + (size_t)min(t0 + 8 * j + (lane >> 3), M - 1) * (size_t)K;
+    ckq_v4i xn[4];
+    auto fetch_x = [&](int s, int p) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) xn[j] = *reinterpret_cast<const ckq_v4i *>(xsrc[j] + F::src_elem(s, p, lane & 7, K));
+    };
+    auto take_x = [&]() {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int t = 8 * j + (lane >> 3);
+            *reinterpret_cast<ckq_v4i *>(xs + 128 * t + 16 * ((lane & 7) ^ (t >> 1 & 7))) = xn[j];
+        }
+        __builtin_amdgcn_wave_barrier();
+    };
+
+    ckq_v16f acc[R], two[R], zero;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) zero[i] = 0.0f;
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = two[r] = zero;
+
+    if (s0 < s1) {
+        fetch_w(s0 / F::RUN);
+        fetch_x(s0, 0);
+    }
+    for (int s = s0; s < s1; ++s) {
+        if (s == s0 || s % F::RUN == 0) {
+            take_w(s / F::RUN);
+            if ((s / F::RUN + 1) * F::RUN < s1) fetch_w(s / F::RUN + 1);
+        }
+        typename F::Raw w[R];
+        typename F::Dec dec[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            F::load(w[r], wl + (32 * r + col) * F::PITCH, s, half);
+            F::decode(dec[r], w[r], s, K);
+        }
+        /* two phases of 32 elements a token: a scale group each, or two groups of 16 */
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            constexpr int NG = F::NG / 2;                    /* groups of a phase */
+            take_x();
+            if (p == 0) fetch_x(s, 1);
+            else if (s + 1 < s1) fetch_x(s + 1, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            Cut c[NG][F::NK];
+#pragma unroll
+            for (int g = 0; g < NG; ++g) {
+                float x[F::NK * 8];
+#pragma unroll
+                for (int i = 0; i < 2 * F::NK; ++i) {
+                    const int ch = NG == 1 ? 4 * half + i : 4 * g + 2 * half + i;
+                    const ckq_v4i v = *reinterpret_cast<const ckq_v4i *>(xs + 128 * col + 16 * (ch ^ (col >> 1 & 7)));
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int e = v[j];
+                        x[4 * i + j] = __builtin_bit_cast(float, e) * x_up(NG == 1 ? p : g);
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < F::NK; ++k) cut8(x + 8 * k, c[g][k]);
+            }
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                if constexpr (NG == 1) {
+                    ckq_v16f sum = zero;
+#pragma unroll
+                    for (int k = 0; k < 2; ++k) {
+                        const ckq_v4i b = F::operand(w[r], dec[r], p, k);
+                        sum = mfma_bf16(c[0][k].lo, b, sum);
+                        sum = mfma_bf16(c[0][k].mid, b, sum);
+                        sum = mfma_bf16(c[0][k].hi, b, sum);
+                    }
+                    /* two groups are added before they meet the sum so far */
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) two[r][i] = p ? fmaf(dec[r].s[p], sum[i], two[r][i]) : dec[r].s[p] * sum[i];
+                    if (p) {
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) acc[r][i] += two[r][i];
+                    }
+                } else {
+#pragma unroll
+                    for (int g = 0; g < NG; ++g) {
+                        const ckq_v4i b = F::operand(w[r], dec[r], 2 * p + g, 0);
+                        ckq_v16f sum = mfma_bf16(c[g][0].lo, b, zero);
+                        sum = mfma_bf16(c[g][0].mid, b, sum);
+                        sum = mfma_bf16(c[g][0].hi, b, sum);
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) two[r][i] = g ? fmaf(dec[r].s[2 * p + g], sum[i], two[r][i]) : dec[r].s[2 * p + g] * sum[i];
+                    }
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) acc[r][i] += two[r][i];
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+
+    constexpr int RP = R < 2 ? 1 : 2;
+    float *const red = reinterpret_cast<float *>(smem);      /* [wave][RP * 16][64] */
+    bool fix = false;
+    __syncthreads();                         /* every wave is done with its weights and activations */
+    /* the eight partial tiles through LDS, two row tiles at a time; wave w finishes sixteenths 2 w .. of every lane */
+#pragma unroll
+    for (int q = 0; q < R; q += RP) {
+        __syncthreads();                     /* every wave is done with the buffer (and its loads have landed) */
+#pragma unroll
+        for (int r = 0; r < RP; ++r)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) red[(wave * RP * 16 + 16 * r + i) * 64 + lane] = acc[q + r][i];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 2 * RP; ++j) {
+            const int o = 2 * RP * wave + j, i = o & 15;
+            float p[F32_WAVES];
+#pragma unroll
+            for (int k = 0; k < F32_WAVES; ++k) p[k] = red[(k * RP * 16 + o) * 64 + lane];
+            const float v = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+            const int n = n0 + 32 * (q + (o >> 4)) + col, t = t0 + 8 * (i >> 2) + 4 * half + (i & 3);
+            fix = fix || !(fabsf(v) < __builtin_inff());
+            if (n < N && t < M) C[(size_t)t * ldc + n] = bias ? v + bias[n] : v;
+        }
+    }
+    if (fix) {
+#pragma unroll 1
+        for (int j = 0; j < 2 * R; ++j) {
+            const int o = 2 * RP * wave + j % (2 * RP), i = o & 15;
+            const int n = n0 + 32 * (j / (2 * RP) * RP + (o >> 4)) + col, t = t0 + 8 * (i >> 2) + 4 * half + (i & 3);
+            if (n >= N || t >= M) continue;
+            float *const out = C + (size_t)t * ldc + n;
+            if (fabsf(*out) < __builtin_inff()) continue;
+            const float v = exact_output<F>(B + (size_t)n * (size_t)wrow, A + (size_t)t * (size_t)K, K);
+            *out = bias ? v + bias[n] : v;
+        }
+    }
+}
+
 template <class F>
 int launch_f32act(const float *A, const uint8_t *B, const float *bias, float *C, int M, int N, int K, long wrow, long ldc, hipStream_t s)
 {
@@ -426,8 +652,11 @@ int launch_f32act(const float *A, const uint8_t *B, const float *bias, float *C,
     const int R = ntg * ((N + 63) / 64) >= 192 ? 2 : 1;
     const long long grid = ntg * ((N + 32 * R - 1) / (32 * R));
     if (grid > 0x7fffffffll) return CKQ_ESHAPE;
-    if (R == 2) hipLaunchKernelGGL((gemm_f32act_kernel<F, 2>), dim3((unsigned)grid), dim3(64 * F32_WAVES), 0, s, A, B, bias, C, M, N, K, wrow, ldc, (int)ntg);
-    else hipLaunchKernelGGL((gemm_f32act_kernel<F, 1>), dim3((unsigned)grid), dim3(64 * F32_WAVES), 0, s, A, B, bias, C, M, N, K, wrow, ldc, (int)ntg);
+    const auto kernel = [&] {
+        if constexpr (std::is_same<F, F32Q4K>::value) return R == 2 ? gemm_f32act_q4k_kernel<2> : gemm_f32act_q4k_kernel<1>;
+        else return R == 2 ? gemm_f32run_kernel<F, 2> : gemm_f32run_kernel<F, 1>;
+    }();
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(64 * F32_WAVES), 0, s, A, B, bias, C, M, N, K, wrow, ldc, (int)ntg);
     return (int)hipGetLastError();
 }
 

@@ -1328,6 +1328,37 @@ def test_f32act_matrix_cores_infinite_huge_and_tiny_activations(fmt):
             assert float(np.abs(got[t][fin].astype(np.float64) - want[t][fin]).max()) <= 1e-5 * scale + 1024 * 2.0 ** -149, t
 
 
+@pytest.mark.parametrize("fmt,blocks", [("q6_k", (1, 2, 7, 8, 9, 17)), ("q8_0", (1, 2, 3, 5, 15, 33, 34, 67))])
+@pytest.mark.parametrize("ofs", [0, 2])
+def test_f32act_weights_by_runs(fmt, blocks, ofs):
+    """Weights that come in runs of one Q6_K or four Q8_0 blocks, from matrices on a dword and two bytes off: block counts that end
+    within a run, within a wave's share, or leave waves without one; one and two row tiles per wave, the last row of the matrix
+    in each place.  The buffer ends with the matrix.  Against float64; the result of fp32 sums of up to 2176 products has an
+    rms error below 2e-7 of the result's, its largest below 2e-6."""
+    import torch
+    L = ckq.lib()
+    B = T.ELEMS[fmt]
+    L.ckq_set_gemm_policy(1)
+    try:
+        for nb in blocks:
+            for M, N in ((33, 1), (2, 33), (200, 1793)):
+                K = nb * B
+                W = T.random_blocks(fmt, N * nb, 50 + nb)
+                buf = torch.zeros(W.size + ofs, dtype=torch.uint8, device="cuda")
+                buf[ofs:] = P.to_device(W)
+                x = T.normal(M * K, 0.5, 1.0, seed=nb)
+                x_d = P.to_device(x)
+                c = torch.full((M, N), 7.0, dtype=torch.float32, device="cuda")
+                say("f32act runs", fmt, nb, M, N, ofs)
+                P.check(L.ckq_gemm_nt_f32act_dev(P.FMT[fmt], P._dp(x_d), ctypes.c_void_p(buf.data_ptr() + ofs), None, P._dp(c), M, N, K, N, P._stream()), "f32act")
+                want = x_d.view(M, K).double() @ torch.from_numpy(T.np_dequant(fmt, W).reshape(N, K)).cuda().double().T
+                rms = float(want.pow(2).mean().sqrt())
+                assert float((c - want).pow(2).mean().sqrt()) <= 2e-7 * rms, (nb, M, N)
+                assert float((c - want).abs().max()) <= 2e-6 * float(want.abs().max()), (nb, M, N)
+    finally:
+        L.ckq_set_gemm_policy(0)
+
+
 # ---- 16-row tiles: a few to a few dozen tokens of the K-quants -------------------------------------
 
 @pytest.mark.parametrize("fmt", ["q4_k", "q5_k", "q6_k"])
