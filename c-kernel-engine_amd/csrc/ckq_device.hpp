@@ -144,6 +144,8 @@ __device__ __forceinline__ void q8k_quantize_block(const float (&e)[4], int lane
     const u32 packed = (u32)(q[0] & 0xff) | ((u32)(q[1] & 0xff) << 8) | ((u32)(q[2] & 0xff) << 16) | ((u32)(q[3] & 0xff) << 24);
     reinterpret_cast<u32 *>(out + 4)[lane] = packed;
     s = group_sum<4>(s);                       /* 16 consecutive elements = 4 lanes */
-    if ((lane & 3) == 3) reinterpret_cast<int16_t *>(out + 260)[lane >> 2] = (int16_t)s;
+    /* two sums a store, so that the block leaves in whole dwords: the host looks for them one by one (ckq_host.c) */
+    const u32 pair = ((u32)dpp_get<0x114>(s) & 0xffffu) | ((u32)s << 16);                /* row_shr:4 */
+    if ((lane & 7) == 7) reinterpret_cast<u32 *>(out + 260)[lane >> 3] = pair;
     if (lane == 0) *reinterpret_cast<float *>(out) = 1.0f / iscale;
 }

@@ -1515,3 +1515,31 @@ def test_gemm_mfma_q8_0_row_alignment_and_k_remainders(blocks):
             assert T.norm_err(np.where(ok, got[:, :N], 0.0), np.where(ok, ref, 0.0)) <= TOL, (M, N, K)
     finally:
         L.ckq_set_gemm_policy(0)
+
+
+@pytest.mark.parametrize("rows", [1, 3, 15, 16, 17, 33, 16384, 16385])
+def test_host_results_as_they_arrive(rows):
+    """Host-pointer GEMVs whose results the CPU waits for word by word (up to 64 KiB): sizes around its sixteen words at a time and
+    its limit, several calls through one twin, inputs of their own each; the bits are the device entry point's."""
+    K = 256
+    say("arrive", rows)
+    W, _, _ = make_case("q4_k", rows, K, "rand", 9500 + rows)
+    for seed in range(3):
+        xq = P.quantize(T.normal(K, 0.0, 1.0, 9600 + seed))
+        assert np.array_equal(xq, T.oracle_quantize(T.normal(K, 0.0, 1.0, 9600 + seed), "q8_k"))
+        y = P.gemv("q4_k", W, xq, rows, K)
+        ref = P.dev_gemm_nt("q4_k", P.to_device(xq), P.to_device(W), None, 1, rows, K).cpu().numpy().reshape(-1)
+        assert np.array_equal(y, ref)
+
+
+def test_host_result_equal_to_the_mark():
+    """Quants that spell the word the CPU takes for "not there yet": the call ends all the same, with the right bytes."""
+    x = T.normal(5 * 256, 0.0, 1.0, 9700)
+    for b in (0, 2, 4):
+        x[256 * b:256 * (b + 1)] = 0.0
+        x[256 * b] = -127.0                                     # iscale = 1
+        x[256 * b + 60:256 * b + 64] = (-63, -45, -91, 127)     # c1 d3 a5 7f
+    for _ in range(2):
+        got = P.quantize(x)
+        assert np.array_equal(got, T.oracle_quantize(x, "q8_k"))
+        assert (got.view(np.uint32) == 0x7FA5D3C1).sum() == 3
