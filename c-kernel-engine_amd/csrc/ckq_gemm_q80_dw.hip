@@ -16,21 +16,28 @@
  * - Tokens are the A operand, weight rows the B operand: lane 16 q + i holds ONE weight row and tokens 4 q .. 4 q + 3 of a
  *   16 x 16 result.  LDS row 64 h + 16 g + i is weight row 64 h + 4 i + g, so a lane ends with four adjacent rows.
  * - K advances 128 (four blocks) per iteration, two stages.  Of the eight waves, four take two of the blocks and four the
- *   other two, each 64 rows x 32 tokens; the partial tiles are added through LDS at the end.  That gives a tile alone on its
+ *   other two, each 64 rows x 16 TG tokens; the partial tiles are added through LDS at the end.  That gives a tile alone on its
  *   CU two waves per SIMD and two tiles four.
+ * - The scales, as fp32, lie beside the rows as [block][row] and [block][token], so that a lane's four rows or tokens are one
+ *   16-byte read.
  *
- * Measured, us, the other kernel (weights two bytes off) -> this one: 333 tokens x 4864 x 4096 51.3 -> 37.8, 512 x 9728 x 896
- * 34.7 -> 25.5, 2048 x 11008 x 4096 426 -> 322, 464 x 37134 x 2048 218 -> 154, 24 x 4864 x 4096 15.7 -> 13.9.  At 2048 tokens a block's
- * iteration takes 1970 cycles of its CU, of which the vector instructions issue 1260 and the matrix instructions 510 (counters).
- *
- * Block = 8 waves = 64 tokens x 128 weight rows.
+ * Tile = 32 TG tokens x 128 weight rows; the copies (a run of a row costs the address path its five cycles whatever the run's length), the
+ * fp32 operations, the LDS reads and the matrix instructions of an iteration weigh about the same, so nothing is hidden to the
+ * end and what counts is how many of each there are and whether a CU has another tile's to fill in:
+ * - 96 tokens save weights copied and read per product and, for some sizes, a round of tiles: 2048 x 11008 x 4096 (tokens,
+ *   rows, K) 321 -> 290 us against 64 tokens, 464 x 37134 x 2048 161 -> 131, 512 x 9728 x 896 26.2 -> 22.6.
+ * - 32 tokens do half the work where no more tokens are there: 32 x 37134 x 2048 33.8 -> 24.9.
+ * - Two TEAMS of eight waves, each with one half of K and its own stages, where a tile would be alone on its CU anyway: 333 x 4864 x 4096
+ *   42.5 -> 34.6, 70 x 11008 x 4096 42.4 -> 32.0, 256 x 4096 x 4096 29.1 -> 24.6.  The second team runs half an iteration behind the
+ *   first (one barrier more before, one less after), so that one computes while the other waits for its copies and
+ *   finishes them; in step they gain half of that (36.9 for the first).
+ * Against ckq_gemm_q80.hip (weights two bytes off): 333 x 4864 x 4096 51.3, 512 x 9728 x 896 34.7, 2048 x 11008 x 4096 426.
  */
 #include "ckq_gemm_common.hpp"
 
-constexpr int GEMM8_BM = 64, GEMM8_BN = 128, GEMM8_KB = 4;   /* tokens, rows, 32-blocks per iteration */
-constexpr int GEMM8_THREADS = 512;
+constexpr int GEMM8_BN = 128, GEMM8_KB = 4;      /* rows, 32-blocks per iteration */
+constexpr int GEMM8_THREADS = 512;               /* of a team */
 constexpr int GEMM8_PITCH = 144;                 /* bytes of an operand row's image in LDS: see below */
-constexpr int GEMM8_REGION = 24 * GEMM8_PITCH;   /* the rows a wave brings in: sixteen weight rows, eight tokens */
 typedef float ckq_v4f __attribute__((ext_vector_type(4)));
 
 /* Output (weight row w, activation row x) over blocks [j0, j1), one term at a time. */
@@ -59,16 +66,19 @@ __device__ __forceinline__ u32 lds_address(const void *p) { return (u32)(uintptr
  * nine 16-byte chunks (adjacent lanes of a copy fetch adjacent chunks, all from dword-aligned addresses).  Chunk 8 holds the last
  * sixteen, so dwords 30 to 33 of the run lie at 32 to 35.  A pair of blocks is 17 dwords: [d0 q0q1] seven of quants [q30q31 d1]
  * eight of quants.  Once a row has landed, the lane in charge makes [q0q1 q30q31] of the first and the ninth - the order of
- * the 32 products of a block is free as long as both operands have the same - and leaves the scales as fp32 in dwords nobody
- * reads (slot).  Lane quarter q takes dwords q and q + 4 of a block: with rows 36 dwords apart every bank then serves two lanes.
+ * the 32 products of a block is free as long as both operands have the same - and leaves the scales as fp32.  Lane quarter q takes
+ * dwords q and q + 4 of a block: with rows 36 dwords apart, and the waves' regions a multiple of four rows, every bank serves one lane.
  */
-template <bool DUMP>
-__global__ void __launch_bounds__(GEMM8_THREADS, DUMP ? 2 : 4) gemm_q80_dw_kernel(GemmArgs a)
+template <int TG, int TEAMS, bool DUMP>
+__global__ void __launch_bounds__(GEMM8_THREADS * TEAMS, DUMP ? 2 : 4) gemm_q80_dw_kernel(GemmArgs a)
 {
-    constexpr int BM = GEMM8_BM, BN = GEMM8_BN, KB = GEMM8_KB, PITCH = GEMM8_PITCH, MAGIC = 0x4B400000;
-    __shared__ __attribute__((aligned(16))) uint8_t stage[2][8 * GEMM8_REGION];
+    constexpr int BM = 32 * TG, BN = GEMM8_BN, KB = GEMM8_KB, PITCH = GEMM8_PITCH, MAGIC = 0x4B400000;
+    constexpr int XR = 4 * TG, REGION = (16 + XR) * PITCH;  /* a wave brings in sixteen weight rows and XR tokens */
+    constexpr int WSCALES = 8 * REGION, XSCALES = WSCALES + KB * BN * 4, STAGE = XSCALES + KB * BM * 4;     /* fp32 scales, [block][row], [block][token] */
+    __shared__ __attribute__((aligned(16))) uint8_t stages[TEAMS][2][STAGE];
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = wave_in_block();
+    const int tid = threadIdx.x, lane = tid & 63, wave = wave_in_block() & 7, team = TEAMS == 1 ? 0 : wave_in_block() >> 3;
+    uint8_t (*const stage)[STAGE] = stages[team];
     const int i16 = lane & 15, q = lane >> 4;
     const int kh = wave >> 2, rh = (wave >> 1) & 1, th = wave & 1;
 
@@ -92,47 +102,49 @@ __global__ void __launch_bounds__(GEMM8_THREADS, DUMP ? 2 : 4) gemm_q80_dw_kerne
     auto w_row = [&](int l) { return (u32)min(64 * (l >> 6) + 4 * (l & 15) + ((l >> 4) & 3), work.N - 1 - n0) * stride; };
     auto x_row = [&](int t) { return (u32)min(t, a.M - 1 - t0) * stride; };
 
-    /* A wave copies sixteen weight rows (144 chunks, three instructions) and eight tokens (72 chunks, two) into its region of a
-     * stage, and finishes the same rows when they have landed. */
-    u32 c_src[5];
-    bool c_on[5];
+    /* A wave copies sixteen weight rows (144 chunks, three instructions) and XR tokens (36 chunks for four, one instruction;
+     * 72 and 108, two) into its region of a stage, and finishes the same rows when they have landed. */
+    constexpr int NC = 3 + (9 * XR + 63) / 64;
+    u32 c_src[NC];
+    bool c_on[NC];
 #pragma unroll
-    for (int i = 0; i < 5; ++i) {
+    for (int i = 0; i < NC; ++i) {
         const int ci = 64 * (i < 3 ? i : i - 3) + lane, r = ci / 9, c = ci % 9;
-        c_on[i] = ci < (i < 3 ? 144 : 72);
-        c_src[i] = (i < 3 ? w_row(16 * wave + min(r, 15)) : x_row(8 * wave + min(r, 7))) + (u32)min(16 * c, 120);
+        c_on[i] = ci < (i < 3 ? 144 : 9 * XR);
+        c_src[i] = (i < 3 ? w_row(16 * wave + min(r, 15)) : x_row(XR * wave + min(r, XR - 1))) + (u32)min(16 * c, 120);
     }
     auto copy = [&](int it, uint8_t *sg) {
-        const u32 dst = lds_address(sg + GEMM8_REGION * wave);
+        const u32 dst = lds_address(sg + REGION * wave);
 #pragma unroll
-        for (int i = 0; i < 5; ++i)
+        for (int i = 0; i < NC; ++i)
             if (c_on[i]) lds_copy16(i < 3 ? bw : bx, dst + (u32)(i < 3 ? 1024 * i : 16 * PITCH + 1024 * (i - 3)), c_src[i], it * (KB * 34));
     };
     /* K ends after 17 dwords of the iteration: fetched one by one, a 16-byte chunk could pass the end of the matrix */
     auto copy_tail = [&](int it, uint8_t *sg) {
-        for (int e = lane; e < 24 * 17; e += 64) {
+        for (int e = lane; e < (16 + XR) * 17; e += 64) {
             const int r = e / 17, d = e % 17;
-            const uint8_t *const src = r < 16 ? wbase + w_row(16 * wave + r) : xbase + x_row(8 * wave + r - 16);
-            *reinterpret_cast<u32 *>(sg + GEMM8_REGION * wave + PITCH * r + 4 * d) = ld4<4>(src + (u32)it * (KB * 34u) + 4u * (u32)d);
+            const uint8_t *const src = r < 16 ? wbase + w_row(16 * wave + r) : xbase + x_row(XR * wave + r - 16);
+            *reinterpret_cast<u32 *>(sg + REGION * wave + PITCH * r + 4 * d) = ld4<4>(src + (u32)it * (KB * 34u) + 4u * (u32)d);
         }
     };
-    /* the dword with the scale of block 2 p + o of a row whose number has bit 3 = s: rows 8 apart start on the same bank */
-    auto slot = [](int p, int o_xor_s) { return p ? 30 + o_xor_s : o_xor_s ? 25 : 8; };
     /* two lanes per row, one for each pair of blocks */
-    const int f_row = lane >> 1, f_p = lane & 1, f_s = f_row < 16 ? f_row >> 3 : wave & 1;
+    const int f_row = lane >> 1, f_p = lane & 1;
+    const int f_w = f_row < 16 ? WSCALES + 4 * (64 * (wave >> 2) + 4 * f_row + (wave & 3)) : XSCALES + 4 * (XR * wave + f_row - 16);
+    const int f_pitch = f_row < 16 ? 4 * BN : 4 * BM;
     auto finish = [&](int it, uint8_t *sg) {
-        if (f_row >= 24) return;
-        u32 *const d = reinterpret_cast<u32 *>(sg + GEMM8_REGION * wave + PITCH * f_row);
+        if (f_row >= 16 + XR) return;
+        u32 *const d = reinterpret_cast<u32 *>(sg + REGION * wave + PITCH * f_row);
         const bool live = 2 * f_p < nblk - it * KB;
         const u32 d0 = d[17 * f_p], d8 = d[17 * f_p + 8];
         d[17 * f_p] = __builtin_amdgcn_alignbyte(d8, d0, 2);
-        d[slot(f_p, f_s)] = live ? __builtin_bit_cast(u32, h2f(d0 & 0xffff)) : 0u;
-        d[slot(f_p, 1 ^ f_s)] = live ? __builtin_bit_cast(u32, h2f(d8 >> 16)) : 0u;
+        float *const sc = reinterpret_cast<float *>(sg + f_w + 2 * f_p * f_pitch);
+        *sc = live ? h2f(d0 & 0xffff) : 0.0f;
+        *reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(sc) + f_pitch) = live ? h2f(d8 >> 16) : 0.0f;
     };
 
-    ckq_v4f acc[2][4];                                      /* [token group][row group] */
+    ckq_v4f acc[TG][4];                                     /* [token group][row group] */
 #pragma unroll
-    for (int tg = 0; tg < 2; ++tg)
+    for (int tg = 0; tg < TG; ++tg)
 #pragma unroll
         for (int g = 0; g < 4; ++g) acc[tg][g] = ckq_v4f{0.0f, 0.0f, 0.0f, 0.0f};
     ckq_v4i magic = {MAGIC, MAGIC, MAGIC, MAGIC};
@@ -144,59 +156,54 @@ __global__ void __launch_bounds__(GEMM8_THREADS, DUMP ? 2 : 4) gemm_q80_dw_kerne
         const u32 *const d = reinterpret_cast<const u32 *>(p);
         return (long)((uint64_t)d[lo] | ((uint64_t)d[hi] << 32));
     };
-    auto compute = [&](const uint8_t *sg, int it) {
-        const uint8_t *const wl = sg + 4 * rh * GEMM8_REGION + i16 * PITCH;
-        const uint8_t *const xl = sg + (4 * th + (i16 >> 3)) * GEMM8_REGION + (16 + (i16 & 7)) * PITCH;
-        const uint8_t *const xs = sg + (4 * th + (q >> 1)) * GEMM8_REGION + (16 + 4 * (q & 1)) * PITCH;
+    auto compute_block = [&](const uint8_t *sg, int it, int jj) __attribute__((always_inline)) {
+        const uint8_t *const wl = sg + 4 * rh * REGION + i16 * PITCH;
+        /* token t of the tile is row 16 + t % XR of wave t / XR */
+        auto token = [&](int t) { return sg + (t / XR) * REGION + (16 + t % XR) * PITCH; };
+        const int tw = 16 * TG * th;
+        const int lo = jj ? opd + 9 : opd, hi = jj ? opd_hi : opd + 4;
+        long w[4], x[TG];
 #pragma unroll
-        for (int jj = 0; jj < 2; ++jj) {
-            const int lo = jj ? opd + 9 : opd, hi = jj ? opd_hi : opd + 4;
-            long w[4], x[2];
-            u32 dwb[4], dxb[2][4];                          
+        for (int tg = 0; tg < TG; ++tg) x[tg] = operand(token(tw + 16 * tg + i16), lo, hi);
 #pragma unroll
-            for (int tg = 0; tg < 2; ++tg) x[tg] = operand(xl + 2 * GEMM8_REGION * tg, lo, hi);
+        for (int g = 0; g < 4; ++g) w[g] = operand(wl + REGION * g, lo, hi);
+        const ckq_v4f dwb = *reinterpret_cast<const ckq_v4f *>(sg + WSCALES + 4 * ((2 * kh + jj) * BN + 64 * rh + 4 * i16));
+        float dwm[4];
 #pragma unroll
-            for (int g = 0; g < 4; ++g) w[g] = operand(wl + GEMM8_REGION * g, lo, hi);
+        for (int g = 0; g < 4; ++g) dwm[g] = dwb[g] * -12582912.0f;
 #pragma unroll
-            for (int g = 0; g < 4; ++g) dwb[g] = reinterpret_cast<const u32 *>(wl + GEMM8_REGION * g)[slot(kh, jj ^ (i16 >> 3))];
+        for (int tg = 0; tg < TG; ++tg) {
+            const ckq_v4f dxb = *reinterpret_cast<const ckq_v4f *>(sg + XSCALES + 4 * ((2 * kh + jj) * BM + tw + 16 * tg + 4 * q));
+            ckq_v4i d[4];
 #pragma unroll
-            for (int tg = 0; tg < 2; ++tg)
+            for (int g = 0; g < 4; ++g) d[g] = __builtin_amdgcn_mfma_i32_16x16x32_i8(x[tg], w[g], magic, 0, 0, 0);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) dxb[tg][r] = reinterpret_cast<const u32 *>(xs + 2 * GEMM8_REGION * tg + PITCH * r)[slot(kh, jj ^ (q >> 1))];
-            float dwm[4];
+            for (int g = 0; g < 4; ++g) {
+                float t[4];
 #pragma unroll
-            for (int g = 0; g < 4; ++g) dwm[g] = __builtin_bit_cast(float, dwb[g]) * -12582912.0f;
-#pragma unroll
-            for (int tg = 0; tg < 2; ++tg) {
-                ckq_v4i d[4];
-#pragma unroll
-                for (int g = 0; g < 4; ++g) d[g] = __builtin_amdgcn_mfma_i32_16x16x32_i8(x[tg], w[g], magic, 0, 0, 0);
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    float t[4];
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int di = d[g][r];
-                        t[r] = __builtin_fmaf(__builtin_bit_cast(float, dwb[g]), __builtin_bit_cast(float, di), dwm[g]);
-                        if constexpr (DUMP) {
-                            int tr = t0 + 32 * th + 16 * tg + 4 * q + r;
-                            asm volatile("" : "+v"(tr));   /* store addresses formed here, not kept in registers */
-                            const int n = n0 + 64 * rh + 4 * i16 + g, b = it * KB + 2 * kh + jj;
-                            if (tr < a.M && n < work.N && b < nblk) a.dump[((size_t)tr * work.N + n) * nblk + (size_t)b] = di - MAGIC;
-                        }
+                for (int r = 0; r < 4; ++r) {
+                    const int di = d[g][r];
+                    t[r] = __builtin_fmaf(dwb[g], __builtin_bit_cast(float, di), dwm[g]);
+                    if constexpr (DUMP) {
+                        int tr = t0 + tw + 16 * tg + 4 * q + r;
+                        asm volatile("" : "+v"(tr));   /* store addresses formed here, not kept in registers */
+                        const int n = n0 + 64 * rh + 4 * i16 + g, b = it * KB + 2 * kh + jj;
+                        if (tr < a.M && n < work.N && b < nblk) a.dump[((size_t)tr * work.N + n) * nblk + (size_t)b] = di - MAGIC;
                     }
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) acc[tg][g][r] = __builtin_fmaf(__builtin_bit_cast(float, dxb[tg][r]), t[r], acc[tg][g][r]);
                 }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[tg][g][r] = __builtin_fmaf(dxb[r], t[r], acc[tg][g][r]);
             }
-            /* block by block: scheduled together, the two would need more registers than four waves per SIMD have */
-            asm volatile("" : "+v"(acc[0][0]), "+v"(acc[0][1]), "+v"(acc[0][2]), "+v"(acc[0][3]),
-                              "+v"(acc[1][0]), "+v"(acc[1][1]), "+v"(acc[1][2]), "+v"(acc[1][3]) :: "memory");
         }
+        /* block by block: scheduled together, the two would need more registers than four waves per SIMD have */
+#pragma unroll
+        for (int tg = 0; tg < TG; ++tg) asm volatile("" : "+v"(acc[tg][0]), "+v"(acc[tg][1]), "+v"(acc[tg][2]), "+v"(acc[tg][3]) :: "memory");
     };
 
-    const int nfull = min(niter, nblk / KB);
-    if (it0 < nfull) {
+    /* the whole iterations, in TEAMS runs; a team that has one less still comes to the barriers */
+    const int nfull = min(niter, nblk / KB), nrun = (max(nfull - it0, 0) + TEAMS - 1) / TEAMS;
+    const int run0 = it0 + team * nrun, run1 = min(run0 + nrun, nfull);
+    if (nrun > 0) {
         auto landed = [] {                                  /* vmcnt(0) lgkmcnt(0) */
             __builtin_amdgcn_s_waitcnt(0x0070);
             asm volatile("" ::: "memory");
@@ -206,91 +213,194 @@ __global__ void __launch_bounds__(GEMM8_THREADS, DUMP ? 2 : 4) gemm_q80_dw_kerne
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
         };
-        copy(it0, stage[0]);
+        auto at = [&](int it) { return min(it, nfull - 1); };
+        copy(at(run0), stage[0]);
         landed();
-        finish(it0, stage[0]);
+        finish(at(run0), stage[0]);
         meet();
+        if (TEAMS == 2 && team) __builtin_amdgcn_s_barrier();
         auto step = [&](int it, uint8_t *cur, uint8_t *next) {
-            copy(min(it + 1, nfull - 1), next);
+            copy(at(it + 1), next);
             __builtin_amdgcn_sched_barrier(0);
-            compute(cur, it);
+            if (TEAMS == 1 || it < run1) compute_block(cur, it, 0);
+            if (TEAMS == 2) __builtin_amdgcn_s_barrier();
+            if (TEAMS == 1 || it < run1) compute_block(cur, it, 1);
             __builtin_amdgcn_sched_barrier(0);
             landed();
-            finish(min(it + 1, nfull - 1), next);
+            finish(at(it + 1), next);
             meet();
         };
         if constexpr (DUMP) {                               /* one copy of the stores */
-            for (int it = it0; it < nfull; ++it) step(it, stage[(it - it0) & 1], stage[(it - it0 + 1) & 1]);
-        } else for (int it = it0; it < nfull; it += 2) {
-            step(it, stage[0], stage[1]);
-            if (it + 1 < nfull) step(it + 1, stage[1], stage[0]);
+            for (int k = 0; k < nrun; ++k) step(run0 + k, stage[k & 1], stage[(k + 1) & 1]);
+        } else for (int k = 0; k < nrun; k += 2) {
+            step(run0 + k, stage[0], stage[1]);
+            if (k + 1 < nrun) step(run0 + k + 1, stage[1], stage[0]);
         }
+        if (TEAMS == 2 && !team) __builtin_amdgcn_s_barrier();
     }
     if (nfull < niter) {
-        copy_tail(nfull, stage[0]);
-        finish(nfull, stage[0]);
+        const bool mine = team == TEAMS - 1;
+        if (mine) {
+            copy_tail(nfull, stage[0]);
+            finish(nfull, stage[0]);
+        }
         __syncthreads();
-        compute(stage[0], nfull);
+        if (mine) {
+            compute_block(stage[0], nfull, 0);
+            compute_block(stage[0], nfull, 1);
+        }
         __syncthreads();
     }
 
-    /* the two halves of K: waves kh keep token group kh and hand the other one over */
-    ckq_v4f *const give = reinterpret_cast<ckq_v4f *>(kh ? stage[1] : stage[0]) + (wave & 3) * 256 + lane;
-    const ckq_v4f *const take = reinterpret_cast<const ckq_v4f *>(kh ? stage[0] : stage[1]) + (wave & 3) * 256 + lane;
+    /* the parts of K: of the 2 TEAMS waves of a sub-tile, wave `part` keeps token groups tg with tg % (2 TEAMS) == part and hands
+     * the others over */
+    constexpr int PARTS = 2 * TEAMS;
+    const int part = 2 * team + kh;
+    ckq_v4f *const meet_at = reinterpret_cast<ckq_v4f *>(stages[0][0]) + (wave & 3) * 256 + lane;     /* [token group][part but the keeper][wave of the part][row group][lane] */
+    static_assert(TG * (PARTS - 1) * 16384 <= (int)sizeof(stages), "");
+    auto place = [&](int tg, int p) { return meet_at + 1024 * ((PARTS - 1) * tg + p - (p > tg % PARTS ? 1 : 0)); };
 #pragma unroll
-    for (int g = 0; g < 4; ++g) give[64 * g] = kh ? acc[0][g] : acc[1][g];
+    for (int tg = 0; tg < TG; ++tg)
+        if (tg % PARTS != part) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) place(tg, part)[64 * g] = acc[tg][g];
+        }
     __syncthreads();
-    ckq_v4f o4[4];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) o4[g] = (kh ? acc[1][g] : acc[0][g]) + take[64 * g];
 
     /* lane: rows n .. n + 3, tokens t .. t + 3 */
     const GemmOut o = work.out;
     const bool vec_ok = (o.ldc % 4 == 0) && (((uintptr_t)o.C) % 16 == 0) && (n0 + BN <= work.N);
-    const int n = n0 + 64 * rh + 4 * i16, t = t0 + 32 * th + 16 * kh + 4 * q;
+    const int n = n0 + 64 * rh + 4 * i16;
     float bv[4];
 #pragma unroll
     for (int g = 0; g < 4; ++g) bv[g] = o.bias && n + g < work.N ? o.bias[n + g] : 0.0f;
-    bool fix = false;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        if (t + r >= a.M) continue;
-        float *dst = o.C + (size_t)(t + r) * o.ldc + n;
-        float v[4];
+    for (int tg = 0; tg < TG; ++tg) {
+        if (tg % PARTS != part) continue;
+        const int t = t0 + 16 * (TG * th + tg) + 4 * q;
+        ckq_v4f o4[4];
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            fix = fix || o4[g][r] != o4[g][r];
-            v[g] = o4[g][r] + bv[g];
-        }
-        if (vec_ok) *reinterpret_cast<float4 *>(dst) = make_float4(v[0], v[1], v[2], v[3]);
-        else {
+            ckq_v4f v[PARTS];
 #pragma unroll
-            for (int g = 0; g < 4; ++g) if (n + g < work.N) dst[g] = v[g];
+            for (int p = 0; p < PARTS; ++p) v[p] = p == tg % PARTS ? acc[tg][g] : place(tg, p)[64 * g];
+            o4[g] = v[0] + v[1];
+            if constexpr (TEAMS == 2) o4[g] += v[2] + v[3];
         }
-    }
-    if (fix) {
-        for (int e = 0; e < 16; ++e) {
-            const int tr = t + (e >> 2), nr = n + (e & 3);
-            if (tr >= a.M || nr >= work.N) continue;
-            float *dst = o.C + (size_t)tr * o.ldc + nr;
-            if (*dst == *dst) continue;
-            *dst = q80_output(work.B + (size_t)nr * stride, a.A + (size_t)tr * stride, it0 * KB, min(nblk, niter * KB)) +
-                   (o.bias ? o.bias[nr] : 0.0f);
+        bool fix = false;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if (t + r >= a.M) continue;
+            float *dst = o.C + (size_t)(t + r) * o.ldc + n;
+            float v[4];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                fix = fix || o4[g][r] != o4[g][r];
+                v[g] = o4[g][r] + bv[g];
+            }
+            if (vec_ok) *reinterpret_cast<float4 *>(dst) = make_float4(v[0], v[1], v[2], v[3]);
+            else {
+#pragma unroll
+                for (int g = 0; g < 4; ++g) if (n + g < work.N) dst[g] = v[g];
+            }
+        }
+        if (fix) {
+            for (int e = 0; e < 16; ++e) {
+                const int tr = t + (e >> 2), nr = n + (e & 3);
+                if (tr >= a.M || nr >= work.N) continue;
+                float *dst = o.C + (size_t)tr * o.ldc + nr;
+                if (*dst == *dst) continue;
+                *dst = q80_output(work.B + (size_t)nr * stride, a.A + (size_t)tr * stride, it0 * KB, min(nblk, niter * KB)) +
+                       (o.bias ? o.bias[nr] : 0.0f);
+            }
         }
     }
 }
 
-/* g: operands, sizes, ntt and nnt set by the caller (ckq_gemm_q80.hip). */
-int gemm_q80_dw_launch(GemmArgs &g, hipStream_t s)
+/* The forms of the kernel: token groups of 16 per wave, teams; blocks of it that fit a CU; and what a launch takes, in us:
+ * launch + iterations of a team x (wait x rounds of the fullest CU + work x blocks on it) + round x rounds, 1.45 per million
+ * floats written and read again, 2.4 for the launch that adds a K split.  Fitted to 110 launches of all five (9 to 1500 tokens, 300 to
+ * 152000 rows, K of 256 to 8192; 9 to 12 % rms): the choice is 2 % slower than the best form of each on average, and
+ * 12 % faster than 64 tokens and one team throughout. */
+struct DwForm { int tg, teams, fit; float launch, wait, work, round; };
+static const DwForm dw_forms[5] = {{1, 1, 3, 4.0f, 0.40f, 0.39f, 0.0f}, {2, 1, 2, 4.7f, 0.45f, 0.575f, 0.0f}, {3, 1, 2, 5.3f, 0.74f, 0.58f, 0.0f},
+                                   {1, 2, 1, 3.1f, 1.18f, 0.0f, 1.9f}, {2, 2, 1, 3.2f, 1.6f, 0.0f, 2.5f}};
+
+/* The form for `row_tiles` tiles of weight rows in all; single: one matrix, which may be split along K.  64 tokens and one team
+ * are always possible; another form only if its chains of multiply-adds are no longer (fewer splits of K would make them so, and the
+ * error larger) and, if it is split, with no more scratch than that form or the entry point that allocates nothing has. */
+static int dw_form(int M, int nb, long rows, long row_tiles, bool single, float *time)
 {
+    const int steps = (nb + GEMM8_KB - 1) / GEMM8_KB;
+    const float out = 1e-6f * (float)M * (float)rows;
+    int best = 0, chain = 0;
+    float least = 0.0f;
+    size_t scratch = 0;
+    for (int k : {1, 0, 2, 3, 4}) {
+        const DwForm &f = dw_forms[k];
+        const long tiles = (long)((M + 32 * f.tg - 1) / (32 * f.tg)) * row_tiles;
+        int s = single && tiles < 160 ? gemm_choose_splits((int)tiles, steps) : 1;
+        const int per = (steps + s - 1) / s, iters = (per + f.teams - 1) / f.teams;
+        s = (steps + per - 1) / per;
+        const size_t need = s > 1 ? (size_t)s * (size_t)M * (size_t)rows * 4 : 0;
+        if (k == 1) {
+            chain = iters;
+            scratch = need > CKQ_NOALLOC_SCRATCH_BYTES ? need : CKQ_NOALLOC_SCRATCH_BYTES;
+        } else if (iters > chain || need > scratch || (f.teams > 1 && (s > 1 || !single))) continue;
+        const long on_cu = (tiles * s + 255) / 256, rounds = (on_cu + f.fit - 1) / f.fit;
+        const float t = f.launch + (float)iters * (f.wait * (float)rounds + f.work * (float)on_cu) + f.round * (float)rounds +
+                        1.45f * out * (float)(s > 1 ? 1 + 2 * s : 1) + (s > 1 ? 2.4f : 0.0f);
+        if (k == 1 || t < least) { least = t; best = k; }
+    }
+    if (time) *time = least;
+    return best;
+}
+
+/* g: operands, sizes, nnt set by the caller (ckq_gemm_q80.hip). */
+template <int TG, int TEAMS>
+static int dw_launch(GemmArgs &g, hipStream_t s)
+{
+    g.ntt = (g.M + 32 * TG - 1) / (32 * TG);
     const unsigned grid = (unsigned)(g.ntt * ((g.nnt + 7) / 8 * 8));
     const int steps = (g.nb + GEMM8_KB - 1) / GEMM8_KB;
 #if CKQ_WITH_DUMP
-    if (g.dump) return gemm_launch_split(gemm_q80_dw_kernel<true>, g, grid, steps, s, GEMM8_THREADS);
+    if (g.dump) return gemm_launch_split(gemm_q80_dw_kernel<TG, TEAMS, true>, g, grid, steps, s, GEMM8_THREADS * TEAMS);
 #endif
-    return gemm_launch_split(gemm_q80_dw_kernel<false>, g, grid, steps, s, GEMM8_THREADS);
+    return gemm_launch_split(gemm_q80_dw_kernel<TG, TEAMS, false>, g, grid, steps, s, GEMM8_THREADS * TEAMS);
+}
+int gemm_q80_dw_launch(GemmArgs &g, hipStream_t s)
+{
+    switch (dw_form(g.M, g.nb, g.N, g.nnt, true, nullptr)) {
+    case 0: return dw_launch<1, 1>(g, s);
+    case 1: return dw_launch<2, 1>(g, s);
+    case 2: return dw_launch<3, 1>(g, s);
+    case 3: return dw_launch<1, 2>(g, s);
+    default: return dw_launch<2, 2>(g, s);
+    }
+}
+template <int TG>
+static int dw_launch_group(GemmArgs &g, const GemmGroupIn &in, hipStream_t s)
+{
+    g.ntt = (g.M + 32 * TG - 1) / (32 * TG);
+    return gemm_launch_grouped(gemm_q80_dw_kernel<TG, 1, false>, g, in, s, GEMM8_THREADS);
 }
 int gemm_q80_dw_launch_group(GemmArgs &g, const GemmGroupIn &in, hipStream_t s)
 {
-    return gemm_launch_grouped(gemm_q80_dw_kernel<false>, g, in, s, GEMM8_THREADS);
+    long rows = 0, tiles = 0;
+    for (int p = 0; p < in.n; ++p) {
+        rows += in.N[p];
+        tiles += (in.N[p] + GEMM8_BN - 1) / GEMM8_BN;
+    }
+    switch (dw_form(g.M, g.nb, rows, tiles, false, nullptr)) {
+    case 0: return dw_launch_group<1>(g, in, s);
+    case 1: return dw_launch_group<2>(g, in, s);
+    default: return dw_launch_group<3>(g, in, s);
+    }
+}
+
+float gemm_q80_dw_time(int M, long rows, int nb)
+{
+    float t;
+    dw_form(M, nb, rows, (rows + GEMM8_BN - 1) / GEMM8_BN, true, &t);
+    return t;
 }

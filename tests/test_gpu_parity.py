@@ -1543,3 +1543,24 @@ def test_host_result_equal_to_the_mark():
         got = P.quantize(x)
         assert np.array_equal(got, T.oracle_quantize(x, "q8_k"))
         assert (got.view(np.uint32) == 0x7FA5D3C1).sum() == 3
+
+
+@pytest.mark.parametrize("M,N,K", [(9, 131, 64), (33, 300, 192), (63, 1030, 2112), (129, 2050, 576), (192, 21001, 640), (350, 24484, 256), (385, 24499, 320),
+                                   (128, 8000, 1984), (16, 21000, 2112), (130, 8001, 1984), (65, 12000, 2240)])
+def test_gemm_mfma_q8_0_tiles_and_teams(M, N, K):
+    """Tiles of 32, 64 and 96 tokens, one and two teams, K ending inside a step and with one step more for the first team, against
+    fp64.  An output is nb terms, each rounded twice and added once: (nb + 4) 2^-24 of the sum of the terms' magnitudes."""
+    import torch
+    x, w = T.random_blocks("q8_0", M * (K // 32), 9800 + M), T.random_blocks("q8_0", N * (K // 32), 9801 + N)
+
+    def real(b, rows):
+        b = P.to_device(b).view(rows, K // 32, 34)
+        d = b[:, :, :2].contiguous().view(torch.float16).double()
+        return (d * b[:, :, 2:].contiguous().view(torch.int8).double()).reshape(rows, K)
+    say("q8_0 tiles", M, N, K)
+    bias = P.to_device(T.normal(N, 0.0, 0.5, seed=N))
+    y = P.dev_gemm_nt("q8_0", P.to_device(x), P.to_device(w), bias, M, N, K).view(M, N).double() - bias.double()
+    A, B = real(x, M), real(w, N)
+    bound = (A.abs() @ B.abs().T) * (K // 32 + 4) * 2.0 ** -24 + bias.abs().double() * 2.0 ** -23
+    assert bool((torch.isfinite(bound)).all())
+    assert float(((y - A @ B.T).abs() / bound).max()) <= 1.0
