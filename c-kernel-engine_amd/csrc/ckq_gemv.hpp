@@ -10,6 +10,7 @@
 
 #include "ckq_blocks.h"
 #include "ckq_formats.hpp"
+#include "ckq_producers.hpp"
 #include "ckq_launch.h"
 
 constexpr int CKQ_GROUP_MAX = 4;   /* independent matmuls of one shape in one launch */
@@ -36,6 +37,11 @@ struct GemvGroup {
 };
 
 
+/* The producer step of a launch that has one (gemv_pro_kernel): RMSNorm (gamma non-null) or the quantizer, rows of x stride
+ * floats apart -> Q8_K blocks, in LDS for the launch's own matmuls and at out. */
+struct GemvPro { const float *x, *gamma; uint8_t *out; long stride; float eps; };
+__host__ __device__ __forceinline__ constexpr size_t pro_image_bytes(size_t tile_bytes) { return (tile_bytes + 15) & ~(size_t)15; }
+
 /*
  * Tiled kernel (token tiles MT >= 1; DUMP: the same instantiation also stores
  * the raw integer sub-block dots of every (token, row), for the exactness tests).  One wave
@@ -46,10 +52,10 @@ struct GemvGroup {
  * summed over the LPR lanes with a fixed DPP tree; the last lane of the group
  * stores.
  */
-template <class F, int LPR, int PPL, int MT, int RPI, bool DUMP, int WPB, bool LDSX, bool GRP = false>
-__global__ void __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(DUMP ? 1 : MT == 1 && PPL == 1 && RPI == 1 ? F::OCC1 : MT == 1 && PPL == 1 && RPI == 2 && LPR == 64 ? F::OCC2 : MT >= 4 && PPL == 1 ? 4 : 1)))
-gemv_kernel(const uint8_t *W, const uint8_t *X, long wrow, long xrow, int row0, int row1, int npos, int ntok,
-            float *y, const float *bias, long ldy, int32_t *sub, int nsub_row, int nrows, GemvGroup grp)
+template <class F, int LPR, int PPL, int MT, int RPI, bool DUMP, int WPB, bool LDSX, bool GRP, bool PRO>
+__device__ __forceinline__ void gemv_body(const uint8_t *W, const uint8_t *X, long wrow, long xrow, int row0, int row1, int npos, int ntok,
+                                          float *y, const float *bias, long ldy, int32_t *sub, int nsub_row, int nrows, const GemvGroup &grp,
+                                          const GemvPro &pro)
 {
     /* The arguments are scalars, those the first loads need in front: the
      * first fourteen registers' worth arrive preloaded with the wave (build
@@ -73,6 +79,7 @@ gemv_kernel(const uint8_t *W, const uint8_t *X, long wrow, long xrow, int row0, 
     const int wave_row = a.row0 + (blockIdx.x * WPB + wave) * (SLOTS * RPI);   /* uniform */
     const bool live = wave_row < a.row1;
     if (!LDSX && !live) return;
+    if (GRP && a.row0 + (int)blockIdx.x * (WPB * SLOTS * RPI) >= a.row1) return;      /* all of the block: a narrower problem of the group */
     const int wrow_c = min(wave_row, a.row1 - 1);
     const int rbase = wave_row + slot * RPI;
     const int t0 = blockIdx.y * MT;
@@ -90,7 +97,22 @@ gemv_kernel(const uint8_t *W, const uint8_t *X, long wrow, long xrow, int row0, 
     const int xbytes = (int)((long)mt_live * a.xrow), xn = xbytes / F::XS_SRC;   /* staging units */
     const u32 xcap = (u32)((long)MT * a.xrow / F::XS_SRC);                                     /* units of a full tile */
     u32 xv[XU][F::XS_REGS];
-    if (LDSX) {
+    /* PRO: wave w turns 256-blocks w, w + WPB, ... of the tile's rows into Q8_K, block column by block column */
+    constexpr int XC = PRO ? (LPR / 4 + WPB - 1) / WPB : 1;
+    float4 px[XC][MT], pg[XC];
+    const int pnb = a.npos / 4;
+    if constexpr (PRO) {
+#pragma unroll
+        for (int c = 0; c < XC; ++c)
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+                px[c][t] = reinterpret_cast<const float4 *>(pro.x + (size_t)(t0 + min(t, mt_live - 1)) * (size_t)pro.stride + 256 * min(wave + WPB * c, pnb - 1))[lane];
+        if (pro.gamma) {
+#pragma unroll
+            for (int c = 0; c < XC; ++c) pg[c] = reinterpret_cast<const float4 *>(pro.gamma + 256 * min(wave + WPB * c, pnb - 1))[lane];
+        }
+    }
+    if (LDSX && !PRO) {
 #pragma unroll
         for (int u = 0; u < XU; ++u) {
             const int i = u * XNT + (int)threadIdx.x;                 /* units past the tile re-read its last one */
@@ -122,7 +144,43 @@ gemv_kernel(const uint8_t *W, const uint8_t *X, long wrow, long xrow, int row0, 
                 F::load_w(w[r][p], wbase, orow);
             }
         }
-        if (LDSX && p0 == 0) {
+        if constexpr (PRO) {
+            float *const rows = reinterpret_cast<float *>(xs + pro_image_bytes((size_t)MT * (size_t)a.xrow));
+            const int D = 64 * a.npos, rfl = (int)(rms_lds_bytes((size_t)D) / 4);
+#pragma unroll
+            for (int c = 0; c < XC; ++c)
+#pragma unroll
+                for (int t = 0; t < MT; ++t)
+                    if (t < mt_live && wave + WPB * c < pnb) rms_stage(rows + t * rfl, D, wave + WPB * c, lane, px[c][t]);
+            if (pro.gamma) {
+                __syncthreads();
+                const int ct = wave + WPB * (lane >> 3);              /* eight lanes walk a token's eight chains */
+                if (ct < mt_live) rms_chain(rows + ct * rfl, D, lane & 7);
+                __syncthreads();
+            }
+            /* the rows come back from LDS: held in registers beside the weights they would not fit */
+#pragma unroll 1
+            for (int t = 0; t < mt_live; ++t) {
+                const float rstd = pro.gamma ? rms_rstd(rows + t * rfl, D, pro.eps) : 0.0f;
+#pragma unroll
+                for (int c = 0; c < XC; ++c) {
+                    const int b = wave + WPB * c;
+                    if (b >= pnb) continue;
+                    const float4 v = rms_unstage(rows + t * rfl, D, b, lane);
+                    uint8_t *const out = xs + (u32)t * (u32)a.xrow + 292u * (u32)b;
+                    if (pro.gamma) rms_quant_block(v, pg[c], rstd, lane, out);
+                    else {
+                        const float e[4] = {v.x, v.y, v.z, v.w};
+                        q8k_quantize_block(e, lane, out);
+                    }
+                }
+            }
+            __syncthreads();
+            if (blockIdx.x == 0 && (!GRP || g == 0)) {                /* the step's own result */
+                u32 *const out = reinterpret_cast<u32 *>(pro.out + (size_t)t0 * (size_t)a.xrow);
+                for (int i = threadIdx.x; i < xbytes / 4; i += XNT) out[i] = reinterpret_cast<const u32 *>(xs)[i];
+            }
+        } else if (LDSX && p0 == 0) {
             /* the staged activations' loads are older than the weight loads
              * just issued, so waiting for them does not wait for the weights */
 #pragma unroll
@@ -230,6 +288,23 @@ gemv_kernel(const uint8_t *W, const uint8_t *X, long wrow, long xrow, int row0, 
         }
 }
 
+template <class F, int LPR, int PPL, int MT, int RPI, bool DUMP, int WPB, bool LDSX, bool GRP = false>
+__global__ void __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(DUMP ? 1 : MT == 1 && PPL == 1 && RPI == 1 ? F::OCC1 : MT == 1 && PPL == 1 && RPI == 2 && LPR == 64 ? F::OCC2 : MT >= 4 && PPL == 1 ? 4 : 1)))
+gemv_kernel(const uint8_t *W, const uint8_t *X, long wrow, long xrow, int row0, int row1, int npos, int ntok,
+            float *y, const float *bias, long ldy, int32_t *sub, int nsub_row, int nrows, GemvGroup grp)
+{
+    gemv_body<F, LPR, PPL, MT, RPI, DUMP, WPB, LDSX, GRP, false>(W, X, wrow, xrow, row0, row1, npos, ntok, y, bias, ldy, sub, nsub_row, nrows, grp, GemvPro{});
+}
+
+/* A producer step and the matmuls that read its result in one launch. */
+template <class F, int LPR, int MT, int RPI>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MT >= 4 || RPI == 2 ? 3 : 4)))
+gemv_pro_kernel(const uint8_t *W, long wrow, long xrow, int row1, int npos, int ntok, GemvPro pro,
+                float *y, const float *bias, long ldy, int nrows, GemvGroup grp)
+{
+    gemv_body<F, LPR, 1, MT, RPI, false, 4, true, true, true>(W, nullptr, wrow, xrow, 0, row1, npos, ntok, y, bias, ldy, nullptr, 0, nrows, grp, pro);
+}
+
 /* Rows the grid has to cover: the computed range, or the largest problem of a group. */
 static int launch_rows(const GemvArgs &a, const GemvGroup &grp) { return grp.n > 1 ? a.nrows : a.row1 - a.row0; }
 
@@ -293,6 +368,22 @@ static int launch_tile(const GemvArgs &a, const GemvGroup &grp, hipStream_t s)
     return launch_one<F, LPR, PPL, MT, RPI, false, WPB, false>(a, grp, s);
 }
 
+/* Two rows per slot serve the staged tokens twice, but leave CUs without a block where the matrix is small: then one row
+ * per slot, and smaller token tiles while that too leaves some.  Measured (us; 2, 4 and 7 tokens): Q5_K 1024 x 4864
+ * 3.9 -> 3.2, 5.2 -> 3.9, 7.5 -> 5.2; 4096 x 1024 at 4 and 7 3.5 -> 2.8, 4.5 -> 3.3; Q6_K 1024 x 11008 at 2 and 4 6.5 -> 5.2,
+ * 9.0 -> 7.3; Q4_K 2048 x 2048 at 7 4.5 -> 3.2; 12000 x 1024 at 4 4.4 -> 4.1, Q8_0 at 7 6.7 -> 5.8.  Rows that take a wave
+ * each lose from 256 blocks of two rows per slot on (2048 x 8192, Q6_K at 4: 7.4 -> 8.2), shorter ones from 512. */
+static void gemv_token_tile(int lpr, int rows, int n, int ntok, int *mt, int *rpi)
+{
+    const long few = lpr < 64 ? 512 : 256;
+    const long slots = ((long)rows * lpr + 255) / 256 * (long)n;      /* blocks of one row per slot and a token tile */
+    *mt = ntok == 2 ? 2 : ntok <= 4 ? 4 : 8;
+    *rpi = 2;                        /* the staged tile serves twice the weights */
+    if (slots >= 2 * few) return;
+    *rpi = 1;
+    while (*mt > 2 && slots * ((ntok + *mt - 1) / *mt) <= 256) *mt /= 2;
+}
+
 /* Rows per wave-slot and waves per block for each token tile: one row per
  * slot in 256-thread blocks for the bandwidth-bound single-token case (as many
  * of the matrix's loads in flight as the CUs can hold, small barrier groups),
@@ -315,23 +406,16 @@ static int launch_mt(const GemvArgs &a, const GemvGroup &grp, int max_mt, hipStr
         return launch_tile<F, LPR, PPL, 1, 1, 4>(a, grp, s);
     }
     if constexpr (F::TOKEN_TILES) {
-        /* Two rows per slot serve the staged tokens twice, but leave CUs without a block where the matrix is small: then one row
-         * per slot, and smaller token tiles while that too leaves some.  Measured (us; 2, 4 and 7 tokens): Q5_K 1024 x 4864
-         * 3.9 -> 3.2, 5.2 -> 3.9, 7.5 -> 5.2; 4096 x 1024 at 4 and 7 3.5 -> 2.8, 4.5 -> 3.3; Q6_K 1024 x 11008 at 2 and 4 6.5 -> 5.2,
-         * 9.0 -> 7.3; Q4_K 2048 x 2048 at 7 4.5 -> 3.2; 12000 x 1024 at 4 4.4 -> 4.1, Q8_0 at 7 6.7 -> 5.8.  Rows that take a wave
-         * each lose from 256 blocks of two rows per slot on (2048 x 8192, Q6_K at 4: 7.4 -> 8.2), shorter ones from 512. */
-        constexpr long few = LPR < 64 ? 512 : 256;
-        const long slots = ((long)launch_rows(a, grp) * LPR + 255) / 256 * (long)grp.n;      /* blocks of one row per slot and a token tile */
-        if (slots < 2 * few) {
-            int mt = a.ntok == 2 ? 2 : a.ntok <= 4 ? 4 : 8;
-            while (mt > 2 && slots * ((a.ntok + mt - 1) / mt) <= 256) mt /= 2;
+        int mt, rpi;
+        gemv_token_tile(LPR, launch_rows(a, grp), grp.n, a.ntok, &mt, &rpi);
+        if (rpi == 1) {
             if (mt == 2) return launch_tile<F, LPR, PPL, 2, 1, 4>(a, grp, s);
             if (mt == 4) return launch_tile<F, LPR, PPL, 4, 1, 4>(a, grp, s);
             return launch_tile<F, LPR, PPL, 8, 1, 4>(a, grp, s);
         }
-        if (a.ntok == 2) return launch_tile<F, LPR, PPL, 2, 2, 4>(a, grp, s);
-        if (a.ntok <= 4) return launch_tile<F, LPR, PPL, 4, 2, 4>(a, grp, s);
-        return launch_tile<F, LPR, PPL, 8, 2, 4>(a, grp, s);   /* two rows per slot: the staged tile serves twice the weights */
+        if (mt == 2) return launch_tile<F, LPR, PPL, 2, 2, 4>(a, grp, s);
+        if (mt == 4) return launch_tile<F, LPR, PPL, 4, 2, 4>(a, grp, s);
+        return launch_tile<F, LPR, PPL, 8, 2, 4>(a, grp, s);
     }
     return CKQ_EINVAL;   /* formats without token tiles are always launched with max_mt == 1 */
 }
@@ -351,6 +435,46 @@ static int launch_fmt(const GemvArgs &a, const GemvGroup &grp, int max_mt, hipSt
     return launch_mt<F, 64, 4>(a, grp, max_mt, s);   /* longer rows loop in passes of 256 positions */
 }
 
+/*
+ * Producer step and matmuls in one launch: rows of up to 32 positions (K of up to 2048).  Where a step is a few microseconds, half
+ * of which are a launch's beginning and end, every block makes the quantized rows for itself, in LDS, while its weights are on their way;
+ * the first block of a token tile stores them as the step's own result.  The arithmetic is that of the producer kernels, so every
+ * buffer keeps its bits.  It pays while the fullest CU makes no more than PRO_UNITS 256-blocks that way (blocks on it x tokens of a tile x
+ * 256-blocks of a row).  Measured, us per layer of a decode chain (RMSNorm, Q/K/V, quantizer, O, RMSNorm, gate and up, SwiGLU, down; K and V narrow),
+ * separate -> joined: one token, 768 wide 20.0 -> 14.8, 1024 wide 20.4 -> 16.6, 2048 wide 24.4 -> 23.6; four tokens, 1024 wide 25.0 -> 23.4
+ * without gate and up (48 units), 25.9 with them; 2048 wide 31.4, with RMSNorm and Q/K/V joined (64 units) 35.7.
+ */
+constexpr int PRO_UNITS = 16;
+template <class F, int LPR, int MT, int RPI>
+static int launch_pro_one(const GemvArgs &a, const GemvGroup &grp, const GemvPro &pro, hipStream_t s)
+{
+    constexpr int rows_per_block = 4 * (64 / LPR) * RPI;
+    const size_t lds = pro_image_bytes((size_t)MT * (size_t)a.xrow) + MT * rms_lds_bytes((size_t)a.npos * 64);
+    if (lds > 65536) return CKQ_ENOGROUP;
+    long blocks = (a.row1 + rows_per_block - 1) / rows_per_block;
+    for (int i = 0; i + 1 < grp.n; ++i) blocks += (grp.nrows[i] + rows_per_block - 1) / rows_per_block;
+    blocks *= (a.ntok + MT - 1) / MT;
+    if ((blocks + 255) / 256 * MT * (a.npos / 4) > PRO_UNITS) return CKQ_ENOGROUP;
+    const dim3 grid((a.nrows + rows_per_block - 1) / rows_per_block, (a.ntok + MT - 1) / MT, (unsigned)grp.n);
+    hipLaunchKernelGGL((gemv_pro_kernel<F, LPR, MT, RPI>), grid, dim3(256), lds, s, a.W, a.wrow, a.xrow, a.row1, a.npos, a.ntok, pro, a.y, a.bias, a.ldy, a.nrows, grp);
+    return (int)hipGetLastError();
+}
+template <class F, int LPR>
+static int launch_pro_lpr(const GemvArgs &a, const GemvGroup &grp, const GemvPro &pro, hipStream_t s)
+{
+    int mt = 1, rpi = 1;
+    if (a.ntok > 1) gemv_token_tile(LPR, a.nrows, grp.n, a.ntok, &mt, &rpi);
+    /* tiles of four at most: eight tokens' rows beside the weights would not fit the registers */
+    if (rpi == 2) return mt == 2 ? launch_pro_one<F, LPR, 2, 2>(a, grp, pro, s) : launch_pro_one<F, LPR, 4, 2>(a, grp, pro, s);
+    return mt == 1 ? launch_pro_one<F, LPR, 1, 1>(a, grp, pro, s) : mt == 2 ? launch_pro_one<F, LPR, 2, 1>(a, grp, pro, s) : launch_pro_one<F, LPR, 4, 1>(a, grp, pro, s);
+}
+template <class F>
+static int launch_pro(const GemvArgs &a, const GemvGroup &grp, const GemvPro &pro, hipStream_t s)
+{
+    if (a.npos > 32) return CKQ_ENOGROUP;
+    return a.npos <= 8 ? launch_pro_lpr<F, 8>(a, grp, pro, s) : a.npos <= 16 ? launch_pro_lpr<F, 16>(a, grp, pro, s) : launch_pro_lpr<F, 32>(a, grp, pro, s);
+}
+
 /* One function per trait, each defined in its own translation unit. */
 int ckq_gemv_launch_q4k(const GemvArgs &a, const GemvGroup &grp, hipStream_t s);
 int ckq_gemv_launch_q5k(const GemvArgs &a, const GemvGroup &grp, hipStream_t s);
@@ -361,3 +485,6 @@ int ckq_gemv_launch_q50(const GemvArgs &a, const GemvGroup &grp, hipStream_t s);
 int ckq_gemv_launch_q80_f32(const GemvArgs &a, const GemvGroup &grp, hipStream_t s);
 int ckq_gemv_launch_q4k_f32(const GemvArgs &a, const GemvGroup &grp, hipStream_t s);
 int ckq_gemv_launch_q6k_f32(const GemvArgs &a, const GemvGroup &grp, hipStream_t s);
+int ckq_gemv_pro_launch_q4k(const GemvArgs &a, const GemvGroup &grp, const GemvPro &pro, hipStream_t s);
+int ckq_gemv_pro_launch_q5k(const GemvArgs &a, const GemvGroup &grp, const GemvPro &pro, hipStream_t s);
+int ckq_gemv_pro_launch_q6k(const GemvArgs &a, const GemvGroup &grp, const GemvPro &pro, hipStream_t s);

@@ -2,3 +2,4 @@
 #include "ckq_gemv.hpp"
 
 int ckq_gemv_launch_q5k(const GemvArgs &a, const GemvGroup &grp, hipStream_t s) { return launch_fmt<FmtQ5K>(a, grp, 8, s); }
+int ckq_gemv_pro_launch_q5k(const GemvArgs &a, const GemvGroup &grp, const GemvPro &pro, hipStream_t s) { return launch_pro<FmtQ5K>(a, grp, pro, s); }

@@ -1517,6 +1517,35 @@ static int group_length(const ckq_matmul_op *ops, int i, int nops)
     return n;
 }
 
+/* A producer entry together with the matmul entries behind it that read its result, up to eight tokens: the number of entries
+ * issued, 0 if they go out one by one, or an error. */
+static int issue_fused(const ckq_matmul_op *ops, int i, int nops, void *stream, int *taken)
+{
+    enum { GROUP_MAX = 4 };
+    const ckq_matmul_op *p = &ops[i], *o = p + 1;
+    *taken = 0;
+    if ((p->fmt != CKQ_STEP_QUANTIZE_Q8_K && p->fmt != CKQ_STEP_RMSNORM_Q8_K) || i + 1 >= nops || p->M > 8 || o->M != p->M || o->K != p->K ||
+        (o->fmt != CKQ_FMT_Q4_K && o->fmt != CKQ_FMT_Q5_K && o->fmt != CKQ_FMT_Q6_K) || (const void *)p->C != o->A_q8 ||
+        (p->fmt == CKQ_STEP_RMSNORM_Q8_K && !p->B))
+        return 0;
+    const int n = group_length(ops, i + 1, nops);
+    float *y[GROUP_MAX];
+    const void *W[GROUP_MAX];
+    const float *b[GROUP_MAX];
+    int rows[GROUP_MAX];
+    long ld[GROUP_MAX];
+    for (int j = 0; j < n; ++j) {
+        if (o[j].A_q8 != o->A_q8) return 0;
+        y[j] = o[j].C; W[j] = o[j].B; b[j] = o[j].bias; rows[j] = o[j].N; ld[j] = o[j].ldc;
+    }
+    const int rms = p->fmt == CKQ_STEP_RMSNORM_Q8_K;
+    const int rc = ckq_launch_gemv_pro(o->fmt, n, y, W, b, rows, ld, o->K, o->M, (const float *)p->A_q8, rms ? (const float *)p->B : NULL, p->eps,
+                                       rms && p->ldc ? p->ldc : p->K, p->C, stream);
+    if (rc == CKQ_ENOGROUP) return 0;
+    *taken = 1 + n;
+    return rc;
+}
+
 int ckq_matmul_sequence_dev(const ckq_matmul_op *ops, int nops, int repeat, void *stream)
 {
     if (!ops || nops <= 0 || repeat <= 0) return CKQ_EINVAL;
@@ -1525,9 +1554,14 @@ int ckq_matmul_sequence_dev(const ckq_matmul_op *ops, int nops, int repeat, void
         for (int i = 0; i < nops;) {
             const ckq_matmul_op *o = &ops[i];
             if (o->fmt >= CKQ_STEP_QUANTIZE_Q8_K && o->fmt <= CKQ_STEP_SWIGLU_Q8_K) {
-                const int rc = issue_producer(o, stream);
+                int taken;
+                int rc = issue_fused(ops, i, nops, stream, &taken);
+                if (!rc && !taken) {
+                    rc = issue_producer(o, stream);
+                    taken = 1;
+                }
                 if (rc) return rc;
-                ++i;
+                i += taken;
                 continue;
             }
             if (o->fmt & CKQ_ACT_F32) {              /* fp32 activations: the dequant-dot kernels, one launch per entry */

@@ -490,6 +490,36 @@ extern "C" int ckq_launch_gemv_group(int fmt, int n, float *const *y, const void
     return launch_gemv_args(fmt, a, grp, K, stream);
 }
 
+extern "C" int ckq_launch_gemv_pro(int fmt, int n, float *const *y, const void *const *W, const float *const *bias, const int *rows, const long *ldys,
+                                   int K, int ntok, const float *x, const float *gamma, float eps, long stride, void *xq, void *stream)
+{
+    if (n < 1 || n > CKQ_GROUP_MAX || ntok < 1 || ntok > CKQ_STREAM_TOKENS || K < 256 || K > 2048 || K % 256 || stride < K || stride % 4) return CKQ_ENOGROUP;
+    const size_t wblock = fmt == CKQ_FMT_Q4_K ? 144 : fmt == CKQ_FMT_Q5_K ? 176 : fmt == CKQ_FMT_Q6_K ? 210 : 0;
+    if (!wblock || !x || !xq) return CKQ_ENOGROUP;
+    const size_t xbytes = ((size_t)(ntok - 1) * (size_t)stride + (size_t)K) * 4, qbytes = (size_t)ntok * (size_t)(K / 256) * 292;
+    if (ckq_ranges_overlap(xq, qbytes, x, xbytes) || (gamma && ckq_ranges_overlap(xq, qbytes, gamma, (size_t)K * 4))) return CKQ_ENOGROUP;
+    GemvArgs a = {};
+    GemvGroup grp = k_no_group;
+    for (int i = 0; i < n; ++i) {
+        if (!y[i] || !W[i] || rows[i] <= 0 || ldys[i] < rows[i] || ldys[i] > 0x7fffffff || take_rows16(fmt, ntok, (size_t)rows[i], K, false)) return CKQ_ENOGROUP;
+        /* every block reads x: nothing it is made of may be written by the launch before the last has, nor xq read */
+        const size_t ybytes = ((size_t)(ntok - 1) * (size_t)ldys[i] + (size_t)rows[i]) * 4;
+        if (ckq_ranges_overlap(y[i], ybytes, x, xbytes) || (gamma && ckq_ranges_overlap(y[i], ybytes, gamma, (size_t)K * 4)) || ckq_ranges_overlap(y[i], ybytes, xq, qbytes) ||
+            ckq_ranges_overlap(xq, qbytes, W[i], (size_t)rows[i] * (size_t)(K / 256) * wblock) || (bias[i] && ckq_ranges_overlap(xq, qbytes, bias[i], (size_t)rows[i] * 4)))
+            return CKQ_ENOGROUP;
+        if (rows[i] > a.nrows) a.nrows = rows[i];
+        if (i) {
+            grp.y[i - 1] = y[i]; grp.W[i - 1] = (const uint8_t *)W[i]; grp.bias[i - 1] = bias[i]; grp.nrows[i - 1] = rows[i]; grp.ldy[i - 1] = (int)ldys[i];
+        }
+    }
+    grp.n = n;
+    a.y = y[0]; a.W = (const uint8_t *)W[0]; a.bias = bias[0]; a.ntok = ntok; a.row1 = rows[0]; a.ldy = ldys[0];
+    a.npos = K / 64; a.wrow = (long)((size_t)(K / 256) * wblock); a.xrow = (long)(K / 256) * 292;
+    const GemvPro pro = {x, gamma, (uint8_t *)xq, stride, eps};
+    return fmt == CKQ_FMT_Q4_K ? ckq_gemv_pro_launch_q4k(a, grp, pro, (hipStream_t)stream) : fmt == CKQ_FMT_Q5_K ? ckq_gemv_pro_launch_q5k(a, grp, pro, (hipStream_t)stream)
+         : ckq_gemv_pro_launch_q6k(a, grp, pro, (hipStream_t)stream);
+}
+
 static int launch_gemv_args(int fmt_flags, GemvArgs &a, const GemvGroup &grp, int K, void *stream, const GemmOpts &opts)
 {
     int fmt = fmt_flags;

@@ -62,6 +62,12 @@ int ckq_launch_gemv_group(int fmt, int n, float *const *y, const void *const *W,
                           const float *const *bias, const int *rows, const long *ldys, int K, int ntok,
                           int32_t *subdots, void *stream);
 
+/* A producer step and the n (1..4) matmuls that read its result as one launch: xq = Q8_K blocks of RMSNorm(x) gamma (gamma
+ * non-NULL) or of x, `ntok` rows of K floats `stride` apart, and y[i] = W[i] xq (+ bias[i]), every buffer with the bits of the steps one
+ * by one.  CKQ_ENOGROUP where they are better (or have to be) launched one by one. */
+int ckq_launch_gemv_pro(int fmt, int n, float *const *y, const void *const *W, const float *const *bias, const int *rows, const long *ldys,
+                        int K, int ntok, const float *x, const float *gamma, float eps, long stride, void *xq, void *stream);
+
 /* n (2..4) weight matrices of one format against the same M x K quantized activations as one
  * matrix-core launch (tile kernels or 16-row tiles); CKQ_ENOGROUP when the matrices should be launched one by one instead. */
 int ckq_launch_gemm_group(int fmt, int n, float *const *C, const void *const *B, const void *A,

@@ -57,6 +57,12 @@ __device__ __forceinline__ void rms_stage(float *xs, int D, int b, int lane, con
     p[3 * rms_pitch(D)] = v.w;
 }
 
+__device__ __forceinline__ float4 rms_unstage(const float *xs, int D, int b, int lane)
+{
+    const float *p = xs + 4 * (lane & 1) * rms_pitch(D) + 32 * b + (lane >> 1);
+    return make_float4(p[0], p[rms_pitch(D)], p[2 * rms_pitch(D)], p[3 * rms_pitch(D)]);
+}
+
 /* Thread j < 8 of the block walks chain j and leaves its sum behind the row.  The chain is serial, one multiply-add
  * after another; the 32 values of the next 256-block are read while those of this one are added. */
 __device__ __forceinline__ void rms_chain(float *xs, int D, int j)

@@ -1564,3 +1564,42 @@ def test_gemm_mfma_q8_0_tiles_and_teams(M, N, K):
     bound = (A.abs() @ B.abs().T) * (K // 32 + 4) * 2.0 ** -24 + bias.abs().double() * 2.0 ** -23
     assert bool((torch.isfinite(bound)).all())
     assert float(((y - A @ B.T).abs() / bound).max()) <= 1.0
+
+
+@pytest.mark.parametrize("fmt,M,D,N", [("q4_k", 1, 768, (768, 64, 64)), ("q5_k", 1, 1024, (1024, 128, 128)), ("q6_k", 1, 2048, (2048, 17)), ("q5_k", 2, 1280, (200, 130, 7, 64)),
+                                       ("q4_k", 3, 1024, (1000, 128, 1)), ("q5_k", 4, 1024, (1024, 128, 128)), ("q6_k", 4, 1792, (31,)), ("q4_k", 5, 1024, (130, 130)),
+                                       ("q5_k", 8, 768, (65, 3)), ("q4_k", 1, 512, (512,)), ("q6_k", 4, 256, (300, 9)), ("q4_k", 1, 2304, (300,)), ("q5_k", 1, 1024, (40000,))])
+@pytest.mark.parametrize("step", ["rms", "quantize"])
+def test_sequence_producer_joined_with_its_matmuls(fmt, M, D, N, step):
+    """A producer step and the matmuls behind it, narrow ones among them, on both sides of the sizes that share a launch: every buffer has the bits
+    of the steps one by one.  Rows of zeros, a row stride, bias, and results that overlap the input (never one launch)."""
+    import torch
+    L = ckq.lib()
+    ld = D + 8 if step == "rms" else D
+    tag = P.STEP["rmsnorm_q8_k" if step == "rms" else "quantize_q8_k"]
+    x = T.normal(M * ld, 0.0, 1.0, 9900 + D).reshape(M, ld)
+    if M > 1:
+        x[1, :] = 0.0
+    x[0, 256:512] = 0.0
+    gamma = P.to_device(T.normal(D, 1.0, 0.2, 9901))
+    Ws = [P.to_device(T.random_blocks(fmt, n * (D // 256), 9902 + n)) for n in N]
+    bias = P.to_device(T.normal(N[0], 0.0, 0.5, 9903))
+
+    def run(one_by_one, overlap):
+        xd = P.to_device(x.reshape(-1))
+        xq = torch.full((M * (D // 256) * 292,), 77, dtype=torch.uint8, device="cuda")
+        ys = [torch.full((M, n + 3), 7.0, device="cuda") for n in N]
+        ops = [P.MatmulOp(tag, M, 0, D, ld, xd.data_ptr(), gamma.data_ptr() if step == "rms" else None, None, xq.data_ptr(), 1e-5)]
+        for i, n in enumerate(N):
+            y = xd if overlap and i == 0 else ys[i]
+            ops.append(P.MatmulOp(P.FMT[fmt], M, n, D, n + 3, xq.data_ptr(), Ws[i].data_ptr(), bias.data_ptr() if i == 0 else None, y.data_ptr(), 0.0))
+        for part in ([[o] for o in ops] if one_by_one else [ops]):
+            arr = (P.MatmulOp * len(part))(*part)
+            P.check(L.ckq_matmul_sequence_dev(ctypes.cast(arr, ctypes.c_void_p), len(part), 1, P._stream()), "sequence")
+        return [xd, xq] + ys
+    say("joined", fmt, M, D, N, step)
+    for overlap in (False, True):
+        if overlap and (N[0] + 3) * M > M * ld:
+            continue
+        for a, b in zip(run(False, overlap), run(True, overlap)):
+            assert torch.equal(a, b)
