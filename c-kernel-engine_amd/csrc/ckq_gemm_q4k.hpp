@@ -25,6 +25,7 @@ __device__ __forceinline__ u32 bf16_pair(float lo, float hi)
 
 /* 96-token tiles, one block per tile, no K split (ckq_gemm_q4k_t96.hip).  g: A, B, bias, C, M, N, nb, ldc, nnt
  * and the dump pointer set by the caller; for the grouped form A, M and nb. */
+constexpr int T96_TOKENS = 96;
 int gemm_q4k_t96_token_tiles(int M);
 int launch_gemm_q4k_t96(GemmArgs g, hipStream_t s);
 int launch_gemm_q4k_t96_group(GemmArgs g, const GemmGroupIn &in, hipStream_t s);

@@ -20,7 +20,7 @@
 #include "ckq_gemm_q4k.hpp"
 #include <type_traits>
 
-constexpr int T96_BM = 96;
+constexpr int T96_BM = T96_TOKENS;
 constexpr int T96_BN = GEMM_TILE_ROWS;
 
 /* Token scales and bsums of one 256-block of 96 tokens: as stored (filled by global->LDS copies; the second
@@ -200,14 +200,33 @@ __global__ void __launch_bounds__(256, DUMP ? 1 : WPE) gemm_q4k_t96_kernel(GemmA
     const int tid = threadIdx.x, lane = tid & 63;
     const int col = lane & 31, half = lane >> 5;
 
-    /* tile of this block: full token tiles first (token tiles fastest, so neighbours share weights), then
-     * the partial token tile of every weight-row tile */
-    const GemmWork work = gemm_work(a, a.nb);
-    const int id = work.id, xcd = id & 7, seq = id >> 3;
-    const int nfull = a.M / BM, ncg = (work.nnt + 7) >> 3;
-    int cg, tt;
-    if (seq < ncg * nfull) { cg = seq / nfull; tt = seq - cg * nfull; }
-    else { cg = seq - ncg * nfull; tt = nfull; }
+    /* tile of this block: full token tiles first (token tiles fastest, so neighbours share weights), of a group those of
+     * all matrices, then the partial token tile of every weight-row tile */
+    GemmWork work = gemm_work(a, a.nb);
+    const int nfull = a.M / BM;
+    int id = work.id;
+    bool whole;
+    if (a.ngroup > 1) {
+        auto cols8 = [](const GemmProblem &p) { return (p.nnt + 7) & ~7; };
+        int wholes = cols8(a.grp[0]) + cols8(a.grp[1]);
+        if (a.ngroup > 2) wholes += cols8(a.grp[2]);
+        if (a.ngroup > 3) wholes += cols8(a.grp[3]);
+        wholes *= nfull;
+        id = blockIdx.x;
+        whole = id < wholes;
+        if (!whole) id -= wholes;
+        const int per = whole ? nfull : 1;
+        GemmProblem g = a.grp[0];
+        int n = per * cols8(g);
+        if (id >= n) { id -= n; g = a.grp[1]; n = per * cols8(g); }
+        if (a.ngroup > 2 && id >= n) { id -= n; g = a.grp[2]; n = per * cols8(g); }
+        if (a.ngroup > 3 && id >= n) { id -= n; g = a.grp[3]; }
+        work = {id, 0, a.nb, {g.C, g.ldc, g.bias}, g.B, g.N, g.nnt};
+    } else {
+        whole = id < nfull * ((work.nnt + 7) & ~7);
+        if (!whole) id -= nfull * ((work.nnt + 7) & ~7);
+    }
+    const int xcd = id & 7, seq = id >> 3, cg = whole ? seq / nfull : seq, tt = whole ? seq - cg * nfull : nfull;
     const int nt = cg * 8 + xcd;
     if (nt >= work.nnt) return;
     const int t0 = tt * BM, n0 = nt * T96_BN;

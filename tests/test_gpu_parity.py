@@ -1603,3 +1603,29 @@ def test_sequence_producer_joined_with_its_matmuls(fmt, M, D, N, step):
             continue
         for a, b in zip(run(False, overlap), run(True, overlap)):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("M,Ns,K", [(97, (22016,), 1024), (160, (16777,), 1024), (192, (11008,), 768), (512, (5120,), 1536), (481, (6100,), 1024), (300, (6701,), 2816),
+                                    (90, (26000,), 1024), (225, (9728, 9728), 1536), (288, (4096, 1024, 1024, 3000), 1280), (512, (6400,), 512)])
+def test_gemm_q4_k_token_tile_choice(M, Ns, K):
+    """Sizes on both sides of the choice between 64- and 96-token tiles (blocks of an XCD on its CUs), single matrices and groups: the bits of
+    64-token tiles."""
+    import torch
+    L = ckq.lib()
+    say("q4_k tile choice", M, Ns, K)
+    xq = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, 9950)), "q8_k", M)
+    Ws = [P.to_device(T.random_blocks("q4_k", n * (K // 256), 9951 + n)) for n in Ns]
+    got = {}
+    try:
+        L.ckq_set_gemm_policy(1)
+        for tile in (0, 64, 96):
+            L.ckq_set_prefill_variant(P.FMT["q4_k"], tile)
+            ys = [torch.full((M, n), 7.0, device="cuda") for n in Ns]
+            P.dev_matmul_sequence([("q4_k", xq, W, None, y, M, n, K) for W, y, n in zip(Ws, ys, Ns)])
+            got[tile] = ys
+    finally:
+        L.ckq_set_gemm_policy(0)
+        L.ckq_set_prefill_variant(P.FMT["q4_k"], 0)
+    for tile in (0, 96):
+        for a, b in zip(got[tile], got[64]):
+            assert torch.equal(a, b)
