@@ -17,7 +17,7 @@ typedef __attribute__((address_space(3))) void ckq_lds_void;
 typedef const __attribute__((address_space(1))) void ckq_glb_void;
 
 /* One weight matrix of a grouped launch: several matrices that multiply the same activations (Q/K/V,
- * gate/up) share a grid; a matrix owns the block ids [id0, id0 + ntt * round_up(nnt, 8)). */
+ * gate/up) share a grid; a matrix owns the block ids [id0, id0 + gemm_blocks(ntt, nnt)). */
 constexpr int GEMM_GROUP_MAX = 4;
 struct GemmProblem {
     const uint8_t *B;
@@ -103,6 +103,20 @@ __device__ __forceinline__ GemmWork gemm_work(const GemmArgs &a, int k_steps)
     return {id, k0, min(k_steps, k0 + a.k_per),
             {a.part + (size_t)blockIdx.y * (size_t)a.M * (size_t)a.N, (long)a.N, nullptr}, a.B, a.N, a.nnt};
 }
+
+/* The tiles of a launch, ntt token tiles of nnt tiles of weight rows, token tiles fastest so that neighbours share weights, are dealt
+ * to the XCDs in eight equal runs (blocks go round the XCDs in turn, and each has an L2 of its own): whole rows of
+ * tiles per XCD leave some with a row more, and with few rows CUs there with two or three tiles beside others with one (us, rows of
+ * tiles -> runs: Q6_K 680 tokens x 2111 rows x 4352 57.8 -> 32.6, Q5_K 67 x 1509 x 10240 32.6 -> 21.3, Q4_K 339 x 1432 x 6656 33.0 -> 20.8;
+ * 60 random sizes 0.5 to 5 % on average, the same bits).  gemm_blocks: block ids to launch; false: no tile. */
+__device__ __forceinline__ bool gemm_tile(int id, int ntt, int nnt, int &nt, int &tt)
+{
+    const int total = ntt * nnt, xcd = id & 7, seq = id >> 3, t = xcd * (total >> 3) + min(xcd, total & 7) + seq;
+    nt = t / ntt;
+    tt = t - nt * ntt;
+    return seq < (total >> 3) + (xcd < (total & 7) ? 1 : 0);
+}
+__host__ __device__ __forceinline__ constexpr int gemm_blocks(int ntt, int nnt) { return (ntt * nnt + 7) & ~7; }
 
 /* Split K when the tile grid leaves most of the chip idle: `tiles` blocks of
  * `k_steps` loop iterations each.  Returns the number of splits (1 = none) so
@@ -222,7 +236,8 @@ __device__ __forceinline__ void gemm_store(float *p, float v)
 }
 
 /* Grouped launch: the matrices of `in` against the same M x K activations, as one grid (no K split; the
- * callers group only what fills the chip without one).  rows_per_tile = weight rows of a block's tile. */
+ * callers group only what fills the chip without one).  rows_per_tile = weight rows of a block's tile; last_apart: the last token tile
+ * of every matrix has block ids of its own (ckq_gemm_q4k_t96.hip). */
 struct GemmGroupIn {
     int          n;
     const void  *B[GEMM_GROUP_MAX];
@@ -241,14 +256,14 @@ static int gemm_group_tiles(const GemmGroupIn &in, int M, int tokens_per_tile, i
     return tiles;
 }
 template <class Kernel>
-static int gemm_launch_grouped(Kernel kernel, GemmArgs &g, const GemmGroupIn &in, hipStream_t s, unsigned threads = 256)
+static int gemm_launch_grouped(Kernel kernel, GemmArgs &g, const GemmGroupIn &in, hipStream_t s, unsigned threads = 256, int last_apart = 0)
 {
     unsigned grid = 0;
     g.ngroup = in.n;
     for (int p = 0; p < in.n; ++p) {
         const int nnt = (in.N[p] + GEMM_TILE_ROWS - 1) / GEMM_TILE_ROWS;
         g.grp[p] = {(const uint8_t *)in.B[p], in.bias[p], in.C[p], in.ldc[p], in.N[p], nnt, (int)grid};
-        grid += (unsigned)g.ntt * (unsigned)((nnt + 7) / 8 * 8);
+        grid += (unsigned)gemm_blocks(g.ntt - last_apart, nnt) + (last_apart ? (unsigned)gemm_blocks(1, nnt) : 0u);
     }
     g.B = g.grp[0].B; g.bias = g.grp[0].bias; g.C = g.grp[0].C; g.N = g.grp[0].N; g.ldc = g.grp[0].ldc; g.nnt = g.grp[0].nnt;
     g.splits = 1; g.k_per = 0; g.part = nullptr;

@@ -203,10 +203,8 @@ __global__ void __launch_bounds__(256 * KG, KG == 2 ? 1 : WPE) gemm_q4k_mfma_ker
     GemmStage *const stage = stage_all[grp];
 
     const GemmWork work = gemm_work(a, a.nb);
-    const int id = work.id, xcd = id & 7, seq = id >> 3;
-    const int tt = seq % a.ntt;
-    const int nt = (seq / a.ntt) * 8 + xcd;
-    if (nt >= work.nnt) return;
+    int nt, tt;
+    if (!gemm_tile(work.id, a.ntt, work.nnt, nt, tt)) return;
     const int t0 = tt * BM, n0 = nt * GEMM_BN;
     const u32 wstride = (u32)a.nb * 144u, xstride = (u32)a.nb * 292u;
     const int b0 = work.k0, b1 = work.k1, last = b1 - 1;
@@ -354,23 +352,31 @@ __global__ void __launch_bounds__(256 * KG, KG == 2 ? 1 : WPE) gemm_q4k_mfma_ker
 }
 
 /* Which token tile a launch takes.  A 96-token tile (ckq_gemm_q4k_t96.hip) costs less per token but comes in blocks that run longer and
- * leaves a remainder of 32, 64 or 96 columns, so it is a matter of how the blocks of an XCD (32 CUs, two slots each; `cols` tiles of
- * weight rows on the fullest one) fall on its CUs.  us for nb 256-blocks of K, from launches of 64 to 600 tokens and K of 512 to 11008:
+ * leaves a remainder of 32, 64 or 96 columns, so it is a matter of how the blocks of an XCD (32 CUs, two
+ * slots each) fall on its CUs.  us for nb 256-blocks of K, from launches of 64 to 600 tokens and K of 512 to 11008:
  *   64 tokens   6.1 + 2.2 nb up to two blocks on a CU, 9.2 + 3.3 nb up to three, 11 + 4.6 nb beyond
  *   96 tokens   8 + 1.6 nb with a CU per block, 2.0 / 2.35 / 2.85 nb where only a remainder of 32 / 64 / 96 tokens doubles up, 2.85 nb up to two
  * Measured, us, 64 -> 96: 512 x 5120 x 4096 (tokens, rows, K) 40.5 -> 33.7, 160 x 22016 x 4096 59.5 -> 45.1, 192 x 22016 x 4096 61.0 -> 54.5,
- * 512 x 6144 x 4096 42.6 -> 39.1, 384 x 11008 x 1024 22.1 -> 20.0; but 512 x 6400 x 4096 (35 whole tiles on an XCD) 42.9 -> 52.6,
- * 256 x 22016 x 4096 63.5 -> 74.4.  Deeper grids: from a round and a half of its blocks and 576 tokens on (512 x 22016 121.2 -> 121.4).  Up to 256 tiles of 64 tokens two groups of waves per tile stand against it (512 x 4096: 25.5, 31.8). */
+ * 512 x 6144 x 4096 42.6 -> 39.1, 384 x 11008 x 1024 22.1 -> 20.0; 512 x 6400 x 4096 42.7 -> 40.1; but
+ * 320 x 10900 x 4096 (33 whole tiles on an XCD) 43.3 -> 53.1, 256 x 22016 x 4096 63.5 -> 74.4.  Deeper grids: from a round and a half of its
+ * blocks and 576 tokens on (512 x 22016 121.2 -> 121.4).  Up to 256 tiles of 64 tokens two groups of waves per tile stand against it
+ * (512 x 4096: 25.5, 31.8). */
 static std::atomic<int> g_q4k_tile{0};
 extern "C" void ckq_launch_set_q4k_tile(int tokens) { g_q4k_tile.store(tokens == 64 || tokens == 96 ? tokens : 0); }
 bool gemm_q4k_forced() { return g_q4k_tile.load(std::memory_order_relaxed) != 0; }
-static bool q4k_take_t96(int M, int nb, int tiles64, int cols, int blocks96)
+static bool q4k_take_t96(int M, int nb, int tiles64, int blocks96, const int *nnt, int n)
 {
     const int forced = g_q4k_tile.load(std::memory_order_relaxed);
     if (forced) return forced == 96;
     if (tiles64 <= 256) return false;
     constexpr int CUS = 32;                   /* of an XCD; two slots each */
-    const int left = M % T96_TOKENS, whole = cols * (M / T96_TOKENS), part = left ? cols : 0, t64 = cols * ((M + GEMM_BM - 1) / GEMM_BM);
+    const int left = M % T96_TOKENS;
+    auto on_xcd = [&](int ntt) {              /* tiles that one gets */
+        int t = 0;
+        for (int p = 0; p < n; ++p) t += gemm_blocks(ntt, nnt[p]) / 8;
+        return t;
+    };
+    const int whole = on_xcd(M / T96_TOKENS), part = left ? on_xcd(1) : 0, t64 = on_xcd((M + GEMM_BM - 1) / GEMM_BM);
     if (whole > 2 * CUS || whole + part > 2 * CUS) return M >= 576 && 2 * blocks96 >= 3 * (16 * CUS);
     const float k = (float)nb, c64 = t64 <= 2 * CUS ? 6.1f + 2.2f * k : t64 <= 3 * CUS ? 9.2f + 3.3f * k : 11.0f + 4.6f * k;
     const float c96 = 8.0f + k * (whole + part <= CUS ? 1.6f : whole > CUS || left > 64 ? 2.85f : left > 32 ? 2.35f : 2.0f);
@@ -400,7 +406,6 @@ int launch_gemm_q4k_mfma(const void *A, const void *B, const float *bias, float 
     if ((long long)g.nb * 292 * GEMM_BN >= (1ll << 31)) return (int)hipErrorInvalidValue;
     g.ntt = (M + GEMM_BM - 1) / GEMM_BM;
     g.nnt = (N + GEMM_BN - 1) / GEMM_BN;
-    const int nnt8 = (g.nnt + 7) / 8 * 8;
     /* One tile per CU at most (with the K split the launch will choose) and a
      * long enough K: two groups of waves per tile put a second wave on every
      * SIMD (4096x11008 at M = 512: 80 -> 70 us).  With more tiles than CUs two
@@ -408,17 +413,17 @@ int launch_gemm_q4k_mfma(const void *A, const void *B, const float *bias, float 
      * (11008x4096: 78 us against 88). */
     const int tiles = g.ntt * g.nnt, sp = gemm_choose_splits(tiles, g.nb);
     const bool two_groups = tiles * sp <= 256 && (g.nb + sp - 1) / sp >= 8;
-    if (q4k_take_t96(M, g.nb, tiles, nnt8 / 8, gemm_q4k_t96_token_tiles(M) * g.nnt)) return launch_gemm_q4k_t96(g, s);
+    if (q4k_take_t96(M, g.nb, tiles, gemm_q4k_t96_token_tiles(M) * g.nnt, &g.nnt, 1)) return launch_gemm_q4k_t96(g, s);
     if (sums) {
 #if CKQ_WITH_DUMP
-        if (two_groups) return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 2, true>, g, (unsigned)(g.ntt * nnt8), g.nb, s, 512);
-        return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 1, true>, g, (unsigned)(g.ntt * nnt8), g.nb, s, 256);
+        if (two_groups) return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 2, true>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s, 512);
+        return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 1, true>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s, 256);
 #else
         return CKQ_ENODUMP;
 #endif
     }
-    if (two_groups) return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 2>, g, (unsigned)(g.ntt * nnt8), g.nb, s, 512);
-    return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 1>, g, (unsigned)(g.ntt * nnt8), g.nb, s, 256);
+    if (two_groups) return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 2>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s, 512);
+    return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 1>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s, 256);
 }
 
 bool gemm_q4k_group_chains(const GemmGroupIn &in, int M, int K, GemmChains *ch)
@@ -435,9 +440,9 @@ int launch_gemm_q4k_mfma_group(const void *A, const GemmGroupIn &in, int M, int 
     GemmArgs g = {};
     g.A = (const uint8_t *)A; g.M = M; g.nb = K / 256;
     if ((long long)g.nb * 292 * GEMM_BN >= (1ll << 31)) return (int)hipErrorInvalidValue;
-    int cols = 0;
-    for (int p = 0; p < in.n; ++p) cols += ((in.N[p] + GEMM_BN - 1) / GEMM_BN + 7) / 8;
-    if (q4k_take_t96(M, g.nb, tiles, cols, gemm_group_tiles(in, M, T96_TOKENS))) return launch_gemm_q4k_t96_group(g, in, s);
+    int nnt[GEMM_GROUP_MAX];
+    for (int p = 0; p < in.n; ++p) nnt[p] = (in.N[p] + GEMM_BN - 1) / GEMM_BN;
+    if (q4k_take_t96(M, g.nb, tiles, gemm_group_tiles(in, M, T96_TOKENS), nnt, in.n)) return launch_gemm_q4k_t96_group(g, in, s);
     g.ntt = (M + GEMM_BM - 1) / GEMM_BM;
     /* as for one matrix: two groups of waves per tile while every tile gets a CU of its own */
     if (tiles <= 256 && g.nb >= 8) return gemm_launch_grouped(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 2>, g, in, s, 512);

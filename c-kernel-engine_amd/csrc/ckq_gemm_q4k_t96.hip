@@ -204,31 +204,30 @@ __global__ void __launch_bounds__(256, DUMP ? 1 : WPE) gemm_q4k_t96_kernel(GemmA
      * all matrices, then the partial token tile of every weight-row tile */
     GemmWork work = gemm_work(a, a.nb);
     const int nfull = a.M / BM;
+    auto wholes = [&](int nnt) { return gemm_blocks(nfull, nnt); };
     int id = work.id;
     bool whole;
     if (a.ngroup > 1) {
-        auto cols8 = [](const GemmProblem &p) { return (p.nnt + 7) & ~7; };
-        int wholes = cols8(a.grp[0]) + cols8(a.grp[1]);
-        if (a.ngroup > 2) wholes += cols8(a.grp[2]);
-        if (a.ngroup > 3) wholes += cols8(a.grp[3]);
-        wholes *= nfull;
+        int all = wholes(a.grp[0].nnt) + wholes(a.grp[1].nnt);
+        if (a.ngroup > 2) all += wholes(a.grp[2].nnt);
+        if (a.ngroup > 3) all += wholes(a.grp[3].nnt);
         id = blockIdx.x;
-        whole = id < wholes;
-        if (!whole) id -= wholes;
-        const int per = whole ? nfull : 1;
+        whole = id < all;
+        if (!whole) id -= all;
+        auto blocks = [&](const GemmProblem &p) { return whole ? wholes(p.nnt) : gemm_blocks(1, p.nnt); };
         GemmProblem g = a.grp[0];
-        int n = per * cols8(g);
-        if (id >= n) { id -= n; g = a.grp[1]; n = per * cols8(g); }
-        if (a.ngroup > 2 && id >= n) { id -= n; g = a.grp[2]; n = per * cols8(g); }
+        int n = blocks(g);
+        if (id >= n) { id -= n; g = a.grp[1]; n = blocks(g); }
+        if (a.ngroup > 2 && id >= n) { id -= n; g = a.grp[2]; n = blocks(g); }
         if (a.ngroup > 3 && id >= n) { id -= n; g = a.grp[3]; }
         work = {id, 0, a.nb, {g.C, g.ldc, g.bias}, g.B, g.N, g.nnt};
     } else {
-        whole = id < nfull * ((work.nnt + 7) & ~7);
-        if (!whole) id -= nfull * ((work.nnt + 7) & ~7);
+        whole = id < wholes(work.nnt);
+        if (!whole) id -= wholes(work.nnt);
     }
-    const int xcd = id & 7, seq = id >> 3, cg = whole ? seq / nfull : seq, tt = whole ? seq - cg * nfull : nfull;
-    const int nt = cg * 8 + xcd;
-    if (nt >= work.nnt) return;
+    int nt, tt;
+    if (!gemm_tile(id, whole ? nfull : 1, work.nnt, nt, tt)) return;
+    if (!whole) tt = nfull;
     const int t0 = tt * BM, n0 = nt * T96_BN;
     const int ng = min(3, (a.M - t0 + 31) >> 5);
     const int tlim = a.M - 1 - t0;                 /* last token of the matrix, counted from t0 */
@@ -395,7 +394,8 @@ int launch_gemm_q4k_t96(GemmArgs g, hipStream_t s)
 {
     g.ntt = gemm_q4k_t96_token_tiles(g.M);
     g.ngroup = 0; g.splits = 1; g.k_per = 0; g.part = nullptr;
-    const unsigned grid = (unsigned)g.ntt * (unsigned)((g.nnt + 7) / 8 * 8);
+    const int last = g.M % T96_BM != 0;
+    const unsigned grid = (unsigned)(gemm_blocks(g.ntt - last, g.nnt) + (last ? gemm_blocks(1, g.nnt) : 0));
     if (g.dump) {
 #if CKQ_WITH_DUMP
         hipLaunchKernelGGL((gemm_q4k_t96_kernel<CKQ_GEMM_WPE, true>), dim3(grid), dim3(256), 0, s, g);
@@ -412,5 +412,5 @@ int launch_gemm_q4k_t96(GemmArgs g, hipStream_t s)
 int launch_gemm_q4k_t96_group(GemmArgs g, const GemmGroupIn &in, hipStream_t s)
 {
     g.ntt = gemm_q4k_t96_token_tiles(g.M);
-    return gemm_launch_grouped(gemm_q4k_t96_kernel<CKQ_GEMM_WPE, false>, g, in, s, 256);
+    return gemm_launch_grouped(gemm_q4k_t96_kernel<CKQ_GEMM_WPE, false>, g, in, s, 256, g.M % T96_BM != 0);
 }

@@ -192,10 +192,8 @@ __global__ void __launch_bounds__(256, 1) gemm_q5k_mfma_kernel(GemmArgs a)
 
     /* token tiles fastest inside an XCD, so each XCD's L2 sees a weight tile once */
     const GemmWork work = gemm_work(a, a.nb);
-    const int id = work.id, xcd = id & 7, seq = id >> 3;
-    const int tt = seq % a.ntt;
-    const int nt = (seq / a.ntt) * 8 + xcd;
-    if (nt >= work.nnt) return;
+    int nt, tt;
+    if (!gemm_tile(work.id, a.ntt, work.nnt, nt, tt)) return;
     const int t0 = tt * BM, n0 = nt * GEMM5_BN;
     const u32 wstride = (u32)a.nb * 176u, xstride = (u32)a.nb * 292u;
     const int b0 = work.k0, b1 = work.k1, last = b1 - 1;
@@ -336,10 +334,8 @@ __global__ void __launch_bounds__(256, 2) gemm_q5k_pair_kernel(GemmArgs a)
     const int col = lane & 31, half = lane >> 5;
 
     const GemmWork work = gemm_work(a, a.nb);
-    const int id = work.id, xcd = id & 7, seq = id >> 3;
-    const int tt = seq % a.ntt;
-    const int nt = (seq / a.ntt) * 8 + xcd;
-    if (nt >= work.nnt) return;
+    int nt, tt;
+    if (!gemm_tile(work.id, a.ntt, work.nnt, nt, tt)) return;
     const int t0 = tt * BM, n0 = nt * GEMM5_BN;
     const u32 wstride = (u32)a.nb * 176u, xstride = (u32)a.nb * 292u;
     const int b0 = work.k0, b1 = work.k1, last = b1 - 1;
@@ -472,21 +468,20 @@ int launch_gemm_q5k_mfma(const void *A, const void *B, const float *bias, float 
     if ((long long)g.nb * 292 * 128 >= (1ll << 31)) return (int)hipErrorInvalidValue;
     g.ntt = (M + GEMM5_BM - 1) / GEMM5_BM;
     g.nnt = (N + GEMM5_BN - 1) / GEMM5_BN;
-    const int nnt8 = (g.nnt + 7) / 8 * 8;
     if (q5k_take_pair(g.ntt * g.nnt)) {
 #if CKQ_WITH_DUMP
-        if (sums) return gemm_launch_split(gemm_q5k_pair_kernel<true>, g, (unsigned)(g.ntt * nnt8), g.nb, s);
+        if (sums) return gemm_launch_split(gemm_q5k_pair_kernel<true>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s);
 #else
         if (sums) return CKQ_ENODUMP;
 #endif
-        return gemm_launch_split(gemm_q5k_pair_kernel<false>, g, (unsigned)(g.ntt * nnt8), g.nb, s);
+        return gemm_launch_split(gemm_q5k_pair_kernel<false>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s);
     }
 #if CKQ_WITH_DUMP
-    if (sums) return gemm_launch_split(gemm_q5k_mfma_kernel<true>, g, (unsigned)(g.ntt * nnt8), g.nb, s);
+    if (sums) return gemm_launch_split(gemm_q5k_mfma_kernel<true>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s);
 #else
     if (sums) return CKQ_ENODUMP;
 #endif
-    return gemm_launch_split(gemm_q5k_mfma_kernel<false>, g, (unsigned)(g.ntt * nnt8), g.nb, s);
+    return gemm_launch_split(gemm_q5k_mfma_kernel<false>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s);
 }
 
 bool gemm_q5k_group_chains(const GemmGroupIn &in, int M, int K, GemmChains *ch)

@@ -184,10 +184,8 @@ __global__ void __launch_bounds__(256, 1) gemm_q6k_mfma_kernel(GemmArgs a)
 
     /* token tiles fastest inside an XCD, so each XCD's L2 sees a weight tile once */
     const GemmWork work = gemm_work(a, a.nb);
-    const int id = work.id, xcd = id & 7, seq = id >> 3;
-    const int tt = seq % a.ntt;
-    const int nt = (seq / a.ntt) * 8 + xcd;
-    if (nt >= work.nnt) return;
+    int nt, tt;
+    if (!gemm_tile(work.id, a.ntt, work.nnt, nt, tt)) return;
     const int t0 = tt * BM, n0 = nt * GEMM6_BN;
     const u32 wstride = (u32)a.nb * 210u, xstride = (u32)a.nb * 292u;
     const int b0 = work.k0, b1 = work.k1, last = b1 - 1;
@@ -346,10 +344,8 @@ __global__ void __launch_bounds__(256, 2) gemm_q6k_pair_kernel(GemmArgs a)
     const int col = lane & 31, half = lane >> 5;
 
     const GemmWork work = gemm_work(a, a.nb);
-    const int id = work.id, xcd = id & 7, seq = id >> 3;
-    const int tt = seq % a.ntt;
-    const int nt = (seq / a.ntt) * 8 + xcd;
-    if (nt >= work.nnt) return;
+    int nt, tt;
+    if (!gemm_tile(work.id, a.ntt, work.nnt, nt, tt)) return;
     const int t0 = tt * BM, n0 = nt * GEMM6_BN;
     const u32 wstride = (u32)a.nb * 210u, xstride = (u32)a.nb * 292u;
     const int b0 = work.k0, b1 = work.k1, last = b1 - 1;
@@ -489,34 +485,33 @@ int launch_gemm_q6k_mfma(const void *A, const void *B, const float *bias, float 
     /* lane offsets inside a tile are 32-bit */
     if ((long long)g.nb * 292 * 128 >= (1ll << 31)) return (int)hipErrorInvalidValue;
     g.nnt = (N + GEMM6_BN - 1) / GEMM6_BN;
-    const int nnt8 = (g.nnt + 7) / 8 * 8;
     if (q6k_take_pair(((M + 127) / 128) * g.nnt, ((M + 63) / 64) * g.nnt)) {
         g.ntt = (M + 63) / 64;
 #if CKQ_WITH_DUMP
-        if (sums) return gemm_launch_split(gemm_q6k_pair_kernel<2, true>, g, (unsigned)(g.ntt * nnt8), g.nb, s);
+        if (sums) return gemm_launch_split(gemm_q6k_pair_kernel<2, true>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s);
 #else
         if (sums) return CKQ_ENODUMP;
 #endif
-        return gemm_launch_split(gemm_q6k_pair_kernel<2>, g, (unsigned)(g.ntt * nnt8), g.nb, s);
+        return gemm_launch_split(gemm_q6k_pair_kernel<2>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s);
     }
     /* tiles of 128 tokens where they still give every CU work, else 64 */
     const int ntt4 = (M + 127) / 128;
     if (ntt4 * g.nnt > 128) {
         g.ntt = ntt4;
 #if CKQ_WITH_DUMP
-        if (sums) return gemm_launch_split(gemm_q6k_mfma_kernel<4, true>, g, (unsigned)(g.ntt * nnt8), g.nb, s);
+        if (sums) return gemm_launch_split(gemm_q6k_mfma_kernel<4, true>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s);
 #else
         if (sums) return CKQ_ENODUMP;
 #endif
-        return gemm_launch_split(gemm_q6k_mfma_kernel<4>, g, (unsigned)(g.ntt * nnt8), g.nb, s);
+        return gemm_launch_split(gemm_q6k_mfma_kernel<4>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s);
     }
     g.ntt = (M + 63) / 64;
 #if CKQ_WITH_DUMP
-    if (sums) return gemm_launch_split(gemm_q6k_mfma_kernel<2, true>, g, (unsigned)(g.ntt * nnt8), g.nb, s);
+    if (sums) return gemm_launch_split(gemm_q6k_mfma_kernel<2, true>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s);
 #else
     if (sums) return CKQ_ENODUMP;
 #endif
-    return gemm_launch_split(gemm_q6k_mfma_kernel<2>, g, (unsigned)(g.ntt * nnt8), g.nb, s);
+    return gemm_launch_split(gemm_q6k_mfma_kernel<2>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s);
 }
 
 bool gemm_q6k_group_chains(const GemmGroupIn &in, int M, int K, GemmChains *ch)

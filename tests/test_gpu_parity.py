@@ -1629,3 +1629,32 @@ def test_gemm_q4_k_token_tile_choice(M, Ns, K):
     for tile in (0, 96):
         for a, b in zip(got[tile], got[64]):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("M", [9, 65, 129, 200, 673])
+def test_gemm_mfma_tiles_over_the_xcds(fmt, M):
+    """Every tile is computed once whatever the numbers of tiles: 1 to 17 tiles of weight rows, 1 to 11 of tokens, split along K and not, one
+    matrix and a group.  Against the streaming kernel, whose terms and order differ: the bar of the other parity tests."""
+    import torch
+    L = ckq.lib()
+    for K in (256, 2304):
+        xq = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, 9960)), T.act_fmt(fmt), M)
+        Ns = (1, 129, 700, 900, 1100, 2049, 2100)
+        Ws = [P.to_device(T.random_blocks(fmt, n * (K // T.ELEMS[fmt]), 9961 + n)) for n in Ns]
+        say("tiles over the XCDs", fmt, M, K)
+
+        def run(policy, group):
+            L.ckq_set_gemm_policy(policy)
+            ys = [torch.full((M, n), 7.0, device="cuda") for n in Ns]
+            ops = [(fmt, xq, W, None, y, M, n, K) for W, y, n in zip(Ws, ys, Ns)]
+            for part in ([ops[:4], ops[4:]] if group else [[o] for o in ops]):
+                P.dev_matmul_sequence(part)
+            return ys
+        try:
+            want, one, grp = run(2, False), run(1, False), run(1, True)
+        finally:
+            L.ckq_set_gemm_policy(0)
+        for w, a, b in zip(want, one, grp):
+            bar = TOL * float(w.abs().max())
+            assert float((a - w).abs().max()) <= bar and float((b - w).abs().max()) <= bar
