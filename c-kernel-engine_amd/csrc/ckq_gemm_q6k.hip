@@ -449,27 +449,36 @@ __global__ void __launch_bounds__(256, 2) gemm_q6k_pair_kernel(GemmArgs a)
     }
 }
 
-/* Which launches take the paired kernel.  It spends 12 % more per token than the 128-token tiles at one block per CU
- * and about as much as the three-stage 64-token kernel, but its grid has 512 slots of 64 tokens instead of 256 of 128, and
- * a partly filled last round runs faster instead of costing a whole block time: it is taken when the 128-token grid
- * would waste a quarter or more of its last round (512 tokens x 11008 rows, K = 4096: 344 tiles on 256 CUs, 94.8 us;
- * paired 78.7) and there are at least 512 blocks of 64 tokens.  variant: 0 = by shape, 1 = never, 2 = always. */
+/* Which kernel a launch takes: 64-token tiles of one block per CU, 128-token tiles of one block per CU, or 64-token tiles of two
+ * (paired).  us for nb 256-blocks of K, from 70 launches of 33 to 900 tokens, 2000 to 40000 rows and K of 512 to 11008:
+ *   64 tokens    6.5 + 1.5 nb a round of 256 tiles
+ *   128 tokens   10 + 2.35 nb a round of 256 tiles
+ *   paired       7 + 2.9 nb a round of 512 tiles, a last round of up to 256 0.55 and a fuller one 0.85 of that
+ * Measured, us, 128 tokens -> 64: 48 x 32000 x 4096 (tokens, rows, K) 46.4 -> 32.1, 160 x 10000 x 4096 47.2 -> 31.3, 56 x 25595 x 6144
+ * 63.3 -> 43.0; 128 tokens -> paired: 266 x 35817 x 768 62.7 -> 45.8, 345 x 10391 x 512 16.6 -> 13.7, 473 x 20320 x 2304 92.1 -> 81.6;
+ * 512 x 11008 x 4096 95.6 -> 85.4; 128 tokens stay the fastest at 247 x 10593 x 3584 (43.2; 64 54.3, paired 48.9).  Every kernel gives the
+ * same bits where nothing is split along K, and up to 256 tiles of 64 tokens, where something may be, it is always the first.
+ * variant: 0 = by shape, 1 = never paired, 2 = always. */
 static std::atomic<int> g_q6k_variant{0};
 extern "C" void ckq_launch_set_q6k_variant(int variant) { g_q6k_variant.store(variant == 1 || variant == 2 ? variant : 0); }
 bool gemm_q6k_forced() { return g_q6k_variant.load(std::memory_order_relaxed) != 0; }
-static bool q6k_take_pair(int tiles128, int tiles64)
+enum { Q6K_64, Q6K_128, Q6K_PAIRED };
+static int q6k_form(int tiles64, int tiles128, int nb)
 {
     const int forced = g_q6k_variant.load(std::memory_order_relaxed);
-    if (forced) return forced == 2;
-    if (tiles64 < 512 || tiles128 <= 256) return false;
-    const int rounds = (tiles128 + 255) / 256;
-    return 4 * rounds * 256 >= 5 * tiles128;        /* ceil(r) / r >= 1.25 */
+    if (forced == 2) return Q6K_PAIRED;
+    if (tiles64 <= 256) return Q6K_64;
+    const float k = (float)nb, rest = (float)(tiles64 % 512 == 0 ? 0.0f : tiles64 < 512 ? 1.0f : tiles64 % 512 <= 256 ? 0.55f : 0.85f);
+    const float t64 = (float)((tiles64 + 255) / 256) * (6.5f + 1.5f * k), t128 = (float)((tiles128 + 255) / 256) * (10.0f + 2.35f * k);
+    const float paired = ((float)(tiles64 / 512) + rest) * (7.0f + 2.9f * k);
+    if (forced != 1 && paired <= t64 && paired <= 0.98f * t128) return Q6K_PAIRED;
+    return t64 < t128 ? Q6K_64 : Q6K_128;
 }
 
 GemmChains gemm_q6k_chains(int M, int N, int K)
 {
-    const int nnt = (N + GEMM6_BN - 1) / GEMM6_BN, t4 = (M + 127) / 128 * nnt, t2 = (M + 63) / 64 * nnt;
-    return gemm_chains_split(q6k_take_pair(t4, t2) || t4 <= 128 ? t2 : t4, K / 256);
+    const int tiles64 = (M + 63) / 64 * ((N + GEMM6_BN - 1) / GEMM6_BN);
+    return tiles64 <= 256 ? gemm_chains_split(tiles64, K / 256) : GemmChains{1, K / 256, 1};
 }
 
 int launch_gemm_q6k_mfma(const void *A, const void *B, const float *bias, float *C,
@@ -485,33 +494,21 @@ int launch_gemm_q6k_mfma(const void *A, const void *B, const float *bias, float 
     /* lane offsets inside a tile are 32-bit */
     if ((long long)g.nb * 292 * 128 >= (1ll << 31)) return (int)hipErrorInvalidValue;
     g.nnt = (N + GEMM6_BN - 1) / GEMM6_BN;
-    if (q6k_take_pair(((M + 127) / 128) * g.nnt, ((M + 63) / 64) * g.nnt)) {
-        g.ntt = (M + 63) / 64;
+    const int form = q6k_form((M + 63) / 64 * g.nnt, (M + 127) / 128 * g.nnt, g.nb);
+    g.ntt = form == Q6K_128 ? (M + 127) / 128 : (M + 63) / 64;
+    const unsigned grid = (unsigned)gemm_blocks(g.ntt, g.nnt);
+    if (sums) {
 #if CKQ_WITH_DUMP
-        if (sums) return gemm_launch_split(gemm_q6k_pair_kernel<2, true>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s);
+        if (form == Q6K_PAIRED) return gemm_launch_split(gemm_q6k_pair_kernel<2, true>, g, grid, g.nb, s);
+        if (form == Q6K_128) return gemm_launch_split(gemm_q6k_mfma_kernel<4, true>, g, grid, g.nb, s);
+        return gemm_launch_split(gemm_q6k_mfma_kernel<2, true>, g, grid, g.nb, s);
 #else
-        if (sums) return CKQ_ENODUMP;
+        return CKQ_ENODUMP;
 #endif
-        return gemm_launch_split(gemm_q6k_pair_kernel<2>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s);
     }
-    /* tiles of 128 tokens where they still give every CU work, else 64 */
-    const int ntt4 = (M + 127) / 128;
-    if (ntt4 * g.nnt > 128) {
-        g.ntt = ntt4;
-#if CKQ_WITH_DUMP
-        if (sums) return gemm_launch_split(gemm_q6k_mfma_kernel<4, true>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s);
-#else
-        if (sums) return CKQ_ENODUMP;
-#endif
-        return gemm_launch_split(gemm_q6k_mfma_kernel<4>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s);
-    }
-    g.ntt = (M + 63) / 64;
-#if CKQ_WITH_DUMP
-    if (sums) return gemm_launch_split(gemm_q6k_mfma_kernel<2, true>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s);
-#else
-    if (sums) return CKQ_ENODUMP;
-#endif
-    return gemm_launch_split(gemm_q6k_mfma_kernel<2>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s);
+    if (form == Q6K_PAIRED) return gemm_launch_split(gemm_q6k_pair_kernel<2>, g, grid, g.nb, s);
+    if (form == Q6K_128) return gemm_launch_split(gemm_q6k_mfma_kernel<4>, g, grid, g.nb, s);
+    return gemm_launch_split(gemm_q6k_mfma_kernel<2>, g, grid, g.nb, s);
 }
 
 bool gemm_q6k_group_chains(const GemmGroupIn &in, int M, int K, GemmChains *ch)
@@ -525,12 +522,11 @@ int launch_gemm_q6k_mfma_group(const void *A, const GemmGroupIn &in, int M, int 
     GemmArgs g = {};
     g.A = (const uint8_t *)A; g.M = M; g.nb = K / 256;
     if ((long long)g.nb * 292 * 128 >= (1ll << 31)) return (int)hipErrorInvalidValue;
-    /* tiles of 128 tokens where they fill the chip, else 64 */
-    if (gemm_group_tiles(in, M, 128) >= GEMM_GROUP_MIN_TILES) {
-        g.ntt = (M + 127) / 128;
-        return gemm_launch_grouped(gemm_q6k_mfma_kernel<4>, g, in, s);
-    }
-    if (gemm_group_tiles(in, M, 64) < GEMM_GROUP_MIN_TILES) return CKQ_ENOGROUP;
-    g.ntt = (M + 63) / 64;
+    const int tiles64 = gemm_group_tiles(in, M, 64);
+    if (tiles64 < GEMM_GROUP_MIN_TILES) return CKQ_ENOGROUP;
+    const int form = q6k_form(tiles64, gemm_group_tiles(in, M, 128), g.nb);
+    g.ntt = form == Q6K_128 ? (M + 127) / 128 : (M + 63) / 64;
+    if (form == Q6K_PAIRED) return gemm_launch_grouped(gemm_q6k_pair_kernel<2>, g, in, s);
+    if (form == Q6K_128) return gemm_launch_grouped(gemm_q6k_mfma_kernel<4>, g, in, s);
     return gemm_launch_grouped(gemm_q6k_mfma_kernel<2>, g, in, s);
 }

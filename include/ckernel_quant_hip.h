@@ -436,16 +436,16 @@ void ckq_set_gemm_policy(int policy);
  * the same sums in the same order: results are bit-identical wherever neither launch splits K or puts two wave groups
  * on a tile.
  *   CKQ_FMT_Q4_K: 64 or 96 = tiles of 128 rows x 64 tokens, or x 96 tokens - fewer instructions per token in blocks that run
- *                 longer, taken where they fit one round that 64-token tiles would not, or the grid is a round and a half deep
+ *                 longer, taken where an estimate of how the blocks fall on the CUs says so
  *                 (CKQ_Q4K_TILE=64|96 in the environment);
  *   CKQ_FMT_Q6_K: 1 = one block per CU (64-token tiles three LDS stages deep, 128-token tiles two), 2 = two blocks per CU
- *                 on 64-token tiles with one LDS image of the weights, taken where the 128-token grid would waste a
- *                 quarter or more of its last round (CKQ_Q6K_VARIANT=1|2);
+ *                 on 64-token tiles with one LDS image of the weights; the fastest of the three by an estimate
+ *                 from the numbers of tiles and K (CKQ_Q6K_VARIANT=1|2);
  *   CKQ_FMT_Q5_K: 1 = one block per CU, three LDS stages deep, 2 = two blocks per CU with one LDS image of the weights,
  *                 taken for more tiles than CUs (CKQ_Q5K_VARIANT=1|2).
  *   16 with any of the three: matmuls of two and more tokens run on 16-row tiles whatever their shape (taken by default from
  *                 three to a few dozen tokens, by shape; K up to 16384).  The bits are those of the kernel it stands in for.
- * Q8_0 has one variant. */
+ * Q8_0 chooses among its own (32-, 64- and 96-token tiles) by shape. */
 void ckq_set_prefill_variant(int fmt, int variant);
 /* Last error of the calling process (0 = none), its text, and a reset for
  * callers that run with CKQ_ABORT_ON_ERROR=0 and handle errors themselves. */

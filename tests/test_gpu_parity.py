@@ -1658,3 +1658,29 @@ def test_gemm_mfma_tiles_over_the_xcds(fmt, M):
         for w, a, b in zip(want, one, grp):
             bar = TOL * float(w.abs().max())
             assert float((a - w).abs().max()) <= bar and float((b - w).abs().max()) <= bar
+
+
+@pytest.mark.parametrize("M,Ns,K", [(64, (20000,), 512), (40, (16700,), 1024), (160, (10000,), 768), (190, (4096, 2048, 3000), 512), (345, (10391,), 512), (266, (9000, 9000), 768),
+                                    (247, (10593,), 2304), (129, (16300,), 256), (600, (3000,), 1280)])
+def test_gemm_q6_k_kernel_choice(M, Ns, K):
+    """Sizes on the sides of the choice between 64-token, 128-token and paired tiles, single matrices and groups, not split along K: one set of
+    bits, that of the paired kernel."""
+    import torch
+    L = ckq.lib()
+    say("q6_k kernel choice", M, Ns, K)
+    xq = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, 9970)), "q8_k", M)
+    Ws = [P.to_device(T.random_blocks("q6_k", n * (K // 256), 9971 + n)) for n in Ns]
+    got = {}
+    try:
+        L.ckq_set_gemm_policy(1)
+        for variant in (0, 1, 2):
+            L.ckq_set_prefill_variant(P.FMT["q6_k"], variant)
+            ys = [torch.full((M, n), 7.0, device="cuda") for n in Ns]
+            P.dev_matmul_sequence([("q6_k", xq, W, None, y, M, n, K) for W, y, n in zip(Ws, ys, Ns)])
+            got[variant] = ys
+    finally:
+        L.ckq_set_gemm_policy(0)
+        L.ckq_set_prefill_variant(P.FMT["q6_k"], 0)
+    for variant in (0, 1):
+        for a, b in zip(got[variant], got[2]):
+            assert torch.equal(a, b)
