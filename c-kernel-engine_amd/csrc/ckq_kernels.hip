@@ -42,6 +42,7 @@
  * Q8_0 4864x896 streams up to 32 tokens. */
 constexpr int CKQ_STREAM_TOKENS = 8;
 #include <atomic>
+#include <type_traits>
 static std::atomic<int> g_gemm_policy{0};      /* 0 automatic, 1 matrix cores above one pass, 2 always stream */
 
 extern "C" void ckq_launch_set_gemm_policy(int policy) { g_gemm_policy.store(policy < 0 || policy > 2 ? 0 : policy); }
@@ -105,16 +106,34 @@ static bool f32act_on_matrix_cores(int fmt, int ntok, int nrows, int K)
 #include "ckq_gemm_rows16.hpp"
 
 /* C = bias + partial 0 + partial 1 + ... in that order: the result does not
- * depend on which block finished first.  One thread per output. */
+ * depend on which block finished first.  A thread adds V (4 or 1) adjacent
+ * outputs.  The loads of eight, four or two partials go out together; one by
+ * one, each was a trip to memory of its own (whole launches, us: Q4_K 20 x 512 x 8192
+ * 13.5 -> 11.7, Q5_K 200 x 1024 x 8192 20.1 -> 17.9, Q4_K 225 x 3072 x 3072 17.8 -> 17.0). */
+template <int V>
 __global__ void __launch_bounds__(256) gemm_splitk_reduce_kernel(float *__restrict__ C, long ldc, const float *__restrict__ part,
                                                                  const float *__restrict__ bias, int M, int N, int splits)
 {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, mn = (size_t)M * (size_t)N;
+    typedef float vec __attribute__((ext_vector_type(V)));
+    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * V, mn = (size_t)M * (size_t)N;
     if (i >= mn) return;
     const int t = (int)(i / (size_t)N), n = (int)(i % (size_t)N);
-    float v = part[i];
-    for (int s = 1; s < splits; ++s) v += part[(size_t)s * mn + i];
-    C[(size_t)t * ldc + n] = bias ? v + bias[n] : v;
+    vec v = {}, b = {};
+    if (bias) b = *reinterpret_cast<const vec *>(bias + n);
+    auto add = [&](auto group, int s) {
+        constexpr int G = decltype(group)::value;
+        vec p[G];
+#pragma unroll
+        for (int k = 0; k < G; ++k) p[k] = *reinterpret_cast<const vec *>(part + (size_t)(s + k) * mn + i);
+#pragma unroll
+        for (int k = 0; k < G; ++k) v = s + k ? v + p[k] : p[k];
+    };
+    int s = 0;
+    for (; s + 8 <= splits; s += 8) add(std::integral_constant<int, 8>{}, s);
+    if (s + 4 <= splits) { add(std::integral_constant<int, 4>{}, s); s += 4; }
+    if (s + 2 <= splits) { add(std::integral_constant<int, 2>{}, s); s += 2; }
+    if (s < splits) add(std::integral_constant<int, 1>{}, s);
+    *reinterpret_cast<vec *>(C + (size_t)t * ldc + n) = bias ? v + b : v;
 }
 
 
@@ -215,8 +234,10 @@ extern "C" int ckq_launch_release_stream(void *stream)
 int gemm_launch_reduce(float *C, long ldc, const float *part, const float *bias, int M, int N, int splits, hipStream_t s)
 {
     const size_t mn = (size_t)M * (size_t)N;
-    hipLaunchKernelGGL(gemm_splitk_reduce_kernel, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, s,
-                       C, ldc, part, bias, M, N, splits);
+    if (N % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)C | (uintptr_t)part | (uintptr_t)bias) % 16 == 0)
+        hipLaunchKernelGGL(gemm_splitk_reduce_kernel<4>, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, s, C, ldc, part, bias, M, N, splits);
+    else
+        hipLaunchKernelGGL(gemm_splitk_reduce_kernel<1>, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, s, C, ldc, part, bias, M, N, splits);
     return (int)hipGetLastError();
 }
 

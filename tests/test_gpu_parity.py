@@ -1684,3 +1684,32 @@ def test_gemm_q6_k_kernel_choice(M, Ns, K):
     for variant in (0, 1):
         for a, b in zip(got[variant], got[2]):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("N,K", [(128, 2048), (128, 3072), (300, 5120), (64, 7168), (132, 8192), (260, 16384), (200, 9216)])
+def test_gemm_split_k_partials_added(N, K):
+    """K splits of two to sixteen, added four outputs a thread where rows of C start on 16 bytes and one elsewhere, with a bias that is and is not
+    so aligned and without: one set of bits, the same as on a second call."""
+    import torch
+    L = ckq.lib()
+    M = 70
+    xq = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, 9980)), "q8_k", M)
+    W = P.to_device(T.random_blocks("q4_k", N * (K // 256), 9981))
+    b = P.to_device(T.normal(N + 1, 0.0, 0.5, 9982))
+    say("split partials", N, K)
+
+    def run(ldc, bias):
+        c = torch.full((M, ldc), 7.0, device="cuda")
+        P.check(L.ckq_gemm_nt_dev(P.FMT["q4_k"], P._dp(xq), P._dp(W), bias, P._dp(c), M, N, K, ldc, P._stream()), "ckq_gemm_nt_dev")
+        assert bool((c[:, N:] == 7.0).all())
+        return c[:, :N].clone()
+    try:
+        L.ckq_set_gemm_policy(1)
+        plain = run(N, None)
+        assert torch.equal(plain, run(N + 1, None)) and torch.equal(plain, run(N, None))
+        for ofs in (0, 1):
+            p = ctypes.c_void_p(b.data_ptr() + 4 * ofs)
+            want = plain + b[ofs:ofs + N]
+            assert torch.equal(run(N, p), want) and torch.equal(run(N + 3, p), want)
+    finally:
+        L.ckq_set_gemm_policy(0)
