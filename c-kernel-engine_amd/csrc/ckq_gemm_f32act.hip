@@ -31,7 +31,7 @@
  * the lane's share of the group's sum of x against the row's factor, both cut in three.
  *
  * Block = 8 waves on one tile of 32 tokens x 32 R weight rows; the waves cut K into eight contiguous runs and add
- * their partial tiles through LDS, in pairs.  Each wave loads its own activations one step (Q4_K) or half a step ahead, a
+ * their partial tiles through LDS, in pairs.  Each wave loads its own activations half a step or a step ahead, a
  * contiguous run per token, and turns them through LDS (a lane loading its own row would touch 64 cache lines per instruction: 40 us
  * instead of 36 at 96 x 4096 x 4096, Q6_K; one token per pass over the weights, as the streaming kernel does it, 245 us);
  * no other wave reads them, so the loop has no barrier.  Cutting the activations in a launch of its own and reading the
@@ -40,8 +40,11 @@
  * Weights.  The address path takes a wave's load in 16 to 22 cycles where quads of lanes read adjacent bytes, in 64 where every lane
  * has a row of its own, and in 160 where the rows' bytes are not on dwords either (measured, 16 bytes a lane, L2).  Q6_K
  * and Q8_0, whose blocks are only 2-byte aligned, therefore come in memory order like the activations (gemm_f32run_kernel, 96 x 4096 x
- * 4096: Q6_K 36.1 -> 31.7 us, Q8_0 36.3 -> 28.2, same bits; 40 shapes of 1..158 tokens 1.03 on average).  Q4_K, 16-byte
- * aligned and two loads a step, loses that way (27.5 -> 29.3) and keeps its own loads (gemm_f32act_q4k_kernel).
+ * 4096: Q6_K 36.1 -> 31.1 us, Q8_0 36.3 -> 27.6; 200 x 5000 x 8192 Q6_K 207 -> 162, Q8_0 187 -> 145; same bits).  Where a wave's share is
+ * shorter than a run (SHORT) that would load the same weights up to four times and wait for them in turn: the block loads them once, all
+ * loads under way together, and the smaller tile leaves room for a second block on the CU (Q6_K 75 x 7670 x 512 12.1 -> 10.5 us,
+ * 200 x 5000 x 1536 42.1 -> 31.9; a run per wave 14.2 and 42.1).  A row per lane stays (gemm_f32row_kernel) for Q4_K, 16-byte aligned and two
+ * loads a step, which loses in memory order (27.5 -> 29.3), and for the sizes named at the launcher.
  *
  * Grid: token groups fastest, so the blocks that share weights run side by side.
  * Bound: VALU issue: per 64 elements 220-260 operations to cut x, shared by the R row tiles, and per row tile some 210 / 230 / 130 for
@@ -125,18 +128,19 @@ __device__ __forceinline__ ckq_v4i bytes_to_bf16(u32 b0, u32 b1)
  *   scale(g)        fp32 factor of the group; MIN: rest(g), the factor of the group's sum of x
  *   weight(blk, e, i)  element e + i of a block, e a multiple of 16 and i below 16, for exact_output */
 struct F32Q4K {
-    static constexpr int STEP = 64, NK = 2;
+    static constexpr int STEP = 64, NG = 2, NK = 2;
+    static constexpr bool MIN = true;
     struct Raw { u32 hdr[4], qs[4]; };
-    static __device__ __forceinline__ void load(Raw &w, const uint8_t *row, int step, int h)
+    static __device__ __forceinline__ void load_row(Raw &w, const uint8_t *row, int step, int h, int)
     {
         const uint8_t *blk = row + (u32)(step >> 2) * 144u;
         ld16<4>(w.hdr, blk);
         ld16<4>(w.qs, blk + 16 + 32 * (step & 3) + 16 * h);
     }
-    static __device__ __forceinline__ u32 src_elem(int step, int c) { return 64u * (u32)step + 4u * c; }
+    static __device__ __forceinline__ u32 src_elem(int step, int c, int) { return 64u * (u32)step + 4u * c; }
     static __device__ __forceinline__ int chunk(int g, int h, int i) { return 8 * g + 4 * h + i; }
     struct Dec { float s[2], rest[2]; u32 off[2]; };          /* off: 128 - c in every byte */
-    static __device__ __forceinline__ void decode(Dec &d, const Raw &w, int step)
+    static __device__ __forceinline__ void decode(Dec &d, const Raw &w, int step, int)
     {
         u32 sc2, mn2;
         k4_scale_pair(w.hdr[1], w.hdr[2], w.hdr[3], step & 3, &sc2, &mn2);
@@ -176,9 +180,24 @@ struct F32Q4K {
 
 struct F32Q6K {
     static constexpr int STEP = 64, NG = 4, NK = 1;       /* a step: 16-runs o of the four 32-runs of one 128-half n */
-    static constexpr int RUN = 4, BYTES = 210, LANES = 16, PITCH = 240;
-    static constexpr bool SHIFT = true;
+    static constexpr int RUN = 4, BYTES = 210, LANES = 16, PITCH = 240, SHORT_RUNS = 6;
+    static constexpr bool SHIFT = true, MIN = false;
     struct Raw { u32 ql0[2], ql1[2], qh[2], sc[2], d; };
+    static __device__ __forceinline__ void load_row(Raw &w, const uint8_t *row, int step, int h, int)
+    {
+        const uint8_t *blk = row + (u32)(step >> 2) * 210u;
+        const int n = (step >> 1) & 1, o = step & 1;
+        ld8<2>(w.ql0, blk + 64 * n + 16 * o + 8 * h);
+        ld8<2>(w.ql1, blk + 64 * n + 32 + 16 * o + 8 * h);
+        ld8<2>(w.qh, blk + 128 + 32 * n + 16 * o + 8 * h);
+        ld8<2>(w.sc, blk + 192 + 8 * n);
+        w.d = ld2(blk + 208);
+    }
+    static __device__ __forceinline__ u32 src_elem(int step, int c, int)
+    {
+        return 128u * (u32)(step >> 1) + 16u * (step & 1) + 32u * (c >> 2) + 4u * (c & 3);
+    }
+    static __device__ __forceinline__ int chunk(int g, int h, int i) { return 4 * g + 2 * h + i; }
     static __device__ __forceinline__ void load(Raw &w, const uint8_t *row, int step, int h)
     {
         const int n = (step >> 1) & 1, o = step & 1;
@@ -229,9 +248,23 @@ struct F32Q6K {
 
 struct F32Q80 {
     static constexpr int STEP = 64, NG = 2, NK = 2;       /* two 32-blocks; the second is missing in the last step of an odd count */
-    static constexpr int RUN = 2, BYTES = 136, LANES = 9, PITCH = 144;
-    static constexpr bool SHIFT = false;
+    static constexpr int RUN = 2, BYTES = 136, LANES = 9, PITCH = 144, SHORT_RUNS = 10;
+    static constexpr bool SHIFT = false, MIN = false;
     struct Raw { u32 q[2][4]; u32 d[2]; };
+    static __device__ __forceinline__ void load_row(Raw &w, const uint8_t *row, int step, int h, int K)
+    {
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            const uint8_t *blk = row + (u32)min(2 * step + g, K / 32 - 1) * 34u;
+            w.d[g] = ld2(blk);
+            ld16<2>(w.q[g], blk + 2 + 16 * h);
+        }
+    }
+    static __device__ __forceinline__ u32 src_elem(int step, int c, int K)
+    {
+        return 32u * (u32)min(2 * step + (c >> 3), K / 32 - 1) + 4u * (c & 7);
+    }
+    static __device__ __forceinline__ int chunk(int g, int h, int i) { return 8 * g + 4 * h + i; }
     static __device__ __forceinline__ void load(Raw &w, const uint8_t *row, int step, int h)
     {
         /* quants of block j start at byte 34 j + 2: two aligned reads around them */
@@ -279,13 +312,11 @@ __device__ __forceinline__ float exact_output(const uint8_t *w, const float *x, 
     return sum;
 }
 
-/* Q4_K */
-template <int R>
+template <class F, int R>
 __global__ void __launch_bounds__(64 * F32_WAVES, 2)
-gemm_f32act_q4k_kernel(const float *__restrict__ A, const uint8_t *__restrict__ B, const float *__restrict__ bias, float *__restrict__ C,
+gemm_f32row_kernel(const float *__restrict__ A, const uint8_t *__restrict__ B, const float *__restrict__ bias, float *__restrict__ C,
                    int M, int N, int K, long wrow, long ldc, int ntg)
 {
-    typedef F32Q4K F;
     /* a wave's activations of one step, token t at 256 t, chunk c in slot c ^ (t & 15); at the end the partial tiles */
     __shared__ __attribute__((aligned(16))) uint8_t xs_all[F32_WAVES][32 * 256];
     const int lane = threadIdx.x & 63, wave = wave_in_block();
@@ -312,9 +343,9 @@ gemm_f32act_q4k_kernel(const float *__restrict__ A, const uint8_t *__restrict__ 
     ckq_v4i xn[8];
     auto fetch = [&](int s) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) xn[j] = *reinterpret_cast<const ckq_v4i *>(xsrc[j] + F::src_elem(s, lane & 15));
+        for (int j = 0; j < 8; ++j) xn[j] = *reinterpret_cast<const ckq_v4i *>(xsrc[j] + F::src_elem(s, lane & 15, K));
 #pragma unroll
-        for (int r = 0; r < R; ++r) F::load(wn[r], wr[r], s, half);
+        for (int r = 0; r < R; ++r) F::load_row(wn[r], wr[r], s, half, K);
     };
     auto take = [&]() {
 #pragma unroll
@@ -328,9 +359,10 @@ gemm_f32act_q4k_kernel(const float *__restrict__ A, const uint8_t *__restrict__ 
     auto compute = [&](int s) {
         typename F::Dec dec[R];
 #pragma unroll
-        for (int r = 0; r < R; ++r) F::decode(dec[r], w[r], s);
-        /* the step's two groups: their two terms are added before they meet the sum so far */
-        {
+        for (int r = 0; r < R; ++r) F::decode(dec[r], w[r], s, K);
+        /* two groups at a time: their two terms are added before they meet the sum so far */
+#pragma unroll
+        for (int g0 = 0; g0 < F::NG; g0 += 2) {
             Cut c[2][F::NK];
             ckq_v4i pa[2];
 #pragma unroll
@@ -338,7 +370,7 @@ gemm_f32act_q4k_kernel(const float *__restrict__ A, const uint8_t *__restrict__ 
                 float x[F::NK * 8];
 #pragma unroll
                 for (int i = 0; i < 2 * F::NK; ++i) {
-                    const ckq_v4i v = *reinterpret_cast<const ckq_v4i *>(xs + 256 * col + 16 * (F::chunk(g, half, i) ^ (col & 15)));
+                    const ckq_v4i v = *reinterpret_cast<const ckq_v4i *>(xs + 256 * col + 16 * (F::chunk(g0 + g, half, i) ^ (col & 15)));
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
                         const int e = v[j];
@@ -347,7 +379,7 @@ gemm_f32act_q4k_kernel(const float *__restrict__ A, const uint8_t *__restrict__ 
                 }
 #pragma unroll
                 for (int k = 0; k < F::NK; ++k) cut8(x + 8 * k, c[g][k]);
-                {
+                if constexpr (F::MIN) {
                     /* this half's share of the group's sum of x, cut in three; against the cut rest of the min, the six
                      * products that matter in one MFMA, which also adds the halves */
                     const float p = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7])) +
@@ -358,25 +390,28 @@ gemm_f32act_q4k_kernel(const float *__restrict__ A, const uint8_t *__restrict__ 
             }
 #pragma unroll
             for (int r = 0; r < R; ++r) {
-                ckq_v16f two = zero, sum;
+                ckq_v16f two, sum;
+                if constexpr (F::MIN) {
+                    two = zero;
 #pragma unroll
-                for (int g = 0; g < 2; ++g) {
-                    const float h = dec[r].rest[g], m = h - top16(h), l = m - top16(m);
-                    two = mfma_bf16(pa[g], ckq_v4i{(int)pack_bf16(h, m), (int)pack_bf16(h, m), (int)pack_bf16(l, h), 0}, two);
+                    for (int g = 0; g < 2; ++g) {
+                        const float h = dec[r].rest[g0 + g], m = h - top16(h), l = m - top16(m);
+                        two = mfma_bf16(pa[g], ckq_v4i{(int)pack_bf16(h, m), (int)pack_bf16(h, m), (int)pack_bf16(l, h), 0}, two);
+                    }
                 }
 #pragma unroll
                 for (int g = 0; g < 2; ++g) {
                     sum = zero;
 #pragma unroll
                     for (int k = 0; k < F::NK; ++k) {
-                        const ckq_v4i b = F::operand(w[r], dec[r], g, k);
+                        const ckq_v4i b = F::operand(w[r], dec[r], g0 + g, k);
                         sum = mfma_bf16(c[g][k].lo, b, sum);
                         sum = mfma_bf16(c[g][k].mid, b, sum);
                         sum = mfma_bf16(c[g][k].hi, b, sum);
                     }
 #pragma unroll
                     for (int i = 0; i < 16; ++i)
-                        two[i] = fmaf(dec[r].s[g], sum[i], g ? two[i] : -two[i]);
+                        two[i] = F::MIN || g ? fmaf(dec[r].s[g0 + g], sum[i], F::MIN && !g ? -two[i] : two[i]) : dec[r].s[g0 + g] * sum[i];
                 }
 #pragma unroll
                 for (int i = 0; i < 16; ++i) acc[r][i] += two[i];
@@ -432,22 +467,26 @@ gemm_f32act_q4k_kernel(const float *__restrict__ A, const uint8_t *__restrict__ 
     }
 }
 
-template <class F, int R>
-__global__ void __launch_bounds__(64 * F32_WAVES, 2)
+template <class F, int R, bool SHORT> constexpr bool f32_two_blocks = R == 1 && SHORT;
+
+template <class F, int R, bool SHORT>
+__global__ void __launch_bounds__(64 * F32_WAVES, (f32_two_blocks<F, R, SHORT> ? 4 : 2))
 gemm_f32run_kernel(const float *__restrict__ A, const uint8_t *__restrict__ B, const float *__restrict__ bias, float *__restrict__ C,
                    int M, int N, int K, long wrow, long ldc, int ntg)
 {
     constexpr int ROWS = 32 * R, RPI = 64 / F::LANES, NWL = (ROWS + RPI - 1) / RPI;      /* rows per load instruction, instructions per run */
     constexpr int WLDS = ROWS * F::PITCH, XLDS = 32 * 128, RED = F32_WAVES * (R < 2 ? 1 : 2) * 16 * 64 * 4;
-    /* of each wave: the weights of a run, and the activations of a phase, token t at 128 t, chunk c in slot c ^ (t / 2 % 8); at
-     * the end the partial tiles */
-    __shared__ __attribute__((aligned(16))) uint8_t smem[F32_WAVES * (WLDS + XLDS) > RED ? F32_WAVES * (WLDS + XLDS) : RED];
+    constexpr int RUNS = SHORT ? F::SHORT_RUNS : F32_WAVES, USED = RUNS * WLDS + F32_WAVES * XLDS;
+    constexpr int AHEAD = SHORT || R == 1 || std::is_same<F, F32Q80>::value ? 2 : 1;      /* phases of activations on their way, as registers allow */
+    /* weights of a run each wave, or (SHORT) of all runs; of each wave the activations of a phase, token t at 128 t, chunk c in slot
+     * c ^ (t / 2 % 8); at the end the partial tiles */
+    __shared__ __attribute__((aligned(16))) uint8_t smem[USED > RED ? USED : RED];
     const int lane = threadIdx.x & 63, wave = wave_in_block();
     const int col = lane & 31, half = lane >> 5;
     const int t0 = (int)(blockIdx.x % (u32)ntg) * 32, n0 = (int)(blockIdx.x / (u32)ntg) * ROWS;
     const int steps = (K + F::STEP - 1) / F::STEP, per = (steps + F32_WAVES - 1) / F32_WAVES;
     const int s0 = wave * per, s1 = min(steps, s0 + per);
-    uint8_t *const wl = smem + wave * (WLDS + XLDS), *const xs = wl + WLDS;
+    uint8_t *const wl = smem + wave * WLDS, *const xs = smem + RUNS * WLDS + wave * XLDS;
 
     /* weights: row and chunk of this lane in load instruction j */
     const int w_row = lane / F::LANES, w_chunk = lane % F::LANES;
@@ -461,63 +500,67 @@ gemm_f32run_kernel(const float *__restrict__ A, const uint8_t *__restrict__ B, c
         asm volatile("" : "+v"(r));                          /* formed when it is needed, not kept for every j */
         return (size_t)min(r, left) * row_bytes + (u32)run * (u32)F::BYTES;
     };
+    auto load_w = [&](int j, int run) {
+        u32 t[4];
+        if constexpr (F::SHIFT) {
+            /* from the dword the block starts in; the last chunk from byte 196 of it, so that no load passes the dword the block ends in */
+            ld16<4>(t, wbase - par + (((w_src(j, run) + par) & ~(size_t)3) + (u32)(w_chunk < 13 ? 16 * w_chunk : 196)));
+        } else ld16<2>(t, wbase + (w_src(j, run) + min(16u * (u32)w_chunk, run_bytes(run) - 16u)));
+        return ckq_v4i{(int)t[0], (int)t[1], (int)t[2], (int)t[3]};
+    };
+    auto put_w = [&](uint8_t *dst, int j, int run, ckq_v4i b) {
+        const int row = RPI * j + w_row;
+        uint8_t *const d = dst + row * F::PITCH;
+        const bool on = w_row < RPI && row < ROWS;
+        if constexpr (F::SHIFT) {
+            const u32 sh = ((u32)w_src(j, run) + par) & 2u;
+            u32 v[5];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = (u32)b[i];
+            /* the neighbour's first dword; lane 13 holds dwords 49 .. 52 of the block's 53 */
+            v[4] = (u32)dpp_get<0x101>((int)(w_chunk == 13 ? v[3] : v[0]));
+            ckq_v4i o;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[i] = (int)__builtin_amdgcn_alignbyte(v[i + 1], v[i], sh);
+            if (on && w_chunk < 13) *reinterpret_cast<ckq_v4i *>(d + 16 * w_chunk) = o;
+            if (on && w_chunk == 13) *reinterpret_cast<u32 *>(d + 208) = v[3] >> (8 * sh);
+        } else if (run_bytes(run) == (u32)F::BYTES) {
+            if (on && 16 * w_chunk + 16 <= F::BYTES) *reinterpret_cast<ckq_v4i *>(d + 16 * w_chunk) = b;
+            else if (on) *reinterpret_cast<int2 *>(d + 16 * w_chunk) = int2{b[2], b[3]};         /* the last 16 of 136 bytes */
+        } else if (on) {
+            uint16_t *const e = reinterpret_cast<uint16_t *>(d + min(16u * (u32)w_chunk, run_bytes(run) - 16u));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                e[2 * i] = (uint16_t)((u32)b[i] & 0xffffu);
+                e[2 * i + 1] = (uint16_t)((u32)b[i] >> 16);
+            }
+        }
+    };
     auto fetch_w = [&](int run) {
 #pragma unroll
-        for (int j = 0; j < NWL; ++j) {
-            u32 t[4];
-            if constexpr (F::SHIFT) {
-                /* from the dword the block starts in; the last chunk from byte 196 of it, so that no load passes the dword the block ends in */
-                ld16<4>(t, wbase - par + (((w_src(j, run) + par) & ~(size_t)3) + (u32)(w_chunk < 13 ? 16 * w_chunk : 196)));
-            } else ld16<2>(t, wbase + (w_src(j, run) + min(16u * (u32)w_chunk, run_bytes(run) - 16u)));
-            wn[j] = ckq_v4i{(int)t[0], (int)t[1], (int)t[2], (int)t[3]};
-        }
+        for (int j = 0; j < NWL; ++j) wn[j] = load_w(j, run);
     };
     auto take_w = [&](int run) {
 #pragma unroll
-        for (int j = 0; j < NWL; ++j) {
-            const int row = RPI * j + w_row;
-            uint8_t *const d = wl + row * F::PITCH;
-            const bool on = w_row < RPI && row < ROWS;
-            if constexpr (F::SHIFT) {
-                const u32 sh = ((u32)w_src(j, run) + par) & 2u;
-                u32 v[5];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) v[i] = (u32)wn[j][i];
-                /* the neighbour's first dword; lane 13 holds dwords 49 .. 52 of the block's 53 */
-                v[4] = (u32)dpp_get<0x101>((int)(w_chunk == 13 ? v[3] : v[0]));
-                ckq_v4i o;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) o[i] = (int)__builtin_amdgcn_alignbyte(v[i + 1], v[i], sh);
-                if (on && w_chunk < 13) *reinterpret_cast<ckq_v4i *>(d + 16 * w_chunk) = o;
-                if (on && w_chunk == 13) *reinterpret_cast<u32 *>(d + 208) = v[3] >> (8 * sh);
-            } else if (run_bytes(run) == (u32)F::BYTES) {
-                if (on && 16 * w_chunk + 16 <= F::BYTES) *reinterpret_cast<ckq_v4i *>(d + 16 * w_chunk) = wn[j];
-                else if (on) *reinterpret_cast<int2 *>(d + 16 * w_chunk) = int2{wn[j][2], wn[j][3]};         /* the last 16 of 136 bytes */
-            } else if (on) {
-                uint16_t *const e = reinterpret_cast<uint16_t *>(d + min(16u * (u32)w_chunk, run_bytes(run) - 16u));
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    e[2 * i] = (uint16_t)((u32)wn[j][i] & 0xffffu);
-                    e[2 * i + 1] = (uint16_t)((u32)wn[j][i] >> 16);
-                }
-            }
-        }
+        for (int j = 0; j < NWL; ++j) put_w(wl, j, run, wn[j]);
         __builtin_amdgcn_wave_barrier();                     /* the wave's own LDS accesses stay in this order */
     };
 
-    const float *xsrc[4];          /* row of the token this lane fetches in load instruction j */
+    /* row of the token this lane fetches in load instruction j */
+    const float *const xbase = A + (size_t)t0 * (size_t)K;
+    typename std::conditional<SHORT, u32, size_t>::type xsrc[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) xsrc[j] = A + (size_t)min(t0 + 8 * j + (lane >> 3), M - 1) * (size_t)K;
-    ckq_v4i xn[4];
+    for (int j = 0; j < 4; ++j) xsrc[j] = (size_t)min(8 * j + (lane >> 3), M - 1 - t0) * (size_t)K;
+    ckq_v4i xn[AHEAD][4];
     auto fetch_x = [&](int s, int p) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) xn[j] = *reinterpret_cast<const ckq_v4i *>(xsrc[j] + F::src_elem(s, p, lane & 7, K));
+        for (int j = 0; j < 4; ++j) xn[p % AHEAD][j] = *reinterpret_cast<const ckq_v4i *>(xbase + (xsrc[j] + F::src_elem(s, p, lane & 7, K)));
     };
-    auto take_x = [&]() {
+    auto take_x = [&](int p) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int t = 8 * j + (lane >> 3);
-            *reinterpret_cast<ckq_v4i *>(xs + 128 * t + 16 * ((lane & 7) ^ (t >> 1 & 7))) = xn[j];
+            *reinterpret_cast<ckq_v4i *>(xs + 128 * t + 16 * ((lane & 7) ^ (t >> 1 & 7))) = xn[p % AHEAD][j];
         }
         __builtin_amdgcn_wave_barrier();
     };
@@ -529,28 +572,47 @@ gemm_f32run_kernel(const float *__restrict__ A, const uint8_t *__restrict__ B, c
     for (int r = 0; r < R; ++r) acc[r] = two[r] = zero;
 
     if (s0 < s1) {
-        fetch_w(s0 / F::RUN);
+        if constexpr (!SHORT) fetch_w(s0 / F::RUN);
         fetch_x(s0, 0);
+        if constexpr (AHEAD == 2) fetch_x(s0, 1);
+    }
+    if constexpr (SHORT) {
+        constexpr int SHARE = (RUNS * NWL + F32_WAVES - 1) / F32_WAVES;        /* load instructions of a wave, all under way together */
+        const int n = (steps + F::RUN - 1) / F::RUN * NWL;
+        ckq_v4i v[SHARE];
+#pragma unroll
+        for (int q = 0; q < SHARE; ++q) {
+            const int i = wave + F32_WAVES * q;
+            if (i < n) v[q] = load_w(i % NWL, i / NWL);
+        }
+#pragma unroll
+        for (int q = 0; q < SHARE; ++q) {
+            const int i = wave + F32_WAVES * q, run = i / NWL;
+            if (i < n) put_w(smem + run * WLDS, i % NWL, run, v[q]);
+        }
+        __syncthreads();
     }
     for (int s = s0; s < s1; ++s) {
-        if (s == s0 || s % F::RUN == 0) {
-            take_w(s / F::RUN);
-            if ((s / F::RUN + 1) * F::RUN < s1) fetch_w(s / F::RUN + 1);
-        }
+        if constexpr (!SHORT)
+            if (s == s0 || s % F::RUN == 0) {
+                take_w(s / F::RUN);
+                if ((s / F::RUN + 1) * F::RUN < s1) fetch_w(s / F::RUN + 1);
+            }
         typename F::Raw w[R];
         typename F::Dec dec[R];
+        const uint8_t *const ws = SHORT ? smem + s / F::RUN * WLDS : wl;
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            F::load(w[r], wl + (32 * r + col) * F::PITCH, s, half);
+            F::load(w[r], ws + (32 * r + col) * F::PITCH, s, half);
             F::decode(dec[r], w[r], s, K);
         }
         /* two phases of 32 elements a token: a scale group each, or two groups of 16 */
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
             constexpr int NG = F::NG / 2;                    /* groups of a phase */
-            take_x();
-            if (p == 0) fetch_x(s, 1);
-            else if (s + 1 < s1) fetch_x(s + 1, 0);
+            take_x(p);
+            if (AHEAD == 1 && p == 0) fetch_x(s, 1);
+            else if (s + 1 < s1) fetch_x(s + 1, AHEAD == 1 ? 0 : p);
             __builtin_amdgcn_sched_barrier(0);
             Cut c[NG][F::NK];
 #pragma unroll
@@ -649,13 +711,40 @@ int launch_f32act(const float *A, const uint8_t *B, const float *bias, float *C,
 {
     const long long ntg = (M + 31) / 32;
     /* two row tiles per wave share the cut of x; one where that would leave CUs without a block */
-    const int R = ntg * ((N + 63) / 64) >= 192 ? 2 : 1;
+    int R = ntg * ((N + 63) / 64) >= 192 ? 2 : 1;
+    auto kernel = gemm_f32row_kernel<F, 1>;
+    if constexpr (std::is_same<F, F32Q4K>::value) {
+        if (R == 2) kernel = gemm_f32row_kernel<F, 2>;
+    } else {
+        /* Same bits from all of them.  Measured over 7 grids of 63..1099 tiles of 32 rows, Q6_K at 16 and Q8_0 at 24 widths of 256..8192:
+         *  - up to SHORT_RUNS runs: weights loaded once a block, two blocks on a CU; Q6_K 1.02..1.31 times the row kernel (75 x 7670 x 1024
+         *    20.9 -> 16.0 us), Q8_0 1.03..1.18 where there is more than a block per CU.  A block alone on its CU gains nothing from the
+         *    second place and pays the way through LDS and the barrier: Q8_0 0.82..0.93, Q6_K 0.92..0.96 where a wave has but one step (512).
+         *  - longer: a wave whose share does not begin and end with a run loads runs that its neighbours load too, which the row kernel
+         *    does not: Q6_K 0.97..1.00 at one row tile and a second round of blocks, 1.02..1.26 otherwise; Q8_0 (runs of 128) 0.89..0.98 up to five steps a
+         *    wave (two bytes off a dword up to eight, at one row tile up to nine: 0.94..0.99), 1.01..1.29 beyond and at four.
+         *  - Q8_0 rows that are a multiple of 64 bytes apart: the row kernel's 64 rows fall on few cache sets; 1.00..1.29. */
+        const int per = ((K + F::STEP - 1) / F::STEP + F32_WAVES - 1) / F32_WAVES;
+        const bool filled = ntg * ((N + 31) / 32) > 256, fits = K <= F::SHORT_RUNS * F::RUN * F::STEP;
+        bool once, runs;
+        if constexpr (std::is_same<F, F32Q6K>::value) {
+            once = fits && (filled || per > 1);
+            runs = !fits && !(R == 1 && filled && per % F::RUN);
+        } else {
+            once = fits && filled;
+            runs = K % 1024 == 0 || per >= 10 || (R == 2 && (per == 4 || per >= (K % 64 ? 9 : 6)));
+        }
+        if (once) {
+            R = 1;
+            kernel = gemm_f32run_kernel<F, 1, true>;
+        } else if (runs)
+            kernel = R == 2 ? gemm_f32run_kernel<F, 2, false> : gemm_f32run_kernel<F, 1, false>;
+        else if constexpr (std::is_same<F, F32Q80>::value) {
+            if (R == 2) kernel = gemm_f32row_kernel<F, 2>;
+        }                                    /* Q6_K: R is 1 here */
+    }
     const long long grid = ntg * ((N + 32 * R - 1) / (32 * R));
     if (grid > 0x7fffffffll) return CKQ_ESHAPE;
-    const auto kernel = [&] {
-        if constexpr (std::is_same<F, F32Q4K>::value) return R == 2 ? gemm_f32act_q4k_kernel<2> : gemm_f32act_q4k_kernel<1>;
-        else return R == 2 ? gemm_f32run_kernel<F, 2> : gemm_f32run_kernel<F, 1>;
-    }();
     hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(64 * F32_WAVES), 0, s, A, B, bias, C, M, N, K, wrow, ldc, (int)ntg);
     return (int)hipGetLastError();
 }

@@ -86,7 +86,7 @@ static bool gemm_on_matrix_cores(int ntok, size_t weight_bytes, size_t budget_mb
  * of 512..8192 and 1..200 tokens (us): streaming 4 + 0.125 / 0.18 / 0.16 (Q4_K / Q6_K / Q8_0) per million products; matrix cores
  * 6 + 0.020 / 0.024 / 0.024 per million products of the tokens rounded up to 32, but never less than 5 + 1.35 (Q4_K 1.5) for every
  * 64 elements a wave walks through (an eighth of K).  4096 x 4096 Q6_K: 4 tokens 14.5 against 19 (streams), 8 tokens 26 against
- * 19, 96 tokens 270 against 36; 141 x 8192 streams up to 96 tokens. */
+ * 19, 96 tokens 270 against 31; 141 x 8192 streams up to 96 tokens. */
 static bool f32act_on_matrix_cores(int fmt, int ntok, int nrows, int K)
 {
     const int policy = g_gemm_policy.load(std::memory_order_relaxed);

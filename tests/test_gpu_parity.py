@@ -1359,6 +1359,32 @@ def test_f32act_weights_by_runs(fmt, blocks, ofs):
         L.ckq_set_gemm_policy(0)
 
 
+@pytest.mark.parametrize("fmt,widths", [("q6_k", (256, 512, 768, 1536, 1792, 2304)),
+                                        ("q8_0", (32, 416, 512, 544, 1024, 1280, 1312, 1536, 1568, 2080, 2592))])
+def test_f32act_short_rows(fmt, widths):
+    """Rows that a block loads once for all its waves, and both sides of the choices around them: widths that end with and within a
+    run, waves with none, one and several steps; grids of a block, of a block per CU and of more, at one and two row tiles.  Against
+    float64; an output is a sum of at most 41 fp32 additions over 8 waves, each rounded by 2^-24 of a partial sum, which random signs
+    keep far below S, the sum of the magnitudes: 3e-7 S is five such roundings of S itself."""
+    import torch
+    L = ckq.lib()
+    B = T.ELEMS[fmt]
+    L.ckq_set_gemm_policy(1)
+    try:
+        for K in widths:
+            for M, N in ((1, 1), (3, 35), (64, 4096), (33, 4129), (96, 4097)):
+                W = T.random_blocks(fmt, N * K // B, 60 + K // B)
+                x = T.normal(M * K, 0.5, 1.0, seed=K)
+                W_d, x_d = P.to_device(W), P.to_device(x)
+                c = torch.full((M, N), 7.0, dtype=torch.float32, device="cuda")
+                say("f32act short", fmt, K, M, N)
+                P.check(L.ckq_gemm_nt_f32act_dev(P.FMT[fmt], P._dp(x_d), P._dp(W_d), None, P._dp(c), M, N, K, N, P._stream()), "f32act")
+                X, V = x_d.view(M, K).double(), torch.from_numpy(T.np_dequant(fmt, W).reshape(N, K)).cuda().double()
+                assert bool(((c - X @ V.T).abs() <= 3e-7 * (X.abs() @ V.abs().T)).all()), (K, M, N)
+    finally:
+        L.ckq_set_gemm_policy(0)
+
+
 # ---- 16-row tiles: a few to a few dozen tokens of the K-quants -------------------------------------
 
 @pytest.mark.parametrize("fmt", ["q4_k", "q5_k", "q6_k"])
