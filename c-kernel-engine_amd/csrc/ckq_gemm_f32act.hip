@@ -712,23 +712,22 @@ int launch_f32act(const float *A, const uint8_t *B, const float *bias, float *C,
     const long long ntg = (M + 31) / 32;
     /* two row tiles per wave share the cut of x; one where that would leave CUs without a block */
     int R = ntg * ((N + 63) / 64) >= 192 ? 2 : 1;
-    auto kernel = gemm_f32row_kernel<F, 1>;
-    if constexpr (std::is_same<F, F32Q4K>::value) {
-        if (R == 2) kernel = gemm_f32row_kernel<F, 2>;
-    } else {
+    auto kernel = R == 2 ? gemm_f32row_kernel<F, 2> : gemm_f32row_kernel<F, 1>;
+    if constexpr (!std::is_same<F, F32Q4K>::value) {
         /* Same bits from all of them.  Measured over 7 grids of 63..1099 tiles of 32 rows, Q6_K at 16 and Q8_0 at 24 widths of 256..8192:
          *  - up to SHORT_RUNS runs: weights loaded once a block, two blocks on a CU; Q6_K 1.02..1.31 times the row kernel (75 x 7670 x 1024
          *    20.9 -> 16.0 us), Q8_0 1.03..1.18 where there is more than a block per CU.  A block alone on its CU gains nothing from the
-         *    second place and pays the way through LDS and the barrier: Q8_0 0.82..0.93, Q6_K 0.92..0.96 where a wave has but one step (512).
+         *    second place and pays the way through LDS and the barrier: Q8_0 0.82..0.93, Q6_K 0.92..0.96 where a wave has but one step (512)
+         *    and 0.94..1.00 where two row tiles fill the CUs once (96 x 4096 x 1024 11.3 -> 11.7).
          *  - longer: a wave whose share does not begin and end with a run loads runs that its neighbours load too, which the row kernel
          *    does not: Q6_K 0.97..1.00 at one row tile and a second round of blocks, 1.02..1.26 otherwise; Q8_0 (runs of 128) 0.89..0.98 up to five steps a
          *    wave (two bytes off a dword up to eight, at one row tile up to nine: 0.94..0.99), 1.01..1.29 beyond and at four.
          *  - Q8_0 rows that are a multiple of 64 bytes apart: the row kernel's 64 rows fall on few cache sets; 1.00..1.29. */
         const int per = ((K + F::STEP - 1) / F::STEP + F32_WAVES - 1) / F32_WAVES;
-        const bool filled = ntg * ((N + 31) / 32) > 256, fits = K <= F::SHORT_RUNS * F::RUN * F::STEP;
+        const bool filled = ntg * ((N + 32 * R - 1) / (32 * R)) > 256, fits = K <= F::SHORT_RUNS * F::RUN * F::STEP;
         bool once, runs;
         if constexpr (std::is_same<F, F32Q6K>::value) {
-            once = fits && (filled || per > 1);
+            once = fits && (filled || (R == 1 && per > 1));
             runs = !fits && !(R == 1 && filled && per % F::RUN);
         } else {
             once = fits && filled;
@@ -739,9 +738,6 @@ int launch_f32act(const float *A, const uint8_t *B, const float *bias, float *C,
             kernel = gemm_f32run_kernel<F, 1, true>;
         } else if (runs)
             kernel = R == 2 ? gemm_f32run_kernel<F, 2, false> : gemm_f32run_kernel<F, 1, false>;
-        else if constexpr (std::is_same<F, F32Q80>::value) {
-            if (R == 2) kernel = gemm_f32row_kernel<F, 2>;
-        }                                    /* Q6_K: R is 1 here */
     }
     const long long grid = ntg * ((N + 32 * R - 1) / (32 * R));
     if (grid > 0x7fffffffll) return CKQ_ESHAPE;
