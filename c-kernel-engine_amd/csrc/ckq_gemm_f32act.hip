@@ -720,9 +720,13 @@ int launch_f32act(const float *A, const uint8_t *B, const float *bias, float *C,
          *    second place and pays the way through LDS and the barrier: Q8_0 0.82..0.93, Q6_K 0.92..0.96 where a wave has but one step (512)
          *    and 0.94..1.00 where two row tiles fill the CUs once (96 x 4096 x 1024 11.3 -> 11.7).
          *  - longer: a wave whose share does not begin and end with a run loads runs that its neighbours load too, which the row kernel
-         *    does not: Q6_K 0.97..1.00 at one row tile and a second round of blocks, 1.02..1.26 otherwise; Q8_0 (runs of 128) 0.89..0.98 up to five steps a
-         *    wave (two bytes off a dword up to eight, at one row tile up to nine: 0.94..0.99), 1.01..1.29 beyond and at four.
-         *  - Q8_0 rows that are a multiple of 64 bytes apart: the row kernel's 64 rows fall on few cache sets; 1.00..1.29. */
+         *    does not: Q6_K 0.97..1.00 at one row tile and a second round of blocks, 1.02..1.26 otherwise; Q8_0 two bytes off a dword 0.94..0.99 up to
+         *    eight steps a wave (at one row tile up to nine), 1.11..1.19 beyond (6 to 64 tokens, widths 9184 and 10272).
+         *  - longer Q8_0 on a dword (runs of 128), whose rows a lane reads in whole dwords: 0.85..1.02 up to nine steps. From ten on it depends on
+         *    the tokens, since the run kernel's way is as long for one as for 32, and on the blocks: one row tile, 6 and 16 tokens 0.92..1.00; from 28
+         *    on 0.98..1.08 up to 129 blocks, 0.95..1.05 at 179 to 194, 0.90..0.95 at 258; two row tiles 1.03..1.05 (40 to 160 tokens).
+         *  - Q8_0 rows that are a multiple of 64 bytes apart: the row kernel's 64 rows fall on few cache sets; 1.00..1.29 (an odd multiple, 5120,
+         *    at 6 and 16 tokens 0.95..1.03). */
         const int per = ((K + F::STEP - 1) / F::STEP + F32_WAVES - 1) / F32_WAVES;
         const bool filled = ntg * ((N + 32 * R - 1) / (32 * R)) > 256, fits = K <= F::SHORT_RUNS * F::RUN * F::STEP;
         bool once, runs;
@@ -731,7 +735,8 @@ int launch_f32act(const float *A, const uint8_t *B, const float *bias, float *C,
             runs = !fits && !(R == 1 && filled && per % F::RUN);
         } else {
             once = fits && filled;
-            runs = K % 1024 == 0 || per >= 10 || (R == 2 && (per == 4 || per >= (K % 64 ? 9 : 6)));
+            runs = K % 2048 == 0 || (K % 64 ? per >= (R == 2 ? 9 : 10)
+                                            : M >= 28 && (K % 1024 == 0 || (per >= 10 && (R == 2 || ntg * ((N + 31) / 32) <= 160))));
         }
         if (once) {
             R = 1;

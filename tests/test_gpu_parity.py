@@ -1385,6 +1385,31 @@ def test_f32act_short_rows(fmt, widths):
         L.ckq_set_gemm_policy(0)
 
 
+@pytest.mark.parametrize("K,N,few,more", [(4672, 70, 27, 28), (4672, 5120, 27, 28), (4672, 5121, 27, 28), (4704, 70, 27, 28), (4672, 70, 29, 33),
+                                          (4672, 4097, 64, 96), (4608, 4097, 64, 96), (5120, 70, 27, 28)])
+def test_f32act_q8_0_token_tiles_partly_filled(K, N, few, more):
+    """Both sides of the choice between a row per lane and weights in memory order by tokens, blocks and width: the tokens that both calls
+    have keep their bits, and all are right against float64 (a sum of at most 28 additions, as in the test above)."""
+    import torch
+    L = ckq.lib()
+    W = T.random_blocks("q8_0", N * K // 32, 70 + N)
+    x = T.normal(more * K, 0.5, 1.0, seed=K)
+    W_d, x_d = P.to_device(W), P.to_device(x)
+    L.ckq_set_gemm_policy(1)
+    try:
+        got = []
+        for M in (few, more):
+            c = torch.full((M, N), 7.0, dtype=torch.float32, device="cuda")
+            say("f32act q8_0 partly filled", K, M, N)
+            P.check(L.ckq_gemm_nt_f32act_dev(P.FMT["q8_0"], P._dp(x_d), P._dp(W_d), None, P._dp(c), M, N, K, N, P._stream()), "f32act")
+            got.append(c)
+    finally:
+        L.ckq_set_gemm_policy(0)
+    assert torch.equal(got[0].view(torch.int32), got[1][:few].view(torch.int32))
+    X, V = x_d.view(more, K).double(), torch.from_numpy(T.np_dequant("q8_0", W).reshape(N, K)).cuda().double()
+    assert bool(((got[1] - X @ V.T).abs() <= 3e-7 * (X.abs() @ V.abs().T)).all())
+
+
 # ---- 16-row tiles: a few to a few dozen tokens of the K-quants -------------------------------------
 
 @pytest.mark.parametrize("fmt", ["q4_k", "q5_k", "q6_k"])
