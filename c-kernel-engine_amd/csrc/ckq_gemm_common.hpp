@@ -25,6 +25,7 @@ struct GemmProblem {
     float         *C;
     long           ldc;
     int            N, nnt, id0;
+    int            tt0, ntt;   /* its token tiles: all of the matrix, or the whole ones, or the ragged one (gemm_deal_ragged_last) */
 };
 
 struct GemmArgs {
@@ -86,7 +87,7 @@ struct GemmOpts {
 /* What one block of a GEMM launch does: which tile id, which K-steps, where it
  * writes and whether it adds the bias. */
 struct GemmOut { float *C; long ldc; const float *bias; };
-struct GemmWork { int id, k0, k1; GemmOut out; const uint8_t *B; int N, nnt; };
+struct GemmWork { int id, k0, k1; GemmOut out; const uint8_t *B; int N, nnt, tt0, ntt; };
 __device__ __forceinline__ GemmWork gemm_work(const GemmArgs &a, int k_steps)
 {
     const int id = blockIdx.x;
@@ -96,12 +97,12 @@ __device__ __forceinline__ GemmWork gemm_work(const GemmArgs &a, int k_steps)
         if (id >= a.grp[1].id0) g = a.grp[1];
         if (a.ngroup > 2 && id >= a.grp[2].id0) g = a.grp[2];
         if (a.ngroup > 3 && id >= a.grp[3].id0) g = a.grp[3];
-        return {id - g.id0, 0, k_steps, {g.C, g.ldc, g.bias}, g.B, g.N, g.nnt};
+        return {id - g.id0, 0, k_steps, {g.C, g.ldc, g.bias}, g.B, g.N, g.nnt, g.tt0, g.ntt};
     }
-    if (a.splits <= 1) return {id, 0, k_steps, {a.C, a.ldc, a.bias}, a.B, a.N, a.nnt};
+    if (a.splits <= 1) return {id, 0, k_steps, {a.C, a.ldc, a.bias}, a.B, a.N, a.nnt, 0, a.ntt};
     const int k0 = (int)blockIdx.y * a.k_per;
     return {id, k0, min(k_steps, k0 + a.k_per),
-            {a.part + (size_t)blockIdx.y * (size_t)a.M * (size_t)a.N, (long)a.N, nullptr}, a.B, a.N, a.nnt};
+            {a.part + (size_t)blockIdx.y * (size_t)a.M * (size_t)a.N, (long)a.N, nullptr}, a.B, a.N, a.nnt, 0, a.ntt};
 }
 
 /* The tiles of a launch, ntt token tiles of nnt tiles of weight rows, token tiles fastest so that neighbours share weights, are dealt
@@ -109,9 +110,9 @@ __device__ __forceinline__ GemmWork gemm_work(const GemmArgs &a, int k_steps)
  * tiles per XCD leave some with a row more, and with few rows CUs there with two or three tiles beside others with one (us, rows of
  * tiles -> runs: Q6_K 680 tokens x 2111 rows x 4352 57.8 -> 32.6, Q5_K 67 x 1509 x 10240 32.6 -> 21.3, Q4_K 339 x 1432 x 6656 33.0 -> 20.8;
  * 60 random sizes 0.5 to 5 % on average, the same bits).  gemm_blocks: block ids to launch; false: no tile. */
-__device__ __forceinline__ bool gemm_tile(int id, int ntt, int nnt, int &nt, int &tt)
+__host__ __device__ __forceinline__ bool gemm_tile(int id, int ntt, int nnt, int &nt, int &tt)
 {
-    const int total = ntt * nnt, xcd = id & 7, seq = id >> 3, t = xcd * (total >> 3) + min(xcd, total & 7) + seq;
+    const int total = ntt * nnt, xcd = id & 7, seq = id >> 3, t = xcd * (total >> 3) + (xcd < (total & 7) ? xcd : total & 7) + seq;
     nt = t / ntt;
     tt = t - nt * ntt;
     return seq < (total >> 3) + (xcd < (total & 7) ? 1 : 0);
@@ -262,12 +263,54 @@ static int gemm_launch_grouped(Kernel kernel, GemmArgs &g, const GemmGroupIn &in
     g.ngroup = in.n;
     for (int p = 0; p < in.n; ++p) {
         const int nnt = (in.N[p] + GEMM_TILE_ROWS - 1) / GEMM_TILE_ROWS;
-        g.grp[p] = {(const uint8_t *)in.B[p], in.bias[p], in.C[p], in.ldc[p], in.N[p], nnt, (int)grid};
+        g.grp[p] = {(const uint8_t *)in.B[p], in.bias[p], in.C[p], in.ldc[p], in.N[p], nnt, (int)grid, 0, g.ntt};
         grid += (unsigned)gemm_blocks(g.ntt - last_apart, nnt) + (last_apart ? (unsigned)gemm_blocks(1, nnt) : 0u);
     }
     g.B = g.grp[0].B; g.bias = g.grp[0].bias; g.C = g.grp[0].C; g.N = g.grp[0].N; g.ldc = g.grp[0].ldc; g.nnt = g.grp[0].nnt;
     g.splits = 1; g.k_per = 0; g.part = nullptr;
     hipLaunchKernelGGL(kernel, dim3(grid, 1u), dim3(threads), 0, s, g);
+    return (int)hipGetLastError();
+}
+
+/* Kernels with two blocks on a CU: whether the ragged token tiles (a matrix' last, of M % bm tokens, at most half a tile: less of everything
+ * but the arithmetic) belong behind the whole ones of all matrices.  They do where the whole tiles of an XCD just fill its 32 CUs, or
+ * once or twice its 64 slots, and the ragged ones are too many: what is left over is then short blocks alone.  us, in turn with the
+ * ragged ones | last: Q5_K 405 tokens x 2 x 11008 rows x 2816 97.6 | 93.1, 276 x 2 x 7680 x 2048 47.1 | 43.0, 139 x 2 x 5888 x 1536 24.6 | 22.6;
+ * Q4_K 405 x 2 x 11008 x 4096 109.9 | 106.0.  Where a few whole ones are left over as well those come late (Q5_K 341 x 2 x 6912 x 2048, 68 of an XCD,
+ * 44.9 | 47.6; after two rounds blocks are out of step and four more do no harm), and so do tiles of more than half (227 x 2 x 8960 x 2816
+ * 59.0 | 63.6); beyond that there is nothing to gain (99 launches outside the rule: 1.00 on average). */
+static bool gemm_ragged_last(const GemmGroupIn &in, int M, int bm)
+{
+    if (M < bm || M % bm == 0 || M % bm > bm / 2 || 2 * in.n > GEMM_GROUP_MAX) return false;
+    int whole = 0, all = 0;                    /* tiles of the fullest XCD */
+    for (int p = 0; p < in.n; ++p) {
+        const int nnt = (in.N[p] + GEMM_TILE_ROWS - 1) / GEMM_TILE_ROWS;
+        whole += gemm_blocks(M / bm, nnt) / 8;
+        all += gemm_blocks(M / bm + 1, nnt) / 8;
+    }
+    return (whole <= 32 && all > 32) || (whole <= 64 && all > 64) || (whole <= 132 && all > 128);
+}
+
+/* One matrix or a group with the ragged token tiles as problems of their own behind the whole ones; returns the blocks to launch. */
+static int gemm_deal_ragged_last(GemmArgs &g, const GemmGroupIn &in, int bm)
+{
+    const int nfull = g.M / bm;
+    int grid = 0;
+    g.ngroup = 0;
+    for (int ragged = 0; ragged < 2; ++ragged)
+        for (int p = 0; p < in.n; ++p) {
+            const int nnt = (in.N[p] + GEMM_TILE_ROWS - 1) / GEMM_TILE_ROWS, ntt = ragged ? 1 : nfull;
+            g.grp[g.ngroup++] = {(const uint8_t *)in.B[p], in.bias[p], in.C[p], in.ldc[p], in.N[p], nnt, grid, ragged ? nfull : 0, ntt};
+            grid += gemm_blocks(ntt, nnt);
+        }
+    g.splits = 1; g.k_per = 0; g.part = nullptr;
+    return grid;
+}
+template <class Kernel>
+static int gemm_launch_ragged_last(Kernel kernel, GemmArgs &g, const GemmGroupIn &in, int bm, hipStream_t s)
+{
+    const int grid = gemm_deal_ragged_last(g, in, bm);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid, 1u), dim3(256u), 0, s, g);
     return (int)hipGetLastError();
 }
 

@@ -204,7 +204,8 @@ __global__ void __launch_bounds__(256 * KG, KG == 2 ? 1 : WPE) gemm_q4k_mfma_ker
 
     const GemmWork work = gemm_work(a, a.nb);
     int nt, tt;
-    if (!gemm_tile(work.id, a.ntt, work.nnt, nt, tt)) return;
+    if (!gemm_tile(work.id, work.ntt, work.nnt, nt, tt)) return;
+    tt += work.tt0;
     const int t0 = tt * BM, n0 = nt * GEMM_BN;
     const u32 wstride = (u32)a.nb * 144u, xstride = (u32)a.nb * 292u;
     const int b0 = work.k0, b1 = work.k1, last = b1 - 1;
@@ -423,6 +424,8 @@ int launch_gemm_q4k_mfma(const void *A, const void *B, const float *bias, float 
 #endif
     }
     if (two_groups) return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 2>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s, 512);
+    const GemmGroupIn one = {1, {B}, {bias}, {C}, {N}, {ldc}};
+    if (tiles > 256 && gemm_ragged_last(one, M, GEMM_BM)) return gemm_launch_ragged_last(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 1>, g, one, GEMM_BM, s);
     return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 1>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s, 256);
 }
 
@@ -446,5 +449,6 @@ int launch_gemm_q4k_mfma_group(const void *A, const GemmGroupIn &in, int M, int 
     g.ntt = (M + GEMM_BM - 1) / GEMM_BM;
     /* as for one matrix: two groups of waves per tile while every tile gets a CU of its own */
     if (tiles <= 256 && g.nb >= 8) return gemm_launch_grouped(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 2>, g, in, s, 512);
+    if (gemm_ragged_last(in, M, GEMM_BM)) return gemm_launch_ragged_last(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 1>, g, in, GEMM_BM, s);
     return gemm_launch_grouped(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 1>, g, in, s, 256);
 }

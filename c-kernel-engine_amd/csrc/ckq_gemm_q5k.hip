@@ -335,7 +335,8 @@ __global__ void __launch_bounds__(256, 2) gemm_q5k_pair_kernel(GemmArgs a)
 
     const GemmWork work = gemm_work(a, a.nb);
     int nt, tt;
-    if (!gemm_tile(work.id, a.ntt, work.nnt, nt, tt)) return;
+    if (!gemm_tile(work.id, work.ntt, work.nnt, nt, tt)) return;
+    tt += work.tt0;
     const int t0 = tt * BM, n0 = nt * GEMM5_BN;
     const u32 wstride = (u32)a.nb * 176u, xstride = (u32)a.nb * 292u;
     const int b0 = work.k0, b1 = work.k1, last = b1 - 1;
@@ -449,6 +450,22 @@ static bool q5k_take_pair(int tiles)
     return forced ? forced == 2 : tiles > 256;
 }
 
+extern "C" int ckq_launch_ragged_last(int M, int n, const int *N, int id, int *matrix, int *nt, int *tt)
+{
+    GemmGroupIn in = {};
+    GemmArgs g = {};
+    in.n = n;
+    for (int p = 0; p < n; ++p) in.N[p] = N[p];
+    if (!gemm_ragged_last(in, M, GEMM5_BM)) return 0;
+    g.M = M;
+    const int grid = gemm_deal_ragged_last(g, in, GEMM5_BM);
+    int p = 0;
+    while (p + 1 < g.ngroup && id >= g.grp[p + 1].id0) ++p;
+    *matrix = gemm_tile(id - g.grp[p].id0, g.grp[p].ntt, g.grp[p].nnt, *nt, *tt) ? p % n : -1;
+    *tt += g.grp[p].tt0;
+    return grid;
+}
+
 GemmChains gemm_q5k_chains(int M, int N, int K)
 {
     return gemm_chains_split(((M + GEMM5_BM - 1) / GEMM5_BM) * ((N + GEMM5_BN - 1) / GEMM5_BN), K / 256);
@@ -474,6 +491,8 @@ int launch_gemm_q5k_mfma(const void *A, const void *B, const float *bias, float 
 #else
         if (sums) return CKQ_ENODUMP;
 #endif
+        const GemmGroupIn one = {1, {B}, {bias}, {C}, {N}, {ldc}};
+        if (g.ntt * g.nnt > 256 && gemm_ragged_last(one, M, GEMM5_BM)) return gemm_launch_ragged_last(gemm_q5k_pair_kernel<false>, g, one, GEMM5_BM, s);
         return gemm_launch_split(gemm_q5k_pair_kernel<false>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s);
     }
 #if CKQ_WITH_DUMP
@@ -497,6 +516,9 @@ int launch_gemm_q5k_mfma_group(const void *A, const GemmGroupIn &in, int M, int 
     g.A = (const uint8_t *)A; g.M = M; g.nb = K / 256;
     if ((long long)g.nb * 292 * 128 >= (1ll << 31)) return (int)hipErrorInvalidValue;
     g.ntt = (M + GEMM5_BM - 1) / GEMM5_BM;
-    if (q5k_take_pair(gemm_group_tiles(in, M, GEMM5_BM))) return gemm_launch_grouped(gemm_q5k_pair_kernel<false>, g, in, s);
+    if (q5k_take_pair(gemm_group_tiles(in, M, GEMM5_BM))) {
+        if (gemm_ragged_last(in, M, GEMM5_BM)) return gemm_launch_ragged_last(gemm_q5k_pair_kernel<false>, g, in, GEMM5_BM, s);
+        return gemm_launch_grouped(gemm_q5k_pair_kernel<false>, g, in, s);
+    }
     return gemm_launch_grouped(gemm_q5k_mfma_kernel<false>, g, in, s);
 }

@@ -96,6 +96,9 @@ void ckq_launch_set_q6k_variant(int variant);
 /* Q5_K x Q8_K matrix-core GEMM: 0 = by tile count (default), 1 = one block per CU, 2 = the paired kernel,
  * wherever the GEMM is taken. */
 void ckq_launch_set_q5k_variant(int variant);
+/* Whether n (1..4) matrices of N[i] rows against M tokens have their ragged 64-token tiles dealt last (Q5_K paired, Q4_K 64-token kernel):
+ * 0, or the blocks of the launch, and then which tile block `id` has (*matrix -1: none).  Host arithmetic; exported for the test of the rule. */
+int ckq_launch_ragged_last(int M, int n, const int *N, int id, int *matrix, int *nt, int *tt);
 /* K-quants: 1 = the 16-row tiles take every matmul of two and more tokens (K up to 16384), 0 = by shape (default). */
 void ckq_launch_set_rows16(int fmt, int on);
 

@@ -216,6 +216,29 @@ def test_16_row_tiles_where_they_are_the_faster_ones(L, fmt, n, k, tokens, want)
     assert route(L, fmt, n, k, tokens) == want
 
 
+@pytest.mark.parametrize("M,Ns,last", [(405, (11008, 11008), True), (276, (7680, 7680), True), (139, (5888, 5888), True), (282, (7041,), True), (65, (17000,), True),
+                                       (88, (9000, 7700), True), (341, (6912, 6912), False), (384, (11008, 11008), False), (227, (8960, 8960), False),
+                                       (405, (4096, 1024, 1024), False), (9, (34000,), False), (400, (28672,), False)])
+def test_ragged_token_tiles_dealt_last(L, M, Ns, last):
+    """Sizes at which the order of a launch's tiles was timed.  Dealt last, the ragged tiles have the highest block ids, every tile
+    has one block, and an XCD (block id modulo 8) has at most two more of a matrix than another."""
+    N, out = (ctypes.c_int * len(Ns))(*Ns), [ctypes.c_int() for _ in range(3)]
+
+    def tile(i):
+        grid = L.ckq_launch_ragged_last(M, len(Ns), N, i, *map(ctypes.byref, out))
+        return grid, tuple(o.value for o in out)
+    grid = tile(0)[0]
+    assert bool(grid) == last
+    if last:
+        dealt = [(i, t) for i, t in ((i, tile(i)[1]) for i in range(grid)) if t[0] >= 0]
+        whole, tiles = M // 64, [-(-n // 128) for n in Ns]
+        assert sorted(t for _, t in dealt) == [(p, r, c) for p, n in enumerate(tiles) for r in range(n) for c in range(whole + 1)]
+        order = [c == whole for _, (_, _, c) in dealt]
+        assert order == sorted(order)
+        per_xcd = [sum(i % 8 == x for i, _ in dealt) for x in range(8)]
+        assert max(per_xcd) - min(per_xcd) <= 2 * len(Ns)
+
+
 def test_workspace_slot_bookkeeping(L):
     """Slot choice of the per-(device, stream, kind) scratch table of the K-split
     GEMMs: a known key finds its slot, a new key takes the first free slot, and

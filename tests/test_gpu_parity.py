@@ -1711,6 +1711,32 @@ def test_gemm_mfma_tiles_over_the_xcds(fmt, M):
             assert float((a - w).abs().max()) <= bar and float((b - w).abs().max()) <= bar
 
 
+@pytest.mark.parametrize("fmt,variants", [("q5_k", (2, 1)), ("q4_k", (64, 96))])
+@pytest.mark.parametrize("M,Ns,K", [(405, (11008, 11008), 768), (65, (17000,), 512), (88, (9000, 7700), 256), (282, (7041,), 1024), (257, (6657, 300), 512)])
+def test_gemm_ragged_token_tiles_dealt_last(fmt, variants, M, Ns, K):
+    """Launches whose ragged token tiles come last, one matrix and two, with a bias and a padded C: the bits of the other tile kernel of the
+    format, which deals its tiles otherwise, and nothing beside C's columns."""
+    import torch
+    L = ckq.lib()
+    say("ragged tiles last", fmt, M, Ns, K)
+    xq = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, 9990)), "q8_k", M)
+    Ws = [P.to_device(T.random_blocks(fmt, n * (K // 256), 9991 + n)) for n in Ns]
+    bs = [P.to_device(T.normal(n, 0.0, 0.5, 9992 + n)) for n in Ns]
+    got = []
+    try:
+        L.ckq_set_gemm_policy(1)
+        for v in variants:
+            L.ckq_set_prefill_variant(P.FMT[fmt], v)
+            ys = [torch.full((M, n + 3), 7.0, device="cuda") for n in Ns]
+            P.dev_matmul_sequence([(fmt, xq, W, b, y, M, n, K, n + 3) for W, b, y, n in zip(Ws, bs, ys, Ns)])
+            got.append(ys)
+    finally:
+        L.ckq_set_gemm_policy(0)
+        L.ckq_set_prefill_variant(P.FMT[fmt], 0)
+    for a, b, n in zip(got[0], got[1], Ns):
+        assert torch.equal(a, b) and bool((a[:, n:] == 7.0).all())
+
+
 @pytest.mark.parametrize("M,Ns,K", [(64, (20000,), 512), (40, (16700,), 1024), (160, (10000,), 768), (190, (4096, 2048, 3000), 512), (345, (10391,), 512), (266, (9000, 9000), 768),
                                     (247, (10593,), 2304), (129, (16300,), 256), (600, (3000,), 1280)])
 def test_gemm_q6_k_kernel_choice(M, Ns, K):
