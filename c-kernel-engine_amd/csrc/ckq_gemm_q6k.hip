@@ -453,10 +453,13 @@ __global__ void __launch_bounds__(256, 2) gemm_q6k_pair_kernel(GemmArgs a)
  * (paired).  us for nb 256-blocks of K, from 70 launches of 33 to 900 tokens, 2000 to 40000 rows and K of 512 to 11008:
  *   64 tokens    6.5 + 1.5 nb a round of 256 tiles
  *   128 tokens   10 + 2.35 nb a round of 256 tiles
- *   paired       7 + 2.9 nb a round of 512 tiles, a last round of up to 256 0.55 and a fuller one 0.85 of that
+ *   paired       7.6 + 2.8 nb a round of 512 tiles, the second and later ones 0.86 of that; a last round of a part f of the tiles 0.8 + 0.23 f where it is the
+ *                only one and 0.37 + 0.65 f after others (fitted to 110 launches of 33 to 1000 tokens: 3 % rms, choosing by it costs 0.15 % more than always
+ *                taking the faster one, at most 6 %)
  * Measured, us, 128 tokens -> 64: 48 x 32000 x 4096 (tokens, rows, K) 46.4 -> 32.1, 160 x 10000 x 4096 47.2 -> 31.3, 56 x 25595 x 6144
  * 63.3 -> 43.0; 128 tokens -> paired: 266 x 35817 x 768 62.7 -> 45.8, 345 x 10391 x 512 16.6 -> 13.7, 473 x 20320 x 2304 92.1 -> 81.6;
- * 512 x 11008 x 4096 95.6 -> 85.4; 128 tokens stay the fastest at 247 x 10593 x 3584 (43.2; 64 54.3, paired 48.9).  Every kernel gives the
+ * 512 x 11008 x 4096 95.6 -> 85.4, 252 x 8318 x 1280 22.5 -> 20.1, 600 x 31833 x 1536 119.6 -> 109.2; 128 tokens stay the fastest at 247 x 10593 x 3584 (43.2; 64 54.3,
+ * paired 48.9) and 241 x 13644 x 5632 (61.7; paired 67.6).  Every kernel gives the
  * same bits where nothing is split along K, and up to 256 tiles of 64 tokens, where something may be, it is always the first.
  * variant: 0 = by shape, 1 = never paired, 2 = always. */
 static std::atomic<int> g_q6k_variant{0};
@@ -468,11 +471,19 @@ static int q6k_form(int tiles64, int tiles128, int nb)
     const int forced = g_q6k_variant.load(std::memory_order_relaxed);
     if (forced == 2) return Q6K_PAIRED;
     if (tiles64 <= 256) return Q6K_64;
-    const float k = (float)nb, rest = (float)(tiles64 % 512 == 0 ? 0.0f : tiles64 < 512 ? 1.0f : tiles64 % 512 <= 256 ? 0.55f : 0.85f);
+    const int rounds = tiles64 / 512;
+    const float k = (float)nb, f = (float)(tiles64 % 512) / 512.0f;
     const float t64 = (float)((tiles64 + 255) / 256) * (6.5f + 1.5f * k), t128 = (float)((tiles128 + 255) / 256) * (10.0f + 2.35f * k);
-    const float paired = ((float)(tiles64 / 512) + rest) * (7.0f + 2.9f * k);
-    if (forced != 1 && paired <= t64 && paired <= 0.98f * t128) return Q6K_PAIRED;
+    const float n = rounds ? 1.0f + 0.86f * (float)(rounds - 1) + (f > 0.0f ? 0.37f + 0.65f * f : 0.0f) : 0.8f + 0.23f * f;
+    const float paired = n * (7.6f + 2.8f * k);
+    if (forced != 1 && paired <= t64 && paired <= 1.01f * t128) return Q6K_PAIRED;
     return t64 < t128 ? Q6K_64 : Q6K_128;
+}
+
+extern "C" int ckq_launch_q6k_form(int M, int N, int K)
+{
+    const int nnt = (N + GEMM6_BN - 1) / GEMM6_BN;
+    return q6k_form((M + 63) / 64 * nnt, (M + 127) / 128 * nnt, K / 256);
 }
 
 GemmChains gemm_q6k_chains(int M, int N, int K)

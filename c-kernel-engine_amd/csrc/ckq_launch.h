@@ -93,6 +93,8 @@ void ckq_launch_set_q4k_tile(int tokens);
 /* Q6_K x Q8_K matrix-core GEMM: 0 = by shape (default), 1 = one block per CU, 2 = the paired 64-token kernel,
  * wherever the GEMM is taken. */
 void ckq_launch_set_q6k_variant(int variant);
+/* Which kernel one Q6_K matrix has there: 0 = 64-token tiles, 1 = 128-token tiles, 2 = paired.  Host arithmetic; exported for the test of the rule. */
+int ckq_launch_q6k_form(int M, int N, int K);
 /* Q5_K x Q8_K matrix-core GEMM: 0 = by tile count (default), 1 = one block per CU, 2 = the paired kernel,
  * wherever the GEMM is taken. */
 void ckq_launch_set_q5k_variant(int variant);

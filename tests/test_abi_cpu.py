@@ -239,6 +239,13 @@ def test_ragged_token_tiles_dealt_last(L, M, Ns, last):
         assert max(per_xcd) - min(per_xcd) <= 2 * len(Ns)
 
 
+@pytest.mark.parametrize("M,N,K,form", [(326, 17318, 2816, 2), (252, 8318, 1280, 2), (162, 10958, 2816, 2), (600, 31833, 1536, 2), (266, 35817, 768, 2), (512, 11008, 4096, 2),
+                                        (247, 10593, 3584, 1), (241, 13644, 5632, 1), (105, 28675, 4864, 1), (48, 32000, 4096, 0), (160, 10000, 4096, 0), (93, 4096, 4096, 0)])
+def test_q6_k_kernel_is_the_fastest_one(L, M, N, K, form):
+    """Sizes at which the three kernels were timed against each other; the fastest one is taken."""
+    assert L.ckq_launch_q6k_form(M, N, K) == form
+
+
 def test_workspace_slot_bookkeeping(L):
     """Slot choice of the per-(device, stream, kind) scratch table of the K-split
     GEMMs: a known key finds its slot, a new key takes the first free slot, and
