@@ -327,7 +327,7 @@ static const DwForm dw_forms[5] = {{1, 1, 3, 4.0f, 0.40f, 0.39f, 0.0f}, {2, 1, 2
 /* The form for `row_tiles` tiles of weight rows in all; single: one matrix, which may be split along K.  64 tokens and one team
  * are always possible; another form only if its chains of multiply-adds are no longer (fewer splits of K would make them so, and the
  * error larger) and, if it is split, with no more scratch than that form or the entry point that allocates nothing has. */
-static int dw_form(int M, int nb, long rows, long row_tiles, bool single, float *time)
+static int dw_form(int M, int nb, long rows, long row_tiles, bool single)
 {
     const int steps = (nb + GEMM8_KB - 1) / GEMM8_KB;
     const float out = 1e-6f * (float)M * (float)rows;
@@ -350,7 +350,6 @@ static int dw_form(int M, int nb, long rows, long row_tiles, bool single, float 
                         1.45f * out * (float)(s > 1 ? 1 + 2 * s : 1) + (s > 1 ? 2.4f : 0.0f);
         if (k == 1 || t < least) { least = t; best = k; }
     }
-    if (time) *time = least;
     return best;
 }
 
@@ -368,7 +367,7 @@ static int dw_launch(GemmArgs &g, hipStream_t s)
 }
 int gemm_q80_dw_launch(GemmArgs &g, hipStream_t s)
 {
-    switch (dw_form(g.M, g.nb, g.N, g.nnt, true, nullptr)) {
+    switch (dw_form(g.M, g.nb, g.N, g.nnt, true)) {
     case 0: return dw_launch<1, 1>(g, s);
     case 1: return dw_launch<2, 1>(g, s);
     case 2: return dw_launch<3, 1>(g, s);
@@ -389,16 +388,9 @@ int gemm_q80_dw_launch_group(GemmArgs &g, const GemmGroupIn &in, hipStream_t s)
         rows += in.N[p];
         tiles += (in.N[p] + GEMM8_BN - 1) / GEMM8_BN;
     }
-    switch (dw_form(g.M, g.nb, rows, tiles, false, nullptr)) {
+    switch (dw_form(g.M, g.nb, rows, tiles, false)) {
     case 0: return dw_launch_group<1>(g, in, s);
     case 1: return dw_launch_group<2>(g, in, s);
     default: return dw_launch_group<3>(g, in, s);
     }
-}
-
-float gemm_q80_dw_time(int M, long rows, int nb)
-{
-    float t;
-    dw_form(M, nb, rows, (rows + GEMM8_BN - 1) / GEMM8_BN, true, &t);
-    return t;
 }

@@ -47,27 +47,19 @@ static std::atomic<int> g_gemm_policy{0};      /* 0 automatic, 1 matrix cores ab
 
 extern "C" void ckq_launch_set_gemm_policy(int policy) { g_gemm_policy.store(policy < 0 || policy > 2 ? 0 : policy); }
 
-static int stream_lanes(int positions);
-float gemm_q80_dw_time(int M, long rows, int nb);
-
 /* Q8_0 has its own estimate (us, weight bytes in MB): streaming 4.8 + passes * MB / 5.0 (MB / 3.6 for rows it must read with
  * 2-byte-aligned loads), matrix cores max(14, 9 + MB / 2.5), measured with ckq_gemm_q80.hip.  LM head 151936x896 (145 MB):
  * 9-16 tokens stream, 17 and more go to the matrix cores; 4864x896 (4.6 MB) streams up to 72 tokens.  Rows on dwords run the
  * faster ckq_gemm_q80_dw.hip since, which is ahead earlier (two passes over large matrices: 16 tokens, 32000x4096 60 against 28; the
- * second kernel's 8 to 14 us for small ones), but the line also says which order of sums a size has, so it stays.  It moves
- * where eight tokens do not fit the streaming kernel's LDS and it slows down several times over: there it takes
- * 4.1 + 0.23 K / 1000 + 6.15 per million lanes of all rows and passes (stream_lanes) + 0.52 MB and pass (11 tokens, 16532x7296: 174
- * against 41), and the estimate of the other kernel's forms, 6 % on the low side, stands against it. */
-static bool gemm_q80_on_matrix_cores(int ntok, size_t rows, int K, bool aligned_rows)
+ * second kernel's 8 to 14 us for small ones), but the line also says which order of sums a size has, whether it may be split along K and
+ * so needs scratch, and stays where it is at every K: the tile kernel's one chain of additions over a row is less exact than the streaming
+ * kernel's terms per lane and tree (rms error of the rms result at K = 7296: 1.9e-7, with two teams 1.4e-7, against 0.8e-7). */
+static bool gemm_q80_on_matrix_cores(int ntok, size_t weight_bytes, bool aligned_rows)
 {
     const int policy = g_gemm_policy.load(std::memory_order_relaxed);
     if (ntok <= CKQ_STREAM_TOKENS || policy == 2) return false;
     if (policy == 1) return true;
-    const float passes = (float)((ntok + CKQ_STREAM_TOKENS - 1) / CKQ_STREAM_TOKENS), mb = (float)(rows * (size_t)(K / 32)) * 34e-6f;
-    if (aligned_rows && (size_t)CKQ_STREAM_TOKENS * (size_t)(K / 32) * 36 > 65536) {
-        const float t_stream = 4.1f + 0.23e-3f * (float)K + 6.15e-6f * passes * (float)rows * (float)stream_lanes(K / 32) + 0.52f * passes * mb;
-        return t_stream > 1.05f * gemm_q80_dw_time(ntok, (long)rows, K / 32);
-    }
+    const float passes = (float)((ntok + CKQ_STREAM_TOKENS - 1) / CKQ_STREAM_TOKENS), mb = (float)weight_bytes * 1e-6f;
     return 4.8f + passes * mb / (aligned_rows ? 5.0f : 3.6f) > fmaxf(14.0f, 9.0f + mb / 2.5f);
 }
 
@@ -356,7 +348,7 @@ extern "C" int ckq_launch_route(int fmt, int nrows, int K, int ntok, int aligned
         tiles = kquant_on_matrix_cores(fmt, ntok, (size_t)nrows, K);
         if (take_rows16(fmt, ntok, (size_t)nrows, K, tiles)) return tiles ? CKQ_ROUTE_ROWS16_TILES : CKQ_ROUTE_ROWS16_STREAM;
         break;
-    case CKQ_FMT_Q8_0: tiles = gemm_q80_on_matrix_cores(ntok, (size_t)nrows, K, K % 64 == 0 && aligned); break;
+    case CKQ_FMT_Q8_0: tiles = gemm_q80_on_matrix_cores(ntok, (size_t)nrows * (K / 32) * 34, K % 64 == 0 && aligned); break;
     case CKQ_FMT_Q5_0: tiles = gemm_on_matrix_cores(ntok, (size_t)nrows * (K / 32) * 22, 20); break;
     case CKQ_KERNEL_Q80_F32: case CKQ_KERNEL_Q4K_F32: case CKQ_KERNEL_Q6K_F32: tiles = f32act_on_matrix_cores(fmt, ntok, nrows, K); break;
     default: return CKQ_EFORMAT;
@@ -674,7 +666,7 @@ extern "C" int ckq_launch_gemm_group(int fmt, int n, float *const *C, const void
         return launch_gemm_q6k_mfma_group(A, in, M, K, s);
     case CKQ_FMT_Q8_0:
         if (K % 32) return CKQ_ESHAPE;
-        if (!gemm_q80_on_matrix_cores(M, rows, K, K % 64 == 0 && aligned)) return CKQ_ENOGROUP;
+        if (!gemm_q80_on_matrix_cores(M, rows * (K / 32) * 34, K % 64 == 0 && aligned)) return CKQ_ENOGROUP;
         return launch_gemm_q80_mfma_group(A, in, M, K, s);
     default:
         return CKQ_ENOGROUP;

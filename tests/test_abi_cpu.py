@@ -239,6 +239,18 @@ def test_ragged_token_tiles_dealt_last(L, M, Ns, last):
         assert max(per_xcd) - min(per_xcd) <= 2 * len(Ns)
 
 
+def test_q8_0_order_of_sums_does_not_hang_on_the_width(L):
+    """Long rows on dwords stream where shorter rows of as many bytes do, up to 16 tokens always: the tile kernel's chains of additions are longer, and
+    it may need scratch for a split along K.  Host arithmetic of the same line."""
+    for k in (3648, 7232, 7296, 8192, 9728, 11008, 16384):
+        for n in (200, 600, 1200, 4096, 16532):
+            mb = n * (k // 32) * 34e-6
+            for t in (9, 11, 16, 17, 24, 40, 64):
+                tiles = 4.8 + -(-t // 8) * mb / 5.0 > max(14.0, 9.0 + mb / 2.5)
+                assert route(L, "q8_0", n, k, t) == (TILES if tiles else STREAM), (n, k, t)
+                assert t > 16 or not tiles
+
+
 @pytest.mark.parametrize("M,N,K,form", [(326, 17318, 2816, 2), (252, 8318, 1280, 2), (162, 10958, 2816, 2), (600, 31833, 1536, 2), (266, 35817, 768, 2), (512, 11008, 4096, 2),
                                         (247, 10593, 3584, 1), (241, 13644, 5632, 1), (105, 28675, 4864, 1), (48, 32000, 4096, 0), (160, 10000, 4096, 0), (93, 4096, 4096, 0)])
 def test_q6_k_kernel_is_the_fastest_one(L, M, N, K, form):

@@ -1493,6 +1493,37 @@ def test_streamed_tokens_have_the_bits_of_single_ones(fmt, N, K):
         L.ckq_set_gemm_policy(0)
 
 
+@pytest.mark.parametrize("M,N,K", [(9, 500, 7296), (16, 4100, 7296), (11, 1500, 9728), (13, 300, 11008), (40, 200, 8192)])
+def test_q8_0_long_rows_of_several_tokens_stream(M, N, K):
+    """The automatic choice for long Q8_0 rows has the streaming kernel's bits, from the entry point that allocates nothing too, and an error
+    against 64 bits no larger than that of one token at a time (rms; a tenth for the spread over some thousand outputs)."""
+    import torch
+    L = ckq.lib()
+    say("q8_0 long rows", M, N, K)
+    xq = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, seed=M)), "q8_0", rows=M)
+    W = P.to_device(T.random_blocks("q8_0", N * K // 32, 9720))
+    auto = P.dev_gemm_nt("q8_0", xq, W, None, M, N, K).view(M, N).clone()
+    bare = torch.full((M, N), 7.0, device="cuda")
+    P.check(L.ckq_gemm_nt_noalloc_dev(P.FMT["q8_0"], P._dp(xq), P._dp(W), None, P._dp(bare), M, N, K, N, P._stream()), "ckq_gemm_nt_noalloc_dev")
+    try:
+        L.ckq_set_gemm_policy(2)
+        streamed = P.dev_gemm_nt("q8_0", xq, W, None, M, N, K).view(M, N)
+    finally:
+        L.ckq_set_gemm_policy(0)
+    assert torch.equal(auto, streamed) and torch.equal(auto, bare)
+
+    def values(blocks, rows):
+        b = blocks.cpu().view(rows, K // 32, 34)
+        d = b[:, :, :2].contiguous().view(torch.float16).double()
+        return (b[:, :, 2:].contiguous().view(torch.int8).double() * d).view(rows, K)
+    exact = values(xq, M) @ values(W, N).T
+    one = torch.stack([P.dev_gemm_nt("q8_0", xq.view(M, -1)[m].clone(), W, None, 1, N, K).view(N) for m in range(M)])
+
+    def rms(y):
+        return float((y.double().cpu() - exact).square().mean().sqrt())
+    assert rms(auto) <= 1.1 * rms(one)
+
+
 @pytest.mark.parametrize("fmt", ["q4_k", "q5_k", "q6_k"])
 def test_16_row_tiles_of_short_rows_and_several_token_groups(fmt):
     """The kernel that keeps the planes of its weights across token groups: one to eight K-blocks (waves), two groups and many,
