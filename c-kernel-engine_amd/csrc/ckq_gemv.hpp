@@ -408,6 +408,10 @@ static int launch_mt(const GemvArgs &a, const GemvGroup &grp, int max_mt, hipStr
     if constexpr (F::TOKEN_TILES) {
         int mt, rpi;
         gemv_token_tile(LPR, launch_rows(a, grp), grp.n, a.ntok, &mt, &rpi);
+        /* a tile that LDS does not hold is read from memory again by every wave, position by position: a smaller one that it does hold is up to
+         * three times as fast although the weights are read more often (us: Q8_0 11 x 16532 x 7296 174 -> 69, 8 x 4096 x 7296 25.2 -> 14.3, 5 x 1500 x 11008
+         * 30.9 -> 11.4, Q5_0 8 x 11000 x 8192 62.1 -> 33.8, Q5_K 8 x 1500 x 8192 10.9 -> 8.0; Q5_0 12 x 1500 x 11008 23.8 -> 24.4); the bits of a token are the same */
+        while (mt > 2 && F::xs_lds_bytes((size_t)mt * (size_t)a.xrow) > 65536) mt /= 2;
         if (rpi == 1) {
             if (mt == 2) return launch_tile<F, LPR, PPL, 2, 1, 4>(a, grp, s);
             if (mt == 4) return launch_tile<F, LPR, PPL, 4, 1, 4>(a, grp, s);

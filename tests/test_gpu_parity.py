@@ -1493,6 +1493,28 @@ def test_streamed_tokens_have_the_bits_of_single_ones(fmt, N, K):
         L.ckq_set_gemm_policy(0)
 
 
+@pytest.mark.parametrize("fmt,K", [("q8_0", 7232), ("q8_0", 7264), ("q8_0", 7296), ("q8_0", 14528), ("q8_0", 14592), ("q5_0", 7264), ("q5_0", 7296), ("q5_0", 14592), ("q5_0", 30720),
+                                   ("q4_k", 7168), ("q4_k", 7424), ("q5_k", 7424), ("q6_k", 14336), ("q6_k", 14592), ("q5_k", 30720)])
+def test_streamed_token_tiles_at_the_limit_of_lds(fmt, K):
+    """Rows of which eight, four or two tokens just fit the staged tile or just do not, with and without two rows per slot: every token's outputs
+    are those of a call with that token alone, in the sense of the test above."""
+    import torch
+    L = ckq.lib()
+    try:
+        L.ckq_set_gemm_policy(2)
+        for N, M in ((70, 13), (2100, 5)):
+            say("streamed tiles at the limit", fmt, M, N, K)
+            W = P.to_device(T.random_blocks(fmt, N * K // ckq.api.BLOCK_ELEMS[fmt], 9730 + N % 97))
+            xq = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, seed=M)), P.act_format(fmt), rows=M).view(M, -1)
+            y = P.dev_gemm_nt(fmt, xq.view(-1), W, None, M, N, K).view(M, N)
+            for m in range(M):
+                one = P.dev_gemm_nt(fmt, xq[m].clone(), W, None, 1, N, K).view(N)
+                same = torch.equal(y[m], one) if fmt[-1] == "k" else torch.allclose(y[m], one, rtol=0, atol=2e-6 * float(one.abs().max()))
+                assert same, (M, m)
+    finally:
+        L.ckq_set_gemm_policy(0)
+
+
 @pytest.mark.parametrize("M,N,K", [(9, 500, 7296), (16, 4100, 7296), (11, 1500, 9728), (13, 300, 11008), (40, 200, 8192)])
 def test_q8_0_long_rows_of_several_tokens_stream(M, N, K):
     """The automatic choice for long Q8_0 rows has the streaming kernel's bits, from the entry point that allocates nothing too, and an error
