@@ -468,10 +468,14 @@ static int launch_pro_lpr(const GemvArgs &a, const GemvGroup &grp, const GemvPro
 {
     int mt = 1, rpi = 1;
     if (a.ntok > 1) gemv_token_tile(LPR, a.nrows, grp.n, a.ntok, &mt, &rpi);
-    /* tiles of four at most: eight tokens' rows beside the weights would not fit the registers */
-    if (rpi == 2) return mt == 2 ? launch_pro_one<F, LPR, 2, 2>(a, grp, pro, s) : launch_pro_one<F, LPR, 4, 2>(a, grp, pro, s);
-    return mt == 1 ? launch_pro_one<F, LPR, 1, 1>(a, grp, pro, s) : mt == 2 ? launch_pro_one<F, LPR, 2, 1>(a, grp, pro, s) : launch_pro_one<F, LPR, 4, 1>(a, grp, pro, s);
+    if (mt == 1) return launch_pro_one<F, LPR, 1, 1>(a, grp, pro, s);
+    if (mt == 2) return rpi == 2 ? launch_pro_one<F, LPR, 2, 2>(a, grp, pro, s) : launch_pro_one<F, LPR, 2, 1>(a, grp, pro, s);
+    /* tiles of four at most: eight tokens' rows beside the weights would not fit the registers.  Rows of 32 lanes, five 256-blocks and more, are past
+     * PRO_UNITS in such a tile whatever the grid */
+    if constexpr (LPR == 32) return CKQ_ENOGROUP;
+    else return rpi == 2 ? launch_pro_one<F, LPR, 4, 2>(a, grp, pro, s) : launch_pro_one<F, LPR, 4, 1>(a, grp, pro, s);
 }
+static_assert(PRO_UNITS < 4 * 5, "rows of 32 lanes and a tile of four tokens: launch_pro_lpr");
 template <class F>
 static int launch_pro(const GemvArgs &a, const GemvGroup &grp, const GemvPro &pro, hipStream_t s)
 {

@@ -1709,6 +1709,34 @@ def test_sequence_producer_joined_with_its_matmuls(fmt, M, D, N, step):
             assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("fmt,M,D,N", [("q4_k", 2, 1024, (8192, 64, 64)), ("q5_k", 4, 1024, (8000, 40, 40)), ("q6_k", 3, 768, (7990, 33, 5)), ("q4_k", 2, 512, (11000, 70, 9)),
+                                       ("q5_k", 3, 512, (11000, 70, 9)), ("q6_k", 2, 1280, (2800, 33, 16)), ("q5_k", 2, 2048, (3000, 500, 64)), ("q4_k", 2, 1024, (16384,))])
+def test_producer_joined_with_two_rows_a_slot(fmt, M, D, N):
+    """Wide matrices, narrow ones beside them, that take one launch with their producer at two rows a slot: it is taken, and every buffer has the
+    bits of the steps one by one."""
+    import torch
+    L = ckq.lib()
+    n, nb = len(N), D // 256
+    say("joined, two rows", fmt, M, D, N)
+    x = P.to_device(T.normal(M * D, 0.0, 1.0, 9910 + D))
+    gamma = P.to_device(T.normal(D, 1.0, 0.2, 9911))
+    Ws = [P.to_device(T.random_blocks(fmt, r * nb, 9912 + r)) for r in N]
+    bias = P.to_device(T.normal(N[0], 0.0, 0.5, 9913))
+
+    def buffers():
+        return [torch.full((M * nb * 292,), 77, dtype=torch.uint8, device="cuda")] + [torch.full((M, r), 7.0, device="cuda") for r in N]
+    one, two = buffers(), buffers()
+    P.check(L.ckq_rmsnorm_q8_k_fused_dev(P._dp(x), P._dp(gamma), P._dp(one[0]), M, D, D, 1e-5, P._stream()), "rmsnorm")
+    for i, r in enumerate(N):
+        P.check(L.ckq_gemm_nt_dev(P.FMT[fmt], P._dp(one[0]), P._dp(Ws[i]), P._dp(bias) if i == 0 else None, P._dp(one[1 + i]), M, r, D, r, P._stream()), "gemm")
+    ptrs = ctypes.c_void_p * n
+    rc = L.ckq_launch_gemv_pro(P.FMT[fmt], n, ptrs(*[y.data_ptr() for y in two[1:]]), ptrs(*[W.data_ptr() for W in Ws]), ptrs(bias.data_ptr(), *[None] * (n - 1)),
+                               (ctypes.c_int * n)(*N), (ctypes.c_long * n)(*N), D, M, P._dp(x), P._dp(gamma), ctypes.c_float(1e-5), ctypes.c_long(D), P._dp(two[0]), P._stream())
+    assert rc == 0
+    for a, b in zip(one, two):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("M,Ns,K", [(97, (22016,), 1024), (160, (16777,), 1024), (192, (11008,), 768), (512, (5120,), 1536), (481, (6100,), 1024), (300, (6701,), 2816),
                                     (90, (26000,), 1024), (225, (9728, 9728), 1536), (288, (4096, 1024, 1024, 3000), 1280), (512, (6400,), 512)])
 def test_gemm_q4_k_token_tile_choice(M, Ns, K):
