@@ -503,7 +503,8 @@ gemm_f32run_kernel(const float *__restrict__ A, const uint8_t *__restrict__ B, c
     auto load_w = [&](int j, int run) {
         u32 t[4];
         if constexpr (F::SHIFT) {
-            /* from the dword the block starts in; the last chunk from byte 196 of it, so that no load passes the dword the block ends in */
+            /* from the dword the block starts in; the last chunk from byte 196 of it, so that no load passes the dword the block ends in.  Of a
+             * matrix that begins or ends within a dword the two bytes beside it are read too (no allocation ends within a dword) and shifted away */
             ld16<4>(t, wbase - par + (((w_src(j, run) + par) & ~(size_t)3) + (u32)(w_chunk < 13 ? 16 * w_chunk : 196)));
         } else ld16<2>(t, wbase + (w_src(j, run) + min(16u * (u32)w_chunk, run_bytes(run) - 16u)));
         return ckq_v4i{(int)t[0], (int)t[1], (int)t[2], (int)t[3]};

@@ -214,7 +214,10 @@ int  ck_get_qk_k(void);
  * stream); work is enqueued, never synchronized.  Outputs must not overlap
  * inputs.  Return 0, or a negative CKQ_E* / positive hipError_t code.
  * Alignment: Q4_K/Q5_K weights and Q8_K activations 4 bytes, Q6_K/Q8_0 2
- * bytes, fp32 inputs of the quantizers 16 bytes, other fp32 4 bytes. */
+ * bytes, fp32 inputs of the quantizers 16 bytes, other fp32 4 bytes.  Q6_K
+ * weights that begin or end two bytes off a dword may be read in whole dwords:
+ * the two bytes that share the first or last dword with them are then read
+ * too, and not used. */
 
 int ckq_quantize_q8_k_dev(const float *x, void *y, int num_rows, int k, void *stream);
 int ckq_quantize_q8_0_dev(const float *x, void *y, int num_rows, int k, void *stream);

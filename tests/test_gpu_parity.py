@@ -1359,6 +1359,31 @@ def test_f32act_weights_by_runs(fmt, blocks, ofs):
         L.ckq_set_gemm_policy(0)
 
 
+@pytest.mark.parametrize("fmt,nb", [("q6_k", 1), ("q6_k", 9), ("q8_0", 5), ("q8_0", 67)])
+@pytest.mark.parametrize("ofs", [0, 2])
+def test_f32act_bytes_beside_the_weights(fmt, nb, ofs):
+    """A matrix of an odd number of blocks, on a dword or two bytes off, between bytes of zeros and between bytes of ones: one set of bits."""
+    import torch
+    L = ckq.lib()
+    L.ckq_set_gemm_policy(1)
+    try:
+        for M, N in ((33, 1), (200, 1793)):
+            K = nb * T.ELEMS[fmt]
+            W = T.random_blocks(fmt, N * nb, 60 + nb)
+            x_d = P.to_device(T.normal(M * K, 0.5, 1.0, seed=nb))
+            got = []
+            for fill in (0, 255):
+                buf = torch.full((W.size + ofs + 6,), fill, dtype=torch.uint8, device="cuda")
+                buf[ofs:ofs + W.size] = P.to_device(W)
+                c = torch.full((M, N), 7.0, dtype=torch.float32, device="cuda")
+                say("f32act neighbours", fmt, nb, M, N, ofs, fill)
+                P.check(L.ckq_gemm_nt_f32act_dev(P.FMT[fmt], P._dp(x_d), ctypes.c_void_p(buf.data_ptr() + ofs), None, P._dp(c), M, N, K, N, P._stream()), "f32act")
+                got.append(c)
+            assert torch.equal(*got)
+    finally:
+        L.ckq_set_gemm_policy(0)
+
+
 @pytest.mark.parametrize("fmt,widths", [("q6_k", (256, 512, 768, 1536, 1792, 2304)),
                                         ("q8_0", (32, 416, 512, 544, 1024, 1280, 1312, 1536, 1568, 2080, 2592))])
 def test_f32act_short_rows(fmt, widths):
