@@ -710,34 +710,34 @@ gemm_f32run_kernel(const float *__restrict__ A, const uint8_t *__restrict__ B, c
 template <class F>
 int launch_f32act(const float *A, const uint8_t *B, const float *bias, float *C, int M, int N, int K, long wrow, long ldc, hipStream_t s)
 {
-    const long long ntg = (M + 31) / 32;
-    /* two row tiles per wave share the cut of x; one where that would leave CUs without a block */
-    int R = ntg * ((N + 63) / 64) >= 192 ? 2 : 1;
+    const long long ntg = (M + 31) / 32, tiles = ntg * ((N + 31) / 32);
+    /* Two row tiles per wave share the cut of x.  A round of 256 blocks, one on a CU, then takes about half as long again, so they pay where they
+     * leave at most two thirds of the rounds.  Of 1585 launches of 2..256 tokens, 128..11008 rows and widths of 256..11008 the choice of all three
+     * formats, forms below included, costs 0.1 (Q4_K), 0.5 (Q6_K) and 1.2 % (Q8_0) more than always taking the fastest, single ones up to 28 %;
+     * from 192 blocks of two on, as it was, 2.0, 1.3 and 2.6 % and up to 48 (us, one tile -> two: Q4_K 31 x 8410 x 1280 15.0 -> 11.3, Q6_K 103 x 2275 x
+     * 3584 36.7 -> 27.9, Q8_0 204 x 1431 x 6080 49.9 -> 37.6). */
+    const long long rounds = (tiles + 255) / 256, rounds2 = (ntg * ((N + 63) / 64) + 255) / 256;
+    int R = 2 * rounds >= 3 * rounds2 ? 2 : 1;
     auto kernel = R == 2 ? gemm_f32row_kernel<F, 2> : gemm_f32row_kernel<F, 1>;
     if constexpr (!std::is_same<F, F32Q4K>::value) {
-        /* Same bits from all of them.  Measured over 7 grids of 63..1099 tiles of 32 rows, Q6_K at 16 and Q8_0 at 24 widths of 256..8192:
-         *  - up to SHORT_RUNS runs: weights loaded once a block, two blocks on a CU; Q6_K 1.02..1.31 times the row kernel (75 x 7670 x 1024
-         *    20.9 -> 16.0 us), Q8_0 1.03..1.18 where there is more than a block per CU.  A block alone on its CU gains nothing from the
-         *    second place and pays the way through LDS and the barrier: Q8_0 0.82..0.93, Q6_K 0.92..0.96 where a wave has but one step (512)
-         *    and 0.94..1.00 where two row tiles fill the CUs once (96 x 4096 x 1024 11.3 -> 11.7).
-         *  - longer: a wave whose share does not begin and end with a run loads runs that its neighbours load too, which the row kernel
-         *    does not: Q6_K 0.97..1.00 at one row tile and a second round of blocks, 1.02..1.26 otherwise; Q8_0 two bytes off a dword 0.94..0.99 up to
-         *    eight steps a wave (at one row tile up to nine), 1.11..1.19 beyond (6 to 64 tokens, widths 9184 and 10272).
-         *  - longer Q8_0 on a dword (runs of 128), whose rows a lane reads in whole dwords: 0.85..1.02 up to nine steps. From ten on it depends on
-         *    the tokens, since the run kernel's way is as long for one as for 32, and on the blocks: one row tile, 6 and 16 tokens 0.92..1.00; from 28
-         *    on 0.98..1.08 up to 129 blocks, 0.95..1.05 at 179 to 194, 0.90..0.95 at 258; two row tiles 1.03..1.05 (40 to 160 tokens).
-         *  - Q8_0 rows that are a multiple of 64 bytes apart: the row kernel's 64 rows fall on few cache sets; 1.00..1.29 (an odd multiple, 5120,
-         *    at 6 and 16 tokens 0.95..1.03). */
+        /* Same bits from all of them.
+         *  - `once`, rows of up to SHORT_RUNS runs: weights loaded once a block, two blocks on a CU.  Where there is more than a block per CU
+         *    1.02..1.31 (Q6_K, 75 x 7670 x 1024 20.9 -> 16.0 us) and 1.03..1.18 times (Q8_0) as fast as the row kernel; a block alone on its CU pays for
+         *    the way through LDS and the barrier: Q6_K gains from two steps a wave on, Q8_0 never.
+         *  - `runs`, weights in memory order.  Q6_K, whose row per lane is misaligned and takes the address path 160 cycles a load: always, as Q8_0 two bytes
+         *    off a dword from nine steps a wave on (1.11..1.19; below, a wave loads runs that its neighbours load too: 0.94..0.99).  Q8_0 on a dword, whose
+         *    rows a lane reads in whole dwords, gains where rows a multiple of 1024 elements apart fall on few cache sets (1.00..1.29), and else from ten
+         *    steps on if the tokens fill the tile, since the way is as long for one as for 32 (6 and 16 tokens 0.92..1.00, from 28 on
+         *    1.03..1.10), with two row tiles or not much more than half the CUs loading (179 to 194 blocks 0.95..1.05, 258 0.90..0.95). */
         const int per = ((K + F::STEP - 1) / F::STEP + F32_WAVES - 1) / F32_WAVES;
-        const bool filled = ntg * ((N + 32 * R - 1) / (32 * R)) > 256, fits = K <= F::SHORT_RUNS * F::RUN * F::STEP;
+        const bool fits = K <= F::SHORT_RUNS * F::RUN * F::STEP;
         bool once, runs;
         if constexpr (std::is_same<F, F32Q6K>::value) {
-            once = fits && (filled || (R == 1 && per > 1));
-            runs = !fits && !(R == 1 && filled && per % F::RUN);
+            once = fits && (tiles > 256 || per > 1);
+            runs = !fits;
         } else {
-            once = fits && filled;
-            runs = K % 2048 == 0 || (K % 64 ? per >= (R == 2 ? 9 : 10)
-                                            : M >= 28 && (K % 1024 == 0 || (per >= 10 && (R == 2 || ntg * ((N + 31) / 32) <= 160))));
+            once = fits && ntg * ((N + 32 * R - 1) / (32 * R)) > 256;
+            runs = K % 64 ? per >= 9 : K % 1024 == 0 || (M >= 28 && per >= 10 && (R == 2 || tiles <= 160));
         }
         if (once) {
             R = 1;

@@ -1359,6 +1359,28 @@ def test_f32act_weights_by_runs(fmt, blocks, ofs):
         L.ckq_set_gemm_policy(0)
 
 
+@pytest.mark.parametrize("fmt,M,N,K", [("q4_k", 5, 8250, 1280), ("q4_k", 97, 2090, 512), ("q4_k", 70, 5500, 768), ("q6_k", 5, 8250, 2304), ("q6_k", 97, 2090, 1792), ("q6_k", 40, 4128, 256),
+                                       ("q6_k", 70, 5500, 2048), ("q8_0", 5, 8250, 1408), ("q8_0", 40, 4128, 1024), ("q8_0", 97, 2090, 5120), ("q8_0", 33, 4128, 4672), ("q8_0", 70, 5500, 2080)])
+def test_f32act_row_tiles_by_rounds_of_blocks(fmt, M, N, K):
+    """Sizes on both sides of the choice between one and two row tiles a wave: the rows in one call have the bits of two calls of a part each,
+    which fill the chip less and choose otherwise."""
+    import torch
+    L = ckq.lib()
+    say("f32act row tiles", fmt, M, N, K)
+    x_d = P.to_device(T.normal(M * K, 0.5, 1.0, seed=K))
+    W = P.to_device(T.random_blocks(fmt, N * K // T.ELEMS[fmt], 70)).view(N, -1)
+
+    def run(w):
+        c = torch.full((M, w.shape[0]), 7.0, dtype=torch.float32, device="cuda")
+        P.check(L.ckq_gemm_nt_f32act_dev(P.FMT[fmt], P._dp(x_d), P._dp(w), None, P._dp(c), M, w.shape[0], K, w.shape[0], P._stream()), "f32act")
+        return c
+    try:
+        L.ckq_set_gemm_policy(1)
+        assert torch.equal(run(W), torch.cat([run(W[:1056].contiguous()), run(W[1056:].contiguous())], 1))
+    finally:
+        L.ckq_set_gemm_policy(0)
+
+
 @pytest.mark.parametrize("fmt,nb", [("q6_k", 1), ("q6_k", 9), ("q8_0", 5), ("q8_0", 67)])
 @pytest.mark.parametrize("ofs", [0, 2])
 def test_f32act_bytes_beside_the_weights(fmt, nb, ofs):
