@@ -47,9 +47,11 @@
  * loads a step, which loses in memory order (27.5 -> 29.3), and for the sizes named at the launcher.
  *
  * Grid: token groups fastest, so the blocks that share weights run side by side.
- * Bound: VALU issue: per 64 elements 220-260 operations to cut x, shared by the R row tiles, and per row tile some 210 / 230 / 130 for
- * Q4_K / Q6_K / Q8_0 to form the integers and apply the scales, half of them at half rate (conversions, byte permutes); the matrix
- * cores are busy a quarter of the time.  The centring of Q4_K is about 60 of them: 96 x 4096 x 4096 23 -> 27 us.
+ * Bound: VALU issue, on the CUs that have a block.  By the counters at 96 x 4096 x 4096 (two row tiles, 192 blocks) a wave issues 714 / 760 / 519 vector
+ * operations per 64 elements in Q4_K / Q6_K / Q8_0: 220-260 cut x, shared by the row tiles, some 60 turn weights and activations
+ * through LDS, and per row tile 210-230 / 230 / 110 form the integers and apply the scales, half of them at half rate (conversions, byte permutes).
+ * They issue in 78 / 72 / 56 % of the cycles; the matrix cores are busy in 23 / 18 / 20 %, LDS bank conflicts take 0 / 4 / 4 %.  The
+ * centring of Q4_K is about 60 of the operations: 96 x 4096 x 4096 23 -> 27 us.
  */
 #include "ckq_gemm_common.hpp"
 #include "ckq_gemm_f32act.hpp"

@@ -21,9 +21,10 @@
  * - The scales, as fp32, lie beside the rows as [block][row] and [block][token], so that a lane's four rows or tokens are one
  *   16-byte read.
  *
- * Tile = 32 TG tokens x 128 weight rows; the copies (a run of a row costs the address path its five cycles whatever the run's length), the
- * fp32 operations, the LDS reads and the matrix instructions of an iteration weigh about the same, so nothing is hidden to the
- * end and what counts is how many of each there are and whether a CU has another tile's to fill in:
+ * Tile = 32 TG tokens x 128 weight rows.  With two tiles on a CU vector instructions issue in 83 % of its cycles (2048 x 11008 x 4096, 96 tokens; matrix
+ * instructions 32 %, LDS bank conflicts 23 %); with one of two teams in 66 % (333 x 4864 x 4096; 23 and 22 %), with one of one team in 52.  What
+ * counts is how many operations, copies (a run of a row costs the address path its five cycles whatever the run's length) and LDS reads there are per product, and
+ * whether a CU has another tile's to fill in:
  * - 96 tokens save weights copied and read per product and, for some sizes, a round of tiles: 2048 x 11008 x 4096 (tokens,
  *   rows, K) 321 -> 290 us against 64 tokens, 464 x 37134 x 2048 161 -> 131, 512 x 9728 x 896 26.2 -> 22.6.
  * - 32 tokens do half the work where no more tokens are there: 32 x 37134 x 2048 33.8 -> 24.9.
