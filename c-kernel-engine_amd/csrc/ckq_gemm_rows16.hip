@@ -29,6 +29,7 @@
 #include "ckq_gemm_rows16.hpp"
 #include "ckq_gemm_q4k.hpp"
 #include <atomic>
+#include <type_traits>
 
 namespace {
 
@@ -399,6 +400,256 @@ gemm_rows16_kernel(const uint8_t *W, const uint8_t *X, int N, Rows16Shape S, flo
     }
 }
 
+/* Short rows, one group of tokens, many row tiles: the activations stay in registers.  Wave w of a block multiplies 256-block w of
+ * every row tile the block goes through (nb of them, at most HOLD_NB), so the activations of that block are fetched once, in the
+ * order of the instruction and never through LDS, and only weights stream: two blocks of a wave are on their way while one is worked on,
+ * across tiles too, and the waves of a block read its rows as they lie in memory.  The terms of a round of `round` tiles gather in
+ * LDS; then the waves meet at a barrier and four of them add up each tile.  The terms and their order are those of the kernel above.
+ * Bound: HBM, and the vector operations of all waves at once when a tile arrives (11008 x 4096 twice, Q4_K: loads alone 10.2 us,
+ * with the terms 14, with the sums and stores 16.8).  Against the kernel above, 13 tokens, weights from HBM (us): Q4_K 2 x 11008 x 4096
+ * 20.5 -> 16.8, Q6_K 32000 x 4096 35.4 -> 29.2, Q5_K 2 x 11008 x 4096 23.5 -> 21.5, 151936 x 1024 39 -> 31.
+ * A wave with a whole chain of blocks to itself, activations in LDS, was as fast on the first two (16.7, 29.2) and 26 on the third;
+ * two blocks a wave (eight waves, two such blocks a CU) 20.5, 36.2 and 25.6. */
+constexpr int HOLD_NB = 16;
+template <class F, bool TREE, bool GRP>
+__global__ void __launch_bounds__(64 * HOLD_NB)
+gemm_rows16_hold_kernel(const uint8_t *W, const uint8_t *X, int N, int M, int nb, int tiles, int round, float *y, const float *bias, long ldy, GemmChains ch, Rows16Args grp)
+{
+    constexpr int NT = 16;
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const int tid = threadIdx.x, nthr = blockDim.x, nwave = nthr >> 6;
+    const int lane = tid & 63, wave = wave_in_block();
+    const int i16 = lane & 15, q = lane >> 4;
+    const u32 xrow = (u32)nb * 292u, wpitch = (u32)nb * (u32)F::WBLOCK;
+    uint8_t *const wl = smem + wave * (16 * F::PITCH);                     /* this wave's weights */
+    float *const dxs = reinterpret_cast<float *>(smem + nwave * (16 * F::PITCH)), *const us = dxs + HOLD_NB * NT;
+    const uint8_t *const wrow = wl + i16 * F::PITCH;
+    struct Tile { const uint8_t *w; float *y; const float *bias; long ldy; int n0, N, own; GemmChains ch; };
+    auto tile_at = [&](int t) {
+        Tile r = {W, y, bias, ldy, t, N, 0, ch};
+        if constexpr (GRP) {
+            if (t >= grp.p[1].id0) {
+                Rows16Problem p = grp.p[1];
+                if (grp.n > 2 && t >= grp.p[2].id0) p = grp.p[2];
+                if (grp.n > 3 && t >= grp.p[3].id0) p = grp.p[3];
+                r = {p.W, p.y, p.bias, p.ldy, t - p.id0, p.N, 0, p.ch};
+            }
+        }
+        r.own = 16 * r.n0;
+        r.n0 = min(r.own, r.N - 16);                /* the last tile starts early rather than end late; its rows before `own` are another's */
+        r.w += (size_t)r.n0 * wpitch;
+        return r;
+    };
+
+    constexpr int NWL = (16 * F::CHUNKS + 63) / 64;
+    u32 wsrc[NWL];
+#pragma unroll
+    for (int j = 0; j < NWL; ++j) {
+        const int e = min(64 * j + lane, 16 * F::CHUNKS - 1);
+        wsrc[j] = (u32)(e / F::CHUNKS) * wpitch + F::chunk_ofs(e % F::CHUNKS);
+    }
+    auto fetch_w = [&](ckq_v4i (&v4)[NWL], int tile) {
+        const uint8_t *wb = tile_at(tile).w + (u32)wave * (u32)F::WBLOCK;
+#pragma unroll
+        for (int j = 0; j < NWL; ++j) {
+            u32 v[4];
+            ld16<F::WBLOCK % 4 == 0 ? 4 : 2>(v, wb + wsrc[j]);
+            v4[j] = ckq_v4i{(int)v[0], (int)v[1], (int)v[2], (int)v[3]};
+        }
+    };
+    auto take = [&](const ckq_v4i (&v4)[NWL]) {
+#pragma unroll
+        for (int j = 0; j < NWL; ++j) {
+            const int e = min(64 * j + lane, 16 * F::CHUNKS - 1);
+            *reinterpret_cast<ckq_v4i *>(wl + (e / F::CHUNKS) * F::PITCH + 16 * (e % F::CHUNKS)) = v4[j];
+        }
+    };
+    const u32 xlane = (u32)min(i16, M - 1) * xrow;
+    auto fetch_a = [&](ckq_v4i (&v4)[4], int2 &bs) {
+        const uint8_t *xb = X + (u32)wave * 292u;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            u32 v[4];
+            ld16<4>(v, xb + 4 + F::a_elem(g, 0) + (xlane + F::a_elem(0, q)));
+            v4[g] = ckq_v4i{(int)v[0], (int)v[1], (int)v[2], (int)v[3]};
+        }
+        if constexpr (F::MIN) {
+            u32 v[2];
+            ld8<4>(v, xb + 260 + (xlane + 8u * (u32)q));
+            bs = int2{(int)v[0], (int)v[1]};
+        }
+    };
+    auto bsum_operand = [&](const int2 &bs) {
+        const int p0 = (int)(int16_t)(bs.x & 0xffff) + (bs.x >> 16), p1 = (int)(int16_t)(bs.y & 0xffff) + (bs.y >> 16);
+        return int2{(int)bf16_pair((float)(p0 & 63), (float)(p1 & 63)), (int)bf16_pair((float)(64 * (p0 >> 6)), (float)(64 * (p1 >> 6)))};
+    };
+    auto min_mfma = [&](const int2 &am, const ckq_v4i &mins) {
+        const ckq_v4f z = {0.0f, 0.0f, 0.0f, 0.0f};
+        const ckq_v4i a = {am.x, am.y, 0, 0};
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(ckq_v8bf, a), __builtin_bit_cast(ckq_v8bf, mins), z, 0, 0, 0);
+    };
+    const ckq_v4i zero = {0, 0, 0, 0};
+    ckq_v4i a[4];                                  /* the activations of this wave's block, in the order of the instruction */
+    int2 am = {};
+    /* the terms of the block whose weights lie in wl */
+    auto terms = [&](float *u) {
+        Head hd;
+        F::head(hd, wrow, q);
+        float out[4];
+        if constexpr (TREE) {
+            const ckq_v4i dxi = lds16(reinterpret_cast<const uint8_t *>(dxs + wave * NT + 4 * q));
+            float acc[4][4];
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[g][r] = 0.0f;
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                ckq_v4i ph, pl;
+                F::planes(ph, pl, hd, wrow, g, q);
+                const ckq_v4i sh = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[g], ph, zero, 0, 0, 0);
+                const ckq_v4i sl = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[g], pl, zero, 0, 0, 0);
+                ckq_v4f i2;
+                if constexpr (F::MIN) i2 = min_mfma(am, q == g ? hd.mins : zero);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int di = dxi[r];
+                    const float dx = __builtin_bit_cast(float, di), f = (float)((sh[r] << F::SHIFT) + sl[r]);
+                    float v;
+                    if constexpr (F::MIN) v = (hd.dw * dx) * f - (hd.dmin * dx) * i2[r];
+                    else                  v = (hd.dw * dx) * f;
+                    asm volatile("" : "+v"(v));                  /* rounded before it is added, as there */
+                    acc[g][r] += v;
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) out[r] = (acc[0][r] + acc[1][r]) + (acc[2][r] + acc[3][r]);
+        } else {
+            ckq_v4i sh, sl;
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                ckq_v4i ph, pl;
+                F::planes(ph, pl, hd, wrow, g, q);
+                sh = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[g], ph, g ? sh : zero, 0, 0, 0);
+                sl = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[g], pl, g ? sl : zero, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if constexpr (F::MIN) {
+                const ckq_v4f i2 = min_mfma(am, hd.mins);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float f = (float)((sh[r] << F::SHIFT) + sl[r]);
+                    out[r] = hd.dw * f - hd.dmin * i2[r];
+                }
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) out[r] = hd.dw * (float)((sh[r] << F::SHIFT) + sl[r]);
+            }
+        }
+        *reinterpret_cast<float4 *>(u + wave * (NT * 16) + 4 * lane) = float4{out[0], out[1], out[2], out[3]};
+    };
+    /* the outputs of the tile whose terms lie at u: e is output e % 4 of lane e / 4 */
+    auto finish = [&](const float *u, int tile, int first, int step) {
+        const Tile tl = tile_at(tile);
+        for (int e = first; e < NT * 16; e += step) {
+            const int tok = 4 * (e >> 6) + (e & 3), n = tl.n0 + ((e >> 2) & 15);
+            const float *ue = u + e;
+            float v = 0.0f;
+            if constexpr (TREE) {
+                float x[16];
+#pragma unroll
+                for (int b = 0; b < 16; ++b) x[b] = b < nb ? ue[b * (NT * 16)] : 0.0f;
+#pragma unroll
+                for (int w = 1; w < 16; w *= 2)
+#pragma unroll
+                    for (int b = 0; b < 16; b += 2 * w) x[b] += x[b + w];
+                v = x[0];
+            } else {
+                const float *dx = dxs + tok;
+                for (int sp = 0; sp < tl.ch.splits; ++sp) {
+                    const int b0 = sp * tl.ch.per, b1 = min(nb, b0 + tl.ch.per);
+                    float c0 = 0.0f, c1 = 0.0f;
+                    int b = b0;
+                    for (; b + 8 <= b1; b += 8) {
+                        float uu[8], dd[8];
+#pragma unroll
+                        for (int k = 0; k < 8; ++k) { uu[k] = ue[(b + k) * (NT * 16)]; dd[k] = dx[(b + k) * NT]; }
+                        if (tl.ch.kg == 2) {
+#pragma unroll
+                            for (int k = 0; k < 8; k += 2) { c0 = fmaf(dd[k], uu[k], c0); c1 = fmaf(dd[k + 1], uu[k + 1], c1); }
+                        } else {
+#pragma unroll
+                            for (int k = 0; k < 8; ++k) c0 = fmaf(dd[k], uu[k], c0);
+                        }
+                    }
+                    for (; b < b1; ++b) {
+                        const float uu = ue[b * (NT * 16)], dd = dx[b * NT];
+                        if (tl.ch.kg == 2 && ((b - b0) & 1)) c1 = fmaf(dd, uu, c1);
+                        else                                 c0 = fmaf(dd, uu, c0);
+                    }
+                    if (tl.ch.kg == 2) c0 += c1;
+                    v = sp ? v + c0 : c0;
+                }
+            }
+            if (tl.bias) v += tl.bias[n];          /* no load without a bias: waiting for it would wait for the stores before it */
+            if (n >= tl.own && tok < M) tl.y[(size_t)tok * tl.ldy + n] = v;
+        }
+    };
+
+    /* the tokens' block scales, [block][token]: the first loads go out before all others, so that waiting for them waits for nothing else */
+    auto load_dx = [&](int e) {
+        return __builtin_bit_cast(float, ld4<4>(X + (size_t)((u32)min(e & 15, M - 1) * xrow + (u32)(e >> 4) * 292u)));
+    };
+    const int ndx = nb * NT, tstep = (int)gridDim.x, tile0 = (int)blockIdx.x, mine = (tiles - tile0 + tstep - 1) / tstep;
+    const float dx0 = load_dx(min(tid, ndx - 1));
+
+    constexpr int D = 2;                           /* blocks of a wave on their way; with three 29.5 -> 31.8 us for the 32000 x 4096 above */
+    ckq_v4i w[D][NWL];
+    int left = mine, ft = tile0;                   /* tiles still to do; the next to fetch */
+    auto fetch = [&](int r) {
+        fetch_w(w[r], ft);
+        ft += tstep;
+    };
+    fetch(0);
+#pragma unroll
+    for (int r = 1; r < D; ++r)
+        if (left > r) fetch(r);
+    fetch_a(a, am);
+    if (tid < ndx) dxs[tid] = dx0;
+    for (int e = tid + nthr; e < ndx; e += nthr) dxs[e] = load_dx(e);
+    if (F::MIN) am = bsum_operand(am);
+    if constexpr (TREE) __syncthreads();
+    const int teams = max(nwave >> 2, 1), team = nwave >= 4 ? wave >> 2 : 0, usize = nb * (NT * 16);
+    int i = 0, t = tile0;                          /* tiles of this round that are done; the current tile */
+    auto step = [&](int r, auto more) {
+        take(w[r]);
+        if (more) fetch(r);
+        __builtin_amdgcn_sched_barrier(0);
+        terms(us + i * usize);
+        __builtin_amdgcn_sched_barrier(0);
+        ++i;
+        const bool last = t + tstep >= tiles;
+        if (i == round || last) {
+            __syncthreads();
+            if (team < teams)
+                for (int j = team; j < i; j += teams) finish(us + j * usize, t - (i - 1 - j) * tstep, nwave >= 4 ? tid & 255 : tid, nwave >= 4 ? 256 : nthr);
+            if (!last) __syncthreads();
+            i = 0;
+        }
+        t += tstep;
+    };
+    for (; left >= 2 * D; left -= D) {
+#pragma unroll
+        for (int r = 0; r < D; ++r) step(r, std::true_type{});
+    }
+    for (; left > 0; left -= D) {
+#pragma unroll
+        for (int r = 0; r < D; ++r)
+            if (left > r) step(r, left > r + D);
+    }
+}
+
 /* Short rows, several token groups: a block has a wave for every 256-block of its 16 rows (at most KEEP_NB of them) and goes
  * through `per` groups of 16 tokens, the planes and scales of its weights formed once and kept in registers.  The kernel above
  * forms them again for every group, and they are a good third of what bounds it there, VALU issue (Q5_K, 93 tokens: 480 vector
@@ -675,6 +926,62 @@ int launch_rows16_keep(Rows16Args &a, int parts, hipStream_t s)
     return (int)hipGetLastError();
 }
 
+/* Blocks of a launch of the kernel that holds its activations, and their tiles a round; false: another kernel.  `tree` has four times the fp32 terms
+ * and gains less.  Fitted to 200 launches of both kernels, 5 to 16 tokens, 1024 x 256 to 150000 x 1024 (time of the kernel above over this one's): up to
+ * four 256-blocks a row and eight, which fill the 16 waves of a CU, 1.0-2.0 at any size (Q4_K 3328 x 1024 4.8 -> 4.1, Q6_K 79808 x 256 15.4 -> 8.3,
+ * 39872 x 2048 23.8 -> 20.3), one or two blocks below a quarter of a round 0.95-1.0; five to seven 0.74-1.1 (they leave waves of the CU
+ * idle); above eight from 1.7 rounds of the CUs on with the tile kernels' sums 1.0-1.47 where 14 to 16 waves are at work, from 4 on 1.04-1.26 with fewer;
+ * with the streaming kernel's from 5 and 8, 0.99-1.09 (below: 0.88-1.03). */
+template <class F>
+bool rows16_hold(const Rows16Args &a, bool tree, int tiles, int *grid, int *round, size_t *lds)
+{
+    if (a.nb > HOLD_NB || a.M > 16) return false;
+    for (int i = 0; i < a.n; ++i)
+        if (a.p[i].X != a.p[0].X || a.p[i].N < 16) return false;
+    const int occ = HOLD_NB / a.nb;                /* blocks on a CU */
+    const float rounds = (float)tiles / (float)(256 * occ);
+    float least = 0.0f;
+    if (a.nb <= 2) least = 0.25f;
+    else if (a.nb > 8) least = a.nb >= 14 ? (tree ? 5.0f : 1.7f) : (tree ? 8.0f : 4.0f);
+    else if (a.nb > 4 && a.nb < 8) return false;
+    if (rounds < least) return false;
+    const size_t tile = (size_t)a.nb * 1024, fixed = (size_t)a.nb * (16 * F::PITCH) + HOLD_NB * 64;
+    *grid = tiles < 256 * occ ? tiles : 256 * occ;
+    const int most = (tiles + *grid - 1) / *grid, fit = (int)((160 * 1024 / occ - fixed) / tile), turns = (most + fit - 1) / fit;
+    *round = (most + turns - 1) / turns;
+    *lds = fixed + *round * tile;
+    return true;
+}
+
+template <class F, bool TREE>
+int launch_rows16_hold(Rows16Args &a, int tiles, int grid, int round, size_t lds, hipStream_t s)
+{
+    int id = 0;
+    for (int i = 0; i < a.n; ++i) {
+        a.p[i].id0 = id;
+        id += (a.p[i].N + 15) / 16;
+    }
+    if (lds > 64 * 1024) {
+        static std::atomic<uint64_t> done[2];      /* as in launch_rows16_nt */
+        int dev = 0;
+        hipError_t e = hipGetDevice(&dev);
+        if (e != hipSuccess) return (int)e;
+        const uint64_t bit = 1ull << (dev & 63);
+        if (!(done[a.n > 1].load(std::memory_order_acquire) & bit)) {
+            e = hipFuncSetAttribute(a.n > 1 ? (const void *)gemm_rows16_hold_kernel<F, TREE, true> : (const void *)gemm_rows16_hold_kernel<F, TREE, false>,
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+            if (e != hipSuccess) return (int)e;
+            done[a.n > 1].fetch_or(bit, std::memory_order_release);
+        }
+    }
+    const Rows16Problem &p = a.p[0];
+    if (a.n > 1)
+        hipLaunchKernelGGL((gemm_rows16_hold_kernel<F, TREE, true>), dim3((unsigned)grid), dim3((unsigned)(64 * a.nb)), lds, s, p.W, p.X, p.N, a.M, a.nb, tiles, round, p.y, p.bias, p.ldy, p.ch, a);
+    else
+        hipLaunchKernelGGL((gemm_rows16_hold_kernel<F, TREE, false>), dim3((unsigned)grid), dim3((unsigned)(64 * a.nb)), lds, s, p.W, p.X, p.N, a.M, a.nb, tiles, round, p.y, p.bias, p.ldy, p.ch, a);
+    return (int)hipGetLastError();
+}
+
 template <class F>
 int launch_rows16(int fmt, Rows16Args &a, hipStream_t s)
 {
@@ -682,6 +989,10 @@ int launch_rows16(int fmt, Rows16Args &a, hipStream_t s)
     for (int i = 0; i < a.n; ++i) tiles += (a.p[i].N + 15) / 16;
     const int parts = rows16_keep_parts(fmt, tiles, (a.M + 15) / 16, a.nb, nullptr);
     if (parts) return a.tree ? launch_rows16_keep<F, true>(a, parts, s) : launch_rows16_keep<F, false>(a, parts, s);
+    int grid, round;
+    size_t lds;
+    if (tiles < 1 << 20 && rows16_hold<F>(a, a.tree, (int)tiles, &grid, &round, &lds))
+        return a.tree ? launch_rows16_hold<F, true>(a, (int)tiles, grid, round, lds, s) : launch_rows16_hold<F, false>(a, (int)tiles, grid, round, lds, s);
     if (a.tree) return a.M <= 8 ? launch_rows16_nt<F, 8, true>(a, s) : launch_rows16_nt<F, 16, true>(a, s);
     return launch_rows16_nt<F, 16, false>(a, s);           /* the tile kernels start above eight tokens */
 }

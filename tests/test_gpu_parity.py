@@ -1634,6 +1634,55 @@ def test_16_row_tiles_of_short_rows_and_several_token_groups(fmt):
         L.ckq_set_prefill_variant(tag, 0)
 
 
+@pytest.mark.parametrize("fmt", ["q4_k", "q5_k", "q6_k"])
+def test_16_row_tiles_with_held_activations(fmt):
+    """The kernel that goes through several row tiles with its activations in registers: one wave a block and sixteen, blocks of one
+    tile, of some more than others and of several rounds of the tiles whose terms fit the LDS, last tiles that start early (row counts
+    past a multiple of 16), a bias and a padded C, one token short of the group and all sixteen.  In the order of the tile
+    kernels (policy 1) bit for bit what they give, in that of the streaming kernel (2) what one token at a time gives; and several matrices in one launch."""
+    import torch
+    L = ckq.lib()
+    tag = P.FMT[fmt]
+
+    def forced(policy, call):
+        L.ckq_set_prefill_variant(tag, 16)
+        L.ckq_set_gemm_policy(policy)
+        try:
+            return call()
+        finally:
+            L.ckq_set_prefill_variant(tag, 0)
+            L.ckq_set_gemm_policy(0)
+    for M, N, K in [(3, 16, 1024), (16, 4111, 1024), (15, 17, 768), (9, 140001, 256), (16, 33000, 512), (13, 130017, 768), (16, 40007, 1024), (12, 12303, 2048),
+                    (16, 16401, 3072), (11, 9001, 3584), (16, 7003, 4096), (8, 21001, 4096)]:
+        xq = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, seed=M)), "q8_k", rows=M)
+        W, bias = P.to_device(T.random_blocks(fmt, N * K // 256, 9600 + M)), P.to_device(T.normal(N, 0.0, 0.5, seed=N))
+        say("16-row tiles, held activations", fmt, M, N, K)
+        c = torch.full((M, N + 5), 7.0, dtype=torch.float32, device="cuda")
+        forced(2, lambda: P.check(L.ckq_gemm_nt_dev(tag, P._dp(xq), P._dp(W), P._dp(bias), P._dp(c), M, N, K, N + 5, P._stream()), "ckq_gemm_nt_dev"))
+        assert bool((c[:, N:] == 7.0).all()), (M, N, K)
+        rb = xq.numel() // M
+        for m in range(0, M, 3):
+            one = P.dev_gemm_nt(fmt, xq[m * rb:(m + 1) * rb].clone(), W, bias, 1, N, K)
+            assert torch.equal(c[m, :N], one.view(N)), (M, N, K, m)
+        if M > 8:
+            chain = forced(1, lambda: P.dev_gemm_nt(fmt, xq, W, bias, M, N, K).clone())
+            L.ckq_set_gemm_policy(1)
+            try:
+                tiles = P.dev_gemm_nt(fmt, xq, W, bias, M, N, K)
+            finally:
+                L.ckq_set_gemm_policy(0)
+            assert torch.equal(chain, tiles), (M, N, K)
+    for M, K, Ns in ((13, 1024, [9000, 33, 4861, 250]), (16, 4096, [5000, 3003])):
+        xq = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, seed=5)), "q8_k", rows=M)
+        Ws = [P.to_device(T.random_blocks(fmt, n * K // 256, 9650 + i)) for i, n in enumerate(Ns)]
+        for policy in (2, 1, 0):
+            ys = [torch.zeros(M, n, dtype=torch.float32, device="cuda") for n in Ns]
+            say("16-row tiles, held activations, grouped", fmt, M, policy)
+            forced(policy, lambda: P.dev_matmul_sequence([(fmt, xq, W, None, y, M, n, K) for W, y, n in zip(Ws, ys, Ns)]))
+            for W, y, n in zip(Ws, ys, Ns):
+                assert torch.allclose(y, P.dev_gemm_nt(fmt, xq, W, None, M, n, K).view(M, n), rtol=0, atol=2e-6 * float(y.abs().max())), (policy, n)
+
+
 @pytest.mark.parametrize("blocks", [1, 2, 3, 4, 5, 6, 7, 8, 13, 37, 64])
 def test_gemm_mfma_q8_0_row_alignment_and_k_remainders(blocks):
     """Rows of odd and even numbers of 32-blocks (odd ones start on dwords every other row), K ending after one, two, three
