@@ -111,6 +111,33 @@ __device__ __forceinline__ int rne_sat_i8(float p)
     return (int)fminf(fmaxf(r, -128.0f), 127.0f);
 }
 
+/* q = RNE(e * scale) as rne_sat_i8 has it, four to a dword.  Adding 1.5 * 2^23 rounds to the nearest even integer and leaves it in the
+ * low bits: a multiplication and an addition a value, and its byte as it is needed, where rne_sat_i8 takes six operations.  That holds
+ * for |e * scale| <= 127.x, which is every value unless the block's scale or the value is infinite or NaN; then a result has an
+ * exponent other than that of 2^23, and the wave goes through rne_sat_i8. */
+template <int N>
+__device__ __forceinline__ void q8_round(const float (&e)[N], float scale, u32 (&packed)[N / 4])
+{
+#pragma clang fp contract(off)
+    u32 b[N], any = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const float p = e[i] * scale;
+        b[i] = __builtin_bit_cast(u32, p + 12582912.0f);
+        any |= b[i];
+    }
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64((any & 0xB4800000u) != 0) != 0, 0)) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const float p = e[i] * scale;
+            b[i] = (u32)rne_sat_i8(p);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < N / 4; ++k)
+        packed[k] = __builtin_amdgcn_perm(b[4 * k + 1], b[4 * k], 0x0c0c0400u) | __builtin_amdgcn_perm(b[4 * k + 3], b[4 * k + 2], 0x04000c0cu);
+}
+
 /* One wave turns 256 fp32 values (lane l holds elements 4l..4l+3 in e) into
  * the 292-byte Q8_K block at `out` (global or LDS), with the reference's rules
  * (quantize_row_q8_k_sse.c:22-82): the scale comes from the FIRST element of
@@ -135,14 +162,10 @@ __device__ __forceinline__ void q8k_quantize_block(const float (&e)[4], int lane
         return;
     }
     const float iscale = -127.0f / smax;
-    int q[4], s = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        q[i] = rne_sat_i8(__fmul_rn(e[i], iscale));
-        s += q[i];
-    }
-    const u32 packed = (u32)(q[0] & 0xff) | ((u32)(q[1] & 0xff) << 8) | ((u32)(q[2] & 0xff) << 16) | ((u32)(q[3] & 0xff) << 24);
-    reinterpret_cast<u32 *>(out + 4)[lane] = packed;
+    u32 packed[1];
+    q8_round(e, iscale, packed);
+    int s = dot4((int)packed[0], 0x01010101, 0);
+    reinterpret_cast<u32 *>(out + 4)[lane] = packed[0];
     s = group_sum<4>(s);                       /* 16 consecutive elements = 4 lanes */
     /* two sums a store, so that the block leaves in whole dwords: the host looks for them one by one (ckq_host.c) */
     const u32 pair = ((u32)dpp_get<0x114>(s) & 0xffffu) | ((u32)s << 16);                /* row_shr:4 */

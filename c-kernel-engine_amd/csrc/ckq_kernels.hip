@@ -237,10 +237,8 @@ int gemm_launch_reduce(float *C, long ldc, const float *part, const float *bias,
 
 /* Q5_0 block -> Q8_0 block: the scale is kept, the 32 values become int8
  * q - 16.  One thread per block. */
-__global__ void __launch_bounds__(256) q5_0_to_q8_0_kernel(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, size_t nblocks)
+__device__ __forceinline__ void q5_0_to_q8_0_block(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, size_t i)
 {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= nblocks) return;
     FmtQ50::Wt w;
     FmtQ50::Off o;
     o.blk = 0;
@@ -254,6 +252,11 @@ __global__ void __launch_bounds__(256) q5_0_to_q8_0_kernel(const uint8_t *__rest
         reinterpret_cast<uint16_t *>(out + 2)[2 * k] = (uint16_t)((u32)d.q[k] & 0xffffu);
         reinterpret_cast<uint16_t *>(out + 2)[2 * k + 1] = (uint16_t)((u32)d.q[k] >> 16);
     }
+}
+__global__ void __launch_bounds__(256) q5_0_to_q8_0_kernel(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, size_t nblocks)
+{
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < nblocks) q5_0_to_q8_0_block(src, dst, i);
 }
 
 static int launch_gemm_q50_via_q80(const void *A, const void *B, const float *bias, float *C,
@@ -760,14 +763,25 @@ extern "C" int ckq_launch_gemm_block_sums(int fmt, const void *A, const void *B,
 /* fp32 -> Q8_K, one wave per 256-element block, lane l owns elements 4l..4l+3
  * (q8k_quantize_block holds the reference's rules).  SWIGLU: the quantizer's
  * input is SiLU(x) * up instead of x.  Rows of the input are ldx floats apart,
- * bpr blocks of 256 per row. */
+ * bpr blocks of 256 per row.  Bound: memory once rows are many (us, inputs not in the L2: 2048 x 4096 11.1 -> 9.7, SwiGLU 512 x 4864 8.0 -> 7.4,
+ * 512 x 11008 13.3 -> 12.2, 2048 x 11008 47.0 -> 43.7 = 4.8 TB/s, when a value's rounding went from six operations to two and
+ * block numbers from 64 bits to 32: 219 -> 93 and 366 -> 243 vector instructions), launch and latency below.  Four blocks a wave, sixteen lanes
+ * each, their divisions and maxima shared: 9.8, 7.2, 12.7, 40.6, and 3.2 -> 3.7 for SwiGLU 93 x 4864. */
 template <bool SWIGLU>
 __global__ void __launch_bounds__(256) quantize_q8_k_kernel(const float *__restrict__ x, const float *__restrict__ up,
-                                                            uint8_t *__restrict__ y, long nblocks, int bpr, long ldx)
+                                                            uint8_t *__restrict__ y, u32 nblocks, u32 bpr, long ldx)
 {
-    const long blk = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const u32 blk = blockIdx.x * 4 + (u32)wave_in_block();
     if (blk >= nblocks) return;
     pro_quantize_block<SWIGLU>(x, up, y, blk, bpr, ldx, threadIdx.x & 63);
+}
+
+template <bool SWIGLU>
+static int launch_quantize_q8_k(const float *x, const float *up, void *y, long nblocks, int bpr, long ldx, hipStream_t s)
+{
+    if (nblocks > 0x7fffffffl) return CKQ_ESHAPE;
+    hipLaunchKernelGGL(quantize_q8_k_kernel<SWIGLU>, dim3((unsigned)((nblocks + 3) / 4)), dim3(256), 0, s, x, up, (uint8_t *)y, (u32)nblocks, (u32)bpr, ldx);
+    return (int)hipGetLastError();
 }
 
 /*
@@ -775,10 +789,9 @@ __global__ void __launch_bounds__(256) quantize_q8_k_kernel(const float *__restr
  * gemm_kernels_q8_0.c:70-146).  d = amax/127 stored as fp16 (RNE);
  * id = amax ? 127/amax : 0; q = RNE(x*id) saturated.
  */
-__global__ void __launch_bounds__(256) quantize_q8_0_kernel(const float *__restrict__ x, uint8_t *__restrict__ y,
-                                                            long nblocks)
+__device__ __forceinline__ void quantize_q8_0_blocks(const float *__restrict__ x, uint8_t *__restrict__ y, long nblocks, u32 block)
 {
-    const long t = (long)blockIdx.x * 256 + threadIdx.x;
+    const long t = (long)block * 256 + threadIdx.x;
     const long blk = t >> 3;
     const int  j = (int)(t & 7);
     const bool live = blk < nblocks;
@@ -786,19 +799,24 @@ __global__ void __launch_bounds__(256) quantize_q8_0_kernel(const float *__restr
     const float4 v = reinterpret_cast<const float4 *>(x + b * 32)[j];
     const float e[4] = {v.x, v.y, v.z, v.w};
     float amax = fmaxf(fmaxf(fabsf(e[0]), fabsf(e[1])), fmaxf(fabsf(e[2]), fabsf(e[3])));
-#pragma unroll
-    for (int off = 1; off < 8; off <<= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+    amax = fmaxf(amax, dpp_get<0xB1>(amax));                 /* eight lanes: quad_perm twice, row_half_mirror */
+    amax = fmaxf(amax, dpp_get<0x4E>(amax));
+    amax = fmaxf(amax, dpp_get<0x141>(amax));
     const float d  = amax / 127.0f;
     const float id = amax != 0.0f ? 127.0f / amax : 0.0f;
-    int q[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) q[i] = rne_sat_i8(__fmul_rn(e[i], id));
+    u32 packed[1];
+    q8_round(e, id, packed);
     if (!live) return;
     uint8_t *out = y + b * 34;
     uint16_t *o16 = reinterpret_cast<uint16_t *>(out + 2 + 4 * j);   /* 2-byte aligned */
-    o16[0] = (uint16_t)((q[0] & 0xff) | ((q[1] & 0xff) << 8));
-    o16[1] = (uint16_t)((q[2] & 0xff) | ((q[3] & 0xff) << 8));
+    o16[0] = (uint16_t)packed[0];
+    o16[1] = (uint16_t)(packed[0] >> 16);
     if (j == 0) *reinterpret_cast<uint16_t *>(out) = __builtin_bit_cast(uint16_t, (_Float16)d);
+}
+
+__global__ void __launch_bounds__(256) quantize_q8_0_kernel(const float *__restrict__ x, uint8_t *__restrict__ y, long nblocks)
+{
+    quantize_q8_0_blocks(x, y, nblocks, blockIdx.x);
 }
 
 extern "C" int ckq_launch_quantize_q8_k(const float *x, void *y, int rows, int k, void *stream)
@@ -806,9 +824,7 @@ extern "C" int ckq_launch_quantize_q8_k(const float *x, void *y, int rows, int k
     if (!x || !y || rows <= 0 || k <= 0) return CKQ_EINVAL;
     if (k % 256) return CKQ_ESHAPE;
     const long nblocks = (long)rows * (k / 256);
-    hipLaunchKernelGGL(quantize_q8_k_kernel<false>, dim3((unsigned)((nblocks + 3) / 4)), dim3(256), 0, (hipStream_t)stream,
-                       x, (const float *)nullptr, (uint8_t *)y, nblocks, k / 256, (long)k);
-    return (int)hipGetLastError();
+    return launch_quantize_q8_k<false>(x, nullptr, y, nblocks, k / 256, (long)k, (hipStream_t)stream);
 }
 
 /* y[row] = Q8_K(SiLU(gate[row]) * up[row]), rows of gate and up ld floats apart. */
@@ -817,9 +833,7 @@ extern "C" int ckq_launch_swiglu_q8_k(const float *gate, const float *up, void *
     if (!gate || !up || !y || rows <= 0 || k <= 0 || ld < k) return CKQ_EINVAL;
     if (k % 256 || ld % 4 || ((uintptr_t)gate | (uintptr_t)up) % 16) return CKQ_ESHAPE;
     const long nblocks = (long)rows * (k / 256);
-    hipLaunchKernelGGL(quantize_q8_k_kernel<true>, dim3((unsigned)((nblocks + 3) / 4)), dim3(256), 0, (hipStream_t)stream,
-                       gate, up, (uint8_t *)y, nblocks, k / 256, ld);
-    return (int)hipGetLastError();
+    return launch_quantize_q8_k<true>(gate, up, y, nblocks, k / 256, ld, (hipStream_t)stream);
 }
 
 extern "C" int ckq_launch_quantize_q8_0(const float *x, void *y, int rows, int k, void *stream)

@@ -18,13 +18,13 @@ __device__ __forceinline__ float swiglu_value(float g, float u)
     return s * u;
 }
 
-/* One wave: 256-block `blk` (of bpr per row, rows ldx floats apart) of x, or of
- * SiLU(x) * up, -> the Q8_K block at y + blk * 292. */
+/* One wave: 256-block `blk` (of bpr per row, rows ldx floats apart) of x, or of SiLU(x) * up, -> the Q8_K block at y + blk * 292.
+ * Without SWIGLU rows lie end to end.  Block numbers have 32 bits (2 TB of input): the division by bpr in 64 was a fifth of the kernel's instructions. */
 template <bool SWIGLU>
 __device__ __forceinline__ void pro_quantize_block(const float *__restrict__ x, const float *__restrict__ up,
-                                                   uint8_t *__restrict__ y, long blk, int bpr, long ldx, int lane)
+                                                   uint8_t *__restrict__ y, u32 blk, u32 bpr, long ldx, int lane)
 {
-    const long src = (blk / bpr) * ldx + (blk % bpr) * 256;
+    const size_t src = SWIGLU ? (size_t)(blk / bpr) * ldx + (blk % bpr) * 256u : (size_t)blk * 256u;
     const float4 v = reinterpret_cast<const float4 *>(x + src)[lane];
     float e[4] = {v.x, v.y, v.z, v.w};
     if constexpr (SWIGLU) {
@@ -32,7 +32,7 @@ __device__ __forceinline__ void pro_quantize_block(const float *__restrict__ x, 
         e[0] = swiglu_value(e[0], w.x); e[1] = swiglu_value(e[1], w.y);
         e[2] = swiglu_value(e[2], w.z); e[3] = swiglu_value(e[3], w.w);
     }
-    q8k_quantize_block(e, lane, y + blk * 292);
+    q8k_quantize_block(e, lane, y + (size_t)blk * 292);
 }
 
 /* ---- RMSNorm -> Q8_K (reference: src/kernels/fused/rmsnorm_q8_k_fused.c:54-142
@@ -115,14 +115,10 @@ __device__ __forceinline__ void rms_quant_block(const float4 xv, const float4 gv
         return;
     }
     const float iscale = __fdiv_rn(-127.0f, amax);
-    int q[4], sum = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        q[i] = rne_sat_i8(__fmul_rn(e[i], iscale));
-        sum += q[i];
-    }
-    reinterpret_cast<u32 *>(out + 4)[lane] =
-        (u32)(q[0] & 0xff) | ((u32)(q[1] & 0xff) << 8) | ((u32)(q[2] & 0xff) << 16) | ((u32)(q[3] & 0xff) << 24);
+    u32 packed[1];
+    q8_round(e, iscale, packed);
+    int sum = dot4((int)packed[0], 0x01010101, 0);
+    reinterpret_cast<u32 *>(out + 4)[lane] = packed[0];
     sum = group_sum<4>(sum);
     if ((lane & 3) == 3) reinterpret_cast<int16_t *>(out + 260)[lane >> 2] = (int16_t)sum;
     if (lane == 0) *reinterpret_cast<float *>(out) = __fdiv_rn(1.0f, iscale);

@@ -103,6 +103,30 @@ def test_quantize_bit_exact_vs_oracle_large(std, seed):
         assert np.array_equal(got, want), fmt
 
 
+@pytest.mark.parametrize("fmt", ["q8_k", "q8_0"])
+def test_quantizers_round_blocks_of_one_wave_the_short_and_the_long_way(fmt):
+    """Blocks whose values round by one addition beside blocks that need the saturating conversion: values half way between two
+    quants (the largest 127 makes the scale 1), an infinity, a block whose inverse scale is infinite, the smallest whose
+    is not, the largest finite values, and (Q8_K, whose rule for them is the order of comparisons) NaNs, alone and beside zeros only."""
+    k = 4096
+    x = T.normal(64 * k, 0.0, 1.0, seed=77).reshape(-1, 256)
+    x[1] = np.arange(256) % 127 + 0.5
+    x[1, ::2] *= -1
+    x[1, 31::32] = 127.0
+    x[3, 40], x[5, 200] = np.inf, -np.inf
+    x[7] *= np.float32(1e-38)
+    x[9] = np.where(np.arange(256) % 3 == 0, np.float32(3.8e-37), np.float32(-1.3e-37))
+    x[11] *= np.float32(3e38) / np.abs(x[11]).max()
+    if fmt == "q8_k":
+        x[13, 17] = np.nan
+        x[14] = 0.0
+        x[14, 3] = np.nan
+    x = np.ascontiguousarray(x.reshape(-1))
+    say("quantizers, short and long rounding", fmt)
+    got, want = P.dev_quantize(P.to_device(x), fmt, rows=64).cpu().numpy(), T.oracle_quantize(x, fmt, rows=64)
+    assert np.array_equal(got, want), np.nonzero(got != want)[0][:8]
+
+
 def test_quantize_batch_equals_rows_host():
     x = T.normal(7 * 768, seed=12)
     whole = P.quantize(x, "q8_k", rows=7)
