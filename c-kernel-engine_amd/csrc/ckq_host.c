@@ -1248,11 +1248,8 @@ void fused_mlp_swiglu_prefill_w1w2_quant(const float *x, const void *W1, const f
         const int out_on_dev = is_device_ptr(output);
         void *dout = output;
         if (!out_on_dev && buf_reserve(BUF_Y, out_bytes, &dout)) break;
-        int rc = ckq_launch_quantize_q8_0((const float *)dx, dq, seq_len, E, g_stream);
-        if (rc) { fail(rc, "quantize launch"); break; }
-        rc = ckq_launch_gemv(fmt1, (float *)dgu, dW1, dq, (const float *)dB1, 2 * I, E, seq_len, 2L * I, 0, 2 * I,
-                             NULL, g_stream);
-        if (rc) { fail(rc, "gate/up GEMM launch"); break; }
+        int rc = ckq_launch_quantize_gemv_q8_0(fmt1, (const float *)dx, dq, (float *)dgu, dW1, (const float *)dB1, 2 * I, E, seq_len, 2L * I, g_stream);
+        if (rc) { fail(rc, "quantize and gate/up GEMM launch"); break; }
         rc = ckq_launch_swiglu_q8_k((const float *)dgu, (const float *)dgu + I, dh, seq_len, I, 2L * I, g_stream);
         if (rc) { fail(rc, "swiglu launch"); break; }
         rc = ckq_launch_gemv(fmt2, (float *)dout, dW2, dh, (const float *)dB2, E, I, seq_len, (long)E, 0, E, NULL, g_stream);

@@ -819,6 +819,18 @@ __global__ void __launch_bounds__(256) quantize_q8_0_kernel(const float *__restr
     quantize_q8_0_blocks(x, y, nblocks, blockIdx.x);
 }
 
+/* Both of what a Q5_0 matmul on the matrix cores waits for: weights rewritten as Q8_0 blocks (the first `wgrid` blocks, the longer part) and
+ * activations quantized.  Neither fills the chip, and neither needs the other: two launches of 5.4 and 2.9 us in one of about 6 (512 tokens, 9728 x 896). */
+__global__ void __launch_bounds__(256) q5_0_operands_kernel(const uint8_t *__restrict__ W, uint8_t *__restrict__ W8, size_t wblocks, u32 wgrid,
+                                                            const float *__restrict__ x, uint8_t *__restrict__ xq, long xblocks)
+{
+    if (blockIdx.x < wgrid) {
+        const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+        if (i < wblocks) q5_0_to_q8_0_block(W, W8, i);
+    } else
+        quantize_q8_0_blocks(x, xq, xblocks, blockIdx.x - wgrid);
+}
+
 extern "C" int ckq_launch_quantize_q8_k(const float *x, void *y, int rows, int k, void *stream)
 {
     if (!x || !y || rows <= 0 || k <= 0) return CKQ_EINVAL;
@@ -844,6 +856,27 @@ extern "C" int ckq_launch_quantize_q8_0(const float *x, void *y, int rows, int k
     hipLaunchKernelGGL(quantize_q8_0_kernel, dim3((unsigned)((nblocks * 8 + 255) / 256)), dim3(256), 0,
                        (hipStream_t)stream, x, (uint8_t *)y, nblocks);
     return (int)hipGetLastError();
+}
+
+/* y = x W^T with x quantized to Q8_0 at xq on the way, as ckq_launch_quantize_q8_0 and ckq_launch_gemv one after the other give it. */
+extern "C" int ckq_launch_quantize_gemv_q8_0(int fmt, const float *x, void *xq, float *y, const void *W, const float *bias, int nrows, int K, int ntok, long ldy, void *stream)
+{
+    const size_t wblocks = (size_t)nrows * (size_t)(K / 32);
+    const long xblocks = (long)ntok * (K / 32);
+    const unsigned wgrid = (unsigned)((wblocks + 255) / 256), xgrid = (unsigned)((xblocks * 8 + 255) / 256);
+    if (fmt != CKQ_FMT_Q5_0 || !x || !xq || !y || !W || nrows <= 0 || K <= 0 || K % 32 || ntok <= 0 || (wblocks + 255) / 256 + (size_t)xgrid > 0x7fffffffu ||
+        ckq_launch_route(fmt, nrows, K, ntok, 1) != CKQ_ROUTE_TILES) {
+        const int rc = ckq_launch_quantize_q8_0(x, xq, ntok, K, stream);
+        return rc ? rc : ckq_launch_gemv(fmt, y, W, xq, bias, nrows, K, ntok, ldy, 0, nrows, nullptr, stream);
+    }
+    hipStream_t const s = (hipStream_t)stream;
+    std::lock_guard<std::recursive_mutex> lock(g_split_mu);   /* the scratch is shared by launches on this stream */
+    float *tmp = nullptr;
+    int rc = gemm_workspace(1, s, wblocks * 34, &tmp);
+    if (rc) return rc;
+    hipLaunchKernelGGL(q5_0_operands_kernel, dim3(wgrid + xgrid), dim3(256), 0, s, (const uint8_t *)W, (uint8_t *)tmp, wblocks, wgrid, x, (uint8_t *)xq, xblocks);
+    rc = (int)hipGetLastError();
+    return rc ? rc : launch_gemm_q80_mfma(xq, tmp, bias, y, ntok, nrows, K, ldy, GemmOpts{}, s);
 }
 
 /*

@@ -107,6 +107,9 @@ void ckq_launch_set_rows16(int fmt, int on);
 /* fp32 [rows x k] -> Q8_K / Q8_0 blocks, row-major. */
 int ckq_launch_quantize_q8_k(const float *x, void *y, int rows, int k, void *stream);
 int ckq_launch_quantize_q8_0(const float *x, void *y, int rows, int k, void *stream);
+/* ckq_launch_quantize_q8_0(x -> xq) and ckq_launch_gemv of a whole Q8_0 or Q5_0 matrix with xq, in fewer launches where both sides of a matmul are
+ * rewritten first (Q5_0 on the matrix cores). */
+int ckq_launch_quantize_gemv_q8_0(int fmt, const float *x, void *xq, float *y, const void *W, const float *bias, int nrows, int K, int ntok, long ldy, void *stream);
 
 /* y[row] = Q8_K(SiLU(gate[row]) * up[row]), k floats per row, rows ld floats apart. */
 int ckq_launch_swiglu_q8_k(const float *gate, const float *up, void *y, int rows, int k, long ld, void *stream);

@@ -1110,6 +1110,25 @@ def test_fused_mlp_q5_0_gate_up_golden_case():
     assert T.norm_err(got, G["mlp_out_q5_0w1_q4_k_avx2"].reshape(SEQ, AED)) <= TOL
 
 
+@pytest.mark.parametrize("seq,E,I", [(70, 64, 4864), (200, 896, 1024), (129, 928, 1280), (512, 896, 4864), (9, 256, 512)])
+def test_fused_mlp_q5_0_equals_its_steps(seq, E, I):
+    """Activations quantized and weights rewritten by one launch (gate and up on the matrix cores; even and odd numbers of blocks a row, last
+    blocks of either part partly filled; the last size streams): the output is that of the steps called one by one, to the bit."""
+    import torch
+    L = ckq.lib()
+    x = P.to_device(T.normal(seq * E, 0.0, 1.0, seed=E))
+    W1, W2 = P.to_device(T.random_blocks("q5_0", 2 * I * E // 32, 81)), P.to_device(T.synth_weights("q4_k", E, I, seed=82))
+    b1, b2 = P.to_device(T.normal(2 * I, 0.0, 0.1, seed=83)), P.to_device(T.normal(E, 0.0, 0.1, seed=84))
+    y, scr = torch.zeros(seq, E, device="cuda"), torch.zeros(16, dtype=torch.uint8, device="cuda")
+    say("fused mlp q5_0, one launch for both operands", seq, E, I)
+    L.fused_mlp_swiglu_prefill_w1w2_quant(P._dp(x), P._dp(W1), P._dp(b1), P.CK_DT["q5_0"], P._dp(W2), P._dp(b2), P.CK_DT["q4_k"], P._dp(y),
+                                          seq, E, E, I, I, P._dp(scr))
+    gu = P.dev_gemm_nt("q5_0", P.dev_quantize(x, "q8_0", rows=seq), W1, b1, seq, 2 * I, E).view(seq, 2 * I)
+    h = P.dev_swiglu_q8_k(gu.view(-1), gu.view(-1)[I:], seq, I, 2 * I)
+    want = P.dev_gemm_nt("q4_k", h, W2, b2, seq, E, I).view(seq, E)
+    assert bool(torch.isfinite(want).all()) and torch.equal(y, want)
+
+
 # ---- automatic choice between the streaming kernel and the matrix cores --------------------------
 
 @pytest.mark.parametrize("fmt,N,K,expect", [
