@@ -514,6 +514,23 @@ def test_embedding_forward_golden_and_oracle(fmt, add_pos):
     assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
 
 
+@pytest.mark.parametrize("fmt", ["q4_k", "q6_k", "q8_0"])
+@pytest.mark.parametrize("n_row,n_valid", [(256, 256), (512, 511), (768, 2), (4096, 4093), (4352, 4352), (8448, 8447)])
+def test_dequant_rows_at_the_edges_of_their_units(fmt, n_row, n_valid):
+    """Rows of one block, of a whole number of thread blocks and of some threads more; zeros from an element on that is inside a run of four; rows
+    behind the last token; ids outside the vocabulary; positions."""
+    voc, rows, tokens = 40, 7, 5
+    tab = T.random_blocks(fmt, voc * (n_row // T.ELEMS[fmt]), n_row)
+    ids = np.array([0, voc - 1, voc, -1, 17], np.int32)
+    pos = T.normal(rows * n_row, 0.0, 0.1, seed=n_row)
+    for add_pos in (0, 1):
+        ref = np.full(rows * n_row, 9.0, np.float32)
+        T.oracle().orc_embedding_forward(T.FMT[fmt], T.ptr(ids), tokens, voc, T.ptr(tab), T.ptr(pos), T.ptr(ref), n_valid, n_row, rows, add_pos)
+        say("dequant rows", fmt, n_row, n_valid, add_pos)
+        got = P.dev_dequant_rows(fmt, P.to_device(tab), P.to_device(ids), voc, P.to_device(pos) if add_pos else None, n_valid, n_row, tokens, rows)
+        assert np.array_equal(got.cpu().numpy().reshape(-1).view(np.uint32), ref.view(np.uint32))
+
+
 # ---- prefill GEMM on the matrix cores (Q4_K, token counts above 16) -------------------------
 
 @pytest.mark.parametrize("M,N,K", [(17, 128, 256), (33, 200, 1024), (64, 96, 512), (100, 333, 2048),
