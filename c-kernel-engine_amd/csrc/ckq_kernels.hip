@@ -885,29 +885,35 @@ extern "C" int ckq_launch_quantize_gemv_q8_0(int fmt, const float *x, void *xq, 
  * maximum goes through DPP, and x stays in registers: 4096 wide, one row 5.1 -> 4.2 us, 512 rows 7.1 -> 6.0,
  * 2048 rows 23.3 -> 12.1.
  */
-template <int GREG>
+template <int GREG, bool ALONE>
 __global__ void __launch_bounds__(1024) rmsnorm_q8_k_fused_kernel(const float *__restrict__ input, const float *__restrict__ gamma,
                                                                   uint8_t *__restrict__ y, int d_model, long in_stride, float eps)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    rms_row<GREG>(input + (size_t)blockIdx.x * in_stride, gamma, y + (size_t)blockIdx.x * (d_model / 256) * 292,
+    rms_row<GREG, ALONE>(input + (size_t)blockIdx.x * in_stride, gamma, y + (size_t)blockIdx.x * (d_model / 256) * 292,
                   d_model, eps, reinterpret_cast<float *>(smem));
 }
 
 constexpr int RMS_FEW_TOKENS = 512;
-template <int GREG>
-static int launch_rms(const float *input, const float *gamma, uint8_t *y, int tokens, int d_model, long stride, float eps, int waves, hipStream_t s)
+template <int GREG, bool ALONE>
+static int launch_rms_form(const float *input, const float *gamma, uint8_t *y, int tokens, int d_model, long stride, float eps, int waves, hipStream_t s)
 {
     const size_t lds = rms_lds_bytes((size_t)d_model);
     if (lds > 64 * 1024) {
         /* more than 64 KB of dynamic LDS is an opt-in per function and per device: set on every
          * such call for the device that is current (rows this long are rare; the call is cheap) */
-        hipError_t e = hipFuncSetAttribute((const void *)rmsnorm_q8_k_fused_kernel<GREG>,
+        hipError_t e = hipFuncSetAttribute((const void *)rmsnorm_q8_k_fused_kernel<GREG, ALONE>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         if (e != hipSuccess) return (int)e;
     }
-    hipLaunchKernelGGL(rmsnorm_q8_k_fused_kernel<GREG>, dim3((unsigned)tokens), dim3(64 * waves), lds, s, input, gamma, y, d_model, stride, eps);
+    hipLaunchKernelGGL((rmsnorm_q8_k_fused_kernel<GREG, ALONE>), dim3((unsigned)tokens), dim3(64 * waves), lds, s, input, gamma, y, d_model, stride, eps);
     return (int)hipGetLastError();
+}
+template <int GREG>
+static int launch_rms(const float *input, const float *gamma, uint8_t *y, int tokens, int d_model, long stride, float eps, int waves, hipStream_t s)
+{
+    return tokens <= 256 ? launch_rms_form<GREG, true>(input, gamma, y, tokens, d_model, stride, eps, waves, s)
+                         : launch_rms_form<GREG, false>(input, gamma, y, tokens, d_model, stride, eps, waves, s);
 }
 
 extern "C" int ckq_launch_rmsnorm_q8_k_fused(const float *input, const float *gamma, void *y, int tokens, int d_model,

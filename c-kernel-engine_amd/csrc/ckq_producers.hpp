@@ -90,6 +90,45 @@ __device__ __forceinline__ void rms_chain(float *xs, int D, int j)
     xs[8 * rms_pitch(D) + j] = acc;
 }
 
+/* The same for a row that has its CU to itself.  A multiply-add of the chain takes some eight cycles, and the values should be there
+ * before it: 32 are read while the 32 before them are added.  The reads are volatile because the compiler moves ordinary ones to
+ * where they are used, as it does above, where every 32 values wait for LDS.  4096 wide, one row 4.2 -> 3.9 us, 256 rows 5.4 -> 5.1, 8192 wide 7.2 -> 6.3; but
+ * the 64 registers keep a second block of sixteen waves off the CU (512 rows 6.8 -> 8.5).  Sixteen values ahead 4.1 and 6.8; a ring of
+ * 32 filled four at a time 4.4 and 7.3; whole waves, a chain to every sixteen lanes that broadcast it their values, 4.4 and 7.0. */
+typedef float rms_v4f __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void rms_chain_alone(float *xs, int D, int j)
+{
+    typedef const volatile __attribute__((address_space(3))) rms_v4f *lds_ptr;
+    const lds_ptr x = (lds_ptr)(const rms_v4f *)(xs + j * rms_pitch(D));
+    float acc = 0.0f;
+    rms_v4f even[8], odd[8];
+    auto load = [&](rms_v4f (&v)[8], int b) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = x[8 * b + u];
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto add = [&](const rms_v4f (&v)[8]) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) acc = __builtin_fmaf(v[u][k], v[u][k], acc);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const int nb = D / 256;
+    load(even, 0);
+    int b = 0;
+    for (; b + 2 < nb; b += 2) {
+        load(odd, b + 1);
+        add(even);
+        load(even, b + 2);
+        add(odd);
+    }
+    if (b + 1 < nb) load(odd, b + 1);
+    add(even);
+    if (b + 1 < nb) add(odd);
+    xs[8 * rms_pitch(D) + j] = acc;
+}
+
 /* rstd from the eight chain sums (every thread derives the same value).
  * sqrtf and '/' are the correctly rounded ones (the __fsqrt_rn intrinsic is not). */
 __device__ __forceinline__ float rms_rstd(const float *xs, int D, float eps)
@@ -126,8 +165,8 @@ __device__ __forceinline__ void rms_quant_block(const float4 xv, const float4 gv
 
 /* A block of nw waves turns row x (D floats) into its D/256 Q8_K blocks at y.  Wave w owns 256-blocks w, w + nw, ...;
  * the x and gamma of its first GREG blocks are loaded at the start and kept in registers across the chain, so a row of
- * up to GREG * nw blocks costs one round trip to memory.  smem: rms_lds_bytes(D). */
-template <int GREG>
+ * up to GREG * nw blocks costs one round trip to memory.  ALONE: there is no more than one row for a CU.  smem: rms_lds_bytes(D). */
+template <int GREG, bool ALONE>
 __device__ __forceinline__ void rms_row(const float *__restrict__ x, const float *__restrict__ gamma,
                                         uint8_t *__restrict__ y, int D, float eps, float *xs)
 {
@@ -143,7 +182,10 @@ __device__ __forceinline__ void rms_row(const float *__restrict__ x, const float
         if (wave + nw * r < nb) rms_stage(xs, D, wave + nw * r, lane, xv[r]);
     for (int b = wave + nw * GREG; b < nb; b += nw) rms_stage(xs, D, b, lane, reinterpret_cast<const float4 *>(x + 256 * b)[lane]);
     __syncthreads();
-    if (tid < 8) rms_chain(xs, D, tid);
+    if (tid < 8) {
+        if constexpr (ALONE) rms_chain_alone(xs, D, tid);
+        else                 rms_chain(xs, D, tid);
+    }
     __syncthreads();
     const float rstd = rms_rstd(xs, D, eps);
 #pragma unroll

@@ -471,6 +471,17 @@ def test_rmsnorm_q8_k_fused_bit_exact_vs_oracle(tokens, D, std, seed):
         y = P.dev_gemm_nt("q4_k", P.to_device(out), P.to_device(W), None, tokens, 64, D).cpu().numpy()
         assert T.norm_err(y, T.oracle_gemm_nt("q4_k", ref, W, None, tokens, 64, D)) <= TOL
 
+@pytest.mark.parametrize("tokens,D", [(1, 256), (2, 512), (5, 768), (256, 1280), (257, 1280), (3, 4096), (256, 4352), (1, 16640)])
+def test_rmsnorm_q8_k_fused_rows_alone_on_their_cu_bit_exact(tokens, D):
+    """Rows that have a CU to themselves read their chains further ahead: one, two, an odd and an even number of runs of 32
+    values, the last number of tokens that does so and the first that does not."""
+    x, g = T.normal(tokens * D, 0.1, 1.0, seed=D), T.normal(D, 1.0, 0.3, seed=D + 1)
+    say("rmsnorm_q8_k_fused, rows alone", tokens, D)
+    ref = np.zeros(tokens * (D // 256) * 292, np.uint8)
+    T.oracle().orc_rmsnorm_q8_k_fused(T.ptr(x), T.ptr(g), T.ptr(ref), tokens, D, D, ctypes.c_float(1e-6))
+    assert np.array_equal(P.dev_rmsnorm_q8_k_fused(P.to_device(x), P.to_device(g), tokens, D).cpu().numpy(), ref)
+
+
 # ---- row dequantizers and quantized embedding lookup, bit-exact -----------------------------
 
 @pytest.mark.parametrize("fmt", ["q4_k", "q6_k", "q8_0"])
