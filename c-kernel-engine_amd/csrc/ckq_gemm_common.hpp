@@ -132,6 +132,15 @@ static int gemm_choose_splits(int tiles, int k_steps)
     return s < 2 ? 1 : s;
 }
 
+/* Global -> LDS, 16 bytes per lane from rs + ofs + k to dst + 16 lane.  Written out because the compiler, which cannot know which
+ * bytes of an LDS object a copy in flight still has to write, waits for all of them before the next read of that object; the
+ * one wait there has to be is the loop's. */
+__device__ __forceinline__ void lds_copy16(const ckq_v4i &rs, u32 dst, u32 ofs, int k)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(dst), "v"(ofs), "s"(rs), "s"(k) : "memory");
+}
+__device__ __forceinline__ u32 lds_address(const void *p) { return (u32)(uintptr_t)(__attribute__((address_space(3))) const void *)p; }
+
 constexpr int GEMM_TILE_ROWS = 128;    /* weight rows per tile, all four kernels */
 
 /* Scratch for the partial tiles of K-split launches (kind 0) and for weights

@@ -53,15 +53,6 @@ __device__ __forceinline__ float q80_output(const uint8_t *w, const uint8_t *x, 
     return acc;
 }
 
-/* Global -> LDS, 16 bytes per lane from rs + ofs + k to dst + 16 lane.  Written out because the compiler, which cannot know which
- * bytes of an LDS object a copy in flight still has to write, waits for all of them before the next read of that object; the
- * one wait there has to be is the loop's. */
-__device__ __forceinline__ void lds_copy16(const ckq_v4i &rs, u32 dst, u32 ofs, int k)
-{
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(dst), "v"(ofs), "s"(rs), "s"(k) : "memory");
-}
-__device__ __forceinline__ u32 lds_address(const void *p) { return (u32)(uintptr_t)(__attribute__((address_space(3))) const void *)p; }
-
 /*
  * LDS image of an operand row, 144 bytes for the four blocks of an iteration: the 136 bytes as they are in memory, 34 dwords, in
  * nine 16-byte chunks (adjacent lanes of a copy fetch adjacent chunks, all from dword-aligned addresses).  Chunk 8 holds the last

@@ -651,12 +651,16 @@ gemm_rows16_hold_kernel(const uint8_t *W, const uint8_t *X, int N, int M, int nb
 }
 
 /* Short rows, several token groups: a block has a wave for every 256-block of its 16 rows (at most KEEP_NB of them) and goes
- * through `per` groups of 16 tokens, the planes and scales of its weights formed once and kept in registers.  The kernel above
+ * through `per` groups of 16 tokens, the planes and scales of its weights formed once and kept in registers.  The first kernel
  * forms them again for every group, and they are a good third of what bounds it there, VALU issue (Q5_K, 93 tokens: 480 vector
- * instructions a 256-block and group at 1024 x 4864, 64 % of the busy CUs' issue cycles; here 301 and 63 % at 2 x 4864 x 1024, which took
- * 20.9 us in the kernel above and takes 15.1).  The terms and their order are the same. */
-constexpr int KEEP_NB = 8;
-template <class F> constexpr int rows16_keep_wave_lds() { return 16 * (F::PITCH > 288 ? F::PITCH : 288); }
+ * instructions a 256-block and group at 1024 x 4864, 64 % of the busy CUs' issue cycles).  The terms and their order are the same.
+ * A group's quants and bsums are copied to LDS without passing through registers, as they lie in memory, as soon as the wave has read the group before: 240
+ * instructions a 256-block and group where fetching them to registers and writing them took 301, and two thirds of the LDS instructions.  2 x 4864 x 1024
+ * Q5_K at 93 tokens 20.9 us in the first kernel, 13.2 through registers, 11.2 now; over 400 launches of 17 to 256 tokens, 256 to 30000 rows, this against
+ * through registers 1.06 on average (five 256-blocks a row, large 1.28-1.43; eight 1.03; all 0.86-1.59).  A lane loading its operands
+ * itself needs no LDS and fewer instructions still, but its 64-byte pieces of sixteen tokens are twice the accesses of the L1, which bound
+ * large launches (12.2; 64 x 11008 x 2048 Q6_K 17.8 -> 18.5). */
+constexpr int KEEP_NB = 8, KEEP_WAVE_LDS = 16 * 288;            /* a group's quants and bsums; before them the 16 weight blocks */
 template <class F, bool TREE, bool GRP>
 __global__ void __launch_bounds__(64 * KEEP_NB)
 gemm_rows16_keep_kernel(const uint8_t *W, const uint8_t *X, int N, int M, int parts, int per, float *y, const float *bias, long ldy, GemmChains ch, Rows16Args grp)
@@ -682,40 +686,36 @@ gemm_rows16_keep_kernel(const uint8_t *W, const uint8_t *X, int N, int M, int pa
     }
     const int n0 = tile * 16;
     const u32 xrow = (u32)nb * 292u, wpitch = (u32)nb * (u32)F::WBLOCK;
-    uint8_t *const al = smem + wave * rows16_keep_wave_lds<F>(), *const bl = al + NT * 256;   /* the weights first, then each group's quants and bsums */
-    float *const us = reinterpret_cast<float *>(smem + nb * rows16_keep_wave_lds<F>());       /* two groups' terms: one written while the other is read */
-    float *const dxs = us + 2 * nb * (NT * 16);
+    uint8_t *const al = smem + wave * KEEP_WAVE_LDS, *const bl = al + NT * 256;           /* this wave's weights first, then each group's quants and bsums */
+    float *const us = reinterpret_cast<float *>(smem + nb * KEEP_WAVE_LDS);               /* two groups' terms: one written while the other is read */
+    const int slots = nb <= 2 ? 2 : nb <= 4 ? 4 : 8;      /* of the tree; the last stay zero */
+    float *const dxs = us + 2 * slots * (NT * 16);
     const uint8_t *const wbase = W + (size_t)n0 * wpitch + (u32)wave * (u32)F::WBLOCK;
-    const uint8_t *xbase = X + (size_t)(g0 * NT) * xrow + (u32)wave * 292u;
+    const uint8_t *const xbase = X + (u32)wave * 292u;
 
-    /* copy roles as in gemm_rows16_kernel; lanes 0..15 fetch the tokens' scales */
-    constexpr int NWL = (16 * F::CHUNKS + 63) / 64, NAL = (NT * 18 + 63) / 64;
-    u32 asrc[NAL], adst[NAL], dsrc = 0;
+    /* 16-byte chunk c of token t goes to slot c ^ t; j = 4: the bsums */
+    u32 asrc[5], dsrc;
     auto token_offsets = [&](int last) {
 #pragma unroll
-        for (int j = 0; j < NAL; ++j) {
-            const int e = min(64 * j + lane, NT * 18 - 1);
-            asrc[j] = (u32)min(e / 18, last) * xrow + 4u + 16u * (u32)(e % 18);
-        }
+        for (int j = 0; j < 4; ++j) asrc[j] = (u32)min(4 * j + q, last) * xrow + 4u + 16u * (u32)(i16 ^ (4 * j + q));
+        asrc[4] = (u32)min(lane >> 1, last) * xrow + 260u + 16u * (u32)(lane & 1);
         dsrc = (u32)min(i16, last) * xrow;
     };
-#pragma unroll
-    for (int j = 0; j < NAL; ++j) {
-        const int e = min(64 * j + lane, NT * 18 - 1), t = e / 18, c = e % 18;
-        adst[j] = (u32)(c < 16 ? 256 * t + 16 * (c ^ (t & 15)) : NT * 256 + 32 * t + 16 * (c - 16));
-    }
     token_offsets(min(NT, M - g0 * NT) - 1);
-    ckq_v4i wr[NWL], ar[NAL];
-    float dr;
-    auto fetch = [&]() {
+    const ckq_v4i xsrd = {__builtin_amdgcn_readfirstlane((int)(u32)(uintptr_t)xbase), __builtin_amdgcn_readfirstlane((int)(u32)((uintptr_t)xbase >> 32)), 0x7fffffff, 0x00020000};
+    const u32 adst = lds_address(al);
+    u32 dr;
+    auto fetch = [&](int gr) {
+        const int k = gr * NT * (int)xrow;
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 0; j < NAL; ++j) {
-            u32 t[4];
-            ld16<4>(t, xbase + asrc[j]);
-            ar[j] = ckq_v4i{(int)t[0], (int)t[1], (int)t[2], (int)t[3]};
-        }
-        dr = __builtin_bit_cast(float, ld4<4>(xbase + dsrc));
+        for (int j = 0; j < 4; ++j) lds_copy16(xsrd, adst + 1024u * j, asrc[j], k);
+        if (F::MIN && lane < 32) lds_copy16(xsrd, adst + 4096u, asrc[4], k);
+        dr = ld4<4>(xbase + (size_t)(u32)k + dsrc);         /* last: once it is there, all are */
+        __builtin_amdgcn_sched_barrier(0);
     };
+    constexpr int NWL = (16 * F::CHUNKS + 63) / 64;
+    ckq_v4i wr[NWL];
     u32 wdst[NWL];
 #pragma unroll
     for (int j = 0; j < NWL; ++j) {
@@ -725,7 +725,6 @@ gemm_rows16_keep_kernel(const uint8_t *W, const uint8_t *X, int N, int M, int pa
         wr[j] = ckq_v4i{(int)t[0], (int)t[1], (int)t[2], (int)t[3]};
         wdst[j] = (u32)(r * F::PITCH + 16 * c);
     }
-    fetch();
 #pragma unroll
     for (int j = 0; j < NWL; ++j) *reinterpret_cast<ckq_v4i *>(al + wdst[j]) = wr[j];
     __builtin_amdgcn_wave_barrier();
@@ -735,51 +734,65 @@ gemm_rows16_keep_kernel(const uint8_t *W, const uint8_t *X, int N, int M, int pa
     F::head(hd, wrow, q);
 #pragma unroll
     for (int g = 0; g < 4; ++g) F::planes(ph[g], pl[g], hd, wrow, g, q);
-    __builtin_amdgcn_wave_barrier();                  /* the wave's own LDS accesses stay in this order */
+    for (int e = tid; e < (slots - nb) * (NT * 16); e += nthr) us[nb * (NT * 16) + e] = us[(slots + nb) * (NT * 16) + e] = 0.0f;
+    __builtin_amdgcn_s_waitcnt(0xc07f);           /* lgkmcnt(0): the weights have been read */
+    asm volatile("" ::: "memory");
+    fetch(g0);
+    /* vmcnt(0): in the loop a group's loads are older than the stores of the group before, and only with nothing on its way here can
+     * the compiler tell, and wait for the loads alone */
+    __builtin_amdgcn_s_waitcnt(0x0f70);
 
     const ckq_v4i zero = {0, 0, 0, 0};
     for (int gr = g0, p = 0; gr < g1; ++gr, p ^= 1) {
-        float *const u = us + p * nb * (NT * 16), *const dx = dxs + p * nb * NT;
-#pragma unroll
-        for (int j = 0; j < NAL; ++j) *reinterpret_cast<ckq_v4i *>(al + adst[j]) = ar[j];
-        if (lane < NT) dx[wave * NT + lane] = dr;
-        if (gr + 1 < g1) {
-            xbase += (size_t)NT * xrow;
-            if ((gr + 2) * NT > M) token_offsets(M - 1 - (gr + 1) * NT);
-            fetch();
-        }
+        float *const u = us + p * slots * (NT * 16), *const dx = dxs + p * nb * NT;
+        asm volatile("" : "+v"(dr));
+        if (lane < NT) dx[wave * NT + lane] = __builtin_bit_cast(float, dr);
         __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_wave_barrier();
-        ckq_v4f i2s = {0.0f, 0.0f, 0.0f, 0.0f};
-        ckq_v4i am = zero;
+        asm volatile("" ::: "memory");
+        int2 am = {};
         if constexpr (F::MIN) {
-            const int2 bs = *reinterpret_cast<const int2 *>(bl + 32 * i16 + 8 * q);
-            const int p0 = (int)(int16_t)(bs.x & 0xffff) + (bs.x >> 16), p1 = (int)(int16_t)(bs.y & 0xffff) + (bs.y >> 16);
-            am = ckq_v4i{(int)bf16_pair((float)(p0 & 63), (float)(p1 & 63)), (int)bf16_pair((float)(64 * (p0 >> 6)), (float)(64 * (p1 >> 6))), 0, 0};
+            const int2 b = *reinterpret_cast<const int2 *>(bl + 32 * i16 + 8 * q);
+            const int p0 = (int)(int16_t)(b.x & 0xffff) + (b.x >> 16), p1 = (int)(int16_t)(b.y & 0xffff) + (b.y >> 16);
+            am = int2{(int)bf16_pair((float)(p0 & 63), (float)(p1 & 63)), (int)bf16_pair((float)(64 * (p0 >> 6)), (float)(64 * (p1 >> 6)))};
+        }
+        ckq_v4i a[4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) a[g] = lds16(al + 256 * i16 + 16 * ((int)(F::a_elem(g, q) >> 4) ^ i16));
+        /* the next group comes where this one lay once it has been read: lgkmcnt(0) */
+        __builtin_amdgcn_s_waitcnt(0xc07f);
+        asm volatile("" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(am.x), "+v"(am.y) :: "memory");
+        if (gr + 1 < g1) {
+            if ((gr + 2) * NT > M) token_offsets(M - 1 - (gr + 1) * NT);
+            fetch(gr + 1);
         }
         auto min_mfma = [&](const ckq_v4i &mins) {
             const ckq_v4f z = {0.0f, 0.0f, 0.0f, 0.0f};
-            return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(ckq_v8bf, am), __builtin_bit_cast(ckq_v8bf, mins), z, 0, 0, 0);
+            const ckq_v4i am4 = {am.x, am.y, 0, 0};
+            return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(ckq_v8bf, am4), __builtin_bit_cast(ckq_v8bf, mins), z, 0, 0, 0);
         };
         float out[4];
         if constexpr (TREE) {
             const ckq_v4i dxi = lds16(reinterpret_cast<const uint8_t *>(dx + wave * NT + 4 * q));
             float t[4][4];
+            ckq_v4i sh[4], sl[4];
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                const ckq_v4i a = lds16(al + 256 * i16 + 16 * ((int)(F::a_elem(g, q) >> 4) ^ i16));
-                const ckq_v4i sh = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, ph[g], zero, 0, 0, 0);
-                const ckq_v4i sl = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, pl[g], zero, 0, 0, 0);
-                if constexpr (F::MIN) i2s = min_mfma(q == g ? hd.mins : zero);
+                sh[g] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[g], ph[g], zero, 0, 0, 0);
+                sl[g] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[g], pl[g], zero, 0, 0, 0);
+            }
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                ckq_v4f i2;
+                if constexpr (F::MIN) i2 = min_mfma(q == g ? hd.mins : zero);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int di = dxi[r];
-                    const float d = __builtin_bit_cast(float, di), f = (float)((sh[r] << F::SHIFT) + sl[r]);
+                    const float d = __builtin_bit_cast(float, di), f = (float)((sh[g][r] << F::SHIFT) + sl[g][r]);
                     float v;
-                    if constexpr (F::MIN) v = (hd.dw * d) * f - (hd.dmin * d) * i2s[r];
+                    if constexpr (F::MIN) v = (hd.dw * d) * f - (hd.dmin * d) * i2[r];
                     else                  v = (hd.dw * d) * f;
                     asm volatile("" : "+v"(v));              /* rounded before it is added, as in the streaming kernel */
-                    t[g][r] = 0.0f + v;
+                    t[g][r] = v;                             /* which adds it to a zero: made up for by the zero at the end */
                 }
             }
 #pragma unroll
@@ -788,49 +801,58 @@ gemm_rows16_keep_kernel(const uint8_t *W, const uint8_t *X, int N, int M, int pa
             ckq_v4i sh, sl;
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                const ckq_v4i a = lds16(al + 256 * i16 + 16 * ((int)(F::a_elem(g, q) >> 4) ^ i16));
-                sh = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, ph[g], g ? sh : zero, 0, 0, 0);
-                sl = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, pl[g], g ? sl : zero, 0, 0, 0);
+                sh = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[g], ph[g], g ? sh : zero, 0, 0, 0);
+                sl = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[g], pl[g], g ? sl : zero, 0, 0, 0);
             }
-            if constexpr (F::MIN) i2s = min_mfma(hd.mins);
+            ckq_v4f i2;
+            if constexpr (F::MIN) i2 = min_mfma(hd.mins);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const float f = (float)((sh[r] << F::SHIFT) + sl[r]);
-                out[r] = F::MIN ? hd.dw * f - hd.dmin * i2s[r] : hd.dw * f;
+                if constexpr (F::MIN) out[r] = hd.dw * f - hd.dmin * i2[r];
+                else                  out[r] = hd.dw * f;
             }
         }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) u[wave * (NT * 16) + 64 * r + lane] = out[r];
+        *reinterpret_cast<float4 *>(u + wave * (NT * 16) + 4 * lane) = float4{out[0], out[1], out[2], out[3]};
         /* one barrier a group: the terms of the group after next overwrite these, behind the next group's barrier */
         __syncthreads();
-        for (int e = tid; e < NT * 16; e += nthr) {
-            const int tok = 4 * ((e & 63) >> 4) + (e >> 6), n = n0 + (e & 15), t = gr * NT + tok;
+        const __amdgpu_buffer_rsrc_t yb = __builtin_amdgcn_make_buffer_rsrc(y + (size_t)(gr * NT) * ldy, 0, 0x7fffffff, 0x00020000);
+        /* Four waves add the terms up, of eight the two fours in turn.  All store, the others past the buffer's end: a store that not every
+         * way through the loop has would make the loads of the next group wait for it. */
+        const bool mine = nthr <= NT * 16 || wave >> 2 == (nb == 8 ? gr & 1 : 0);
+        int done = 0;
+        do {
+            const int e = min(done + (tid & (NT * 16 - 1)), NT * 16 - 1);          /* output e % 4 of lane e / 4 */
+            const int tok = 4 * (e >> 6) + (e & 3), n = n0 + ((e >> 2) & 15);
+            const bool live = mine && done + (tid & (NT * 16 - 1)) < NT * 16 && n < N && gr * NT + tok < M;
+            const float *ue = u + e;
             float v = 0.0f;
-            if constexpr (TREE) {
-                float w[KEEP_NB];
-#pragma unroll
-                for (int b = 0; b < KEEP_NB; ++b) w[b] = b < nb ? u[b * (NT * 16) + e] : 0.0f;
-#pragma unroll
-                for (int k = 1; k < KEEP_NB; k *= 2)
-#pragma unroll
-                    for (int b = 0; b < KEEP_NB; b += 2 * k) w[b] += w[b + k];
-                v = w[0] + 0.0f;                      /* the other half of the tree, empty */
-            } else {
-                for (int sp = 0; sp < ch.splits; ++sp) {
-                    const int b0 = sp * ch.per, b1 = min(nb, b0 + ch.per);
-                    float c[2] = {0.0f, 0.0f};
-                    for (int b = b0; b < b1; ++b) {
-                        const int k = ch.kg == 2 ? (b - b0) & 1 : 0;
-                        const float uu = u[b * (NT * 16) + e], dd = dx[b * NT + tok];
-                        if (k) c[1] = fmaf(dd, uu, c[1]);
-                        else   c[0] = fmaf(dd, uu, c[0]);
+            if (mine) {
+                if constexpr (TREE) {
+                    auto pair = [&](int b) { return ue[b * (NT * 16)] + ue[(b + 1) * (NT * 16)]; };
+                    v = pair(0);
+                    if (nb > 2) v += pair(2);
+                    if (nb > 4) v += pair(4) + pair(6);
+                    v += 0.0f;                    /* the rest of the tree, empty */
+                } else {
+                    for (int sp = 0; sp < ch.splits; ++sp) {
+                        const int b0 = sp * ch.per, b1 = min(nb, b0 + ch.per);
+                        float c[2] = {0.0f, 0.0f};
+                        for (int b = b0; b < b1; ++b) {
+                            const int k = ch.kg == 2 ? (b - b0) & 1 : 0;
+                            const float uu = ue[b * (NT * 16)], dd = dx[b * NT + tok];
+                            if (k) c[1] = fmaf(dd, uu, c[1]);
+                            else   c[0] = fmaf(dd, uu, c[0]);
+                        }
+                        if (ch.kg == 2) c[0] += c[1];
+                        v = sp ? v + c[0] : c[0];
                     }
-                    if (ch.kg == 2) c[0] += c[1];
-                    v = sp ? v + c[0] : c[0];
                 }
+                if (bias) v += bias[min(n, N - 1)];
             }
-            if (n < N && t < M) y[(size_t)t * ldy + n] = bias ? v + bias[n] : v;
-        }
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(u32, v), yb, live ? 4 * (tok * (int)ldy + n) : -4, 0, 0);
+            done += nthr;
+        } while (done < NT * 16);
     }
 }
 
@@ -916,7 +938,7 @@ int launch_rows16_keep(Rows16Args &a, int parts, hipStream_t s)
         tiles += (a.p[i].N + 15) / 16;
     }
     const int groups = (a.M + 15) / 16, per = (groups + parts - 1) / parts;
-    const size_t lds = (size_t)a.nb * (rows16_keep_wave_lds<F>() + 2 * 1024 + 2 * 64);
+    const size_t lds = (size_t)a.nb * (KEEP_WAVE_LDS + 2 * 64) + (a.nb <= 2 ? 2 : a.nb <= 4 ? 4 : 8) * 2 * 1024;
     const Rows16Problem &p = a.p[0];
     const dim3 grid((unsigned)(tiles * parts)), block((unsigned)(64 * a.nb));
     if (a.n > 1)
@@ -987,7 +1009,9 @@ int launch_rows16(int fmt, Rows16Args &a, hipStream_t s)
 {
     long tiles = 0;
     for (int i = 0; i < a.n; ++i) tiles += (a.p[i].N + 15) / 16;
-    const int parts = rows16_keep_parts(fmt, tiles, (a.M + 15) / 16, a.nb, nullptr);
+    bool near = true;                              /* the kernel that keeps its planes has 32 bits for where a group's outputs lie */
+    for (int i = 0; i < a.n; ++i) near = near && a.p[i].ldy < 1 << 25;
+    const int parts = near ? rows16_keep_parts(fmt, tiles, (a.M + 15) / 16, a.nb, nullptr) : 0;
     if (parts) return a.tree ? launch_rows16_keep<F, true>(a, parts, s) : launch_rows16_keep<F, false>(a, parts, s);
     int grid, round;
     size_t lds;

@@ -1706,6 +1706,44 @@ def test_16_row_tiles_of_short_rows_and_several_token_groups(fmt):
 
 
 @pytest.mark.parametrize("fmt", ["q4_k", "q5_k", "q6_k"])
+def test_16_row_tiles_of_several_token_groups_copied_to_lds(fmt):
+    """Where the kernel that keeps its planes copies a group while the one before is at work: three groups and more for one block, one
+    to eight waves (sums by part of the waves, by all, by two fours in turn), a last group of one token, and an output pitch past what its
+    stores reach, which another kernel serves.  In both orders bit for bit, with a bias and a padded C."""
+    import torch
+    L = ckq.lib()
+    tag = P.FMT[fmt]
+    try:
+        for M, N, K, ldy in [(161, 2033, 256, 2040), (49, 5000, 512, 5000), (113, 900, 768, 901), (97, 3001, 1024, 3001), (65, 2100, 1536, 2111), (81, 1300, 2048, 1300),
+                             (18, 40, 1024, 1 << 25)]:
+            if fmt == "q4_k" and K > 1024:
+                continue
+            xq = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, seed=M)), "q8_k", rows=M)
+            W, bias = P.to_device(T.random_blocks(fmt, N * K // 256, 9450 + M)), P.to_device(T.normal(N, 0.0, 0.5, seed=N))
+            say("16-row tiles, groups copied to LDS", fmt, M, N, K, ldy)
+
+            def call(policy, forced):
+                L.ckq_set_prefill_variant(tag, 16 if forced else 0)
+                L.ckq_set_gemm_policy(policy)
+                c = torch.full(((M - 1) * ldy + N,), 7.0, device="cuda")
+                P.check(L.ckq_gemm_nt_dev(tag, P._dp(xq), P._dp(W), P._dp(bias), P._dp(c), M, N, K, ldy, P._stream()), "ckq_gemm_nt_dev")
+                return c.as_strided((M, N), (ldy, 1)), c
+            (tree, all_), (chain, _), (tiles, _) = call(2, True), call(1, True), call(1, False)
+            assert torch.equal(chain, tiles), (M, N, K)
+            if ldy > N:
+                assert bool((all_[N:ldy] == 7.0).all()), (M, N, K)
+            L.ckq_set_prefill_variant(tag, 0)
+            L.ckq_set_gemm_policy(0)
+            rb = xq.numel() // M
+            for m in {0, 15, 16, M // 2, M - 1}:
+                one = P.dev_gemm_nt(fmt, xq[m * rb:(m + 1) * rb].clone(), W, bias, 1, N, K)
+                assert torch.equal(tree[m], one.view(N)), (M, N, K, m)
+    finally:
+        L.ckq_set_gemm_policy(0)
+        L.ckq_set_prefill_variant(tag, 0)
+
+
+@pytest.mark.parametrize("fmt", ["q4_k", "q5_k", "q6_k"])
 def test_16_row_tiles_with_held_activations(fmt):
     """The kernel that goes through several row tiles with its activations in registers: one wave a block and sixteen, blocks of one
     tile, of some more than others and of several rounds of the tiles whose terms fit the LDS, last tiles that start early (row counts
