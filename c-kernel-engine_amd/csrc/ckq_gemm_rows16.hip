@@ -29,6 +29,7 @@
 #include "ckq_gemm_rows16.hpp"
 #include "ckq_gemm_q4k.hpp"
 #include <atomic>
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -650,6 +651,230 @@ gemm_rows16_hold_kernel(const uint8_t *W, const uint8_t *X, int N, int M, int nb
     }
 }
 
+/* Rows too long to keep their planes, several token groups: two groups of 16 tokens a block, so that the planes of a weight
+ * block are formed once for both.  As in the first kernel wave w takes 256-blocks w, w + waves, ..., the next one's weights on their way;
+ * a lane loads its own activations, in the order of the instruction.  Of TREE's terms, those of a position whose lane of the streaming
+ * kernel has two blocks of the row (`wide` positions: blocks 0 .. wide - 1 and those from 16 on) go to LDS one by one, all others summed over their block.
+ * Bound: VALU issue, 257 instructions a 256-block and group (Q5_K, TREE; 480 in the first kernel).  us against the first kernel: Q6_K 1024 x 4864 at 93
+ * tokens 14.2 -> 9.0, Q5_K 11.4 -> 10.5, Q4_K 4096 x 4096 at 24 8.1 -> 7.0. */
+template <class F, bool TREE, bool GRP>
+__global__ void __launch_bounds__(768)
+gemm_rows16_pair_kernel(const uint8_t *W, const uint8_t *X, int N, int M, int nb, float *y, const float *bias, long ldy, GemmChains ch, Rows16Args grp)
+{
+    constexpr int NT = 16, G = 2, OUT = G * NT * 16;
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const int tid = threadIdx.x, nthr = blockDim.x, nwave = nthr >> 6;
+    const int lane = tid & 63, wave = wave_in_block();
+    const int i16 = lane & 15, q = lane >> 4;
+    int bid = (int)blockIdx.x;
+    if constexpr (GRP) {
+        if (bid >= grp.p[1].id0) {
+            Rows16Problem p = grp.p[1];
+            if (grp.n > 2 && bid >= grp.p[2].id0) p = grp.p[2];
+            if (grp.n > 3 && bid >= grp.p[3].id0) p = grp.p[3];
+            W = p.W; X = p.X; N = p.N; y = p.y; bias = p.bias; ldy = p.ldy; ch = p.ch;
+            bid -= p.id0;
+        }
+    }
+    const int n0 = bid * 16, t0 = (int)blockIdx.y * (G * NT);
+    const u32 xrow = (u32)nb * 292u, wpitch = (u32)nb * (u32)F::WBLOCK;
+    uint8_t *const wl = smem + wave * (16 * F::PITCH);                     /* this wave's weights */
+    float *const dxs = reinterpret_cast<float *>(smem + nwave * (16 * F::PITCH)), *const us = dxs + nb * (G * NT);
+    const int wide = TREE ? max(nb - 16, 0) : 0;                           /* leaves of more than one block */
+    /* terms: [block][output], or, of TREE, leaves wide .. 15 and then the four positions of the other leaves' blocks */
+    float *const up = us + (min(nb, 16) - wide) * OUT;
+    const uint8_t *const wbase = W + (size_t)n0 * wpitch;
+
+    constexpr int NWL = (16 * F::CHUNKS + 63) / 64;
+    u32 wsrc[NWL], wdst[NWL];
+#pragma unroll
+    for (int j = 0; j < NWL; ++j) {
+        const int e = min(64 * j + lane, 16 * F::CHUNKS - 1), r = e / F::CHUNKS, c = e % F::CHUNKS;
+        wsrc[j] = (u32)min(r, N - 1 - n0) * wpitch + F::chunk_ofs(c);
+        wdst[j] = (u32)(r * F::PITCH + 16 * c);
+    }
+    ckq_v4i wr[NWL], a[G][4];
+    u32 bs[G][2] = {}, xo[G];
+#pragma unroll
+    for (int k = 0; k < G; ++k) xo[k] = (u32)min(t0 + k * NT + i16, M - 1) * xrow;
+    auto fetch_w = [&](int b) {
+        const uint8_t *const wb = wbase + (size_t)((u32)b * (u32)F::WBLOCK);
+#pragma unroll
+        for (int j = 0; j < NWL; ++j) {
+            u32 t[4];
+            ld16<F::WBLOCK % 4 == 0 ? 4 : 2>(t, wb + wsrc[j]);
+            wr[j] = ckq_v4i{(int)t[0], (int)t[1], (int)t[2], (int)t[3]};
+        }
+    };
+    auto fetch_a = [&](int b) {
+        __builtin_amdgcn_sched_barrier(0);
+        const uint8_t *const xb = X + (size_t)((u32)b * 292u);
+#pragma unroll
+        for (int k = 0; k < G; ++k) {
+            if constexpr (F::MIN) ld8<4>(bs[k], xb + 260 + (xo[k] + 8u * (u32)q));
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                u32 t[4];
+                ld16<4>(t, xb + 4 + F::a_elem(g, 0) + (xo[k] + F::a_elem(0, q)));
+                a[k][g] = ckq_v4i{(int)t[0], (int)t[1], (int)t[2], (int)t[3]};
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const int nd = nb * (G * NT);
+    auto dx_load = [&](int e) {
+        return __builtin_bit_cast(float, ld4<4>(X + (size_t)((u32)min(t0 + (e & (G * NT - 1)), M - 1) * xrow + (u32)(e / (G * NT)) * 292u)));
+    };
+    const float dx0 = dx_load(min(tid, nd - 1)), dx1 = dx_load(min(tid + nthr, nd - 1));
+    if (wave < nb) { fetch_w(wave); fetch_a(wave); }
+    if (tid < nd) dxs[tid] = dx0;
+    if (tid + nthr < nd) dxs[tid + nthr] = dx1;
+    for (int e = tid + 2 * nthr; e < nd; e += nthr) dxs[e] = dx_load(e);
+    if constexpr (TREE) __syncthreads();
+
+    const ckq_v4i zero = {0, 0, 0, 0};
+    const uint8_t *const wrow = wl + i16 * F::PITCH;
+    auto min_mfma = [&](const int2 &am, const ckq_v4i &mins) {
+        const ckq_v4f z = {0.0f, 0.0f, 0.0f, 0.0f};
+        const ckq_v4i am4 = {am.x, am.y, 0, 0};
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(ckq_v8bf, am4), __builtin_bit_cast(ckq_v8bf, mins), z, 0, 0, 0);
+    };
+    for (int b = wave; b < nb; b += nwave) {
+#pragma unroll
+        for (int j = 0; j < NWL; ++j) *reinterpret_cast<ckq_v4i *>(wl + wdst[j]) = wr[j];
+        if (b + nwave < nb) fetch_w(b + nwave);
+        __builtin_amdgcn_sched_barrier(0);
+        Head hd;
+        F::head(hd, wrow, q);
+        int2 am[G];
+#pragma unroll
+        for (int k = 0; k < G; ++k) {
+            const int b0 = (int)bs[k][0], b1 = (int)bs[k][1], p0 = (int)(int16_t)(b0 & 0xffff) + (b0 >> 16), p1 = (int)(int16_t)(b1 & 0xffff) + (b1 >> 16);
+            am[k] = F::MIN ? int2{(int)bf16_pair((float)(p0 & 63), (float)(p1 & 63)), (int)bf16_pair((float)(64 * (p0 >> 6)), (float)(64 * (p1 >> 6)))} : int2{};
+        }
+        if constexpr (TREE) {
+            const bool apart = b < wide || b >= 16;
+            float *const u4 = up + (b < wide ? b : b - 16 + wide) * (4 * OUT) + 4 * lane;
+            float t[G][4], s01[G][4];
+            ckq_v4f dx[G];
+#pragma unroll
+            for (int k = 0; k < G; ++k) dx[k] = *reinterpret_cast<const ckq_v4f *>(dxs + b * (G * NT) + k * NT + 4 * q);
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                ckq_v4i ph, pl;
+                F::planes(ph, pl, hd, wrow, g, q);
+#pragma unroll
+                for (int k = 0; k < G; ++k) {
+                    const ckq_v4i sh = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[k][g], ph, zero, 0, 0, 0);
+                    const ckq_v4i sl = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[k][g], pl, zero, 0, 0, 0);
+                    ckq_v4f i2;
+                    if constexpr (F::MIN) i2 = min_mfma(am[k], q == g ? hd.mins : zero);
+                    float v[4];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float f = (float)((sh[r] << F::SHIFT) + sl[r]);
+                        if constexpr (F::MIN) v[r] = (hd.dw * dx[k][r]) * f - (hd.dmin * dx[k][r]) * i2[r];
+                        else                  v[r] = (hd.dw * dx[k][r]) * f;
+                        asm volatile("" : "+v"(v[r]));              /* rounded before it is added, as in the streaming kernel */
+                    }
+                    if (apart) *reinterpret_cast<float4 *>(u4 + g * OUT + k * (NT * 16)) = float4{v[0], v[1], v[2], v[3]};
+                    else {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            if (g == 0) t[k][r] = v[r];
+                            if (g == 1) s01[k][r] = t[k][r] + v[r];
+                            if (g == 2) t[k][r] = v[r];
+                            if (g == 3) t[k][r] = s01[k][r] + (t[k][r] + v[r]);
+                        }
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (!apart) {
+#pragma unroll
+                for (int k = 0; k < G; ++k) *reinterpret_cast<float4 *>(us + (b - wide) * OUT + k * (NT * 16) + 4 * lane) = float4{t[k][0], t[k][1], t[k][2], t[k][3]};
+            }
+        } else {
+            ckq_v4i sh[G], sl[G];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                ckq_v4i ph, pl;
+                F::planes(ph, pl, hd, wrow, g, q);
+#pragma unroll
+                for (int k = 0; k < G; ++k) {
+                    sh[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[k][g], ph, g ? sh[k] : zero, 0, 0, 0);
+                    sl[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[k][g], pl, g ? sl[k] : zero, 0, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int k = 0; k < G; ++k) {
+                ckq_v4f i2;
+                if constexpr (F::MIN) i2 = min_mfma(am[k], hd.mins);
+                float out[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float f = (float)((sh[k][r] << F::SHIFT) + sl[k][r]);
+                    if constexpr (F::MIN) out[r] = hd.dw * f - hd.dmin * i2[r];
+                    else                  out[r] = hd.dw * f;
+                }
+                *reinterpret_cast<float4 *>(us + b * OUT + k * (NT * 16) + 4 * lane) = float4{out[0], out[1], out[2], out[3]};
+            }
+        }
+        if (b + nwave < nb) fetch_a(b + nwave);
+    }
+    __syncthreads();
+    for (int e = tid; e < OUT; e += nthr) {        /* output e % 4 of lane e / 4 of group e / 256 */
+        const int tok = 16 * (e >> 8) + 4 * ((e >> 6) & 3) + (e & 3), n = n0 + ((e >> 2) & 15), t = t0 + tok;
+        float v = 0.0f;
+        if constexpr (TREE) {
+            float x[16];
+#pragma unroll
+            for (int l = 0; l < 16; ++l) {
+                if (l >= nb) x[l] = 0.0f;
+                else if (l >= wide) x[l] = us[(l - wide) * OUT + e];
+                else {
+                    const float *const u0 = up + l * (4 * OUT) + e, *const u1 = u0 + wide * (4 * OUT);
+                    float p[4];
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) p[g] = u0[g * OUT] + u1[g * OUT];
+                    x[l] = (p[0] + p[1]) + (p[2] + p[3]);
+                }
+            }
+#pragma unroll
+            for (int w = 1; w < 16; w *= 2)
+#pragma unroll
+                for (int l = 0; l < 16; l += 2 * w) x[l] += x[l + w];
+            v = x[0] + 0.0f;                      /* the streaming kernel adds each term to a zero */
+        } else {
+            const float *ue = us + e, *dx = dxs + tok;
+            for (int sp = 0; sp < ch.splits; ++sp) {
+                const int b0 = sp * ch.per, b1 = min(nb, b0 + ch.per);
+                float c[2] = {0.0f, 0.0f};
+                for (int b = b0; b < b1; b += 4) {
+                    float uu[4], dd[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const int bk = min(b + k, b1 - 1);
+                        uu[k] = ue[bk * OUT];
+                        dd[k] = dx[bk * (G * NT)];
+                    }
+                    if (ch.kg == 2) {
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) c[k & 1] = b + k < b1 ? fmaf(dd[k], uu[k], c[k & 1]) : c[k & 1];
+                    } else {
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) c[0] = b + k < b1 ? fmaf(dd[k], uu[k], c[0]) : c[0];
+                    }
+                }
+                if (ch.kg == 2) c[0] += c[1];
+                v = sp ? v + c[0] : c[0];
+            }
+        }
+        if (n < N && t < M) y[(size_t)t * ldy + n] = bias ? v + bias[n] : v;
+    }
+}
+
 /* Short rows, several token groups: a block has a wave for every 256-block of its 16 rows (at most KEEP_NB of them) and goes
  * through `per` groups of 16 tokens, the planes and scales of its weights formed once and kept in registers.  The first kernel
  * forms them again for every group, and they are a good third of what bounds it there, VALU issue (Q5_K, 93 tokens: 480 vector
@@ -1004,6 +1229,55 @@ int launch_rows16_hold(Rows16Args &a, int tiles, int grid, int round, size_t lds
     return (int)hipGetLastError();
 }
 
+/* Waves and LDS of a launch of the kernel that takes groups in pairs; 0: another kernel.  From 420 launches of both, 17 to 130 tokens, rows of 9 to 43 blocks
+ * (Q4_K 5): as long as a block for every group and row tile finds a CU of its own it loses (0.69-1.0, two groups in a row where there
+ * could be two CUs), past that it wins while the pairs still do: Q4_K 1.01-1.36, Q5_K 1.12-1.45, Q6_K 1.22-1.67, in the streaming kernel's order 0.99-1.15 (there twelve waves
+ * are 2-4 % ahead of eight).  With more pairs than CUs, eight waves: Q6_K 1.18-1.37 on average (0.94-1.61), Q5_K 1.07-1.16 but for three groups, 0.97;
+ * Q4_K, whose planes are quickly formed, 0.92-1.09, and the streaming kernel's order 0.72-0.83.  Rows of which only one such block fits a CU lose too
+ * (Q5_K 914 x 7168 at 175: tile kernel 18.6, this 23.2). */
+int rows16_pair_waves(int fmt, bool tree, long tiles, int groups, int nb, size_t *lds)
+{
+    const int wide = tree && nb > 16 ? nb - 16 : 0;
+    const long pairs = tiles * ((groups + 1) / 2);
+    if (groups < 2 || groups > 1 << 10 || tiles * groups <= 256 || wide > 16) return 0;
+    if (pairs > 256 && (tree || fmt == CKQ_FMT_Q4_K || (fmt == CKQ_FMT_Q5_K && groups == 3))) return 0;
+    const int waves = std::min(pairs <= 256 ? 12 : 8, nb);
+    const size_t pitch = fmt == CKQ_FMT_Q4_K ? R16Q4K::PITCH : fmt == CKQ_FMT_Q5_K ? R16Q5K::PITCH : R16Q6K::PITCH;
+    const size_t terms = tree ? (size_t)(std::min(nb, 16) - wide) + 8 * wide : (size_t)nb;
+    *lds = waves * (16 * pitch) + (size_t)nb * 128 + terms * 2048;
+    return *lds > (pairs > 256 ? 80 : 160) * 1024 ? 0 : waves;
+}
+
+template <class F, bool TREE>
+int launch_rows16_pair(Rows16Args &a, int waves, size_t lds, hipStream_t s)
+{
+    unsigned grid = 0;
+    for (int i = 0; i < a.n; ++i) {
+        a.p[i].id0 = (int)grid;
+        grid += (unsigned)((a.p[i].N + 15) / 16);
+    }
+    const unsigned gy = (unsigned)((a.M + 31) / 32);
+    if (lds > 64 * 1024) {
+        static std::atomic<uint64_t> done[2];      /* as in launch_rows16_nt */
+        int dev = 0;
+        hipError_t e = hipGetDevice(&dev);
+        if (e != hipSuccess) return (int)e;
+        const uint64_t bit = 1ull << (dev & 63);
+        if (!(done[a.n > 1].load(std::memory_order_acquire) & bit)) {
+            e = hipFuncSetAttribute(a.n > 1 ? (const void *)gemm_rows16_pair_kernel<F, TREE, true> : (const void *)gemm_rows16_pair_kernel<F, TREE, false>,
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+            if (e != hipSuccess) return (int)e;
+            done[a.n > 1].fetch_or(bit, std::memory_order_release);
+        }
+    }
+    const Rows16Problem &p = a.p[0];
+    if (a.n > 1)
+        hipLaunchKernelGGL((gemm_rows16_pair_kernel<F, TREE, true>), dim3(grid, gy), dim3((unsigned)(64 * waves)), lds, s, p.W, p.X, p.N, a.M, a.nb, p.y, p.bias, p.ldy, p.ch, a);
+    else
+        hipLaunchKernelGGL((gemm_rows16_pair_kernel<F, TREE, false>), dim3(grid, gy), dim3((unsigned)(64 * waves)), lds, s, p.W, p.X, p.N, a.M, a.nb, p.y, p.bias, p.ldy, p.ch, a);
+    return (int)hipGetLastError();
+}
+
 template <class F>
 int launch_rows16(int fmt, Rows16Args &a, hipStream_t s)
 {
@@ -1017,6 +1291,8 @@ int launch_rows16(int fmt, Rows16Args &a, hipStream_t s)
     size_t lds;
     if (tiles < 1 << 20 && rows16_hold<F>(a, a.tree, (int)tiles, &grid, &round, &lds))
         return a.tree ? launch_rows16_hold<F, true>(a, (int)tiles, grid, round, lds, s) : launch_rows16_hold<F, false>(a, (int)tiles, grid, round, lds, s);
+    if (const int waves = rows16_pair_waves(fmt, a.tree, tiles, (a.M + 15) / 16, a.nb, &lds))
+        return a.tree ? launch_rows16_pair<F, true>(a, waves, lds, s) : launch_rows16_pair<F, false>(a, waves, lds, s);
     if (a.tree) return a.M <= 8 ? launch_rows16_nt<F, 8, true>(a, s) : launch_rows16_nt<F, 16, true>(a, s);
     return launch_rows16_nt<F, 16, false>(a, s);           /* the tile kernels start above eight tokens */
 }
@@ -1027,6 +1303,17 @@ float gemm_rows16_keep_time(int fmt, size_t rows, int ntok, int nb)
 {
     float t = 0.0f;
     return rows16_keep_parts(fmt, (long)((rows + 15) / 16), (ntok + 15) / 16, nb, &t) ? t : 0.0f;
+}
+
+/* Fitted to the launches of the rule above in the tile kernels' order, 12-15 % rms. */
+float gemm_rows16_pair_time(int fmt, size_t rows, int ntok, int nb)
+{
+    static const float fit[3][3] = {{3.2f, 0.04f, 0.27f}, {3.4f, 0.11f, 0.29f}, {2.6f, 0.09f, 0.30f}};
+    size_t lds;
+    const long tiles = (long)((rows + 15) / 16), groups = (ntok + 15) / 16;
+    if (tiles > 1 << 20 || !rows16_pair_waves(fmt, false, tiles, (int)groups, nb, &lds)) return 0.0f;
+    const float *f = fit[fmt == CKQ_FMT_Q4_K ? 0 : fmt == CKQ_FMT_Q5_K ? 1 : 2], on_cu = (float)(tiles * ((groups + 1) / 2)) / 256.0f;
+    return f[0] + (f[1] + f[2] * fmaxf(on_cu, 1.0f)) * (float)nb;
 }
 
 int launch_gemm_rows16(int fmt, Rows16Args &a, hipStream_t s)

@@ -45,6 +45,8 @@ struct Rows16Args {
 };
 /* Estimated time in us of such a launch where its kernel for short rows and several token groups runs, else 0. */
 float gemm_rows16_keep_time(int fmt, size_t rows, int ntok, int nb);
+/* The same for its kernel that takes token groups in pairs, in the order of the tile kernels. */
+float gemm_rows16_pair_time(int fmt, size_t rows, int ntok, int nb);
 /* One launch over a.n problems of one format, width and token count (id0 is filled in). */
 int launch_gemm_rows16(int fmt, Rows16Args &a, hipStream_t s);
 constexpr int ROWS16_MAX_K = 64 * 256;      /* the terms of a longer row would not fit the LDS */

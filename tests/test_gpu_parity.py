@@ -1744,6 +1744,52 @@ def test_16_row_tiles_of_several_token_groups_copied_to_lds(fmt):
 
 
 @pytest.mark.parametrize("fmt", ["q4_k", "q5_k", "q6_k"])
+def test_16_row_tiles_of_token_groups_in_pairs(fmt):
+    """Longer rows, two token groups a block: an even and an odd number of groups, a last group of one token, ragged rows, fewer blocks of the row than
+    waves and more, row tiles that just have a CU each as pairs and ones that do not; in the tile kernels' order bit for bit what they
+    give, in the streaming kernel's what one token at a time gives, with no, some and all but a few positions that hold two blocks of the row."""
+    import torch
+    L = ckq.lib()
+    tag = P.FMT[fmt]
+    try:
+        for M, N, K in [(32, 4096, 9 * 256), (33, 3003, 11 * 256), (64, 2039, 16 * 256), (93, 1024, 19 * 256), (17, 4095, 20 * 256), (50, 1500, 24 * 256), (32, 2100, 43 * 256),
+                        (70, 9000, 10 * 256), (40, 6001, 16 * 256), (64, 5000, 19 * 256), (129, 700, 9 * 256)]:
+            xq = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, seed=M)), "q8_k", rows=M)
+            W, bias = P.to_device(T.random_blocks(fmt, N * K // 256, 9480 + M)), P.to_device(T.normal(N, 0.0, 0.5, seed=N))
+            say("16-row tiles, token groups in pairs", fmt, M, N, K)
+
+            def call(policy, forced):
+                L.ckq_set_prefill_variant(tag, 16 if forced else 0)
+                L.ckq_set_gemm_policy(policy)
+                c = torch.full((M, N + 3), 7.0, device="cuda")
+                P.check(L.ckq_gemm_nt_dev(tag, P._dp(xq), P._dp(W), P._dp(bias), P._dp(c), M, N, K, N + 3, P._stream()), "ckq_gemm_nt_dev")
+                assert bool((c[:, N:] == 7.0).all()), (M, N, K)
+                return c[:, :N]
+            tree, chain, tiles = call(2, True), call(1, True), call(1, False)
+            assert torch.equal(chain, tiles), (M, N, K)
+            L.ckq_set_prefill_variant(tag, 0)
+            L.ckq_set_gemm_policy(0)
+            rb = xq.numel() // M
+            for m in {0, 15, 16, M // 2, M - 1}:
+                one = P.dev_gemm_nt(fmt, xq[m * rb:(m + 1) * rb].clone(), W, bias, 1, N, K)
+                assert torch.equal(tree[m], one.view(N)), (M, N, K, m)
+        M, K, Ns = 40, 4096, [3000, 700, 333]
+        xq = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, seed=6)), "q8_k", rows=M)
+        Ws = [P.to_device(T.random_blocks(fmt, n * K // 256, 9490 + i)) for i, n in enumerate(Ns)]
+        for policy in (2, 1, 0):
+            L.ckq_set_prefill_variant(tag, 16)
+            L.ckq_set_gemm_policy(policy)
+            ys = [torch.zeros(M, n, dtype=torch.float32, device="cuda") for n in Ns]
+            say("16-row tiles, token groups in pairs, grouped", fmt, policy)
+            P.dev_matmul_sequence([(fmt, xq, W, None, y, M, n, K) for W, y, n in zip(Ws, ys, Ns)])
+            for W, y, n in zip(Ws, ys, Ns):
+                assert torch.allclose(y, P.dev_gemm_nt(fmt, xq, W, None, M, n, K).view(M, n), rtol=0, atol=2e-6 * float(y.abs().max())), (policy, n)
+    finally:
+        L.ckq_set_gemm_policy(0)
+        L.ckq_set_prefill_variant(tag, 0)
+
+
+@pytest.mark.parametrize("fmt", ["q4_k", "q5_k", "q6_k"])
 def test_16_row_tiles_with_held_activations(fmt):
     """The kernel that goes through several row tiles with its activations in registers: one wave a block and sixteen, blocks of one
     tile, of some more than others and of several rounds of the tiles whose terms fit the LDS, last tiles that start early (row counts
