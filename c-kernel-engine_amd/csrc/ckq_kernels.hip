@@ -289,9 +289,9 @@ static bool weights_dword_aligned(const GemvArgs &a, const GemvGroup &grp)
  * shapes up to a third (Q6_K 14911 x 1536 at 75 tokens: 22, tiles 17; Q4_K 4556 x 9984 at 30: 22, tiles 18):
  *   rows16     3.6 + 0.12 nb + (Q4_K 0.36, Q5_K 0.65, Q6_K 0.71) n16; up to 256 tokens of short rows gemm_rows16_keep_time
  *              (Q5_K 4864 x 1024 at 192 tokens: 10.3, tiles 13.7; 4096 x 2048 at 256: 17.2, tiles 19.5); groups of tokens in pairs gemm_rows16_pair_time
- *   tiles      Q4_K 11 + 0.2 mb + 0.0015 tokens mb, an under-estimate almost everywhere; Q5_K 13.3 + 0.164 mb + 0.0048 tokens mb and
- *              Q6_K 13.8 + 0.083 mb + 0.0044 tokens mb (11 % rms over 207 launches of 9 to 200 tokens; with Q4_K's these two cost 4.1 and 7.3 % more
- *              than the faster kernel, so 1.5 and 0.6; Q4_K's own fit would cost 5.2 instead of 1.0)
+ *   tiles      11 + 0.2 mb + 0.0015 tokens mb, an under-estimate almost everywhere; against groups in pairs Q5_K 13.3 + 0.164 mb + 0.0048 tokens mb and
+ *              Q6_K 13.8 + 0.083 mb + 0.0044 tokens mb (11 % rms over 207 launches of 9 to 200 tokens, where the first cost 4.1 and 7.3 % more than the
+ *              faster kernel and these cost 1.5 and 0.6; Q4_K's own fit would cost 5.2 instead of 1.0)
  *   streaming  above eight tokens the larger of 2.9 and 2.2 + 0.0075 lanes + (23.5, 23.5, 29) million lanes of all rows and passes,
  *              a row's 64-element positions being dealt to 8, 16, 32 or 64 lanes or to 2 to 4 passes of 64 (stream_lanes): small
  *              matrices stream at up to some 60 tokens (Q5_K 290 x 1792 at 25: 3.0, here 4.6; Q6_K 435 x 1536 at 13 3.0, here 4.8);
@@ -330,7 +330,7 @@ static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles, int l
     const float t_pair = tiles && t_keep <= 0.0f ? gemm_rows16_pair_time(fmt, rows, ntok, K / 256) : 0.0f;
     const float t_rows = t_keep > 0.0f ? t_keep : t_pair > 0.0f ? t_pair : 3.6f + 0.12f * nb + per_block[f] * 1e-3f * nb * (float)((rows + 15) / 16) * (float)((ntok + 15) / 16);
     float t_else;
-    if (tiles) t_else = f == 0 ? 11.0f + (0.2f + 0.0015f * (float)ntok) * mb : f == 1 ? 13.3f + (0.164f + 0.0048f * (float)ntok) * mb : 13.8f + (0.083f + 0.0044f * (float)ntok) * mb;
+    if (tiles) t_else = f == 0 || t_pair <= 0.0f ? 11.0f + (0.2f + 0.0015f * (float)ntok) * mb : f == 1 ? 13.3f + (0.164f + 0.0048f * (float)ntok) * mb : 13.8f + (0.083f + 0.0044f * (float)ntok) * mb;
     else if (ntok <= 8) t_else = fmaxf(3.5f + 0.07f * nb, 3.05f + 0.11f * nb + 1.25f * per_pass[f] * mb);
     else {
         const float t_launch = 2.2f + 0.0075f * (float)lanes;
