@@ -888,34 +888,33 @@ extern "C" int ckq_launch_quantize_gemv_q8_0(int fmt, const float *x, void *xq, 
  * maximum goes through DPP, and x stays in registers: 4096 wide, one row 5.1 -> 4.2 us, 512 rows 7.1 -> 6.0,
  * 2048 rows 23.3 -> 12.1.
  */
-template <int GREG, bool ALONE>
+template <int GREG, bool AHEAD>
 __global__ void __launch_bounds__(1024) rmsnorm_q8_k_fused_kernel(const float *__restrict__ input, const float *__restrict__ gamma,
                                                                   uint8_t *__restrict__ y, int d_model, long in_stride, float eps)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    rms_row<GREG, ALONE>(input + (size_t)blockIdx.x * in_stride, gamma, y + (size_t)blockIdx.x * (d_model / 256) * 292,
+    rms_row<GREG, AHEAD>(input + (size_t)blockIdx.x * in_stride, gamma, y + (size_t)blockIdx.x * (d_model / 256) * 292,
                   d_model, eps, reinterpret_cast<float *>(smem));
 }
 
-constexpr int RMS_FEW_TOKENS = 512;
-template <int GREG, bool ALONE>
+template <int GREG, bool AHEAD>
 static int launch_rms_form(const float *input, const float *gamma, uint8_t *y, int tokens, int d_model, long stride, float eps, int waves, hipStream_t s)
 {
     const size_t lds = rms_lds_bytes((size_t)d_model);
     if (lds > 64 * 1024) {
         /* more than 64 KB of dynamic LDS is an opt-in per function and per device: set on every
          * such call for the device that is current (rows this long are rare; the call is cheap) */
-        hipError_t e = hipFuncSetAttribute((const void *)rmsnorm_q8_k_fused_kernel<GREG, ALONE>,
+        hipError_t e = hipFuncSetAttribute((const void *)rmsnorm_q8_k_fused_kernel<GREG, AHEAD>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         if (e != hipSuccess) return (int)e;
     }
-    hipLaunchKernelGGL((rmsnorm_q8_k_fused_kernel<GREG, ALONE>), dim3((unsigned)tokens), dim3(64 * waves), lds, s, input, gamma, y, d_model, stride, eps);
+    hipLaunchKernelGGL((rmsnorm_q8_k_fused_kernel<GREG, AHEAD>), dim3((unsigned)tokens), dim3(64 * waves), lds, s, input, gamma, y, d_model, stride, eps);
     return (int)hipGetLastError();
 }
 template <int GREG>
 static int launch_rms(const float *input, const float *gamma, uint8_t *y, int tokens, int d_model, long stride, float eps, int waves, hipStream_t s)
 {
-    return tokens <= 256 ? launch_rms_form<GREG, true>(input, gamma, y, tokens, d_model, stride, eps, waves, s)
+    return tokens <= 512 ? launch_rms_form<GREG, true>(input, gamma, y, tokens, d_model, stride, eps, waves, s)
                          : launch_rms_form<GREG, false>(input, gamma, y, tokens, d_model, stride, eps, waves, s);
 }
 
@@ -925,10 +924,12 @@ extern "C" int ckq_launch_rmsnorm_q8_k_fused(const float *input, const float *ga
     if (!input || !gamma || !y || tokens <= 0 || d_model <= 0 || aligned_embed_dim < d_model) return CKQ_EINVAL;
     if (d_model % 256 || aligned_embed_dim % 4) return CKQ_ESHAPE;
     if (rms_lds_bytes((size_t)d_model) > 160 * 1024) return CKQ_ESHAPE;        /* the row is staged in LDS */
-    /* A wave for every 256-block of the row, up to sixteen, while the rows have the chip to themselves: two such blocks fit a
-     * CU.  More rows than that take four waves each, or their serial chains would run in rounds of two per CU (4096 wide, sixteen
-     * waves against four: 513 rows 8.0 us against 6.5, 1024 rows 10.3 against 7.8, 2048 rows 19.4 against 12.1). */
-    const int nb = d_model / 256, most = tokens <= RMS_FEW_TOKENS ? 16 : 4, waves = nb < most ? nb : most, per = (nb + waves - 1) / waves;
+    /* A wave for every 256-block of the row, up to sixteen while a row has a CU to itself, up to eight for two and four rows on a CU, whose chains
+     * then run side by side.  More rows take four waves each, so that more of them fit, unless their image in LDS leaves room for four anyway (8192 and wider).  The
+     * chains read ahead up to two rows a CU.  us, up to 512 rows sixteen waves without reading ahead -> eight with it: 4096 wide 300 rows 6.6 -> 6.2,
+     * 512 rows 7.1 -> 6.5, 8192 wide 512 rows 11.8 -> 11.1, 2048 wide 4.4 -> 4.2; beyond, four -> eight: 700 rows, 4096 wide 7.9 -> 7.6, 8192 wide
+     * 15.7 -> 13.1, 2048 rows of 8192 32.2 -> 28.1 (eight: of 4096 13.7 -> 15.0, 1500 rows of 6144 17.0 -> 17.8). */
+    const int nb = d_model / 256, most = tokens <= 256 ? 16 : tokens <= 1024 || nb >= 32 ? 8 : 4, waves = nb < most ? nb : most, per = (nb + waves - 1) / waves;
     uint8_t *const out = (uint8_t *)y;
     hipStream_t const s = (hipStream_t)stream;
     if (per == 1) return launch_rms<1>(input, gamma, out, tokens, d_model, (long)aligned_embed_dim, eps, waves, s);

@@ -90,13 +90,13 @@ __device__ __forceinline__ void rms_chain(float *xs, int D, int j)
     xs[8 * rms_pitch(D) + j] = acc;
 }
 
-/* The same for a row that has its CU to itself.  A multiply-add of the chain takes some eight cycles, and the values should be there
+/* The same for rows that share their CU with one other at most.  A multiply-add of the chain takes some eight cycles, and the values should be there
  * before it: 32 are read while the 32 before them are added.  The reads are volatile because the compiler moves ordinary ones to
  * where they are used, as it does above, where every 32 values wait for LDS.  4096 wide, one row 4.2 -> 3.9 us, 256 rows 5.4 -> 5.1, 8192 wide 7.2 -> 6.3; but
- * the 64 registers keep a second block of sixteen waves off the CU (512 rows 6.8 -> 8.5).  Sixteen values ahead 4.1 and 6.8; a ring of
+ * the 64 registers keep a second block of sixteen waves off the CU (512 rows 6.8 -> 8.5, of eight waves 6.9 -> 6.5).  Sixteen values ahead 4.1 and 6.8; a ring of
  * 32 filled four at a time 4.4 and 7.3; whole waves, a chain to every sixteen lanes that broadcast it their values, 4.4 and 7.0. */
 typedef float rms_v4f __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ void rms_chain_alone(float *xs, int D, int j)
+__device__ __forceinline__ void rms_chain_ahead(float *xs, int D, int j)
 {
     typedef const volatile __attribute__((address_space(3))) rms_v4f *lds_ptr;
     const lds_ptr x = (lds_ptr)(const rms_v4f *)(xs + j * rms_pitch(D));
@@ -165,8 +165,8 @@ __device__ __forceinline__ void rms_quant_block(const float4 xv, const float4 gv
 
 /* A block of nw waves turns row x (D floats) into its D/256 Q8_K blocks at y.  Wave w owns 256-blocks w, w + nw, ...;
  * the x and gamma of its first GREG blocks are loaded at the start and kept in registers across the chain, so a row of
- * up to GREG * nw blocks costs one round trip to memory.  ALONE: there is no more than one row for a CU.  smem: rms_lds_bytes(D). */
-template <int GREG, bool ALONE>
+ * up to GREG * nw blocks costs one round trip to memory.  AHEAD: which form of the chain.  smem: rms_lds_bytes(D). */
+template <int GREG, bool AHEAD>
 __device__ __forceinline__ void rms_row(const float *__restrict__ x, const float *__restrict__ gamma,
                                         uint8_t *__restrict__ y, int D, float eps, float *xs)
 {
@@ -183,7 +183,7 @@ __device__ __forceinline__ void rms_row(const float *__restrict__ x, const float
     for (int b = wave + nw * GREG; b < nb; b += nw) rms_stage(xs, D, b, lane, reinterpret_cast<const float4 *>(x + 256 * b)[lane]);
     __syncthreads();
     if (tid < 8) {
-        if constexpr (ALONE) rms_chain_alone(xs, D, tid);
+        if constexpr (AHEAD) rms_chain_ahead(xs, D, tid);
         else                 rms_chain(xs, D, tid);
     }
     __syncthreads();

@@ -482,6 +482,17 @@ def test_rmsnorm_q8_k_fused_rows_alone_on_their_cu_bit_exact(tokens, D):
     assert np.array_equal(P.dev_rmsnorm_q8_k_fused(P.to_device(x), P.to_device(g), tokens, D).cpu().numpy(), ref)
 
 
+@pytest.mark.parametrize("tokens,D", [(257, 256), (512, 2304), (512, 4096), (513, 2048), (513, 4352), (700, 8192), (1024, 4096), (1025, 2304), (1025, 8192), (300, 16640)])
+def test_rmsnorm_q8_k_fused_rows_that_share_a_cu_bit_exact(tokens, D):
+    """More rows than CUs: eight waves a row and four, with and without reading ahead, rows of fewer blocks than waves, of a multiple and of some
+    more, rows whose LDS image leaves room for four of them, and one that takes the CU for itself."""
+    x, g = T.normal(tokens * D, 0.1, 1.0, seed=D), T.normal(D, 1.0, 0.3, seed=D + 1)
+    say("rmsnorm_q8_k_fused, rows that share a CU", tokens, D)
+    ref = np.zeros(tokens * (D // 256) * 292, np.uint8)
+    T.oracle().orc_rmsnorm_q8_k_fused(T.ptr(x), T.ptr(g), T.ptr(ref), tokens, D, D, ctypes.c_float(1e-6))
+    assert np.array_equal(P.dev_rmsnorm_q8_k_fused(P.to_device(x), P.to_device(g), tokens, D).cpu().numpy(), ref)
+
+
 # ---- row dequantizers and quantized embedding lookup, bit-exact -----------------------------
 
 @pytest.mark.parametrize("fmt", ["q4_k", "q6_k", "q8_0"])
