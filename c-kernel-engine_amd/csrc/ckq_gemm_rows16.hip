@@ -1082,16 +1082,19 @@ gemm_rows16_keep_kernel(const uint8_t *W, const uint8_t *X, int N, int M, int pa
 }
 
 /* Waves per block: with two tiles per CU and more, blocks of four waves overlap each other's beginnings and ends
- * (32000 x 4096, 13 tokens: 27 us, with eight 41); with fewer, a tile's blocks spread over more waves. */
-int rows16_waves(int tiles, int nb)
+ * (32000 x 4096, 13 tokens: 27 us, with eight 41); with fewer, a tile's blocks spread over more waves.  A tile alone on its CU takes twelve
+ * for rows of more than twelve 256-blocks: 44 launches of 64 to 256 tiles 1.02 on average, up to 1.11 (us, eight -> twelve: Q4_K 4096 x 4096 at 13
+ * tokens 7.08 -> 6.81, Q5_K 3568 x 5888 10.2 -> 9.2, Q6_K 2048 x 5632 10.5 -> 9.3; sixteen 1.017; up to twelve blocks 0.98); but Q6_K rows of more than 32, whose
+ * blocks come in more bytes, 0.97 (704 x 10496 at 15 14.6 -> 15.2). */
+int rows16_waves(int fmt, int tiles, int nb)
 {
-    int waves = tiles >= 512 ? 4 : tiles > 64 ? 8 : 16;
+    int waves = tiles >= 512 ? 4 : tiles > 256 ? 8 : tiles > 64 ? (nb > 12 && (fmt != CKQ_FMT_Q6_K || nb <= 32) ? 12 : 8) : 16;
     while (waves > 4 && waves / 2 >= nb) waves /= 2;
     return waves;
 }
 
 template <class F, int NT, bool TREE>
-int launch_rows16_nt(Rows16Args &a, hipStream_t s)
+int launch_rows16_nt(int fmt, Rows16Args &a, hipStream_t s)
 {
     unsigned grid = 0;
     for (int i = 0; i < a.n; ++i) {
@@ -1101,7 +1104,7 @@ int launch_rows16_nt(Rows16Args &a, hipStream_t s)
     const unsigned gy = (unsigned)((a.M + NT - 1) / NT);
     if (gy > 65535) return CKQ_ESHAPE;
     auto lds_bytes = [&](int w) { return (size_t)w * rows16_wave_lds<F, NT>() + (size_t)(TREE && a.nb > 16 ? 16 : a.nb) * (NT * 64) + (size_t)a.nb * (NT * 4); };
-    int waves = rows16_waves((int)(grid * gy), TREE ? (a.nb < 16 ? a.nb : 16) : a.nb);
+    int waves = rows16_waves(fmt, (int)(grid * gy), TREE ? (a.nb < 16 ? a.nb : 16) : a.nb);
     while (waves > 4 && lds_bytes(waves) > 160 * 1024) waves -= 4;
     const size_t lds = lds_bytes(waves);
     if (lds > 160 * 1024) return CKQ_ESHAPE;
@@ -1293,8 +1296,8 @@ int launch_rows16(int fmt, Rows16Args &a, hipStream_t s)
         return a.tree ? launch_rows16_hold<F, true>(a, (int)tiles, grid, round, lds, s) : launch_rows16_hold<F, false>(a, (int)tiles, grid, round, lds, s);
     if (const int waves = rows16_pair_waves(fmt, a.tree, tiles, (a.M + 15) / 16, a.nb, &lds))
         return a.tree ? launch_rows16_pair<F, true>(a, waves, lds, s) : launch_rows16_pair<F, false>(a, waves, lds, s);
-    if (a.tree) return a.M <= 8 ? launch_rows16_nt<F, 8, true>(a, s) : launch_rows16_nt<F, 16, true>(a, s);
-    return launch_rows16_nt<F, 16, false>(a, s);           /* the tile kernels start above eight tokens */
+    if (a.tree) return a.M <= 8 ? launch_rows16_nt<F, 8, true>(fmt, a, s) : launch_rows16_nt<F, 16, true>(fmt, a, s);
+    return launch_rows16_nt<F, 16, false>(fmt, a, s);           /* the tile kernels start above eight tokens */
 }
 
 } // namespace

@@ -1755,6 +1755,43 @@ def test_16_row_tiles_of_several_token_groups_copied_to_lds(fmt):
 
 
 @pytest.mark.parametrize("fmt", ["q4_k", "q5_k", "q6_k"])
+def test_16_row_tiles_alone_on_their_cu(fmt):
+    """Row tiles that have a CU each, one token group and rows too few for groups in pairs: blocks of eight waves, of twelve and (rows longer than
+    the LDS has room for) in between; fewer 256-blocks than waves in the last turn, one, and none.  In the tile kernels' order bit for bit what
+    they give, in the streaming kernel's what one token at a time gives."""
+    import torch
+    L = ckq.lib()
+    tag = P.FMT[fmt]
+    try:
+        for M, N, K in [(13, 1500, 12 * 256), (16, 1040, 13 * 256), (9, 4096, 16 * 256), (40, 1033, 17 * 256), (13, 2048, 24 * 256), (8, 1100, 25 * 256), (15, 1056, 32 * 256),
+                        (13, 1056, 33 * 256), (12, 1200, 43 * 256), (11, 1200, 64 * 256)]:
+            xq = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, seed=M)), "q8_k", rows=M)
+            W, bias = P.to_device(T.random_blocks(fmt, N * K // 256, 9520 + M)), P.to_device(T.normal(N, 0.0, 0.5, seed=N))
+            say("16-row tiles, alone on their CU", fmt, M, N, K)
+
+            def call(policy, forced):
+                L.ckq_set_prefill_variant(tag, 16 if forced else 0)
+                L.ckq_set_gemm_policy(policy)
+                c = torch.full((M, N + 3), 7.0, device="cuda")
+                P.check(L.ckq_gemm_nt_dev(tag, P._dp(xq), P._dp(W), P._dp(bias), P._dp(c), M, N, K, N + 3, P._stream()), "ckq_gemm_nt_dev")
+                assert bool((c[:, N:] == 7.0).all()), (M, N, K)
+                return c[:, :N]
+            tree = call(2, True)
+            if M > 8:
+                chain, tiles = call(1, True), call(1, False)
+                assert torch.equal(chain, tiles), (M, N, K)
+            L.ckq_set_prefill_variant(tag, 0)
+            L.ckq_set_gemm_policy(0)
+            rb = xq.numel() // M
+            for m in {0, M // 2, M - 1}:
+                one = P.dev_gemm_nt(fmt, xq[m * rb:(m + 1) * rb].clone(), W, bias, 1, N, K)
+                assert torch.equal(tree[m], one.view(N)), (M, N, K, m)
+    finally:
+        L.ckq_set_gemm_policy(0)
+        L.ckq_set_prefill_variant(tag, 0)
+
+
+@pytest.mark.parametrize("fmt", ["q4_k", "q5_k", "q6_k"])
 def test_16_row_tiles_of_token_groups_in_pairs(fmt):
     """Longer rows, two token groups a block: an even and an odd number of groups, a last group of one token, ragged rows, fewer blocks of the row than
     waves and more, row tiles that just have a CU each as pairs and ones that do not; in the tile kernels' order bit for bit what they
