@@ -234,22 +234,25 @@ enum { PTR_CACHE = 64 };
 static const void *g_host_ptr[PTR_CACHE];
 static void ptr_cache_clear(void) { memset(g_host_ptr, 0, sizeof g_host_ptr); }
 
-static int is_device_ptr(const void *p)
+enum { PTR_HOST = 0, PTR_DEVICE, PTR_MANAGED };
+static int ptr_kind(const void *p)
 {
     const size_t slot = ((uintptr_t)p >> 6) % PTR_CACHE;
-    if (p && g_host_ptr[slot] == p) return 0;
+    if (p && g_host_ptr[slot] == p) return PTR_HOST;
     hipPointerAttribute_t at;
     memset(&at, 0, sizeof(at));
     hipError_t e = hipPointerGetAttributes(&at, p);
     if (e != hipSuccess) {
         (void)hipGetLastError(); /* plain host memory: clear the sticky error */
         g_host_ptr[slot] = p;
-        return 0;
+        return PTR_HOST;
     }
-    if (at.type == hipMemoryTypeDevice || at.type == hipMemoryTypeManaged) return 1;
+    if (at.type == hipMemoryTypeDevice) return PTR_DEVICE;
+    if (at.type == hipMemoryTypeManaged) return PTR_MANAGED;
     if (at.type == hipMemoryTypeUnregistered) g_host_ptr[slot] = p;
-    return 0;
+    return PTR_HOST;
 }
+static int is_device_ptr(const void *p) { return ptr_kind(p) != PTR_HOST; }
 
 /* Waits for the work enqueued on the library's stream so far. */
 static int stream_wait(void)
@@ -282,6 +285,16 @@ static int stream_wait(void)
             g_done_ok = 0;
         }
     }
+    HIP_TRY(hipStreamSynchronize(g_stream));
+    return 0;
+}
+
+/* The same where the results are in the caller's own memory.  Device memory is read by the GPU and its copy engines, which see what a kernel has
+ * written once it has ended; managed memory the CPU may read as well, which only the synchronisation call promises.  The word instead of
+ * that call: fused MLP of 512 tokens, 896 x 4864 65.3 -> 62.9 us. */
+static int result_wait(int kind)
+{
+    if (kind == PTR_DEVICE) return stream_wait();
     HIP_TRY(hipStreamSynchronize(g_stream));
     return 0;
 }
@@ -876,8 +889,7 @@ static void matmul_locked(int fmt, const void *A, const void *B, const float *bi
             if (stage_out_sync(BUF_Y, C + row0, (size_t)ldc * sizeof(float), (size_t)ld * sizeof(float),
                                (size_t)(row1 - row0) * sizeof(float), (size_t)ntok)) break;
         } else {
-            hipError_t e = hipStreamSynchronize(g_stream);
-            if (e != hipSuccess) { fail((int)e, "hipStreamSynchronize"); break; }
+            if (result_wait(c_on_dev)) break;
         }
         done = 1;
     } while (0);
@@ -940,8 +952,7 @@ static void host_quantize(int q8k, const float *x, void *y, int rows, int k)
         } else if (!y_on_dev) {
             if (stage_out_sync(BUF_Y, y, out_bytes, out_bytes, out_bytes, 1)) break;
         } else {
-            hipError_t e = hipStreamSynchronize(g_stream);
-            if (e != hipSuccess) { fail((int)e, "hipStreamSynchronize"); break; }
+            if (result_wait(y_on_dev)) break;
         }
         done = 1;
     } while (0);
@@ -1119,8 +1130,7 @@ static void host_dequant_rows(int fmt, const void *table, size_t table_rows, con
         if (!on_dev) {
             if (stage_out_sync(BUF_Y, out, out_bytes, out_bytes, out_bytes, 1)) break;
         } else {
-            hipError_t e = hipStreamSynchronize(g_stream);
-            if (e != hipSuccess) { fail((int)e, "hipStreamSynchronize"); break; }
+            if (result_wait(on_dev)) break;
         }
         done = 1;
     } while (0);
@@ -1184,8 +1194,7 @@ void rmsnorm_q8_k_fused(const float *input, const float *gamma, void *vy, int to
         if (!y_on_dev) {
             if (stage_out_sync(BUF_Y, vy, out_bytes, out_bytes, out_bytes, 1)) break;
         } else {
-            hipError_t e = hipStreamSynchronize(g_stream);
-            if (e != hipSuccess) { fail((int)e, "hipStreamSynchronize"); break; }
+            if (result_wait(y_on_dev)) break;
         }
         done = 1;
     } while (0);
@@ -1257,8 +1266,7 @@ void fused_mlp_swiglu_prefill_w1w2_quant(const float *x, const void *W1, const f
         if (!out_on_dev) {
             if (stage_out_sync(BUF_Y, output, out_bytes, out_bytes, out_bytes, 1)) break;
         } else {
-            hipError_t e = hipStreamSynchronize(g_stream);
-            if (e != hipSuccess) { fail((int)e, "hipStreamSynchronize"); break; }
+            if (result_wait(out_on_dev)) break;
         }
         done = 1;
     } while (0);

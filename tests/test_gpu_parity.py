@@ -781,6 +781,30 @@ def test_fused_mlp_golden_case(fmt):
     assert np.array_equal(out_d.cpu().numpy().reshape(SEQ, AED), got)
 
 
+def test_results_in_device_memory_are_there_when_a_call_returns():
+    """The synchronous symbols on device pointers: the result is read at once on another stream, which nothing orders behind the library's, and by a
+    copy to the host; short calls and one that takes longer than the library looks for its completion word."""
+    import torch
+    L = ckq.lib()
+    other = torch.cuda.Stream()
+    for seq, E, I in [(9, 256, 512), (200, 896, 1024), (4096, 2048, 8192)]:
+        x = P.to_device(T.normal(seq * E, 0.0, 1.0, seed=E))
+        W1, W2 = P.to_device(T.synth_weights("q8_0", 2 * I, E, seed=85)), P.to_device(T.synth_weights("q4_k", E, I, seed=86))
+        scr, want = torch.zeros(16, dtype=torch.uint8, device="cuda"), None
+        say("results in device memory", seq, E, I)
+        for _ in range(6):
+            y = torch.full((seq, E), 7.0, device="cuda")
+            torch.cuda.synchronize()
+            L.fused_mlp_swiglu_prefill_w1w2_quant(P._dp(x), P._dp(W1), None, P.CK_DT["q8_0"], P._dp(W2), None, P.CK_DT["q4_k"], P._dp(y), seq, E, E, I, I, P._dp(scr))
+            with torch.cuda.stream(other):
+                seen = y.clone()
+            other.synchronize()
+            if want is None:
+                want = y.cpu()
+                assert bool(torch.isfinite(want).all()) and not bool((want == 7.0).any())
+            assert torch.equal(seen.cpu(), want) and torch.equal(y.cpu(), want), (seq, E, I)
+
+
 @pytest.mark.parametrize("fmt,seq,E,I,bias", [("q4_k", 130, 896, 4864, True), ("q6_k", 33, 256, 1024, False),
                                               ("q4_k", 1, 64, 256, True), ("q6_k", 512, 128, 512, True)])
 def test_fused_mlp_vs_oracle(fmt, seq, E, I, bias):
