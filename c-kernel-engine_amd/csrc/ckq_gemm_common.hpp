@@ -139,6 +139,11 @@ __device__ __forceinline__ void lds_copy16(const ckq_v4i &rs, u32 dst, u32 ofs, 
 {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(dst), "v"(ofs), "s"(rs), "s"(k) : "memory");
 }
+/* The same, four bytes per lane to dst + 4 lane. */
+__device__ __forceinline__ void lds_copy4(const ckq_v4i &rs, u32 dst, u32 ofs, int k)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(dst), "v"(ofs), "s"(rs), "s"(k) : "memory");
+}
 __device__ __forceinline__ u32 lds_address(const void *p) { return (u32)(uintptr_t)(__attribute__((address_space(3))) const void *)p; }
 
 constexpr int GEMM_TILE_ROWS = 128;    /* weight rows per tile, all four kernels */

@@ -59,21 +59,20 @@ struct GemmStage {
  * of sub-blocks 0-3 are expanded during pass 1, those of 4-7 during pass 2,
  * and the fp32 combine of tokens 0-31 runs under pass 4.  Activation operands
  * are read from LDS two steps ahead.  Scheduling barriers pin that order. */
+/* A lane's part of its row's raw block: the header and its half's nibble runs. */
+struct GemmRaw { ckq_v4i hv, qv[4]; };
 template <bool DUMP, class CopyFn>
-__device__ __forceinline__ void gemm_block_pipe(const GemmStage &st, u32 wofs, const u32 (&aofs)[8], int col, int half,
-                                                ckq_v16f (&acc)[2], CopyFn copy_one, const GemmDumpLane &dl)
+__device__ __forceinline__ void gemm_block_pipe(const GemmRaw &raw, const uint8_t *st_q, const float *st_d, const uint16_t *st_b, const u32 (&aofs)[8],
+                                                int col, int half, ckq_v16f (&acc)[2], CopyFn copy_one, const GemmDumpLane &dl)
 {
 #define CKQ_PIN() __builtin_amdgcn_sched_barrier(0)
     auto lds16 = [&](const uint8_t *p) { return *reinterpret_cast<const ckq_v4i *>(p); };
     /* step s = 0..15: pass order (ts, j) = (0,0..3) (1,0..3) (0,4..7) (1,4..7) */
     auto step_ts = [](int s) { return (s >> 2) & 1; };
     auto step_j  = [](int s) { return (s & 3) | ((s >> 3) << 2); };
-    auto a_read = [&](int s) { return lds16(&st.q[aofs[step_j(s)] + 32 * 256 * step_ts(s)]); };
+    auto a_read = [&](int s) { return lds16(&st_q[aofs[step_j(s)] + 32 * 256 * step_ts(s)]); };
 
-    const ckq_v4i hv = lds16(&st.w[wofs]);
-    ckq_v4i qv[4];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) qv[g] = lds16(&st.w[wofs + 16 + 32 * g + 16 * half]);
+    const ckq_v4i hv = raw.hv, (&qv)[4] = raw.qv;
     ckq_v4i av[3];
     av[0] = a_read(0);
     av[1] = a_read(1);
@@ -131,7 +130,7 @@ __device__ __forceinline__ void gemm_block_pipe(const GemmStage &st, u32 wofs, c
      * load); the multiply-add of output r then takes lane r of the row as its factor */
     const int dx_tok = mfma32_row_of_lane(col + 32 * half);
     auto load_dx = [&](int ts) {
-        dxl = __builtin_bit_cast(float, *reinterpret_cast<const int *>(&st.d[32 * ts + dx_tok]));
+        dxl = __builtin_bit_cast(float, *reinterpret_cast<const int *>(&st_d[32 * ts + dx_tok]));
     };
     auto min_mfma = [&](int ts) {
         ckq_v16f zero;
@@ -163,13 +162,13 @@ __device__ __forceinline__ void gemm_block_pipe(const GemmStage &st, u32 wofs, c
             }
             const ckq_v4i t = {(int)m[0], (int)m[1], (int)m[2], (int)m[3]};
             bm = __builtin_bit_cast(ckq_v8bf, t);
-            ab[0] = lds16(reinterpret_cast<const uint8_t *>(&st.b[(col) * 16 + 8 * half]));
-            ab[1] = lds16(reinterpret_cast<const uint8_t *>(&st.b[(32 + col) * 16 + 8 * half]));
+            ab[0] = lds16(reinterpret_cast<const uint8_t *>(&st_b[col * 16 + 8 * half]));
+            ab[1] = lds16(reinterpret_cast<const uint8_t *>(&st_b[(32 + col) * 16 + 8 * half]));
         } else if (s == 10) load_dx(0);
         else if (s >= 12) { combine(0, 4 * (s - 12)); combine(0, 4 * (s - 12) + 1); }
         CKQ_PIN();
         aL[ts] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[s % 3], bL[j], (s == 0 || s == 4) ? zero16 : aL[ts], 0, 0, 0);
-        if (s < 9) copy_one(s);                      /* one global->LDS copy of the next block per step */
+        copy_one(s);                                 /* this step's global->LDS copies of the next block */
         if (s == 11) min_mfma(0);                    /* tokens 0-31 are complete after this step */
         if (s >= 12) { combine(0, 4 * (s - 12) + 2); combine(0, 4 * (s - 12) + 3); }
         if (s == 15) asm volatile("" : "+v"(acc[0]));   /* the combine of tokens 0-31 stays under pass 4 */
@@ -253,6 +252,7 @@ __global__ void __launch_bounds__(256 * KG, KG == 2 ? 1 : WPE) gemm_q4k_mfma_ker
         cp_buf = buf;
     };
     auto copy_one = [&](int i) {
+        if (i >= NWI + NQI) return;
         if (i < NWI)      /* weight slots past 17 repeat slot 17: same bytes, no branch */
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_w, (ckq_lds_void *)(stage[cp_buf].w + 1024 * min(wave + 4 * i, 17)), 16,
                                                      (int)wofs_g[i], cp_w, 0, 0);
@@ -260,7 +260,7 @@ __global__ void __launch_bounds__(256 * KG, KG == 2 ? 1 : WPE) gemm_q4k_mfma_ker
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_x, (ckq_lds_void *)(stage[cp_buf].q + 1024 * (wave + 4 * (i - NWI))), 16,
                                                      (int)qofs_g[i - NWI], cp_x, 0, 0);
     };
-    static_assert(NWI + NQI == 9, "the pipelined block issues nine copies");
+    static_assert(NWI + NQI <= 16, "the pipelined block issues one copy a step");
     auto side_store = [&](int buf) {
         if (!st_live) return;
         if (st_q == 0) stage[buf].d[st_tok] = nd;
@@ -309,7 +309,14 @@ __global__ void __launch_bounds__(256 * KG, KG == 2 ? 1 : WPE) gemm_q4k_mfma_ker
             dl.tok_left = a.M - tf;
             dl.row_ok = n < work.N && b < b1;
         }
-        if (KG == 1 || b < b1) gemm_block_pipe<DUMP>(stage[cur], wofs_l, aofs, col, half, acc, copy_one, dl);
+        if (KG == 1 || b < b1) {
+            auto lds16 = [&](u32 ofs) { return *reinterpret_cast<const ckq_v4i *>(&stage[cur].w[wofs_l + ofs]); };
+            GemmRaw raw;
+            raw.hv = lds16(0);
+#pragma unroll
+            for (int g = 0; g < 4; ++g) raw.qv[g] = lds16(16 + 32 * g + 16 * half);
+            gemm_block_pipe<DUMP>(raw, stage[cur].q, stage[cur].d, stage[cur].b, aofs, col, half, acc, copy_one, dl);
+        }
         __builtin_amdgcn_sched_barrier(0);
         side_store(cur ^ 1);
         __builtin_amdgcn_s_waitcnt(0x0070);
@@ -349,6 +356,138 @@ __global__ void __launch_bounds__(256 * KG, KG == 2 ? 1 : WPE) gemm_q4k_mfma_ker
                 const int t = t0 + 32 * ts + 8 * (r >> 2) + 4 * half + (r & 3);
                 if (t < a.M) gemm_store(&o.C[(size_t)t * o.ldc + n], acc[ts][r] + bias);
             }
+    }
+}
+
+/* K-split launches of two to four splits without partial tiles in memory and the launch that adds them.  A block is 64 tokens x 32 rows, and its waves
+ * are the pieces of K that a wave of as many blocks of the kernel above would take: the same work in as many waves, but their partial tiles meet
+ * in LDS, in the order of the splits (the same bits), and until then no wave waits for another.  What the four waves of a tile shared - the
+ * activations - each copies for itself: rows and bsums in one image, which the next block's fill once they have been read, quants and scales in two, 40 KB a wave.
+ * All copies are contiguous runs; a lane loading its row and its token's bsums itself keeps the address path busy for 64 cycles a load (512 x 4864 x 896
+ * 18.8 us instead of 15.5).
+ * Bound: a lone wave's issue and the copies, 1.7 us a 256-block, next to a beginning and an end of 7.  us against partial tiles (tokens, K, rows):
+ * 512 x 4864 x 896 18.7 -> 15.5, 256 x 4096 x 2048 17.4 -> 13.9, 1024 x 2048 x 1024 18.5 -> 12.5, 512 x 3072 x 2048 20.5 -> 16.2; 50 launches 1.22 on average, 1.03 and more. */
+template <int SPLITS>
+__global__ void __launch_bounds__(64 * SPLITS, 1) gemm_q4k_ksplit_kernel(GemmArgs a)
+{
+    __shared__ __attribute__((aligned(16))) uint8_t xs[SPLITS][2][GEMM_BM * 256], ws[SPLITS][32 * 144], bs[SPLITS][GEMM_BM * 32];
+    __shared__ float ds[SPLITS][2][GEMM_BM];
+    const int lane = threadIdx.x & 63, wave = wave_in_block();
+    const int col = lane & 31, half = lane >> 5;
+    int nt, tt;
+    if (!gemm_tile((int)blockIdx.x, a.ntt, a.nnt, nt, tt)) return;
+    const int t0 = tt * GEMM_BM, n0 = nt * 32;
+    const u32 wstride = (u32)a.nb * 144u, xstride = (u32)a.nb * 292u;
+    const int b0 = wave * a.k_per, b1 = min(a.nb, b0 + a.k_per), last = b1 - 1;
+    auto buffer = [](const uint8_t *p) {
+        return ckq_v4i{__builtin_amdgcn_readfirstlane((int)(u32)(uintptr_t)p), __builtin_amdgcn_readfirstlane((int)(u32)((uintptr_t)p >> 32)), 0x7fffffff, 0x00020000};
+    };
+    const ckq_v4i rs_w = buffer(a.B + (size_t)n0 * wstride), rs_x = buffer(a.A + (size_t)t0 * xstride);
+
+    /* copies of a 256-block: of the quants (four tokens each), the rows (288 chunks, the last copy half a wave), the bsums, the scales */
+    constexpr int NQ = GEMM_BM / 4, NW = 5;
+    u32 qofs[NQ], wofs[NW], bofs[2];
+    auto token = [&](int t) { return (u32)min(t, a.M - 1 - t0) * xstride; };
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+        const int t = 4 * i + (lane >> 4);
+        qofs[i] = token(t) + 4u + 16u * (u32)((lane & 15) ^ (t & 15));
+    }
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+        const int e = min(64 * i + lane, 287);
+        wofs[i] = (u32)min(e / 9, a.N - 1 - n0) * wstride + 16u * (u32)(e % 9);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) bofs[i] = token(32 * i + (lane >> 1)) + 260u + 16u * (u32)(lane & 1);
+    const u32 dofs = token(lane);
+    const u32 wdst = lds_address(ws[wave]), bdst = lds_address(bs[wave]);
+    auto copy_q = [&](int b, int buf, int i) { lds_copy16(rs_x, lds_address(xs[wave][buf]) + 1024u * (u32)i, qofs[i], b * 292); };
+    auto copy_w = [&](int b, int i) { if (i < NW - 1 || lane < 32) lds_copy16(rs_w, wdst + 1024u * (u32)i, wofs[i], b * 144); };
+    auto copy_b = [&](int b, int i) { lds_copy16(rs_x, bdst + 1024u * (u32)i, bofs[i], b * 292); };
+    auto copy_d = [&](int b, int buf) { lds_copy4(rs_x, lds_address(ds[wave][buf]), dofs, b * 292); };
+    auto reads_done = [] {                         /* lgkmcnt(0) */
+        __builtin_amdgcn_s_waitcnt(0xc07f);
+        asm volatile("" ::: "memory");
+    };
+    u32 aofs[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) aofs[j] = (u32)col * 256u + 16u * (u32)((2 * j + half) ^ (col & 15));
+    /* what the wave has copied is there (no other wave reads it); lane t puts the bsums of token t into the form of the min MFMA */
+    auto landed = [&] {
+        __builtin_amdgcn_s_waitcnt(0x0f70);
+        asm volatile("" ::: "memory");
+        ckq_v4i *const o = reinterpret_cast<ckq_v4i *>(&bs[wave][lane * 32]);
+        const ckq_v4i s[2] = {o[0], o[1]};
+        ckq_v4i lo, hi;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int u = s[i >> 1][2 * (i & 1)], v = s[i >> 1][2 * (i & 1) + 1];
+            const int p0 = (int)(int16_t)(u & 0xffff) + (u >> 16), p1 = (int)(int16_t)(v & 0xffff) + (v >> 16);
+            lo[i] = (int)bf16_pair((float)(p0 & 63), (float)(p1 & 63));
+            hi[i] = (int)bf16_pair((float)(64 * (p0 >> 6)), (float)(64 * (p1 >> 6)));
+        }
+        o[0] = lo;
+        o[1] = hi;
+        __builtin_amdgcn_wave_barrier();
+    };
+    ckq_v16f acc[2];
+#pragma unroll
+    for (int ts = 0; ts < 2; ++ts)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[ts][r] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) copy_w(b0, i);
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) copy_q(b0, 0, i);
+    copy_b(b0, 0);
+    copy_b(b0, 1);
+    copy_d(b0, 0);
+    landed();
+    auto kstep = [&](int b, auto curc) {
+        constexpr int cur = decltype(curc)::value;
+        const int bn = min(b + 1, last);
+        auto lds16 = [&](int ofs) { return *reinterpret_cast<const ckq_v4i *>(&ws[wave][144 * col + ofs]); };
+        GemmRaw raw;
+        raw.hv = lds16(0);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) raw.qv[g] = lds16(16 + 32 * g + 16 * half);
+        gemm_block_pipe<false>(raw, xs[wave][cur], ds[wave][cur], reinterpret_cast<const uint16_t *>(bs[wave]), aofs, col, half, acc, [&](int s) {
+            auto q2 = [&](int i) { copy_q(bn, cur ^ 1, i); copy_q(bn, cur ^ 1, i + 1); };
+            if (s == 1) {                          /* the rows are in registers: the next ones come in their place */
+                asm volatile("" : "+v"(raw.hv), "+v"(raw.qv[0]), "+v"(raw.qv[1]), "+v"(raw.qv[2]), "+v"(raw.qv[3]));
+                reads_done();
+            }
+            if (s == 9) reads_done();              /* the bsums have been read (step 8) */
+            if (s == 1 || s == 2) { copy_w(bn, 2 * s - 2); copy_w(bn, 2 * s - 1); }
+            if (s == 3) copy_w(bn, 4);
+            if (s >= 3 && s < 9) q2(2 * s - 6);
+            if (s == 9) { copy_b(bn, 0); copy_b(bn, 1); }
+            if (s == 10) { q2(12); q2(14); }
+            if (s == 11) copy_d(bn, cur ^ 1);
+        }, GemmDumpLane{});
+        __builtin_amdgcn_sched_barrier(0);
+        landed();
+    };
+    for (int b = b0; b < b1; b += 2) {
+        kstep(b, std::integral_constant<int, 0>{});
+        if (b + 1 < b1) kstep(b + 1, std::integral_constant<int, 1>{});
+    }
+
+    float *const red = reinterpret_cast<float *>(&xs[0][0][0]);      /* [split][output of a lane][lane]; a wave writes where its own activations lay */
+    constexpr int PART = 2 * GEMM_BM * 256 / 4;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) red[wave * PART + 64 * i + lane] = acc[i >> 4][i & 15];
+    __syncthreads();
+    const int n = n0 + col;
+    if (n >= a.N) return;
+    const float bias = a.bias ? a.bias[n] : 0.0f;
+    for (int i = wave; i < 32; i += SPLITS) {
+        float v = red[64 * i + lane];
+#pragma unroll
+        for (int sp = 1; sp < SPLITS; ++sp) v += red[sp * PART + 64 * i + lane];
+        const int r = i & 15, t = t0 + 32 * (i >> 4) + 8 * (r >> 2) + 4 * half + (r & 3);
+        if (t < a.M) gemm_store(&a.C[(size_t)t * a.ldc + n], a.bias ? v + bias : v);
     }
 }
 
@@ -393,6 +532,14 @@ GemmChains gemm_q4k_chains(int M, int N, int K)
     return c;
 }
 
+/* The splits of K of a launch whose waves add them up, 0: another kernel.  Four waves fill a CU's LDS, so every block gets a place at once: a second round
+ * would cost more than the second launch (300 tokens x 3840 x 2000: 320 blocks of three waves). */
+static int gemm_q4k_ksplit(const GemmArgs &g, int tiles)
+{
+    const int s = gemm_choose_splits(tiles, g.nb), per = (g.nb + s - 1) / s, k = (g.nb + per - 1) / per;
+    return k >= 2 && k <= 4 && g.ntt * ((g.N + 31) / 32) <= (k == 2 ? 512 : 256) ? k : 0;
+}
+
 int launch_gemm_q4k_mfma(const void *A, const void *B, const float *bias, float *C,
                          int M, int N, int K, long ldc, const GemmOpts &opts, hipStream_t s)
 {
@@ -424,6 +571,17 @@ int launch_gemm_q4k_mfma(const void *A, const void *B, const float *bias, float 
 #endif
     }
     if (two_groups) return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 2>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s, 512);
+    if (const int k = gemm_q4k_ksplit(g, tiles)) {
+        g.k_per = (g.nb + k - 1) / k;
+        /* what has no room for the partial tiles of the kernel above is refused as before */
+        if (g.ext_part && (size_t)k * (size_t)M * (size_t)N * sizeof(float) > g.ext_part_bytes) return CKQ_ESCRATCH;
+        g.nnt = (N + 31) / 32;
+        const dim3 grid((unsigned)gemm_blocks(g.ntt, g.nnt)), block((unsigned)(64 * k));
+        if (k == 2) hipLaunchKernelGGL(gemm_q4k_ksplit_kernel<2>, grid, block, 0, s, g);
+        else if (k == 3) hipLaunchKernelGGL(gemm_q4k_ksplit_kernel<3>, grid, block, 0, s, g);
+        else hipLaunchKernelGGL(gemm_q4k_ksplit_kernel<4>, grid, block, 0, s, g);
+        return (int)hipGetLastError();
+    }
     const GemmGroupIn one = {1, {B}, {bias}, {C}, {N}, {ldc}};
     if (tiles > 256 && gemm_ragged_last(one, M, GEMM_BM)) return gemm_launch_ragged_last(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 1>, g, one, GEMM_BM, s);
     return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 1>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s, 256);

@@ -1778,6 +1778,49 @@ def test_16_row_tiles_of_several_token_groups_copied_to_lds(fmt):
         L.ckq_set_prefill_variant(tag, 0)
 
 
+@pytest.mark.parametrize("fmt", ["q4_k"])
+def test_k_split_whose_pieces_meet_in_lds(fmt):
+    """Two, three and four pieces of K, of two blocks and more, the last one shorter; one token and one row more than a tile, a single row; as many
+    blocks as the CUs have places for.  Bit for bit the chains of the tile kernels as the 16-row tiles run them, within the tolerance the oracle's result, nothing outside the
+    matrix; and the entry point that allocates nothing refuses what it refused when the partial tiles lay in memory."""
+    import torch
+    L = ckq.lib()
+    tag = P.FMT[fmt]
+    try:
+        for M, N, nb in [(9, 1, 8), (64, 128, 8), (65, 33, 9), (130, 1000, 11), (512, 2048, 8), (200, 257, 12), (449, 1025, 13), (33, 4096, 15), (512, 896, 19), (70, 130, 16),
+                         (509, 1024, 17), (1000, 100, 21)]:
+            K = nb * 256
+            xh = T.normal(M * K, 0.0, 1.0, seed=M)
+            xq, Wh = P.dev_quantize(P.to_device(xh), "q8_k", rows=M), T.synth_weights(fmt, N, K, seed=9700 + nb)
+            W, bias = P.to_device(Wh), P.to_device(T.normal(N, 0.0, 0.5, seed=N))
+            say("K split, pieces meet in LDS", fmt, M, N, K)
+
+            def call(forced, b=bias):
+                L.ckq_set_prefill_variant(tag, 16 if forced else 0)
+                L.ckq_set_gemm_policy(1)
+                c = torch.full((M + 1, N + 3), 7.0, device="cuda")
+                P.check(L.ckq_gemm_nt_dev(tag, P._dp(xq), P._dp(W), None if b is None else P._dp(b), P._dp(c), M, N, K, N + 3, P._stream()), "ckq_gemm_nt_dev")
+                assert bool((c[:, N:] == 7.0).all()) and bool((c[M] == 7.0).all()), (M, N, K)
+                return c[:M, :N]
+            assert torch.equal(call(False), call(True)), (M, N, K)
+            assert torch.equal(call(False, None), call(True, None)), (M, N, K)
+            if M * N * K < 1 << 28:
+                want = T.oracle_gemm_nt(fmt, xq.cpu().numpy(), Wh, bias.cpu().numpy(), M, N, K)
+                assert T.norm_err(call(False).cpu().numpy(), want) <= TOL
+        for M, N, nb, refused in [(512, 896, 19, True), (65, 33, 9, False)]:
+            K = nb * 256
+            xq, W = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, seed=3)), "q8_k", rows=M), P.to_device(T.random_blocks(fmt, N * nb, 9750))
+            L.ckq_set_prefill_variant(tag, 0)
+            c = torch.full((M, N), 7.0, device="cuda")
+            rc = L.ckq_gemm_nt_noalloc_dev(tag, P._dp(xq), P._dp(W), None, P._dp(c), M, N, K, N, P._stream())
+            assert (rc != 0) == refused and bool((c == 7.0).all()) == refused, (rc, M, N)
+            if not refused:
+                assert torch.equal(c, P.dev_gemm_nt(fmt, xq, W, None, M, N, K).view(M, N))
+    finally:
+        L.ckq_set_gemm_policy(0)
+        L.ckq_set_prefill_variant(tag, 0)
+
+
 @pytest.mark.parametrize("fmt", ["q4_k", "q5_k", "q6_k"])
 def test_16_row_tiles_alone_on_their_cu(fmt):
     """Row tiles that have a CU each, one token group and rows too few for groups in pairs: blocks of eight waves, of twelve and (rows longer than
