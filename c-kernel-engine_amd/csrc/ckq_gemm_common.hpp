@@ -139,6 +139,11 @@ __device__ __forceinline__ void lds_copy16(const ckq_v4i &rs, u32 dst, u32 ofs, 
 {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(dst), "v"(ofs), "s"(rs), "s"(k) : "memory");
 }
+/* The source of such copies: a uniform address. */
+__device__ __forceinline__ ckq_v4i gemm_buffer(const uint8_t *p)
+{
+    return ckq_v4i{__builtin_amdgcn_readfirstlane((int)(u32)(uintptr_t)p), __builtin_amdgcn_readfirstlane((int)(u32)((uintptr_t)p >> 32)), 0x7fffffff, 0x00020000};
+}
 /* The same, four bytes per lane to dst + 4 lane. */
 __device__ __forceinline__ void lds_copy4(const ckq_v4i &rs, u32 dst, u32 ofs, int k)
 {
@@ -248,6 +253,45 @@ __device__ __forceinline__ void gemm_store(float *p, float v)
 #else
     *p = v;
 #endif
+}
+
+/* K split in SPLITS pieces by the waves of a block (gemm_q4k_ksplit_kernel and its siblings): the pieces of a tile of 64 tokens x 32 rows meet in LDS, which
+ * the block has done with but for its own wave's part at red + wave * part, and are added in the order of the splits. */
+template <int SPLITS>
+__device__ __forceinline__ void gemm_ksplit_store(const GemmArgs &a, float *red, int part, const ckq_v16f (&acc)[2], int t0, int n0, int wave, int lane)
+{
+#pragma unroll
+    for (int i = 0; i < 32; ++i) red[wave * part + 64 * i + lane] = acc[i >> 4][i & 15];
+    __syncthreads();
+    const int n = n0 + (lane & 31);
+    if (n >= a.N) return;
+    const float bias = a.bias ? a.bias[n] : 0.0f;
+    for (int i = wave; i < 32; i += SPLITS) {
+        float v = red[64 * i + lane];
+#pragma unroll
+        for (int sp = 1; sp < SPLITS; ++sp) v += red[sp * part + 64 * i + lane];
+        const int r = i & 15, t = t0 + 32 * (i >> 4) + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+        if (t < a.M) gemm_store(&a.C[(size_t)t * a.ldc + n], a.bias ? v + bias : v);
+    }
+}
+
+/* The pieces of such a launch in place of one of `tiles` tiles of 64 tokens x 128 rows and up to max_per 256-blocks a piece, 0: no.  Four waves
+ * fill a CU's LDS, so every block gets a place at once: a second round would cost more than the second launch it saves (Q4_K, 300 tokens x 3840 x
+ * 2000: 320 blocks of three waves). */
+static int gemm_ksplit_pieces(const GemmArgs &g, int tiles, int max_per)
+{
+    const int s = gemm_choose_splits(tiles, g.nb), per = (g.nb + s - 1) / s, k = (g.nb + per - 1) / per;
+    return k >= 2 && k <= 4 && per <= max_per && g.ntt * ((g.N + 31) / 32) <= (k == 2 ? 512 : 256) ? k : 0;
+}
+template <class Kernel>
+static int gemm_launch_ksplit(Kernel k2, Kernel k3, Kernel k4, GemmArgs &g, int k, hipStream_t s)
+{
+    g.k_per = (g.nb + k - 1) / k;
+    /* what has no room for the partial tiles of a split among blocks is refused as there */
+    if (g.ext_part && (size_t)k * (size_t)g.M * (size_t)g.N * sizeof(float) > g.ext_part_bytes) return CKQ_ESCRATCH;
+    g.nnt = (g.N + 31) / 32;
+    hipLaunchKernelGGL(k == 2 ? k2 : k == 3 ? k3 : k4, dim3((unsigned)gemm_blocks(g.ntt, g.nnt)), dim3((unsigned)(64 * k)), 0, s, g);
+    return (int)hipGetLastError();
 }
 
 /* Grouped launch: the matrices of `in` against the same M x K activations, as one grid (no K split; the

@@ -379,10 +379,7 @@ __global__ void __launch_bounds__(64 * SPLITS, 1) gemm_q4k_ksplit_kernel(GemmArg
     const int t0 = tt * GEMM_BM, n0 = nt * 32;
     const u32 wstride = (u32)a.nb * 144u, xstride = (u32)a.nb * 292u;
     const int b0 = wave * a.k_per, b1 = min(a.nb, b0 + a.k_per), last = b1 - 1;
-    auto buffer = [](const uint8_t *p) {
-        return ckq_v4i{__builtin_amdgcn_readfirstlane((int)(u32)(uintptr_t)p), __builtin_amdgcn_readfirstlane((int)(u32)((uintptr_t)p >> 32)), 0x7fffffff, 0x00020000};
-    };
-    const ckq_v4i rs_w = buffer(a.B + (size_t)n0 * wstride), rs_x = buffer(a.A + (size_t)t0 * xstride);
+    const ckq_v4i rs_w = gemm_buffer(a.B + (size_t)n0 * wstride), rs_x = gemm_buffer(a.A + (size_t)t0 * xstride);
 
     /* copies of a 256-block: of the quants (four tokens each), the rows (288 chunks, the last copy half a wave), the bsums, the scales */
     constexpr int NQ = GEMM_BM / 4, NW = 5;
@@ -474,21 +471,7 @@ __global__ void __launch_bounds__(64 * SPLITS, 1) gemm_q4k_ksplit_kernel(GemmArg
         if (b + 1 < b1) kstep(b + 1, std::integral_constant<int, 1>{});
     }
 
-    float *const red = reinterpret_cast<float *>(&xs[0][0][0]);      /* [split][output of a lane][lane]; a wave writes where its own activations lay */
-    constexpr int PART = 2 * GEMM_BM * 256 / 4;
-#pragma unroll
-    for (int i = 0; i < 32; ++i) red[wave * PART + 64 * i + lane] = acc[i >> 4][i & 15];
-    __syncthreads();
-    const int n = n0 + col;
-    if (n >= a.N) return;
-    const float bias = a.bias ? a.bias[n] : 0.0f;
-    for (int i = wave; i < 32; i += SPLITS) {
-        float v = red[64 * i + lane];
-#pragma unroll
-        for (int sp = 1; sp < SPLITS; ++sp) v += red[sp * PART + 64 * i + lane];
-        const int r = i & 15, t = t0 + 32 * (i >> 4) + 8 * (r >> 2) + 4 * half + (r & 3);
-        if (t < a.M) gemm_store(&a.C[(size_t)t * a.ldc + n], a.bias ? v + bias : v);
-    }
+    gemm_ksplit_store<SPLITS>(a, reinterpret_cast<float *>(xs), 2 * GEMM_BM * 256 / 4, acc, t0, n0, wave, lane);
 }
 
 /* Which token tile a launch takes.  A 96-token tile (ckq_gemm_q4k_t96.hip) costs less per token but comes in blocks that run longer and
@@ -532,14 +515,6 @@ GemmChains gemm_q4k_chains(int M, int N, int K)
     return c;
 }
 
-/* The splits of K of a launch whose waves add them up, 0: another kernel.  Four waves fill a CU's LDS, so every block gets a place at once: a second round
- * would cost more than the second launch (300 tokens x 3840 x 2000: 320 blocks of three waves). */
-static int gemm_q4k_ksplit(const GemmArgs &g, int tiles)
-{
-    const int s = gemm_choose_splits(tiles, g.nb), per = (g.nb + s - 1) / s, k = (g.nb + per - 1) / per;
-    return k >= 2 && k <= 4 && g.ntt * ((g.N + 31) / 32) <= (k == 2 ? 512 : 256) ? k : 0;
-}
-
 int launch_gemm_q4k_mfma(const void *A, const void *B, const float *bias, float *C,
                          int M, int N, int K, long ldc, const GemmOpts &opts, hipStream_t s)
 {
@@ -571,17 +546,7 @@ int launch_gemm_q4k_mfma(const void *A, const void *B, const float *bias, float 
 #endif
     }
     if (two_groups) return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 2>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s, 512);
-    if (const int k = gemm_q4k_ksplit(g, tiles)) {
-        g.k_per = (g.nb + k - 1) / k;
-        /* what has no room for the partial tiles of the kernel above is refused as before */
-        if (g.ext_part && (size_t)k * (size_t)M * (size_t)N * sizeof(float) > g.ext_part_bytes) return CKQ_ESCRATCH;
-        g.nnt = (N + 31) / 32;
-        const dim3 grid((unsigned)gemm_blocks(g.ntt, g.nnt)), block((unsigned)(64 * k));
-        if (k == 2) hipLaunchKernelGGL(gemm_q4k_ksplit_kernel<2>, grid, block, 0, s, g);
-        else if (k == 3) hipLaunchKernelGGL(gemm_q4k_ksplit_kernel<3>, grid, block, 0, s, g);
-        else hipLaunchKernelGGL(gemm_q4k_ksplit_kernel<4>, grid, block, 0, s, g);
-        return (int)hipGetLastError();
-    }
+    if (const int k = gemm_ksplit_pieces(g, tiles, 7)) return gemm_launch_ksplit(gemm_q4k_ksplit_kernel<2>, gemm_q4k_ksplit_kernel<3>, gemm_q4k_ksplit_kernel<4>, g, k, s);
     const GemmGroupIn one = {1, {B}, {bias}, {C}, {N}, {ldc}};
     if (tiles > 256 && gemm_ragged_last(one, M, GEMM_BM)) return gemm_launch_ragged_last(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 1>, g, one, GEMM_BM, s);
     return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 1>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s, 256);

@@ -438,6 +438,85 @@ __global__ void __launch_bounds__(256, 2) gemm_q5k_pair_kernel(GemmArgs a)
     }
 }
 
+/* K split among the waves of a block, as gemm_q4k_ksplit_kernel has it: 64 tokens x 32 rows, a wave a piece of K, 39.75 KB of LDS each: one image of
+ * all but the quants, which the next block's take once they have been read, at the start of a block.  us against partial tiles in memory (tokens,
+ * K, rows): 512 x 4864 x 896 21.2 -> 17.3, 256 x 5632 x 2048 23.0 -> 19.0, 512 x 2048 x 2048 20.0 -> 12.6; 35 launches of four to nine 256-blocks a piece 1.30 on average, 1.05 and
+ * more; of ten to 21 0.91 to 1.12. */
+template <int SPLITS>
+__global__ void __launch_bounds__(64 * SPLITS, 1) gemm_q5k_ksplit_kernel(GemmArgs a)
+{
+    constexpr int BM = GEMM5_BM;
+    __shared__ __attribute__((aligned(16))) uint8_t xs[SPLITS][2][BM * 256], ws[SPLITS][32 * GEMM5_ROW], bs[SPLITS][BM * 32];
+    __shared__ __attribute__((aligned(16))) float ds[SPLITS][BM];
+    const int lane = threadIdx.x & 63, wave = wave_in_block();
+    const int col = lane & 31, half = lane >> 5;
+    int nt, tt;
+    if (!gemm_tile((int)blockIdx.x, a.ntt, a.nnt, nt, tt)) return;
+    const int t0 = tt * BM, n0 = nt * 32;
+    const u32 wstride = (u32)a.nb * 176u, xstride = (u32)a.nb * 292u;
+    const int b0 = wave * a.k_per, b1 = min(a.nb, b0 + a.k_per), last = b1 - 1;
+    const ckq_v4i rs_w = gemm_buffer(a.B + (size_t)n0 * wstride), rs_x = gemm_buffer(a.A + (size_t)t0 * xstride);
+
+    constexpr int NW = 6, NQ = BM / 4, NC = NW + NQ + 3;      /* copies of a 256-block: rows (the last half a wave), quants of four tokens each, bsums, scales */
+    static_assert(NC == 25, "nine slots of two copies and seven of one");
+    u32 wofs[NW], qofs[NQ], bofs[2];
+    auto token = [&](int t) { return (u32)min(t, a.M - 1 - t0) * xstride; };
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+        const int e = min(64 * i + lane, 32 * 11 - 1);
+        wofs[i] = (u32)min(e / 11, a.N - 1 - n0) * wstride + 16u * (u32)(e % 11);
+    }
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+        const int t = 4 * i + (lane >> 4);
+        qofs[i] = token(t) + 4u + 16u * (u32)((lane & 15) ^ (t & 15));
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) bofs[i] = token(32 * i + (lane >> 1)) + 260u + 16u * (u32)(lane & 1);
+    const u32 dofs = token(lane), wdst = lds_address(ws[wave]), bdst = lds_address(bs[wave]);
+    auto copy = [&](int b, int buf, int i) {
+        if (i < NW - 1 || (i == NW - 1 && lane < 32)) lds_copy16(rs_w, wdst + 1024u * (u32)i, wofs[i], b * 176);
+        else if (i == NW - 1) ;
+        else if (i < NW + NQ)     lds_copy16(rs_x, lds_address(xs[wave][buf]) + 1024u * (u32)(i - NW), qofs[i - NW], b * 292);
+        else if (i < NW + NQ + 2) lds_copy16(rs_x, bdst + 1024u * (u32)(i - NW - NQ), bofs[i - NW - NQ], b * 292);
+        else                      lds_copy4(rs_x, lds_address(ds[wave]), dofs, b * 292);
+    };
+    u32 aofs[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) aofs[s] = (u32)col * 256u + 16u * (u32)((2 * s + half) ^ (col & 15));
+    auto landed = [] {                             /* vmcnt(0): this wave's copies are there, and no other wave reads them */
+        __builtin_amdgcn_s_waitcnt(0x0f70);
+        asm volatile("" ::: "memory");
+    };
+    ckq_v16f acc[2];
+#pragma unroll
+    for (int ts = 0; ts < 2; ++ts)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[ts][r] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) copy(b0, 0, i);
+    landed();
+    auto kstep = [&](int b, auto curc) __attribute__((always_inline)) {
+        constexpr int cur = decltype(curc)::value;
+        const int bn = min(b + 1, last);
+        gemm5_block<16, false>(ws[wave], xs[wave][cur], bs[wave], ds[wave], (u32)(col * GEMM5_ROW), aofs, col, half, acc, [&](int i) __attribute__((always_inline)) {
+            const int slot = 2 * (i & 7) + (i >> 3);          /* in time: i and i + 8 are the two of a slab */
+            if (slot < 9) { copy(bn, cur ^ 1, 2 * slot); copy(bn, cur ^ 1, 2 * slot + 1); }
+            else copy(bn, cur ^ 1, 9 + slot);
+        }, []() __attribute__((always_inline)) {
+            __builtin_amdgcn_s_waitcnt(0xc07f);    /* lgkmcnt(0): rows, bsums and scales are in registers */
+            asm volatile("" ::: "memory");
+        }, GemmDumpLane{});
+        __builtin_amdgcn_sched_barrier(0);
+        landed();
+    };
+    for (int b = b0; b < b1; b += 2) {
+        kstep(b, std::integral_constant<int, 0>{});
+        if (b + 1 < b1) kstep(b + 1, std::integral_constant<int, 1>{});
+    }
+    gemm_ksplit_store<SPLITS>(a, reinterpret_cast<float *>(xs), 2 * BM * 256 / 4, acc, t0, n0, wave, lane);
+}
+
 /* More tiles than CUs: the paired kernel (512 x 11008, K = 4096: 99.2 -> 85.3 us; 2048 tokens: 374 -> 320; 512 x 8192:
  * 67.9 -> 60.4); up to one tile per CU the three-stage kernel, whose deeper pipeline serves a block that has its CU to
  * itself (256 tiles: 81.7 against 83.0).  variant: 0 = by tile count, 1 = one block per CU always, 2 = paired always. */
@@ -500,6 +579,7 @@ int launch_gemm_q5k_mfma(const void *A, const void *B, const float *bias, float 
 #else
     if (sums) return CKQ_ENODUMP;
 #endif
+    if (const int k = gemm_ksplit_pieces(g, g.ntt * g.nnt, 9)) return gemm_launch_ksplit(gemm_q5k_ksplit_kernel<2>, gemm_q5k_ksplit_kernel<3>, gemm_q5k_ksplit_kernel<4>, g, k, s);
     return gemm_launch_split(gemm_q5k_mfma_kernel<false>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s);
 }
 

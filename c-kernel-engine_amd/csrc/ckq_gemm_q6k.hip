@@ -449,6 +449,88 @@ __global__ void __launch_bounds__(256, 2) gemm_q6k_pair_kernel(GemmArgs a)
     }
 }
 
+/* K split among the waves of a block, as gemm_q4k_ksplit_kernel has it: 64 tokens x 32 rows, a wave a piece of K, 39.5 KB of LDS each.  The next
+ * block's rows fill the one image once the wave has the last ones in registers; copies in memory order, two a slot until all rows and half of the quants are on
+ * their way.  us against partial tiles in memory (tokens, K, rows): 512 x 4864 x 896 20.3 -> 18.1, 512 x 2048 x 2048 19.3 -> 14.2, 131 x 4096 x 2250 18.0 -> 15.6; 37 launches
+ * of four to seven 256-blocks a piece 1.22 on average, 1.05 and more; of eight 1.04, of nine to 21 0.87 to 0.96 (a 256-block takes a lone wave 2.3 us here, 1.6 where
+ * three stages are shared). */
+template <int SPLITS>
+__global__ void __launch_bounds__(64 * SPLITS, 1) gemm_q6k_ksplit_kernel(GemmArgs a)
+{
+    constexpr int BM = 64;
+    __shared__ __attribute__((aligned(16))) uint8_t xs[SPLITS][2][BM * 256], ws[SPLITS][32 * GEMM6_ROW];
+    __shared__ __attribute__((aligned(16))) float ds[SPLITS][2][BM];
+    const int lane = threadIdx.x & 63, wave = wave_in_block();
+    const int col = lane & 31, half = lane >> 5;
+    int nt, tt;
+    if (!gemm_tile((int)blockIdx.x, a.ntt, a.nnt, nt, tt)) return;
+    const int t0 = tt * BM, n0 = nt * 32;
+    const u32 wstride = (u32)a.nb * 210u, xstride = (u32)a.nb * 292u;
+    const int b0 = wave * a.k_per, b1 = min(a.nb, b0 + a.k_per), last = b1 - 1;
+    const ckq_v4i rs_w = gemm_buffer(a.B + (size_t)n0 * wstride), rs_x = gemm_buffer(a.A + (size_t)t0 * xstride);
+
+    constexpr int NW = 7, NQ = BM / 4, NC = NW + NQ + 1;      /* copies of a 256-block: rows, quants of four tokens each, scales */
+    static_assert(NW * 64 == 32 * 14 && NC == 24, "eight slots of two copies and eight of one");
+    u32 wofs[NW], qofs[NQ];
+    auto token = [&](int t) { return (u32)min(t, a.M - 1 - t0) * xstride; };
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+        const int e = 64 * i + lane, part = e % 14;
+        wofs[i] = (u32)min(e / 14, a.N - 1 - n0) * wstride + (part < 13 ? 16u * (u32)part : 194u);
+    }
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+        const int t = 4 * i + (lane >> 4);
+        qofs[i] = token(t) + 4u + 16u * (u32)((lane & 15) ^ (t & 15));
+    }
+    const u32 dofs = token(lane), wdst = lds_address(ws[wave]);
+    auto copy = [&](int b, int buf, int i) {
+        if (i < NW)           lds_copy16(rs_w, wdst + 1024u * (u32)i, wofs[i], b * 210);
+        else if (i < NW + NQ) lds_copy16(rs_x, lds_address(xs[wave][buf]) + 1024u * (u32)(i - NW), qofs[i - NW], b * 292);
+        else                  lds_copy4(rs_x, lds_address(ds[wave][buf]), dofs, b * 292);
+    };
+    u32 aofs[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) aofs[s] = (u32)col * 256u + 16u * (u32)((2 * s + half) ^ (col & 15));
+    auto landed = [] {                             /* vmcnt(0): this wave's copies are there, and no other wave reads them */
+        __builtin_amdgcn_s_waitcnt(0x0f70);
+        asm volatile("" ::: "memory");
+    };
+    ckq_v16f acc[2];
+#pragma unroll
+    for (int ts = 0; ts < 2; ++ts)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[ts][r] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) copy(b0, 0, i);
+    landed();
+    Gemm6Head<2> head;
+    gemm6_head_read<2>(ws[wave], xs[wave][0], (u32)(col * GEMM6_ROW), aofs[0], half, head);
+    auto kstep = [&](int b, auto curc) __attribute__((always_inline)) {
+        constexpr int cur = decltype(curc)::value;
+        const int bn = min(b + 1, last);
+        __builtin_amdgcn_s_waitcnt(0xc07f);        /* lgkmcnt(0): the rows are in registers */
+        asm volatile("" ::: "memory");
+        Gemm6Sums<2> sums;
+        gemm6_slabs<2, 16>(xs[wave][cur], ds[wave][cur], head, aofs, half, sums, [&](int i) __attribute__((always_inline)) {
+            const int slot = 2 * (i & 7) + (i >> 3);          /* in time: i and i + 8 are the two of a slab */
+            if (slot < 8) { copy(bn, cur ^ 1, 2 * slot); copy(bn, cur ^ 1, 2 * slot + 1); }
+            else copy(bn, cur ^ 1, 8 + slot);
+        });
+        __builtin_amdgcn_sched_barrier(0);
+        landed();
+        gemm6_head_read<2>(ws[wave], xs[wave][cur ^ 1], (u32)(col * GEMM6_ROW), aofs[0], half, head);
+        __builtin_amdgcn_sched_barrier(0);
+        gemm6_combine<2, false>(sums, acc, GemmDumpLane{});
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int b = b0; b < b1; b += 2) {
+        kstep(b, std::integral_constant<int, 0>{});
+        if (b + 1 < b1) kstep(b + 1, std::integral_constant<int, 1>{});
+    }
+    gemm_ksplit_store<SPLITS>(a, reinterpret_cast<float *>(xs), 2 * BM * 256 / 4, acc, t0, n0, wave, lane);
+}
+
 /* Which kernel a launch takes: 64-token tiles of one block per CU, 128-token tiles of one block per CU, or 64-token tiles of two
  * (paired).  us for nb 256-blocks of K, from 70 launches of 33 to 900 tokens, 2000 to 40000 rows and K of 512 to 11008:
  *   64 tokens    6.5 + 1.5 nb a round of 256 tiles
@@ -519,6 +601,7 @@ int launch_gemm_q6k_mfma(const void *A, const void *B, const float *bias, float 
     }
     if (form == Q6K_PAIRED) return gemm_launch_split(gemm_q6k_pair_kernel<2>, g, grid, g.nb, s);
     if (form == Q6K_128) return gemm_launch_split(gemm_q6k_mfma_kernel<4>, g, grid, g.nb, s);
+    if (const int k = gemm_ksplit_pieces(g, g.ntt * g.nnt, 7)) return gemm_launch_ksplit(gemm_q6k_ksplit_kernel<2>, gemm_q6k_ksplit_kernel<3>, gemm_q6k_ksplit_kernel<4>, g, k, s);
     return gemm_launch_split(gemm_q6k_mfma_kernel<2>, g, grid, g.nb, s);
 }
 

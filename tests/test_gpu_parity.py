@@ -1778,7 +1778,7 @@ def test_16_row_tiles_of_several_token_groups_copied_to_lds(fmt):
         L.ckq_set_prefill_variant(tag, 0)
 
 
-@pytest.mark.parametrize("fmt", ["q4_k"])
+@pytest.mark.parametrize("fmt", ["q4_k", "q5_k", "q6_k"])
 def test_k_split_whose_pieces_meet_in_lds(fmt):
     """Two, three and four pieces of K, of two blocks and more, the last one shorter; one token and one row more than a tile, a single row; as many
     blocks as the CUs have places for.  Bit for bit the chains of the tile kernels as the 16-row tiles run them, within the tolerance the oracle's result, nothing outside the
@@ -1787,7 +1787,7 @@ def test_k_split_whose_pieces_meet_in_lds(fmt):
     L = ckq.lib()
     tag = P.FMT[fmt]
     try:
-        for M, N, nb in [(9, 1, 8), (64, 128, 8), (65, 33, 9), (130, 1000, 11), (512, 2048, 8), (200, 257, 12), (449, 1025, 13), (33, 4096, 15), (512, 896, 19), (70, 130, 16),
+        for M, N, nb in [(9, 1, 8), (64, 128, 8), (65, 33, 9), (130, 1000, 11), (512, 2048, 8), (200, 257, 12), (449, 1025, 13), (33, 4096, 15), (512, 896, 19), (70, 130, 16), (500, 900, 28),
                          (509, 1024, 17), (1000, 100, 21)]:
             K = nb * 256
             xh = T.normal(M * K, 0.0, 1.0, seed=M)
