@@ -275,13 +275,16 @@ __device__ __forceinline__ void gemm_ksplit_store(const GemmArgs &a, float *red,
     }
 }
 
-/* The pieces of such a launch in place of one of `tiles` tiles of 64 tokens x 128 rows and up to max_per 256-blocks a piece, 0: no.  Four waves
+/* The pieces of such a launch in place of one of tiles of 64 tokens x 128 rows, up to max_per 256-blocks a piece, 0: no.  Four waves
  * fill a CU's LDS, so every block gets a place at once: a second round would cost more than the second launch it saves (Q4_K, 300 tokens x 3840 x
  * 2000: 320 blocks of three waves). */
-static int gemm_ksplit_pieces(const GemmArgs &g, int tiles, int max_per)
+constexpr int GEMM_KSPLIT_Q4K = 7, GEMM_KSPLIT_Q5K = 9, GEMM_KSPLIT_Q6K = 7;       /* measured at the kernels */
+static int gemm_ksplit_pieces(int M, long N, int nb, int max_per)
 {
-    const int s = gemm_choose_splits(tiles, g.nb), per = (g.nb + s - 1) / s, k = (g.nb + per - 1) / per;
-    return k >= 2 && k <= 4 && per <= max_per && g.ntt * ((g.N + 31) / 32) <= (k == 2 ? 512 : 256) ? k : 0;
+    const long ntt = (M + 63) / 64, tiles = ntt * ((N + GEMM_TILE_ROWS - 1) / GEMM_TILE_ROWS);
+    if (tiles >= 160) return 0;
+    const int s = gemm_choose_splits((int)tiles, nb), per = (nb + s - 1) / s, k = (nb + per - 1) / per;
+    return k >= 2 && k <= 4 && per <= max_per && ntt * ((N + 31) / 32) <= (k == 2 ? 512 : 256) ? k : 0;
 }
 template <class Kernel>
 static int gemm_launch_ksplit(Kernel k2, Kernel k3, Kernel k4, GemmArgs &g, int k, hipStream_t s)

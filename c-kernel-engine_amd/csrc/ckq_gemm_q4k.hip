@@ -546,7 +546,7 @@ int launch_gemm_q4k_mfma(const void *A, const void *B, const float *bias, float 
 #endif
     }
     if (two_groups) return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 2>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s, 512);
-    if (const int k = gemm_ksplit_pieces(g, tiles, 7)) return gemm_launch_ksplit(gemm_q4k_ksplit_kernel<2>, gemm_q4k_ksplit_kernel<3>, gemm_q4k_ksplit_kernel<4>, g, k, s);
+    if (const int k = gemm_ksplit_pieces(M, N, g.nb, GEMM_KSPLIT_Q4K)) return gemm_launch_ksplit(gemm_q4k_ksplit_kernel<2>, gemm_q4k_ksplit_kernel<3>, gemm_q4k_ksplit_kernel<4>, g, k, s);
     const GemmGroupIn one = {1, {B}, {bias}, {C}, {N}, {ldc}};
     if (tiles > 256 && gemm_ragged_last(one, M, GEMM_BM)) return gemm_launch_ragged_last(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 1>, g, one, GEMM_BM, s);
     return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 1>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s, 256);

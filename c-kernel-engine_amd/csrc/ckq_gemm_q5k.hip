@@ -579,7 +579,7 @@ int launch_gemm_q5k_mfma(const void *A, const void *B, const float *bias, float 
 #else
     if (sums) return CKQ_ENODUMP;
 #endif
-    if (const int k = gemm_ksplit_pieces(g, g.ntt * g.nnt, 9)) return gemm_launch_ksplit(gemm_q5k_ksplit_kernel<2>, gemm_q5k_ksplit_kernel<3>, gemm_q5k_ksplit_kernel<4>, g, k, s);
+    if (const int k = gemm_ksplit_pieces(M, N, g.nb, GEMM_KSPLIT_Q5K)) return gemm_launch_ksplit(gemm_q5k_ksplit_kernel<2>, gemm_q5k_ksplit_kernel<3>, gemm_q5k_ksplit_kernel<4>, g, k, s);
     return gemm_launch_split(gemm_q5k_mfma_kernel<false>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s);
 }
 

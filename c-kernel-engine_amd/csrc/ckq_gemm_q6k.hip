@@ -601,7 +601,7 @@ int launch_gemm_q6k_mfma(const void *A, const void *B, const float *bias, float 
     }
     if (form == Q6K_PAIRED) return gemm_launch_split(gemm_q6k_pair_kernel<2>, g, grid, g.nb, s);
     if (form == Q6K_128) return gemm_launch_split(gemm_q6k_mfma_kernel<4>, g, grid, g.nb, s);
-    if (const int k = gemm_ksplit_pieces(g, g.ntt * g.nnt, 7)) return gemm_launch_ksplit(gemm_q6k_ksplit_kernel<2>, gemm_q6k_ksplit_kernel<3>, gemm_q6k_ksplit_kernel<4>, g, k, s);
+    if (const int k = gemm_ksplit_pieces(M, N, g.nb, GEMM_KSPLIT_Q6K)) return gemm_launch_ksplit(gemm_q6k_ksplit_kernel<2>, gemm_q6k_ksplit_kernel<3>, gemm_q6k_ksplit_kernel<4>, g, k, s);
     return gemm_launch_split(gemm_q6k_mfma_kernel<2>, g, grid, g.nb, s);
 }
 

@@ -292,6 +292,12 @@ static bool weights_dword_aligned(const GemvArgs &a, const GemvGroup &grp)
  *   tiles      11 + 0.2 mb + 0.0015 tokens mb, an under-estimate almost everywhere; against groups in pairs Q5_K 13.3 + 0.164 mb + 0.0048 tokens mb and
  *              Q6_K 13.8 + 0.083 mb + 0.0044 tokens mb (11 % rms over 207 launches of 9 to 200 tokens, where the first cost 4.1 and 7.3 % more than the
  *              faster kernel and these cost 1.5 and 0.6; Q4_K's own fit would cost 5.2 instead of 1.0)
+ *   K split    where the pieces of K are waves of a block (gemm_ksplit_pieces), fitted to 450 launches of 17 to 700 tokens, 5 to 11 % rms: 4.1 + 1.44 per + 0.16 mb + 3.3 out
+ *              (per: 256-blocks of a piece, out: millions of outputs; Q5_K 3.7, 1.83, 0.12, 2.8, Q6_K 3.75, 1.73, 0.18, 3.7), and rows16 there 3.4 + 0.11 nb +
+ *              0.6 n16 (2.8, 0.154, 0.85; 2.8, 0.26, 0.22), groups in pairs 3.7 + (0.135 + 0.135 blocks on a CU) nb (3.4, 0.09, 0.32; 4.6, -0.024,
+ *              0.344).  By the estimates above the choice cost 5.6, 7.1 and 4.5 % more than the faster kernel, single sizes 48; by these 0.4 (us: Q4_K 172 tokens x 2560 x 3385
+ *              18.8 -> 13.5, Q5_K 146 x 3840 x 2084 18.7 -> 13.7, Q6_K 329 x 3328 x 1257 20.2 -> 13.7).  Not for calls that bring their scratch: which of
+ *              them are refused for want of it stays as it was (`own_scratch`), and no call on the K split is refused that a 16-row kernel took.
  *   streaming  above eight tokens the larger of 2.9 and 2.2 + 0.0075 lanes + (23.5, 23.5, 29) million lanes of all rows and passes,
  *              a row's 64-element positions being dealt to 8, 16, 32 or 64 lanes or to 2 to 4 passes of 64 (stream_lanes): small
  *              matrices stream at up to some 60 tokens (Q5_K 290 x 1792 at 25: 3.0, here 4.6; Q6_K 435 x 1536 at 13 3.0, here 4.8);
@@ -314,7 +320,7 @@ extern "C" void ckq_launch_set_rows16(int fmt, int on)
     if (on) g_rows16_forced.fetch_or(1 << fmt);
     else g_rows16_forced.fetch_and(~(1 << fmt));
 }
-static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles, int launches = 1)
+static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles, int launches = 1, bool own_scratch = false)
 {
     if (ntok < 2 || K > ROWS16_MAX_K) return false;
     if (g_rows16_forced.load(std::memory_order_relaxed) >> fmt & 1) return true;
@@ -330,6 +336,17 @@ static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles, int l
     const float t_pair = tiles && t_keep <= 0.0f ? gemm_rows16_pair_time(fmt, rows, ntok, K / 256) : 0.0f;
     const float t_rows = t_keep > 0.0f ? t_keep : t_pair > 0.0f ? t_pair : 3.6f + 0.12f * nb + per_block[f] * 1e-3f * nb * (float)((rows + 15) / 16) * (float)((ntok + 15) / 16);
     float t_else;
+    if (const int pieces = tiles && launches == 1 && !own_scratch && rows < 1 << 24
+                               ? gemm_ksplit_pieces(ntok, (long)rows, K / 256, f == 0 ? GEMM_KSPLIT_Q4K : f == 1 ? GEMM_KSPLIT_Q5K : GEMM_KSPLIT_Q6K) : 0) {
+        static const float split[3][4] = {{4.1f, 1.44f, 0.16f, 3.3f}, {3.7f, 1.83f, 0.12f, 2.8f}, {3.75f, 1.73f, 0.18f, 3.7f}},
+                           single[3][3] = {{3.4f, 0.11f, 0.6f}, {2.8f, 0.154f, 0.85f}, {2.8f, 0.26f, 0.22f}},
+                           pair[3][3] = {{3.7f, 0.135f, 0.135f}, {3.4f, 0.09f, 0.32f}, {4.6f, -0.024f, 0.344f}};
+        const float r16 = (float)((rows + 15) / 16), groups = (float)((ntok + 15) / 16), per = (float)((K / 256 + pieces - 1) / pieces);
+        const float t = split[f][0] + split[f][1] * per + split[f][2] * mb + split[f][3] * 1e-6f * (float)ntok * (float)rows;
+        if (t_keep > 0.0f) return t_keep < t;
+        if (t_pair > 0.0f) return pair[f][0] + (pair[f][1] + pair[f][2] * fmaxf(r16 * (float)((ntok + 31) / 32) / 256.0f, 1.0f)) * nb < t;
+        return single[f][0] + single[f][1] * nb + single[f][2] * 1e-3f * nb * r16 * groups < t;
+    }
     if (tiles) t_else = f == 0 || t_pair <= 0.0f ? 11.0f + (0.2f + 0.0015f * (float)ntok) * mb : f == 1 ? 13.3f + (0.164f + 0.0048f * (float)ntok) * mb : 13.8f + (0.083f + 0.0044f * (float)ntok) * mb;
     else if (ntok <= 8) t_else = fmaxf(3.5f + 0.07f * nb, 3.05f + 0.11f * nb + 1.25f * per_pass[f] * mb);
     else {
@@ -346,13 +363,13 @@ static bool kquant_on_matrix_cores(int fmt, int ntok, size_t rows, int K)
 }
 
 /* Where a matmul of a whole matrix goes. */
-extern "C" int ckq_launch_route(int fmt, int nrows, int K, int ntok, int aligned)
+static int launch_route(int fmt, int nrows, int K, int ntok, int aligned, bool own_scratch)
 {
     bool tiles;
     switch (fmt) {
     case CKQ_FMT_Q4_K: case CKQ_FMT_Q5_K: case CKQ_FMT_Q6_K:
         tiles = kquant_on_matrix_cores(fmt, ntok, (size_t)nrows, K);
-        if (take_rows16(fmt, ntok, (size_t)nrows, K, tiles)) return tiles ? CKQ_ROUTE_ROWS16_TILES : CKQ_ROUTE_ROWS16_STREAM;
+        if (take_rows16(fmt, ntok, (size_t)nrows, K, tiles, 1, own_scratch)) return tiles ? CKQ_ROUTE_ROWS16_TILES : CKQ_ROUTE_ROWS16_STREAM;
         break;
     case CKQ_FMT_Q8_0: tiles = gemm_q80_on_matrix_cores(ntok, (size_t)nrows * (K / 32) * 34, K % 64 == 0 && aligned); break;
     case CKQ_FMT_Q5_0: tiles = gemm_on_matrix_cores(ntok, (size_t)nrows * (K / 32) * 22, 20); break;
@@ -361,6 +378,8 @@ extern "C" int ckq_launch_route(int fmt, int nrows, int K, int ntok, int aligned
     }
     return tiles ? CKQ_ROUTE_TILES : CKQ_ROUTE_STREAM;
 }
+
+extern "C" int ckq_launch_route(int fmt, int nrows, int K, int ntok, int aligned) { return launch_route(fmt, nrows, K, ntok, aligned, false); }
 
 /* The chains of multiply-adds of such a launch: those of the tile kernel where it stands in for one, so that the result
  * has the tile kernel's bits. */
@@ -551,7 +570,7 @@ static int launch_gemv_args(int fmt_flags, GemvArgs &a, const GemvGroup &grp, in
     const bool dump = a.sub != nullptr;
     const bool whole = !dump && grp.n == 1 && row0 == 0 && row1 == nrows;   /* what a matrix-core GEMM can take */
     const bool aligned = weights_dword_aligned(a, grp);
-    const int route = whole ? ckq_launch_route(fmt, nrows, K, ntok, aligned) : CKQ_ROUTE_STREAM;
+    const int route = whole ? launch_route(fmt, nrows, K, ntok, aligned, opts.scratch != nullptr) : CKQ_ROUTE_STREAM;
     switch (fmt) {
     case CKQ_FMT_Q4_K:
         if (K % 256) return CKQ_ESHAPE;

@@ -1782,7 +1782,8 @@ def test_16_row_tiles_of_several_token_groups_copied_to_lds(fmt):
 def test_k_split_whose_pieces_meet_in_lds(fmt):
     """Two, three and four pieces of K, of two blocks and more, the last one shorter; one token and one row more than a tile, a single row; as many
     blocks as the CUs have places for.  Bit for bit the chains of the tile kernels as the 16-row tiles run them, within the tolerance the oracle's result, nothing outside the
-    matrix; and the entry point that allocates nothing refuses what it refused when the partial tiles lay in memory."""
+    matrix; and the entry point that allocates nothing refuses what it refused when the partial tiles lay in memory, and takes what the
+    16-row tiles took although others go to the K split now."""
     import torch
     L = ckq.lib()
     tag = P.FMT[fmt]
@@ -1807,10 +1808,11 @@ def test_k_split_whose_pieces_meet_in_lds(fmt):
             if M * N * K < 1 << 28:
                 want = T.oracle_gemm_nt(fmt, xq.cpu().numpy(), Wh, bias.cpu().numpy(), M, N, K)
                 assert T.norm_err(call(False).cpu().numpy(), want) <= TOL
-        for M, N, nb, refused in [(512, 896, 19, True), (65, 33, 9, False)]:
+        for M, N, nb, refused in [(512, 896, 19, True), (65, 33, 9, False), {"q4_k": (172, 3385, 10, False), "q5_k": (182, 3139, 10, False), "q6_k": (191, 3084, 10, False)}[fmt]]:
             K = nb * 256
             xq, W = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, seed=3)), "q8_k", rows=M), P.to_device(T.random_blocks(fmt, N * nb, 9750))
             L.ckq_set_prefill_variant(tag, 0)
+            L.ckq_set_gemm_policy(0)
             c = torch.full((M, N), 7.0, device="cuda")
             rc = L.ckq_gemm_nt_noalloc_dev(tag, P._dp(xq), P._dp(W), None, P._dp(c), M, N, K, N, P._stream())
             assert (rc != 0) == refused and bool((c == 7.0).all()) == refused, (rc, M, N)
