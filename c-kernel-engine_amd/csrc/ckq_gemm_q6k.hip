@@ -450,8 +450,8 @@ __global__ void __launch_bounds__(256, 2) gemm_q6k_pair_kernel(GemmArgs a)
 }
 
 /* K split among the waves of a block, as gemm_q4k_ksplit_kernel has it: 64 tokens x 32 rows, a wave a piece of K, 39.5 KB of LDS each.  The next
- * block's rows fill the one image once the wave has the last ones in registers; copies in memory order, two a slot until all rows and half of the quants are on
- * their way.  us against partial tiles in memory (tokens, K, rows): 512 x 4864 x 896 20.3 -> 18.1, 512 x 2048 x 2048 19.3 -> 14.2, 131 x 4096 x 2250 18.0 -> 15.6; 37 launches
+ * block's rows fill the one image once the wave has the last ones in registers; copies in memory order, three a slot, so that all are on their way by the
+ * middle of the block (over all of it, as Q4_K has them: 512 x 4864 x 896 18.2 us instead of 17.2, 100 x 2048 x 600 11.1 instead of 10.6; Q4_K loses 3 % this way).  us against partial tiles in memory (tokens, K, rows): 512 x 4864 x 896 20.3 -> 17.2, 512 x 2048 x 2048 19.3 -> 14.2, 128 x 4096 x 4096 18.0 -> 15.5; 37 launches
  * of four to seven 256-blocks a piece 1.22 on average, 1.05 and more; of eight 1.04, of nine to 21 0.87 to 0.96 (a 256-block takes a lone wave 2.3 us here, 1.6 where
  * three stages are shared). */
 template <int SPLITS>
@@ -470,7 +470,7 @@ __global__ void __launch_bounds__(64 * SPLITS, 1) gemm_q6k_ksplit_kernel(GemmArg
     const ckq_v4i rs_w = gemm_buffer(a.B + (size_t)n0 * wstride), rs_x = gemm_buffer(a.A + (size_t)t0 * xstride);
 
     constexpr int NW = 7, NQ = BM / 4, NC = NW + NQ + 1;      /* copies of a 256-block: rows, quants of four tokens each, scales */
-    static_assert(NW * 64 == 32 * 14 && NC == 24, "eight slots of two copies and eight of one");
+    static_assert(NW * 64 == 32 * 14 && NC == 24, "eight slots of three copies");
     u32 wofs[NW], qofs[NQ];
     auto token = [&](int t) { return (u32)min(t, a.M - 1 - t0) * xstride; };
 #pragma unroll
@@ -514,8 +514,7 @@ __global__ void __launch_bounds__(64 * SPLITS, 1) gemm_q6k_ksplit_kernel(GemmArg
         Gemm6Sums<2> sums;
         gemm6_slabs<2, 16>(xs[wave][cur], ds[wave][cur], head, aofs, half, sums, [&](int i) __attribute__((always_inline)) {
             const int slot = 2 * (i & 7) + (i >> 3);          /* in time: i and i + 8 are the two of a slab */
-            if (slot < 8) { copy(bn, cur ^ 1, 2 * slot); copy(bn, cur ^ 1, 2 * slot + 1); }
-            else copy(bn, cur ^ 1, 8 + slot);
+            if (slot < 8) { copy(bn, cur ^ 1, 3 * slot); copy(bn, cur ^ 1, 3 * slot + 1); copy(bn, cur ^ 1, 3 * slot + 2); }
         });
         __builtin_amdgcn_sched_barrier(0);
         landed();
