@@ -451,7 +451,7 @@ __global__ void __launch_bounds__(256, 2) gemm_q6k_pair_kernel(GemmArgs a)
 
 /* K split among the waves of a block, as gemm_q4k_ksplit_kernel has it: 64 tokens x 32 rows, a wave a piece of K, 39.5 KB of LDS each.  The next
  * block's rows fill the one image once the wave has the last ones in registers; copies in memory order, three a slot, so that all are on their way by the
- * middle of the block (over all of it, as Q4_K has them: 512 x 4864 x 896 18.2 us instead of 17.2, 100 x 2048 x 600 11.1 instead of 10.6; Q4_K loses 3 % this way).  us against partial tiles in memory (tokens, K, rows): 512 x 4864 x 896 20.3 -> 17.2, 512 x 2048 x 2048 19.3 -> 14.2, 128 x 4096 x 4096 18.0 -> 15.5; 37 launches
+ * middle of the block (over all of it, as Q4_K has them: 512 x 4864 x 896 18.2 us instead of 17.2, 100 x 2048 x 600 11.1 instead of 10.6; Q4_K loses 3 % this way).  us against partial tiles in memory (tokens, K, rows): 512 x 4864 x 896 20.3 -> 17.2, 512 x 2048 x 2048 19.8 -> 14.2; 37 launches
  * of four to seven 256-blocks a piece 1.22 on average, 1.05 and more; of eight 1.04, of nine to 21 0.87 to 0.96 (a 256-block takes a lone wave 2.3 us here, 1.6 where
  * three stages are shared). */
 template <int SPLITS>
