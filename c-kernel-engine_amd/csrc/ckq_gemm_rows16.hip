@@ -1132,28 +1132,34 @@ int launch_rows16_nt(int fmt, Rows16Args &a, hipStream_t s)
     return (int)hipGetLastError();
 }
 
-/* Blocks per row tile of the kernel that keeps its planes, 0: the other kernel; its time in us.  Both times are fitted to launches
- * of 1024 x 1024 to 12000 x 2048, 17 to 256 tokens, one to eight blocks a row tile, mostly within 15 %: here 2.5 (Q4_K 3) +
- * (groups of a block + 1.5) (0.45 + 0.27 waves a SIMD of the fullest CU + 0.25 (4 / nb - 1) where nb < 4), there 3.2 + 0.15 nb +
- * (a nb + b) thousands of tiles.  Against the other kernel (us): Q5_K 4864 x 1024 at 64 / 96 / 128 tokens 8.3 -> 6.5,
- * 10.8 -> 7.9, 10.9 -> 8.6, 12000 x 1024 at 32 / 96 9.8 -> 6.8, 19.0 -> 11.6, 4096 x 2048 at 96 12.0 -> 9.1; Q6_K 11008 x 2048
- * at 64 22.0 -> 16.4; Q4_K, whose planes are quickly formed, 12000 x 1024 at 64 11.1 -> 8.7.  It loses where the other's waves
- * have a SIMD to themselves anyway (Q4_K 1782 x 1536 at 43: 5.1 against 7.0) and for Q4_K rows of five blocks and more (11008 x 2048
- * at 32: 9.6 against 10.3). */
-int rows16_keep_parts(int fmt, long tiles, int groups, int nb, float *time)
+/* Blocks per row tile of the kernel that keeps its planes, 0: another kernel; its time in us.  With n blocks on the fullest CU, as many at once as sixteen waves
+ * are, a block takes (its groups + per0) (a + short_row (1 / nb - 1/4) where nb < 4 + s waves a SIMD), what comes after the first round `later` of that, a launch t0 more; the
+ * other kernels together 3.3..3.8 + ...: `other`, by nb and by thousands of tiles of 16 rows and tokens.  Fitted to 210 launches of 16 to 224 x 16 tokens and rows up to 14000, one to
+ * eight blocks a row tile, in either order of the sums: 6 to 7 % rms (other: 7 to 11).  Over further launches the choice costs 0.2 to 0.5 % more than the best of all in
+ * the streaming kernel's order, 0.9 to 2.6 in the tile kernels'; an older fit, to an older kernel and without rounds, cost 7.2 to 16.4 and 2.4 to 6.0, at most 75 (us: Q4_K 4630 x 512 at
+ * 82 tokens 7.0 -> 5.1, Q5_K 993 x 256 at 194 6.0 -> 4.2, 2069 x 1280 at 219 9.7 -> 8.4). */
+struct KeepFit { float t0, per0, a, s, short_row, later, other[4]; };
+const KeepFit keep_fit[3][2] = {
+    {{2.21f, 0.56f, 0.55f, 0.315f, 0.60f, 0.92f, {3.35f, -0.072f, 0.334f, 1.65f}}, {2.11f, 0.88f, 0.50f, 0.318f, 0.30f, 0.81f, {3.74f, 0.022f, 0.363f, 1.97f}}},
+    {{1.84f, 1.65f, 0.64f, 0.246f, 0.41f, 0.72f, {3.27f, 0.115f, 0.571f, 1.22f}}, {1.66f, 2.00f, 0.57f, 0.230f, 0.26f, 0.68f, {3.82f, 0.088f, 0.706f, 1.49f}}},
+    {{2.25f, 1.68f, 0.55f, 0.238f, 0.53f, 0.65f, {2.73f, 0.197f, 0.632f, 1.40f}}, {2.01f, 2.40f, 0.42f, 0.201f, 0.22f, 0.86f, {3.82f, 0.075f, 0.850f, 0.45f}}}};
+int rows16_keep_parts(int fmt, bool tree, long tiles, int groups, int nb, float *time)
 {
     if (nb > (fmt == CKQ_FMT_Q4_K ? 4 : KEEP_NB) || groups < 2 || tiles > 1 << 20 || groups > 1 << 10) return 0;
+    const KeepFit &f = keep_fit[fmt == CKQ_FMT_Q4_K ? 0 : fmt == CKQ_FMT_Q5_K ? 1 : 2][tree];
+    const int at_once = 16 / nb;
+    const float block = f.a + (nb < 4 ? f.short_row * (1.0f / (float)nb - 0.25f) : 0.0f), wave = 0.25f * f.s * (float)nb;
     int best = 0;
     float least = 0.0f;
-    for (int parts = 1; parts <= groups / 2 + 1; ++parts) {
-        const int per = (groups + parts - 1) / parts;
-        if (per < 2) break;
-        const float waves = 0.25f * (float)((tiles * parts + 255) / 256) * (float)nb;
-        const float t = (fmt == CKQ_FMT_Q4_K ? 3.0f : 2.5f) + (1.5f + (float)per) * (0.45f + 0.27f * waves + (nb < 4 ? 1.0f / (float)nb - 0.25f : 0.0f));
-        if (!best || t <= least) { least = t; best = (groups + per - 1) / per; }
+    for (int per = groups; per >= 1; --per) {
+        const int parts = (groups + per - 1) / per;
+        if (per > 1 && (groups + per - 2) / (per - 1) == parts) continue;          /* fewer groups a block in as many blocks */
+        const long n = (tiles * parts + 255) / 256, full = n / at_once, rest = n % at_once;
+        const float t = f.t0 + ((float)per + f.per0) * ((float)full * (block + wave * (float)at_once) + (rest ? (block + wave * (float)rest) * (full ? f.later : 1.0f) : 0.0f));
+        if (!best || t < 1.02f * least) { least = best ? std::min(t, least) : t; best = parts; }       /* of two alike the shorter blocks */
     }
-    const float a = fmt == CKQ_FMT_Q4_K ? 0.29f : fmt == CKQ_FMT_Q5_K ? 0.36f : 0.59f, b = fmt == CKQ_FMT_Q4_K ? 1.6f : fmt == CKQ_FMT_Q5_K ? 2.1f : 1.1f;
-    if (least >= 3.2f + 0.15f * (float)nb + 1e-3f * (a * (float)nb + b) * (float)(tiles * groups)) return 0;
+    const float n16 = 1e-3f * (float)(tiles * groups);
+    if (least >= f.other[0] + f.other[1] * (float)nb + (f.other[2] * (float)nb + f.other[3]) * n16) return 0;
     if (time) *time = least;
     return best;
 }
@@ -1238,12 +1244,12 @@ int launch_rows16_hold(Rows16Args &a, int tiles, int grid, int round, size_t lds
  * could be two CUs), past that it wins while the pairs still do: Q4_K 1.01-1.36, Q5_K 1.12-1.45, Q6_K 1.22-1.67, in the streaming kernel's order 0.99-1.15 (there twelve waves
  * are 2-4 % ahead of eight).  With more pairs than CUs, eight waves: Q6_K 1.18-1.37 on average (0.94-1.61), Q5_K 1.07-1.16 but for three groups, 0.97;
  * Q4_K, whose planes are quickly formed, 0.92-1.09, and the streaming kernel's order 0.72-0.83.  Rows of which only one such block fits a CU lose too
- * (Q5_K 914 x 7168 at 175: tile kernel 18.6, this 23.2). */
+ * (Q5_K 914 x 7168 at 175: tile kernel 18.6, this 23.2), and rows of up to four blocks, which have as many waves (Q4_K 2757 x 256 at 28: 5.1, planes kept 3.7). */
 int rows16_pair_waves(int fmt, bool tree, long tiles, int groups, int nb, size_t *lds)
 {
     const int wide = tree && nb > 16 ? nb - 16 : 0;
     const long pairs = tiles * ((groups + 1) / 2);
-    if (groups < 2 || groups > 1 << 10 || tiles * groups <= 256 || wide > 16) return 0;
+    if (nb < 5 || groups < 2 || groups > 1 << 10 || tiles * groups <= 256 || wide > 16) return 0;
     if (pairs > 256 && (tree || fmt == CKQ_FMT_Q4_K || (fmt == CKQ_FMT_Q5_K && groups == 3))) return 0;
     const int waves = std::min(pairs <= 256 ? 12 : 8, nb);
     const size_t pitch = fmt == CKQ_FMT_Q4_K ? R16Q4K::PITCH : fmt == CKQ_FMT_Q5_K ? R16Q5K::PITCH : R16Q6K::PITCH;
@@ -1289,7 +1295,7 @@ int launch_rows16(int fmt, Rows16Args &a, hipStream_t s)
     for (int i = 0; i < a.n; ++i) tiles += (a.p[i].N + 15) / 16;
     bool near = true;                              /* the kernel that keeps its planes has 32 bits for where a group's outputs lie */
     for (int i = 0; i < a.n; ++i) near = near && a.p[i].ldy < 1 << 25;
-    const int parts = near ? rows16_keep_parts(fmt, tiles, (a.M + 15) / 16, a.nb, nullptr) : 0;
+    const int parts = near ? rows16_keep_parts(fmt, a.tree, tiles, (a.M + 15) / 16, a.nb, nullptr) : 0;
     if (parts) return a.tree ? launch_rows16_keep<F, true>(a, parts, s) : launch_rows16_keep<F, false>(a, parts, s);
     int grid, round;
     size_t lds;
@@ -1303,10 +1309,10 @@ int launch_rows16(int fmt, Rows16Args &a, hipStream_t s)
 
 } // namespace
 
-float gemm_rows16_keep_time(int fmt, size_t rows, int ntok, int nb)
+float gemm_rows16_keep_time(int fmt, bool tree, size_t rows, int ntok, int nb)
 {
     float t = 0.0f;
-    return rows16_keep_parts(fmt, (long)((rows + 15) / 16), (ntok + 15) / 16, nb, &t) ? t : 0.0f;
+    return rows16_keep_parts(fmt, tree, (long)((rows + 15) / 16), (ntok + 15) / 16, nb, &t) ? t : 0.0f;
 }
 
 /* Fitted to the launches of the rule above in the tile kernels' order, 12-15 % rms. */

@@ -44,7 +44,7 @@ struct Rows16Args {
     Rows16Problem p[GEMM_GROUP_MAX];
 };
 /* Estimated time in us of such a launch where its kernel for short rows and several token groups runs, else 0. */
-float gemm_rows16_keep_time(int fmt, size_t rows, int ntok, int nb);
+float gemm_rows16_keep_time(int fmt, bool tree, size_t rows, int ntok, int nb);
 /* The same for its kernel that takes token groups in pairs, in the order of the tile kernels. */
 float gemm_rows16_pair_time(int fmt, size_t rows, int ntok, int nb);
 /* One launch over a.n problems of one format, width and token count (id0 is filled in). */

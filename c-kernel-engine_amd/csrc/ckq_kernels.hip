@@ -320,6 +320,19 @@ extern "C" void ckq_launch_set_rows16(int fmt, int on)
     if (on) g_rows16_forced.fetch_or(1 << fmt);
     else g_rows16_forced.fetch_and(~(1 << fmt));
 }
+/* gemm_rows16_keep_time as it was fitted before, for calls that bring their scratch: rows of eight blocks are the only ones that this kernel and a split of K
+ * both take, and which calls are refused for want of scratch is not to follow an estimate of time. */
+static float keep_time_own_scratch(int f, size_t rows, int ntok)
+{
+    const long tiles = (long)((rows + 15) / 16), groups = (ntok + 15) / 16;
+    if (f == 0 || groups < 2 || tiles > 1 << 20) return 0.0f;
+    float least = 0.0f;
+    for (long parts = 1; (groups + parts - 1) / parts >= 2; ++parts) {
+        const float t = 2.5f + (1.5f + (float)((groups + parts - 1) / parts)) * (0.45f + 0.54f * (float)((tiles * parts + 255) / 256));
+        if (parts == 1 || t <= least) least = t;
+    }
+    return least < 4.4f + 1e-3f * (f == 1 ? 4.98f : 5.82f) * (float)(tiles * groups) ? least : 0.0f;
+}
 static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles, int launches = 1, bool own_scratch = false)
 {
     if (ntok < 2 || K > ROWS16_MAX_K) return false;
@@ -332,7 +345,7 @@ static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles, int l
     const float nb = (float)(K / 256), mb = (float)rows * nb * (f == 0 ? 144e-6f : f == 1 ? 176e-6f : 210e-6f);
     const int lanes = stream_lanes(K / 64);
     if (ntok <= 4) return f == 2 && K > 4096 && mb >= 20.0f && 10 * lanes >= 11 * (K / 64);
-    const float t_keep = ntok <= 256 ? gemm_rows16_keep_time(fmt, rows, ntok, K / 256) : 0.0f;
+    const float t_keep = ntok > 256 ? 0.0f : own_scratch && tiles && K == 2048 ? keep_time_own_scratch(f, rows, ntok) : gemm_rows16_keep_time(fmt, !tiles, rows, ntok, K / 256);
     const float t_pair = tiles && t_keep <= 0.0f ? gemm_rows16_pair_time(fmt, rows, ntok, K / 256) : 0.0f;
     const float t_rows = t_keep > 0.0f ? t_keep : t_pair > 0.0f ? t_pair : 3.6f + 0.12f * nb + per_block[f] * 1e-3f * nb * (float)((rows + 15) / 16) * (float)((ntok + 15) / 16);
     float t_else;

@@ -1824,6 +1824,36 @@ def test_k_split_whose_pieces_meet_in_lds(fmt):
 
 
 @pytest.mark.parametrize("fmt", ["q4_k", "q5_k", "q6_k"])
+def test_16_row_tiles_with_planes_kept_for_one_group(fmt):
+    """Few row tiles and many groups: the kernel that keeps its planes in blocks of one group each, and of two, the last of one; one block a row to
+    eight.  In both orders bit for bit."""
+    import torch
+    L = ckq.lib()
+    tag = P.FMT[fmt]
+    try:
+        for M, N, K in [(113, 40, 256), (194, 993, 256), (50, 300, 768), (33, 17, 1024), (82, 4630, 512), (250, 90, 2048), (219, 2069, 1280), (256, 16, 1792)]:
+            xq = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, seed=M)), "q8_k", rows=M)
+            W, bias = P.to_device(T.random_blocks(fmt, N * K // 256, 9560 + M)), P.to_device(T.normal(N, 0.0, 0.5, seed=N))
+            say("16-row tiles, planes kept for one group", fmt, M, N, K)
+
+            def call(policy, forced):
+                L.ckq_set_prefill_variant(tag, 16 if forced else 0)
+                L.ckq_set_gemm_policy(policy)
+                return P.dev_gemm_nt(fmt, xq, W, bias, M, N, K).view(M, N).clone()
+            tree, chain, tiles = call(2, True), call(1, True), call(1, False)
+            assert torch.equal(chain, tiles), (M, N, K)
+            L.ckq_set_prefill_variant(tag, 0)
+            L.ckq_set_gemm_policy(0)
+            rb = xq.numel() // M
+            for m in {0, 15, 16, M // 2, M - 1}:
+                one = P.dev_gemm_nt(fmt, xq[m * rb:(m + 1) * rb].clone(), W, bias, 1, N, K)
+                assert torch.equal(tree[m], one.view(N)), (M, N, K, m)
+    finally:
+        L.ckq_set_gemm_policy(0)
+        L.ckq_set_prefill_variant(tag, 0)
+
+
+@pytest.mark.parametrize("fmt", ["q4_k", "q5_k", "q6_k"])
 def test_16_row_tiles_alone_on_their_cu(fmt):
     """Row tiles that have a CU each, one token group and rows too few for groups in pairs: blocks of eight waves, of twelve and (rows longer than
     the LDS has room for) in between; fewer 256-blocks than waves in the last turn, one, and none.  In the tile kernels' order bit for bit what
