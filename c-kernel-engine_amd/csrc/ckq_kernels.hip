@@ -974,14 +974,13 @@ extern "C" int ckq_launch_rmsnorm_q8_k_fused(const float *input, const float *ga
 /* ========================================================================= */
 
 /* Elements of a quantized row with the reference's operation order; products and differences are rounded one by one
- * (reference: dequant_kernels.c:276-296 Q8_0, :336-385 Q4_K, :396-430 Q6_K).  A thread takes unit `u` of the row, what one load of its
- * quants holds, as runs of four elements: run i is elements at(u, i) .. + 3. */
-template <int FMT> struct DequantUnit;
+ * (reference: dequant_kernels.c:276-296 Q8_0, :336-385 Q4_K, :396-430 Q6_K).  A thread takes unit `u` of the row, RUNS runs of
+ * four elements: run i is elements at(u, i) .. + 3. */
+template <int FMT, int RUNS> struct DequantUnit;
 
-template <> struct DequantUnit<CKQ_FMT_Q8_0> {
-    static constexpr int RUNS = 1;
+template <> struct DequantUnit<CKQ_FMT_Q8_0, 1> {
     static __device__ __forceinline__ u32 at(u32 u, int) { return 4 * u; }
-    static __device__ __forceinline__ void get(float4 (&v)[RUNS], const uint8_t *row, u32 u)
+    static __device__ __forceinline__ void get(float4 (&v)[1], const uint8_t *row, u32 u)
     {
 #pragma clang fp contract(off)
         const uint8_t *blk = row + (u >> 3) * 34u;
@@ -991,11 +990,43 @@ template <> struct DequantUnit<CKQ_FMT_Q8_0> {
     }
 };
 
+template <> struct DequantUnit<CKQ_FMT_Q4_K, 1> {
+    static __device__ __forceinline__ u32 at(u32 u, int) { return 4 * u; }
+    static __device__ __forceinline__ void get(float4 (&v)[1], const uint8_t *row, u32 u)
+    {
+#pragma clang fp contract(off)
+        const uint8_t *blk = row + (u >> 6) * 144u;
+        const u32 j = (u >> 3) & 7, l = 4 * (u & 7);         /* sub-block j, element l of it */
+        const u32 hdr0 = ld4<4>(blk);
+        u32 sc2, mn2;
+        k4_scale_pair(ld4<4>(blk + 4), ld4<4>(blk + 8), ld4<4>(blk + 12), (int)(j >> 1), &sc2, &mn2);
+        const u32 sc = (sc2 >> (8 * (j & 1))) & 0xff, mn = (mn2 >> (8 * (j & 1))) & 0xff;
+        const float dj = h2f(hdr0 & 0xffff) * (float)sc, mj = h2f(hdr0 >> 16) * (float)mn;
+        const u32 qs = ld4<4>(blk + 16 + 32 * (j >> 1) + l);
+        const u32 nib = (j & 1) ? (qs >> 4) & 0x0f0f0f0fu : qs & 0x0f0f0f0fu;
+        v[0] = make_float4(dj * (float)(nib & 0xff) - mj, dj * (float)((nib >> 8) & 0xff) - mj, dj * (float)((nib >> 16) & 0xff) - mj, dj * (float)(nib >> 24) - mj);
+    }
+};
+
+template <> struct DequantUnit<CKQ_FMT_Q6_K, 1> {
+    static __device__ __forceinline__ u32 at(u32 u, int) { return 4 * u; }
+    static __device__ __forceinline__ void get(float4 (&v)[1], const uint8_t *row, u32 u)
+    {
+#pragma clang fp contract(off)
+        const uint8_t *blk = row + (u >> 6) * 210u;
+        const u32 n = (u >> 5) & 1, r = (u >> 3) & 3, l = 4 * (u & 7);       /* half n, run r, element l */
+        const u32 lo = ld4<2>(blk + 64 * n + l + 32 * (r & 1)), hi = ld4<2>(blk + 128 + 32 * n + l);
+        const u32 q = ((r >> 1) ? (lo >> 4) & 0x0f0f0f0fu : lo & 0x0f0f0f0fu) | (((hi >> (2 * r)) & 0x03030303u) << 4);
+        const float ds = h2f(ld2(blk + 208)) * (float)(int8_t)blk[192 + 8 * n + 2 * r + (l >> 4)];
+        v[0] = make_float4(ds * (float)((int)(q & 0xff) - 32), ds * (float)((int)((q >> 8) & 0xff) - 32),
+                           ds * (float)((int)((q >> 16) & 0xff) - 32), ds * (float)((int)(q >> 24) - 32));
+    }
+};
+
 /* Eight bytes of a 64-element group: their low nibbles are in one sub-block, their high ones in the next. */
-template <> struct DequantUnit<CKQ_FMT_Q4_K> {
-    static constexpr int RUNS = 4;
+template <> struct DequantUnit<CKQ_FMT_Q4_K, 4> {
     static __device__ __forceinline__ u32 at(u32 u, int i) { return 64 * (u >> 2) + 32 * (i >> 1) + 8 * (u & 3) + 4 * (i & 1); }
-    static __device__ __forceinline__ void get(float4 (&v)[RUNS], const uint8_t *row, u32 u)
+    static __device__ __forceinline__ void get(float4 (&v)[4], const uint8_t *row, u32 u)
     {
 #pragma clang fp contract(off)
         const uint8_t *blk = row + (u >> 4) * 144u;
@@ -1016,10 +1047,9 @@ template <> struct DequantUnit<CKQ_FMT_Q4_K> {
 };
 
 /* Four bytes of the high bits of a 128-element half and what belongs to them: one run in each of its four runs of 32. */
-template <> struct DequantUnit<CKQ_FMT_Q6_K> {
-    static constexpr int RUNS = 4;
+template <> struct DequantUnit<CKQ_FMT_Q6_K, 4> {
     static __device__ __forceinline__ u32 at(u32 u, int i) { return 128 * (u >> 3) + 32 * i + 4 * (u & 7); }
-    static __device__ __forceinline__ void get(float4 (&v)[RUNS], const uint8_t *row, u32 u)
+    static __device__ __forceinline__ void get(float4 (&v)[4], const uint8_t *row, u32 u)
     {
 #pragma clang fp contract(off)
         const uint8_t *blk = row + (u >> 4) * 210u;
@@ -1043,29 +1073,27 @@ template <> struct DequantUnit<CKQ_FMT_Q6_K> {
  * source row (ids ? clamp(ids[t]) : t), plus pos[t] where asked, zero from
  * n_valid on; rows from `tokens` on are zero (reference:
  * src/kernels/embedding_kernels.c:76-196).  Bound: two latencies, the id's and its row's, and the stores.
- * Sixteen elements a thread need a third of the loads of four a thread (2000 rows of 8192 Q6_K 22.5 -> 17.3 us, Q4_K 21.0 -> 18.5).
  */
-template <int FMT>
+template <int FMT, int RUNS>
 __global__ void __launch_bounds__(256) dequant_rows_kernel(const uint8_t *__restrict__ table, const int32_t *__restrict__ ids,
-                                                           int vocab, const float *__restrict__ pos, float *__restrict__ out,
-                                                           int n_valid, int n_row, long row_bytes, int tokens, int col_blocks)
+                                                           const float *__restrict__ pos, float *__restrict__ out, int vocab,
+                                                           int n_valid, int n_row, u32 row_bytes, int tokens, u32 col_blocks, u32 width)
 {
-    typedef DequantUnit<FMT> Unit;
-    constexpr int RUNS = Unit::RUNS;
+    typedef DequantUnit<FMT, RUNS> Unit;
     /* the output row rides in blockIdx.x with the column block (gridDim.y stops at 65 535 rows) */
-    const int t = (int)(blockIdx.x / (u32)col_blocks);
-    const u32 u = (blockIdx.x % (u32)col_blocks) * blockDim.x + threadIdx.x;
+    const int t = (int)(blockIdx.x / col_blocks);
+    const u32 u = (blockIdx.x % col_blocks) * width + threadIdx.x;
     if (u >= (u32)n_row / (4 * RUNS)) return;
     float4 v[RUNS];
 #pragma unroll
     for (int i = 0; i < RUNS; ++i) v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
     if (t < tokens) {
-        long src = t;
+        int src = t;
         if (ids) {
             const int id = ids[t];
             src = (id < 0 || id >= vocab) ? 0 : id;
         }
-        Unit::get(v, table + src * row_bytes, u);
+        Unit::get(v, table + (size_t)src * row_bytes, u);
 #pragma unroll
         for (int i = 0; i < RUNS; ++i) {
             const u32 e = Unit::at(u, i);
@@ -1083,6 +1111,23 @@ __global__ void __launch_bounds__(256) dequant_rows_kernel(const uint8_t *__rest
     for (int i = 0; i < RUNS; ++i) *reinterpret_cast<float4 *>(out + (size_t)t * n_row + Unit::at(u, i)) = v[i];
 }
 
+/* Elements a thread takes, and the threads of a block: as many as an equal share of the row needs, whole waves.
+ * Sixteen elements a thread need a third of the loads but leave a quarter of the threads: they win once a launch of four each, 1024 to a block, has
+ * more blocks than the chip holds at once (2048; Q4_K, whose loads are wider as it is, twice that), while a narrow row's sixteens leave lanes of its last wave without work,
+ * all but sixteen of a row of 256.  From 130 launches a format of 1 to 40000 rows, 256 to 8192 wide, random ids (us, four -> sixteen): Q6_K 1024 rows of 4096 7.6 -> 6.3,
+ * 2048 of 8192 24.3 -> 19.0, 1024 of 2048 4.2 -> 4.3, 3000 of 256 3.1 -> 3.5; Q4_K 1500 of 4096 10.0 -> 9.6, 2048 of 8192 23.5 -> 19.7, 384 of 5120 4.0 -> 4.7, 2048
+ * of 1024 4.2 -> 4.7.  The rule's choices are within 1.5 % of the faster form, but for Q4_K 3000 of 1280 (7.2 -> 7.7) and 1024 of 5120 (9.0 -> 9.3).
+ * Blocks of 256 threads whatever the row: four a thread 4096 of 256 3.4 -> 3.8, sixteen a thread 1024 of 5120 Q6_K 7.6 -> 9.5. */
+extern "C" int ckq_launch_dequant_form(int fmt, int n_row, int n_out_rows, int *width)
+{
+    const bool q4 = fmt == CKQ_FMT_Q4_K;
+    const long long most = n_row <= (q4 ? 1024 : 512) ? 8ll << 20 : q4 ? 4ll << 20 : 2ll << 20;
+    const int e = fmt != CKQ_FMT_Q8_0 && n_row >= 512 && (long long)n_row * n_out_rows > most ? 16 : 4;
+    const int units = n_row / e, col_blocks = (units + 255) / 256;
+    *width = ((units + col_blocks - 1) / col_blocks + 63) & ~63;
+    return e;
+}
+
 extern "C" int ckq_launch_dequant_rows(int fmt, const void *table, const int32_t *ids, int vocab, const float *pos,
                                        float *out, int n_valid, int n_row, int tokens, int n_out_rows, void *stream)
 {
@@ -1091,21 +1136,20 @@ extern "C" int ckq_launch_dequant_rows(int fmt, const void *table, const int32_t
     if (n_row % (fmt == CKQ_FMT_Q8_0 ? 32 : 256)) return CKQ_ESHAPE;
     if (tokens > n_out_rows) tokens = n_out_rows;
     if (n_valid > n_row) n_valid = n_row;
-    const long rb = (long)ckq_row_bytes(fmt, n_row);
-    const int units = n_row / (fmt == CKQ_FMT_Q8_0 ? 4 : 16), col_blocks = (units + 255) / 256;
+    const u32 rb = (u32)ckq_row_bytes(fmt, n_row);
+    int width;
+    const bool wide = ckq_launch_dequant_form(fmt, n_row, n_out_rows, &width) == 16;
+    const int col_blocks = (n_row / (wide ? 16 : 4) + 255) / 256;
     if ((long long)col_blocks * n_out_rows > 0x7fffffffll) return CKQ_ESHAPE;
-    const dim3 grid((unsigned)((long long)col_blocks * n_out_rows)), block(256);
+    const dim3 grid((unsigned)((long long)col_blocks * n_out_rows)), block((unsigned)width);
     hipStream_t s = (hipStream_t)stream;
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, block, 0, s, (const uint8_t *)table, ids, pos, out, vocab, n_valid, n_row, rb, tokens, (u32)col_blocks, (u32)width);
+    };
     switch (fmt) {
-    case CKQ_FMT_Q4_K:
-        hipLaunchKernelGGL(dequant_rows_kernel<CKQ_FMT_Q4_K>, grid, block, 0, s, (const uint8_t *)table, ids, vocab, pos, out, n_valid, n_row, rb, tokens, col_blocks);
-        break;
-    case CKQ_FMT_Q6_K:
-        hipLaunchKernelGGL(dequant_rows_kernel<CKQ_FMT_Q6_K>, grid, block, 0, s, (const uint8_t *)table, ids, vocab, pos, out, n_valid, n_row, rb, tokens, col_blocks);
-        break;
-    default:
-        hipLaunchKernelGGL(dequant_rows_kernel<CKQ_FMT_Q8_0>, grid, block, 0, s, (const uint8_t *)table, ids, vocab, pos, out, n_valid, n_row, rb, tokens, col_blocks);
-        break;
+    case CKQ_FMT_Q4_K: launch(wide ? dequant_rows_kernel<CKQ_FMT_Q4_K, 4> : dequant_rows_kernel<CKQ_FMT_Q4_K, 1>); break;
+    case CKQ_FMT_Q6_K: launch(wide ? dequant_rows_kernel<CKQ_FMT_Q6_K, 4> : dequant_rows_kernel<CKQ_FMT_Q6_K, 1>); break;
+    default:           launch(dequant_rows_kernel<CKQ_FMT_Q8_0, 1>); break;
     }
     return (int)hipGetLastError();
 }

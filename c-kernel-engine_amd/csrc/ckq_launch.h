@@ -126,6 +126,9 @@ int ckq_launch_rmsnorm_q8_k_fused(const float *input, const float *gamma, void *
 int ckq_launch_dequant_rows(int fmt, const void *table, const int32_t *ids, int vocab, const float *pos,
                             float *out, int n_valid, int n_row, int tokens, int n_out_rows, void *stream);
 
+/* Elements of a row that a thread of that launch takes, 4 or 16, and the threads of a block (*width).  Host arithmetic; exported for the test of the rule. */
+int ckq_launch_dequant_form(int fmt, int n_row, int n_out_rows, int *width);
+
 /* ckq_launch_gemv for callers that must not allocate: a K-split matrix-core
  * GEMM takes its partial tiles from a static device array of
  * CKQ_NOALLOC_SCRATCH_BYTES instead of the grow-only workspace; a split that

@@ -258,6 +258,16 @@ def test_q6_k_kernel_is_the_fastest_one(L, M, N, K, form):
     assert L.ckq_launch_q6k_form(M, N, K) == form
 
 
+@pytest.mark.parametrize("fmt,n_row,rows,elems,width", [
+    ("q4_k", 256, 512, 4, 64), ("q4_k", 512, 2048, 4, 128), ("q4_k", 4096, 384, 4, 256), ("q4_k", 5120, 384, 4, 256), ("q4_k", 1024, 6000, 4, 256), ("q4_k", 8192, 2048, 16, 256),
+    ("q4_k", 6144, 1024, 16, 192), ("q4_k", 4096, 1500, 16, 256), ("q6_k", 256, 40000, 4, 64), ("q6_k", 1024, 2048, 4, 256), ("q6_k", 512, 10000, 4, 128), ("q6_k", 5120, 1024, 16, 192),
+    ("q6_k", 4096, 700, 16, 256), ("q6_k", 4096, 512, 4, 256), ("q8_0", 896, 20000, 4, 256), ("q8_0", 32, 1, 4, 64)])
+def test_dequantizer_form_is_the_faster_one(L, fmt, n_row, rows, elems, width):
+    """Sizes at which four and sixteen elements a thread were timed against each other; blocks no larger than their share of the row needs."""
+    w = ctypes.c_int()
+    assert (L.ckq_launch_dequant_form(ckq.parity.FMT[fmt], n_row, rows, ctypes.byref(w)), w.value) == (elems, width)
+
+
 def test_workspace_slot_bookkeeping(L):
     """Slot choice of the per-(device, stream, kind) scratch table of the K-split
     GEMMs: a known key finds its slot, a new key takes the first free slot, and

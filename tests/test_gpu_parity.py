@@ -553,6 +553,26 @@ def test_dequant_rows_at_the_edges_of_their_units(fmt, n_row, n_valid):
         assert np.array_equal(got.cpu().numpy().reshape(-1).view(np.uint32), ref.view(np.uint32))
 
 
+@pytest.mark.parametrize("fmt,n_row,rows", [("q4_k", 512, 16400), ("q4_k", 1280, 3300), ("q4_k", 5376, 800), ("q6_k", 512, 16400), ("q6_k", 768, 2800),
+                                            ("q6_k", 5376, 400), ("q8_0", 96, 9), ("q8_0", 1312, 9)])
+def test_dequant_rows_of_large_launches_and_uneven_blocks(fmt, n_row, rows):
+    """Launches large enough for sixteen elements a thread, and blocks of fewer threads than 256: rows of one block and of two with a last wave that is part
+    empty; zeros from an element on that is inside a run of four, rows behind the last token, ids outside the vocabulary, positions."""
+    voc, tokens, n_valid = 300, rows - 3, n_row - 5
+    width = ctypes.c_int()
+    assert ckq.lib().ckq_launch_dequant_form(P.FMT[fmt], n_row, rows, ctypes.byref(width)) == (4 if fmt == "q8_0" else 16)
+    assert width.value < 256
+    tab = T.random_blocks(fmt, voc * (n_row // T.ELEMS[fmt]), n_row)
+    ids = np.random.default_rng(n_row).integers(-2, voc + 2, size=tokens).astype(np.int32)
+    pos = T.normal(rows * n_row, 0.0, 0.1, seed=n_row)
+    for add_pos in (0, 1):
+        ref = np.full(rows * n_row, 9.0, np.float32)
+        T.oracle().orc_embedding_forward(T.FMT[fmt], T.ptr(ids), tokens, voc, T.ptr(tab), T.ptr(pos), T.ptr(ref), n_valid, n_row, rows, add_pos)
+        say("dequant rows, large launches", fmt, n_row, rows, add_pos)
+        got = P.dev_dequant_rows(fmt, P.to_device(tab), P.to_device(ids), voc, P.to_device(pos) if add_pos else None, n_valid, n_row, tokens, rows)
+        assert np.array_equal(got.cpu().numpy().reshape(-1).view(np.uint32), ref.view(np.uint32))
+
+
 # ---- prefill GEMM on the matrix cores (Q4_K, token counts above 16) -------------------------
 
 @pytest.mark.parametrize("M,N,K", [(17, 128, 256), (33, 200, 1024), (64, 96, 512), (100, 333, 2048),
