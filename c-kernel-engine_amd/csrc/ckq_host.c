@@ -66,6 +66,7 @@ static int          g_cache_on = 1;
 #define CKQ_PARALLEL_WHOLE_DEFAULT 0
 static int          g_parallel_whole = CKQ_PARALLEL_WHOLE_DEFAULT;
 static hipStream_t  g_stream = NULL;
+static int          g_device = -1;        /* the GPU of g_stream */
 static dev_buf      g_buf[BUF_COUNT];
 /* Pinned host twins of the staging buffers.  Small transfers (a decode step's
  * activation vector up, its outputs down) go through them: a copy between
@@ -171,6 +172,7 @@ static int init_locked(void)
         return fail((int)hipErrorInvalidDeviceFunction, "architecture check");
     }
     HIP_TRY(hipStreamCreateWithFlags(&g_stream, hipStreamNonBlocking));
+    g_device = dev;
     const char *c = getenv("CKQ_WEIGHT_CACHE");
     if (c && strcmp(c, "0") == 0) g_cache_on = 0;
     const char *mb = getenv("CKQ_WEIGHT_CACHE_MB");
@@ -234,8 +236,9 @@ enum { PTR_CACHE = 64 };
 static const void *g_host_ptr[PTR_CACHE];
 static void ptr_cache_clear(void) { memset(g_host_ptr, 0, sizeof g_host_ptr); }
 
-enum { PTR_HOST = 0, PTR_DEVICE, PTR_MANAGED };
-static int ptr_kind(const void *p)
+/* What a kernel may use as it is: ordinary memory of the library's GPU, and all other (managed, fine-grained or uncached memory, another GPU's). */
+typedef enum { PTR_HOST = 0, PTR_OWN, PTR_OTHER } ptr_kind_t;
+static ptr_kind_t ptr_kind(const void *p)
 {
     const size_t slot = ((uintptr_t)p >> 6) % PTR_CACHE;
     if (p && g_host_ptr[slot] == p) return PTR_HOST;
@@ -247,8 +250,8 @@ static int ptr_kind(const void *p)
         g_host_ptr[slot] = p;
         return PTR_HOST;
     }
-    if (at.type == hipMemoryTypeDevice) return PTR_DEVICE;
-    if (at.type == hipMemoryTypeManaged) return PTR_MANAGED;
+    if (at.type == hipMemoryTypeDevice) return at.device == g_device && at.allocationFlags == hipDeviceMallocDefault ? PTR_OWN : PTR_OTHER;
+    if (at.type == hipMemoryTypeManaged) return PTR_OTHER;
     if (at.type == hipMemoryTypeUnregistered) g_host_ptr[slot] = p;
     return PTR_HOST;
 }
@@ -289,12 +292,12 @@ static int stream_wait(void)
     return 0;
 }
 
-/* The same where the results are in the caller's own memory.  Device memory is read by the GPU and its copy engines, which see what a kernel has
- * written once it has ended; managed memory the CPU may read as well, which only the synchronisation call promises.  The word instead of
- * that call: fused MLP of 512 tokens, 896 x 4864 65.3 -> 62.9 us. */
-static int result_wait(int kind)
+/* The same where the results are in the caller's own memory.  Ordinary memory of this GPU is read by its kernels and copy engines, which see what a kernel has
+ * written once it has ended.  Other memory the CPU may read where it lies (managed, fine-grained), or another GPU through caches of its own: only
+ * the synchronisation call promises that they see it.  The word instead of that call: fused MLP of 512 tokens, 896 x 4864 65.3 -> 62.9 us. */
+static int result_wait(ptr_kind_t kind)
 {
-    if (kind == PTR_DEVICE) return stream_wait();
+    if (kind == PTR_OWN) return stream_wait();
     HIP_TRY(hipStreamSynchronize(g_stream));
     return 0;
 }
@@ -858,11 +861,11 @@ static void matmul_locked(int fmt, const void *A, const void *B, const float *bi
         if (weights_resolve(0, B, (size_t)nrows * weight_row_bytes(fmt, K), &dB)) break;
         if (stage_in(BUF_X, A, (size_t)ntok * act_row_bytes(fmt, K), &dA)) break;
         if (bias && stage_in(BUF_BIAS, bias, (size_t)nrows * sizeof(float), &dbias)) break;
-        const int c_on_dev = is_device_ptr(C);
+        const ptr_kind_t c_kind = ptr_kind(C);
         float *dC = C;
         long   ld = ldc;
         void  *ypin = NULL;      /* small results are written by the kernel straight into the pinned twin */
-        if (!c_on_dev) {
+        if (c_kind == PTR_HOST) {
             void *t;
             ld = row1 - row0; /* compact staging: only the computed rows */
             const size_t ybytes = (size_t)ntok * (size_t)ld * sizeof(float);
@@ -885,11 +888,11 @@ static void matmul_locked(int fmt, const void *A, const void *B, const float *bi
             if (stream_wait()) break;
             const size_t w = (size_t)(row1 - row0) * sizeof(float);
             for (int t = 0; t < ntok; ++t) memcpy(C + (size_t)t * ldc + row0, (const uint8_t *)ypin + (size_t)t * w, w);
-        } else if (!c_on_dev) {
+        } else if (c_kind == PTR_HOST) {
             if (stage_out_sync(BUF_Y, C + row0, (size_t)ldc * sizeof(float), (size_t)ld * sizeof(float),
                                (size_t)(row1 - row0) * sizeof(float), (size_t)ntok)) break;
         } else {
-            if (result_wait(c_on_dev)) break;
+            if (result_wait(c_kind)) break;
         }
         done = 1;
     } while (0);
@@ -937,22 +940,22 @@ static void host_quantize(int q8k, const float *x, void *y, int rows, int k)
         if (init_locked()) break;
         const void *dx;
         if (stage_in(BUF_X, x, in_bytes, &dx)) break;
-        const int y_on_dev = is_device_ptr(y);
+        const ptr_kind_t y_kind = ptr_kind(y);
         void *dy = y, *ypin = NULL;      /* Q8_K leaves its kernel in whole dwords: straight into the pinned twin if small */
-        if (!y_on_dev && q8k && out_bytes <= ARRIVE_MAX_BYTES) {
+        if (y_kind == PTR_HOST && q8k && out_bytes <= ARRIVE_MAX_BYTES) {
             if (pin_reserve(BUF_Y, round16(out_bytes), &ypin)) break;
             dy = g_pin[BUF_Y].dev;
             arrive_expect(ypin, out_bytes);
-        } else if (!y_on_dev && buf_reserve(BUF_Y, out_bytes, &dy)) break;
+        } else if (y_kind == PTR_HOST && buf_reserve(BUF_Y, out_bytes, &dy)) break;
         int rc = q8k ? ckq_launch_quantize_q8_k((const float *)dx, dy, rows, k, g_stream)
                      : ckq_launch_quantize_q8_0((const float *)dx, dy, rows, k, g_stream);
         if (rc) { fail(rc, "quantize launch"); break; }
         if (ypin) {
             if (arrive_collect(y, ypin, out_bytes)) break;
-        } else if (!y_on_dev) {
+        } else if (y_kind == PTR_HOST) {
             if (stage_out_sync(BUF_Y, y, out_bytes, out_bytes, out_bytes, 1)) break;
         } else {
-            if (result_wait(y_on_dev)) break;
+            if (result_wait(y_kind)) break;
         }
         done = 1;
     } while (0);
@@ -1121,16 +1124,16 @@ static void host_dequant_rows(int fmt, const void *table, size_t table_rows, con
         if (ids && tokens > 0 && stage_in(BUF_X, ids, (size_t)tokens * sizeof(int32_t), &dids)) break;
         if (pos && tokens > 0 && stage_in(BUF_BIAS, pos, (size_t)tokens * n_row * sizeof(float), &dpos)) break;
         const size_t out_bytes = (size_t)n_out_rows * n_row * sizeof(float);
-        const int on_dev = is_device_ptr(out);
+        const ptr_kind_t out_kind = ptr_kind(out);
         void *dout = out;
-        if (!on_dev && buf_reserve(BUF_Y, out_bytes, &dout)) break;
+        if (out_kind == PTR_HOST && buf_reserve(BUF_Y, out_bytes, &dout)) break;
         int rc = ckq_launch_dequant_rows(fmt, dT, ids ? (const int32_t *)dids : NULL, vocab, (const float *)dpos,
                                          (float *)dout, n_valid, n_row, tokens, n_out_rows, g_stream);
         if (rc) { fail(rc, "ckq_launch_dequant_rows"); break; }
-        if (!on_dev) {
+        if (out_kind == PTR_HOST) {
             if (stage_out_sync(BUF_Y, out, out_bytes, out_bytes, out_bytes, 1)) break;
         } else {
-            if (result_wait(on_dev)) break;
+            if (result_wait(out_kind)) break;
         }
         done = 1;
     } while (0);
@@ -1185,16 +1188,16 @@ void rmsnorm_q8_k_fused(const float *input, const float *gamma, void *vy, int to
         const void *dx, *dg;
         if (stage_in(BUF_X, input, in_bytes, &dx)) break;
         if (stage_in(BUF_BIAS, gamma, (size_t)d_model * 4, &dg)) break;
-        const int y_on_dev = is_device_ptr(vy);
+        const ptr_kind_t y_kind = ptr_kind(vy);
         void *dy = vy;
-        if (!y_on_dev && buf_reserve(BUF_Y, out_bytes, &dy)) break;
+        if (y_kind == PTR_HOST && buf_reserve(BUF_Y, out_bytes, &dy)) break;
         int rc = ckq_launch_rmsnorm_q8_k_fused((const float *)dx, (const float *)dg, dy, tokens, d_model,
                                                aligned_embed_dim, eps, g_stream);
         if (rc) { fail(rc, "rmsnorm_q8_k_fused launch"); break; }
-        if (!y_on_dev) {
+        if (y_kind == PTR_HOST) {
             if (stage_out_sync(BUF_Y, vy, out_bytes, out_bytes, out_bytes, 1)) break;
         } else {
-            if (result_wait(y_on_dev)) break;
+            if (result_wait(y_kind)) break;
         }
         done = 1;
     } while (0);
@@ -1254,19 +1257,19 @@ void fused_mlp_swiglu_prefill_w1w2_quant(const float *x, const void *W1, const f
         if (buf_reserve(BUF_Q, (size_t)seq_len * act_row_bytes(CKQ_FMT_Q8_0, E), &dq)) break;
         if (buf_reserve(BUF_GU, (size_t)seq_len * 2 * I * 4, &dgu)) break;
         if (buf_reserve(BUF_H, (size_t)seq_len * act_row_bytes(fmt2, I), &dh)) break;
-        const int out_on_dev = is_device_ptr(output);
+        const ptr_kind_t out_kind = ptr_kind(output);
         void *dout = output;
-        if (!out_on_dev && buf_reserve(BUF_Y, out_bytes, &dout)) break;
+        if (out_kind == PTR_HOST && buf_reserve(BUF_Y, out_bytes, &dout)) break;
         int rc = ckq_launch_quantize_gemv_q8_0(fmt1, (const float *)dx, dq, (float *)dgu, dW1, (const float *)dB1, 2 * I, E, seq_len, 2L * I, g_stream);
         if (rc) { fail(rc, "quantize and gate/up GEMM launch"); break; }
         rc = ckq_launch_swiglu_q8_k((const float *)dgu, (const float *)dgu + I, dh, seq_len, I, 2L * I, g_stream);
         if (rc) { fail(rc, "swiglu launch"); break; }
         rc = ckq_launch_gemv(fmt2, (float *)dout, dW2, dh, (const float *)dB2, E, I, seq_len, (long)E, 0, E, NULL, g_stream);
         if (rc) { fail(rc, "down GEMM launch"); break; }
-        if (!out_on_dev) {
+        if (out_kind == PTR_HOST) {
             if (stage_out_sync(BUF_Y, output, out_bytes, out_bytes, out_bytes, 1)) break;
         } else {
-            if (result_wait(out_on_dev)) break;
+            if (result_wait(out_kind)) break;
         }
         done = 1;
     } while (0);

@@ -825,6 +825,47 @@ def test_results_in_device_memory_are_there_when_a_call_returns():
             assert torch.equal(seen.cpu(), want) and torch.equal(y.cpu(), want), (seq, E, I)
 
 
+def test_results_of_every_call_are_there_where_the_caller_reads_them():
+    """The five kinds of synchronous call with a result of their own, in ordinary device memory (read at once on another stream, and by a copy) and in
+    managed memory (read at once by the CPU): the same bytes as through host memory."""
+    import torch
+    with open("/proc/self/maps") as f:
+        hip = ctypes.CDLL(next(l.split()[-1] for l in f if "libamdhip64" in l))
+    L, other = ckq.lib(), torch.cuda.Stream()
+    M, K, D, seq, E, I = 96, 1024, 4096, 40, 256, 512
+    h = {"W": T.random_blocks("q4_k", M * K // 256, 31), "x": T.oracle_quantize(T.normal(K, 0.0, 1.0, 32), "q8_k"), "f": T.normal(4 * D, 0.0, 1.0, 33),
+         "g": T.normal(D, 1.0, 0.1, 34), "xm": T.normal(seq * E, 0.0, 1.0, 35), "W1": T.synth_weights("q8_0", 2 * I, E, seed=36), "W2": T.synth_weights("q4_k", E, I, seed=37),
+         "s": np.zeros(16, np.uint8)}
+    calls = [("matmul", 4 * M, lambda p, y: L.gemv_q4_k_q8_k(y, p("W"), p("x"), M, K)),
+             ("quantize", 4 * D // 256 * 292, lambda p, y: L.quantize_batch_q8_k(p("f"), y, 4, D)),
+             ("dequantize", 4 * M * K, lambda p, y: L.dequant_q4_k_row(p("W"), y, M * K)),
+             ("rmsnorm", 4 * D // 256 * 292, lambda p, y: L.rmsnorm_q8_k_fused(p("f"), p("g"), y, 4, D, D, 1e-5)),
+             ("fused mlp", 4 * seq * E, lambda p, y: L.fused_mlp_swiglu_prefill_w1w2_quant(p("xm"), p("W1"), None, P.CK_DT["q8_0"], p("W2"), None, P.CK_DT["q4_k"], y,
+                                                                                           seq, E, E, I, I, p("s")))]
+    d = {k: P.to_device(v) for k, v in h.items()}
+    managed = ctypes.c_void_p()
+    assert hip.hipMallocManaged(ctypes.byref(managed), ctypes.c_size_t(4 * M * K), 1) == 0
+    try:
+        for name, n, call in calls:
+            say("results where the caller reads them", name)
+            want = np.zeros(n, np.uint8)
+            call(lambda k: T.ptr(h[k]), T.ptr(want))
+            for _ in range(4):
+                y = torch.full((n,), 0x55, dtype=torch.uint8, device="cuda")
+                torch.cuda.synchronize()
+                call(lambda k: P._dp(d[k]), P._dp(y))
+                with torch.cuda.stream(other):
+                    seen = y.clone()
+                other.synchronize()
+                assert np.array_equal(seen.cpu().numpy(), want) and np.array_equal(y.cpu().numpy(), want), name
+                ctypes.memset(managed, 0x55, n)
+                call(lambda k: P._dp(d[k]), managed)
+                assert ctypes.string_at(managed, n) == want.tobytes(), name
+    finally:
+        torch.cuda.synchronize()
+        assert hip.hipFree(managed) == 0
+
+
 @pytest.mark.parametrize("fmt,seq,E,I,bias", [("q4_k", 130, 896, 4864, True), ("q6_k", 33, 256, 1024, False),
                                               ("q4_k", 1, 64, 256, True), ("q6_k", 512, 128, 512, True)])
 def test_fused_mlp_vs_oracle(fmt, seq, E, I, bias):
