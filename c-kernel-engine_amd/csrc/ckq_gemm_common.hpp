@@ -290,7 +290,7 @@ template <class Kernel>
 static int gemm_launch_ksplit(Kernel k2, Kernel k3, Kernel k4, GemmArgs &g, int k, hipStream_t s)
 {
     g.k_per = (g.nb + k - 1) / k;
-    /* what has no room for the partial tiles of a split among blocks is refused as there */
+    /* refused as a split among blocks is where its partial tiles have no room, though none are written here: what a size is answered does not hang on the kernel */
     if (g.ext_part && (size_t)k * (size_t)g.M * (size_t)g.N * sizeof(float) > g.ext_part_bytes) return CKQ_ESCRATCH;
     g.nnt = (g.N + 31) / 32;
     hipLaunchKernelGGL(k == 2 ? k2 : k == 3 ? k3 : k4, dim3((unsigned)gemm_blocks(g.ntt, g.nnt)), dim3((unsigned)(64 * k)), 0, s, g);

@@ -296,8 +296,10 @@ static bool weights_dword_aligned(const GemvArgs &a, const GemvGroup &grp)
  *              (per: 256-blocks of a piece, out: millions of outputs; Q5_K 3.7, 1.83, 0.12, 2.8, Q6_K 3.75, 1.73, 0.18, 3.7), and rows16 there 3.4 + 0.11 nb +
  *              0.6 n16 (2.8, 0.154, 0.85; 2.8, 0.26, 0.22), groups in pairs 3.7 + (0.135 + 0.135 blocks on a CU) nb (3.4, 0.09, 0.32; 4.6, -0.024,
  *              0.344).  By the estimates above the choice cost 5.6, 7.1 and 4.5 % more than the faster kernel, single sizes 48; by these 0.4 (us: Q4_K 172 tokens x 2560 x 3385
- *              18.8 -> 13.5, Q5_K 146 x 3840 x 2084 18.7 -> 13.7, Q6_K 329 x 3328 x 1257 20.2 -> 13.7).  Not for calls that bring their scratch: which of
- *              them are refused for want of it stays as it was (`own_scratch`), and no call on the K split is refused that a 16-row kernel took.
+ *              18.8 -> 13.5, Q5_K 146 x 3840 x 2084 18.7 -> 13.7, Q6_K 329 x 3328 x 1257 20.2 -> 13.7).  Not for calls that bring their scratch
+ *              (`own_scratch`): a 16-row kernel needs none, and what goes to a split of K is refused where the partial tiles would be more than that scratch,
+ *              so these calls keep the estimates above, by which none is refused that a 16-row kernel took before there were splits among waves (the
+ *              groups in pairs take many of Q5_K and Q6_K that were).
  *   streaming  above eight tokens the larger of 2.9 and 2.2 + 0.0075 lanes + (23.5, 23.5, 29) million lanes of all rows and passes,
  *              a row's 64-element positions being dealt to 8, 16, 32 or 64 lanes or to 2 to 4 passes of 64 (stream_lanes): small
  *              matrices stream at up to some 60 tokens (Q5_K 290 x 1792 at 25: 3.0, here 4.6; Q6_K 435 x 1536 at 13 3.0, here 4.8);
@@ -321,7 +323,7 @@ extern "C" void ckq_launch_set_rows16(int fmt, int on)
     else g_rows16_forced.fetch_and(~(1 << fmt));
 }
 /* gemm_rows16_keep_time as it was fitted before, for calls that bring their scratch: rows of eight blocks are the only ones that this kernel and a split of K
- * both take, and which calls are refused for want of scratch is not to follow an estimate of time. */
+ * both take, and no call is to be refused for want of scratch because an estimate of time was fitted again. */
 static float keep_time_own_scratch(int f, size_t rows, int ntok)
 {
     const long tiles = (long)((rows + 15) / 16), groups = (ntok + 15) / 16;

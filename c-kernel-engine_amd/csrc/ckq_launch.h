@@ -18,7 +18,7 @@ extern "C" {
 #define CKQ_EINVAL  (-1)  /* NULL pointer / non-positive dimension */
 #define CKQ_ESHAPE  (-2)  /* K not a multiple of the block size */
 #define CKQ_EFORMAT (-3)  /* unknown format tag */
-#define CKQ_ESCRATCH (-4) /* the call needs more scratch than the entry point that allocates nothing holds */
+#define CKQ_ESCRATCH (-4) /* the call is counted with more scratch than the entry point that allocates nothing holds */
 #define CKQ_ENOGROUP (-7) /* internal: a grouped GEMM launch was declined; the caller launches the matrices one by one */
 #define CKQ_ENODUMP (-6)  /* the integer dumps are compiled into libckernel_quant_hip_dump.so only */
 /* 1 in the test library (same sources, same templates, plus the DUMP instantiations that also
@@ -131,8 +131,8 @@ int ckq_launch_dequant_form(int fmt, int n_row, int n_out_rows, int *width);
 
 /* ckq_launch_gemv for callers that must not allocate: a K-split matrix-core
  * GEMM takes its partial tiles from a static device array of
- * CKQ_NOALLOC_SCRATCH_BYTES instead of the grow-only workspace; a split that
- * needs more returns CKQ_ESCRATCH.  Formats Q4_K, Q5_K, Q6_K, Q8_0.
+ * CKQ_NOALLOC_SCRATCH_BYTES instead of the grow-only workspace; a split whose
+ * partial tiles would take more returns CKQ_ESCRATCH, whether its kernel writes them or not.  Formats Q4_K, Q5_K, Q6_K, Q8_0.
  * ckq_launch_noalloc_setup() resolves the array's address for the current
  * device (once per device; also done by the first call on a device). */
 #define CKQ_NOALLOC_SCRATCH_BYTES ((size_t)4 << 20)

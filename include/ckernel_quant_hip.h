@@ -230,15 +230,17 @@ int ckq_gemm_nt_dev(int fmt, const void *A_q8, const void *B, const float *bias,
 
 /* ckq_gemm_nt_dev for callers that cannot allocate device memory.  It has no
  * counterpart in the reference; it is for code under HIP graph capture, tight
- * serving loops and harnesses that forbid hipMalloc.  Same arithmetic, same
- * kernel choice and the same bits as ckq_gemm_nt_dev (formats CKQ_FMT_Q4_K,
- * _Q5_K, _Q6_K, _Q8_0); the partial tiles of a K-split matrix-core GEMM live in
- * a static device array of 4 MiB (one copy per GPU, held until the process
- * ends) instead of the library's grow-only workspace.  A call whose split
- * needs more (splits x M x N x 4 bytes; up to 16 splits are taken when the
- * tile grid is smaller than the chip) returns CKQ_ESCRATCH (-4) and enqueues
- * nothing: pass fewer tokens per call, or use ckq_gemm_nt_dev; no call allocates,
- * frees or synchronizes.  Every call on a GPU shares that GPU's array: calls
+ * serving loops and harnesses that forbid hipMalloc.  Same arithmetic and the
+ * same bits as ckq_gemm_nt_dev (formats CKQ_FMT_Q4_K, _Q5_K, _Q6_K, _Q8_0),
+ * though not the same kernel at every size; the partial tiles of a K-split
+ * matrix-core GEMM live in a static device array of 4 MiB (one copy per GPU,
+ * held until the process ends) instead of the library's grow-only workspace.
+ * A call that splits K and whose partial tiles would take more (splits x M x N
+ * x 4 bytes; up to 16 splits are taken when the tile grid is smaller than the
+ * chip) returns CKQ_ESCRATCH (-4) and enqueues nothing, also where the pieces
+ * of the split meet inside a block and nothing would be written there: pass
+ * fewer tokens per call, or use ckq_gemm_nt_dev; no call allocates, frees or
+ * synchronizes.  Every call on a GPU shares that GPU's array: calls
  * that overlap on one GPU (two streams, two threads) race.  The array's
  * address is resolved once per device, by ckq_init() or by the first call on
  * that device; resolving it may load the library's code object, so call
