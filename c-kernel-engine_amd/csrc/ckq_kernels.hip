@@ -294,8 +294,9 @@ static bool weights_dword_aligned(const GemvArgs &a, const GemvGroup &grp)
  *              faster kernel and these cost 1.5 and 0.6; Q4_K's own fit would cost 5.2 instead of 1.0)
  *   K split    where the pieces of K are waves of a block (gemm_ksplit_pieces), fitted to 450 launches of 17 to 700 tokens, 5 to 11 % rms: 4.1 + 1.44 per + 0.16 mb + 3.3 out
  *              (per: 256-blocks of a piece, out: millions of outputs; Q5_K 3.7, 1.83, 0.12, 2.8, Q6_K 3.75, 1.73, 0.18, 3.7), and rows16 there 3.4 + 0.11 nb +
- *              0.6 n16 (2.8, 0.154, 0.85; 2.8, 0.26, 0.22), groups in pairs 3.7 + (0.135 + 0.135 blocks on a CU) nb (3.4, 0.09, 0.32; 4.6, -0.024,
- *              0.344).  By the estimates above the choice cost 5.6, 7.1 and 4.5 % more than the faster kernel, single sizes 48; by these 0.4 (us: Q4_K 172 tokens x 2560 x 3385
+ *              0.6 n16 (2.8, 0.154, 0.85; 2.8, 0.26, 0.22 and with more than one block a CU 1.7, 0.43, 0.70: 7 % rms over 22 launches, where the former made
+ *              half of 46 us, and the choice cost up to 113 % instead of none: 111 tokens x 6912 x 3759 46.4 -> 22.8, 29 x 6912 x 7371 30.0 -> 23.4),
+ *              groups in pairs 3.7 + (0.135 + 0.135 blocks on a CU) nb (3.4, 0.09, 0.32; 4.6, -0.024, 0.344).  By the estimates above the choice cost 5.6, 7.1 and 4.5 % more than the faster kernel, single sizes 48; by these 0.4 (us: Q4_K 172 tokens x 2560 x 3385
  *              18.8 -> 13.5, Q5_K 146 x 3840 x 2084 18.7 -> 13.7, Q6_K 329 x 3328 x 1257 20.2 -> 13.7).  Not for calls that bring their scratch
  *              (`own_scratch`): a 16-row kernel needs none, and what goes to a split of K is refused where the partial tiles would be more than that scratch,
  *              so these calls keep the estimates above, by which none is refused that a 16-row kernel took before there were splits among waves (the
@@ -354,13 +355,14 @@ static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles, int l
     if (const int pieces = tiles && launches == 1 && !own_scratch && rows < 1 << 24
                                ? gemm_ksplit_pieces(ntok, (long)rows, K / 256, f == 0 ? GEMM_KSPLIT_Q4K : f == 1 ? GEMM_KSPLIT_Q5K : GEMM_KSPLIT_Q6K) : 0) {
         static const float split[3][4] = {{4.1f, 1.44f, 0.16f, 3.3f}, {3.7f, 1.83f, 0.12f, 2.8f}, {3.75f, 1.73f, 0.18f, 3.7f}},
-                           single[3][3] = {{3.4f, 0.11f, 0.6f}, {2.8f, 0.154f, 0.85f}, {2.8f, 0.26f, 0.22f}},
+                           single[4][3] = {{3.4f, 0.11f, 0.6f}, {2.8f, 0.154f, 0.85f}, {2.8f, 0.26f, 0.22f}, {1.7f, 0.43f, 0.7f}},
                            pair[3][3] = {{3.7f, 0.135f, 0.135f}, {3.4f, 0.09f, 0.32f}, {4.6f, -0.024f, 0.344f}};
         const float r16 = (float)((rows + 15) / 16), groups = (float)((ntok + 15) / 16), per = (float)((K / 256 + pieces - 1) / pieces);
         const float t = split[f][0] + split[f][1] * per + split[f][2] * mb + split[f][3] * 1e-6f * (float)ntok * (float)rows;
         if (t_keep > 0.0f) return t_keep < t;
         if (t_pair > 0.0f) return pair[f][0] + (pair[f][1] + pair[f][2] * fmaxf(r16 * (float)((ntok + 31) / 32) / 256.0f, 1.0f)) * nb < t;
-        return single[f][0] + single[f][1] * nb + single[f][2] * 1e-3f * nb * r16 * groups < t;
+        const float *one = single[f == 2 && r16 * groups > 256.0f ? 3 : f];
+        return one[0] + one[1] * nb + one[2] * 1e-3f * nb * r16 * groups < t;
     }
     if (tiles) t_else = f == 0 || t_pair <= 0.0f ? 11.0f + (0.2f + 0.0015f * (float)ntok) * mb : f == 1 ? 13.3f + (0.164f + 0.0048f * (float)ntok) * mb : 13.8f + (0.083f + 0.0044f * (float)ntok) * mb;
     else if (ntok <= 8) t_else = fmaxf(3.5f + 0.07f * nb, 3.05f + 0.11f * nb + 1.25f * per_pass[f] * mb);
