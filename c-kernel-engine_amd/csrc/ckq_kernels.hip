@@ -301,6 +301,12 @@ static bool weights_dword_aligned(const GemvArgs &a, const GemvGroup &grp)
  *              (`own_scratch`): a 16-row kernel needs none, and what goes to a split of K is refused where the partial tiles would be more than that scratch,
  *              so these calls keep the estimates above, by which none is refused that a 16-row kernel took before there were splits among waves (the
  *              groups in pairs take many of Q5_K and Q6_K that were).
+ *   short rows, up to 256 tokens of two groups and more (t_keep), against the tiles: 6.2 + (0.26 + 0.41 rounds + 0.62 CU) nb + 0.88 out (rounds: of 256 tiles of 64 tokens x 128 rows, CU:
+ *              tiles a CU, one at least, since some kernels have two blocks on a CU; Q5_K 6.6, 0.32, 0.70, 0.78, 1.04, Q6_K 7.3, 0, 1.11, 0.45, 0.77; 4 to 5 % rms over 1146 launches of
+ *              17 to 256 tokens, 200 to 32000 rows, where the line above has 20 to 28) and gemm_rows16_keep_time once more, with the outputs and rows of three blocks, which leave
+ *              a wave's place idle: 0.66 + 0.82 t + 0.97 out + 0.09 t where nb = 3 (0.14, 0.98, 0.47, 0.04; 0.21, 0.985, 0.43, 0.08).  The choice costs 0.2 to 0.3 % more
+ *              than the faster kernel, by the line above 0.8 to 1.5, at most 53 (us: Q4_K 120 tokens x 256 x 27284 13.4 -> 10.1, Q5_K 117 x 256 x 26823 14.5 -> 11.2, 185 x 1792 x
+ *              3199 19.5 -> 15.0).
  *   streaming  above eight tokens the larger of 2.9 and 2.2 + 0.0075 lanes + (23.5, 23.5, 29) million lanes of all rows and passes,
  *              a row's 64-element positions being dealt to 8, 16, 32 or 64 lanes or to 2 to 4 passes of 64 (stream_lanes): small
  *              matrices stream at up to some 60 tokens (Q5_K 290 x 1792 at 25: 3.0, here 4.6; Q6_K 435 x 1536 at 13 3.0, here 4.8);
@@ -363,6 +369,14 @@ static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles, int l
         if (t_pair > 0.0f) return pair[f][0] + (pair[f][1] + pair[f][2] * fmaxf(r16 * (float)((ntok + 31) / 32) / 256.0f, 1.0f)) * nb < t;
         const float *one = single[f == 2 && r16 * groups > 256.0f ? 3 : f];
         return one[0] + one[1] * nb + one[2] * 1e-3f * nb * r16 * groups < t;
+    }
+    const float out = 1e-6f * (float)ntok * (float)rows;
+    if (tiles && t_keep > 0.0f && !(own_scratch && K == 2048)) {
+        static const float tile[3][5] = {{6.18f, 0.26f, 0.41f, 0.62f, 0.88f}, {6.57f, 0.32f, 0.70f, 0.78f, 1.04f}, {7.28f, -0.02f, 1.11f, 0.45f, 0.77f}},
+                           keep[3][4] = {{0.66f, 0.82f, 0.97f, 0.09f}, {0.14f, 0.98f, 0.47f, 0.04f}, {0.21f, 0.985f, 0.43f, 0.08f}};
+        const float on_cu = (float)((rows + 127) / 128) * (float)((ntok + 63) / 64) / 256.0f;
+        return keep[f][0] + (keep[f][1] + (nb == 3.0f ? keep[f][3] : 0.0f)) * t_keep + keep[f][2] * out <
+               tile[f][0] + (tile[f][1] + tile[f][2] * ceilf(on_cu) + tile[f][3] * fmaxf(on_cu, 1.0f)) * nb + tile[f][4] * out;
     }
     if (tiles) t_else = f == 0 || t_pair <= 0.0f ? 11.0f + (0.2f + 0.0015f * (float)ntok) * mb : f == 1 ? 13.3f + (0.164f + 0.0048f * (float)ntok) * mb : 13.8f + (0.083f + 0.0044f * (float)ntok) * mb;
     else if (ntok <= 8) t_else = fmaxf(3.5f + 0.07f * nb, 3.05f + 0.11f * nb + 1.25f * per_pass[f] * mb);
