@@ -310,7 +310,9 @@ static bool weights_dword_aligned(const GemvArgs &a, const GemvGroup &grp)
  *   streaming  above eight tokens the larger of 2.9 and 2.2 + 0.0075 lanes + (23.5, 23.5, 29) million lanes of all rows and passes,
  *              a row's 64-element positions being dealt to 8, 16, 32 or 64 lanes or to 2 to 4 passes of 64 (stream_lanes): small
  *              matrices stream at up to some 60 tokens (Q5_K 290 x 1792 at 25: 3.0, here 4.6; Q6_K 435 x 1536 at 13 3.0, here 4.8);
- *              several matrices take a launch each; 5 to 8 tokens the larger of 3.5 + 0.07 nb and 3.05 + 0.11 nb + (0.24, 0.245, 0.29) mb for 10 tokens
+ *              several matrices take a launch each; against short rows' t_keep 2.4 + 14.9 w + 2.7 sqrt w (w: those lanes; Q5_K 2.2, 10.4, 6.0, Q6_K 2.15, 9.2, 8.65; 5.5 to 11 % rms
+ *              over 900 launches of 17 to 120 tokens) and 1.17 t - 0.8 (1.32 t - 1.6; 1.4 t - 1.95): costs 0.1 to 0.25 % more than the faster kernel instead of 0.6 to 1.9, at most
+ *              27 instead of 60 (us: Q6_K 47 tokens x 2048 x 368 7.0 -> 4.4, Q5_K 64 x 256 x 1141 4.9 -> 3.9); 5 to 8 tokens the larger of 3.5 + 0.07 nb and 3.05 + 0.11 nb + (0.24, 0.245, 0.29) mb for 10 tokens
  * Three and four tokens, one pass of half the width, only move for long rows of large Q6_K matrices whose positions leave a
  * tenth of those lanes idle (4096 x 11008 at 4: 14.2 -> 12.3, at 4 8192 x 4608 13.1 -> 11.4; but 4096 x 8192, no lane idle, 9.6 against
  * 9.9, and Q5_K 4096 x 8192 7.6 against 9.5); two never do.  The forced policies keep their kernels: 1 the tile kernels, 2 the
@@ -381,8 +383,12 @@ static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles, int l
     if (tiles) t_else = f == 0 || t_pair <= 0.0f ? 11.0f + (0.2f + 0.0015f * (float)ntok) * mb : f == 1 ? 13.3f + (0.164f + 0.0048f * (float)ntok) * mb : 13.8f + (0.083f + 0.0044f * (float)ntok) * mb;
     else if (ntok <= 8) t_else = fmaxf(3.5f + 0.07f * nb, 3.05f + 0.11f * nb + 1.25f * per_pass[f] * mb);
     else {
-        const float t_launch = 2.2f + 0.0075f * (float)lanes;
-        t_else = fmaxf(2.9f, t_launch + per_lane[f] * 1e-6f * (float)rows * (float)lanes * (float)((ntok + 7) / 8)) + (float)(launches - 1) * t_launch;
+        const float t_launch = 2.2f + 0.0075f * (float)lanes, w = 1e-6f * (float)rows * (float)lanes * (float)((ntok + 7) / 8);
+        if (t_keep > 0.0f) {
+            static const float stream[3][3] = {{2.39f, 14.9f, 2.69f}, {2.2f, 10.4f, 6.0f}, {2.15f, 9.2f, 8.65f}}, keep[3][2] = {{-0.78f, 1.17f}, {-1.56f, 1.32f}, {-1.95f, 1.4f}};
+            return keep[f][0] + keep[f][1] * t_keep < stream[f][0] + stream[f][1] * w + stream[f][2] * sqrtf(w) + (float)(launches - 1) * t_launch;
+        }
+        t_else = fmaxf(2.9f, t_launch + per_lane[f] * w) + (float)(launches - 1) * t_launch;
     }
     return t_rows < t_else;
 }

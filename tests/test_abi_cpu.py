@@ -213,7 +213,9 @@ def test_forced_variants_keep_their_kernels(L, fmt, variants):
     ("q6_k", 4096, 4096, 13, ROWS16_TILES), ("q5_k", 4864, 1024, 93, ROWS16_STREAM), ("q4_k", 11008, 4096, 512, TILES),
     ("q6_k", 3759, 6912, 111, TILES), ("q6_k", 7371, 6912, 29, TILES), ("q6_k", 292, 6400, 1138, TILES), ("q6_k", 7534, 2560, 10, ROWS16_TILES),
     ("q4_k", 27284, 256, 120, TILES), ("q4_k", 10244, 768, 110, TILES), ("q4_k", 17582, 256, 176, TILES), ("q5_k", 26823, 256, 117, TILES), ("q5_k", 3199, 1792, 185, ROWS16_TILES),
-    ("q4_k", 6552, 1024, 64, ROWS16_TILES), ("q5_k", 5029, 1792, 104, ROWS16_TILES), ("q6_k", 28565, 1024, 62, TILES), ("q6_k", 5000, 2048, 64, ROWS16_TILES)])
+    ("q4_k", 6552, 1024, 64, ROWS16_TILES), ("q5_k", 5029, 1792, 104, ROWS16_TILES), ("q6_k", 28565, 1024, 62, TILES), ("q6_k", 5000, 2048, 64, ROWS16_TILES),
+    ("q5_k", 1141, 256, 64, ROWS16_STREAM), ("q5_k", 948, 256, 80, ROWS16_STREAM), ("q5_k", 3258, 256, 24, ROWS16_STREAM), ("q6_k", 368, 2048, 47, ROWS16_STREAM),
+    ("q6_k", 454, 1792, 34, ROWS16_STREAM), ("q6_k", 1458, 512, 44, ROWS16_STREAM), ("q4_k", 1284, 512, 36, ROWS16_STREAM), ("q4_k", 438, 1024, 36, STREAM), ("q5_k", 177, 1024, 20, STREAM)])
 def test_16_row_tiles_where_they_are_the_faster_ones(L, fmt, n, k, tokens, want):
     """Shapes at which the kernels were timed against each other; the faster one is taken."""
     assert route(L, fmt, n, k, tokens) == want
