@@ -1085,8 +1085,9 @@ gemm_rows16_keep_kernel(const uint8_t *W, const uint8_t *X, int N, int M, int pa
 /* Waves per block: with two tiles per CU and more, blocks of four waves overlap each other's beginnings and ends
  * (32000 x 4096, 13 tokens: 27 us, with eight 41); with fewer, a tile's blocks spread over more waves.  A tile alone on its CU takes twelve
  * for rows of more than twelve 256-blocks: 44 launches of 64 to 256 tiles 1.02 on average, up to 1.11 (us, eight -> twelve: Q4_K 4096 x 4096 at 13
- * tokens 7.08 -> 6.81, Q5_K 3568 x 5888 10.2 -> 9.2, Q6_K 2048 x 5632 10.5 -> 9.3; sixteen 1.017; up to twelve blocks 0.98); but Q6_K rows of more than 32, whose
- * blocks come in more bytes, 0.97 (704 x 10496 at 15 14.6 -> 15.2). */
+ * tokens 7.08 -> 6.81, Q5_K 3568 x 5888 10.2 -> 9.2, Q6_K 2048 x 5632 10.5 -> 9.3; sixteen 1.017; up to twelve blocks 0.98); but Q6_K rows of more than 32 in the
+ * tile kernels' order, whose blocks come in more bytes, 0.986 over 100 launches (2048 x 8448 at 9 11.9 -> 12.6).  In the streaming kernel's order `nb` is
+ * the sums that are dealt, sixteen at most, and twelve waves it is for Q6_K as well: 1.05 over 118 launches of 5 and 8 tokens, rows of 13 to 43 blocks (Q6_K of 33 1.06, of 43 1.01). */
 int rows16_waves(int fmt, int tiles, int nb)
 {
     int waves = tiles >= 512 ? 4 : tiles > 256 ? 8 : tiles > 64 ? (nb > 12 && (fmt != CKQ_FMT_Q6_K || nb <= 32) ? 12 : 8) : 16;

@@ -64,7 +64,7 @@ __device__ __forceinline__ float4 rms_unstage(const float *xs, int D, int b, int
 }
 
 /* Thread j < 8 of the block walks chain j and leaves its sum behind the row.  The chain is serial, one multiply-add
- * after another; the 32 values of the next 256-block are read while those of this one are added. */
+ * after another, and waits for LDS once a 256-block: the compiler moves the reads of the next 32 values to where they are used. */
 __device__ __forceinline__ void rms_chain(float *xs, int D, int j)
 {
     const float4 *x = reinterpret_cast<const float4 *>(xs + j * rms_pitch(D));
