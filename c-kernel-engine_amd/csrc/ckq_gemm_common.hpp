@@ -39,7 +39,9 @@ struct GemmArgs {
     /* grouped launch: ngroup > 1 matrices, never split along K; B, bias, C, N, ldc, nnt above are those of grp[0] */
     int  ngroup;
     GemmProblem grp[GEMM_GROUP_MAX];
-    /* split K: blockIdx.y = s handles K-steps [s * k_per, min(k_steps, (s + 1) * k_per)) and
+    /* what is dealt to the XCDs as one (gemm_work): the tiles of all matrices, times the splits; 0: every matrix by itself, from its id0 on */
+    int    units;
+    /* split K: piece s handles K-steps [s * k_per, min(k_steps, (s + 1) * k_per)) and
      * writes its partial tile, without bias, to part + s * M * N (row pitch N) */
     int    splits, k_per;
     float *part;
@@ -84,25 +86,11 @@ struct GemmOpts {
     size_t   scratch_bytes;
 };
 
-/* What one block of a GEMM launch does: which tile id, which K-steps, where it
- * writes and whether it adds the bias. */
-struct GemmOut { float *C; long ldc; const float *bias; };
-struct GemmWork { int id, k0, k1; GemmOut out; const uint8_t *B; int N, nnt, tt0, ntt; };
-__device__ __forceinline__ GemmWork gemm_work(const GemmArgs &a, int k_steps)
+/* Of `total` things the one that block `id` takes, -1: none: eight equal runs, one for each XCD (blocks go round the XCDs in turn). */
+__host__ __device__ __forceinline__ int gemm_deal(int id, int total)
 {
-    const int id = blockIdx.x;
-    if (a.ngroup > 1) {
-        /* uniform selects, no indexing: the argument block stays in scalar registers */
-        GemmProblem g = a.grp[0];
-        if (id >= a.grp[1].id0) g = a.grp[1];
-        if (a.ngroup > 2 && id >= a.grp[2].id0) g = a.grp[2];
-        if (a.ngroup > 3 && id >= a.grp[3].id0) g = a.grp[3];
-        return {id - g.id0, 0, k_steps, {g.C, g.ldc, g.bias}, g.B, g.N, g.nnt, g.tt0, g.ntt};
-    }
-    if (a.splits <= 1) return {id, 0, k_steps, {a.C, a.ldc, a.bias}, a.B, a.N, a.nnt, 0, a.ntt};
-    const int k0 = (int)blockIdx.y * a.k_per;
-    return {id, k0, min(k_steps, k0 + a.k_per),
-            {a.part + (size_t)blockIdx.y * (size_t)a.M * (size_t)a.N, (long)a.N, nullptr}, a.B, a.N, a.nnt, 0, a.ntt};
+    const int xcd = id & 7, seq = id >> 3;
+    return seq < (total >> 3) + (xcd < (total & 7) ? 1 : 0) ? xcd * (total >> 3) + (xcd < (total & 7) ? xcd : total & 7) + seq : -1;
 }
 
 /* The tiles of a launch, ntt token tiles of nnt tiles of weight rows, token tiles fastest so that neighbours share weights, are dealt
@@ -112,12 +100,47 @@ __device__ __forceinline__ GemmWork gemm_work(const GemmArgs &a, int k_steps)
  * 60 random sizes 0.5 to 5 % on average, the same bits).  gemm_blocks: block ids to launch; false: no tile. */
 __host__ __device__ __forceinline__ bool gemm_tile(int id, int ntt, int nnt, int &nt, int &tt)
 {
-    const int total = ntt * nnt, xcd = id & 7, seq = id >> 3, t = xcd * (total >> 3) + (xcd < (total & 7) ? xcd : total & 7) + seq;
+    const int t = gemm_deal(id, ntt * nnt);
     nt = t / ntt;
     tt = t - nt * ntt;
-    return seq < (total >> 3) + (xcd < (total & 7) ? 1 : 0);
+    return t >= 0;
 }
 __host__ __device__ __forceinline__ constexpr int gemm_blocks(int ntt, int nnt) { return (ntt * nnt + 7) & ~7; }
+
+/* What one block of a GEMM launch does: which tile (weight-row tile nt, token tile tt; -1: none), which K-steps, where it
+ * writes and whether it adds the bias. */
+struct GemmOut { float *C; long ldc; const float *bias; };
+struct GemmWork { int tile, k0, k1; GemmOut out; const uint8_t *B; int N, nnt, tt0, ntt; };
+/* A launch of pieces of K is as wide as the chip (gemm_choose_splits), and takes as long as its fullest XCD: 84 tiles in three pieces, 252 blocks, were 33 for
+ * the 32 CUs of four XCDs, and so two rounds, as long as each piece's tiles were dealt by themselves (three matrices of 84 tiles were 33 where 32 do).  All pieces of all tiles
+ * are dealt as one, piece by piece, so that an XCD has one or two pieces of K of many tiles, which share activations as well as weights.  us, tokens x
+ * rows x K: Q6_K 384 x 1792 x 6400 43.3 -> 30.5, Q5_K 150 x 3584 x 9984 60.7 -> 36.2, Q4_K 379 x 768 x 7168 25.8 -> 21.5, Q8_0 321 x 1792 x 4864 32.3 -> 25.9; 48
+ * sizes of that kind 1.29 on average (1.02 to 1.68), 60 others 1.00.  The sums and their order are the same. */
+__device__ __forceinline__ GemmWork gemm_work(const GemmArgs &a, int k_steps)
+{
+    const int id = blockIdx.x;
+    int u = a.units ? gemm_deal(id, a.units) : id;
+    if (a.ngroup > 1) {
+        /* uniform selects, no indexing: the argument block stays in scalar registers */
+        GemmProblem g = a.grp[0];
+        if (u >= a.grp[1].id0) g = a.grp[1];
+        if (a.ngroup > 2 && u >= a.grp[2].id0) g = a.grp[2];
+        if (a.ngroup > 3 && u >= a.grp[3].id0) g = a.grp[3];
+        u = a.units ? (u < 0 ? -1 : u - g.id0) : gemm_deal(id - g.id0, g.ntt * g.nnt);
+        return {u, 0, k_steps, {g.C, g.ldc, g.bias}, g.B, g.N, g.nnt, g.tt0, g.ntt};
+    }
+    if (a.splits <= 1) return {u, 0, k_steps, {a.C, a.ldc, a.bias}, a.B, a.N, a.nnt, 0, a.ntt};
+    const int tiles = a.ntt * a.nnt, sp = u < 0 ? 0 : u / tiles, k0 = sp * a.k_per;
+    return {u - sp * tiles, k0, min(k_steps, k0 + a.k_per),
+            {a.part + (size_t)sp * (size_t)a.M * (size_t)a.N, (long)a.N, nullptr}, a.B, a.N, a.nnt, 0, a.ntt};
+}
+/* Its tile; false: it has none. */
+__device__ __forceinline__ bool gemm_tile(const GemmWork &w, int &nt, int &tt)
+{
+    nt = w.tile / w.ntt;
+    tt = w.tile - nt * w.ntt + w.tt0;
+    return w.tile >= 0;
+}
 
 /* Split K when the tile grid leaves most of the chip idle: `tiles` blocks of
  * `k_steps` loop iterations each.  Returns the number of splits (1 = none) so
@@ -165,17 +188,19 @@ int gemm_workspace(int kind, hipStream_t s, size_t bytes, float **out);
 /* C = bias + partial 0 + partial 1 + ... in that order (ckq_kernels.hip). */
 int gemm_launch_reduce(float *C, long ldc, const float *part, const float *bias, int M, int N, int splits, hipStream_t s);
 
-/* Common launch tail: sets up the split, launches `kernel` on grid (x, splits)
+/* Common launch tail: sets up the split, launches `kernel` on all pieces of all tiles
  * and, when split, the ordered reduction. */
 template <class Kernel>
-static int gemm_launch_split(Kernel kernel, GemmArgs &g, unsigned grid_x, int k_steps, hipStream_t s, unsigned threads = 256)
+static int gemm_launch_split(Kernel kernel, GemmArgs &g, int k_steps, hipStream_t s, unsigned threads = 256)
 {
     g.splits = gemm_choose_splits(g.ntt * g.nnt, k_steps);
     g.k_per = (k_steps + g.splits - 1) / g.splits;
     g.splits = (k_steps + g.k_per - 1) / g.k_per;          /* no empty split */
+    g.units = g.ntt * g.nnt * g.splits;
     g.part = nullptr;
+    const dim3 grid((unsigned)gemm_blocks(g.units, 1));
     if (g.splits <= 1) {
-        hipLaunchKernelGGL(kernel, dim3(grid_x, 1u), dim3(threads), 0, s, g);
+        hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, s, g);
         return (int)hipGetLastError();
     }
     const size_t need = (size_t)g.splits * (size_t)g.M * (size_t)g.N * sizeof(float);
@@ -186,7 +211,7 @@ static int gemm_launch_split(Kernel kernel, GemmArgs &g, unsigned grid_x, int k_
          * the scratch needs no clearing. */
         if (need > g.ext_part_bytes) return CKQ_ESCRATCH;
         g.part = g.ext_part;
-        hipLaunchKernelGGL(kernel, dim3(grid_x, (unsigned)g.splits), dim3(threads), 0, s, g);
+        hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, s, g);
         const int rc = (int)hipGetLastError();
         if (rc) return rc;
         return gemm_launch_reduce(g.C, g.ldc, g.part, g.bias, g.M, g.N, g.splits, s);
@@ -194,7 +219,7 @@ static int gemm_launch_split(Kernel kernel, GemmArgs &g, unsigned grid_x, int k_
     std::lock_guard<std::recursive_mutex> lock(gemm_split_mutex());
     int rc = gemm_workspace(0, s, need, &g.part);
     if (rc) return rc;
-    hipLaunchKernelGGL(kernel, dim3(grid_x, (unsigned)g.splits), dim3(threads), 0, s, g);
+    hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, s, g);
     rc = (int)hipGetLastError();
     if (rc) return rc;
     return gemm_launch_reduce(g.C, g.ldc, g.part, g.bias, g.M, g.N, g.splits, s);
@@ -298,8 +323,7 @@ static int gemm_launch_ksplit(Kernel k2, Kernel k3, Kernel k4, GemmArgs &g, int 
 }
 
 /* Grouped launch: the matrices of `in` against the same M x K activations, as one grid (no K split; the
- * callers group only what fills the chip without one).  rows_per_tile = weight rows of a block's tile; last_apart: the last token tile
- * of every matrix has block ids of its own (ckq_gemm_q4k_t96.hip). */
+ * callers group only what fills the chip without one).  rows_per_tile = weight rows of a block's tile. */
 struct GemmGroupIn {
     int          n;
     const void  *B[GEMM_GROUP_MAX];
@@ -318,15 +342,17 @@ static int gemm_group_tiles(const GemmGroupIn &in, int M, int tokens_per_tile, i
     return tiles;
 }
 template <class Kernel>
-static int gemm_launch_grouped(Kernel kernel, GemmArgs &g, const GemmGroupIn &in, hipStream_t s, unsigned threads = 256, int last_apart = 0)
+static int gemm_launch_grouped(Kernel kernel, GemmArgs &g, const GemmGroupIn &in, hipStream_t s, unsigned threads = 256)
 {
     unsigned grid = 0;
     g.ngroup = in.n;
     for (int p = 0; p < in.n; ++p) {
         const int nnt = (in.N[p] + GEMM_TILE_ROWS - 1) / GEMM_TILE_ROWS;
         g.grp[p] = {(const uint8_t *)in.B[p], in.bias[p], in.C[p], in.ldc[p], in.N[p], nnt, (int)grid, 0, g.ntt};
-        grid += (unsigned)gemm_blocks(g.ntt - last_apart, nnt) + (last_apart ? (unsigned)gemm_blocks(1, nnt) : 0u);
+        grid += (unsigned)(g.ntt * nnt);
     }
+    g.units = (int)grid;
+    grid = (grid + 7) & ~7u;
     g.B = g.grp[0].B; g.bias = g.grp[0].bias; g.C = g.grp[0].C; g.N = g.grp[0].N; g.ldc = g.grp[0].ldc; g.nnt = g.grp[0].nnt;
     g.splits = 1; g.k_per = 0; g.part = nullptr;
     hipLaunchKernelGGL(kernel, dim3(grid, 1u), dim3(threads), 0, s, g);
@@ -347,8 +373,9 @@ static bool gemm_ragged_last(const GemmGroupIn &in, int M, int bm)
     for (int p = 0; p < in.n; ++p) {
         const int nnt = (in.N[p] + GEMM_TILE_ROWS - 1) / GEMM_TILE_ROWS;
         whole += gemm_blocks(M / bm, nnt) / 8;
-        all += gemm_blocks(M / bm + 1, nnt) / 8;
+        all += (M / bm + 1) * nnt;
     }
+    all = (all + 7) / 8;                       /* all tiles of all matrices are dealt as one (gemm_work) */
     return (whole <= 32 && all > 32) || (whole <= 64 && all > 64) || (whole <= 132 && all > 128);
 }
 
@@ -364,7 +391,7 @@ static int gemm_deal_ragged_last(GemmArgs &g, const GemmGroupIn &in, int bm)
             g.grp[g.ngroup++] = {(const uint8_t *)in.B[p], in.bias[p], in.C[p], in.ldc[p], in.N[p], nnt, grid, ragged ? nfull : 0, ntt};
             grid += gemm_blocks(ntt, nnt);
         }
-    g.splits = 1; g.k_per = 0; g.part = nullptr;
+    g.units = 0; g.splits = 1; g.k_per = 0; g.part = nullptr;
     return grid;
 }
 template <class Kernel>

@@ -203,8 +203,7 @@ __global__ void __launch_bounds__(256 * KG, KG == 2 ? 1 : WPE) gemm_q4k_mfma_ker
 
     const GemmWork work = gemm_work(a, a.nb);
     int nt, tt;
-    if (!gemm_tile(work.id, work.ntt, work.nnt, nt, tt)) return;
-    tt += work.tt0;
+    if (!gemm_tile(work, nt, tt)) return;
     const int t0 = tt * BM, n0 = nt * GEMM_BN;
     const u32 wstride = (u32)a.nb * 144u, xstride = (u32)a.nb * 292u;
     const int b0 = work.k0, b1 = work.k1, last = b1 - 1;
@@ -496,8 +495,8 @@ static bool q4k_take_t96(int M, int nb, int tiles64, int blocks96, const int *nn
     const int left = M % T96_TOKENS;
     auto on_xcd = [&](int ntt) {              /* tiles that one gets */
         int t = 0;
-        for (int p = 0; p < n; ++p) t += gemm_blocks(ntt, nnt[p]) / 8;
-        return t;
+        for (int p = 0; p < n; ++p) t += ntt * nnt[p];
+        return (t + 7) / 8;
     };
     const int whole = on_xcd(M / T96_TOKENS), part = left ? on_xcd(1) : 0, t64 = on_xcd((M + GEMM_BM - 1) / GEMM_BM);
     if (whole > 2 * CUS || whole + part > 2 * CUS) return M >= 576 && 2 * blocks96 >= 3 * (16 * CUS);
@@ -539,17 +538,17 @@ int launch_gemm_q4k_mfma(const void *A, const void *B, const float *bias, float 
     if (q4k_take_t96(M, g.nb, tiles, gemm_q4k_t96_token_tiles(M) * g.nnt, &g.nnt, 1)) return launch_gemm_q4k_t96(g, s);
     if (sums) {
 #if CKQ_WITH_DUMP
-        if (two_groups) return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 2, true>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s, 512);
-        return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 1, true>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s, 256);
+        if (two_groups) return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 2, true>, g, g.nb, s, 512);
+        return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 1, true>, g, g.nb, s, 256);
 #else
         return CKQ_ENODUMP;
 #endif
     }
-    if (two_groups) return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 2>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s, 512);
+    if (two_groups) return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 2>, g, g.nb, s, 512);
     if (const int k = gemm_ksplit_pieces(M, N, g.nb, GEMM_KSPLIT_Q4K)) return gemm_launch_ksplit(gemm_q4k_ksplit_kernel<2>, gemm_q4k_ksplit_kernel<3>, gemm_q4k_ksplit_kernel<4>, g, k, s);
     const GemmGroupIn one = {1, {B}, {bias}, {C}, {N}, {ldc}};
     if (tiles > 256 && gemm_ragged_last(one, M, GEMM_BM)) return gemm_launch_ragged_last(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 1>, g, one, GEMM_BM, s);
-    return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 1>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s, 256);
+    return gemm_launch_split(gemm_q4k_mfma_kernel<CKQ_GEMM_WPE, 1>, g, g.nb, s, 256);
 }
 
 bool gemm_q4k_group_chains(const GemmGroupIn &in, int M, int K, GemmChains *ch)

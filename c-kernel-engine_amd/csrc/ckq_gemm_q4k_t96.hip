@@ -202,32 +202,18 @@ __global__ void __launch_bounds__(256, DUMP ? 1 : WPE) gemm_q4k_t96_kernel(GemmA
 
     /* tile of this block: full token tiles first (token tiles fastest, so neighbours share weights), of a group those of
      * all matrices, then the partial token tile of every weight-row tile */
-    GemmWork work = gemm_work(a, a.nb);
-    const int nfull = a.M / BM;
-    auto wholes = [&](int nnt) { return gemm_blocks(nfull, nnt); };
-    int id = work.id;
-    bool whole;
-    if (a.ngroup > 1) {
-        int all = wholes(a.grp[0].nnt) + wholes(a.grp[1].nnt);
-        if (a.ngroup > 2) all += wholes(a.grp[2].nnt);
-        if (a.ngroup > 3) all += wholes(a.grp[3].nnt);
-        id = blockIdx.x;
-        whole = id < all;
-        if (!whole) id -= all;
-        auto blocks = [&](const GemmProblem &p) { return whole ? wholes(p.nnt) : gemm_blocks(1, p.nnt); };
-        GemmProblem g = a.grp[0];
-        int n = blocks(g);
-        if (id >= n) { id -= n; g = a.grp[1]; n = blocks(g); }
-        if (a.ngroup > 2 && id >= n) { id -= n; g = a.grp[2]; n = blocks(g); }
-        if (a.ngroup > 3 && id >= n) { id -= n; g = a.grp[3]; }
-        work = {id, 0, a.nb, {g.C, g.ldc, g.bias}, g.B, g.N, g.nnt};
-    } else {
-        whole = id < wholes(work.nnt);
-        if (!whole) id -= wholes(work.nnt);
-    }
-    int nt, tt;
-    if (!gemm_tile(id, whole ? nfull : 1, work.nnt, nt, tt)) return;
-    if (!whole) tt = nfull;
+    const int nfull = a.M / BM, nwhole = nfull * a.units, whole_ids = (nwhole + 7) & ~7;
+    const bool whole = (int)blockIdx.x < whole_ids;
+    const int u = whole ? gemm_deal((int)blockIdx.x, nwhole) : gemm_deal((int)blockIdx.x - whole_ids, a.units);
+    if (u < 0) return;
+    int nt = whole ? u / nfull : u;
+    const int tt = whole ? u - nt * nfull : nfull;
+    GemmProblem g = a.grp[0];
+    if (a.ngroup > 1 && nt >= a.grp[1].id0) g = a.grp[1];
+    if (a.ngroup > 2 && nt >= a.grp[2].id0) g = a.grp[2];
+    if (a.ngroup > 3 && nt >= a.grp[3].id0) g = a.grp[3];
+    nt -= g.id0;
+    const GemmWork work = {0, 0, a.nb, {g.C, g.ldc, g.bias}, g.B, g.N, g.nnt, 0, 0};
     const int t0 = tt * BM, n0 = nt * T96_BN;
     const int ng = min(3, (a.M - t0 + 31) >> 5);
     const int tlim = a.M - 1 - t0;                 /* last token of the matrix, counted from t0 */
@@ -388,14 +374,20 @@ __global__ void __launch_bounds__(256, DUMP ? 1 : WPE) gemm_q4k_t96_kernel(GemmA
 
 int gemm_q4k_t96_token_tiles(int M) { return (M + T96_BM - 1) / T96_BM; }
 
-/* g: A, B, bias, C, M, N, nb, ldc, nnt and the dump pointer set; the token tiling is set here.
+/* Blocks over `row_tiles` tiles of weight rows in all: whole token tiles, then the partial one. */
+static unsigned t96_blocks(GemmArgs &g, int row_tiles)
+{
+    g.units = row_tiles;
+    return (unsigned)(gemm_blocks(g.M / T96_BM, row_tiles) + (g.M % T96_BM ? gemm_blocks(1, row_tiles) : 0));
+}
+
+/* g: A, B, bias, C, M, N, nb, ldc, nnt and the dump pointer set.
  * One block per tile, no K split: for launches whose tiles fill the chip. */
 int launch_gemm_q4k_t96(GemmArgs g, hipStream_t s)
 {
-    g.ntt = gemm_q4k_t96_token_tiles(g.M);
-    g.ngroup = 0; g.splits = 1; g.k_per = 0; g.part = nullptr;
-    const int last = g.M % T96_BM != 0;
-    const unsigned grid = (unsigned)(gemm_blocks(g.ntt - last, g.nnt) + (last ? gemm_blocks(1, g.nnt) : 0));
+    g.ngroup = 1; g.splits = 1; g.k_per = 0; g.part = nullptr;
+    g.grp[0] = {g.B, g.bias, g.C, g.ldc, g.N, g.nnt, 0, 0, 0};
+    const unsigned grid = t96_blocks(g, g.nnt);
     if (g.dump) {
 #if CKQ_WITH_DUMP
         hipLaunchKernelGGL((gemm_q4k_t96_kernel<CKQ_GEMM_WPE, true>), dim3(grid), dim3(256), 0, s, g);
@@ -411,6 +403,14 @@ int launch_gemm_q4k_t96(GemmArgs g, hipStream_t s)
 /* The matrices of `in` against the same activations as one grid of 96-token tiles; g: A, M, nb set. */
 int launch_gemm_q4k_t96_group(GemmArgs g, const GemmGroupIn &in, hipStream_t s)
 {
-    g.ntt = gemm_q4k_t96_token_tiles(g.M);
-    return gemm_launch_grouped(gemm_q4k_t96_kernel<CKQ_GEMM_WPE, false>, g, in, s, 256, g.M % T96_BM != 0);
+    int row_tiles = 0;
+    g.ngroup = in.n; g.splits = 1; g.k_per = 0; g.part = nullptr;
+    for (int p = 0; p < in.n; ++p) {
+        const int nnt = (in.N[p] + T96_BN - 1) / T96_BN;
+        g.grp[p] = {(const uint8_t *)in.B[p], in.bias[p], in.C[p], in.ldc[p], in.N[p], nnt, row_tiles, 0, 0};
+        row_tiles += nnt;
+    }
+    const unsigned grid = t96_blocks(g, row_tiles);
+    hipLaunchKernelGGL((gemm_q4k_t96_kernel<CKQ_GEMM_WPE, false>), dim3(grid), dim3(256), 0, s, g);
+    return (int)hipGetLastError();
 }

@@ -193,7 +193,7 @@ __global__ void __launch_bounds__(256, 1) gemm_q5k_mfma_kernel(GemmArgs a)
     /* token tiles fastest inside an XCD, so each XCD's L2 sees a weight tile once */
     const GemmWork work = gemm_work(a, a.nb);
     int nt, tt;
-    if (!gemm_tile(work.id, a.ntt, work.nnt, nt, tt)) return;
+    if (!gemm_tile(work, nt, tt)) return;
     const int t0 = tt * BM, n0 = nt * GEMM5_BN;
     const u32 wstride = (u32)a.nb * 176u, xstride = (u32)a.nb * 292u;
     const int b0 = work.k0, b1 = work.k1, last = b1 - 1;
@@ -335,8 +335,7 @@ __global__ void __launch_bounds__(256, 2) gemm_q5k_pair_kernel(GemmArgs a)
 
     const GemmWork work = gemm_work(a, a.nb);
     int nt, tt;
-    if (!gemm_tile(work.id, work.ntt, work.nnt, nt, tt)) return;
-    tt += work.tt0;
+    if (!gemm_tile(work, nt, tt)) return;
     const int t0 = tt * BM, n0 = nt * GEMM5_BN;
     const u32 wstride = (u32)a.nb * 176u, xstride = (u32)a.nb * 292u;
     const int b0 = work.k0, b1 = work.k1, last = b1 - 1;
@@ -566,21 +565,21 @@ int launch_gemm_q5k_mfma(const void *A, const void *B, const float *bias, float 
     g.nnt = (N + GEMM5_BN - 1) / GEMM5_BN;
     if (q5k_take_pair(g.ntt * g.nnt)) {
 #if CKQ_WITH_DUMP
-        if (sums) return gemm_launch_split(gemm_q5k_pair_kernel<true>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s);
+        if (sums) return gemm_launch_split(gemm_q5k_pair_kernel<true>, g, g.nb, s);
 #else
         if (sums) return CKQ_ENODUMP;
 #endif
         const GemmGroupIn one = {1, {B}, {bias}, {C}, {N}, {ldc}};
         if (g.ntt * g.nnt > 256 && gemm_ragged_last(one, M, GEMM5_BM)) return gemm_launch_ragged_last(gemm_q5k_pair_kernel<false>, g, one, GEMM5_BM, s);
-        return gemm_launch_split(gemm_q5k_pair_kernel<false>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s);
+        return gemm_launch_split(gemm_q5k_pair_kernel<false>, g, g.nb, s);
     }
 #if CKQ_WITH_DUMP
-    if (sums) return gemm_launch_split(gemm_q5k_mfma_kernel<true>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s);
+    if (sums) return gemm_launch_split(gemm_q5k_mfma_kernel<true>, g, g.nb, s);
 #else
     if (sums) return CKQ_ENODUMP;
 #endif
     if (const int k = gemm_ksplit_pieces(M, N, g.nb, GEMM_KSPLIT_Q5K)) return gemm_launch_ksplit(gemm_q5k_ksplit_kernel<2>, gemm_q5k_ksplit_kernel<3>, gemm_q5k_ksplit_kernel<4>, g, k, s);
-    return gemm_launch_split(gemm_q5k_mfma_kernel<false>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), g.nb, s);
+    return gemm_launch_split(gemm_q5k_mfma_kernel<false>, g, g.nb, s);
 }
 
 bool gemm_q5k_group_chains(const GemmGroupIn &in, int M, int K, GemmChains *ch)

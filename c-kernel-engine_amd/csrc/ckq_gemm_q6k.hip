@@ -185,7 +185,7 @@ __global__ void __launch_bounds__(256, 1) gemm_q6k_mfma_kernel(GemmArgs a)
     /* token tiles fastest inside an XCD, so each XCD's L2 sees a weight tile once */
     const GemmWork work = gemm_work(a, a.nb);
     int nt, tt;
-    if (!gemm_tile(work.id, a.ntt, work.nnt, nt, tt)) return;
+    if (!gemm_tile(work, nt, tt)) return;
     const int t0 = tt * BM, n0 = nt * GEMM6_BN;
     const u32 wstride = (u32)a.nb * 210u, xstride = (u32)a.nb * 292u;
     const int b0 = work.k0, b1 = work.k1, last = b1 - 1;
@@ -345,7 +345,7 @@ __global__ void __launch_bounds__(256, 2) gemm_q6k_pair_kernel(GemmArgs a)
 
     const GemmWork work = gemm_work(a, a.nb);
     int nt, tt;
-    if (!gemm_tile(work.id, a.ntt, work.nnt, nt, tt)) return;
+    if (!gemm_tile(work, nt, tt)) return;
     const int t0 = tt * BM, n0 = nt * GEMM6_BN;
     const u32 wstride = (u32)a.nb * 210u, xstride = (u32)a.nb * 292u;
     const int b0 = work.k0, b1 = work.k1, last = b1 - 1;
@@ -588,20 +588,19 @@ int launch_gemm_q6k_mfma(const void *A, const void *B, const float *bias, float 
     g.nnt = (N + GEMM6_BN - 1) / GEMM6_BN;
     const int form = q6k_form((M + 63) / 64 * g.nnt, (M + 127) / 128 * g.nnt, g.nb);
     g.ntt = form == Q6K_128 ? (M + 127) / 128 : (M + 63) / 64;
-    const unsigned grid = (unsigned)gemm_blocks(g.ntt, g.nnt);
     if (sums) {
 #if CKQ_WITH_DUMP
-        if (form == Q6K_PAIRED) return gemm_launch_split(gemm_q6k_pair_kernel<2, true>, g, grid, g.nb, s);
-        if (form == Q6K_128) return gemm_launch_split(gemm_q6k_mfma_kernel<4, true>, g, grid, g.nb, s);
-        return gemm_launch_split(gemm_q6k_mfma_kernel<2, true>, g, grid, g.nb, s);
+        if (form == Q6K_PAIRED) return gemm_launch_split(gemm_q6k_pair_kernel<2, true>, g, g.nb, s);
+        if (form == Q6K_128) return gemm_launch_split(gemm_q6k_mfma_kernel<4, true>, g, g.nb, s);
+        return gemm_launch_split(gemm_q6k_mfma_kernel<2, true>, g, g.nb, s);
 #else
         return CKQ_ENODUMP;
 #endif
     }
-    if (form == Q6K_PAIRED) return gemm_launch_split(gemm_q6k_pair_kernel<2>, g, grid, g.nb, s);
-    if (form == Q6K_128) return gemm_launch_split(gemm_q6k_mfma_kernel<4>, g, grid, g.nb, s);
+    if (form == Q6K_PAIRED) return gemm_launch_split(gemm_q6k_pair_kernel<2>, g, g.nb, s);
+    if (form == Q6K_128) return gemm_launch_split(gemm_q6k_mfma_kernel<4>, g, g.nb, s);
     if (const int k = gemm_ksplit_pieces(M, N, g.nb, GEMM_KSPLIT_Q6K)) return gemm_launch_ksplit(gemm_q6k_ksplit_kernel<2>, gemm_q6k_ksplit_kernel<3>, gemm_q6k_ksplit_kernel<4>, g, k, s);
-    return gemm_launch_split(gemm_q6k_mfma_kernel<2>, g, grid, g.nb, s);
+    return gemm_launch_split(gemm_q6k_mfma_kernel<2>, g, g.nb, s);
 }
 
 bool gemm_q6k_group_chains(const GemmGroupIn &in, int M, int K, GemmChains *ch)

@@ -61,7 +61,7 @@ __global__ void __launch_bounds__(256, 2) gemm_q80_mfma_kernel(GemmArgs a)
     /* token tiles fastest inside an XCD, so each XCD's L2 sees a weight tile once */
     const GemmWork work = gemm_work(a, (a.nb + KB - 1) / KB);
     int nt, tt;
-    if (!gemm_tile(work.id, a.ntt, work.nnt, nt, tt)) return;
+    if (!gemm_tile(work, nt, tt)) return;
     const int t0 = tt * BM, n0 = nt * BN;
     const int nblk = a.nb;                                  /* 32-blocks per row */
     const u32 stride = (u32)nblk * 34u;                     /* bytes per weight row and per activation row */
@@ -265,9 +265,9 @@ int launch_gemm_q80_mfma(const void *A, const void *B, const float *bias, float 
 #endif
     if (gemm_q80_dword_rows(g.nb, A, B)) return gemm_q80_dw_launch(g, s);
 #if CKQ_WITH_DUMP
-    if (sums) return gemm_launch_split(gemm_q80_mfma_kernel<true>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), (g.nb + GEMM8_KB - 1) / GEMM8_KB, s);
+    if (sums) return gemm_launch_split(gemm_q80_mfma_kernel<true>, g, (g.nb + GEMM8_KB - 1) / GEMM8_KB, s);
 #endif
-    return gemm_launch_split(gemm_q80_mfma_kernel<false>, g, (unsigned)gemm_blocks(g.ntt, g.nnt), (g.nb + GEMM8_KB - 1) / GEMM8_KB, s);
+    return gemm_launch_split(gemm_q80_mfma_kernel<false>, g, (g.nb + GEMM8_KB - 1) / GEMM8_KB, s);
 }
 
 int launch_gemm_q80_mfma_group(const void *A, const GemmGroupIn &in, int M, int K, hipStream_t s)

@@ -77,7 +77,7 @@ __global__ void __launch_bounds__(GEMM8_THREADS * TEAMS, DUMP ? 2 : 4) gemm_q80_
     /* token tiles fastest inside an XCD, so each XCD's L2 sees a weight tile once */
     const GemmWork work = gemm_work(a, (a.nb + KB - 1) / KB);
     int nt, tt;
-    if (!gemm_tile(work.id, a.ntt, work.nnt, nt, tt)) return;
+    if (!gemm_tile(work, nt, tt)) return;
     const int t0 = tt * BM, n0 = nt * BN;
     const int nblk = a.nb;                                  /* 32-blocks per row */
     const u32 stride = (u32)nblk * 34u;                     /* bytes per weight row and per activation row */
@@ -350,12 +350,11 @@ template <int TG, int TEAMS>
 static int dw_launch(GemmArgs &g, hipStream_t s)
 {
     g.ntt = (g.M + 32 * TG - 1) / (32 * TG);
-    const unsigned grid = (unsigned)gemm_blocks(g.ntt, g.nnt);
     const int steps = (g.nb + GEMM8_KB - 1) / GEMM8_KB;
 #if CKQ_WITH_DUMP
-    if (g.dump) return gemm_launch_split(gemm_q80_dw_kernel<TG, TEAMS, true>, g, grid, steps, s, GEMM8_THREADS * TEAMS);
+    if (g.dump) return gemm_launch_split(gemm_q80_dw_kernel<TG, TEAMS, true>, g, steps, s, GEMM8_THREADS * TEAMS);
 #endif
-    return gemm_launch_split(gemm_q80_dw_kernel<TG, TEAMS, false>, g, grid, steps, s, GEMM8_THREADS * TEAMS);
+    return gemm_launch_split(gemm_q80_dw_kernel<TG, TEAMS, false>, g, steps, s, GEMM8_THREADS * TEAMS);
 }
 int gemm_q80_dw_launch(GemmArgs &g, hipStream_t s)
 {

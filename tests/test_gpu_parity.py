@@ -2251,6 +2251,27 @@ def test_gemm_mfma_tiles_over_the_xcds(fmt, M):
             assert float((a - w).abs().max()) <= bar and float((b - w).abs().max()) <= bar
 
 
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("M,N,K", [(129, 1500, 7168), (65, 129, 16384), (200, 2700, 2304), (385, 1700, 3328)])
+def test_gemm_pieces_of_k_dealt_with_their_tiles(fmt, M, N, K):
+    """Every piece of K of every tile is computed once where neither their number nor that of the tiles divides by the eight XCDs: 36 tiles in up to seven
+    pieces (the last one shorter), 4 in sixteen, 88 in two, 98 in two.  Against the streaming kernel, whose terms and order differ: the bar of
+    the other parity tests."""
+    import torch
+    L = ckq.lib()
+    say("pieces of K over the XCDs", fmt, M, N, K)
+    xq = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, 9963)), T.act_fmt(fmt), M)
+    W = P.to_device(T.random_blocks(fmt, N * (K // T.ELEMS[fmt]), 9964))
+    try:
+        L.ckq_set_gemm_policy(2)
+        want = P.dev_gemm_nt(fmt, xq, W, None, M, N, K).clone()
+        L.ckq_set_gemm_policy(1)
+        got = P.dev_gemm_nt(fmt, xq, W, None, M, N, K)
+    finally:
+        L.ckq_set_gemm_policy(0)
+    assert float((got - want).abs().max()) <= TOL * float(want.abs().max())
+
+
 @pytest.mark.parametrize("fmt,variants", [("q5_k", (2, 1)), ("q4_k", (64, 96))])
 @pytest.mark.parametrize("M,Ns,K", [(405, (11008, 11008), 768), (65, (17000,), 512), (88, (9000, 7700), 256), (282, (7041,), 1024), (257, (6657, 300), 512)])
 def test_gemm_ragged_token_tiles_dealt_last(fmt, variants, M, Ns, K):
