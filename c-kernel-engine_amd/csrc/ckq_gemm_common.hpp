@@ -409,8 +409,8 @@ int launch_gemm_q4k_mfma_group(const void *A, const GemmGroupIn &in, int M, int 
 int launch_gemm_q5k_mfma_group(const void *A, const GemmGroupIn &in, int M, int K, hipStream_t s);
 int launch_gemm_q6k_mfma_group(const void *A, const GemmGroupIn &in, int M, int K, hipStream_t s);
 int launch_gemm_q80_mfma_group(const void *A, const GemmGroupIn &in, int M, int K, hipStream_t s);
-/* Q8_0 rows that start on dwords and hold an even number of blocks: ckq_gemm_q80_dw.hip */
-static inline bool gemm_q80_dword_rows(int nb, const void *A, const void *B) { return nb % 2 == 0 && ((uintptr_t)A | (uintptr_t)B) % 4 == 0; }
+/* Q8_0 operands that start on dwords: ckq_gemm_q80_dw.hip */
+static inline bool gemm_q80_on_dwords(const void *A, const void *B) { return ((uintptr_t)A | (uintptr_t)B) % 4 == 0; }
 int gemm_q80_dw_launch(GemmArgs &g, hipStream_t s);
 int gemm_q80_dw_launch_group(GemmArgs &g, const GemmGroupIn &in, hipStream_t s);
 int launch_gemm_q4k_mfma(const void *A, const void *B, const float *bias, float *C, int M, int N, int K, long ldc, const GemmOpts &opts, hipStream_t s);

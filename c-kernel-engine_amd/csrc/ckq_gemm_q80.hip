@@ -263,7 +263,7 @@ int launch_gemm_q80_mfma(const void *A, const void *B, const float *bias, float 
 #if !CKQ_WITH_DUMP
     if (sums) return CKQ_ENODUMP;
 #endif
-    if (gemm_q80_dword_rows(g.nb, A, B)) return gemm_q80_dw_launch(g, s);
+    if (gemm_q80_on_dwords(A, B)) return gemm_q80_dw_launch(g, s);
 #if CKQ_WITH_DUMP
     if (sums) return gemm_launch_split(gemm_q80_mfma_kernel<true>, g, (g.nb + GEMM8_KB - 1) / GEMM8_KB, s);
 #endif
@@ -281,7 +281,7 @@ int launch_gemm_q80_mfma_group(const void *A, const GemmGroupIn &in, int M, int 
      * without a K split, so that a group never needs scratch) */
     GemmGroupIn kind[2] = {};
     for (int p = 0; p < in.n; ++p) {
-        GemmGroupIn &k = kind[gemm_q80_dword_rows(g.nb, A, in.B[p])];
+        GemmGroupIn &k = kind[gemm_q80_on_dwords(A, in.B[p])];
         k.B[k.n] = in.B[p]; k.bias[k.n] = in.bias[p]; k.C[k.n] = in.C[p]; k.N[k.n] = in.N[p]; k.ldc[k.n] = in.ldc[p];
         ++k.n;
     }

@@ -1,6 +1,6 @@
 /*
- * ckq_gemm_q80_dw.hip - prefill GEMM, Q8_0 weights x Q8_0 activations, on the gfx950 int8 matrix cores, for rows that start on
- * dwords and hold an even number of blocks (K a multiple of 64); ckq_gemm_q80.hip takes the others.
+ * ckq_gemm_q80_dw.hip - prefill GEMM, Q8_0 weights x Q8_0 activations, on the gfx950 int8 matrix cores, for operands that start on
+ * dwords; ckq_gemm_q80.hip takes the others.
  *
  *   C[t][n] = sum_j dx(t,j) * (dw(n,j) * S(t,n,j))   (+ bias[n]),   S = the integer dot of 32-block j
  *
@@ -33,11 +33,19 @@
  *   first (one barrier more before, one less after), so that one computes while the other waits for its copies and
  *   finishes them; in step they gain half of that (36.9 for the first).
  * Against ckq_gemm_q80.hip (weights two bytes off): 333 x 4864 x 4096 51.3, 512 x 9728 x 896 34.7, 2048 x 11008 x 4096 426.
+ *
+ * Rows of an odd number of blocks (K = 32 mod 64) start on a dword and two bytes behind one in turn.  A wave's sixteen rows of one operand are
+ * therefore all even or all odd ones: of those the quants of one block in two lie on dwords and of the other two bytes off, which costs two more LDS reads
+ * and two byte alignments an operand and block.  With their quantizer, against ckq_gemm_q80.hip: 133 x 5950 x 10272 112.6 -> 71.0, 1628 x 5551 x 6752 336 ->
+ * 251, 512 x 4096 x 8224 103.5 -> 79.8 (K = 8192: 67.5), 118 x 13225 x 4960 61 -> 48; 31 sizes 1.18 on average (1.05 to 1.58).  rms error 0.54 to 0.84 of that kernel's.
+ * A last iteration of fewer blocks is copied like the others while the one before it is multiplied, and reaches into what follows the row: fetched apart,
+ * dword by dword and at the end, it was a round trip to memory that nothing hid (1040 x 672 x 8640 56.1 -> 54.0, odd 487 x 17537 x 1248 88.2 -> 81.5).
  */
 #include "ckq_gemm_common.hpp"
 
 constexpr int GEMM8_BN = 128, GEMM8_KB = 4;      /* rows, 32-blocks per iteration */
 constexpr int GEMM8_THREADS = 512;               /* of a team */
+enum { DW_WHOLE, DW_EVEN, DW_ODD };              /* 32-blocks per row: a multiple of GEMM8_KB, another even number, an odd one */
 constexpr int GEMM8_PITCH = 144;                 /* bytes of an operand row's image in LDS: see below */
 typedef float ckq_v4f __attribute__((ext_vector_type(4)));
 
@@ -56,14 +64,15 @@ __device__ __forceinline__ float q80_output(const uint8_t *w, const uint8_t *x, 
 /*
  * LDS image of an operand row, 144 bytes for the four blocks of an iteration: the 136 bytes as they are in memory, 34 dwords, in
  * nine 16-byte chunks (adjacent lanes of a copy fetch adjacent chunks, all from dword-aligned addresses).  Chunk 8 holds the last
- * sixteen, so dwords 30 to 33 of the run lie at 32 to 35.  A pair of blocks is 17 dwords: [d0 q0q1] seven of quants [q30q31 d1]
+ * sixteen, so dwords 30 to 33 of the run lie at 32 to 35 (of an odd number of blocks, whose run may start two bytes early, dwords 31 to 34).  A pair of blocks is 17 dwords: [d0 q0q1] seven of quants [q30q31 d1]
  * eight of quants.  Once a row has landed, the lane in charge makes [q0q1 q30q31] of the first and the ninth - the order of
  * the 32 products of a block is free as long as both operands have the same - and leaves the scales as fp32.  Lane quarter q takes
  * dwords q and q + 4 of a block: with rows 36 dwords apart, and the waves' regions a multiple of four rows, every bank serves one lane.
  */
-template <int TG, int TEAMS, bool DUMP>
+template <int TG, int TEAMS, int ROWS, bool DUMP>
 __global__ void __launch_bounds__(GEMM8_THREADS * TEAMS, DUMP ? 2 : 4) gemm_q80_dw_kernel(GemmArgs a)
 {
+    constexpr bool ODD = ROWS == DW_ODD, PART = ROWS != DW_WHOLE;
     constexpr int BM = 32 * TG, BN = GEMM8_BN, KB = GEMM8_KB, PITCH = GEMM8_PITCH, MAGIC = 0x4B400000;
     constexpr int XR = 4 * TG, REGION = (16 + XR) * PITCH;  /* a wave brings in sixteen weight rows and XR tokens */
     constexpr int WSCALES = 8 * REGION, XSCALES = WSCALES + KB * BN * 4, STAGE = XSCALES + KB * BM * 4;     /* fp32 scales, [block][row], [block][token] */
@@ -89,33 +98,45 @@ __global__ void __launch_bounds__(GEMM8_THREADS * TEAMS, DUMP ? 2 : 4) gemm_q80_
         return ckq_v4i{__builtin_amdgcn_readfirstlane((int)(u32)b), __builtin_amdgcn_readfirstlane((int)(u32)(b >> 32)), 0x7fffffff, 0x00020000};
     };
     const ckq_v4i bw = buffer(wbase), bx = buffer(xbase);
-    auto w_row = [&](int l) { return (u32)min(64 * (l >> 6) + 4 * (l & 15) + ((l >> 4) & 3), work.N - 1 - n0) * stride; };
-    auto x_row = [&](int t) { return (u32)min(t, a.M - 1 - t0) * stride; };
+    /* token slot l of the tile: of an odd number of blocks, sixteen even tokens and sixteen odd ones in turn */
+    auto token_at = [](int l) { return ODD ? (l & ~31) + 2 * (l & 15) + ((l >> 4) & 1) : l; };
+    /* rows that are not there: the last one that is, of the same parity if there is one (other bytes would be taken for its scales) */
+    auto clamped = [](int r, int last) {
+        const int c = min(r, last);
+        return (u32)(ODD && c > 0 ? c - ((c ^ r) & 1) : c);
+    };
+    auto w_row = [&](int l) { return clamped(64 * (l >> 6) + 4 * (l & 15) + ((l >> 4) & 3), work.N - 1 - n0) * stride; };
+    auto x_row = [&](int l) { return clamped(token_at(l), a.M - 1 - t0) * stride; };
 
     /* A wave copies sixteen weight rows (144 chunks, three instructions) and XR tokens (36 chunks for four, one instruction;
      * 72 and 108, two) into its region of a stage, and finishes the same rows when they have landed. */
-    constexpr int NC = 3 + (9 * XR + 63) / 64;
+    constexpr int NC = 3 + (9 * XR + 63) / 64, LAST_CHUNK = ODD ? 124 : 120;
     u32 c_src[NC];
     bool c_on[NC];
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
         const int ci = 64 * (i < 3 ? i : i - 3) + lane, r = ci / 9, c = ci % 9;
         c_on[i] = ci < (i < 3 ? 144 : 9 * XR);
-        c_src[i] = (i < 3 ? w_row(16 * wave + min(r, 15)) : x_row(XR * wave + min(r, XR - 1))) + (u32)min(16 * c, 120);
+        c_src[i] = ((i < 3 ? w_row(16 * wave + min(r, 15)) : x_row(XR * wave + min(r, XR - 1))) & ~3u) + (u32)min(16 * c, LAST_CHUNK);
     }
+    /* The last iteration may hold fewer blocks.  Its chunks then reach into the rows behind, but not past the end of the operand: those that
+     * would start 16 bytes before it instead, and what its last row needs of them, one dword or two, is fetched when the rest has landed. */
+    const int w_last = work.N - 1 - n0, x_last = a.M - 1 - t0;
+    auto last_chunk_of = [&](int rows) {
+        const size_t bytes = (size_t)rows * stride;
+        return (u32)min((bytes & ~(size_t)3) - 16, (size_t)0x7fffffe0);
+    };
+    const u32 w_end = last_chunk_of(w_last + 1), x_end = last_chunk_of(x_last + 1);
     auto copy = [&](int it, uint8_t *sg) {
         const u32 dst = lds_address(sg + REGION * wave);
+        auto all = [&](auto src, int k) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < NC; ++i)
-            if (c_on[i]) lds_copy16(i < 3 ? bw : bx, dst + (u32)(i < 3 ? 1024 * i : 16 * PITCH + 1024 * (i - 3)), c_src[i], it * (KB * 34));
-    };
-    /* K ends after 17 dwords of the iteration: fetched one by one, a 16-byte chunk could pass the end of the matrix */
-    auto copy_tail = [&](int it, uint8_t *sg) {
-        for (int e = lane; e < (16 + XR) * 17; e += 64) {
-            const int r = e / 17, d = e % 17;
-            const uint8_t *const src = r < 16 ? wbase + w_row(16 * wave + r) : xbase + x_row(XR * wave + r - 16);
-            *reinterpret_cast<u32 *>(sg + REGION * wave + PITCH * r + 4 * d) = ld4<4>(src + (u32)it * (KB * 34u) + 4u * (u32)d);
-        }
+            for (int i = 0; i < NC; ++i)
+                if (c_on[i]) lds_copy16(i < 3 ? bw : bx, dst + (u32)(i < 3 ? 1024 * i : 16 * PITCH + 1024 * (i - 3)), src(i), k);
+        };
+        const int k = __builtin_amdgcn_readfirstlane(it * (KB * 34));
+        if (!PART || it * KB + KB <= nblk) all([&](int i) { return c_src[i]; }, k);
+        else all([&](int i) { return i < 3 ? min(c_src[i] + (u32)k, w_end) : min(c_src[i] + (u32)k, x_end); }, __builtin_amdgcn_readfirstlane(k & 0));
     };
     /* two lanes per row, one for each pair of blocks */
     const int f_row = lane >> 1, f_p = lane & 1;
@@ -124,12 +145,33 @@ __global__ void __launch_bounds__(GEMM8_THREADS * TEAMS, DUMP ? 2 : 4) gemm_q80_
     auto finish = [&](int it, uint8_t *sg) {
         if (f_row >= 16 + XR) return;
         u32 *const d = reinterpret_cast<u32 *>(sg + REGION * wave + PITCH * f_row);
+        if constexpr (ODD) {
+            const int p = f_row < 16 ? wave & 1 : (XR * wave + f_row - 16) >> 4 & 1, left = nblk - it * KB - 2 * f_p;
+            const u32 e0 = d[17 * f_p], e1 = d[17 * f_p + 8 + p];
+            float *const sc = reinterpret_cast<float *>(sg + f_w + 2 * f_p * f_pitch);
+            *sc = left > 0 ? h2f(e0 >> (16 * p) & 0xffff) : 0.0f;
+            *reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(sc) + f_pitch) = left > 1 ? h2f(e1 >> (16 - 16 * p) & 0xffff) : 0.0f;
+            return;
+        }
         const bool live = 2 * f_p < nblk - it * KB;
         const u32 d0 = d[17 * f_p], d8 = d[17 * f_p + 8];
         d[17 * f_p] = __builtin_amdgcn_alignbyte(d8, d0, 2);
         float *const sc = reinterpret_cast<float *>(sg + f_w + 2 * f_p * f_pitch);
         *sc = live ? h2f(d0 & 0xffff) : 0.0f;
         *reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(sc) + f_pitch) = live ? h2f(d8 >> 16) : 0.0f;
+    };
+
+    auto mend = [&](int it, uint8_t *sg) {
+        const int r = lane, slot = r < 16 ? 16 * wave + r : XR * wave + r - 16, row = r < 16 ? 64 * (slot >> 6) + 4 * (slot & 15) + ((slot >> 4) & 3) : token_at(slot);
+        if (r >= 16 + XR || row != (r < 16 ? w_last : x_last)) return;
+        /* 34 bytes a block, from a dword or from two bytes behind one: dwords 8, 16 or 24 and 25, the last of which may be half of one */
+        const int left = nblk - it * KB;
+        const u32 ofs = (u32)row * stride;
+        const u32 at = (ofs & ~3u) + (u32)it * (KB * 34u) + 32u * (u32)left;
+        const uint8_t *const src = r < 16 ? wbase + at : xbase + at;
+        u32 *const d = reinterpret_cast<u32 *>(sg + REGION * wave + PITCH * r) + 8 * left;
+        d[0] = left == 1 && !(ofs & 2) ? ld2(src) : ld4<4>(src);
+        if (left == 3) d[1] = !(ofs & 2) ? ld2(src + 4) : ld4<4>(src + 4);
     };
 
     ckq_v4f acc[TG][4];                                     /* [token group][row group] */
@@ -141,10 +183,18 @@ __global__ void __launch_bounds__(GEMM8_THREADS * TEAMS, DUMP ? 2 : 4) gemm_q80_
     asm volatile("" : "+v"(magic));                         /* kept in registers: as a constant it is copied before every use */
 
     /* this lane's operands of the wave's two blocks, and where their scales are */
-    const int opd = 17 * kh + q, opd_hi = opd + 9 + (kh ? 6 : 4);       /* block 3 ends in the last chunk */
+    const int opd = 17 * kh + q, opd_hi = ODD ? opd + 13 + (kh && q ? 1 : 0) : opd + 9 + (kh ? 6 : 4);       /* block 3 ends in the last chunk */
     auto operand = [](const uint8_t *p, int lo, int hi) {
         const u32 *const d = reinterpret_cast<const u32 *>(p);
         return (long)((uint64_t)d[lo] | ((uint64_t)d[hi] << 32));
+    };
+    /* ODD: of rows of parity p the quants of block jj start on a dword (jj != p) or two bytes behind one */
+    auto odd_operand = [&](const uint8_t *r, int jj, int p) __attribute__((always_inline)) {
+        const u32 *const d = reinterpret_cast<const u32 *>(r);
+        const int lo = jj ? opd + 9 : opd + p, hi = jj ? opd_hi : lo + 4;
+        if (__builtin_constant_p(p) && jj != p) return (long)((uint64_t)d[lo] | ((uint64_t)d[hi] << 32));
+        const u32 sh = jj != p ? 0 : 2;
+        return (long)((uint64_t)__builtin_amdgcn_alignbyte(d[lo + 1], d[lo], sh) | ((uint64_t)__builtin_amdgcn_alignbyte(d[hi + 1], d[hi], sh) << 32));
     };
     auto compute_block = [&](const uint8_t *sg, int it, int jj) __attribute__((always_inline)) {
         const uint8_t *const wl = sg + 4 * rh * REGION + i16 * PITCH;
@@ -153,16 +203,25 @@ __global__ void __launch_bounds__(GEMM8_THREADS * TEAMS, DUMP ? 2 : 4) gemm_q80_
         const int tw = 16 * TG * th;
         const int lo = jj ? opd + 9 : opd, hi = jj ? opd_hi : opd + 4;
         long w[4], x[TG];
+        auto take_x = [&](int tg) __attribute__((always_inline)) {
+            const uint8_t *const r = token(tw + 16 * tg + i16);
+            x[tg] = !ODD ? operand(r, lo, hi) : TG % 2 ? odd_operand(r, jj, (th + tg) & 1) : odd_operand(r, jj, tg & 1);
+        };
+        constexpr int AHEAD = ODD && TG == 3 ? 1 : TG;          /* three groups' operands and their pieces do not fit the registers of four waves per SIMD */
 #pragma unroll
-        for (int tg = 0; tg < TG; ++tg) x[tg] = operand(token(tw + 16 * tg + i16), lo, hi);
+        for (int tg = 0; tg < AHEAD; ++tg) take_x(tg);
 #pragma unroll
-        for (int g = 0; g < 4; ++g) w[g] = operand(wl + REGION * g, lo, hi);
+        for (int g = 0; g < 4; ++g) w[g] = ODD ? odd_operand(wl + REGION * g, jj, g & 1) : operand(wl + REGION * g, lo, hi);
         const ckq_v4f dwb = *reinterpret_cast<const ckq_v4f *>(sg + WSCALES + 4 * ((2 * kh + jj) * BN + 64 * rh + 4 * i16));
         float dwm[4];
 #pragma unroll
         for (int g = 0; g < 4; ++g) dwm[g] = dwb[g] * -12582912.0f;
 #pragma unroll
         for (int tg = 0; tg < TG; ++tg) {
+            if (tg >= AHEAD) {
+                asm volatile("" ::: "memory");
+                take_x(tg);
+            }
             const ckq_v4f dxb = *reinterpret_cast<const ckq_v4f *>(sg + XSCALES + 4 * ((2 * kh + jj) * BM + tw + 16 * tg + 4 * q));
             ckq_v4i d[4];
 #pragma unroll
@@ -175,7 +234,7 @@ __global__ void __launch_bounds__(GEMM8_THREADS * TEAMS, DUMP ? 2 : 4) gemm_q80_
                     const int di = d[g][r];
                     t[r] = __builtin_fmaf(dwb[g], __builtin_bit_cast(float, di), dwm[g]);
                     if constexpr (DUMP) {
-                        int tr = t0 + tw + 16 * tg + 4 * q + r;
+                        int tr = t0 + token_at(tw + 16 * tg + 4 * q + r);
                         asm volatile("" : "+v"(tr));   /* store addresses formed here, not kept in registers */
                         const int n = n0 + 64 * rh + 4 * i16 + g, b = it * KB + 2 * kh + jj;
                         if (tr < a.M && n < work.N && b < nblk) a.dump[((size_t)tr * work.N + n) * nblk + (size_t)b] = di - MAGIC;
@@ -190,10 +249,10 @@ __global__ void __launch_bounds__(GEMM8_THREADS * TEAMS, DUMP ? 2 : 4) gemm_q80_
         for (int tg = 0; tg < TG; ++tg) asm volatile("" : "+v"(acc[tg][0]), "+v"(acc[tg][1]), "+v"(acc[tg][2]), "+v"(acc[tg][3]) :: "memory");
     };
 
-    /* the whole iterations, in TEAMS runs; a team that has one less still comes to the barriers */
-    const int nfull = min(niter, nblk / KB), nrun = (max(nfull - it0, 0) + TEAMS - 1) / TEAMS;
-    const int run0 = it0 + team * nrun, run1 = min(run0 + nrun, nfull);
-    if (nrun > 0) {
+    /* the iterations in TEAMS runs, the whole ones in equal parts and one with fewer blocks to the last team; a team that has one less still comes to the barriers */
+    const int nrun = (max(min(niter, nblk / KB) - it0, 0) + TEAMS - 1) / TEAMS, nstep = TEAMS == 1 ? niter - it0 : max(nrun, niter - it0 - nrun);
+    const int run0 = it0 + team * nrun, run1 = TEAMS == 1 || team ? niter : run0 + nrun;
+    {
         auto landed = [] {                                  /* vmcnt(0) lgkmcnt(0) */
             __builtin_amdgcn_s_waitcnt(0x0070);
             asm volatile("" ::: "memory");
@@ -203,7 +262,7 @@ __global__ void __launch_bounds__(GEMM8_THREADS * TEAMS, DUMP ? 2 : 4) gemm_q80_
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
         };
-        auto at = [&](int it) { return min(it, nfull - 1); };
+        auto at = [&](int it) { return min(it, niter - 1); };
         copy(at(run0), stage[0]);
         landed();
         finish(at(run0), stage[0]);
@@ -220,26 +279,27 @@ __global__ void __launch_bounds__(GEMM8_THREADS * TEAMS, DUMP ? 2 : 4) gemm_q80_
             finish(at(it + 1), next);
             meet();
         };
-        if constexpr (DUMP) {                               /* one copy of the stores */
-            for (int k = 0; k < nrun; ++k) step(run0 + k, stage[k & 1], stage[(k + 1) & 1]);
-        } else for (int k = 0; k < nrun; k += 2) {
+        /* rows of whole iterations go on copying to the end, a step more of one kind: the last step apart costs short rows 1 % (512 x 9728 x 896) */
+        const int nloop = PART ? nstep - 1 : nstep;
+        if constexpr (DUMP || (ODD && TG == 3)) {           /* one copy of the stores; of three groups and an odd number of blocks two spill a register */
+            for (int k = 0; k < nloop; ++k) step(run0 + k, stage[k & 1], stage[(k + 1) & 1]);
+        } else for (int k = 0; k < nloop; k += 2) {
             step(run0 + k, stage[0], stage[1]);
-            if (k + 1 < nrun) step(run0 + k + 1, stage[1], stage[0]);
+            if (k + 1 < nloop) step(run0 + k + 1, stage[1], stage[0]);
+        }
+        if constexpr (PART) {
+            const int it = run0 + nstep - 1;
+            uint8_t *const cur = stage[(nstep - 1) & 1];
+            if (niter * KB > nblk && (w_last < BN || x_last < BM)) {
+                if (it == niter - 1) mend(it, cur);
+                meet();
+            }
+            if (TEAMS == 1 || it < run1) compute_block(cur, it, 0);
+            if (TEAMS == 2) __builtin_amdgcn_s_barrier();
+            if (TEAMS == 1 || it < run1) compute_block(cur, it, 1);
         }
         if (TEAMS == 2 && !team) __builtin_amdgcn_s_barrier();
-    }
-    if (nfull < niter) {
-        const bool mine = team == TEAMS - 1;
-        if (mine) {
-            copy_tail(nfull, stage[0]);
-            finish(nfull, stage[0]);
-        }
-        __syncthreads();
-        if (mine) {
-            compute_block(stage[0], nfull, 0);
-            compute_block(stage[0], nfull, 1);
-        }
-        __syncthreads();
+        if (PART) __syncthreads();                          /* the stages have been read */
     }
 
     /* the parts of K: of the 2 TEAMS waves of a sub-tile, wave `part` keeps token groups tg with tg % (2 TEAMS) == part and hands
@@ -267,7 +327,8 @@ __global__ void __launch_bounds__(GEMM8_THREADS * TEAMS, DUMP ? 2 : 4) gemm_q80_
 #pragma unroll
     for (int tg = 0; tg < TG; ++tg) {
         if (tg % PARTS != part) continue;
-        const int t = t0 + 16 * (TG * th + tg) + 4 * q;
+        constexpr int TSTEP = ODD ? 2 : 1;
+        const int t = t0 + token_at(16 * (TG * th + tg) + 4 * q);
         ckq_v4f o4[4];
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
@@ -280,8 +341,8 @@ __global__ void __launch_bounds__(GEMM8_THREADS * TEAMS, DUMP ? 2 : 4) gemm_q80_
         bool fix = false;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            if (t + r >= a.M) continue;
-            float *dst = o.C + (size_t)(t + r) * o.ldc + n;
+            if (t + TSTEP * r >= a.M) continue;
+            float *dst = o.C + (size_t)(t + TSTEP * r) * o.ldc + n;
             float v[4];
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
@@ -296,7 +357,7 @@ __global__ void __launch_bounds__(GEMM8_THREADS * TEAMS, DUMP ? 2 : 4) gemm_q80_
         }
         if (fix) {
             for (int e = 0; e < 16; ++e) {
-                const int tr = t + (e >> 2), nr = n + (e & 3);
+                const int tr = t + TSTEP * (e >> 2), nr = n + (e & 3);
                 if (tr >= a.M || nr >= work.N) continue;
                 float *dst = o.C + (size_t)tr * o.ldc + nr;
                 if (*dst == *dst) continue;
@@ -318,7 +379,9 @@ static const DwForm dw_forms[5] = {{1, 1, 3, 4.0f, 0.40f, 0.39f, 0.0f}, {2, 1, 2
 
 /* The form for `row_tiles` tiles of weight rows in all; single: one matrix, which may be split along K.  64 tokens and one team
  * are always possible; another form only if its chains of multiply-adds are no longer (fewer splits of K would make them so, and the
- * error larger) and, if it is split, with no more scratch than that form or the entry point that allocates nothing has. */
+ * error larger) and, if it is split, with no more scratch than that form or the entry point that allocates nothing has; rows of an odd number of
+ * blocks, which were another kernel's, never with more than that form.  Their 32-token tiles of two teams take 1.5 us an iteration where the others take 1.18 (four
+ * more LDS reads in a step that waits for itself): 1040 x 672 x 8608 64.5 with them, 57.7 with 64 tokens, one team and a split. */
 static int dw_form(int M, int nb, long rows, long row_tiles, bool single)
 {
     const int steps = (nb + GEMM8_KB - 1) / GEMM8_KB;
@@ -335,10 +398,11 @@ static int dw_form(int M, int nb, long rows, long row_tiles, bool single)
         const size_t need = s > 1 ? (size_t)s * (size_t)M * (size_t)rows * 4 : 0;
         if (k == 1) {
             chain = iters;
-            scratch = need > CKQ_NOALLOC_SCRATCH_BYTES ? need : CKQ_NOALLOC_SCRATCH_BYTES;
+            scratch = nb % 2 || need > CKQ_NOALLOC_SCRATCH_BYTES ? need : CKQ_NOALLOC_SCRATCH_BYTES;
         } else if (iters > chain || need > scratch || (f.teams > 1 && (s > 1 || !single))) continue;
         const long on_cu = (tiles * s + 255) / 256, rounds = (on_cu + f.fit - 1) / f.fit;
-        const float t = f.launch + (float)iters * (f.wait * (float)rounds + f.work * (float)on_cu) + f.round * (float)rounds +
+        const float wait = nb % 2 && k == 3 ? 1.5f : f.wait;       /* 32 tokens, two teams, rows of an odd number of blocks */
+        const float t = f.launch + (float)iters * (wait * (float)rounds + f.work * (float)on_cu) + f.round * (float)rounds +
                         1.45f * out * (float)(s > 1 ? 1 + 2 * s : 1) + (s > 1 ? 2.4f : 0.0f);
         if (k == 1 || t < least) { least = t; best = k; }
     }
@@ -346,18 +410,29 @@ static int dw_form(int M, int nb, long rows, long row_tiles, bool single)
 }
 
 /* g: operands, sizes, nnt set by the caller (ckq_gemm_q80.hip). */
-template <int TG, int TEAMS>
-static int dw_launch(GemmArgs &g, hipStream_t s)
+template <int TG, int TEAMS, int ROWS>
+static int dw_launch_rows(GemmArgs &g, hipStream_t s)
 {
     g.ntt = (g.M + 32 * TG - 1) / (32 * TG);
     const int steps = (g.nb + GEMM8_KB - 1) / GEMM8_KB;
 #if CKQ_WITH_DUMP
-    if (g.dump) return gemm_launch_split(gemm_q80_dw_kernel<TG, TEAMS, true>, g, steps, s, GEMM8_THREADS * TEAMS);
+    if (g.dump) return gemm_launch_split(gemm_q80_dw_kernel<TG, TEAMS, ROWS, true>, g, steps, s, GEMM8_THREADS * TEAMS);
 #endif
-    return gemm_launch_split(gemm_q80_dw_kernel<TG, TEAMS, false>, g, steps, s, GEMM8_THREADS * TEAMS);
+    return gemm_launch_split(gemm_q80_dw_kernel<TG, TEAMS, ROWS, false>, g, steps, s, GEMM8_THREADS * TEAMS);
+}
+template <int TG, int TEAMS>
+static int dw_launch(GemmArgs &g, hipStream_t s)
+{
+    if (g.nb % 2) return dw_launch_rows<TG, TEAMS, DW_ODD>(g, s);
+    return g.nb % GEMM8_KB ? dw_launch_rows<TG, TEAMS, DW_EVEN>(g, s) : dw_launch_rows<TG, TEAMS, DW_WHOLE>(g, s);
 }
 int gemm_q80_dw_launch(GemmArgs &g, hipStream_t s)
 {
+    if (g.nb % 2 && g.ext_part) {
+        /* what a size is answered does not hang on the form: refused where the split of 64-token tiles has no room */
+        const int steps = (g.nb + GEMM8_KB - 1) / GEMM8_KB, sp = gemm_choose_splits((g.M + 63) / 64 * g.nnt, steps), per = (steps + sp - 1) / sp, k = (steps + per - 1) / per;
+        if (k > 1 && (size_t)k * (size_t)g.M * (size_t)g.N * sizeof(float) > g.ext_part_bytes) return CKQ_ESCRATCH;
+    }
     switch (dw_form(g.M, g.nb, g.N, g.nnt, true)) {
     case 0: return dw_launch<1, 1>(g, s);
     case 1: return dw_launch<2, 1>(g, s);
@@ -370,7 +445,9 @@ template <int TG>
 static int dw_launch_group(GemmArgs &g, const GemmGroupIn &in, hipStream_t s)
 {
     g.ntt = (g.M + 32 * TG - 1) / (32 * TG);
-    return gemm_launch_grouped(gemm_q80_dw_kernel<TG, 1, false>, g, in, s, GEMM8_THREADS);
+    if (g.nb % 2) return gemm_launch_grouped(gemm_q80_dw_kernel<TG, 1, DW_ODD, false>, g, in, s, GEMM8_THREADS);
+    if (g.nb % GEMM8_KB) return gemm_launch_grouped(gemm_q80_dw_kernel<TG, 1, DW_EVEN, false>, g, in, s, GEMM8_THREADS);
+    return gemm_launch_grouped(gemm_q80_dw_kernel<TG, 1, DW_WHOLE, false>, g, in, s, GEMM8_THREADS);
 }
 int gemm_q80_dw_launch_group(GemmArgs &g, const GemmGroupIn &in, hipStream_t s)
 {

@@ -52,7 +52,7 @@ extern "C" void ckq_launch_set_gemm_policy(int policy) { g_gemm_policy.store(pol
  * 9-16 tokens stream, 17 and more go to the matrix cores; 4864x896 (4.6 MB) streams up to 72 tokens.  Rows on dwords run the
  * faster ckq_gemm_q80_dw.hip since, which is ahead earlier (two passes over large matrices: 16 tokens, 32000x4096 60 against 28; the
  * second kernel's 8 to 14 us for small ones), but the line also says which order of sums a size has, whether it may be split along K and
- * so needs scratch, and stays where it is at every K: the tile kernel's one chain of additions over a row is less exact than the streaming
+ * so needs scratch, and stays where it is at every K (rows of an odd number of blocks, which it serves too, included): the tile kernel's one chain of additions over a row is less exact than the streaming
  * kernel's terms per lane and tree (rms error of the rms result at K = 7296: 1.9e-7, with two teams 1.4e-7, against 0.8e-7). */
 static bool gemm_q80_on_matrix_cores(int ntok, size_t weight_bytes, bool aligned_rows)
 {

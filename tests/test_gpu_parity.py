@@ -2129,6 +2129,39 @@ def test_gemm_mfma_q8_0_tiles_and_teams(M, N, K):
     assert float(((y - A @ B.T).abs() / bound).max()) <= 1.0
 
 
+@pytest.mark.parametrize("M,N,K", [(9, 131, 32), (10, 1, 224), (33, 300, 96), (63, 1030, 2080), (129, 2050, 608), (192, 21001, 672), (350, 24484, 288), (385, 24499, 352),
+                                   (128, 8000, 1952), (130, 8001, 2016), (65, 12000, 2208), (70, 129, 9248)])
+def test_gemm_mfma_q8_0_rows_of_an_odd_number_of_blocks(M, N, K):
+    """Rows that start on dwords and two bytes behind them in turn, one block or three after the last whole step, in every form of the kernel and split
+    along K: against fp64 at the bound of the test above.  A scale that is infinite makes the outputs of its row what the oracle has."""
+    import torch
+    x, w = T.random_blocks("q8_0", M * (K // 32), 9850 + M), T.random_blocks("q8_0", N * (K // 32), 9851 + N)
+
+    def real(b, rows):
+        b = P.to_device(b).view(rows, K // 32, 34)
+        d = b[:, :, :2].contiguous().view(torch.float16).double()
+        return (d * b[:, :, 2:].contiguous().view(torch.int8).double()).reshape(rows, K)
+    say("q8_0, an odd number of blocks", M, N, K)
+    bias = P.to_device(T.normal(N, 0.0, 0.5, seed=N))
+    L = ckq.lib()
+    try:
+        L.ckq_set_gemm_policy(1)
+        y = P.dev_gemm_nt("q8_0", P.to_device(x), P.to_device(w), bias, M, N, K).view(M, N).double() - bias.double()
+        A, B = real(x, M), real(w, N)
+        bound = (A.abs() @ B.abs().T) * (K // 32 + 4) * 2.0 ** -24 + bias.abs().double() * 2.0 ** -23
+        assert bool((torch.isfinite(bound)).all())
+        assert float(((y - A @ B.T).abs() / bound).max()) <= 1.0
+        if M * N * K < 1 << 21:
+            rows = w.reshape(N, -1)
+            rows[N // 2, 34 * (K // 64):34 * (K // 64) + 2] = (0, 0x7C)
+            got = P.dev_gemm_nt("q8_0", P.to_device(x), P.to_device(w), None, M, N, K).cpu().numpy().reshape(M, N)
+            with np.errstate(all="ignore"):
+                want = T.oracle_gemm_nt("q8_0", x, w, None, M, N, K)
+            assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want)) and not np.isfinite(want[:, N // 2]).any()
+    finally:
+        L.ckq_set_gemm_policy(0)
+
+
 @pytest.mark.parametrize("fmt,M,D,N", [("q4_k", 1, 768, (768, 64, 64)), ("q5_k", 1, 1024, (1024, 128, 128)), ("q6_k", 1, 2048, (2048, 17)), ("q5_k", 2, 1280, (200, 130, 7, 64)),
                                        ("q4_k", 3, 1024, (1000, 128, 1)), ("q5_k", 4, 1024, (1024, 128, 128)), ("q6_k", 4, 1792, (31,)), ("q4_k", 5, 1024, (130, 130)),
                                        ("q5_k", 8, 768, (65, 3)), ("q4_k", 1, 512, (512,)), ("q6_k", 4, 256, (300, 9)), ("q4_k", 1, 2304, (300,)), ("q5_k", 1, 1024, (40000,))])
