@@ -15,11 +15,12 @@
  *   v = 256 * H + L (L = signed low byte of v, H = high byte of v + 128), the
  *   byte lanes of the products gathered with v_perm_b32; both planes are
  *   accumulated over the block, I1 = 256 * IH + IL.
- * - The min term is two more int8 MFMAs per 32x32 tile per block: the eight
- *   bsum pairs of a token, split the same way into low and high bytes, fill 16
- *   of the 32 k slots of the token operand (the other 16 are zero); the weight
- *   operand holds the eight 6-bit mins in the low or in the high slots, giving
- *   sum m * PL and sum m * PH; I2 = 256 * that + this.
+ * - The min term is one bf16 MFMA per 32x32 tile per block, as in the Q4_K kernel: the eight bsum pairs P of a token as P & 63 and P - (P & 63) fill the
+ *   sixteen k slots, the eight mins stand against both halves, and the sum leaves the matrix core as the fp32 number that is wanted, exactly.
+ *   The block's threads turn the stored bsums into that operand where they lie in LDS, a quarter of a token each.  Two int8 MFMAs of bytes of P, formed by every
+ *   wave for itself, and their integers shifted, added and converted were 646 vector instructions a 256-block and wave where this is 545 (matrix 36 -> 34).  What
+ *   bounds the kernel is their issue, least so with one wave per SIMD: us with the quantizer, tokens x rows x K, 512 x 11008 x 4096 92.1 -> 83.9, 2048 x 11008 x 4096 324 ->
+ *   298, 320 x 6784 x 4096 58.5 -> 53.0; up to one tile a CU 256 x 8192 x 4096 41.2 -> 39.0, 700 x 2048 x 6400 55.7 -> 54.0.
  * - Operands reach LDS by global->LDS loads only: a 176-byte block is eleven
  *   16-byte chunks; quants as in the Q4_K kernel (chunks XOR-swizzled by
  *   token); the tokens' block scales as 4-byte loads and their stored bsums as
@@ -30,6 +31,7 @@
  * Block = 4 waves = 64 tokens x 128 weight rows; wave w owns rows 32w..32w+31.
  */
 #include "ckq_gemm_rows16.hpp"
+#include "ckq_gemm_q4k.hpp"
 #include <atomic>
 #include <type_traits>
 
@@ -42,12 +44,31 @@ struct Gemm5Stage {
     float   d[GEMM5_BM];               /* block scale of each token */
 };
 
+/* The token operand of the min term in the place of the stored bsums: of a token's 32 bytes its eight bsum pairs P as P & 63 in the first half and as
+ * P - (P & 63) in the second, exact in bf16.  `quarter`: of the sixteen bsums. */
+__device__ __forceinline__ void gemm5_min_quarter(const int2 &d, u32 &lo, u32 &hi)
+{
+    const int p0 = (int)(int16_t)(d.x & 0xffff) + (d.x >> 16), p1 = (int)(int16_t)(d.y & 0xffff) + (d.y >> 16);
+    lo = bf16_pair((float)(p0 & 63), (float)(p1 & 63));
+    hi = bf16_pair((float)(p0 & ~63), (float)(p1 & ~63));
+}
+/* By the 256 threads of a block, four to a token, which are neighbours in a wave: all of a token is read before any of it is written. */
+__device__ __forceinline__ void gemm5_min_operand(uint8_t *bsum, int tid)
+{
+    uint8_t *const t = bsum + 32 * (tid >> 2);
+    const int qu = tid & 3;
+    u32 lo, hi;
+    gemm5_min_quarter(*reinterpret_cast<const int2 *>(t + 8 * qu), lo, hi);
+    *reinterpret_cast<u32 *>(t + 4 * qu) = lo;
+    *reinterpret_cast<u32 *>(t + 16 + 4 * qu) = hi;
+}
+
 /* One 256-block of a tile.  The planes of slab s+1 are expanded between the
  * MFMAs of slab s; copy_one(i) issues one global->LDS copy of a later block. */
-template <int NCOPY, bool DUMP, class CopyFn, class AfterFn>
+template <int NCOPY, bool DUMP, class CopyFn, class AfterFn, class MinsFn>
 __device__ __forceinline__ void gemm5_block(const uint8_t *w, const uint8_t *q, const uint8_t *bsum, const float *d, u32 wrow,
                                             const u32 (&aofs)[8], int col, int half, ckq_v16f (&acc)[2], CopyFn copy_one,
-                                            AfterFn after_weights, const GemmDumpLane &dl)
+                                            AfterFn after_weights, MinsFn mins_there, const GemmDumpLane &dl)
 {
 #define CKQ_PIN() __builtin_amdgcn_sched_barrier(0)
     auto lds16 = [&](const void *p) { return *reinterpret_cast<const ckq_v4i *>(p); };
@@ -67,17 +88,11 @@ __device__ __forceinline__ void gemm5_block(const uint8_t *w, const uint8_t *q, 
     };
     a_read(0);
 
-    /* token scales and stored bsums, read (through the integer vector type)
-     * before the first copy is issued */
+    /* token scales, read before the first copy is issued */
     float dx[2];      /* per token group: the block scale of the token of output (lane & 15) */
-    ckq_v4i bs[2][2];
     const int dx_tok = mfma32_row_of_lane(col + 32 * half);
 #pragma unroll
-    for (int ts = 0; ts < 2; ++ts) {
-        dx[ts] = __builtin_bit_cast(float, *reinterpret_cast<const int *>(&d[32 * ts + dx_tok]));
-        bs[ts][0] = lds16(&bsum[(col + 32 * ts) * 32]);
-        bs[ts][1] = lds16(&bsum[(col + 32 * ts) * 32 + 16]);
-    }
+    for (int ts = 0; ts < 2; ++ts) dx[ts] = __builtin_bit_cast(float, *reinterpret_cast<const int *>(&d[32 * ts + dx_tok]));
 
     const u32 h0 = (u32)hv[0], h1 = (u32)hv[1], h2 = (u32)hv[2], h3 = (u32)hv[3];
     const u32 sc03 = h1 & 0x3f3f3f3fu;
@@ -106,29 +121,22 @@ __device__ __forceinline__ void gemm5_block(const uint8_t *w, const uint8_t *q, 
         pH[s & 1][i] = (int)__builtin_amdgcn_perm(to, te, 0x07030501u);
     };
 
-    /* token operand of the min term: P_s = bsums[2s] + bsums[2s+1] (one dword
-     * holds the pair), t = P + 128; bytes [PL_0..7 | PH_0..7] for the lanes of
-     * k-half 0, zeros for k-half 1 */
-    auto min_operand = [&](int ts) {
-        u32 u[4];
+    /* weight operand of the min term: the eight mins, for either half of the token operand */
+    auto min_weights = [&]() {
+        ckq_v4i m;
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            const u32 d0 = (u32)bs[ts][p >> 1][2 * (p & 1)], d1 = (u32)bs[ts][p >> 1][2 * (p & 1) + 1];
-            const u32 t0 = d0 + (d0 >> 16) + 128u, t1 = d1 + (d1 >> 16) + 128u;   /* low 16 bits: P + 128 */
-            u[p] = __builtin_amdgcn_perm(t1, t0, 0x05040100u);                     /* [t0.lo16, t1.lo16] */
+        for (int i = 0; i < 4; ++i) {
+            const u32 src = i < 2 ? mn03 : mn47;
+            m[i] = (int)bf16_pair((float)((src >> (16 * (i & 1))) & 0xff), (float)((src >> (16 * (i & 1) + 8)) & 0xff));
         }
-        ckq_v4i a;
-        a[0] = (int)(__builtin_amdgcn_perm(u[1], u[0], 0x06040200u) ^ 0x80808080u);   /* PL_0..3 */
-        a[1] = (int)(__builtin_amdgcn_perm(u[3], u[2], 0x06040200u) ^ 0x80808080u);   /* PL_4..7 */
-        a[2] = (int)__builtin_amdgcn_perm(u[1], u[0], 0x07050301u);                   /* PH_0..3 */
-        a[3] = (int)__builtin_amdgcn_perm(u[3], u[2], 0x07050301u);                   /* PH_4..7 */
-        if (half) a = ckq_v4i{0, 0, 0, 0};
-        return a;
+        return __builtin_bit_cast(ckq_v8bf, m);
     };
 
-    ckq_v16i iL[2], iH[2], mL[2], mH[2];
+    ckq_v16i iL[2], iH[2];
+    ckq_v16f i2[2];
     const ckq_v16i zero16 = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    const ckq_v4i bM1 = {(int)mn03, (int)mn47, 0, 0}, bM2 = {0, 0, (int)mn03, (int)mn47};
+    const ckq_v16f zero16f = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    ckq_v8bf bm;
 
     prep(0);
 #pragma unroll
@@ -155,11 +163,11 @@ __device__ __forceinline__ void gemm5_block(const uint8_t *w, const uint8_t *q, 
             CKQ_PIN();
         }
         /* the min term rides along in slabs 5 and 6, one token group each */
+        if (s == 3) mins_there();
+        if (s == 4) bm = min_weights();
         if (s == 5 || s == 6) {
             const int ts = s - 5;
-            const ckq_v4i aP = min_operand(ts);
-            mL[ts] = __builtin_amdgcn_mfma_i32_32x32x32_i8(aP, bM1, zero16, 0, 0, 0);
-            mH[ts] = __builtin_amdgcn_mfma_i32_32x32x32_i8(aP, bM2, zero16, 0, 0, 0);
+            i2[ts] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(ckq_v8bf, lds16(&bsum[(col + 32 * ts) * 32 + 16 * half])), bm, zero16f, 0, 0, 0);
             CKQ_PIN();
         }
     }
@@ -168,14 +176,13 @@ __device__ __forceinline__ void gemm5_block(const uint8_t *w, const uint8_t *q, 
     for (int ts = 0; ts < 2; ++ts)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const int i1 = (iH[ts][r] << 8) + iL[ts][r], i2 = (mH[ts][r] << 8) + mL[ts][r];
-            const float f1 = (float)i1;
-            const float f2 = (float)i2;
+            const int i1 = (iH[ts][r] << 8) + iL[ts][r];
+            const float f1 = (float)i1, f2 = i2[ts][r];
             acc[ts][r] = fmac_row_lane(acc[ts][r], dx[ts], dw * f1 - dmin * f2, r);
             if constexpr (DUMP) {
                 const int tok = 32 * ts + 8 * (r >> 2) + (r & 3);
                 dl.put(tok, 0, i1);
-                dl.put(tok, 1, i2);
+                dl.put(tok, 1, (int)f2);
             }
         }
 #undef CKQ_PIN
@@ -286,7 +293,12 @@ __global__ void __launch_bounds__(256, 1) gemm_q5k_mfma_kernel(GemmArgs a)
             dl.tok_left = a.M - tf;
             dl.row_ok = n < work.N;
         }
-        gemm5_block<NCOPY, DUMP>(stage[cur].w, stage[cur].q, stage[cur].b, stage[cur].d, wrow, aofs, col, half, acc, copy_one, [] {}, dl);
+        gemm5_min_operand(stage[cur].b, tid);
+        auto mins_there = [] {
+            __builtin_amdgcn_s_waitcnt(0xc07f);      /* lgkmcnt(0) */
+            __builtin_amdgcn_s_barrier();
+        };
+        gemm5_block<NCOPY, DUMP>(stage[cur].w, stage[cur].q, stage[cur].b, stage[cur].d, wrow, aofs, col, half, acc, copy_one, [] {}, mins_there, dl);
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_waitcnt(0x0070 | (NCOPY & 15) | ((NCOPY >> 4) << 14));
         __builtin_amdgcn_s_barrier();
@@ -413,7 +425,8 @@ __global__ void __launch_bounds__(256, 2) gemm_q5k_pair_kernel(GemmArgs a)
         };
         auto copy_next = [&](int i) __attribute__((always_inline)) { copy_one(i, std::integral_constant<int, cur ^ 1>{}); };
         __builtin_amdgcn_sched_barrier(0);
-        gemm5_block<NCOPY, DUMP>(wimg, qst(curc), bst(curc), dst(curc), wrow, aofs, col, half, acc, copy_next, after_weights, dl);
+        gemm5_min_operand(bst(curc), tid);           /* there for all behind after_weights' barrier */
+        gemm5_block<NCOPY, DUMP>(wimg, qst(curc), bst(curc), dst(curc), wrow, aofs, col, half, acc, copy_next, after_weights, [] {}, dl);
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_waitcnt(0x0070);
         __builtin_amdgcn_s_barrier();
@@ -498,14 +511,28 @@ __global__ void __launch_bounds__(64 * SPLITS, 1) gemm_q5k_ksplit_kernel(GemmArg
     auto kstep = [&](int b, auto curc) __attribute__((always_inline)) {
         constexpr int cur = decltype(curc)::value;
         const int bn = min(b + 1, last);
+        {
+            uint8_t *const t = bs[wave] + 32 * lane;
+            const ckq_v4i b0 = *reinterpret_cast<const ckq_v4i *>(t), b1 = *reinterpret_cast<const ckq_v4i *>(t + 16);
+            ckq_v4i lo, hi;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                u32 l, h;
+                gemm5_min_quarter(k < 2 ? int2{b0[2 * k], b0[2 * k + 1]} : int2{b1[2 * k - 4], b1[2 * k - 3]}, l, h);
+                lo[k] = (int)l;
+                hi[k] = (int)h;
+            }
+            *reinterpret_cast<ckq_v4i *>(t) = lo;
+            *reinterpret_cast<ckq_v4i *>(t + 16) = hi;
+        }
         gemm5_block<16, false>(ws[wave], xs[wave][cur], bs[wave], ds[wave], (u32)(col * GEMM5_ROW), aofs, col, half, acc, [&](int i) __attribute__((always_inline)) {
             const int slot = 2 * (i & 7) + (i >> 3);          /* in time: i and i + 8 are the two of a slab */
             if (slot < 9) { copy(bn, cur ^ 1, 2 * slot); copy(bn, cur ^ 1, 2 * slot + 1); }
             else copy(bn, cur ^ 1, 9 + slot);
         }, []() __attribute__((always_inline)) {
-            __builtin_amdgcn_s_waitcnt(0xc07f);    /* lgkmcnt(0): rows, bsums and scales are in registers */
+            __builtin_amdgcn_s_waitcnt(0xc07f);    /* lgkmcnt(0): rows and scales are in registers; the next block's bsums (copies 22 and 23) come in slots 13 and 14, slabs 6 and 7, behind the reads of these */
             asm volatile("" ::: "memory");
-        }, GemmDumpLane{});
+        }, [] {}, GemmDumpLane{});
         __builtin_amdgcn_sched_barrier(0);
         landed();
     };
