@@ -344,7 +344,10 @@ static float keep_time_own_scratch(int f, size_t rows, int ntok)
     }
     return least < 4.4f + 1e-3f * (f == 1 ? 4.98f : 5.82f) * (float)(tiles * groups) ? least : 0.0f;
 }
-static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles, int launches = 1, bool own_scratch = false)
+static float rows16_q4k_time(float nb, size_t rows, int ntok) { return 3.6f + 0.12f * nb + 0.58e-3f * nb * (float)((rows + 15) / 16) * (float)((ntok + 15) / 16); }
+/* A Q4_K matrix of fewer than 160 tiles on its own: split along K or not, or by the 16-row kernel. */
+static float single_q4k_time(float nb, size_t rows, int ntok) { return fminf(nb < 8.0f ? 5.5f + 1.2f * nb : 7.2f + 0.22f * nb + 0.22f * 144e-6f * nb * (float)rows, rows16_q4k_time(nb, rows, ntok)); }
+static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles, int launches = 1, bool own_scratch = false, size_t shared_tiles = 0, float t_singles = 0.0f)
 {
     if (ntok < 2 || K > ROWS16_MAX_K) return false;
     if (g_rows16_forced.load(std::memory_order_relaxed) >> fmt & 1) return true;
@@ -379,6 +382,16 @@ static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles, int l
         const float on_cu = (float)((rows + 127) / 128) * (float)((ntok + 63) / 64) / 256.0f;
         return keep[f][0] + (keep[f][1] + (nb == 3.0f ? keep[f][3] : 0.0f)) * t_keep + keep[f][2] * out <
                tile[f][0] + (tile[f][1] + tile[f][2] * ceilf(on_cu) + tile[f][3] * fmaxf(on_cu, 1.0f)) * nb + tile[f][4] * out;
+    }
+    /* Q4_K, several groups, against ONE launch of unsplit tiles (a single matrix of 160 tiles and more, or several of so many together): the 16-row kernel takes
+     * 0.58 ns a 256-block of 16 rows and 16 tokens there, its blocks all over each other, and not the 0.36 of a few blocks a CU, and the tiles' time goes by rounds of their blocks. 60 launches of
+     * 17 to 300 tokens, rows of 5 to 16 blocks, us, 16-row kernel | tiles: 65 x 2 x 6912 x 1536 19.0 | 14.3, 133 x 2 x 3840 x 1280 17.9 | 12.6, 32 x 2 x 11008 x 3840 28.2 | 22.1,
+     * 257 x 2 x 3584 x 768 16.5 | 11.0; and 32 x 2 x 10240 x 1280 stays (11.6 | 13.0). Where several matrices are fewer tiles than that they go out one by one, and the estimates of those add up:
+     * 98 x (2816, 1408, 1408) x 2816 27.5 one by one, 20.1 together. */
+    const size_t unsplit = launches == 1 ? (rows + 127) / 128 * (size_t)((ntok + 63) / 64) : shared_tiles;
+    if (f == 0 && tiles && !own_scratch && ntok > 16 && t_keep <= 0.0f && t_pair <= 0.0f && (unsplit >= 160 || (launches > 1 && unsplit == 0))) {
+        const float t_tiles = !unsplit ? t_singles : unsplit <= 256 ? (nb < 8.0f ? 6.2f + 1.35f * nb : 8.5f + 0.95f * nb) : unsplit <= 512 ? 6.1f + 2.2f * nb : unsplit <= 768 ? 9.2f + 3.3f * nb : 11.0f + 4.6f * nb;
+        return rows16_q4k_time(nb, rows, ntok) < t_tiles;
     }
     if (tiles) t_else = f == 0 || t_pair <= 0.0f ? 11.0f + (0.2f + 0.0015f * (float)ntok) * mb : f == 1 ? 13.3f + (0.164f + 0.0048f * (float)ntok) * mb : 13.8f + (0.083f + 0.0044f * (float)ntok) * mb;
     else if (ntok <= 8) t_else = fmaxf(3.5f + 0.07f * nb, 3.05f + 0.11f * nb + 1.25f * per_pass[f] * mb);
@@ -706,7 +719,9 @@ extern "C" int ckq_launch_gemm_group(int fmt, int n, float *const *C, const void
             tiles[p] = grouped || kquant_on_matrix_cores(fmt, M, (size_t)N[p], K);
             alike = alike && tiles[p] == tiles[0];
         }
-        if (alike && take_rows16(fmt, M, rows, K, tiles[0], n)) {
+        float t_singles = 0.0f;
+        for (int p = 0; p < n; ++p) t_singles += single_q4k_time((float)(K / 256), (size_t)N[p], M);
+        if (alike && take_rows16(fmt, M, rows, K, tiles[0], n, false, grouped ? (size_t)gemm_group_tiles(in, M, 64) : 0, t_singles)) {
             Rows16Args r = {};
             r.M = M; r.nb = K / 256; r.n = n; r.tree = !tiles[0];
             for (int p = 0; p < n; ++p)

@@ -244,6 +244,13 @@ def test_ragged_token_tiles_dealt_last(L, M, Ns, last):
         assert max(per_xcd) - min(per_xcd) <= 2 * len(Ns)
 
 
+@pytest.mark.parametrize("n,k,tokens,want", [(11000, 1280, 65, TILES), (20480, 1280, 32, ROWS16_TILES), (20480, 1280, 48, TILES), (13824, 1536, 65, TILES), (7680, 1280, 133, TILES),
+                                             (22016, 2816, 24, TILES), (32000, 2048, 40, TILES), (25000, 1536, 20, TILES), (28000, 768, 100, TILES), (8192, 4096, 16, ROWS16_TILES)])
+def test_q4_k_unsplit_tiles_or_16_row_tiles(L, n, k, tokens, want):
+    """160 tiles of 64 tokens and more: sizes at which both kernels were timed, the faster one (within 4 %) is taken; one token group keeps its own rule."""
+    assert route(L, "q4_k", n, k, tokens) == want
+
+
 def test_q8_0_order_of_sums_does_not_hang_on_the_width(L):
     """Long rows on dwords stream where shorter rows of as many bytes do, up to 16 tokens always: the tile kernel's chains of additions are longer, and
     it may need scratch for a split along K.  Host arithmetic of the same line."""
