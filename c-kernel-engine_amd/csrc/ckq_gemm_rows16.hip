@@ -11,7 +11,7 @@
  * v_mfma_i32_16x16x64_i8: A = 16 tokens x 64 k, B = 64 k x 16 weight rows, D = 16 x 16 int32.  Lane l = 16 q + i holds
  * token / row i and the 16 k of quarter q; of D it holds row i and tokens 4 q .. 4 q + 3.  The 64 k of an instruction are
  * those a lane of the streaming kernel takes, ordered so that a lane's sixteen are one 16-byte run of the raw block's
- * quants (low or high nibbles) inside one scale; the activations are read in the same order.  The planes are those of the tile kernels: Q4_K (sc >> 3) q and
+ * quants (low or high nibbles) inside one scale; the activations are read in the same order.  Where several groups of tokens share them, the planes are those of the tile kernels: Q4_K (sc >> 3) q and
  * (sc & 7) q, Q5_K / Q6_K the two bytes of the 16-bit product, each summed over the 256-block; the min term of Q4_K / Q5_K is
  * a bf16 MFMA of the mins and the bsum pairs split in two (ckq_gemm_q4k.hip).  All integers are exact.
  *
@@ -70,6 +70,24 @@ __device__ __forceinline__ void byte_planes(u32 v, u32 sc2, u32 add2, int &lo, i
 
 __device__ __forceinline__ ckq_v4i lds16(const uint8_t *p) { return *reinterpret_cast<const ckq_v4i *>(p); }
 
+/* One group of tokens: the quants as they are against one 32-run (slab) of the block at a time (v_mfma_i32_16x16x32_i8; lane quarter q has elements 32 s + 8 q ..
+ * + 7 of slab s), the integers of a slab then times its scale, which a lane has for its row: four multiply-adds where forming planes and putting their sums
+ * together costs more than the matrix instructions it saves (vector instructions of a 256-block in the first kernel, planes -> slabs: Q4_K 129 -> 121, in the streaming
+ * kernel's order 215 -> 185, Q5_K 247 -> 151 and 333 -> 215, Q6_K 236 -> 207; us, weights from the cache, tokens x rows x K: Q5_K 13 x 6144 x 4096 10.8 -> 9.3, 8 x 11008 x 4096 13.4 ->
+ * 11.2, 6 x 4096 x 11008 12.5 -> 10.2; Q4_K 8 x 11008 x 4096 10.7 -> 10.1; Q6_K 13 x 4096 x 11008 13.9 -> 13.4, 16 x 3584 x 9728 13.2 -> 12.7).  Q6_K has a scale every 16: a second product with the first half of the tokens' run alone, times the
+ * difference of the two scales.  raw(): the operands of SLABS slabs of the row at r, Q6_K 4 (q - 32); scales(): sc[s], or of Q6_K sc[2 s + half]. */
+__device__ __forceinline__ long two_dwords(u32 lo, u32 hi) { return (long)((uint64_t)lo | ((uint64_t)hi << 32)); }
+__device__ __forceinline__ void scales_k45(int (&sc)[16], const uint8_t *r)
+{
+    const ckq_v4i hv = *reinterpret_cast<const ckq_v4i *>(r);
+    const u32 h1 = (u32)hv[1], h3 = (u32)hv[3], lo = h1 & 0x3f3f3f3fu, hi = (h3 & 0x0f0f0f0fu) | ((h1 >> 2) & 0x30303030u);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        sc[k] = (int)((lo >> (8 * k)) & 0xffu);
+        sc[4 + k] = (int)((hi >> (8 * k)) & 0xffu);
+    }
+}
+
 /* Formats.  Position g of a 256-block: the 64 elements of one instruction, of which lane quarter q supplies the sixteen
  * from a_elem(g, q).  planes() forms them from the raw block of the lane's row at r (in LDS). */
 struct R16Q4K {
@@ -89,6 +107,14 @@ struct R16Q4K {
             h[i] = mul_bytes(n, mh);
             l[i] = mul_bytes(n, ml);
         }
+    }
+    static __device__ __forceinline__ void scales(int (&sc)[16], const uint8_t *r) { scales_k45(sc, r); }
+    static constexpr int SLABS = 2;
+    static __device__ __forceinline__ void raw(long (&b)[2], const uint8_t *r, int g, int q)
+    {
+        const uint2 v = *reinterpret_cast<const uint2 *>(r + 16 + 32 * g + 8 * q);
+        b[0] = two_dwords(v.x & 0x0f0f0f0fu, v.y & 0x0f0f0f0fu);
+        b[1] = two_dwords((v.x >> 4) & 0x0f0f0f0fu, (v.y >> 4) & 0x0f0f0f0fu);
     }
 };
 
@@ -110,6 +136,17 @@ struct R16Q5K {
             byte_planes(n | (hb << 4), sc2, 0x00800080u, lo, hi);
             h[i] = hi;
             l[i] = lo;
+        }
+    }
+    static __device__ __forceinline__ void scales(int (&sc)[16], const uint8_t *r) { scales_k45(sc, r); }
+    static constexpr int SLABS = 2;
+    static __device__ __forceinline__ void raw(long (&b)[2], const uint8_t *r, int g, int q)
+    {
+        const uint2 f = *reinterpret_cast<const uint2 *>(r + 16 + 8 * q), v = *reinterpret_cast<const uint2 *>(r + 48 + 32 * g + 8 * q);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            auto five = [&](u32 n, u32 h) { return ((n >> (4 * k)) & 0x0f0f0f0fu) | (((h >> (2 * g + k)) & 0x01010101u) << 4); };
+            b[k] = two_dwords(five(v.x, f.x), five(v.y, f.y));
         }
     }
 };
@@ -145,7 +182,43 @@ struct R16Q6K {
             l[i] = lo;
         }
     }
+    static __device__ __forceinline__ void scales(int (&sc)[16], const uint8_t *r)
+    {
+        const ckq_v4i v = lds16(r + 192);
+#pragma unroll
+        for (int k = 0; k < 16; ++k) sc[k] = __builtin_amdgcn_sbfe(v[k >> 2], 8 * (k & 3), 8);
+    }
+    static constexpr int SLABS = 4;
+    static __device__ __forceinline__ void raw(long (&b)[4], const uint8_t *r, int n, int q)
+    {
+        const uint2 l0 = *reinterpret_cast<const uint2 *>(r + 64 * n + 8 * q), l1 = *reinterpret_cast<const uint2 *>(r + 64 * n + 32 + 8 * q);
+        const uint2 h = *reinterpret_cast<const uint2 *>(r + 128 + 32 * n + 8 * q);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const uint2 l = t & 1 ? l1 : l0;
+            /* 6-bit q in the upper bits of its byte, the top one turned: 4 (q - 32) */
+            auto six = [&](u32 n4, u32 n2) {
+                return ((t < 2 ? n4 << 2 : n4 >> 2) & 0x3c3c3c3cu) | (((n2 << (6 - 2 * t)) & 0xc0c0c0c0u) ^ 0x80808080u);
+            };
+            b[t] = two_dwords(six(l.x, h.x), six(l.y, h.y));
+        }
+    }
 };
+/* The sums of slab s: of the whole of it, and for Q6_K of its first half too; `I` += them times their scales. */
+template <class F>
+__device__ __forceinline__ void slab_sums(int (&I)[4], int s, long a, long ah, long b, const int (&sc)[16])
+{
+    const ckq_v4i zero = {0, 0, 0, 0};
+    const ckq_v4i S = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b, zero, 0, 0, 0);
+    if constexpr (F::MIN) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) I[r] += __mul24(S[r], sc[s]);
+    } else {
+        const ckq_v4i H = __builtin_amdgcn_mfma_i32_16x16x32_i8(ah, b, zero, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) I[r] += __mul24(S[r], sc[2 * s + 1]) + __mul24(H[r], sc[2 * s] - sc[2 * s + 1]);
+    }
+}
 
 /* Shape of a launch: what a block needs besides its problem. */
 struct Rows16Shape { int M, nb; };
@@ -206,11 +279,15 @@ gemm_rows16_kernel(const uint8_t *W, const uint8_t *X, int N, Rows16Shape S, flo
         asrc[j] = (u32)min(t, M - 1 - t0) * xrow + 4u + 16u * (u32)c;
         adst[j] = (u32)(c < 16 ? 256 * t + 16 * (c ^ (t & 15)) : NT * 256 + 32 * t + 16 * (c - 16));
     }
-    u32 aofs[4];
     constexpr int QL = NT / 4;                       /* quarters of the result that hold tokens */
     const int ta = i16 & (NT - 1);
-#pragma unroll
-    for (int m = 0; m < 4; ++m) aofs[m] = (u32)(256 * ta + 16 * ((int)(F::a_elem(m, q) >> 4) ^ ta));
+    const u32 abase = (u32)(256 * ta + 8 * (q & 1)), aslot = 16u * (u32)((q >> 1) ^ ta);        /* slab s: 16-byte chunk 2 s + q / 2 of the token, in slot (its number) ^ ta */
+    const u32 first = q < 2 ? ~0u : 0u;
+    auto slab_a = [&](int s, long &a, long &ah) {
+        const uint2 v = *reinterpret_cast<const uint2 *>(al + abase + (aslot ^ (32u * (u32)s)));
+        a = two_dwords(v.x, v.y);
+        ah = two_dwords(v.x & first, v.y & first);
+    };
 
     ckq_v4i wr[NWL], ar[NAL];
     auto fetch = [&](int b) {
@@ -258,26 +335,30 @@ gemm_rows16_kernel(const uint8_t *W, const uint8_t *X, int N, Rows16Shape S, flo
     auto block_term = [&](int b) {
         Head hd;
         F::head(hd, wrow, q);
-        ckq_v4i sh, sl;
+        int sc[16], I[4] = {0, 0, 0, 0};
+        F::scales(sc, wrow);
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            ckq_v4i ph, pl;
-            F::planes(ph, pl, hd, wrow, g, q);
-            const ckq_v4i a = lds16(al + aofs[g]);
-            sh = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, ph, g ? sh : zero, 0, 0, 0);
-            sl = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, pl, g ? sl : zero, 0, 0, 0);
+        for (int k = 0; k < 8 / F::SLABS; ++k) {
+            long w[F::SLABS];
+            F::raw(w, wrow, k, q);
+#pragma unroll
+            for (int j = 0; j < F::SLABS; ++j) {
+                long a, ah;
+                slab_a(F::SLABS * k + j, a, ah);
+                slab_sums<F>(I, F::SLABS * k + j, a, ah, w[j], sc);
+            }
         }
         float out[4];
         if constexpr (F::MIN) {
             const ckq_v4f i2 = min_mfma(bsum_operand(), hd.mins);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float f = (float)((sh[r] << F::SHIFT) + sl[r]);
+                const float f = (float)I[r];
                 out[r] = hd.dw * f - hd.dmin * i2[r];
             }
         } else {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) out[r] = hd.dw * (float)((sh[r] << F::SHIFT) + sl[r]);
+            for (int r = 0; r < 4; ++r) out[r] = hd.dw * (float)(I[r] >> 2);
         }
         put(b, out);
     };
@@ -289,24 +370,57 @@ gemm_rows16_kernel(const uint8_t *W, const uint8_t *X, int N, Rows16Shape S, flo
         const ckq_v4i dxi = lds16(reinterpret_cast<const uint8_t *>(dxs + b * NT + 4 * (q & (QL - 1))));
         ckq_v4i am;
         if (F::MIN) am = bsum_operand();
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            ckq_v4i ph, pl;
-            F::planes(ph, pl, hd, wrow, g, q);
-            const ckq_v4i a = lds16(al + aofs[g]);
-            const ckq_v4i sh = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, ph, zero, 0, 0, 0);
-            const ckq_v4i sl = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, pl, zero, 0, 0, 0);
+        int sc[16];
+        F::scales(sc, wrow);
+        auto term = [&](int g, const int (&I)[4]) {
             ckq_v4f i2;
             if constexpr (F::MIN) i2 = min_mfma(am, q == g ? hd.mins : zero);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int di = dxi[r];
-                const float dx = __builtin_bit_cast(float, di), f = (float)((sh[r] << F::SHIFT) + sl[r]);
+                const float dx = __builtin_bit_cast(float, di), f = (float)(F::MIN ? I[r] : I[r] >> 2);
                 float v;
                 if constexpr (F::MIN) v = (hd.dw * dx) * f - (hd.dmin * dx) * i2[r];
                 else                  v = (hd.dw * dx) * f;
                 asm volatile("" : "+v"(v));                  /* rounded before it is added, as there */
                 acc[g][r] += v;
+            }
+        };
+        if constexpr (F::MIN) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {                    /* slabs 2 g and 2 g + 1 */
+                int I[4] = {0, 0, 0, 0};
+                long w[F::SLABS];
+                F::raw(w, wrow, g, q);
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    long a, ah;
+                    slab_a(2 * g + j, a, ah);
+                    slab_sums<F>(I, 2 * g + j, a, ah, w[j], sc);
+                }
+                term(g, I);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+#pragma unroll
+            for (int n = 0; n < 2; ++n) {                    /* position 2 n + odd: the halves `odd` of slabs 4 n .. 4 n + 3 */
+                int even[4] = {0, 0, 0, 0}, odd[4] = {0, 0, 0, 0};
+                long w[F::SLABS];
+                F::raw(w, wrow, n, q);
+#pragma unroll
+                for (int s = 4 * n; s < 4 * n + 4; ++s) {
+                    long a, ah;
+                    slab_a(s, a, ah);
+                    const ckq_v4i S = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, w[s & 3], zero, 0, 0, 0), H = __builtin_amdgcn_mfma_i32_16x16x32_i8(ah, w[s & 3], zero, 0, 0, 0);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        even[r] += __mul24(H[r], sc[2 * s]);
+                        odd[r] += __mul24(S[r] - H[r], sc[2 * s + 1]);
+                    }
+                }
+                term(2 * n, even);
+                term(2 * n + 1, odd);
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
     };
