@@ -19,7 +19,7 @@
  * would otherwise run on: the streaming kernel's term per 64 elements and tree (TREE), or the tile kernels' term per
  * 256-block and chains (GemmChains).  The terms meet in LDS; one thread per output adds them.
  *
- * Bound: VALU issue (150-300 operations per 256-block of 16 rows) next to HBM and, for small matrices, one latency after
+ * Bound: VALU issue (110-260 operations per 256-block of 16 rows) next to HBM and, for small matrices, one latency after
  * another.  Measured, weights from HBM, against the kernel that served the shape before (us): Q4_K 4096 x 4096 at 8 / 13 / 32
  * tokens 7.5 -> 6.1, 10.0 -> 6.5, 13.1 -> 8.1; 11008 x 4096 at 8 / 13: 14.7 -> 10.3, 15.6 -> 9.7; Q6_K 32000 x 4096 at
  * 8 / 13: 40.6 -> 27.1, 46.2 -> 28.3; 4096 x 11008 at 13: 20.7 -> 15.8; Q5_K 1024 x 4864 at 64: 16.8 -> 8.0.
@@ -72,9 +72,9 @@ __device__ __forceinline__ ckq_v4i lds16(const uint8_t *p) { return *reinterpret
 
 /* One group of tokens: the quants as they are against one 32-run (slab) of the block at a time (v_mfma_i32_16x16x32_i8; lane quarter q has elements 32 s + 8 q ..
  * + 7 of slab s), the integers of a slab then times its scale, which a lane has for its row: four multiply-adds where forming planes and putting their sums
- * together costs more than the matrix instructions it saves (vector instructions of a 256-block in the first kernel, planes -> slabs: Q4_K 129 -> 121, in the streaming
- * kernel's order 215 -> 185, Q5_K 247 -> 151 and 333 -> 215, Q6_K 236 -> 207; us, weights from the cache, tokens x rows x K: Q5_K 13 x 6144 x 4096 10.8 -> 9.3, 8 x 11008 x 4096 13.4 ->
- * 11.2, 6 x 4096 x 11008 12.5 -> 10.2; Q4_K 8 x 11008 x 4096 10.7 -> 10.1; Q6_K 13 x 4096 x 11008 13.9 -> 13.4, 16 x 3584 x 9728 13.2 -> 12.7).  Q6_K has a scale every 16: a second product with the first half of the tokens' run alone, times the
+ * together costs more than the matrix instructions it saves (vector instructions of a 256-block in the first kernel, planes -> slabs: Q4_K 129 -> 110, in the streaming
+ * kernel's order 215 -> 184, Q5_K 247 -> 140 and 333 -> 214, Q6_K 236 -> 186 and 292 -> 256; us, weights from the cache, tokens x rows x K: Q5_K 13 x 6144 x 4096 10.8 -> 9.3, 8 x 11008 x 4096 13.4 ->
+ * 11.1, 6 x 4096 x 11008 12.5 -> 10.1; Q4_K 8 x 11008 x 4096 10.8 -> 10.2, 13 x 4096 x 11008 11.8 -> 11.4; Q6_K 13 x 4096 x 11008 14.0 -> 13.3, 16 x 3584 x 9728 13.2 -> 12.8).  Q6_K has a scale every 16: a second product with the first half of the tokens' run alone, times the
  * difference of the two scales.  raw(): the operands of SLABS slabs of the row at r, Q6_K 4 (q - 32); scales(): sc[s], or of Q6_K sc[2 s + half]. */
 __device__ __forceinline__ long two_dwords(u32 lo, u32 hi) { return (long)((uint64_t)lo | ((uint64_t)hi << 32)); }
 __device__ __forceinline__ void scales_k45(int (&sc)[16], const uint8_t *r)
@@ -212,11 +212,31 @@ __device__ __forceinline__ void slab_sums(int (&I)[4], int s, long a, long ah, l
     const ckq_v4i S = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b, zero, 0, 0, 0);
     if constexpr (F::MIN) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) I[r] += __mul24(S[r], sc[s]);
+        for (int r = 0; r < 4; ++r) {
+            I[r] += __mul24(S[r], sc[s]);
+            asm("" : "+v"(I[r]));               /* one multiply-add, not two products and an addition of three */
+        }
     } else {
         const ckq_v4i H = __builtin_amdgcn_mfma_i32_16x16x32_i8(ah, b, zero, 0, 0, 0);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) I[r] += __mul24(S[r], sc[2 * s + 1]) + __mul24(H[r], sc[2 * s] - sc[2 * s + 1]);
+        for (int r = 0; r < 4; ++r) {
+            I[r] += __mul24(S[r], sc[2 * s + 1]);
+            asm("" : "+v"(I[r]));
+            I[r] += __mul24(H[r], sc[2 * s] - sc[2 * s + 1]);
+            asm("" : "+v"(I[r]));
+        }
+    }
+}
+/* Q6_K, the two halves of slab s apart: ah, ao are the tokens' with the other half zero. */
+__device__ __forceinline__ void slab_halves(int (&even)[4], int (&odd)[4], int s, long ah, long ao, long b, const int (&sc)[16])
+{
+    const ckq_v4i zero = {0, 0, 0, 0};
+    const ckq_v4i H = __builtin_amdgcn_mfma_i32_16x16x32_i8(ah, b, zero, 0, 0, 0), O = __builtin_amdgcn_mfma_i32_16x16x32_i8(ao, b, zero, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        even[r] += __mul24(H[r], sc[2 * s]);
+        odd[r] += __mul24(O[r], sc[2 * s + 1]);
+        asm("" : "+v"(even[r]), "+v"(odd[r]));
     }
 }
 
@@ -411,12 +431,7 @@ gemm_rows16_kernel(const uint8_t *W, const uint8_t *X, int N, Rows16Shape S, flo
                 for (int s = 4 * n; s < 4 * n + 4; ++s) {
                     long a, ah;
                     slab_a(s, a, ah);
-                    const ckq_v4i S = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, w[s & 3], zero, 0, 0, 0), H = __builtin_amdgcn_mfma_i32_16x16x32_i8(ah, w[s & 3], zero, 0, 0, 0);
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        even[r] += __mul24(H[r], sc[2 * s]);
-                        odd[r] += __mul24(S[r] - H[r], sc[2 * s + 1]);
-                    }
+                    slab_halves(even, odd, s, ah, two_dwords((u32)a & ~first, (u32)((uint64_t)a >> 32) & ~first), w[s & 3], sc);
                 }
                 term(2 * n, even);
                 term(2 * n + 1, odd);
@@ -524,6 +539,8 @@ gemm_rows16_kernel(const uint8_t *W, const uint8_t *X, int N, Rows16Shape S, flo
  * Bound: HBM, and the vector operations of all waves at once when a tile arrives (11008 x 4096 twice, Q4_K: loads alone 10.2 us,
  * with the terms 14, with the sums and stores 16.8).  Against the kernel above, 13 tokens, weights from HBM (us): Q4_K 2 x 11008 x 4096
  * 20.5 -> 16.8, Q6_K 32000 x 4096 35.4 -> 29.2, Q5_K 2 x 11008 x 4096 23.5 -> 21.5, 151936 x 1024 39 -> 31.
+ * Since then, slabs instead of planes (vector instructions a 256-block: Q4_K 126 -> 106, Q5_K 236 -> 128, Q6_K 241 -> 191), weights from the cache: 14.1 -> 13.8, 30.8 -> 29.6 (30000 x 3072 at
+ * 16 tokens 24.8 -> 23.2), 19.4 -> 16.0, 34.1 -> 30.3.
  * A wave with a whole chain of blocks to itself, activations in LDS, was as fast on the first two (16.7, 29.2) and 26 on the third;
  * two blocks a wave (eight waves, two such blocks a CU) 20.5, 36.2 and 25.6. */
 constexpr int HOLD_NB = 16;
@@ -581,13 +598,13 @@ gemm_rows16_hold_kernel(const uint8_t *W, const uint8_t *X, int N, int M, int nb
         }
     };
     const u32 xlane = (u32)min(i16, M - 1) * xrow;
-    auto fetch_a = [&](ckq_v4i (&v4)[4], int2 &bs) {
+    auto fetch_a = [&](long (&a8)[8], int2 &bs) {
         const uint8_t *xb = X + (u32)wave * 292u;
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            u32 v[4];
-            ld16<4>(v, xb + 4 + F::a_elem(g, 0) + (xlane + F::a_elem(0, q)));
-            v4[g] = ckq_v4i{(int)v[0], (int)v[1], (int)v[2], (int)v[3]};
+        for (int s = 0; s < 8; ++s) {
+            u32 v[2];
+            ld8<4>(v, xb + 4 + 32 * s + (xlane + 8u * (u32)q));
+            a8[s] = two_dwords(v[0], v[1]);
         }
         if constexpr (F::MIN) {
             u32 v[2];
@@ -605,62 +622,83 @@ gemm_rows16_hold_kernel(const uint8_t *W, const uint8_t *X, int N, int M, int nb
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(ckq_v8bf, a), __builtin_bit_cast(ckq_v8bf, mins), z, 0, 0, 0);
     };
     const ckq_v4i zero = {0, 0, 0, 0};
-    ckq_v4i a[4];                                  /* the activations of this wave's block, in the order of the instruction */
+    long a[8];                                     /* the activations of this wave's block, in the order of the instruction */
+    const u32 first_half = q < 2 ? ~0u : 0u;
     int2 am = {};
     /* the terms of the block whose weights lie in wl */
     auto terms = [&](float *u) {
         Head hd;
         F::head(hd, wrow, q);
+        u32 first = first_half;
+        if (!F::MIN) asm volatile("" : "+v"(first));             /* Q6_K: the first halves of the slabs are formed for every tile; kept like the whole ones, they would spill */
+        int sc[16];
+        F::scales(sc, wrow);
         float out[4];
         if constexpr (TREE) {
             const ckq_v4i dxi = lds16(reinterpret_cast<const uint8_t *>(dxs + wave * NT + 4 * q));
             float acc[4][4];
-#pragma unroll
-            for (int g = 0; g < 4; ++g)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) acc[g][r] = 0.0f;
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                ckq_v4i ph, pl;
-                F::planes(ph, pl, hd, wrow, g, q);
-                const ckq_v4i sh = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[g], ph, zero, 0, 0, 0);
-                const ckq_v4i sl = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[g], pl, zero, 0, 0, 0);
+            auto term = [&](int g, const int (&I)[4]) {
                 ckq_v4f i2;
                 if constexpr (F::MIN) i2 = min_mfma(am, q == g ? hd.mins : zero);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int di = dxi[r];
-                    const float dx = __builtin_bit_cast(float, di), f = (float)((sh[r] << F::SHIFT) + sl[r]);
+                    const float dx = __builtin_bit_cast(float, di), f = (float)(F::MIN ? I[r] : I[r] >> 2);
                     float v;
                     if constexpr (F::MIN) v = (hd.dw * dx) * f - (hd.dmin * dx) * i2[r];
                     else                  v = (hd.dw * dx) * f;
                     asm volatile("" : "+v"(v));                  /* rounded before it is added, as there */
-                    acc[g][r] += v;
+                    acc[g][r] = 0.0f + v;
                 }
                 __builtin_amdgcn_sched_barrier(0);
+            };
+            if constexpr (F::MIN) {
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    int I[4] = {0, 0, 0, 0};
+                    long w[F::SLABS];
+                    F::raw(w, wrow, g, q);
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) slab_sums<F>(I, 2 * g + j, a[2 * g + j], 0, w[j], sc);
+                    term(g, I);
+                }
+            } else {
+#pragma unroll
+                for (int n = 0; n < 2; ++n) {
+                    int even[4] = {0, 0, 0, 0}, odd[4] = {0, 0, 0, 0};
+                    long w[F::SLABS];
+                    F::raw(w, wrow, n, q);
+#pragma unroll
+                    for (int s = 4 * n; s < 4 * n + 4; ++s) slab_halves(even, odd, s, two_dwords((u32)a[s] & first, (u32)((uint64_t)a[s] >> 32) & first), two_dwords((u32)a[s] & ~first, (u32)((uint64_t)a[s] >> 32) & ~first), w[s & 3], sc);
+                    term(2 * n, even);
+                    term(2 * n + 1, odd);
+                }
             }
 #pragma unroll
             for (int r = 0; r < 4; ++r) out[r] = (acc[0][r] + acc[1][r]) + (acc[2][r] + acc[3][r]);
         } else {
-            ckq_v4i sh, sl;
+            int I[4] = {0, 0, 0, 0};
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                ckq_v4i ph, pl;
-                F::planes(ph, pl, hd, wrow, g, q);
-                sh = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[g], ph, g ? sh : zero, 0, 0, 0);
-                sl = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[g], pl, g ? sl : zero, 0, 0, 0);
+            for (int k = 0; k < 8 / F::SLABS; ++k) {
+                long w[F::SLABS];
+                F::raw(w, wrow, k, q);
+#pragma unroll
+                for (int j = 0; j < F::SLABS; ++j) {
+                    const long x = a[F::SLABS * k + j];
+                    slab_sums<F>(I, F::SLABS * k + j, x, two_dwords((u32)x & first, (u32)((uint64_t)x >> 32) & first), w[j], sc);
+                }
                 __builtin_amdgcn_sched_barrier(0);
             }
             if constexpr (F::MIN) {
                 const ckq_v4f i2 = min_mfma(am, hd.mins);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float f = (float)((sh[r] << F::SHIFT) + sl[r]);
+                    const float f = (float)I[r];
                     out[r] = hd.dw * f - hd.dmin * i2[r];
                 }
             } else {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) out[r] = hd.dw * (float)((sh[r] << F::SHIFT) + sl[r]);
+                for (int r = 0; r < 4; ++r) out[r] = hd.dw * (float)(I[r] >> 2);
             }
         }
         *reinterpret_cast<float4 *>(u + wave * (NT * 16) + 4 * lane) = float4{out[0], out[1], out[2], out[3]};
