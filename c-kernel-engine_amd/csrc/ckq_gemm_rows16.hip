@@ -11,7 +11,7 @@
  * v_mfma_i32_16x16x64_i8: A = 16 tokens x 64 k, B = 64 k x 16 weight rows, D = 16 x 16 int32.  Lane l = 16 q + i holds
  * token / row i and the 16 k of quarter q; of D it holds row i and tokens 4 q .. 4 q + 3.  The 64 k of an instruction are
  * those a lane of the streaming kernel takes, ordered so that a lane's sixteen are one 16-byte run of the raw block's
- * quants (low or high nibbles) inside one scale; the activations are read in the same order.  Where several groups of tokens share them, the planes are those of the tile kernels: Q4_K (sc >> 3) q and
+ * quants (low or high nibbles) inside one scale; the activations are read in the same order.  Where several groups of tokens share them (but for Q5_K in the kernel of two groups), the planes are those of the tile kernels: Q4_K (sc >> 3) q and
  * (sc & 7) q, Q5_K / Q6_K the two bytes of the 16-bit product, each summed over the 256-block; the min term of Q4_K / Q5_K is
  * a bf16 MFMA of the mins and the bsum pairs split in two (ckq_gemm_q4k.hip).  All integers are exact.
  *
@@ -92,7 +92,7 @@ __device__ __forceinline__ void scales_k45(int (&sc)[16], const uint8_t *r)
  * from a_elem(g, q).  planes() forms them from the raw block of the lane's row at r (in LDS). */
 struct R16Q4K {
     static constexpr int WBLOCK = 144, SHIFT = 3, CHUNKS = 9, PITCH = 144;
-    static constexpr bool MIN = true;
+    static constexpr bool MIN = true, HALVES = false;
     static __device__ __forceinline__ u32 chunk_ofs(int c) { return 16u * (u32)c; }
     static __device__ __forceinline__ u32 a_elem(int g, int q) { return 64u * g + 16u * q; }
     static __device__ __forceinline__ void head(Head &p, const uint8_t *r, int q) { head_k45(p, r, q); }
@@ -120,7 +120,18 @@ struct R16Q4K {
 
 struct R16Q5K {
     static constexpr int WBLOCK = 176, SHIFT = 8, CHUNKS = 11, PITCH = 176;
-    static constexpr bool MIN = true;
+    static constexpr bool MIN = true, HALVES = true;
+    /* for the kernel of two groups: the quants of position g, and those of its first 32 elements alone (lane quarters 0 and 1) */
+    static __device__ __forceinline__ void halves(ckq_v4i &all, ckq_v4i &first, const uint8_t *r, int g, int q)
+    {
+        const ckq_v4i qs = lds16(r + 48 + 32 * g + 16 * (q & 1)), qh = lds16(r + 16 + 16 * (q & 1));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const u32 n = ((u32)qs[i] >> (4 * (q >> 1))) & 0x0f0f0f0fu, v = n | ((((u32)qh[i] >> (2 * g + (q >> 1))) & 0x01010101u) << 4);
+            all[i] = (int)v;
+            first[i] = q < 2 ? (int)v : 0;
+        }
+    }
     static __device__ __forceinline__ u32 chunk_ofs(int c) { return 16u * (u32)c; }
     static __device__ __forceinline__ u32 a_elem(int g, int q) { return 64u * g + 16u * q; }
     static __device__ __forceinline__ void head(Head &p, const uint8_t *r, int q) { head_k45(p, r, q); }
@@ -154,7 +165,7 @@ struct R16Q5K {
 struct R16Q6K {
     /* a 210-byte block as fourteen chunks, the last from byte 194 so that no load passes the block's end */
     static constexpr int WBLOCK = 210, SHIFT = 8, CHUNKS = 14, PITCH = 240;
-    static constexpr bool MIN = false;
+    static constexpr bool MIN = false, HALVES = false;
     static __device__ __forceinline__ u32 chunk_ofs(int c) { return c < 13 ? 16u * (u32)c : 194u; }
     /* position g = 2 n + odd: the halves `odd` of the four 32-runs of 128-half n */
     static __device__ __forceinline__ u32 a_elem(int g, int q) { return 128u * (g >> 1) + 32u * q + 16u * (g & 1); }
@@ -238,6 +249,13 @@ __device__ __forceinline__ void slab_halves(int (&even)[4], int (&odd)[4], int s
         odd[r] += __mul24(O[r], sc[2 * s + 1]);
         asm("" : "+v"(even[r]), "+v"(odd[r]));
     }
+}
+/* A position's integer from the sums over all of its 64 elements and over the first 32. */
+__device__ __forceinline__ int halves_sum(int all, int first, int sc0, int sc1)
+{
+    int v = __mul24(first, sc0 - sc1);
+    asm("" : "+v"(v));
+    return v + __mul24(all, sc1);
 }
 
 /* Shape of a launch: what a block needs besides its problem. */
@@ -808,8 +826,11 @@ gemm_rows16_hold_kernel(const uint8_t *W, const uint8_t *X, int N, int M, int nb
  * block are formed once for both.  As in the first kernel wave w takes 256-blocks w, w + waves, ..., the next one's weights on their way;
  * a lane loads its own activations, in the order of the instruction.  Of TREE's terms, those of a position whose lane of the streaming
  * kernel has two blocks of the row (`wide` positions: blocks 0 .. wide - 1 and those from 16 on) go to LDS one by one, all others summed over their block.
- * Bound: VALU issue, 257 instructions a 256-block and group (Q5_K, TREE; 480 in the first kernel).  us against the first kernel: Q6_K 1024 x 4864 at 93
- * tokens 14.2 -> 9.0, Q5_K 11.4 -> 10.5, Q4_K 4096 x 4096 at 24 8.1 -> 7.0. */
+ * Bound: VALU issue.  us against the first kernel: Q6_K 1024 x 4864 at 93 tokens 14.2 -> 9.0, Q5_K 11.4 -> 10.5, Q4_K 4096 x 4096 at 24 8.1 -> 7.0.
+ * Q5_K's planes cost more than the 16-bit products they save (two scalings, a carry between the planes and a sum put together again), so its operands are
+ * the quants themselves, once whole and once with the second scale's half zero: instructions of a pair and 256-block 286 -> 275 in the tile kernels' order, about
+ * 420 -> 350 in TREE; us at 20 / 32 tokens: 2048 x 8192 10.7 -> 8.9, 1024 x 11008 13.0 -> 10.8, 2758 x 6400 at 22 14.2 -> 11.7, others 1.00-1.05.  Q4_K, whose planes are
+ * two multiplications, would need more (TREE 0.99, tile kernels' order 168 -> 227), and the kernel that keeps its planes, which forms them once, gains nothing. */
 template <class F, bool TREE, bool GRP>
 __global__ void __launch_bounds__(768)
 gemm_rows16_pair_kernel(const uint8_t *W, const uint8_t *X, int N, int M, int nb, float *y, const float *bias, long ldy, GemmChains ch, Rows16Args grp)
@@ -899,6 +920,12 @@ gemm_rows16_pair_kernel(const uint8_t *W, const uint8_t *X, int N, int M, int nb
         __builtin_amdgcn_sched_barrier(0);
         Head hd;
         F::head(hd, wrow, q);
+        int sc[16];
+        if constexpr (F::HALVES) F::scales(sc, wrow);
+        auto operands = [&](ckq_v4i &ph, ckq_v4i &pl, int g) {
+            if constexpr (F::HALVES) F::halves(ph, pl, wrow, g, q);
+            else F::planes(ph, pl, hd, wrow, g, q);
+        };
         int2 am[G];
 #pragma unroll
         for (int k = 0; k < G; ++k) {
@@ -915,7 +942,7 @@ gemm_rows16_pair_kernel(const uint8_t *W, const uint8_t *X, int N, int M, int nb
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 ckq_v4i ph, pl;
-                F::planes(ph, pl, hd, wrow, g, q);
+                operands(ph, pl, g);
 #pragma unroll
                 for (int k = 0; k < G; ++k) {
                     const ckq_v4i sh = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[k][g], ph, zero, 0, 0, 0);
@@ -925,7 +952,7 @@ gemm_rows16_pair_kernel(const uint8_t *W, const uint8_t *X, int N, int M, int nb
                     float v[4];
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        const float f = (float)((sh[r] << F::SHIFT) + sl[r]);
+                        const float f = (float)(F::HALVES ? halves_sum(sh[r], sl[r], sc[2 * g], sc[2 * g + 1]) : (sh[r] << F::SHIFT) + sl[r]);
                         if constexpr (F::MIN) v[r] = (hd.dw * dx[k][r]) * f - (hd.dmin * dx[k][r]) * i2[r];
                         else                  v[r] = (hd.dw * dx[k][r]) * f;
                         asm volatile("" : "+v"(v[r]));              /* rounded before it is added, as in the streaming kernel */
@@ -949,14 +976,19 @@ gemm_rows16_pair_kernel(const uint8_t *W, const uint8_t *X, int N, int M, int nb
             }
         } else {
             ckq_v4i sh[G], sl[G];
+            int I[G][4] = {};
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 ckq_v4i ph, pl;
-                F::planes(ph, pl, hd, wrow, g, q);
+                operands(ph, pl, g);
 #pragma unroll
                 for (int k = 0; k < G; ++k) {
-                    sh[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[k][g], ph, g ? sh[k] : zero, 0, 0, 0);
-                    sl[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[k][g], pl, g ? sl[k] : zero, 0, 0, 0);
+                    sh[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[k][g], ph, !F::HALVES && g ? sh[k] : zero, 0, 0, 0);
+                    sl[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[k][g], pl, !F::HALVES && g ? sl[k] : zero, 0, 0, 0);
+                    if constexpr (F::HALVES) {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) I[k][r] += halves_sum(sh[k][r], sl[k][r], sc[2 * g], sc[2 * g + 1]);
+                    }
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -967,7 +999,7 @@ gemm_rows16_pair_kernel(const uint8_t *W, const uint8_t *X, int N, int M, int nb
                 float out[4];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float f = (float)((sh[k][r] << F::SHIFT) + sl[k][r]);
+                    const float f = (float)(F::HALVES ? I[k][r] : (sh[k][r] << F::SHIFT) + sl[k][r]);
                     if constexpr (F::MIN) out[r] = hd.dw * f - hd.dmin * i2[r];
                     else                  out[r] = hd.dw * f;
                 }
