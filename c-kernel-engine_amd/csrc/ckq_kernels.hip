@@ -312,7 +312,12 @@ static bool weights_dword_aligned(const GemvArgs &a, const GemvGroup &grp)
  *              matrices stream at up to some 60 tokens (Q5_K 290 x 1792 at 25: 3.0, here 4.6; Q6_K 435 x 1536 at 13 3.0, here 4.8);
  *              several matrices take a launch each; against short rows' t_keep 2.4 + 14.9 w + 2.7 sqrt w (w: those lanes; Q5_K 2.2, 10.4, 6.0, Q6_K 2.15, 9.2, 8.65; 5.5 to 11 % rms
  *              over 900 launches of 17 to 120 tokens) and 1.17 t - 0.8 (1.32 t - 1.6; 1.4 t - 1.95): costs 0.1 to 0.25 % more than the faster kernel instead of 0.6 to 1.9, at most
- *              27 instead of 60 (us: Q6_K 47 tokens x 2048 x 368 7.0 -> 4.4, Q5_K 64 x 256 x 1141 4.9 -> 3.9); 5 to 8 tokens the larger of 3.5 + 0.07 nb and 3.05 + 0.11 nb + (0.24, 0.245, 0.29) mb for 10 tokens
+ *              27 instead of 60 (us: Q6_K 47 tokens x 2048 x 368 7.0 -> 4.4, Q5_K 64 x 256 x 1141 4.9 -> 3.9)
+ *   5 to 8 tokens, one to three matrices in a launch, weights from HBM: 2.64 + 0.0043 lanes + 7.6 million lanes of all rows + 0.237 mb + 0.022 lanes where the grid (the largest
+ *              matrix's for each) is more than a block a CU, 65536 lanes (Q5_K 2.71, 0.006, 8.0, 0.206, 0.0254; Q6_K 2.88, 0.0085, 11.7, 0.182, 0.0348: 10 to 11 % rms), against the 16-row
+ *              tiles' larger of 3.38 + 0.116 nb and 3.71 + 0.327 mb (3.45, 0.133, 3.83, 0.296; 3.39, 0.181, 3.76, 0.291: 7 % rms): 4692 launches of 64 to 40000 rows, widths of 256 to
+ *              16384. The choice costs 0.2 to 0.3 % more than the faster kernel; by a line without lanes, each matrix of a group for itself, it cost 7 to 8, at most 130 (us:
+ *              Q6_K 6 tokens x (4352, 1088, 1088) x 4352 25.5 -> 11.1, Q5_K 8 x (4352, 1088, 1088) x 4352 21.0 -> 10.1, Q4_K 8 x (5120, 1280, 1280) x 5120 21.1 -> 10.3, 8 x 2304 x 2304 6.7 -> 5.2)
  * Three and four tokens, one pass of half the width, only move for long rows of large Q6_K matrices whose positions leave a
  * tenth of those lanes idle (4096 x 11008 at 4: 14.2 -> 12.3, at 4 8192 x 4608 13.1 -> 11.4; but 4096 x 8192, no lane idle, 9.6 against
  * 9.9, and Q5_K 4096 x 8192 7.6 against 9.5); two never do.  The forced policies keep their kernels: 1 the tile kernels, 2 the
@@ -347,6 +352,40 @@ static float keep_time_own_scratch(int f, size_t rows, int ntok)
 static float rows16_q4k_time(float nb, size_t rows, int ntok) { return 3.6f + 0.12f * nb + 0.58e-3f * nb * (float)((rows + 15) / 16) * (float)((ntok + 15) / 16); }
 /* A Q4_K matrix of fewer than 160 tiles on its own: split along K or not, or by the 16-row kernel. */
 static float single_q4k_time(float nb, size_t rows, int ntok) { return fminf(nb < 8.0f ? 5.5f + 1.2f * nb : 7.2f + 0.22f * nb + 0.22f * 144e-6f * nb * (float)rows, rows16_q4k_time(nb, rows, ntok)); }
+/* Five to eight tokens, `rows` rows in one launch of either kernel; the streaming kernel's grid follows the largest of its matrices: `grid_rows`, their number times its
+ * rows. The figures are described above. */
+static float rows16_one_pass_time(int f, size_t rows, int K)
+{
+    static const float c[3][4] = {{3.38f, 0.116f, 3.71f, 0.327f}, {3.45f, 0.133f, 3.83f, 0.296f}, {3.39f, 0.181f, 3.76f, 0.291f}}, block[3] = {144e-6f, 176e-6f, 210e-6f};
+    const float nb = (float)(K / 256);
+    return fmaxf(c[f][0] + c[f][1] * nb, c[f][2] + c[f][3] * nb * (float)rows * block[f]);
+}
+static float stream_one_pass_time(int f, size_t rows, size_t grid_rows, int K)
+{
+    static const float c[3][5] = {{2.64f, 0.0043f, 7.6f, 0.237f, 0.0220f}, {2.71f, 0.0060f, 8.0f, 0.206f, 0.0254f}, {2.88f, 0.0085f, 11.7f, 0.182f, 0.0348f}}, block[3] = {144e-6f, 176e-6f, 210e-6f};
+    const int lanes = stream_lanes(K / 64);
+    const bool second_round = grid_rows * (size_t)(lanes < 16 ? 16 : lanes > 64 ? 64 : lanes) > 65536;
+    return c[f][0] + c[f][1] * (float)lanes + c[f][2] * 1e-6f * (float)rows * (float)lanes + c[f][3] * (float)(K / 256) * (float)rows * block[f] + (second_round ? c[f][4] * (float)lanes : 0.0f);
+}
+/* Several matrices of five to eight tokens, which have one order of their sums in either kernel: all of them to the 16-row tiles, or none (a choice by matrix sent Q and K/V of
+ * one group to two launches, or all to a streaming launch that each alone was too small to be faster than). */
+static bool rows16_as_one(int fmt, int ntok, int K)
+{
+    return ntok > 4 && ntok <= CKQ_STREAM_TOKENS && K <= ROWS16_MAX_K && g_gemm_policy.load(std::memory_order_relaxed) != 2 && !(g_rows16_forced.load(std::memory_order_relaxed) >> fmt & 1);
+}
+static bool group_takes_rows16(int fmt, int n, const int *rows, int K, bool streams_as_one)
+{
+    const int f = fmt == CKQ_FMT_Q4_K ? 0 : fmt == CKQ_FMT_Q5_K ? 1 : 2;
+    size_t all = 0, largest = 0;
+    float apart = 0.0f;
+    for (int i = 0; i < n; ++i) {
+        const size_t r = (size_t)rows[i];
+        all += r;
+        if (r > largest) largest = r;
+        apart += fminf(rows16_one_pass_time(f, r, K), stream_one_pass_time(f, r, r, K));
+    }
+    return rows16_one_pass_time(f, all, K) < (streams_as_one ? stream_one_pass_time(f, all, largest * (size_t)n, K) : apart);
+}
 static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles, int launches = 1, bool own_scratch = false, size_t shared_tiles = 0, float t_singles = 0.0f)
 {
     if (ntok < 2 || K > ROWS16_MAX_K) return false;
@@ -355,10 +394,11 @@ static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles, int l
     const int f = fmt == CKQ_FMT_Q4_K ? 0 : fmt == CKQ_FMT_Q5_K ? 1 : 2;
     const bool tile_forced = f == 0 ? gemm_q4k_forced() : f == 1 ? gemm_q5k_forced() : gemm_q6k_forced();
     if (ntok < 3 || policy == 2 || (tiles && (policy == 1 || tile_forced))) return false;
-    static const float per_block[3] = {0.36f, 0.65f, 0.71f}, per_pass[3] = {0.24f, 0.245f, 0.29f}, per_lane[3] = {23.5f, 23.5f, 29.0f};
+    static const float per_block[3] = {0.36f, 0.65f, 0.71f}, per_lane[3] = {23.5f, 23.5f, 29.0f};
     const float nb = (float)(K / 256), mb = (float)rows * nb * (f == 0 ? 144e-6f : f == 1 ? 176e-6f : 210e-6f);
     const int lanes = stream_lanes(K / 64);
     if (ntok <= 4) return f == 2 && K > 4096 && mb >= 20.0f && 10 * lanes >= 11 * (K / 64);
+    if (ntok <= CKQ_STREAM_TOKENS) return rows16_one_pass_time(f, rows, K) < stream_one_pass_time(f, rows, rows, K);
     const float t_keep = ntok > 256 ? 0.0f : own_scratch && tiles && K == 2048 ? keep_time_own_scratch(f, rows, ntok) : gemm_rows16_keep_time(fmt, !tiles, rows, ntok, K / 256);
     const float t_pair = tiles && t_keep <= 0.0f ? gemm_rows16_pair_time(fmt, rows, ntok, K / 256) : 0.0f;
     const float t_rows = t_keep > 0.0f ? t_keep : t_pair > 0.0f ? t_pair : 3.6f + 0.12f * nb + per_block[f] * 1e-3f * nb * (float)((rows + 15) / 16) * (float)((ntok + 15) / 16);
@@ -394,7 +434,6 @@ static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles, int l
         return rows16_q4k_time(nb, rows, ntok) < t_tiles;
     }
     if (tiles) t_else = f == 0 || t_pair <= 0.0f ? 11.0f + (0.2f + 0.0015f * (float)ntok) * mb : f == 1 ? 13.3f + (0.164f + 0.0048f * (float)ntok) * mb : 13.8f + (0.083f + 0.0044f * (float)ntok) * mb;
-    else if (ntok <= 8) t_else = fmaxf(3.5f + 0.07f * nb, 3.05f + 0.11f * nb + 1.25f * per_pass[f] * mb);
     else {
         const float t_launch = 2.2f + 0.0075f * (float)lanes, w = 1e-6f * (float)rows * (float)lanes * (float)((ntok + 7) / 8);
         if (t_keep > 0.0f) {
@@ -510,6 +549,15 @@ extern "C" int ckq_launch_gemv_group(int fmt, int n, float *const *y, const void
         if (ldys[i] < rows[i] || ldys[i] > 0x7fffffff || !y[i]) return CKQ_EINVAL;
     for (int i = 0; i < n; ++i)
         if (!W[i] || !X[i]) return CKQ_EINVAL;
+    /* K-quants at five to eight tokens: one choice for all matrices; at fewer, below, one for each. */
+    const bool kquant = !subdots && (fmt == CKQ_FMT_Q4_K || fmt == CKQ_FMT_Q5_K || fmt == CKQ_FMT_Q6_K) && K % 256 == 0;
+    const bool as_one = kquant && n > 1 && rows16_as_one(fmt, ntok, K);
+    if (as_one && group_takes_rows16(fmt, n, rows, K, group_tile_fits_lds(fmt, K, ntok))) {
+        Rows16Args r = {};
+        r.M = ntok; r.nb = K / 256; r.tree = true; r.n = n;
+        for (int i = 0; i < n; ++i) r.p[i] = {(const uint8_t *)W[i], (const uint8_t *)X[i], y[i], bias ? bias[i] : nullptr, ldys[i], rows[i], 0, {}};
+        return launch_gemm_rows16(fmt, r, (hipStream_t)stream);
+    }
     /* Every grouped kernel stages its token tile in LDS.  A tile that does not
      * fit (the tile is the token count rounded up to 1, 2, 4 or 8 rows of
      * activations) goes out as n separate launches, which stream it instead. */
@@ -536,7 +584,7 @@ extern "C" int ckq_launch_gemv_group(int fmt, int n, float *const *y, const void
     };
     /* Matrices that the 16-row tiles take when launched alone share a launch of theirs, the others one of the streaming
      * kernel: every result keeps the bits of its single launch. */
-    if (!subdots && (fmt == CKQ_FMT_Q4_K || fmt == CKQ_FMT_Q5_K || fmt == CKQ_FMT_Q6_K) && K % 256 == 0) {
+    if (kquant && !as_one) {
         Rows16Args r = {};
         r.M = ntok; r.nb = K / 256; r.tree = true;
         int rest[CKQ_GROUP_MAX], nrest = 0;
@@ -584,12 +632,16 @@ extern "C" int ckq_launch_gemv_pro(int fmt, int n, float *const *y, const void *
     if (n < 1 || n > CKQ_GROUP_MAX || ntok < 1 || ntok > CKQ_STREAM_TOKENS || K < 256 || K > 2048 || K % 256 || stride < K || stride % 4) return CKQ_ENOGROUP;
     const size_t wblock = fmt == CKQ_FMT_Q4_K ? 144 : fmt == CKQ_FMT_Q5_K ? 176 : fmt == CKQ_FMT_Q6_K ? 210 : 0;
     if (!wblock || !x || !xq) return CKQ_ENOGROUP;
+    /* The 16-row tiles want quantized activations: the quantizer's launch and theirs. At five to eight tokens this kernel streams the weights for two tiles of tokens, and where they beat ONE
+     * streaming launch they are no slower with the quantizer (layers of 512 to 2048 columns, 5 and 8 tokens, against always this kernel: 0.97-1.09, 1.01 on average). */
+    const bool as_one = rows16_as_one(fmt, ntok, K);
+    if (as_one && group_takes_rows16(fmt, n, rows, K, true)) return CKQ_ENOGROUP;
     const size_t xbytes = ((size_t)(ntok - 1) * (size_t)stride + (size_t)K) * 4, qbytes = (size_t)ntok * (size_t)(K / 256) * 292;
     if (ckq_ranges_overlap(xq, qbytes, x, xbytes) || (gamma && ckq_ranges_overlap(xq, qbytes, gamma, (size_t)K * 4))) return CKQ_ENOGROUP;
     GemvArgs a = {};
     GemvGroup grp = k_no_group;
     for (int i = 0; i < n; ++i) {
-        if (!y[i] || !W[i] || rows[i] <= 0 || ldys[i] < rows[i] || ldys[i] > 0x7fffffff || take_rows16(fmt, ntok, (size_t)rows[i], K, false)) return CKQ_ENOGROUP;
+        if (!y[i] || !W[i] || rows[i] <= 0 || ldys[i] < rows[i] || ldys[i] > 0x7fffffff || (!as_one && take_rows16(fmt, ntok, (size_t)rows[i], K, false))) return CKQ_ENOGROUP;
         /* every block reads x: nothing it is made of may be written by the launch before the last has, nor xq read */
         const size_t ybytes = ((size_t)(ntok - 1) * (size_t)ldys[i] + (size_t)rows[i]) * 4;
         if (ckq_ranges_overlap(y[i], ybytes, x, xbytes) || (gamma && ckq_ranges_overlap(y[i], ybytes, gamma, (size_t)K * 4)) || ckq_ranges_overlap(y[i], ybytes, xq, qbytes) ||

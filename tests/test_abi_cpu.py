@@ -221,6 +221,14 @@ def test_16_row_tiles_where_they_are_the_faster_ones(L, fmt, n, k, tokens, want)
     assert route(L, fmt, n, k, tokens) == want
 
 
+@pytest.mark.parametrize("fmt,n,k,tokens,want", [
+    ("q4_k", 2304, 2304, 8, ROWS16_STREAM), ("q4_k", 1792, 4608, 7, ROWS16_STREAM), ("q4_k", 1024, 3072, 8, STREAM), ("q5_k", 3328, 3328, 8, ROWS16_STREAM), ("q5_k", 1280, 5632, 8, ROWS16_STREAM),
+    ("q5_k", 1024, 2560, 6, STREAM), ("q6_k", 3584, 10752, 5, ROWS16_STREAM), ("q6_k", 1024, 3328, 5, STREAM), ("q6_k", 1792, 1792, 8, STREAM)])
+def test_16_row_tiles_at_five_to_eight_tokens(L, fmt, n, k, tokens, want):
+    """Single matrices on either side of the line, where both kernels were timed."""
+    assert route(L, fmt, n, k, tokens) == want
+
+
 @pytest.mark.parametrize("M,Ns,last", [(405, (11008, 11008), True), (276, (7680, 7680), True), (139, (5888, 5888), True), (282, (7041,), True), (65, (17000,), True),
                                        (88, (9000, 7700), True), (341, (6912, 6912), False), (384, (11008, 11008), False), (227, (8960, 8960), False),
                                        (405, (4096, 1024, 1024), False), (9, (34000,), False), (400, (28672,), False)])
