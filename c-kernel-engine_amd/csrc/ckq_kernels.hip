@@ -318,9 +318,11 @@ static bool weights_dword_aligned(const GemvArgs &a, const GemvGroup &grp)
  *              tiles' larger of 3.38 + 0.116 nb and 3.71 + 0.327 mb (3.45, 0.133, 3.83, 0.296; 3.39, 0.181, 3.76, 0.291: 7 % rms): 4692 launches of 64 to 40000 rows, widths of 256 to
  *              16384. The choice costs 0.2 to 0.3 % more than the faster kernel; by a line without lanes, each matrix of a group for itself, it cost 7 to 8, at most 130 (us:
  *              Q6_K 6 tokens x (4352, 1088, 1088) x 4352 25.5 -> 11.1, Q5_K 8 x (4352, 1088, 1088) x 4352 21.0 -> 10.1, Q4_K 8 x (5120, 1280, 1280) x 5120 21.1 -> 10.3, 8 x 2304 x 2304 6.7 -> 5.2)
- * Three and four tokens, one pass of half the width, only move for long rows of large Q6_K matrices whose positions leave a
- * tenth of those lanes idle (4096 x 11008 at 4: 14.2 -> 12.3, at 4 8192 x 4608 13.1 -> 11.4; but 4096 x 8192, no lane idle, 9.6 against
- * 9.9, and Q5_K 4096 x 8192 7.6 against 9.5); two never do.  The forced policies keep their kernels: 1 the tile kernels, 2 the
+ *   3 and 4 tokens, one pass of half the width: 2.48 + 0.0008 lanes + 4.36 million lanes (1.15 times that for rows above 6144) + 0.141 mb + 0.0129 lanes where the grid is more than two blocks a CU
+ *              (2.62, 0.0004, 6.04, 0.098, 0.0148; 2.70, 0.0043, 7.19, 0.103, 0.0189) against 1.1 times the larger of 3.04 + 0.142 nb and 3.73 + 0.311 mb (3.15, 0.151, 3.88, 0.279; 3.27,
+ *              0.188, 3.86, 0.288): 6 to 8 % rms over 2100 launches. By the rule before, for large Q6_K matrices alone, the choice cost 2.7 % more than the faster kernel, by this 0.8: 332
+ *              launches by more than 5 % faster, 8 by more than 3 % slower (us: Q5_K 4 x 11264 x 2560 13.0 -> 9.8, Q6_K 4 x (4352, 2176, 2176) x 4352 18.3 -> 14.5; not moved, Q5_K 4 x 4096 x 8192 7.6 against 9.5).
+ * Two tokens never move.  The forced policies keep their kernels: 1 the tile kernels, 2 the
  * streaming kernel at any number of tokens; and so does a tile kernel that the caller asked for.  Forced itself
  * (ckq_launch_set_rows16) it goes before all of them, in the order of the kernel that the policy asks for. */
 static int stream_lanes(int positions)
@@ -352,28 +354,32 @@ static float keep_time_own_scratch(int f, size_t rows, int ntok)
 static float rows16_q4k_time(float nb, size_t rows, int ntok) { return 3.6f + 0.12f * nb + 0.58e-3f * nb * (float)((rows + 15) / 16) * (float)((ntok + 15) / 16); }
 /* A Q4_K matrix of fewer than 160 tiles on its own: split along K or not, or by the 16-row kernel. */
 static float single_q4k_time(float nb, size_t rows, int ntok) { return fminf(nb < 8.0f ? 5.5f + 1.2f * nb : 7.2f + 0.22f * nb + 0.22f * 144e-6f * nb * (float)rows, rows16_q4k_time(nb, rows, ntok)); }
-/* Five to eight tokens, `rows` rows in one launch of either kernel; the streaming kernel's grid follows the largest of its matrices: `grid_rows`, their number times its
- * rows. The figures are described above. */
-static float rows16_one_pass_time(int f, size_t rows, int K)
+/* Three to eight tokens, `rows` rows in one launch of either kernel; the streaming kernel's grid follows the largest of its matrices: `grid_rows`, their number times its
+ * rows. The figures are described above; at three and four tokens the 16-row tiles have to be ahead by a tenth, as the times lie closer than
+ * the fits do there. */
+static float rows16_one_pass_time(int f, int ntok, size_t rows, int K)
 {
-    static const float c[3][4] = {{3.38f, 0.116f, 3.71f, 0.327f}, {3.45f, 0.133f, 3.83f, 0.296f}, {3.39f, 0.181f, 3.76f, 0.291f}}, block[3] = {144e-6f, 176e-6f, 210e-6f};
-    const float nb = (float)(K / 256);
-    return fmaxf(c[f][0] + c[f][1] * nb, c[f][2] + c[f][3] * nb * (float)rows * block[f]);
+    static const float c[2][3][4] = {{{3.04f, 0.142f, 3.73f, 0.311f}, {3.15f, 0.151f, 3.88f, 0.279f}, {3.27f, 0.188f, 3.86f, 0.288f}},
+                                     {{3.38f, 0.116f, 3.71f, 0.327f}, {3.45f, 0.133f, 3.83f, 0.296f}, {3.39f, 0.181f, 3.76f, 0.291f}}}, block[3] = {144e-6f, 176e-6f, 210e-6f};
+    const float nb = (float)(K / 256), *t = c[ntok > 4][f];
+    return (ntok > 4 ? 1.0f : 1.1f) * fmaxf(t[0] + t[1] * nb, t[2] + t[3] * nb * (float)rows * block[f]);
 }
-static float stream_one_pass_time(int f, size_t rows, size_t grid_rows, int K)
+static float stream_one_pass_time(int f, int ntok, size_t rows, size_t grid_rows, int K)
 {
-    static const float c[3][5] = {{2.64f, 0.0043f, 7.6f, 0.237f, 0.0220f}, {2.71f, 0.0060f, 8.0f, 0.206f, 0.0254f}, {2.88f, 0.0085f, 11.7f, 0.182f, 0.0348f}}, block[3] = {144e-6f, 176e-6f, 210e-6f};
+    static const float c[2][3][5] = {{{2.48f, 0.0008f, 4.36f, 0.141f, 0.0129f}, {2.62f, 0.0004f, 6.04f, 0.098f, 0.0148f}, {2.70f, 0.0043f, 7.19f, 0.103f, 0.0189f}},
+                                     {{2.64f, 0.0043f, 7.6f, 0.237f, 0.0220f}, {2.71f, 0.0060f, 8.0f, 0.206f, 0.0254f}, {2.88f, 0.0085f, 11.7f, 0.182f, 0.0348f}}}, block[3] = {144e-6f, 176e-6f, 210e-6f};
     const int lanes = stream_lanes(K / 64);
-    const bool second_round = grid_rows * (size_t)(lanes < 16 ? 16 : lanes > 64 ? 64 : lanes) > 65536;
-    return c[f][0] + c[f][1] * (float)lanes + c[f][2] * 1e-6f * (float)rows * (float)lanes + c[f][3] * (float)(K / 256) * (float)rows * block[f] + (second_round ? c[f][4] * (float)lanes : 0.0f);
+    const bool second_round = grid_rows * (size_t)(lanes < 16 ? 16 : lanes > 64 ? 64 : lanes) > (ntok > 4 ? 65536 : 131072);
+    const float *t = c[ntok > 4][f], few_blocks = ntok <= 4 && K > 6144 ? 1.15f : 1.0f;       /* four long tokens fill the LDS of a CU with few blocks */
+    return t[0] + t[1] * (float)lanes + few_blocks * t[2] * 1e-6f * (float)rows * (float)lanes + t[3] * (float)(K / 256) * (float)rows * block[f] + (second_round ? t[4] * (float)lanes : 0.0f);
 }
-/* Several matrices of five to eight tokens, which have one order of their sums in either kernel: all of them to the 16-row tiles, or none (a choice by matrix sent Q and K/V of
+/* Several matrices of three to eight tokens, which have one order of their sums in either kernel: all of them to the 16-row tiles, or none (a choice by matrix sent Q and K/V of
  * one group to two launches, or all to a streaming launch that each alone was too small to be faster than). */
 static bool rows16_as_one(int fmt, int ntok, int K)
 {
-    return ntok > 4 && ntok <= CKQ_STREAM_TOKENS && K <= ROWS16_MAX_K && g_gemm_policy.load(std::memory_order_relaxed) != 2 && !(g_rows16_forced.load(std::memory_order_relaxed) >> fmt & 1);
+    return ntok > 2 && ntok <= CKQ_STREAM_TOKENS && K <= ROWS16_MAX_K && g_gemm_policy.load(std::memory_order_relaxed) != 2 && !(g_rows16_forced.load(std::memory_order_relaxed) >> fmt & 1);
 }
-static bool group_takes_rows16(int fmt, int n, const int *rows, int K, bool streams_as_one)
+static bool group_takes_rows16(int fmt, int ntok, int n, const int *rows, int K, bool streams_as_one)
 {
     const int f = fmt == CKQ_FMT_Q4_K ? 0 : fmt == CKQ_FMT_Q5_K ? 1 : 2;
     size_t all = 0, largest = 0;
@@ -382,9 +388,9 @@ static bool group_takes_rows16(int fmt, int n, const int *rows, int K, bool stre
         const size_t r = (size_t)rows[i];
         all += r;
         if (r > largest) largest = r;
-        apart += fminf(rows16_one_pass_time(f, r, K), stream_one_pass_time(f, r, r, K));
+        apart += fminf(rows16_one_pass_time(f, ntok, r, K), stream_one_pass_time(f, ntok, r, r, K));
     }
-    return rows16_one_pass_time(f, all, K) < (streams_as_one ? stream_one_pass_time(f, all, largest * (size_t)n, K) : apart);
+    return rows16_one_pass_time(f, ntok, all, K) < (streams_as_one ? stream_one_pass_time(f, ntok, all, largest * (size_t)n, K) : apart);
 }
 static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles, int launches = 1, bool own_scratch = false, size_t shared_tiles = 0, float t_singles = 0.0f)
 {
@@ -397,8 +403,7 @@ static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles, int l
     static const float per_block[3] = {0.36f, 0.65f, 0.71f}, per_lane[3] = {23.5f, 23.5f, 29.0f};
     const float nb = (float)(K / 256), mb = (float)rows * nb * (f == 0 ? 144e-6f : f == 1 ? 176e-6f : 210e-6f);
     const int lanes = stream_lanes(K / 64);
-    if (ntok <= 4) return f == 2 && K > 4096 && mb >= 20.0f && 10 * lanes >= 11 * (K / 64);
-    if (ntok <= CKQ_STREAM_TOKENS) return rows16_one_pass_time(f, rows, K) < stream_one_pass_time(f, rows, rows, K);
+    if (ntok <= CKQ_STREAM_TOKENS) return rows16_one_pass_time(f, ntok, rows, K) < stream_one_pass_time(f, ntok, rows, rows, K);
     const float t_keep = ntok > 256 ? 0.0f : own_scratch && tiles && K == 2048 ? keep_time_own_scratch(f, rows, ntok) : gemm_rows16_keep_time(fmt, !tiles, rows, ntok, K / 256);
     const float t_pair = tiles && t_keep <= 0.0f ? gemm_rows16_pair_time(fmt, rows, ntok, K / 256) : 0.0f;
     const float t_rows = t_keep > 0.0f ? t_keep : t_pair > 0.0f ? t_pair : 3.6f + 0.12f * nb + per_block[f] * 1e-3f * nb * (float)((rows + 15) / 16) * (float)((ntok + 15) / 16);
@@ -549,10 +554,10 @@ extern "C" int ckq_launch_gemv_group(int fmt, int n, float *const *y, const void
         if (ldys[i] < rows[i] || ldys[i] > 0x7fffffff || !y[i]) return CKQ_EINVAL;
     for (int i = 0; i < n; ++i)
         if (!W[i] || !X[i]) return CKQ_EINVAL;
-    /* K-quants at five to eight tokens: one choice for all matrices; at fewer, below, one for each. */
+    /* K-quants at three to eight tokens: one choice for all matrices; two never go there, and forced, below, all do. */
     const bool kquant = !subdots && (fmt == CKQ_FMT_Q4_K || fmt == CKQ_FMT_Q5_K || fmt == CKQ_FMT_Q6_K) && K % 256 == 0;
     const bool as_one = kquant && n > 1 && rows16_as_one(fmt, ntok, K);
-    if (as_one && group_takes_rows16(fmt, n, rows, K, group_tile_fits_lds(fmt, K, ntok))) {
+    if (as_one && group_takes_rows16(fmt, ntok, n, rows, K, group_tile_fits_lds(fmt, K, ntok))) {
         Rows16Args r = {};
         r.M = ntok; r.nb = K / 256; r.tree = true; r.n = n;
         for (int i = 0; i < n; ++i) r.p[i] = {(const uint8_t *)W[i], (const uint8_t *)X[i], y[i], bias ? bias[i] : nullptr, ldys[i], rows[i], 0, {}};
@@ -635,7 +640,7 @@ extern "C" int ckq_launch_gemv_pro(int fmt, int n, float *const *y, const void *
     /* The 16-row tiles want quantized activations: the quantizer's launch and theirs. At five to eight tokens this kernel streams the weights for two tiles of tokens, and where they beat ONE
      * streaming launch they are no slower with the quantizer (layers of 512 to 2048 columns, 5 and 8 tokens, against always this kernel: 0.97-1.09, 1.01 on average). */
     const bool as_one = rows16_as_one(fmt, ntok, K);
-    if (as_one && group_takes_rows16(fmt, n, rows, K, true)) return CKQ_ENOGROUP;
+    if (as_one && ntok > 4 && group_takes_rows16(fmt, ntok, n, rows, K, true)) return CKQ_ENOGROUP;
     const size_t xbytes = ((size_t)(ntok - 1) * (size_t)stride + (size_t)K) * 4, qbytes = (size_t)ntok * (size_t)(K / 256) * 292;
     if (ckq_ranges_overlap(xq, qbytes, x, xbytes) || (gamma && ckq_ranges_overlap(xq, qbytes, gamma, (size_t)K * 4))) return CKQ_ENOGROUP;
     GemvArgs a = {};

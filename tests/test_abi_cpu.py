@@ -223,8 +223,9 @@ def test_16_row_tiles_where_they_are_the_faster_ones(L, fmt, n, k, tokens, want)
 
 @pytest.mark.parametrize("fmt,n,k,tokens,want", [
     ("q4_k", 2304, 2304, 8, ROWS16_STREAM), ("q4_k", 1792, 4608, 7, ROWS16_STREAM), ("q4_k", 1024, 3072, 8, STREAM), ("q5_k", 3328, 3328, 8, ROWS16_STREAM), ("q5_k", 1280, 5632, 8, ROWS16_STREAM),
-    ("q5_k", 1024, 2560, 6, STREAM), ("q6_k", 3584, 10752, 5, ROWS16_STREAM), ("q6_k", 1024, 3328, 5, STREAM), ("q6_k", 1792, 1792, 8, STREAM)])
-def test_16_row_tiles_at_five_to_eight_tokens(L, fmt, n, k, tokens, want):
+    ("q5_k", 1024, 2560, 6, STREAM), ("q6_k", 3584, 10752, 5, ROWS16_STREAM), ("q6_k", 1024, 3328, 5, STREAM), ("q6_k", 1792, 1792, 8, STREAM),
+    ("q5_k", 3328, 13568, 3, ROWS16_STREAM), ("q6_k", 4352, 4352, 4, ROWS16_STREAM), ("q6_k", 2560, 2560, 4, STREAM), ("q4_k", 3840, 3840, 4, STREAM), ("q6_k", 14336, 14336, 2, STREAM)])
+def test_16_row_tiles_at_two_to_eight_tokens(L, fmt, n, k, tokens, want):
     """Single matrices on either side of the line, where both kernels were timed."""
     assert route(L, fmt, n, k, tokens) == want
 

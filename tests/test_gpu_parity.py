@@ -1952,18 +1952,19 @@ def test_16_row_tiles_alone_on_their_cu(fmt):
 
 
 @pytest.mark.parametrize("fmt", ["q4_k", "q5_k", "q6_k"])
-def test_matrices_of_five_to_eight_tokens_share_one_choice_of_kernel(fmt):
+def test_matrices_of_three_to_eight_tokens_share_one_choice_of_kernel(fmt):
     """Groups that go to the 16-row tiles and ones that stream, with rows that some or none of the matrices alone would take there, rows too long for a grouped
     streaming launch and the longest, ragged and tiny matrices: bit for bit what the streaming kernel gives each matrix alone."""
     import torch
     L = ckq.lib()
     try:
         for M, K, Ns in [(8, 4352, (4352, 1088, 1088)), (5, 2560, (2560, 640, 640)), (6, 3072, (3072, 1536, 1536)), (7, 512, (512, 128, 128)), (8, 768, (1000, 17, 1)), (5, 2048, (5632, 5632)),
-                         (8, 256, (70, 4000)), (6, 7424, (1500, 1, 300)), (7, 11008, (96, 33)), (5, 16384, (700, 500)), (5, 16640, (64, 32)), (8, 1280, (1280, 320, 320)), (4, 2560, (2560, 640, 640))]:
+                         (8, 256, (70, 4000)), (6, 7424, (1500, 1, 300)), (7, 11008, (96, 33)), (5, 16384, (700, 500)), (5, 16640, (64, 32)), (8, 1280, (1280, 320, 320)), (4, 2560, (2560, 640, 640)),
+                         (4, 4608, (4608, 1152, 1152)), (3, 8192, (2100, 40)), (3, 14592, (300, 17)), (2, 4608, (4608, 600))]:
             xq = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, seed=M + K)), "q8_k", rows=M)
             Ws = [P.to_device(T.random_blocks(fmt, n * K // 256, 9700 + i)) for i, n in enumerate(Ns)]
             bs = [P.to_device(T.normal(n, 0.0, 0.5, seed=n)) for n in Ns]
-            say("groups of five to eight tokens", fmt, M, K, Ns)
+            say("groups of three to eight tokens", fmt, M, K, Ns)
             ys = [torch.full((M, n + 3), 7.0, device="cuda") for n in Ns]
             P.dev_matmul_sequence([(fmt, xq, W, b, y, M, n, K, n + 3) for W, b, y, n in zip(Ws, bs, ys, Ns)])
             L.ckq_set_gemm_policy(2)
