@@ -352,8 +352,14 @@ static float keep_time_own_scratch(int f, size_t rows, int ntok)
     return least < 4.4f + 1e-3f * (f == 1 ? 4.98f : 5.82f) * (float)(tiles * groups) ? least : 0.0f;
 }
 static float rows16_q4k_time(float nb, size_t rows, int ntok) { return 3.6f + 0.12f * nb + 0.58e-3f * nb * (float)((rows + 15) / 16) * (float)((ntok + 15) / 16); }
-/* A Q4_K matrix of fewer than 160 tiles on its own: split along K or not, or by the 16-row kernel. */
-static float single_q4k_time(float nb, size_t rows, int ntok) { return fminf(nb < 8.0f ? 5.5f + 1.2f * nb : 7.2f + 0.22f * nb + 0.22f * 144e-6f * nb * (float)rows, rows16_q4k_time(nb, rows, ntok)); }
+/* A matrix of fewer than 160 tiles on its own: split along K or not, or by the 16-row kernel (Q5_K, Q6_K: fitted to 631 launches of whichever the rule takes, 17 to 130 tokens, 12 % rms). */
+static float single_time(int f, float nb, size_t rows, int ntok)
+{
+    static const float c[2][6] = {{2.09f, 0.224f, 0.218f, 13.8f, 0.50f, 176e-6f}, {2.13f, 0.232f, 0.127f, 15.0f, 0.565f, 210e-6f}};
+    const float out = 1e-6f * (float)ntok * (float)rows;
+    if (f) return c[f - 1][0] + c[f - 1][1] * nb + c[f - 1][2] * c[f - 1][5] * nb * (float)rows + (c[f - 1][3] + c[f - 1][4] * nb) * out;
+    return fminf(nb < 8.0f ? 5.5f + 1.2f * nb : 7.2f + 0.22f * nb + 0.22f * 144e-6f * nb * (float)rows, rows16_q4k_time(nb, rows, ntok));
+}
 /* Three to eight tokens, `rows` rows in one launch of either kernel; the streaming kernel's grid follows the largest of its matrices: `grid_rows`, their number times its
  * rows. The figures are described above; at three and four tokens the 16-row tiles have to be ahead by a tenth, as the times lie closer than
  * the fits do there. */
@@ -408,6 +414,14 @@ static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles, int l
     const float t_pair = tiles && t_keep <= 0.0f ? gemm_rows16_pair_time(fmt, rows, ntok, K / 256) : 0.0f;
     const float t_rows = t_keep > 0.0f ? t_keep : t_pair > 0.0f ? t_pair : 3.6f + 0.12f * nb + per_block[f] * 1e-3f * nb * (float)((rows + 15) / 16) * (float)((ntok + 15) / 16);
     float t_else;
+    /* Q5_K and Q6_K, several matrices that together are too few tiles for a shared launch: the tile kernels would take one or two launches for EACH, and what the estimates below know is one for all.
+     * Where the 16-row tiles are ahead by a tenth they have it (fitted to 699 groups of 17 to 130 tokens, 13 % rms). 529 further groups of up to 400 tokens: 3.2 % faster on average, 54 by more than 5 %,
+     * none by more than 4 % slower (us, one by one -> 16-row tiles in one launch: Q5_K 105 x 3 x 2304 x 2304 30.0 -> 20.5, 98 x (3072, 1536, 1536) x 3072 31.1 -> 21.8, Q6_K 64 x (5120, 1280, 1280) x
+     * 5120 41.8 -> 28.6; left, 34 x (8704, 1088, 1088) x 8704 52.3 | 63.4). */
+    if (f > 0 && tiles && ntok > 16 && launches > 1 && shared_tiles == 0 && !own_scratch) {
+        static const float group[2][3] = {{2.85f, 0.303f, 0.583e-3f}, {2.97f, 0.282f, 0.575e-3f}};
+        if (1.1f * (group[f - 1][0] + group[f - 1][1] * nb + group[f - 1][2] * nb * (float)((rows + 15) / 16) * (float)((ntok + 15) / 16)) < t_singles) return true;
+    }
     if (const int pieces = tiles && launches == 1 && !own_scratch && rows < 1 << 24
                                ? gemm_ksplit_pieces(ntok, (long)rows, K / 256, f == 0 ? GEMM_KSPLIT_Q4K : f == 1 ? GEMM_KSPLIT_Q5K : GEMM_KSPLIT_Q6K) : 0) {
         static const float split[3][4] = {{4.1f, 1.44f, 0.16f, 3.3f}, {3.7f, 1.83f, 0.12f, 2.8f}, {3.75f, 1.73f, 0.18f, 3.7f}},
@@ -777,7 +791,7 @@ extern "C" int ckq_launch_gemm_group(int fmt, int n, float *const *C, const void
             alike = alike && tiles[p] == tiles[0];
         }
         float t_singles = 0.0f;
-        for (int p = 0; p < n; ++p) t_singles += single_q4k_time((float)(K / 256), (size_t)N[p], M);
+        for (int p = 0; p < n; ++p) t_singles += single_time(fmt == CKQ_FMT_Q4_K ? 0 : fmt == CKQ_FMT_Q5_K ? 1 : 2, (float)(K / 256), (size_t)N[p], M);
         if (alike && take_rows16(fmt, M, rows, K, tiles[0], n, false, grouped ? (size_t)gemm_group_tiles(in, M, 64) : 0, t_singles)) {
             Rows16Args r = {};
             r.M = M; r.nb = K / 256; r.n = n; r.tree = !tiles[0];

@@ -1975,6 +1975,27 @@ def test_matrices_of_three_to_eight_tokens_share_one_choice_of_kernel(fmt):
         L.ckq_set_gemm_policy(0)
 
 
+@pytest.mark.parametrize("fmt", ["q5_k", "q6_k"])
+def test_groups_of_too_few_tiles_for_a_shared_launch_keep_their_matrices_bits(fmt):
+    """Q, K and V of 17 to 313 tokens whose tiles together would leave most of the chip idle, on either side of the line between one launch of 16-row tiles and
+    the tile kernels one by one: the bits that each matrix has alone."""
+    import torch
+    for M, K, Ns in [(105, 2304, (2304, 2304, 2304)), (81, 4352, (4352, 1088, 1088)), (38, 3072, (3072, 3072, 3072)), (17, 5120, (4100, 2561)), (313, 2560, (2560, 320, 320)), (34, 8704, (8704, 1088, 1088))]:
+        xq = P.dev_quantize(P.to_device(T.normal(M * K, 0.0, 1.0, seed=M + K)), "q8_k", rows=M)
+        Ws = [P.to_device(T.random_blocks(fmt, n * K // 256, 9800 + i)) for i, n in enumerate(Ns)]
+        bs = [P.to_device(T.normal(n, 0.0, 0.5, seed=n)) for n in Ns]
+        say("groups of few tiles", fmt, M, K, Ns)
+        ys = [torch.full((M, n + 3), 7.0, device="cuda") for n in Ns]
+        P.dev_matmul_sequence([(fmt, xq, W, b, y, M, n, K, n + 3) for W, b, y, n in zip(Ws, bs, ys, Ns)])
+        for W, b, y, n in zip(Ws, bs, ys, Ns):
+            one = P.dev_gemm_nt(fmt, xq, W, b, M, n, K).view(M, n)
+            assert bool((y[:, n:] == 7.0).all())
+            if (M + 7) // 8 * max(n * T.row_bytes(fmt, K), 3 << 20) > (40 if fmt == "q5_k" else 20) << 20:
+                assert torch.equal(y[:, :n], one), (M, K, n)
+            else:                                         # alone it streams, with another order of its sums
+                assert torch.allclose(y[:, :n], one, rtol=0, atol=2e-6 * float(one.abs().max())), (M, K, n)
+
+
 @pytest.mark.parametrize("fmt", ["q4_k", "q5_k", "q6_k"])
 def test_16_row_tiles_of_token_groups_in_pairs(fmt):
     """Longer rows, two token groups a block: an even and an odd number of groups, a last group of one token, ragged rows, fewer blocks of the row than
