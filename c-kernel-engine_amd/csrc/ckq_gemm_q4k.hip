@@ -20,9 +20,9 @@
  *   accumulated over all eight sub-blocks of a block; I1 = 8*H + L exactly.
  *   Nibble unpack and the two multiplies (v_pk_mul_lo_u16 on byte pairs) are
  *   done once per weight and reused for both 32-token halves of the tile.
- * - The min term contracts 8 (min, bsum) pairs per block.  Stored bsums need
- *   13 bits; split as lo + 64*hi (lo in [0,63], hi in [-64,63]) both parts and
- *   the 6-bit mins are exact in bf16, so ONE v_mfma_f32_32x32x16_bf16 per
+ * - The min term contracts 8 (min, bsum) pairs per block.  A pair of stored
+ *   bsums is split in its low eight bits and the rest (min_operand): both parts
+ *   and the 6-bit mins are exact in bf16, so ONE v_mfma_f32_32x32x16_bf16 per
  *   32x32 tile per block yields I2 exactly in fp32 (|I2| < 2^24).
  * - Every operand reaches the matrix cores through LDS, filled by 16-byte
  *   global->LDS loads (no VGPR staging): the raw Q4_K blocks of the tile's
@@ -50,7 +50,7 @@ struct GemmStage {
     uint8_t  w[GEMM_BN * 144];    /* raw Q4_K blocks, row r at byte 144 r */
     uint8_t  q[GEMM_BM * 256];    /* int8 quants: 16-byte chunk c of token t in slot c ^ (t & 15) of its 256 bytes */
     float    d[GEMM_BM];          /* block scale of each token */
-    uint16_t b[GEMM_BM * 16];     /* bf16: lo_0..7, 64*hi_0..7 of the stored bsums */
+    uint16_t b[GEMM_BM * 16];     /* bf16: the two parts (min_operand) of the eight pairs of stored bsums */
 };
 
 /* One 256-block of a 64-token tile, software-pipelined by hand.  The 32 int8
@@ -263,11 +263,8 @@ __global__ void __launch_bounds__(256 * KG, KG == 2 ? 1 : WPE) gemm_q4k_mfma_ker
     auto side_store = [&](int buf) {
         if (!st_live) return;
         if (st_q == 0) stage[buf].d[st_tok] = nd;
-        const int b0 = (int)(int16_t)(nbs[0] & 0xffff) + (int)(int16_t)(nbs[0] >> 16);
-        const int b1 = (int)(int16_t)(nbs[1] & 0xffff) + (int)(int16_t)(nbs[1] >> 16);
         u32 *bd = reinterpret_cast<u32 *>(&stage[buf].b[st_tok * 16]);
-        bd[st_q]     = bf16_pair((float)(b0 & 63), (float)(b1 & 63));
-        bd[4 + st_q] = bf16_pair((float)(64 * (b0 >> 6)), (float)(64 * (b1 >> 6)));
+        min_operand((int)nbs[0], (int)nbs[1], bd[st_q], bd[4 + st_q]);
     };
 
     /* read-side offsets of this lane */
@@ -418,10 +415,10 @@ __global__ void __launch_bounds__(64 * SPLITS, 1) gemm_q4k_ksplit_kernel(GemmArg
         ckq_v4i lo, hi;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int u = s[i >> 1][2 * (i & 1)], v = s[i >> 1][2 * (i & 1) + 1];
-            const int p0 = (int)(int16_t)(u & 0xffff) + (u >> 16), p1 = (int)(int16_t)(v & 0xffff) + (v >> 16);
-            lo[i] = (int)bf16_pair((float)(p0 & 63), (float)(p1 & 63));
-            hi[i] = (int)bf16_pair((float)(64 * (p0 >> 6)), (float)(64 * (p1 >> 6)));
+            u32 l, h;
+            min_operand(s[i >> 1][2 * (i & 1)], s[i >> 1][2 * (i & 1) + 1], l, h);
+            lo[i] = (int)l;
+            hi[i] = (int)h;
         }
         o[0] = lo;
         o[1] = hi;

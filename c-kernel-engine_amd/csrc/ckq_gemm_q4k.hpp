@@ -23,6 +23,16 @@ __device__ __forceinline__ u32 bf16_pair(float lo, float hi)
     return __builtin_amdgcn_perm(__builtin_bit_cast(u32, hi), __builtin_bit_cast(u32, lo), 0x07060302u);
 }
 
+/* The token operand of the min term: two pairs of stored bsums, a dword each, as P & 255 and P - (P & 255).  Both parts have at most eight
+ * significant bits, exact in bf16, whatever the sixteen-bit bsums are, and eight products with 6-bit mins and their sums stay below 2^24, exact in the
+ * matrix core's fp32, up to |P| = 2^15, eight times what sums of int8 quants reach. */
+__device__ __forceinline__ void min_operand(int pair0, int pair1, u32 &lo, u32 &hi)
+{
+    const int p0 = (int)(int16_t)(pair0 & 0xffff) + (pair0 >> 16), p1 = (int)(int16_t)(pair1 & 0xffff) + (pair1 >> 16);
+    lo = bf16_pair((float)(p0 & 255), (float)(p1 & 255));
+    hi = bf16_pair((float)(p0 & ~255), (float)(p1 & ~255));
+}
+
 /* 96-token tiles, one block per tile, no K split (ckq_gemm_q4k_t96.hip).  g: A, B, bias, C, M, N, nb, ldc, nnt
  * and the dump pointer set by the caller; for the grouped form A, M and nb. */
 constexpr int T96_TOKENS = 96;

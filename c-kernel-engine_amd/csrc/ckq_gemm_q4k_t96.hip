@@ -31,7 +31,7 @@ struct T96Raw {
 };
 struct T96Side {
     float    d[T96_BM];          /* block scale of each token */
-    uint16_t b[T96_BM * 16];     /* bf16: lo_0..7, 64*hi_0..7 of the pair sums of the stored bsums */
+    uint16_t b[T96_BM * 16];     /* bf16: the two parts (min_operand) of the eight pairs of stored bsums */
 };
 
 /* The last token group of a 256-block, MFMAs done but not yet combined into the fp32 accumulators: that happens
@@ -265,7 +265,7 @@ __global__ void __launch_bounds__(256, DUMP ? 1 : WPE) gemm_q4k_t96_kernel(GemmA
         }
     };
     /* raw -> side, four threads per token (tokens 64..95: the first 128 threads once more): the scale as it is, the
-     * sixteen bsums as eight pair sums split lo + 64 hi, both exact in bf16 */
+     * sixteen bsums as the two parts of their eight pairs (min_operand) */
     const int st_tok = tid >> 2, st_q = tid & 3;
     const bool st_two = wave < 2 && ng == 3;
     auto side_read = [&](int tok, u32 (&bs)[2], u32 &d) __attribute__((always_inline)) {
@@ -276,11 +276,8 @@ __global__ void __launch_bounds__(256, DUMP ? 1 : WPE) gemm_q4k_t96_kernel(GemmA
     };
     auto side_put = [&](int tok, const u32 (&bs)[2], u32 d) __attribute__((always_inline)) {
         if (st_q == 0) reinterpret_cast<u32 *>(side.d)[tok] = d;
-        const int s0 = (int)(int16_t)(bs[0] & 0xffff) + (int)(int16_t)(bs[0] >> 16);
-        const int s1 = (int)(int16_t)(bs[1] & 0xffff) + (int)(int16_t)(bs[1] >> 16);
         u32 *bd = reinterpret_cast<u32 *>(&side.b[tok * 16]);
-        bd[st_q]     = bf16_pair((float)(s0 & 63), (float)(s1 & 63));
-        bd[4 + st_q] = bf16_pair((float)(64 * (s0 >> 6)), (float)(64 * (s1 >> 6)));
+        min_operand((int)bs[0], (int)bs[1], bd[st_q], bd[4 + st_q]);
     };
 
     const u32 wofs_l = (u32)(32 * wave + col) * 144u;

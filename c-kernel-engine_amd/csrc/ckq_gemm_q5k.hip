@@ -15,7 +15,7 @@
  *   v = 256 * H + L (L = signed low byte of v, H = high byte of v + 128), the
  *   byte lanes of the products gathered with v_perm_b32; both planes are
  *   accumulated over the block, I1 = 256 * IH + IL.
- * - The min term is one bf16 MFMA per 32x32 tile per block, as in the Q4_K kernel: the eight bsum pairs P of a token as P & 63 and P - (P & 63) fill the
+ * - The min term is one bf16 MFMA per 32x32 tile per block, as in the Q4_K kernel: the two parts of a token's eight bsum pairs (min_operand) fill the
  *   sixteen k slots, the eight mins stand against both halves, and the sum leaves the matrix core as the fp32 number that is wanted, exactly.
  *   The block's threads turn the stored bsums into that operand where they lie in LDS, a quarter of a token each.  Two int8 MFMAs of bytes of P, formed by every
  *   wave for itself, and their integers shifted, added and converted were 646 vector instructions a 256-block and wave where this is 545 (matrix 36 -> 34).  What
@@ -44,21 +44,15 @@ struct Gemm5Stage {
     float   d[GEMM5_BM];               /* block scale of each token */
 };
 
-/* The token operand of the min term in the place of the stored bsums: of a token's 32 bytes its eight bsum pairs P as P & 63 in the first half and as
- * P - (P & 63) in the second, exact in bf16.  `quarter`: of the sixteen bsums. */
-__device__ __forceinline__ void gemm5_min_quarter(const int2 &d, u32 &lo, u32 &hi)
-{
-    const int p0 = (int)(int16_t)(d.x & 0xffff) + (d.x >> 16), p1 = (int)(int16_t)(d.y & 0xffff) + (d.y >> 16);
-    lo = bf16_pair((float)(p0 & 63), (float)(p1 & 63));
-    hi = bf16_pair((float)(p0 & ~63), (float)(p1 & ~63));
-}
-/* By the 256 threads of a block, four to a token, which are neighbours in a wave: all of a token is read before any of it is written. */
+/* The token operand of the min term in the place of the stored bsums: of a token's 32 bytes the first half the low parts of its eight pairs, the second half the
+ * high ones (min_operand).  By the 256 threads of a block, four to a token, which are neighbours in a wave: all of a token is read before any of it is written. */
 __device__ __forceinline__ void gemm5_min_operand(uint8_t *bsum, int tid)
 {
     uint8_t *const t = bsum + 32 * (tid >> 2);
     const int qu = tid & 3;
     u32 lo, hi;
-    gemm5_min_quarter(*reinterpret_cast<const int2 *>(t + 8 * qu), lo, hi);
+    const int2 pairs = *reinterpret_cast<const int2 *>(t + 8 * qu);
+    min_operand(pairs.x, pairs.y, lo, hi);
     *reinterpret_cast<u32 *>(t + 4 * qu) = lo;
     *reinterpret_cast<u32 *>(t + 16 + 4 * qu) = hi;
 }
@@ -513,12 +507,12 @@ __global__ void __launch_bounds__(64 * SPLITS, 1) gemm_q5k_ksplit_kernel(GemmArg
         const int bn = min(b + 1, last);
         {
             uint8_t *const t = bs[wave] + 32 * lane;
-            const ckq_v4i b0 = *reinterpret_cast<const ckq_v4i *>(t), b1 = *reinterpret_cast<const ckq_v4i *>(t + 16);
+            const ckq_v4i stored[2] = {*reinterpret_cast<const ckq_v4i *>(t), *reinterpret_cast<const ckq_v4i *>(t + 16)};
             ckq_v4i lo, hi;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 u32 l, h;
-                gemm5_min_quarter(k < 2 ? int2{b0[2 * k], b0[2 * k + 1]} : int2{b1[2 * k - 4], b1[2 * k - 3]}, l, h);
+                min_operand(stored[k >> 1][2 * (k & 1)], stored[k >> 1][2 * (k & 1) + 1], l, h);
                 lo[k] = (int)l;
                 hi[k] = (int)h;
             }

@@ -349,11 +349,12 @@ gemm_rows16_kernel(const uint8_t *W, const uint8_t *X, int N, Rows16Shape S, flo
 #pragma unroll
         for (int j = 0; j < NAL; ++j) *reinterpret_cast<ckq_v4i *>(al + adst[j]) = ar[j];
     };
-    /* the two bsum pairs of position q as lo + 64 hi, exact in bf16 (ckq_gemm_q4k.hip) */
+    /* the two bsum pairs of position q */
     auto bsum_operand = [&]() {
         const int2 bs = *reinterpret_cast<const int2 *>(bl + 32 * ta + 8 * q);
-        const int p0 = (int)(int16_t)(bs.x & 0xffff) + (bs.x >> 16), p1 = (int)(int16_t)(bs.y & 0xffff) + (bs.y >> 16);
-        return ckq_v4i{(int)bf16_pair((float)(p0 & 63), (float)(p1 & 63)), (int)bf16_pair((float)(64 * (p0 >> 6)), (float)(64 * (p1 >> 6))), 0, 0};
+        u32 lo, hi;
+        min_operand(bs.x, bs.y, lo, hi);
+        return ckq_v4i{(int)lo, (int)hi, 0, 0};
     };
     auto min_mfma = [&](const ckq_v4i &am, const ckq_v4i &mins) {
         const ckq_v4f z = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -631,8 +632,9 @@ gemm_rows16_hold_kernel(const uint8_t *W, const uint8_t *X, int N, int M, int nb
         }
     };
     auto bsum_operand = [&](const int2 &bs) {
-        const int p0 = (int)(int16_t)(bs.x & 0xffff) + (bs.x >> 16), p1 = (int)(int16_t)(bs.y & 0xffff) + (bs.y >> 16);
-        return int2{(int)bf16_pair((float)(p0 & 63), (float)(p1 & 63)), (int)bf16_pair((float)(64 * (p0 >> 6)), (float)(64 * (p1 >> 6)))};
+        u32 lo, hi;
+        min_operand(bs.x, bs.y, lo, hi);
+        return int2{(int)lo, (int)hi};
     };
     auto min_mfma = [&](const int2 &am, const ckq_v4i &mins) {
         const ckq_v4f z = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -929,8 +931,12 @@ gemm_rows16_pair_kernel(const uint8_t *W, const uint8_t *X, int N, int M, int nb
         int2 am[G];
 #pragma unroll
         for (int k = 0; k < G; ++k) {
-            const int b0 = (int)bs[k][0], b1 = (int)bs[k][1], p0 = (int)(int16_t)(b0 & 0xffff) + (b0 >> 16), p1 = (int)(int16_t)(b1 & 0xffff) + (b1 >> 16);
-            am[k] = F::MIN ? int2{(int)bf16_pair((float)(p0 & 63), (float)(p1 & 63)), (int)bf16_pair((float)(64 * (p0 >> 6)), (float)(64 * (p1 >> 6)))} : int2{};
+            am[k] = int2{};
+            if constexpr (F::MIN) {
+                u32 lo, hi;
+                min_operand((int)bs[k][0], (int)bs[k][1], lo, hi);
+                am[k] = int2{(int)lo, (int)hi};
+            }
         }
         if constexpr (TREE) {
             const bool apart = b < wide || b >= 16;
@@ -1162,8 +1168,9 @@ gemm_rows16_keep_kernel(const uint8_t *W, const uint8_t *X, int N, int M, int pa
         int2 am = {};
         if constexpr (F::MIN) {
             const int2 b = *reinterpret_cast<const int2 *>(bl + 32 * i16 + 8 * q);
-            const int p0 = (int)(int16_t)(b.x & 0xffff) + (b.x >> 16), p1 = (int)(int16_t)(b.y & 0xffff) + (b.y >> 16);
-            am = int2{(int)bf16_pair((float)(p0 & 63), (float)(p1 & 63)), (int)bf16_pair((float)(64 * (p0 >> 6)), (float)(64 * (p1 >> 6)))};
+            u32 lo, hi;
+            min_operand(b.x, b.y, lo, hi);
+            am = int2{(int)lo, (int)hi};
         }
         ckq_v4i a[4];
 #pragma unroll

@@ -77,7 +77,10 @@ typedef struct {
 } ckq_block_q6_K;
 
 /* Q8_K: activation super-block. fp32 d, 256 x int8, 16 x int16 sums of each
- * run of 16 quants. 292 bytes, 4-byte aligned. */
+ * run of 16 quants. 292 bytes, 4-byte aligned. Matmuls of Q4_K and Q5_K weights
+ * take the stored sums as they are, whatever their sixteen bits; the min term of
+ * a block is exact while pairs (2j, 2j + 1) stay within +-32768 (sums of int8
+ * reach 4096), and rounded like any fp32 sum beyond. */
 typedef struct {
     float    d;
     int8_t   qs[CKQ_QK_K];

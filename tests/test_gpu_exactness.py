@@ -197,6 +197,27 @@ def test_gemm_mfma_block_sums_extremes():
     assert T.norm_err(c.cpu().numpy(), T.oracle_gemm_nt("q4_k", A, W, None, M, N, K)) <= TOL
 
 
+@pytest.mark.parametrize("fmt", ["q4_k", "q5_k"])
+@pytest.mark.parametrize("M,N,K", [(70, 200, 512), (130, 384, 2048), (520, 260, 512)])
+def test_gemm_mfma_min_sums_of_any_stored_bsums(fmt, M, N, K):
+    """Stored bsums of any value whose pairs stay within +-2^15: the min sums of the tile kernels are the integers."""
+    W, A = rand_case(fmt, N, K, 5 * M + K, tokens=M)
+    A = A.copy().reshape(-1, 292)
+    stored = np.random.default_rng(M).integers(-16384, 16384, size=(A.shape[0], 16)).astype(np.int16)
+    stored[0], stored[-1] = 16383, -16384
+    A[:, 260:292] = stored.view(np.uint8)
+    A = A.reshape(-1)
+    say("gemm min sums, any stored bsums", fmt, M, N, K)
+    L = ckq.dump_lib()
+    try:
+        for variant in (64, 96) if fmt == "q4_k" else (1, 2):
+            L.ckq_set_prefill_variant(P.FMT[fmt], variant)
+            _, sums = P.dev_gemm_block_sums(fmt, P.to_device(A), P.to_device(W), None, M, N, K)
+            assert np.array_equal(sums.cpu().numpy().astype(np.int64), np_block_sums(fmt, W, A, M, N, K)), variant
+    finally:
+        L.ckq_set_prefill_variant(P.FMT[fmt], 0)
+
+
 # ---- fp16 scales at the ends of their range ----------------------------------------------------------
 
 def _set_f16(blocks, off, bits):

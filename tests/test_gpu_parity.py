@@ -1011,7 +1011,7 @@ def test_gemm_mfma_q5_k_vs_oracle(M, N, K):
 def test_gemm_mfma_q5_k_stored_bsums_and_extremes():
     """Stored bsums are consumed (zeroed bsums drop the min term), and the
     extreme values (5-bit value 31, scale and min 63, q8 = -128 / 127, bsums at
-    both ends of their range) stay exact through the byte-split operands."""
+    both ends of their range) stay exact through the split operands."""
     M, N, K = 96, 64, 512
     W, _, xq = make_case("q5_k", N, K, "rand", 1311, tokens=M)
     xz = xq.copy().reshape(-1, 292)
@@ -1036,6 +1036,35 @@ def test_gemm_mfma_q5_k_stored_bsums_and_extremes():
         ref = T.oracle_gemm_nt("q5_k", xb, Wb, None, M, N, K)
         c = P.dev_gemm_nt("q5_k", P.to_device(xb), P.to_device(Wb), None, M, N, K).cpu().numpy()
         assert T.norm_err(c, ref) <= TOL, pattern
+
+
+@pytest.mark.parametrize("fmt", ["q4_k", "q5_k"])
+@pytest.mark.parametrize("M,N,K", [(1, 70, 1280), (5, 300, 512), (13, 96, 2816), (16, 4100, 1024), (24, 200, 512), (30, 2100, 2560), (70, 200, 2304), (100, 130, 512)])
+def test_stored_bsums_of_any_sixteen_bits(fmt, M, N, K):
+    """Stored bsums that no int8 quants sum to, pairs of them up to +-2^15: eight times a pair of the quantizer's.  Every kernel that serves the size against the oracle, whose
+    min term is an integer.  The bar: the rounding of up to eleven fp32 terms and their sums, 16 x 2^-24 of the terms' absolute sum, which is at most some five
+    times the largest result here; a part of a pair cut to bf16 that does not fit it errs by 1e-4 and more."""
+    W, _, xq = make_case(fmt, N, K, "rand", 1400 + M, tokens=M)
+    rng = np.random.default_rng(M + K)
+    xb = xq.copy().reshape(-1, 292)
+    stored = rng.integers(-16384, 16384, size=(xb.shape[0], 16)).astype(np.int16)
+    stored[0], stored[-1] = 16383, -16384
+    xb[:, 260:292] = stored.view(np.uint8)
+    xb = xb.reshape(-1)
+    say("stored bsums of any value", fmt, M, N, K)
+    ref = T.oracle_gemm_nt(fmt, xb, W, None, M, N, K)
+    L, tag = ckq.lib(), P.FMT[fmt]
+    Xd, Wd = P.to_device(xb), P.to_device(W)
+    forms = [(0, 0), (2, 0), (2, 16)] + ([(1, v) for v in (0, 16) + ((64, 96) if fmt == "q4_k" else (1, 2))] if M > 8 else [])
+    try:
+        for policy, variant in forms:
+            L.ckq_set_prefill_variant(tag, variant)
+            L.ckq_set_gemm_policy(policy)
+            c = P.dev_gemm_nt(fmt, Xd, Wd, None, M, N, K).cpu().numpy().reshape(M, N)
+            assert T.norm_err(c, ref) <= 5e-6, (policy, variant)
+    finally:
+        L.ckq_set_gemm_policy(0)
+        L.ckq_set_prefill_variant(tag, 0)
 
 
 # ---- loader hook: registered weight regions ---------------------------------------------------
