@@ -379,6 +379,13 @@ static float stream_one_pass_time(int f, int ntok, size_t rows, size_t grid_rows
     const float *t = c[ntok > 4][f], few_blocks = ntok <= 4 && K > 6144 ? 1.15f : 1.0f;       /* four long tokens fill the LDS of a CU with few blocks */
     return t[0] + t[1] * (float)lanes + few_blocks * t[2] * 1e-6f * (float)rows * (float)lanes + t[3] * (float)(K / 256) * (float)rows * block[f] + (second_round ? t[4] * (float)lanes : 0.0f);
 }
+/* Q6_K at three and four tokens, rows of more than 4096, 20 MB of weights and more, a tenth of the streaming kernel's lanes idle: the passes over a row with few blocks on a CU, whose LDS the four
+ * tokens fill, take up to 1.7 times the estimate below, and by it the 16-row tiles lost what they had had (180 such launches of one to three matrices, weights from HBM: streaming / 16-row tiles 1.37
+ * in the middle, 1.77 at most, one 0.94 and two 0.99; us: 4 x 3 x 3831 x 11008 45.6 | 29.3, 3 x 2 x 7984 x 10496 54.7 | 35.2, 4 x (8517, 4258, 4258) x 6912 34.4 | 29.4). */
+static bool q6k_long_rows_of_few_tokens(int f, int ntok, size_t rows, int K)
+{
+    return f == 2 && ntok <= 4 && K > 4096 && (float)rows * (float)(K / 256) * 210e-6f >= 20.0f && 10 * stream_lanes(K / 64) >= 11 * (K / 64);
+}
 /* Several matrices of three to eight tokens, which have one order of their sums in either kernel: all of them to the 16-row tiles, or none (a choice by matrix sent Q and K/V of
  * one group to two launches, or all to a streaming launch that each alone was too small to be faster than). */
 static bool rows16_as_one(int fmt, int ntok, int K)
@@ -396,7 +403,7 @@ static bool group_takes_rows16(int fmt, int ntok, int n, const int *rows, int K,
         if (r > largest) largest = r;
         apart += fminf(rows16_one_pass_time(f, ntok, r, K), stream_one_pass_time(f, ntok, r, r, K));
     }
-    return rows16_one_pass_time(f, ntok, all, K) < (streams_as_one ? stream_one_pass_time(f, ntok, all, largest * (size_t)n, K) : apart);
+    return q6k_long_rows_of_few_tokens(f, ntok, all, K) || rows16_one_pass_time(f, ntok, all, K) < (streams_as_one ? stream_one_pass_time(f, ntok, all, largest * (size_t)n, K) : apart);
 }
 static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles, int launches = 1, bool own_scratch = false, size_t shared_tiles = 0, float t_singles = 0.0f)
 {
@@ -409,7 +416,7 @@ static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles, int l
     static const float per_block[3] = {0.36f, 0.65f, 0.71f}, per_lane[3] = {23.5f, 23.5f, 29.0f};
     const float nb = (float)(K / 256), mb = (float)rows * nb * (f == 0 ? 144e-6f : f == 1 ? 176e-6f : 210e-6f);
     const int lanes = stream_lanes(K / 64);
-    if (ntok <= CKQ_STREAM_TOKENS) return rows16_one_pass_time(f, ntok, rows, K) < stream_one_pass_time(f, ntok, rows, rows, K);
+    if (ntok <= CKQ_STREAM_TOKENS) return q6k_long_rows_of_few_tokens(f, ntok, rows, K) || rows16_one_pass_time(f, ntok, rows, K) < stream_one_pass_time(f, ntok, rows, rows, K);
     const float t_keep = ntok > 256 ? 0.0f : own_scratch && tiles && K == 2048 ? keep_time_own_scratch(f, rows, ntok) : gemm_rows16_keep_time(fmt, !tiles, rows, ntok, K / 256);
     const float t_pair = tiles && t_keep <= 0.0f ? gemm_rows16_pair_time(fmt, rows, ntok, K / 256) : 0.0f;
     const float t_rows = t_keep > 0.0f ? t_keep : t_pair > 0.0f ? t_pair : 3.6f + 0.12f * nb + per_block[f] * 1e-3f * nb * (float)((rows + 15) / 16) * (float)((ntok + 15) / 16);

@@ -230,6 +230,13 @@ def test_16_row_tiles_at_two_to_eight_tokens(L, fmt, n, k, tokens, want):
     assert route(L, fmt, n, k, tokens) == want
 
 
+@pytest.mark.parametrize("n,k,tokens,want", [(11493, 11008, 4, ROWS16_STREAM), (15968, 10496, 3, ROWS16_STREAM), (17034, 6912, 4, ROWS16_STREAM), (16040, 14080, 4, ROWS16_STREAM),
+                                             (567, 9984, 3, STREAM), (8520, 4096, 3, STREAM), (576, 14592, 4, STREAM)])
+def test_q6_k_long_rows_at_three_and_four_tokens(L, n, k, tokens, want):
+    """Rows of two to four passes of the streaming kernel, weights of some megabytes: both kernels were timed (as one matrix or as several of as many rows), the faster one by a seventh and more is taken."""
+    assert route(L, "q6_k", n, k, tokens) == want
+
+
 @pytest.mark.parametrize("M,Ns,last", [(405, (11008, 11008), True), (276, (7680, 7680), True), (139, (5888, 5888), True), (282, (7041,), True), (65, (17000,), True),
                                        (88, (9000, 7700), True), (341, (6912, 6912), False), (384, (11008, 11008), False), (227, (8960, 8960), False),
                                        (405, (4096, 1024, 1024), False), (9, (34000,), False), (400, (28672,), False)])
