@@ -368,7 +368,10 @@ static float rows16_one_pass_time(int f, int ntok, size_t rows, int K)
     static const float c[2][3][4] = {{{3.04f, 0.142f, 3.73f, 0.311f}, {3.15f, 0.151f, 3.88f, 0.279f}, {3.27f, 0.188f, 3.86f, 0.288f}},
                                      {{3.38f, 0.116f, 3.71f, 0.327f}, {3.45f, 0.133f, 3.83f, 0.296f}, {3.39f, 0.181f, 3.76f, 0.291f}}}, block[3] = {144e-6f, 176e-6f, 210e-6f};
     const float nb = (float)(K / 256), *t = c[ntok > 4][f];
-    return (ntok > 4 ? 1.0f : 1.1f) * fmaxf(t[0] + t[1] * nb, t[2] + t[3] * nb * (float)rows * block[f]);
+    /* Q4_K, five to eight tokens, rows of up to four blocks: by the fit alone they streamed where the 16-row tiles are the faster ones and had been taken (us, streaming | 16-row tiles: 8 x 8695 x 1024
+     * 5.55 | 4.77, 5 x 7256 x 1024 4.62 | 4.31; 242 such launches: the choice costs 0.9 % more than the faster kernel, 3.4 without) */
+    const float short_rows = f == 0 && ntok > 4 && nb <= 4.0f ? 0.93f : 1.0f;
+    return (ntok > 4 ? short_rows : 1.1f) * fmaxf(t[0] + t[1] * nb, t[2] + t[3] * nb * (float)rows * block[f]);
 }
 static float stream_one_pass_time(int f, int ntok, size_t rows, size_t grid_rows, int K)
 {

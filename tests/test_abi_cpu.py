@@ -237,6 +237,13 @@ def test_q6_k_long_rows_at_three_and_four_tokens(L, n, k, tokens, want):
     assert route(L, "q6_k", n, k, tokens) == want
 
 
+@pytest.mark.parametrize("n,k,tokens,want", [(8695, 1024, 8, ROWS16_STREAM), (7479, 1024, 8, ROWS16_STREAM), (7256, 1024, 5, ROWS16_STREAM), (7434, 1024, 8, ROWS16_STREAM), (15500, 512, 6, ROWS16_STREAM),
+                                             (9500, 768, 7, ROWS16_STREAM), (3500, 1024, 8, STREAM), (7500, 512, 8, STREAM), (3500, 768, 6, STREAM)])
+def test_q4_k_short_rows_at_five_to_eight_tokens(L, n, k, tokens, want):
+    """Rows of two to four blocks on either side of the line, where both kernels were timed."""
+    assert route(L, "q4_k", n, k, tokens) == want
+
+
 @pytest.mark.parametrize("M,Ns,last", [(405, (11008, 11008), True), (276, (7680, 7680), True), (139, (5888, 5888), True), (282, (7041,), True), (65, (17000,), True),
                                        (88, (9000, 7700), True), (341, (6912, 6912), False), (384, (11008, 11008), False), (227, (8960, 8960), False),
                                        (405, (4096, 1024, 1024), False), (9, (34000,), False), (400, (28672,), False)])
