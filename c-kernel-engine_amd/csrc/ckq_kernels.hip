@@ -507,6 +507,62 @@ static GemmChains rows16_chains(int fmt, int ntok, int nrows, int K, bool tiles)
     return fmt == CKQ_FMT_Q4_K ? gemm_q4k_chains(ntok, nrows, K) : fmt == CKQ_FMT_Q5_K ? gemm_q5k_chains(ntok, nrows, K) : gemm_q6k_chains(ntok, nrows, K);
 }
 
+/* LDS bytes of the staged token tile of a grouped launch against the 64 KB a
+ * block may use: MT rows of activations, MT = token count rounded up to the
+ * tile sizes launch_mt knows (1, 2, 4, 8); Q8_0 activations are re-laid out to
+ * 36 bytes per block. */
+static bool group_tile_fits_lds(int fmt, int K, int ntok)
+{
+    const size_t mt = ntok <= 1 ? 1 : ntok == 2 ? 2 : ntok <= 4 ? 4 : 8;
+    size_t bytes;
+    switch (fmt) {
+    case CKQ_FMT_Q4_K: case CKQ_FMT_Q5_K: case CKQ_FMT_Q6_K: bytes = FmtQ4K::xs_lds_bytes(mt * (size_t)(K / 256) * 292); break;
+    case CKQ_FMT_Q8_0: case CKQ_FMT_Q5_0:                     bytes = FmtQ80::xs_lds_bytes(mt * (size_t)(K / 32) * 34); break;
+    default: return false;
+    }
+    return bytes <= 65536;
+}
+
+/* Where several K-quant matrices against the same `ntok` tokens go.  Up to eight tokens: the 16-row tiles (all of them) or the streaming kernel.  Beyond: the 16-row tiles in the
+ * order of either (one order a launch), in place of the tile kernels' shared launch where they would take it, else of the single launches and with the bits of either; the tile kernels'
+ * shared launch; or CKQ_ENOGROUP, one by one.  *grouped: whether the shared launch would be taken, whose chains *shared then are. */
+static int kquant_group_route(int fmt, const GemmGroupIn &in, int M, int K, bool *grouped, GemmChains *shared)
+{
+    const int f = fmt == CKQ_FMT_Q4_K ? 0 : fmt == CKQ_FMT_Q5_K ? 1 : 2;
+    size_t rows = 0;
+    for (int p = 0; p < in.n; ++p) rows += (size_t)in.N[p];
+    *grouped = kquant_on_matrix_cores(fmt, M, rows, K) &&
+               (f == 0 ? gemm_q4k_group_chains(in, M, K, shared) : f == 1 ? gemm_q5k_group_chains(in, M, K, shared) : gemm_q6k_group_chains(in, M, K, shared));
+    bool tiles[GEMM_GROUP_MAX], alike = true;
+    float t_singles = 0.0f;
+    for (int p = 0; p < in.n; ++p) {
+        tiles[p] = *grouped || kquant_on_matrix_cores(fmt, M, (size_t)in.N[p], K);
+        alike = alike && tiles[p] == tiles[0];
+        t_singles += single_time(f, (float)(K / 256), (size_t)in.N[p], M);
+    }
+    if (alike && take_rows16(fmt, M, rows, K, tiles[0], in.n, false, *grouped ? (size_t)gemm_group_tiles(in, M, 64) : 0, t_singles)) return tiles[0] ? CKQ_ROUTE_ROWS16_TILES : CKQ_ROUTE_ROWS16_STREAM;
+    return *grouped ? CKQ_ROUTE_TILES : CKQ_ENOGROUP;
+}
+static int group_route(int fmt, int n, const int *rows, int K, int ntok)
+{
+    if (ntok <= CKQ_STREAM_TOKENS) {
+        /* two tokens, and the policies that ask for a kernel, have one answer for all sizes */
+        const bool rows16 = rows16_as_one(fmt, ntok, K) ? group_takes_rows16(fmt, ntok, n, rows, K, group_tile_fits_lds(fmt, K, ntok)) : take_rows16(fmt, ntok, (size_t)rows[0], K, false);
+        return rows16 ? CKQ_ROUTE_ROWS16_STREAM : CKQ_ROUTE_STREAM;
+    }
+    GemmGroupIn in = {};
+    in.n = n;
+    for (int p = 0; p < n; ++p) in.N[p] = rows[p];
+    bool grouped;
+    GemmChains shared = {};
+    return kquant_group_route(fmt, in, ntok, K, &grouped, &shared);
+}
+extern "C" int ckq_launch_group_route(int fmt, int n, const int *rows, int K, int ntok)
+{
+    if (n < 2 || n > CKQ_GROUP_MAX || K < 256 || K % 256 || ntok < 1 || (fmt != CKQ_FMT_Q4_K && fmt != CKQ_FMT_Q5_K && fmt != CKQ_FMT_Q6_K)) return CKQ_EINVAL;
+    return group_route(fmt, n, rows, K, ntok);
+}
+
 static int launch_rows16_one(int fmt, const GemvArgs &a, bool tiles, int K, hipStream_t s)
 {
     Rows16Args r = {};
@@ -538,22 +594,6 @@ extern "C" int ckq_launch_gemv(int fmt, float *y, const void *W, const void *X, 
     return launch_gemv_args(fmt, a, k_no_group, K, stream);
 }
 
-/* LDS bytes of the staged token tile of a grouped launch against the 64 KB a
- * block may use: MT rows of activations, MT = token count rounded up to the
- * tile sizes launch_mt knows (1, 2, 4, 8); Q8_0 activations are re-laid out to
- * 36 bytes per block. */
-static bool group_tile_fits_lds(int fmt, int K, int ntok)
-{
-    const size_t mt = ntok <= 1 ? 1 : ntok == 2 ? 2 : ntok <= 4 ? 4 : 8;
-    size_t bytes;
-    switch (fmt) {
-    case CKQ_FMT_Q4_K: case CKQ_FMT_Q5_K: case CKQ_FMT_Q6_K: bytes = FmtQ4K::xs_lds_bytes(mt * (size_t)(K / 256) * 292); break;
-    case CKQ_FMT_Q8_0: case CKQ_FMT_Q5_0:                     bytes = FmtQ80::xs_lds_bytes(mt * (size_t)(K / 32) * 34); break;
-    default: return false;
-    }
-    return bytes <= 65536;
-}
-
 /* `n` (2..CKQ_GROUP_MAX) independent matmuls of one format and input width,
  * each with its own number of rows - the Q/K/V (grouped-query attention makes
  * K and V narrower than Q) or the gate/up projections of a token - as one
@@ -578,10 +618,9 @@ extern "C" int ckq_launch_gemv_group(int fmt, int n, float *const *y, const void
         if (ldys[i] < rows[i] || ldys[i] > 0x7fffffff || !y[i]) return CKQ_EINVAL;
     for (int i = 0; i < n; ++i)
         if (!W[i] || !X[i]) return CKQ_EINVAL;
-    /* K-quants at three to eight tokens: one choice for all matrices; two never go there, and forced, below, all do. */
+    /* K-quants: one choice for all matrices */
     const bool kquant = !subdots && (fmt == CKQ_FMT_Q4_K || fmt == CKQ_FMT_Q5_K || fmt == CKQ_FMT_Q6_K) && K % 256 == 0;
-    const bool as_one = kquant && n > 1 && rows16_as_one(fmt, ntok, K);
-    if (as_one && group_takes_rows16(fmt, ntok, n, rows, K, group_tile_fits_lds(fmt, K, ntok))) {
+    if (kquant && n > 1 && group_route(fmt, n, rows, K, ntok) == CKQ_ROUTE_ROWS16_STREAM) {
         Rows16Args r = {};
         r.M = ntok; r.nb = K / 256; r.tree = true; r.n = n;
         for (int i = 0; i < n; ++i) r.p[i] = {(const uint8_t *)W[i], (const uint8_t *)X[i], y[i], bias ? bias[i] : nullptr, ldys[i], rows[i], 0, {}};
@@ -611,23 +650,6 @@ extern "C" int ckq_launch_gemv_group(int fmt, int n, float *const *y, const void
         }
         return ckq_launch_gemv_group(fmt, count, sy, sW, sX, sb, srows, sld, K, ntok, nullptr, stream);
     };
-    /* Matrices that the 16-row tiles take when launched alone share a launch of theirs, the others one of the streaming
-     * kernel: every result keeps the bits of its single launch. */
-    if (kquant && !as_one) {
-        Rows16Args r = {};
-        r.M = ntok; r.nb = K / 256; r.tree = true;
-        int rest[CKQ_GROUP_MAX], nrest = 0;
-        for (int i = 0; i < n; ++i) {
-            if (take_rows16(fmt, ntok, (size_t)rows[i], K, false))
-                r.p[r.n++] = {(const uint8_t *)W[i], (const uint8_t *)X[i], y[i], bias ? bias[i] : nullptr, ldys[i], rows[i], 0, {}};
-            else
-                rest[nrest++] = i;
-        }
-        if (r.n) {
-            const int rc = launch_gemm_rows16(fmt, r, (hipStream_t)stream);
-            return rc || !nrest ? rc : launch_some(rest, nrest);
-        }
-    }
     /* Q8_0 rows of an even number of blocks: matrices that start on a dword and ones that do not run different kernels */
     if (!subdots && fmt == CKQ_FMT_Q8_0 && K % 64 == 0) {
         int on[CKQ_GROUP_MAX], off[CKQ_GROUP_MAX], non = 0, noff = 0;
@@ -788,29 +810,19 @@ extern "C" int ckq_launch_gemm_group(int fmt, int n, float *const *C, const void
     }
     hipStream_t s = (hipStream_t)stream;
     if ((fmt == CKQ_FMT_Q4_K || fmt == CKQ_FMT_Q5_K || fmt == CKQ_FMT_Q6_K) && K % 256 == 0) {
-        /* 16-row tiles: in place of the tile kernels' shared launch where they would take it, else of the single launches
-         * (of one kind, as a launch has one order of its sums), with the bits of either */
         GemmChains shared = {};
-        const bool grouped = kquant_on_matrix_cores(fmt, M, rows, K) &&
-                             (fmt == CKQ_FMT_Q4_K   ? gemm_q4k_group_chains(in, M, K, &shared)
-                              : fmt == CKQ_FMT_Q5_K ? gemm_q5k_group_chains(in, M, K, &shared)
-                                                    : gemm_q6k_group_chains(in, M, K, &shared));
-        bool tiles[GEMM_GROUP_MAX], alike = true;
-        for (int p = 0; p < n; ++p) {
-            tiles[p] = grouped || kquant_on_matrix_cores(fmt, M, (size_t)N[p], K);
-            alike = alike && tiles[p] == tiles[0];
-        }
-        float t_singles = 0.0f;
-        for (int p = 0; p < n; ++p) t_singles += single_time(fmt == CKQ_FMT_Q4_K ? 0 : fmt == CKQ_FMT_Q5_K ? 1 : 2, (float)(K / 256), (size_t)N[p], M);
-        if (alike && take_rows16(fmt, M, rows, K, tiles[0], n, false, grouped ? (size_t)gemm_group_tiles(in, M, 64) : 0, t_singles)) {
+        bool grouped;
+        const int route = kquant_group_route(fmt, in, M, K, &grouped, &shared);
+        if (route == CKQ_ROUTE_ROWS16_TILES || route == CKQ_ROUTE_ROWS16_STREAM) {
+            const bool tiles = route == CKQ_ROUTE_ROWS16_TILES;
             Rows16Args r = {};
-            r.M = M; r.nb = K / 256; r.n = n; r.tree = !tiles[0];
+            r.M = M; r.nb = K / 256; r.n = n; r.tree = !tiles;
             for (int p = 0; p < n; ++p)
                 r.p[p] = {(const uint8_t *)B[p], (const uint8_t *)A, C[p], bias ? bias[p] : nullptr, ldc[p], N[p], 0,
-                          grouped ? shared : rows16_chains(fmt, M, N[p], K, tiles[p])};
+                          grouped ? shared : rows16_chains(fmt, M, N[p], K, tiles)};
             return launch_gemm_rows16(fmt, r, s);
         }
-        if (!grouped) return CKQ_ENOGROUP;
+        if (route == CKQ_ENOGROUP) return CKQ_ENOGROUP;
     }
     switch (fmt) {
     case CKQ_FMT_Q4_K:

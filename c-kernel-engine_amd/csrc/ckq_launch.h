@@ -52,9 +52,8 @@ int ckq_launch_gemv(int fmt, float *y, const void *W, const void *X, const float
 /* n (at most 4) independent matmuls of one format, input width and token count
  * (at most eight tokens; a token tile that does not fit in LDS is issued as
  * separate launches), problem i with rows[i] weight rows and output row stride
- * ldys[i], in one launch of the streaming kernel (K-quant matrices that run on
- * the 16-row tiles when launched alone share one of those, and Q8_0 matrices on
- * and off dword boundaries have a launch each); the arrays are host arrays
+ * ldys[i], in one launch of the streaming kernel or, K-quants, of the 16-row tiles
+ * (ckq_launch_group_route; Q8_0 matrices on and off dword boundaries have a launch each); the arrays are host arrays
  * (of device pointers), bias may be NULL or hold NULL entries.  `subdots`
  * non-NULL runs the dump build of the grouped kernel instead (y, ldys and bias
  * are then ignored): subdots[((g * ntok + t) * max_rows + row) * nsub + i]. */
@@ -88,6 +87,9 @@ void ckq_launch_set_gemm_policy(int policy);
  * either.  Host arithmetic; exported for the test of the rules. */
 enum { CKQ_ROUTE_STREAM = 0, CKQ_ROUTE_TILES = 1, CKQ_ROUTE_ROWS16_STREAM = 2, CKQ_ROUTE_ROWS16_TILES = 3 };
 int ckq_launch_route(int fmt, int nrows, int K, int ntok, int aligned);
+/* Where n (2..4) K-quant matrices of rows[i] rows against the same tokens go together: up to eight tokens CKQ_ROUTE_STREAM or CKQ_ROUTE_ROWS16_STREAM, beyond any of the routes (one launch for
+ * all) or CKQ_ENOGROUP, one by one.  Host arithmetic; exported for the test of the rules. */
+int ckq_launch_group_route(int fmt, int n, const int *rows, int K, int ntok);
 /* Token tile of the Q4_K x Q8_K matrix-core GEMM: 0 = by shape (default), 64 or 96 = that kernel wherever the GEMM is taken. */
 void ckq_launch_set_q4k_tile(int tokens);
 /* Q6_K x Q8_K matrix-core GEMM: 0 = by shape (default), 1 = one block per CU, 2 = the paired 64-token kernel,

@@ -244,6 +244,43 @@ def test_q4_k_short_rows_at_five_to_eight_tokens(L, n, k, tokens, want):
     assert route(L, "q4_k", n, k, tokens) == want
 
 
+APART = -7
+
+
+def group_route(L, fmt, tokens, k, ns):
+    return L.ckq_launch_group_route(ckq.parity.FMT[fmt], len(ns), (ctypes.c_int * len(ns))(*ns), k, tokens)
+
+
+@pytest.mark.parametrize("fmt", ["q4_k", "q5_k", "q6_k"])
+@pytest.mark.parametrize("tokens,k,ns,want", [
+    (8, 4352, (4352, 1088, 1088), ROWS16_STREAM), (5, 2560, (2560, 640, 640), ROWS16_STREAM), (6, 3072, (3072, 1536, 1536), ROWS16_STREAM), (5, 2048, (5632, 5632), ROWS16_STREAM),
+    (8, 1280, (1280, 320, 320), ROWS16_STREAM), (6, 7424, (1500, 1, 300), ROWS16_STREAM), (5, 16384, (700, 500), ROWS16_STREAM), (4, 4608, (4608, 1152, 1152), ROWS16_STREAM),
+    (7, 512, (512, 128, 128), STREAM), (8, 768, (1000, 17, 1), STREAM), (8, 256, (70, 4000), STREAM), (7, 11008, (96, 33), STREAM), (5, 16640, (64, 32), STREAM),
+    (4, 2560, (2560, 640, 640), STREAM), (3, 8192, (2100, 40), STREAM), (3, 14592, (300, 17), STREAM), (2, 4608, (4608, 600), STREAM)])
+def test_groups_of_few_tokens_have_one_kernel(L, fmt, tokens, k, ns, want):
+    """The sizes whose bits are compared on the GPU (test_matrices_of_three_to_eight_tokens_share_one_choice_of_kernel) lie on both sides of the line."""
+    assert group_route(L, fmt, tokens, k, ns) == want
+
+
+@pytest.mark.parametrize("fmt,tokens,k,ns,want", [
+    # three and four tokens, long rows
+    ("q6_k", 4, 11008, (3831, 3831, 3831), ROWS16_STREAM), ("q6_k", 3, 10496, (7984, 7984), ROWS16_STREAM), ("q6_k", 4, 6912, (8517, 4258, 4258), ROWS16_STREAM),
+    # too few tiles for a shared launch: one launch of 16-row tiles, or one by one
+    ("q5_k", 105, 2304, (2304, 2304, 2304), ROWS16_TILES), ("q6_k", 105, 2304, (2304, 2304, 2304), ROWS16_TILES), ("q5_k", 98, 3072, (3072, 1536, 1536), ROWS16_TILES),
+    ("q6_k", 64, 5120, (5120, 1280, 1280), ROWS16_TILES), ("q5_k", 313, 2560, (2560, 320, 320), ROWS16_TILES), ("q6_k", 17, 5120, (4100, 2561), ROWS16_TILES),
+    ("q5_k", 34, 8704, (8704, 1088, 1088), APART), ("q6_k", 34, 8704, (8704, 1088, 1088), APART), ("q5_k", 81, 4352, (4352, 1088, 1088), APART), ("q5_k", 17, 5120, (4100, 2561), APART),
+    # Q4_K against one launch of unsplit tiles, and against single launches
+    ("q4_k", 65, 1536, (6912, 6912), TILES), ("q4_k", 133, 1280, (3840, 3840), TILES), ("q4_k", 32, 3840, (11008, 11008), TILES), ("q4_k", 257, 768, (3584, 3584), TILES),
+    ("q4_k", 32, 1280, (10240, 10240), ROWS16_TILES), ("q4_k", 98, 2816, (2816, 1408, 1408), ROWS16_TILES)])
+def test_groups_go_where_they_were_timed_to_be_faster(L, fmt, tokens, k, ns, want):
+    assert group_route(L, fmt, tokens, k, ns) == want
+
+
+def test_group_route_refuses_what_is_no_group(L):
+    assert group_route(L, "q4_k", 8, 4096, (4096,)) == -1 and group_route(L, "q8_0", 8, 4096, (4096, 4096)) == -1
+    assert group_route(L, "q4_k", 8, 4000, (64, 64)) == -1 and group_route(L, "q4_k", 0, 4096, (64, 64)) == -1
+
+
 @pytest.mark.parametrize("M,Ns,last", [(405, (11008, 11008), True), (276, (7680, 7680), True), (139, (5888, 5888), True), (282, (7041,), True), (65, (17000,), True),
                                        (88, (9000, 7700), True), (341, (6912, 6912), False), (384, (11008, 11008), False), (227, (8960, 8960), False),
                                        (405, (4096, 1024, 1024), False), (9, (34000,), False), (400, (28672,), False)])
