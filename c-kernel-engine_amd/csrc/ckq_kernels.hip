@@ -683,8 +683,10 @@ extern "C" int ckq_launch_gemv_pro(int fmt, int n, float *const *y, const void *
     if (n < 1 || n > CKQ_GROUP_MAX || ntok < 1 || ntok > CKQ_STREAM_TOKENS || K < 256 || K > 2048 || K % 256 || stride < K || stride % 4) return CKQ_ENOGROUP;
     const size_t wblock = fmt == CKQ_FMT_Q4_K ? 144 : fmt == CKQ_FMT_Q5_K ? 176 : fmt == CKQ_FMT_Q6_K ? 210 : 0;
     if (!wblock || !x || !xq) return CKQ_ENOGROUP;
-    /* The 16-row tiles want quantized activations: the quantizer's launch and theirs. At five to eight tokens this kernel streams the weights for two tiles of tokens, and where they beat ONE
-     * streaming launch they are no slower with the quantizer (layers of 512 to 2048 columns, 5 and 8 tokens, against always this kernel: 0.97-1.09, 1.01 on average). */
+    /* The 16-row tiles want quantized activations: the producer's launch and theirs.  At five to eight tokens this kernel streams the weights for two tiles of tokens, and where they beat ONE
+     * streaming launch they are no slower with the producer: of 867 launches of 256 to 2048 columns that could be joined 7 yield, in two launches 0.74 to 1.00 of the joined time.  (40 more would be 3 to
+     * 24 % faster in two, most of them rows of one block; longer rows of the same models are past PRO_UNITS.)  Whole layers of 512 to 2048 columns, 5 to 8 tokens, against a choice by matrix: 0.945 on
+     * average, the slowest two of 300 1.02 and 1.01. */
     const bool as_one = rows16_as_one(fmt, ntok, K);
     if (as_one && ntok > 4 && group_takes_rows16(fmt, ntok, n, rows, K, true)) return CKQ_ENOGROUP;
     const size_t xbytes = ((size_t)(ntok - 1) * (size_t)stride + (size_t)K) * 4, qbytes = (size_t)ntok * (size_t)(K / 256) * 292;

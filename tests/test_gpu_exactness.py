@@ -173,6 +173,32 @@ def test_gemm_mfma_integer_block_sums_bit_exact(fmt):
         assert T.norm_err(c.cpu().numpy(), T.oracle_gemm_nt(fmt, A, W, None, M, N, K)) <= TOL
 
 
+@pytest.mark.parametrize("wo,xo", [(2, 0), (0, 2), (2, 2)])
+@pytest.mark.parametrize("M,N,K", [(70, 200, 896), (130, 333, 160), (33, 130, 192), (65, 131, 224), (33, 128, 32), (64, 96, 1120)])
+def test_q8_0_integer_block_sums_off_the_dwords(M, N, K, wo, xo):
+    """Operands two bytes behind a dword, which have a kernel of their own: its block dots against brute force, K ending after one to four blocks of a step and split in two; its fp32 result
+    against the oracle, and the production build's the same bits."""
+    import torch
+    W, A = rand_case("q8_0", N, K, 3 * M + N + K, tokens=M)
+    say("q8_0 block sums off the dwords", M, N, K, wo, xo)
+
+    def at(a, o):
+        buf = torch.zeros(len(a) + 4, dtype=torch.uint8, device="cuda")
+        buf[o:o + len(a)] = P.to_device(a)
+        return buf[o:o + len(a)]
+    Ad, Wd, bias = at(A, xo), at(W, wo), T.normal(N, 0.0, 0.5, seed=N)
+    assert Wd.data_ptr() % 4 == wo and Ad.data_ptr() % 4 == xo
+    c, sums = P.dev_gemm_block_sums("q8_0", Ad, Wd, P.to_device(bias), M, N, K)
+    assert np.array_equal(sums.cpu().numpy().astype(np.int64), np_block_sums("q8_0", W, A, M, N, K))
+    L = ckq.lib()
+    L.ckq_set_gemm_policy(1)
+    try:
+        prod = P.dev_gemm_nt("q8_0", Ad, Wd, P.to_device(bias), M, N, K)
+    finally:
+        L.ckq_set_gemm_policy(0)
+    assert torch.equal(c, prod) and T.norm_err(c.cpu().numpy(), T.oracle_gemm_nt("q8_0", A, W, bias, M, N, K)) <= TOL
+
+
 def test_gemm_mfma_block_sums_extremes():
     """Saturating operands: every nibble 15, every scale and min 63, every
     activation -128 / 127 and the largest stored bsums: the integer sums reach

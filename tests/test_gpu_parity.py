@@ -2236,6 +2236,38 @@ def test_gemm_mfma_q8_0_rows_of_an_odd_number_of_blocks(M, N, K):
         L.ckq_set_gemm_policy(0)
 
 
+@pytest.mark.parametrize("K", [160, 192, 224, 256, 1056, 1088, 1120])
+@pytest.mark.parametrize("M,Ns", [(257, (4100, 1, 129)), (70, (9100, 1027, 130)), (333, (3000, 777))])
+def test_grouped_q8_0_rows_of_every_number_of_blocks(M, Ns, K):
+    """One launch for several matrices whose rows end one, two, three or no blocks after the last whole step, one of a single row and odd ones among them (160 tiles and more: never split along K):
+    against fp64 at the bound of the tests of single matrices, and nothing beside C's columns."""
+    import torch
+    assert sum(-(-n // 128) for n in Ns) * -(-M // 64) >= 160
+    x = T.random_blocks("q8_0", M * (K // 32), 9870 + M)
+    ws = [T.random_blocks("q8_0", n * (K // 32), 9871 + n) for n in Ns]
+
+    def real(b, rows):
+        b = P.to_device(b).view(rows, K // 32, 34)
+        d = b[:, :, :2].contiguous().view(torch.float16).double()
+        return (d * b[:, :, 2:].contiguous().view(torch.int8).double()).reshape(rows, K)
+    say("q8_0 groups, blocks of a row", M, Ns, K)
+    xd, Ws = P.to_device(x), [P.to_device(w) for w in ws]
+    bs = [P.to_device(T.normal(n, 0.0, 0.5, seed=n)) for n in Ns]
+    ys = [torch.full((M, n + 3), 7.0, device="cuda") for n in Ns]
+    L = ckq.lib()
+    try:
+        L.ckq_set_gemm_policy(1)
+        P.dev_matmul_sequence([("q8_0", xd, W, b, y, M, n, K, n + 3) for W, b, y, n in zip(Ws, bs, ys, Ns)])
+    finally:
+        L.ckq_set_gemm_policy(0)
+    A = real(x, M)
+    for w, b, y, n in zip(ws, bs, ys, Ns):
+        B = real(w, n)
+        bound = (A.abs() @ B.abs().T) * (K // 32 + 4) * 2.0 ** -24 + b.abs().double() * 2.0 ** -23
+        assert bool(torch.isfinite(bound).all()) and bool((y[:, n:] == 7.0).all())
+        assert float(((y[:, :n].double() - b.double() - A @ B.T).abs() / bound).max()) <= 1.0, n
+
+
 @pytest.mark.parametrize("fmt,M,D,N", [("q4_k", 1, 768, (768, 64, 64)), ("q5_k", 1, 1024, (1024, 128, 128)), ("q6_k", 1, 2048, (2048, 17)), ("q5_k", 2, 1280, (200, 130, 7, 64)),
                                        ("q4_k", 3, 1024, (1000, 128, 1)), ("q5_k", 4, 1024, (1024, 128, 128)), ("q6_k", 4, 1792, (31,)), ("q4_k", 5, 1024, (130, 130)),
                                        ("q5_k", 8, 768, (65, 3)), ("q4_k", 1, 512, (512,)), ("q6_k", 4, 256, (300, 9)), ("q4_k", 1, 2304, (300,)), ("q5_k", 1, 1024, (40000,))])
@@ -2358,12 +2390,35 @@ def test_gemm_mfma_tiles_over_the_xcds(fmt, M):
             assert float((a - w).abs().max()) <= bar and float((b - w).abs().max()) <= bar
 
 
-@pytest.mark.parametrize("fmt", FMTS)
-@pytest.mark.parametrize("M,N,K", [(129, 1500, 7168), (65, 129, 16384), (200, 2700, 2304), (385, 1700, 3328)])
+PIECES_OF_K = [(65, 1100, 7936), (40, 300, 5376), (65, 650, 11008), (129, 1200, 1664), (129, 1200, 5376), (129, 1200, 6656), (129, 1500, 7168), (65, 129, 16384), (200, 2700, 2304), (385, 1700, 3328)]
+
+
+def _pieces_of_k(tiles, steps):
+    """(pieces, steps of each but the last) of a launch of `tiles` tiles that is split along K."""
+    s = max(1, min(256 // tiles, steps // 4, 16)) if tiles < 160 and steps >= 8 else 1
+    per = -(-steps // s)
+    return -(-steps // per), per
+
+
+def test_sizes_of_the_pieces_of_k_are_uneven():
+    """Of the first five sizes below the 64-token tiles of the K-quants, and of the first three and the fourth the 32-, 64- and 96-token tiles of Q8_0: more than four pieces (fewer may be waves of
+    one block instead), a shorter last one, and a number of pieces of all tiles that eight does not divide."""
+    for M, N, K in PIECES_OF_K[:3] + PIECES_OF_K[4:6]:
+        tiles = -(-M // 64) * -(-N // 128)
+        pieces, per = _pieces_of_k(tiles, K // 256)
+        assert pieces > 4 and tiles * pieces % 8 and K // 256 % per, (M, N, K)
+    for M, N, K in PIECES_OF_K[:4]:
+        for tokens in (32, 64, 96):
+            tiles = -(-M // tokens) * -(-N // 128)
+            pieces, per = _pieces_of_k(tiles, -(-K // 128))
+            assert pieces > 1 and tiles * pieces % 8 and -(-K // 128) % per, (M, N, K, tokens)
+
+
+@pytest.mark.parametrize("fmt,M,N,K", [(fmt, *size) for fmt in FMTS for size in PIECES_OF_K if size[2] % T.ELEMS[fmt] == 0])
 def test_gemm_pieces_of_k_dealt_with_their_tiles(fmt, M, N, K):
-    """Every piece of K of every tile is computed once where neither their number nor that of the tiles divides by the eight XCDs: 36 tiles in up to seven
-    pieces (the last one shorter), 4 in sixteen, 88 in two, 98 in two.  Against the streaming kernel, whose terms and order differ: the bar of
-    the other parity tests."""
+    """Every piece of K of every tile is computed once, where eight XCDs divide neither the number of pieces nor that of the tiles and the last piece is shorter (the test above); where they do
+    (36 tiles in seven equal pieces, of Q8_0 in more; 4 in sixteen); and where the K-quants' pieces are waves of one block instead (two of 5 and of 7 blocks, the last two sizes).
+    Against the streaming kernel, whose terms and order differ: the bar of the other parity tests."""
     import torch
     L = ckq.lib()
     say("pieces of K over the XCDs", fmt, M, N, K)

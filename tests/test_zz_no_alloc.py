@@ -76,6 +76,30 @@ def test_noalloc_entry_point_matches_allocating_one(fmt):
         L.ckq_set_gemm_policy(0)
 
 
+def test_noalloc_q8_0_rows_of_an_odd_number_of_blocks():
+    """Rows of an odd number of blocks: refused where the split of 64-token tiles has no room in the scratch, whichever tiles would be taken; else the bits of the allocating entry point."""
+    import torch
+    L = ckq.lib()
+    assert L.ckq_init() == 0
+    L.ckq_set_gemm_policy(1)
+    try:
+        # MiB of partial tiles: 8, 4.005, 0.97, 2.54, 2.56
+        for M, N, K, fits in [(512, 1024, 2592, False), (300, 700, 2592, False), (33, 1100, 4128, True), (512, 260, 2592, True), (64, 2100, 2592, True)]:
+            tiles, steps = -(-M // 64) * -(-N // 128), -(-K // 128)
+            s = min(256 // tiles, steps // 4, 16)
+            pieces = -(-steps // -(-steps // s))
+            assert pieces > 1 and (pieces * M * N * 4 <= 4 << 20) == fits, (tiles, pieces)
+            W, A = T.random_blocks("q8_0", N * (K // 32), 370 + M), T.random_blocks("q8_0", M * (K // 32), 371 + M)
+            say("no-alloc entry point, odd number of blocks", M, N, K)
+            Ad, Wd = P.to_device(A), P.to_device(W)
+            rc, got = noalloc("q8_0", Ad, Wd, None, M, N, K)
+            want = P.dev_gemm_nt("q8_0", Ad, Wd, None, M, N, K)
+            assert rc == (0 if fits else ESCRATCH)
+            assert torch.equal(got, want) if fits else bool((got == 5.0).all())
+    finally:
+        L.ckq_set_gemm_policy(0)
+
+
 def test_noalloc_entry_point_leaves_device_memory_untouched():
     """The free device memory the driver reports is the same before and after
     the calls (operands and output allocated beforehand, ckq_init() done): a
