@@ -352,7 +352,8 @@ static float keep_time_own_scratch(int f, size_t rows, int ntok)
     return least < 4.4f + 1e-3f * (f == 1 ? 4.98f : 5.82f) * (float)(tiles * groups) ? least : 0.0f;
 }
 static float rows16_q4k_time(float nb, size_t rows, int ntok) { return 3.6f + 0.12f * nb + 0.58e-3f * nb * (float)((rows + 15) / 16) * (float)((ntok + 15) / 16); }
-/* A matrix of fewer than 160 tiles on its own: split along K or not, or by the 16-row kernel (Q5_K, Q6_K: fitted to 631 launches of whichever the rule takes, 17 to 130 tokens, 12 % rms). */
+/* A matrix of fewer than 160 tiles on its own: split along K or not, or by the 16-row kernel (Q5_K, Q6_K: fitted to 631 launches of whichever the rule takes, 17 to 130 tokens, 12 % rms; Q4_K rows of
+ * less than eight blocks, never split, by their length alone: one round of tiles). */
 static float single_time(int f, float nb, size_t rows, int ntok)
 {
     static const float c[2][6] = {{2.09f, 0.224f, 0.218f, 13.8f, 0.50f, 176e-6f}, {2.13f, 0.232f, 0.127f, 15.0f, 0.565f, 210e-6f}};
@@ -363,14 +364,15 @@ static float single_time(int f, float nb, size_t rows, int ntok)
 /* Three to eight tokens, `rows` rows in one launch of either kernel; the streaming kernel's grid follows the largest of its matrices: `grid_rows`, their number times its
  * rows. The figures are described above; at three and four tokens the 16-row tiles have to be ahead by a tenth, as the times lie closer than
  * the fits do there. */
-static float rows16_one_pass_time(int f, int ntok, size_t rows, int K)
+static float rows16_one_pass_time(int f, int ntok, size_t rows, int K, bool alone = true)
 {
     static const float c[2][3][4] = {{{3.04f, 0.142f, 3.73f, 0.311f}, {3.15f, 0.151f, 3.88f, 0.279f}, {3.27f, 0.188f, 3.86f, 0.288f}},
                                      {{3.38f, 0.116f, 3.71f, 0.327f}, {3.45f, 0.133f, 3.83f, 0.296f}, {3.39f, 0.181f, 3.76f, 0.291f}}}, block[3] = {144e-6f, 176e-6f, 210e-6f};
     const float nb = (float)(K / 256), *t = c[ntok > 4][f];
     /* Q4_K, five to eight tokens, rows of up to four blocks: by the fit alone they streamed where the 16-row tiles are the faster ones and had been taken (us, streaming | 16-row tiles: 8 x 8695 x 1024
-     * 5.55 | 4.77, 5 x 7256 x 1024 4.62 | 4.31; 242 such launches: the choice costs 0.9 % more than the faster kernel, 3.4 without) */
-    const float short_rows = f == 0 && ntok > 4 && nb <= 4.0f ? 0.93f : 1.0f;
+     * 5.55 | 4.77, 5 x 7256 x 1024 4.62 | 4.31; 242 such launches: the choice costs 0.9 % more than the faster kernel, 3.4 without).  Not against a launch that has the producer too (`alone`): 5 x 13113 x 256
+     * 5.7 in one, 7.2 in two */
+    const float short_rows = alone && f == 0 && ntok > 4 && nb <= 4.0f ? 0.93f : 1.0f;
     return (ntok > 4 ? short_rows : 1.1f) * fmaxf(t[0] + t[1] * nb, t[2] + t[3] * nb * (float)rows * block[f]);
 }
 static float stream_one_pass_time(int f, int ntok, size_t rows, size_t grid_rows, int K)
@@ -395,7 +397,7 @@ static bool rows16_as_one(int fmt, int ntok, int K)
 {
     return ntok > 2 && ntok <= CKQ_STREAM_TOKENS && K <= ROWS16_MAX_K && g_gemm_policy.load(std::memory_order_relaxed) != 2 && !(g_rows16_forced.load(std::memory_order_relaxed) >> fmt & 1);
 }
-static bool group_takes_rows16(int fmt, int ntok, int n, const int *rows, int K, bool streams_as_one)
+static bool group_takes_rows16(int fmt, int ntok, int n, const int *rows, int K, bool streams_as_one, bool alone = true)
 {
     const int f = fmt == CKQ_FMT_Q4_K ? 0 : fmt == CKQ_FMT_Q5_K ? 1 : 2;
     size_t all = 0, largest = 0;
@@ -406,7 +408,7 @@ static bool group_takes_rows16(int fmt, int ntok, int n, const int *rows, int K,
         if (r > largest) largest = r;
         apart += fminf(rows16_one_pass_time(f, ntok, r, K), stream_one_pass_time(f, ntok, r, r, K));
     }
-    return q6k_long_rows_of_few_tokens(f, ntok, all, K) || rows16_one_pass_time(f, ntok, all, K) < (streams_as_one ? stream_one_pass_time(f, ntok, all, largest * (size_t)n, K) : apart);
+    return q6k_long_rows_of_few_tokens(f, ntok, all, K) || rows16_one_pass_time(f, ntok, all, K, alone) < (streams_as_one ? stream_one_pass_time(f, ntok, all, largest * (size_t)n, K) : apart);
 }
 static bool take_rows16(int fmt, int ntok, size_t rows, int K, bool tiles, int launches = 1, bool own_scratch = false, size_t shared_tiles = 0, float t_singles = 0.0f)
 {
@@ -688,7 +690,7 @@ extern "C" int ckq_launch_gemv_pro(int fmt, int n, float *const *y, const void *
      * 24 % faster in two, most of them rows of one block; longer rows of the same models are past PRO_UNITS.)  Whole layers of 512 to 2048 columns, 5 to 8 tokens, against a choice by matrix: 0.945 on
      * average, the slowest two of 300 1.02 and 1.01. */
     const bool as_one = rows16_as_one(fmt, ntok, K);
-    if (as_one && ntok > 4 && group_takes_rows16(fmt, ntok, n, rows, K, true)) return CKQ_ENOGROUP;
+    if (as_one && ntok > 4 && group_takes_rows16(fmt, ntok, n, rows, K, true, false)) return CKQ_ENOGROUP;
     const size_t xbytes = ((size_t)(ntok - 1) * (size_t)stride + (size_t)K) * 4, qbytes = (size_t)ntok * (size_t)(K / 256) * 292;
     if (ckq_ranges_overlap(xq, qbytes, x, xbytes) || (gamma && ckq_ranges_overlap(xq, qbytes, gamma, (size_t)K * 4))) return CKQ_ENOGROUP;
     GemvArgs a = {};

@@ -2308,7 +2308,8 @@ def test_sequence_producer_joined_with_its_matmuls(fmt, M, D, N, step):
 
 
 @pytest.mark.parametrize("fmt,M,D,N", [("q4_k", 2, 1024, (8192, 64, 64)), ("q5_k", 4, 1024, (8000, 40, 40)), ("q6_k", 3, 768, (7990, 33, 5)), ("q4_k", 2, 512, (11000, 70, 9)),
-                                       ("q5_k", 3, 512, (11000, 70, 9)), ("q6_k", 2, 1280, (2800, 33, 16)), ("q5_k", 2, 2048, (3000, 500, 64)), ("q4_k", 2, 1024, (16384,))])
+                                       ("q5_k", 3, 512, (11000, 70, 9)), ("q6_k", 2, 1280, (2800, 33, 16)), ("q5_k", 2, 2048, (3000, 500, 64)), ("q4_k", 2, 1024, (16384,)),
+                                       ("q4_k", 5, 256, (13113,))])
 def test_producer_joined_with_two_rows_a_slot(fmt, M, D, N):
     """Wide matrices, narrow ones beside them, that take one launch with their producer at two rows a slot: it is taken, and every buffer has the
     bits of the steps one by one."""
