@@ -17,7 +17,8 @@ typedef __attribute__((address_space(3))) void ckq_lds_void;
 typedef const __attribute__((address_space(1))) void ckq_glb_void;
 
 /* One weight matrix of a grouped launch: several matrices that multiply the same activations (Q/K/V,
- * gate/up) share a grid; a matrix owns the block ids [id0, id0 + gemm_blocks(ntt, nnt)). */
+ * gate/up) share a grid.  id0 is where a matrix begins: among the tiles of all matrices, which are dealt as one (GemmArgs::units; gemm_launch_grouped); among the tiles of
+ * weight rows (ckq_gemm_q4k_t96.hip); or its first block id, of gemm_blocks(ntt, nnt), where every matrix is dealt by itself (units = 0; gemm_deal_ragged_last). */
 constexpr int GEMM_GROUP_MAX = 4;
 struct GemmProblem {
     const uint8_t *B;
@@ -114,7 +115,7 @@ struct GemmWork { int tile, k0, k1; GemmOut out; const uint8_t *B; int N, nnt, t
 /* A launch of pieces of K is as wide as the chip (gemm_choose_splits), and takes as long as its fullest XCD: 84 tiles in three pieces, 252 blocks, were 33 for
  * the 32 CUs of four XCDs, and so two rounds, as long as each piece's tiles were dealt by themselves (three matrices of 84 tiles were 33 where 32 do).  All pieces of all tiles
  * are dealt as one, piece by piece, so that an XCD has one or two pieces of K of many tiles, which share activations as well as weights.  us, tokens x
- * rows x K: Q6_K 384 x 1792 x 6400 43.3 -> 30.5, Q5_K 150 x 3584 x 9984 60.7 -> 36.2, Q4_K 379 x 768 x 7168 25.8 -> 21.5, Q8_0 321 x 1792 x 4864 32.3 -> 25.9; 48
+ * rows x K: Q6_K 384 x 1792 x 6400 43.3 -> 30.5, Q5_K 150 x 3584 x 9984 60.7 -> 36.2, Q4_K 379 x 768 x 7168 25.8 -> 21.5, Q8_0 321 x 1792 x 4864 32.3 -> 25.9; 49
  * sizes of that kind 1.29 on average (1.02 to 1.68), 60 others 1.00.  The sums and their order are the same. */
 __device__ __forceinline__ GemmWork gemm_work(const GemmArgs &a, int k_steps)
 {
@@ -323,7 +324,7 @@ static int gemm_launch_ksplit(Kernel k2, Kernel k3, Kernel k4, GemmArgs &g, int 
 }
 
 /* Grouped launch: the matrices of `in` against the same M x K activations, as one grid (no K split; the
- * callers group only what fills the chip without one).  rows_per_tile = weight rows of a block's tile. */
+ * callers group only what fills the chip without one). */
 struct GemmGroupIn {
     int          n;
     const void  *B[GEMM_GROUP_MAX];

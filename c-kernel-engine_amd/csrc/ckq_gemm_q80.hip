@@ -32,9 +32,8 @@
  *
  * Block = 4 waves = 64 tokens x 128 weight rows; wave w owns rows 32w..32w+31.
  *
- * Rows that start on dwords and hold an even number of blocks go to ckq_gemm_q80_dw.hip, 1.2 to 1.45 times as fast for
- * copying them in memory order; with an odd number every other row is two bytes off, and moving those in LDS cost what the
- * better copies gave (333 x 4864 x 4064: 52.7 us against 46.6 here).
+ * This kernel has the operands that start two bytes behind a dword.  The others go to ckq_gemm_q80_dw.hip, which copies rows in memory order:
+ * 1.2 to 1.45 times as fast for an even number of blocks a row, 1.05 to 1.58 for an odd one.
  */
 #include "ckq_gemm_common.hpp"
 #include <type_traits>

@@ -12,7 +12,8 @@
  *   exactly M + S (M = 1.5 * 2^23, |S| < 2^20).  t = fma(dw, M + S, -dw M) is dw S rounded once (dw M has 13 bits), and acc =
  *   fma(dx, t, acc): two plain fp32 operations per output and block, against the other kernel's convert, product and
  *   multiply-add with a lane broadcast.
- *   A row whose fp16 scale is infinite gives NaN that way; such outputs are summed again term by term at the end.
+ *   A row whose fp16 scale is infinite gives NaN that way; such outputs are summed again term by term at the end.  That is for broken inputs only:
+ *   where every output is NaN, a launch takes up to 50 times as long (397 x 3 x 2458 x 1696 2030 us).
  * - Tokens are the A operand, weight rows the B operand: lane 16 q + i holds ONE weight row and tokens 4 q .. 4 q + 3 of a
  *   16 x 16 result.  LDS row 64 h + 16 g + i is weight row 64 h + 4 i + g, so a lane ends with four adjacent rows.
  * - K advances 128 (four blocks) per iteration, two stages.  Of the eight waves, four take two of the blocks and four the
@@ -67,7 +68,9 @@ __device__ __forceinline__ float q80_output(const uint8_t *w, const uint8_t *x, 
  * sixteen, so dwords 30 to 33 of the run lie at 32 to 35 (of an odd number of blocks, whose run may start two bytes early, dwords 31 to 34).  A pair of blocks is 17 dwords: [d0 q0q1] seven of quants [q30q31 d1]
  * eight of quants.  Once a row has landed, the lane in charge makes [q0q1 q30q31] of the first and the ninth - the order of
  * the 32 products of a block is free as long as both operands have the same - and leaves the scales as fp32.  Lane quarter q takes
- * dwords q and q + 4 of a block: with rows 36 dwords apart, and the waves' regions a multiple of four rows, every bank serves one lane.
+ * dwords q and q + 4 of a block: a dword at a time, with rows 36 dwords apart and the waves' regions a multiple of four rows, every bank would serve one lane.
+ * But the two are one instruction (ds_read2_b32), and two dwords for each of 32 lanes fall on half of the banks twice: sixteen rows lie on those of one residue modulo 4,
+ * and q and q + 4 have the same one.  Conflicts are 17 to 23 % of the busy cycles by the counters, other kernels here have 0 to 6; two dwords in a row are not tried.
  */
 template <int TG, int TEAMS, int ROWS, bool DUMP>
 __global__ void __launch_bounds__(GEMM8_THREADS * TEAMS, DUMP ? 2 : 4) gemm_q80_dw_kernel(GemmArgs a)

@@ -19,8 +19,8 @@
  * would otherwise run on: the streaming kernel's term per 64 elements and tree (TREE), or the tile kernels' term per
  * 256-block and chains (GemmChains).  The terms meet in LDS; one thread per output adds them.
  *
- * Bound: VALU issue (110-260 operations per 256-block of 16 rows) next to HBM and, for small matrices, one latency after
- * another.  Measured, weights from HBM, against the kernel that served the shape before (us): Q4_K 4096 x 4096 at 8 / 13 / 32
+ * Bound: for one token group nothing alone.  Vector instructions (110-260 per 256-block of 16 rows) issue in 36 to 51 % of the busy CUs' cycles, waves wait in
+ * 35 to 45 %, and a block's loads, terms and sums add up; for several groups it is VALU issue (64 % at 93 tokens x 4864 x 1024).  Measured, weights from HBM, against the kernel that served the shape before (us): Q4_K 4096 x 4096 at 8 / 13 / 32
  * tokens 7.5 -> 6.1, 10.0 -> 6.5, 13.1 -> 8.1; 11008 x 4096 at 8 / 13: 14.7 -> 10.3, 15.6 -> 9.7; Q6_K 32000 x 4096 at
  * 8 / 13: 40.6 -> 27.1, 46.2 -> 28.3; 4096 x 11008 at 13: 20.7 -> 15.8; Q5_K 1024 x 4864 at 64: 16.8 -> 8.0.
  */
@@ -74,7 +74,8 @@ __device__ __forceinline__ ckq_v4i lds16(const uint8_t *p) { return *reinterpret
  * + 7 of slab s), the integers of a slab then times its scale, which a lane has for its row: four multiply-adds where forming planes and putting their sums
  * together costs more than the matrix instructions it saves (vector instructions of a 256-block in the first kernel, planes -> slabs: Q4_K 129 -> 110, in the streaming
  * kernel's order 215 -> 184, Q5_K 247 -> 140 and 333 -> 214, Q6_K 236 -> 186 and 292 -> 256; us, weights from the cache, tokens x rows x K: Q5_K 13 x 6144 x 4096 10.8 -> 9.3, 8 x 11008 x 4096 13.4 ->
- * 11.1, 6 x 4096 x 11008 12.5 -> 10.1; Q4_K 8 x 11008 x 4096 10.8 -> 10.2, 13 x 4096 x 11008 11.8 -> 11.4; Q6_K 13 x 4096 x 11008 14.0 -> 13.3, 16 x 3584 x 9728 13.2 -> 12.8).  Q6_K has a scale every 16: a second product with the first half of the tokens' run alone, times the
+ * 11.1, 6 x 4096 x 11008 12.5 -> 10.1; Q4_K 8 x 11008 x 4096 10.8 -> 10.2, 13 x 4096 x 11008 11.8 -> 11.4; Q6_K 13 x 4096 x 11008 14.0 -> 13.3, 16 x 3584 x 9728 13.2 -> 12.8;
+ * Q6_K rows of two to four blocks lose up to 6 % where there are 8000 to 32000 of them, 8 x 15986 x 768 6.4 -> 6.7, 12 and 16 tokens the same, and gain 1 to 4 beyond).  Q6_K has a scale every 16: a second product with the first half of the tokens' run alone, times the
  * difference of the two scales.  raw(): the operands of SLABS slabs of the row at r, Q6_K 4 (q - 32); scales(): sc[s], or of Q6_K sc[2 s + half]. */
 __device__ __forceinline__ long two_dwords(u32 lo, u32 hi) { return (long)((uint64_t)lo | ((uint64_t)hi << 32)); }
 __device__ __forceinline__ void scales_k45(int (&sc)[16], const uint8_t *r)
